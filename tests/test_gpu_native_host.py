@@ -1,0 +1,69 @@
+"""The native host path (csrc/host_ext.cpp) against the Python launchers it stands in for: the same kernels on the same
+operands, so the same bits, in every layout it takes; and it leaves the operands it does not take to them."""
+import pytest
+import torch
+
+import acsr_helpers as A
+import _splat_hip as hip
+from r_attention import RegularAttention, _AttentionFunction, attention_launcher, attention_with_grad
+
+pytestmark = pytest.mark.gpu
+
+
+def _operands(dev, B, H, L, d, dtype, layout):
+    g = torch.Generator(device="cpu").manual_seed(L + d)
+
+    def one():
+        if layout == "tokens":
+            return torch.randn(B, L, H, d, generator=g).to(dtype).to(dev).transpose(1, 2)
+        if layout == "odd offset":  # rows that do not start on 16-byte boundaries: not an ordinary case
+            return torch.randn(B * H * L * d + 1, generator=g).to(dtype).to(dev)[1:].view(B, H, L, d)
+        return torch.randn(B, H, L, d, generator=g).to(dtype).to(dev)
+    q, k, v = one(), one(), one()
+    kT = k.transpose(2, 3)
+    return q, k, (kT.contiguous() if layout == "keys" else kT), v
+
+
+@pytest.mark.parametrize("layout", ["rows", "tokens", "keys", "odd offset"])
+@pytest.mark.parametrize("L,masks", [(520, lambda L: A.causal_windowed_pattern(L, 99)), (333, lambda L: A.windowed_pattern(L, 40)),
+                                     (384, lambda L: A.strided_patterns(L, 32, 16))])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_native_forward_equals_the_launcher(dev, layout, L, masks, dtype):
+    B, H, d = 2, 3, 64
+    attn = RegularAttention(B, L, H, d, masks(L), 16, 16, dev, dtype, scale=d ** -0.5)
+    q, _, kT, v = _operands(dev, B, H, L, d, dtype, layout)
+    first = attn([q, kT, v]).clone()   # builds the plan: the launcher
+    taken = hip.host().forward(attn._native, q, kT, v, attn.rspmm_output.zero_(), attn.scale)
+    assert taken == (layout != "odd offset")
+    again = attn([q, kT, v])
+    want = attention_launcher(q, kT, v, torch.empty_like(first), attn.segments, attn.scale, attn._plan)
+    assert torch.equal(first, want) and torch.equal(again, want)
+
+
+@pytest.mark.parametrize("layout", ["rows", "tokens", "odd offset"])
+@pytest.mark.parametrize("L,masks", [(520, lambda L: A.causal_windowed_pattern(L, 99)), (8192, lambda L: A.strided_patterns(L, 64, 64))])
+@pytest.mark.parametrize("dtype,d", [(torch.float16, 64), (torch.bfloat16, 128)])
+def test_native_gradients_equal_the_python_function(dev, layout, L, masks, dtype, d):
+    B, H = 2, 2
+    attn = RegularAttention(B, L, H, d, masks(L), 16, 16, dev, dtype, scale=d ** -0.5)
+    q, k, _, v = (t.requires_grad_(True) for t in _operands(dev, B, H, L, d, dtype, layout))
+    go = torch.randn(B, H, L, d, device=dev).to(dtype)
+    out = attention_with_grad(q, k, v, attn)
+    got = torch.autograd.grad(out, (q, k, v), go)
+    ref = _AttentionFunction.apply(q, k, v, attn)
+    want = torch.autograd.grad(ref, (q, k, v), go)
+    assert torch.equal(out, ref) and all(torch.equal(a, b) for a, b in zip(got, want))
+    with torch.no_grad():
+        assert torch.equal(attention_with_grad(q, k, v, attn), ref)
+
+
+def test_native_operators_refuse_what_the_launchers_check(dev):
+    """Operands of the wrong shape or type fall through to the launchers and their messages."""
+    L, d = 256, 64
+    attn = RegularAttention(1, L, 2, d, A.causal_windowed_pattern(L, 31), 16, 16, dev, torch.bfloat16, scale=1.0)
+    q = torch.randn(1, 2, L, d, device=dev).to(torch.bfloat16)
+    attn([q, q.transpose(2, 3), q])
+    with pytest.raises(hip.SplatError):
+        attn([q[:, :, :128], q[:, :, :128].transpose(2, 3), q[:, :, :128]])
+    assert not hip.host().forward(attn._native, q, q.float().transpose(2, 3), q, attn.rspmm_output, 1.0)
+    assert not hip.host().softmax(attn.segments.native(L, dev, False), q, q[:, :1])

@@ -6,6 +6,8 @@ present, every operator raises -- there is no host fallback.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 from typing import Any, Sequence
 
@@ -14,6 +16,7 @@ import torch
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # SPLAT_HIP_LIB selects another build of the same library (e.g. an instrumented one)
 LIB_PATH = os.environ.get("SPLAT_HIP_LIB") or os.path.normpath(os.path.join(_HERE, "..", "lib", "libsplat_hip.so"))
+HOST_PATH = os.path.normpath(os.path.join(_HERE, "..", "lib", "_splat_host.so"))
 
 SPLAT_F32, SPLAT_F16, SPLAT_BF16 = 0, 1, 2
 MAX_SEGMENTS = 4
@@ -35,6 +38,7 @@ class AcsrSeg(ctypes.Structure):
 
 
 _lib = None
+_host = None
 
 _i32, _i64, _f32, _vp = ctypes.c_int32, ctypes.c_int64, ctypes.c_float, ctypes.c_void_p
 _SIGNATURES = {
@@ -99,6 +103,21 @@ def lib() -> ctypes.CDLL:
             fn.argtypes = args
         _lib = handle
     return _lib
+
+
+def host():
+    """The native host path (csrc/host_ext.cpp), loaded once and bound to the library's entry points: operator calls without
+    the interpreter's share of the argument checks, the strides and the C-ABI call, and the differentiable attention."""
+    global _host
+    if _host is None:
+        if not os.path.exists(HOST_PATH):
+            raise SplatError(f"{HOST_PATH} is missing: build it with `python triton-fun_amd/build.py`")
+        loader = importlib.machinery.ExtensionFileLoader("_splat_host", HOST_PATH)
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_splat_host", loader))
+        loader.exec_module(mod)
+        mod.bind({name: ctypes.cast(getattr(lib(), name), _vp).value for name in EXPORTS}, SplatError)
+        _host = mod
+    return _host
 
 
 def check(rc: int, what: str) -> None:

@@ -17,6 +17,7 @@ from dataclasses import dataclass
 from math import ceil
 from typing import Any, Sequence, Type
 
+import ctypes
 import hashlib
 import weakref
 
@@ -412,7 +413,7 @@ class ACSRSegments:
             self.offsets.append(off)
             off += int(t[5])
         self.T = off
-        self._plan_holder = None  # where plan() keeps its tables when not with this object
+        self._plan_holder = None  # where plan() and native() keep what they build when not with this object
         self._arrays = {}  # seg_array()'s results
 
     def __len__(self) -> int:
@@ -462,14 +463,7 @@ class ACSRSegments:
                 _hip.check(rc, "splat_attention_plan")
                 # once, so that later launches may run on any stream without ordering themselves after the plan kernel
                 torch.cuda.current_stream(dev).synchronize()
-                # whether every live row starts on a multiple of 8 positions of its block's walk (blocked masks): one look
-                # at the rows' records of the first variant (gathered walks), which follow its 5 records per block and
-                # segment: [lo, cnt, lin, phase] each
-                n_rb = nbytes // (2 * len(self) * (5 + 128) * 16)
-                recs = table.view(torch.int32).view(-1, 4)
-                rows = recs[n_rb * len(self) * 5:n_rb * len(self) * (5 + 128)]
-                aligned = bool((((rows[:, 0] & 7) == 0) | (rows[:, 1] <= 0)).all())
-            plans[key] = (table, aligned)
+            plans[key] = [table, None]
         return plans[key][0]
 
     def has_plan(self, L: int, device) -> bool:
@@ -479,11 +473,40 @@ class ACSRSegments:
         return (int(L), len(self), tuple(self.offsets), dev.index) in getattr(holder, "splat_plans", {})
 
     def plan_is_aligned(self, L: int, device) -> bool:
-        """Whether every row of the plan for ``L`` rows starts on a multiple of 8 positions (see ``plan``)."""
-        self.plan(L, device)
+        """Whether every live row starts on a multiple of 8 positions of its block's walk in the plan for ``L`` rows (blocked
+        masks): one look at the rows' records of the first variant (gathered walks), which follow its 5 records per block
+        and segment: [lo, cnt, lin, phase] each."""
+        table = self.plan(L, device)
         holder = self._plan_holder if self._plan_holder is not None else self
         dev = _hip.resolve_device(device)
-        return holder.splat_plans[(int(L), len(self), tuple(self.offsets), dev.index)][1]
+        entry = holder.splat_plans[(int(L), len(self), tuple(self.offsets), dev.index)]
+        if entry[1] is None:
+            n_rb = table.numel() // (2 * len(self) * (5 + 128) * 16)
+            recs = table.view(torch.int32).view(-1, 4)
+            rows = recs[n_rb * len(self) * 5:n_rb * len(self) * (5 + 128)]
+            entry[1] = bool((((rows[:, 0] & 7) == 0) | (rows[:, 1] <= 0)).all())
+        return entry[1]
+
+    def native(self, L: int, device, with_plan: bool):
+        """The segments as the native host path takes them (``_splat_hip.host().mask``), with the plan table or without, built
+        on first use and kept where ``plan`` keeps its tables; None under stream capture when it would have to be built
+        (building synchronises).  The metadata is taken to be immutable from then on."""
+        holder = self._plan_holder if self._plan_holder is not None else self
+        kept = holder.__dict__.get("splat_native")
+        if kept is None:
+            kept = holder.__dict__["splat_native"] = {}
+        # (the tensors' addresses: separate tensors may come with one sTod_translations and other companions)
+        key = (L, device.index, with_plan) if holder is self else \
+            (L, device.index, with_plan, *(t.data_ptr() for t in self.tuples[0][:5]))
+        mask = kept.get(key)
+        if mask is None:
+            if torch.cuda.is_current_stream_capturing():
+                return None
+            arr = self.seg_array(L)
+            own = [t for seg in self.seg_args() for t in seg[:6] if t is not None and t is not holder]
+            mask = kept[key] = _hip.host().mask(ctypes.addressof(arr), len(self), L, self.plan(L, device) if with_plan else None,
+                                                self.max_step, tuple(own))
+        return mask
 
     def seg_args(self) -> list[tuple]:
         return [(t[0], t[1], t[2], t[3], t[4], fc, off) for t, fc, off in zip(self.tuples, self.first_cols, self.offsets)]

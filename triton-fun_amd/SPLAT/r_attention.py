@@ -162,6 +162,8 @@ class RegularAttention(nn.Module):
         self._segments_t = None  # ACSR of the transposed mask(s), built on the first backward
         self._plan_t = None  # the fused backward's plan of the transposed mask
         self._lse = None  # the rows' softmax statistics, allocated by the first forward_with_stats
+        self._native = None  # the mask as the native host path takes it, once the plan exists
+        self._native_grad = None  # what the native differentiable path keeps (False: this module cannot use it)
         self._BLOCK_HEIGHT = BLOCK_SIZE_Y
 
     # The two [B, H, L, T] intermediates and the reference's launch geometry exist only for the unfused path.
@@ -198,12 +200,12 @@ class RegularAttention(nn.Module):
         """x = [q, kT, v] after RoPE: q [B, H, L, d], kT [B, H, d, L], v [B, H, L, d].  Returns the module's
         output buffer (reused by every call)."""
         q, k, v = x
+        if self.fused and self._native is not None and \
+                _hip.host().forward(self._native, q, k, v, self.rspmm_output, self.scale):
+            return self.rspmm_output
         fusable = self.fused and q.shape[-1] in (64, 128) and q.dtype == k.dtype == v.dtype == self._out_dtype
         if fusable:
-            if self._plan is None:
-                self._plan = attention_plan(self.segments, self._shape[2], self._device)
-                # once, so that later forwards may run on any stream without ordering themselves after the plan kernel
-                torch.cuda.current_stream(self._device).synchronize()
+            self._ensure_plan()
             return attention_launcher(q, k, v, self.rspmm_output, self.segments, self.scale, self._plan)
 
         multi = self.segments  # (also for one segment: the object keeps what every call would otherwise rebuild and recheck)
@@ -225,6 +227,13 @@ class RegularAttention(nn.Module):
                        self.nnzs, self.rspmm_grid_dim, self.BLOCK_SIZE_Y, self.BLOCK_SIZE_X, segments=multi)
         return self.rspmm_output
 
+    def _ensure_plan(self):
+        """The fused kernel's plan of this mask, and the mask as the native host path takes it."""
+        if self._plan is None:
+            self._plan = attention_plan(self.segments, self._shape[2], self._device)
+        if self._native is None:
+            self._native = self.segments.native(self._shape[2], self._device, True)
+
     def forward_with_stats(self, x):
         """``forward(x)`` through the fused kernel plus every row's softmax statistic: returns ``(output, lse)`` with
         ``lse`` float32 [B, H, L] = log of the row's sum of exp(scale * score) over its live columns (+inf for a row
@@ -233,9 +242,7 @@ class RegularAttention(nn.Module):
         q, k, v = x
         if not (q.shape[-1] in (64, 128) and q.dtype == k.dtype == v.dtype == self._out_dtype):
             raise _hip.SplatError("the softmax statistic comes from the fused kernel: d in {64, 128}, one dtype")
-        if self._plan is None:
-            self._plan = attention_plan(self.segments, self._shape[2], self._device)
-            torch.cuda.current_stream(self._device).synchronize()
+        self._ensure_plan()
         if self._lse is None:
             self._lse = torch.empty(self._shape[:3], dtype=torch.float32, device=self._device)
         attention_launcher(q, k, v, self.rspmm_output, self.segments, self.scale, self._plan, self._lse)
@@ -250,11 +257,9 @@ class RegularAttention(nn.Module):
         (a forward is run here when one is missing); otherwise, or with ``fused=False``, from the operators composed over
         compressed matrices, which ``lse`` spares the softmax pass.  ``sparse_rows``: how the fused kernel takes segments
         of the transposed mask that keep few keys with long columns (``r_backward.attention_backward_fused``)."""
-        from r_backward import attention_backward, attention_backward_fused, transposed_segments
+        from r_backward import attention_backward, attention_backward_fused
         q, kT, v = x
-        if self._segments_t is None:
-            masks = self._mask if _is_segment_list(self._mask) else [self._mask]
-            self._segments_t = transposed_segments(masks, self._BLOCK_HEIGHT, self._GPU_ID)
+        self._ensure_transposed()
         fusable = (self.fused and q.shape[-1] in (64, 128) and q.dtype in (torch.float16, torch.bfloat16) and
                    q.dtype == kT.dtype == v.dtype == grad_out.dtype == self._out_dtype)
         if fused is None:
@@ -265,15 +270,44 @@ class RegularAttention(nn.Module):
             return attention_backward(q, kT, v, grad_out, self.segments, self._segments_t, self.scale, lse)
         if lse is None or out is None:
             out, lse = self.forward_with_stats(x)
-        if self._plan is None or self._plan_t is None:
-            if self._plan is None:
-                self._plan = attention_plan(self.segments, self._shape[2], self._device)
-            if self._plan_t is None:
-                self._plan_t = attention_plan(self._segments_t, self._shape[2], self._device)
-            # once, so that later calls may run on any stream without ordering themselves after the plan kernels
-            torch.cuda.current_stream(self._device).synchronize()
+        self._ensure_plan()
+        if self._plan_t is None:
+            self._plan_t = attention_plan(self._segments_t, self._shape[2], self._device)
         return attention_backward_fused(q, kT, v, out, grad_out, lse, self.segments, self._segments_t, self._plan,
                                         self._plan_t, self.scale, sparse_rows)
+
+
+    def _ensure_transposed(self):
+        from r_backward import transposed_segments
+        if self._segments_t is None:
+            masks = self._mask if _is_segment_list(self._mask) else [self._mask]
+            self._segments_t = transposed_segments(masks, self._BLOCK_HEIGHT, self._GPU_ID)
+
+    def _grad_state(self):
+        """What the native differentiable path (csrc/host_ext.cpp) keeps for this module: the mask and the transposed mask
+        with their plans and the row-sparse segments' schedule.  None where it does not apply (float32, other head
+        dimensions, ``fused=False``, a mask without a transposed ACSR, a first call under stream capture)."""
+        if self._native_grad is None:
+            from r_backward import keys_side_schedule
+            B, H, L, d = self._shape
+            if torch.cuda.is_current_stream_capturing():
+                return None
+            self._native_grad = False
+            if d in (64, 128) and self._out_dtype in (torch.float16, torch.bfloat16):
+                try:
+                    self._ensure_transposed()
+                except _hip.SplatError:
+                    return None  # (raised again by the backward that needs it)
+                self._ensure_plan()
+                dev = self._device
+                sched = keys_side_schedule(self._segments_t, L, dev, B * H)
+                keys = sched.main if sched is not None else self._segments_t
+                self._native_grad = _hip.host().grad_state(
+                    self._native, keys.native(L, dev, True),
+                    None if sched is None else sched.rows.native(sched.n_rows, dev, True),
+                    None if sched is None else sched.key_of_row, 0 if sched is None else sched.per_stretch,
+                    B, H, L, d, self.rspmm_output)
+        return self._native_grad if self.fused and self._native_grad is not False else None
 
 
 class _AttentionFunction(torch.autograd.Function):
@@ -281,9 +315,12 @@ class _AttentionFunction(torch.autograd.Function):
     def forward(ctx, q, k, v, attn):
         ctx.attn = attn
         if attn.fused and q.shape[-1] in (64, 128) and q.dtype == k.dtype == v.dtype == attn._out_dtype:
-            out, lse = attn.forward_with_stats([q, k.transpose(2, 3), v])
-            out = out.clone()  # the module's buffers are reused by the next call
-            ctx.save_for_backward(q, k, v, lse.clone(), out)
+            # (tensors of this call's own: the module's buffers are reused by the next one)
+            attn._ensure_plan()
+            out = torch.empty_like(attn.rspmm_output)
+            lse = torch.empty(attn._shape[:3], dtype=torch.float32, device=out.device)
+            attention_launcher(q, k.transpose(2, 3), v, out, attn.segments, attn.scale, attn._plan, lse)
+            ctx.save_for_backward(q, k, v, lse, out)
             return out
         out = attn([q, k.transpose(2, 3), v])
         ctx.save_for_backward(q, k, v)
@@ -300,6 +337,12 @@ class _AttentionFunction(torch.autograd.Function):
 def attention_with_grad(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, attn: RegularAttention) -> torch.Tensor:
     """``attn([q, k^T, v])`` for q, k, v [B, H, L, d] as a differentiable operation (fused forward, backward from
     ``RegularAttention.backward_pass``)."""
+    if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
+        state = attn._grad_state()
+        if state is not None:
+            out = _hip.host().attend(state, q, k, v, attn.scale)
+            if out is not None:
+                return out
     return _AttentionFunction.apply(q, k, v, attn)
 
 

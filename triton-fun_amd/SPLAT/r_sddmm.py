@@ -64,6 +64,9 @@ def _strides4(t: torch.Tensor, name: str):
     return t.stride()
 
 
+_HALF = (torch.float16, torch.bfloat16)
+
+
 def _takes_a_plan(x, output, y, B: int, H: int, L: int, d: int, T: int, segs: ACSRSegments) -> bool:
     """Whether this launch runs the kernel that reads a plan table (the library decides by the same rules and ignores the
     plan otherwise): 16-bit types, d = 64 / 128, rows of K contiguous, 16-byte alignment, and at least 256 row blocks or rows
@@ -99,6 +102,11 @@ def rsddmm_launcher(x: torch.Tensor, y: torch.Tensor, output: torch.Tensor,
         raise _hip.SplatError("x and y must share a dtype")
     segs = segments or ACSRSegments.single(dTos_linear_transformations, dTos_translations,
                                            sTod_linear_transformations, sTod_translations, nnzs, trailing_dim)
+    if plan is None and x.dim() == 4 and output.shape[-1] == trailing_dim:
+        # (the library uses the table where it has a kernel that reads one: 16-bit types at d = 64 / 128)
+        mask = segs.native(x.shape[2], x.device, x.shape[3] in (64, 128) and x.dtype in _HALF)
+        if mask is not None and _hip.host().sddmm(mask, x, y, output, 1.0 if scale is None else scale, lse):
+            return (output, sTod_linear_transformations, sTod_translations, nnzs)
     B, H, L, d = x.shape
     if y.shape[0] != B or y.shape[1] != H or y.shape[2] != d:
         raise _hip.SplatError(f"y must be [B, H, d, n] = [{B}, {H}, {d}, n], got {tuple(y.shape)}")

@@ -49,6 +49,9 @@ def rsoftmax_launcher(x: torch.Tensor, output: torch.Tensor,
                                            sTod_linear_transformations, sTod_translations, nnzs,
                                            acsr_trailing_dim_true)
     B, H, L, T = x.shape
+    mask = segs.native(L, x.device, False)
+    if mask is not None and _hip.host().softmax(mask, x, output):
+        return (output, sTod_linear_transformations, sTod_translations, nnzs)
     dev = x.device
     arr = segs.seg_array(L, T)
     with torch.cuda.device(dev):

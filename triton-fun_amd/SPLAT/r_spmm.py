@@ -15,6 +15,9 @@ from acsr_helpers import ACSRSegments, build_acsr, create_acsr, create_blocked_m
 from r_sddmm import live_slot_columns
 
 
+_HALF = (torch.float16, torch.bfloat16)
+
+
 def rspmm_preamble(mask, output_shape: tuple[int], BLOCK_SIZE_X: int, BLOCK_SIZE_Y: int, GPU_ID: Any,
                    output_dtype: torch.dtype) -> tuple[torch.Tensor, tuple[int], int]:
     """-> (output [B, H, L, n] uninitialised, grid_dim = (ceil(n / BSX), ceil(L / BSY), B*H), T = max row nnz)."""
@@ -60,6 +63,13 @@ def rspmm_launcher(x: torch.Tensor, y: torch.Tensor, output: torch.Tensor,
                                            sTod_linear_transformations, sTod_translations, nnzs, acsr_trailing_dim)
     vs = y.stride()
     dev = x.device
+    if plan is None:
+        capturing = torch.cuda.is_current_stream_capturing()
+        tabled = x.dtype in _HALF and output.dtype == x.dtype and n_out in (64, 128) \
+            and not (T >= 256 and (segs.has_plan(L, dev) or not capturing) and segs.plan_is_aligned(L, dev))
+        mask = segs.native(L, dev, tabled)
+        if mask is not None and _hip.host().spmm(mask, x, y, output):
+            return (output, sTod_linear_transformations, sTod_translations, nnzs)
     arr = segs.seg_array(L, T)
     if plan is None and x.dtype in (torch.float16, torch.bfloat16) and output.dtype == x.dtype and n_out in (64, 128) \
             and (segs.has_plan(L, dev) or not torch.cuda.is_current_stream_capturing()) \

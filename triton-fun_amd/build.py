@@ -1,5 +1,5 @@
 """Build libsplat_hip.so (the operators) and libsplat_bench.so (bench.py's measurement aids) for gfx950 from csrc/ with
-hipcc.  Usage: python build.py [-j N]"""
+hipcc, and _splat_host.so (the native host path, a Python extension over PyTorch's C++ interface) with g++.  Usage: python build.py [-j N]"""
 from __future__ import annotations
 
 import argparse
@@ -14,6 +14,7 @@ OBJ = os.path.join(HERE, "build")
 LIB_DIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIB_DIR, "libsplat_hip.so")
 BENCH_LIB = os.path.join(LIB_DIR, "libsplat_bench.so")
+HOST_EXT = os.path.join(LIB_DIR, "_splat_host.so")
 
 SOURCES = ["api_common.cpp", "acsr_build.hip", "softmax.hip", "sddmm.hip", "sddmm_lines.hip", "spmm.hip", "spmm_thin.hip", "spmm_tile.hip", "spmm_t_thin.hip", "attention.hip", "backward.hip", "attention_bwd.hip", "transpose.hip"]
 # the measurement aids: a library of their own, so that the operator ABI holds operators only
@@ -55,17 +56,34 @@ def _link(lib: str, objs: list[str]) -> None:
         raise RuntimeError(f"{lib} has undefined symbols of its own: {missing[:4]}")
 
 
+def _host_ext() -> None:
+    """The Python extension of the host path: host code only, so the host compiler builds it."""
+    import sysconfig
+
+    from torch.utils.cpp_extension import ROCM_HOME, include_paths, library_paths
+    rocm = ROCM_HOME or "/opt/rocm"
+    inc = [*include_paths(), os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]
+    cmd = ["g++", "-O2", "-fPIC", "-shared", "-std=c++17", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           *(f"-I{p}" for p in inc), os.path.join(CSRC, "host_ext.cpp"), "-o", HOST_EXT,
+           *(f"-L{p}" for p in library_paths()), "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed on host_ext.cpp:\n{r.stderr}")
+
+
 def build(jobs: int = 8, verbose: bool = True) -> str:
-    """Compile every source and link both shared libraries; always recompiles."""
+    """Compile every source and link the shared libraries; always recompiles."""
     os.makedirs(OBJ, exist_ok=True)
     os.makedirs(LIB_DIR, exist_ok=True)
     names = SOURCES + [s for s in BENCH_SOURCES if s not in SOURCES]
     with ThreadPoolExecutor(max_workers=max(1, min(jobs, 16))) as ex:
+        host = ex.submit(_host_ext)
         objs = dict(zip(names, ex.map(_compile, names)))
+        host.result()
     _link(LIB, [objs[s] for s in SOURCES])
     _link(BENCH_LIB, [objs[s] for s in BENCH_SOURCES])
     if verbose:
-        print(f"built {LIB} and {BENCH_LIB}")
+        print(f"built {LIB}, {BENCH_LIB} and {HOST_EXT}")
     return LIB
 
 

@@ -1,0 +1,459 @@
+// The host path of the operators that a program calls in a loop, in native code: argument checks, strides, allocations and the
+// C-ABI call of one operator, and the differentiable attention as a C++ autograd function.
+//
+// Bound: the host.  A call of the fused forward through ctypes costs the interpreter 14 us, of which the launch itself is 3;
+// sizes whose kernels take less than that (a few hundred row blocks) run at the interpreter's speed, and a training step, whose
+// backward an autograd thread runs under the interpreter's lock, at 90 us.  Here a call reads the tensors' fields directly.
+//
+// Every entry point handles the ordinary case (tensors on the current device, rows in whole 16-byte pieces) and returns False
+// (attend: None) for anything else, before it has done anything: the Python launchers then take the call, with their copies and
+// their messages.  The kernels are reached through the addresses that `bind` receives, so that both layers use one library.
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/custom_class.h>
+
+#include <cstring>
+#include <vector>
+
+#include "../../include/splat_hip.h"
+
+namespace {
+
+// ---- the library's entry points -------------------------------------------------------------------------------------
+struct Api {
+    decltype(&splat_last_error) last_error;
+    decltype(&splat_attention_fwd_planned) fwd_planned;
+    decltype(&splat_attention_fwd_stats) fwd_stats;
+    decltype(&splat_transpose_keys) transpose_keys;
+    decltype(&splat_attention_bwd) bwd;
+    decltype(&splat_attention_bwd_keys) bwd_keys;
+    decltype(&splat_sddmm) sddmm;
+    decltype(&splat_sddmm_probs) sddmm_probs;
+    decltype(&splat_sddmm_planned) sddmm_planned;
+    decltype(&splat_softmax) softmax;
+    decltype(&splat_spmm) spmm;
+    decltype(&splat_spmm_planned) spmm_planned;
+} api;
+PyObject* g_error = nullptr;  // SplatError
+
+int dtype_code(at::ScalarType t) {
+    switch (t) {
+        case at::kFloat: return SPLAT_F32;
+        case at::kHalf: return SPLAT_F16;
+        case at::kBFloat16: return SPLAT_BF16;
+        default: return -1;
+    }
+}
+
+bool aligned16(const at::Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; }
+
+// rows of the last dimension contiguous, in whole 16-byte pieces
+bool rows_in_pieces(const at::Tensor& t, int64_t epc) {
+    return t.stride(3) == 1 && t.stride(0) % epc == 0 && t.stride(1) % epc == 0 && t.stride(2) % epc == 0 && aligned16(t);
+}
+
+bool is_shape(const at::Tensor& t, int64_t a, int64_t b, int64_t c, int64_t d) {
+    return t.size(0) == a && t.size(1) == b && t.size(2) == c && t.size(3) == d;
+}
+
+void* stream_of(const at::Tensor& t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
+
+std::string failure(const char* what, int rc) {
+    return std::string(what) + " failed (code " + std::to_string(rc) + "): " + api.last_error();
+}
+
+// ---- a mask: its segments as the C ABI takes them, the plan table, and the tensors that own the memory -----------------
+struct Mask : torch::CustomClassHolder {
+    splat_acsr_seg segs[SPLAT_MAX_SEGMENTS];
+    int n_seg = 0;
+    int64_t rows = 0;
+    int max_step = 1;
+    at::Tensor plan;               // may be undefined
+    std::vector<at::Tensor> keep;  // the arrays that `segs` points into
+    int device = 0;
+    const void* plan_ptr() const { return plan.data_ptr(); }
+    int64_t plan_bytes() const { return plan.nbytes(); }
+};
+
+// What the differentiable attention needs besides q, k and v.
+struct GradState : torch::CustomClassHolder {
+    c10::intrusive_ptr<Mask> fwd;   // the mask, with its plan
+    c10::intrusive_ptr<Mask> keys;  // the transposed mask's segments that are walked by blocks of keys, with their plan
+    c10::intrusive_ptr<Mask> rows;  // its row-sparse segments, listed row by row (may be null)
+    at::Tensor key_of_row;
+    int64_t per_stretch = 0;
+    int64_t B = 0, H = 0, L = 0, d = 0;
+    at::ScalarType dtype = at::kFloat;
+};
+
+const char* const kMaskName = "splat.mask";
+const char* const kGradName = "splat.grad";
+
+template <typename H>
+void drop(PyObject* cap) {
+    auto* p = static_cast<H*>(PyCapsule_GetPointer(cap, PyCapsule_GetName(cap)));
+    if (p) c10::raw::intrusive_ptr::decref(p);
+}
+template <typename H>
+PyObject* capsule(c10::intrusive_ptr<H> h, const char* name) {
+    return PyCapsule_New(h.release(), name, drop<H>);
+}
+template <typename H>
+c10::intrusive_ptr<H> held(PyObject* cap, const char* name) {
+    auto* p = static_cast<H*>(PyCapsule_GetPointer(cap, name));
+    return p ? c10::intrusive_ptr<H>::reclaim_copy(p) : c10::intrusive_ptr<H>();
+}
+Mask* mask_of(PyObject* cap) { return static_cast<Mask*>(PyCapsule_GetPointer(cap, kMaskName)); }
+
+// A 4-dimensional device tensor on the current device, or null.
+const at::Tensor* tensor4(PyObject* o, int device) {
+    if (!THPVariable_Check(o)) return nullptr;
+    const at::Tensor& t = THPVariable_Unpack(o);
+    if (!t.is_cuda() || t.dim() != 4 || t.layout() != at::kStrided || t.get_device() != device) return nullptr;
+    return &t;
+}
+
+PyObject* raise_rc(const char* what, int rc) {
+    PyErr_SetString(g_error, failure(what, rc).c_str());
+    return nullptr;
+}
+PyObject* raise_std(const std::exception& e) {
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
+    return nullptr;
+}
+
+// K [B, H, L, d] with rows contiguous from K^T [B, H, d, L] with the keys contiguous: one streaming kernel.
+at::Tensor transposed_keys(const at::Tensor& kT, int* rc) {
+    at::Tensor k = at::empty({kT.size(0), kT.size(1), kT.size(3), kT.size(2)}, kT.options());
+    *rc = api.transpose_keys(kT.data_ptr(), kT.stride(0), kT.stride(1), kT.stride(2), k.data_ptr(), kT.size(0), kT.size(1),
+                             kT.size(3), kT.size(2), dtype_code(kT.scalar_type()), stream_of(kT));
+    return k;
+}
+
+// mask(arr_address, n_seg, rows, plan | None, max_step, (tensors...)) -> capsule
+PyObject* py_mask(PyObject*, PyObject* args) {
+    unsigned long long addr;
+    int n_seg, max_step;
+    long long rows;
+    PyObject *plan, *tensors;
+    if (!PyArg_ParseTuple(args, "KiLOiO!", &addr, &n_seg, &rows, &plan, &max_step, &PyTuple_Type, &tensors)) return nullptr;
+    if (n_seg < 1 || n_seg > SPLAT_MAX_SEGMENTS) {
+        PyErr_SetString(PyExc_ValueError, "number of segments");
+        return nullptr;
+    }
+    auto m = c10::make_intrusive<Mask>();
+    std::memcpy(m->segs, reinterpret_cast<const void*>(static_cast<uintptr_t>(addr)), n_seg * sizeof(splat_acsr_seg));
+    m->n_seg = n_seg, m->rows = rows, m->max_step = max_step;
+    for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(tensors); ++i) {
+        PyObject* o = PyTuple_GET_ITEM(tensors, i);
+        if (!THPVariable_Check(o)) continue;
+        m->keep.push_back(THPVariable_Unpack(o));
+        m->device = m->keep.back().get_device();
+    }
+    if (plan != Py_None && THPVariable_Check(plan)) m->plan = THPVariable_Unpack(plan);
+    return capsule(std::move(m), kMaskName);
+}
+
+// ---- fused forward -------------------------------------------------------------------------------------------------------
+// 1: launched, 0: not an ordinary case, < 0 or > 1 after `rc` was set: failed
+enum class Did { kNo, kYes, kFailed };
+
+Did forward(const Mask& m, const at::Tensor& q, at::Tensor kT, const at::Tensor& v, const at::Tensor& out, double scale, float* lse,
+            int* rc) {
+    const auto dt = q.scalar_type();
+    const int code = dtype_code(dt);
+    if (code < 0 || kT.scalar_type() != dt || v.scalar_type() != dt || out.scalar_type() != dt || !m.plan.defined()) return Did::kNo;
+    const int64_t B = q.size(0), H = q.size(1), L = q.size(2), d = q.size(3);
+    if ((d != 64 && d != 128) || L != m.rows || L <= 0 || !is_shape(kT, B, H, d, L) || !is_shape(v, B, H, L, d) || !is_shape(out, B, H, L, d))
+        return Did::kNo;
+    const int64_t epc = 16 / q.element_size();
+    if (!rows_in_pieces(q, epc) || !rows_in_pieces(v, epc) || !rows_in_pieces(out, epc)) return Did::kNo;
+    const bool k_rows = kT.stride(2) == 1 && kT.stride(3) >= d && kT.stride(0) % epc == 0 && kT.stride(1) % epc == 0 &&
+                        kT.stride(3) % epc == 0 && aligned16(kT);
+    if (!k_rows) {
+        if (kT.stride(3) != 1 || kT.stride(2) < L) return Did::kNo;
+        // keys contiguous: taken as they are where every row of keys is whole 16-byte pieces and no row of the mask steps over
+        // columns (dense runs are all this layout can be read in), else turned around first
+        const bool as_is = m.max_step < 2 && L % epc == 0 && kT.stride(0) % epc == 0 && kT.stride(1) % epc == 0 &&
+                           kT.stride(2) % epc == 0 && aligned16(kT);
+        if (!as_is) {
+            kT = transposed_keys(kT, rc).transpose(2, 3);
+            if (*rc) return Did::kFailed;
+        }
+    }
+    void* st = stream_of(q);
+    if (lse)
+        *rc = api.fwd_stats(q.data_ptr(), q.stride(0), q.stride(1), q.stride(2), kT.data_ptr(), kT.stride(0), kT.stride(1), kT.stride(2),
+                            kT.stride(3), v.data_ptr(), v.stride(0), v.stride(1), v.stride(2), out.data_ptr(), out.stride(0),
+                            out.stride(1), out.stride(2), m.segs, m.n_seg, B, H, L, d, (float)scale, code, m.plan_ptr(),
+                            m.plan_bytes(), lse, st);
+    else
+        *rc = api.fwd_planned(q.data_ptr(), q.stride(0), q.stride(1), q.stride(2), kT.data_ptr(), kT.stride(0), kT.stride(1),
+                              kT.stride(2), kT.stride(3), v.data_ptr(), v.stride(0), v.stride(1), v.stride(2), out.data_ptr(),
+                              out.stride(0), out.stride(1), out.stride(2), m.segs, m.n_seg, B, H, L, d, (float)scale, code,
+                              m.plan_ptr(), m.plan_bytes(), st);
+    return *rc ? Did::kFailed : Did::kYes;
+}
+
+// forward(mask, q, kT, v, out, scale) -> bool
+PyObject* py_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 6) return PyErr_Format(PyExc_TypeError, "forward takes 6 arguments");
+    Mask* m = mask_of(a[0]);
+    if (!m) return nullptr;
+    try {
+        const int dev = c10::hip::current_device();
+        const at::Tensor *q = tensor4(a[1], dev), *kT = tensor4(a[2], dev), *v = tensor4(a[3], dev), *out = tensor4(a[4], dev);
+        if (!q || !kT || !v || !out || m->device != dev) Py_RETURN_FALSE;
+        const double scale = PyFloat_AsDouble(a[5]);
+        if (scale == -1.0 && PyErr_Occurred()) return nullptr;
+        int rc = 0;
+        const Did did = forward(*m, *q, *kT, *v, *out, scale, nullptr, &rc);
+        if (did == Did::kFailed) return raise_rc("splat_attention_fwd_planned", rc);
+        return PyBool_FromLong(did == Did::kYes);
+    } catch (const std::exception& e) {
+        return raise_std(e);
+    }
+}
+
+// ---- differentiable attention ----------------------------------------------------------------------------------------------
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+at::Tensor in_pieces(const at::Tensor& t) { return rows_in_pieces(t, 16 / t.element_size()) ? t : t.contiguous(); }
+
+struct Attend : public torch::autograd::Function<Attend> {
+    static at::Tensor forward(AutogradContext* ctx, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
+                              const c10::intrusive_ptr<GradState>& st, double scale) {
+        at::Tensor out = at::empty({st->B, st->H, st->L, st->d}, q.options());
+        at::Tensor lse = at::empty({st->B, st->H, st->L}, q.options().dtype(at::kFloat));
+        int rc = 0;
+        const Did did = ::forward(*st->fwd, q, k.transpose(2, 3), v, out, scale, lse.data_ptr<float>(), &rc);
+        TORCH_CHECK(did == Did::kYes, rc ? failure("splat_attention_fwd_stats", rc) : std::string("attention: unusual operands"));
+        ctx->save_for_backward({q, k, v, lse, out});
+        ctx->saved_data["state"] = c10::IValue::make_capsule(st);
+        ctx->saved_data["scale"] = scale;
+        return out;
+    }
+
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const variable_list s = ctx->get_saved_variables();
+        const at::Tensor &q = s[0], &k = s[1], &v = s[2], &lse = s[3], &out = s[4];
+        auto held = ctx->saved_data["state"].toCapsule();
+        const GradState& st = *static_cast<GradState*>(held.get());
+        const float scale = (float)ctx->saved_data["scale"].toDouble();
+        const at::Tensor g = in_pieces(grads[0].scalar_type() == st.dtype ? grads[0] : grads[0].to(st.dtype));
+        const int64_t B = st.B, H = st.H, L = st.L, d = st.d;
+        const int code = dtype_code(st.dtype);
+        const auto contiguous = q.options().memory_format(c10::nullopt);
+        at::Tensor dq = at::empty({B, H, L, d}, contiguous), dk = at::empty({B, H, L, d}, contiguous), dv = at::empty({B, H, L, d}, contiguous);
+        at::Tensor delta = at::empty({B, H, L}, lse.options());
+        void* stream = stream_of(q);
+        const Mask &m = *st.fwd, &mt = *st.keys;
+        int rc = api.bwd(q.data_ptr(), q.stride(0), q.stride(1), q.stride(2), k.data_ptr(), k.stride(0), k.stride(1), k.stride(2), v.data_ptr(),
+                         v.stride(0), v.stride(1), v.stride(2), out.data_ptr(), out.stride(0), out.stride(1), out.stride(2), g.data_ptr(),
+                         g.stride(0), g.stride(1), g.stride(2), lse.data_ptr<float>(), delta.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(),
+                         dv.data_ptr(), m.segs, m.n_seg, m.plan_ptr(), m.plan_bytes(), mt.segs, mt.n_seg, mt.plan_ptr(), mt.plan_bytes(), B, H,
+                         L, d, scale, code, stream);
+        TORCH_CHECK(rc == 0, failure("splat_attention_bwd", rc));
+        if (st.rows) {  // the row-sparse segments of the transposed mask, row by row, onto what the others gave
+            const Mask& r = *st.rows;
+            at::Tensor part = at::empty({2, B, H, r.rows, d}, contiguous);
+            char* half = static_cast<char*>(part.data_ptr()) + part.nbytes() / 2;
+            rc = api.bwd_keys(q.data_ptr(), q.stride(0), q.stride(1), q.stride(2), k.data_ptr(), k.stride(0), k.stride(1), k.stride(2),
+                              v.data_ptr(), v.stride(0), v.stride(1), v.stride(2), g.data_ptr(), g.stride(0), g.stride(1), g.stride(2),
+                              lse.data_ptr<float>(), delta.data_ptr<float>(), st.key_of_row.data_ptr<int32_t>(), part.data_ptr(), half, r.segs,
+                              r.n_seg, r.plan_ptr(), r.plan_bytes(), B, H, L, r.rows, d, scale, code, dk.data_ptr(), dv.data_ptr(),
+                              st.per_stretch, stream);
+            TORCH_CHECK(rc == 0, failure("splat_attention_bwd_keys", rc));
+        }
+        return {dq, dk, dv, at::Tensor(), at::Tensor()};
+    }
+};
+
+// grad_state(mask, keys_mask, rows_mask | None, key_of_row | None, per_stretch, B, H, L, d, like) -> capsule; `like` a tensor of the type
+PyObject* py_grad_state(PyObject*, PyObject* args) {
+    PyObject *m, *mt, *mr, *key, *like;
+    long long per, B, H, L, d;
+    if (!PyArg_ParseTuple(args, "OOOOLLLLLO", &m, &mt, &mr, &key, &per, &B, &H, &L, &d, &like)) return nullptr;
+    auto st = c10::make_intrusive<GradState>();
+    st->fwd = held<Mask>(m, kMaskName);
+    st->keys = held<Mask>(mt, kMaskName);
+    if (!st->fwd || !st->keys) return nullptr;
+    if (mr != Py_None) {
+        st->rows = held<Mask>(mr, kMaskName);
+        if (!st->rows) return nullptr;
+        st->key_of_row = THPVariable_Unpack(key);
+    }
+    st->per_stretch = per, st->B = B, st->H = H, st->L = L, st->d = d;
+    st->dtype = THPVariable_Unpack(like).scalar_type();
+    return capsule(std::move(st), kGradName);
+}
+
+// attend(state, q, k, v, scale) -> output, or None when the case is not an ordinary one
+PyObject* py_attend(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 5) return PyErr_Format(PyExc_TypeError, "attend takes 5 arguments");
+    try {
+        auto st = held<GradState>(a[0], kGradName);
+        if (!st) return nullptr;
+        const int dev = c10::hip::current_device();
+        const at::Tensor *q = tensor4(a[1], dev), *k = tensor4(a[2], dev), *v = tensor4(a[3], dev);
+        if (!q || !k || !v || st->fwd->device != dev) Py_RETURN_NONE;
+        const int64_t epc = 16 / q->element_size();
+        for (const at::Tensor* t : {q, k, v})
+            if (t->scalar_type() != st->dtype || !is_shape(*t, st->B, st->H, st->L, st->d) || !rows_in_pieces(*t, epc) || t->stride(2) < st->d)
+                Py_RETURN_NONE;
+        const double scale = PyFloat_AsDouble(a[4]);
+        if (scale == -1.0 && PyErr_Occurred()) return nullptr;
+        return THPVariable_Wrap(Attend::apply(*q, *k, *v, st, scale));
+    } catch (const std::exception& e) {
+        return raise_std(e);
+    }
+}
+
+// ---- the three operators ------------------------------------------------------------------------------------------------------
+// sddmm(mask, x, y, output, scale, lse | None) -> bool; a plan in the mask is handed on
+PyObject* py_sddmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 6) return PyErr_Format(PyExc_TypeError, "sddmm takes 6 arguments");
+    Mask* m = mask_of(a[0]);
+    if (!m) return nullptr;
+    try {
+        const int dev = c10::hip::current_device();
+        const at::Tensor *x = tensor4(a[1], dev), *y0 = tensor4(a[2], dev), *out = tensor4(a[3], dev);
+        if (!x || !y0 || !out || m->device != dev) Py_RETURN_FALSE;
+        at::Tensor y = *y0;
+        const int code = dtype_code(x->scalar_type()), out_code = dtype_code(out->scalar_type());
+        const int64_t B = x->size(0), H = x->size(1), L = x->size(2), d = x->size(3), keys = y.size(3), T = out->size(3);
+        if (code < 0 || out_code < 0 || y.scalar_type() != x->scalar_type() || L != m->rows || x->stride(3) != 1 || B * H * L * d * T == 0 ||
+            !is_shape(y, B, H, d, keys) || !is_shape(*out, B, H, L, T) || !out->is_contiguous() || (y.stride(2) != 1 && y.stride(3) != 1))
+            Py_RETURN_FALSE;
+        float* lse = nullptr;
+        if (a[5] != Py_None) {
+            if (!THPVariable_Check(a[5])) Py_RETURN_FALSE;
+            const at::Tensor& t = THPVariable_Unpack(a[5]);
+            if (!t.is_cuda() || t.get_device() != dev || t.scalar_type() != at::kFloat || !t.is_contiguous() || t.dim() != 3 ||
+                t.size(0) != B || t.size(1) != H || t.size(2) != L)
+                Py_RETURN_FALSE;
+            lse = t.data_ptr<float>();
+        }
+        const double scale = PyFloat_AsDouble(a[4]);
+        if (scale == -1.0 && PyErr_Occurred()) return nullptr;
+        int rc = 0;
+        if (m->max_step >= 2 && y.stride(3) == 1 && y.stride(2) != 1) {
+            if (y.stride(2) < keys) Py_RETURN_FALSE;
+            y = transposed_keys(y, &rc).transpose(2, 3);
+            if (rc) return raise_rc("splat_transpose_keys", rc);
+        }
+        void* st = stream_of(*x);
+#define SPLAT_ARGS                                                                                                                     \
+    x->data_ptr(), x->stride(0), x->stride(1), x->stride(2), y.data_ptr(), y.stride(0), y.stride(1), y.stride(2), y.stride(3),        \
+        out->data_ptr(), m->segs, m->n_seg, B, H, L, keys, d, T, (float)scale, code, out_code
+        if (m->plan.defined())
+            rc = api.sddmm_planned(SPLAT_ARGS, lse, m->plan_ptr(), m->plan_bytes(), st);
+        else if (lse)
+            rc = api.sddmm_probs(SPLAT_ARGS, lse, st);
+        else
+            rc = api.sddmm(SPLAT_ARGS, st);
+#undef SPLAT_ARGS
+        if (rc) return raise_rc("splat_sddmm", rc);
+        Py_RETURN_TRUE;
+    } catch (const std::exception& e) {
+        return raise_std(e);
+    }
+}
+
+// softmax(mask, x, output) -> bool
+PyObject* py_softmax(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 3) return PyErr_Format(PyExc_TypeError, "softmax takes 3 arguments");
+    Mask* m = mask_of(a[0]);
+    if (!m) return nullptr;
+    try {
+        const int dev = c10::hip::current_device();
+        const at::Tensor *x = tensor4(a[1], dev), *out = tensor4(a[2], dev);
+        if (!x || !out || m->device != dev || x->sizes() != out->sizes() || !x->is_contiguous() || !out->is_contiguous() ||
+            x->size(2) != m->rows || x->numel() == 0)
+            Py_RETURN_FALSE;
+        const int code = dtype_code(x->scalar_type()), out_code = dtype_code(out->scalar_type());
+        if (code < 0 || out_code < 0) Py_RETURN_FALSE;
+        const int rc = api.softmax(x->data_ptr(), out->data_ptr(), m->segs, m->n_seg, x->size(0) * x->size(1), x->size(2), x->size(3),
+                                   code, out_code, stream_of(*x));
+        if (rc) return raise_rc("splat_softmax", rc);
+        Py_RETURN_TRUE;
+    } catch (const std::exception& e) {
+        return raise_std(e);
+    }
+}
+
+// spmm(mask, x, y, output) -> bool; a plan in the mask is handed on
+PyObject* py_spmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 4) return PyErr_Format(PyExc_TypeError, "spmm takes 4 arguments");
+    Mask* m = mask_of(a[0]);
+    if (!m) return nullptr;
+    try {
+        const int dev = c10::hip::current_device();
+        const at::Tensor *x = tensor4(a[1], dev), *y = tensor4(a[2], dev), *out = tensor4(a[3], dev);
+        if (!x || !y || !out || m->device != dev) Py_RETURN_FALSE;
+        const int code = dtype_code(x->scalar_type()), out_code = dtype_code(out->scalar_type());
+        const int64_t B = x->size(0), H = x->size(1), L = x->size(2), T = x->size(3), keys = y->size(2), w = y->size(3);
+        if (code < 0 || out_code < 0 || y->scalar_type() != x->scalar_type() || L != m->rows || x->numel() == 0 || y->numel() == 0 ||
+            y->size(0) != B || y->size(1) != H || !is_shape(*out, B, H, L, w) || !x->is_contiguous() || !out->is_contiguous() ||
+            y->stride(3) != 1)
+            Py_RETURN_FALSE;
+        void* st = stream_of(*x);
+        int rc;
+        if (m->plan.defined())
+            rc = api.spmm_planned(x->data_ptr(), y->data_ptr(), y->stride(0), y->stride(1), y->stride(2), out->data_ptr(), m->segs, m->n_seg,
+                                  B, H, L, keys, w, T, code, out_code, m->plan_ptr(), m->plan_bytes(), st);
+        else
+            rc = api.spmm(x->data_ptr(), y->data_ptr(), y->stride(0), y->stride(1), y->stride(2), out->data_ptr(), m->segs, m->n_seg, B, H,
+                          L, keys, w, T, code, out_code, st);
+        if (rc) return raise_rc("splat_spmm", rc);
+        Py_RETURN_TRUE;
+    } catch (const std::exception& e) {
+        return raise_std(e);
+    }
+}
+
+// bind({entry point: address}, SplatError)
+PyObject* py_bind(PyObject*, PyObject* args) {
+    PyObject *table, *err;
+    if (!PyArg_ParseTuple(args, "O!O", &PyDict_Type, &table, &err)) return nullptr;
+    auto take = [&](const char* name, auto& fn) {
+        PyObject* o = PyDict_GetItemString(table, name);
+        if (!o) {
+            PyErr_Format(PyExc_KeyError, "%s", name);
+            return false;
+        }
+        fn = reinterpret_cast<std::remove_reference_t<decltype(fn)>>(static_cast<uintptr_t>(PyLong_AsUnsignedLongLong(o)));
+        return !PyErr_Occurred();
+    };
+    if (!take("splat_last_error", api.last_error) || !take("splat_attention_fwd_planned", api.fwd_planned) ||
+        !take("splat_attention_fwd_stats", api.fwd_stats) || !take("splat_transpose_keys", api.transpose_keys) ||
+        !take("splat_attention_bwd", api.bwd) || !take("splat_attention_bwd_keys", api.bwd_keys) || !take("splat_sddmm", api.sddmm) ||
+        !take("splat_sddmm_probs", api.sddmm_probs) || !take("splat_sddmm_planned", api.sddmm_planned) ||
+        !take("splat_softmax", api.softmax) || !take("splat_spmm", api.spmm) || !take("splat_spmm_planned", api.spmm_planned))
+        return nullptr;
+    Py_INCREF(err);
+    Py_XSETREF(g_error, err);
+    Py_RETURN_NONE;
+}
+
+PyMethodDef methods[] = {
+    {"bind", py_bind, METH_VARARGS, "bind({entry point: address}, error class)"},
+    {"mask", py_mask, METH_VARARGS, "the segments of a mask, with its plan"},
+    {"forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_forward)), METH_FASTCALL, "fused forward"},
+    {"grad_state", py_grad_state, METH_VARARGS, "what the differentiable attention keeps"},
+    {"attend", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_attend)), METH_FASTCALL, "differentiable attention"},
+    {"sddmm", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_sddmm)), METH_FASTCALL, "sampled product"},
+    {"softmax", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_softmax)), METH_FASTCALL, "softmax of compressed rows"},
+    {"spmm", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_spmm)), METH_FASTCALL, "compressed rows times dense"},
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_splat_host", nullptr, -1, methods};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__splat_host(void) { return PyModule_Create(&module); }
