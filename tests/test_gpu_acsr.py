@@ -227,3 +227,20 @@ def test_a_trailing_dimension_given_by_the_caller_spares_the_read_back(dev):
     with pytest.raises(hip.SplatError, match="longest row has 100"):
         A.create_acsr(pat, 16, dev, T=p)
     A._MASK_CACHE.clear()
+
+
+@pytest.mark.parametrize("rows,cols,pitch,offset,BH", [(1, 1, 1, 0, 16), (17, 15, 15, 1, 4), (33, 31, 37, 3, 16), (100, 1041, 1048, 5, 16),
+                                                       (64, 8192, 8192, 0, 64), (40, 8209, 8211, 15, 16), (16384, 64, 64, 0, 16)])
+def test_mask_tensors_of_any_pitch_in_one_kernel(dev, rows, cols, pitch, offset, BH):
+    """Mask tensors go through the build that is waited for (one kernel): rows of any pitch and alignment, the same result on
+    the second call (from the kept duplicate), and tensors of the caller's own."""
+    g = torch.Generator().manual_seed(rows + cols)
+    flat = torch.zeros(offset + rows * pitch, dtype=torch.uint8, device=dev)
+    mask = flat[offset:].view(rows, pitch)[:, :cols]
+    mask.copy_(torch.rand(rows, cols, generator=g) < 0.3)
+    if cols > 1000:
+        mask[: rows // 2, : cols - 20] = 0  # first columns in the last pieces
+    got = check_acsr(mask, BH, dev)
+    assert np.array_equal(A.row_extents(mask, dev)[1].cpu().numpy(), O.row_extents(mask.cpu().numpy())[1])
+    got[0].fill_(7.0)
+    check_acsr(mask, BH, dev)

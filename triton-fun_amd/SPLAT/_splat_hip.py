@@ -39,12 +39,14 @@ class AcsrSeg(ctypes.Structure):
 
 _lib = None
 _host = None
+_available = False
 
 _i32, _i64, _f32, _vp = ctypes.c_int32, ctypes.c_int64, ctypes.c_float, ctypes.c_void_p
 _SIGNATURES = {
     "splat_version": (ctypes.c_int, []),
     "splat_last_error": (ctypes.c_char_p, []),
     "splat_acsr_build": (ctypes.c_int, [_vp, _i64, _i64, _i64, _i32] + [_vp] * 10 + [_vp]),
+    "splat_acsr_build_record": (ctypes.c_int, [_vp, _i64, _i64, _i64, _i32, _vp, _i64, _vp, _vp]),
     "splat_mask_generate": (ctypes.c_int, [_vp, _i64, _i64, _i64, _i32, _i64, _i64, _vp]),
     "splat_acsr_build_pattern": (ctypes.c_int, [_i32, _i64, _i64, _i64, _i32] + [_vp] * 10 + [_vp]),
     "splat_sddmm": (ctypes.c_int, [_vp, _i64, _i64, _i64, _vp, _i64, _i64, _i64, _i64, _vp, ctypes.POINTER(AcsrSeg), _i32,
@@ -139,8 +141,11 @@ def resolve_device(GPU_ID: Any) -> torch.device:
     dev = torch.device("cuda", GPU_ID) if isinstance(GPU_ID, int) else torch.device(GPU_ID)
     if dev.type != "cuda":
         raise SplatError(f"GPU_ID={GPU_ID!r}: this implementation runs on a HIP device only (no CPU path)")
-    if not torch.cuda.is_available():
-        raise SplatError("no HIP device is available")
+    global _available
+    if not _available:  # (asking costs a driver call: once a device has been seen it is not asked again)
+        if not torch.cuda.is_available():
+            raise SplatError("no HIP device is available")
+        _available = True
     if dev.index is None:
         dev = torch.device("cuda", torch.cuda.current_device())
     return dev

@@ -190,7 +190,7 @@ def _cache_key(mask, host_bytes: np.ndarray | None = None) -> tuple:
     digest of their bytes, taken from the uint8 copy that the upload needs anyway."""
     if isinstance(mask, torch.Tensor):
         return ("t", mask.data_ptr(), mask._version, tuple(mask.shape), tuple(mask.stride()), mask.storage_offset(),
-                str(mask.dtype), str(mask.device))
+                mask.dtype, mask.device)
     if isinstance(mask, MaskPattern):
         return ("p", mask)
     b = _host_mask_bytes(mask) if host_bytes is None else host_bytes
@@ -202,7 +202,7 @@ def _mask_entry(mask, dev: torch.device) -> tuple[_MaskEntry, np.ndarray | None]
     reference, and share one build) and, for host masks, their uint8 bytes.  Only the small per-row results are kept:
     no rows x cols copy of the mask outlives a build."""
     host = None if isinstance(mask, (torch.Tensor, MaskPattern)) else _host_mask_bytes(mask)
-    key = (_cache_key(mask, host), str(dev))
+    key = (_cache_key(mask, host), dev)
     _MASK_CACHE[:] = [e for e in _MASK_CACHE if e.alive()]
     for e in _MASK_CACHE:
         if e.key == key:
@@ -221,7 +221,7 @@ def _device_mask(mask, host: np.ndarray | None, dev: torch.device) -> torch.Tens
     if isinstance(mask, MaskPattern):
         return None
     if isinstance(mask, torch.Tensor):
-        dm = mask.to(device=dev, dtype=torch.uint8)
+        dm = mask if mask.dtype == torch.uint8 and mask.device == dev else mask.to(device=dev, dtype=torch.uint8)
         return dm if dm.stride(1) == 1 else dm.contiguous()
     return torch.from_numpy(host).to(dev)
 
@@ -262,14 +262,7 @@ class AcsrBuild:
     def resolve(self) -> None:
         if self.summary is None:
             return
-        found = self.summary.cpu()  # the one synchronisation: T is returned as a Python int, like the reference
-        self.summary = None
-        assert int(found[1]) == 0, "Incorrect unpacking of affine-indices."
-        self._T = int(found[0])
-        # rows whose columns step by n and start in phase with the row index (dilated windows): kernels group them by phase
-        self._row_stride = int(found[2]) if (int(found[2]) == int(found[3]) and int(found[3]) > 1 and int(found[4]) == 0) else 1
-        # the largest column step of any row: above 1 some rows are gathered (dilated windows, strided far fields)
-        self._max_step = int(found[3])
+        _checked_summary(self, *self.summary.tolist()[:5])  # the one synchronisation: T is returned as a Python int, like the reference
 
     @property
     def T(self) -> int:
@@ -287,8 +280,31 @@ class AcsrBuild:
         return self._max_step
 
 
-def build_acsr(mask, BLOCK_HEIGHT: int, dev: torch.device) -> AcsrBuild:
-    entry, host = _mask_entry(mask, dev)
+def _checked_summary(b: AcsrBuild, t_max: int, failed: int, step_min: int, step_max: int, off_phase: int) -> None:
+    b.summary = None
+    assert failed == 0, "Incorrect unpacking of affine-indices."
+    b._T = t_max
+    # rows whose columns step by n and start in phase with the row index (dilated windows): kernels group them by phase
+    b._row_stride = step_min if (step_min == step_max and step_max > 1 and off_phase == 0) else 1
+    # the largest column step of any row: above 1 some rows are gathered (dilated windows, strided far fields)
+    b._max_step = step_max
+
+
+def _build_and_wait(entry: _MaskEntry, dm: torch.Tensor, BLOCK_HEIGHT: int):
+    """The build in one kernel that is waited for, kept with the mask's entry: a duplicate of its arrays for the caller, or
+    None where the native host path leaves the case to ``build_acsr``."""
+    found = None if torch.cuda.is_current_stream_capturing() else _hip.host().build(dm, BLOCK_HEIGHT)
+    if found is None:
+        return None
+    b = AcsrBuild()
+    (b.dTos_lin, b.dTos_trans, b.sTod_lin, b.sTod_trans, b.nnz, b.row_first, b.row_last, b.span_start, b.span_end), own = found[:2]
+    _checked_summary(b, *found[2:])
+    entry.builds[BLOCK_HEIGHT] = b
+    return b, own
+
+
+def build_acsr(mask, BLOCK_HEIGHT: int, dev: torch.device, entry_host=None) -> AcsrBuild:
+    entry, host = entry_host or _mask_entry(mask, dev)
     if BLOCK_HEIGHT in entry.builds:
         return entry.builds[BLOCK_HEIGHT]
     dm = _device_mask(mask, host, dev)
@@ -344,13 +360,22 @@ def create_acsr(mask, BLOCK_HEIGHT: int, GPU_ID: Any, *, T: int | None = None):
     hint for patterns whose rows alternate column phase, ``splat_max_step`` the largest column step of any row (both
     convert with ``int()``; after a call with ``T=`` that conversion is what reads the builder's record back)."""
     dev = _hip.resolve_device(GPU_ID)
-    b = build_acsr(mask, BLOCK_HEIGHT, dev)
-    if T is None:
-        b.resolve()
+    found = _mask_entry(mask, dev)
+    both = None
+    if T is None and isinstance(mask, torch.Tensor) and BLOCK_HEIGHT not in found[0].builds:
+        both = _build_and_wait(found[0], _device_mask(mask, None, dev), BLOCK_HEIGHT)
     # every caller gets tensors of its own, as from the reference's create_acsr: a build shared through the cache must
     # not change under one caller because another one wrote into its metadata
-    arrays = [t.clone() for t in (b.dTos_lin, b.dTos_trans, b.sTod_lin, b.sTod_trans, b.nnz, b.span_start, b.span_end)]
-    arrays[3].splat_first_col = b.row_first.clone()
+    if both is not None:
+        b, own = both
+        arrays = [*own[:5], own[7], own[8]]
+        arrays[3].splat_first_col = own[5]
+    else:
+        b = build_acsr(mask, BLOCK_HEIGHT, dev, found)
+        if T is None:
+            b.resolve()
+        arrays = [t.clone() for t in (b.dTos_lin, b.dTos_trans, b.sTod_lin, b.sTod_trans, b.nnz, b.span_start, b.span_end)]
+        arrays[3].splat_first_col = b.row_first.clone()
     if b.summary is None:
         if T is not None and int(T) != b.T:
             raise _hip.SplatError(f"T={T} was given, the mask's longest row has {b.T} live columns")

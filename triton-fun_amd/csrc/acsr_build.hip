@@ -1,12 +1,10 @@
 // ACSR builder and mask generators.
 //
-// splat_acsr_build: one wavefront (short rows) or one workgroup (rows >= 4 KiB) per mask row streams the row once
-// (16-byte loads), reducing the
-// byte sum (nnz), the first two columns whose byte equals 1 (the affine map's anchors a < b) and the
+// splat_acsr_build, splat_acsr_build_record: one wavefront per mask row streams the row once (16-byte loads), reducing the byte sum (nnz), the first two columns whose byte equals 1 (the affine map's anchors a < b) and the
 // first/last nonzero column.  Lane 0 then evaluates the 2x2 solve of acsr_helpers.py:122 in closed
 // form in double precision and rounds to float32, which is what the reference's
-// float64 -> torch.FloatTensor conversion stores.  A second, tiny kernel folds rows into the
-// per-row-block span pairs (acsr_helpers.py:135-140).  HBM-bound: rows*ld bytes in, 28*rows out.
+// float64 -> torch.FloatTensor conversion stores.  The per-row-block span pairs (acsr_helpers.py:135-140) come from the
+// same kernel, or, with the summary on the device, from a second, tiny one.  HBM-bound: rows*ld bytes in, 28*rows out.
 #include "splat_common.hpp"
 
 namespace splat {
@@ -83,18 +81,32 @@ __device__ __forceinline__ void init_summary(int32_t* summary) {
 }
 constexpr float kUnpackFailed = 0.0f;  // stored as a row's sTod_lin (a real step is >= 1) until the span kernel has counted it
 
+// Where a build's arrays go.  `twin`, when not 0, is the distance in elements from every array to its duplicate: a caller
+// that keeps a build and hands out another copy gets both from one kernel.
+struct RowOut {
+    float *dTos_lin, *dTos_trans, *sTod_lin, *sTod_trans, *nnz;
+    int32_t *row_first, *row_last;
+    float *span_start, *span_end;
+    int64_t twin;
+    template <typename T>
+    __device__ __forceinline__ void put(T* p, int i, T x) const {
+        p[i] = x;
+        if (twin) p[i + twin] = x;
+    }
+};
+
 // What one row contributes once its scan is reduced: the closed-form 2x2 solve.  (The summary extrema are
-// reduced by the span kernel: per-row atomics on one address cost more than streaming the whole mask.)
-__device__ __forceinline__ void finish_row(const RowScan& s, int row, int cols, float* dTos_lin, float* dTos_trans,
-                                           float* sTod_lin, float* sTod_trans, float* nnz_out, int32_t* row_first,
-                                           int32_t* row_last) {
+// reduced per row block: per-row atomics on one address cost more than streaming the whole mask.)  Returns whether the
+// row is one the reference asserts on (acsr_helpers.py:119); its stored step is `failed_lin`.
+__device__ __forceinline__ bool finish_row(const RowScan& s, int row, int cols, const RowOut& o, float failed_lin, float* lin_out,
+                                           float* trans_out) {
     const int nnz = (int)s.sum;
     double x0 = 1.0, x1 = 0.0;
     int step = 1;
     bool failed = false;
     if (nnz > 1) {
         if (s.m1 == kInf || s.m2 == kInf) {
-            failed = true;  // the reference asserts here (acsr_helpers.py:119); counted by the span kernel
+            failed = true;
         } else {
             step = s.m2 - s.m1;
             x0 = 1.0 / (double)step;
@@ -102,14 +114,48 @@ __device__ __forceinline__ void finish_row(const RowScan& s, int row, int cols, 
             x1 = (s.m1 == 0) ? 0.0 : -(double)s.m1 / (double)step;
         }
     }
-    dTos_lin[row] = (float)x0;
-    dTos_trans[row] = (float)x1;
-    sTod_lin[row] = failed ? kUnpackFailed : (float)step;
-    sTod_trans[row] = (float)fabs(x1);
-    nnz_out[row] = (float)nnz;
-    if (row_first) row_first[row] = (s.first == kInf) ? cols : s.first;
-    if (row_last) row_last[row] = s.last;
+    *lin_out = failed ? failed_lin : (float)step;
+    *trans_out = (float)fabs(x1);
+    o.put(o.dTos_lin, row, (float)x0);
+    o.put(o.dTos_trans, row, (float)x1);
+    o.put(o.sTod_lin, row, *lin_out);
+    o.put(o.sTod_trans, row, *trans_out);
+    o.put(o.nnz, row, (float)nnz);
+    if (o.row_first) o.put(o.row_first, row, (s.first == kInf) ? cols : s.first);
+    if (o.row_last) o.put(o.row_last, row, s.last);
+    return failed;
 }
+
+// The rows of one span block folded together: span_start = min(cols, min_r trans_r), span_end = max(-1, max_r nnz_r*lin_r +
+// trans_r), evaluated in double from the exact integers (a, lin, nnz) and rounded once to float32, and the block's share of
+// the summary: T = max nnz, smallest / largest column step over rows with nnz > 1, how many rows with nnz > 1 have a first
+// column that is not congruent to the row index modulo their step, and how many the reference would have asserted on.
+struct BlockFold {
+    double lo, hi;
+    int t_max, step_min, step_max, off_phase, failed;
+    __device__ __forceinline__ void init(int cols) {
+        lo = (double)cols, hi = -1.0;
+        t_max = 0, step_min = 0x7fffffff, step_max = 0, off_phase = 0, failed = 0;
+    }
+    __device__ __forceinline__ void row(int r, float linf, float trans, int cnt) {
+        const int lin = (int)linf;
+        const int a = (int)rintf(linf * trans);
+        const double t = (double)a / (double)lin;
+        lo = fmin(lo, t);
+        hi = fmax(hi, (double)((int64_t)cnt * lin) + t);
+        t_max = max(t_max, cnt);
+        if (cnt > 1) {
+            step_min = min(step_min, lin);
+            step_max = max(step_max, lin);
+            off_phase += ((a - r) % lin) != 0;
+        }
+    }
+    __device__ __forceinline__ void merge(const BlockFold& b) {
+        lo = fmin(lo, b.lo), hi = fmax(hi, b.hi);
+        t_max = max(t_max, b.t_max), step_min = min(step_min, b.step_min), step_max = max(step_max, b.step_max);
+        off_phase += b.off_phase, failed += b.failed;
+    }
+};
 
 __device__ __forceinline__ void scan_chunk(RowScan& s, const u32x4& x, int c) {
     if ((x.x | x.y | x.z | x.w) == 0) return;
@@ -119,141 +165,73 @@ __device__ __forceinline__ void scan_chunk(RowScan& s, const u32x4& x, int c) {
     s.dword(x.w, c + 12);
 }
 
-// Short rows: one wavefront per row, four rows per workgroup.
-__global__ __launch_bounds__(256) void acsr_rows_kernel(const uint8_t* __restrict__ mask, int rows, int cols,
-                                                        int64_t ld, int vec_ok, float* __restrict__ dTos_lin,
-                                                        float* __restrict__ dTos_trans, float* __restrict__ sTod_lin,
-                                                        float* __restrict__ sTod_trans, float* __restrict__ nnz_out,
-                                                        int32_t* __restrict__ row_first,
-                                                        int32_t* __restrict__ row_last, int32_t* __restrict__ summary) {
-    init_summary(summary);
+// A workgroup takes `per_block` consecutive rows, a wavefront one row at a time: 16-byte pieces from the row's first aligned
+// address on (rows of any pitch), eight per lane in flight, and single bytes at the two ends.  Sixteen wavefronts and at most
+// 64 registers, so that a CU holds two workgroups and the loads of 32 rows are in flight at once: a mask of 8192 rows is one
+// wave of workgroups over the chip.  No cross-wavefront traffic but the block's fold.
+//
+// FOLD: the workgroup's rows are one span block; its spans and its share of the summary (5 integers, 8 apart, into memory
+// that the host reads) come from the same kernel.  With a second kernel for the spans, which walks 16 rows a thread with
+// few threads, and the summary read back through a copy, an 8192 x 8192 mask took 23 us on the GPU in two kernels and 95 us
+// for the whole call; in this one kernel 16.7 us (4.0 TB/s) and 37 us.
+constexpr int kRowWaves = 16;
+template <bool FOLD>
+__global__ __launch_bounds__(64 * kRowWaves, 8) void acsr_rows_kernel(const uint8_t* __restrict__ mask, int rows, int cols, int64_t ld,
+                                                                      int per_block, RowOut o, int32_t* __restrict__ summary,
+                                                                      int32_t* __restrict__ shares) {
+    __shared__ BlockFold s_fold[kRowWaves];
+    if constexpr (!FOLD) init_summary(summary);
     const int lane = threadIdx.x & 63;
-    const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (row >= rows) return;
-    const uint8_t* p = mask + (int64_t)row * ld;
-    RowScan s;
-    s.init();
-    int done = 0;
-    if (vec_ok) {
-        const int nvec = cols >> 4;
-        const u32x4* pv = reinterpret_cast<const u32x4*>(p);
-        for (int i = lane; i < nvec; i += 64) scan_chunk(s, pv[i], i << 4);
-        done = nvec << 4;
-    }
-    for (int c = done + lane; c < cols; c += 64) s.byte(p[c], c);
-    s.wave_reduce();
-    if (lane == 0) finish_row(s, row, cols, dTos_lin, dTos_trans, sTod_lin, sTod_trans, nnz_out, row_first, row_last);
-}
-
-// Long rows (>= 4 KiB, 16-byte aligned): one workgroup per row, so that the memory system sees a few thousand
-// sequential 4 KiB-wide streams instead of tens of thousands of 1 KiB-wide ones; up to 8 loads in flight per lane.
-__global__ __launch_bounds__(256) void acsr_rows_wide_kernel(const uint8_t* __restrict__ mask, int rows, int cols,
-                                                             int64_t ld, float* __restrict__ dTos_lin,
-                                                             float* __restrict__ dTos_trans, float* __restrict__ sTod_lin,
-                                                             float* __restrict__ sTod_trans, float* __restrict__ nnz_out,
-                                                             int32_t* __restrict__ row_first,
-                                                             int32_t* __restrict__ row_last, int32_t* __restrict__ summary) {
-    init_summary(summary);
-    __shared__ uint32_t s_sum[4];
-    __shared__ int s_m1[4], s_m2[4], s_first[4], s_last[4];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int row = blockIdx.x;
-    const uint8_t* p = mask + (int64_t)row * ld;
-    RowScan s;
-    s.init();
-    const int nvec = cols >> 4;
-    const u32x4* pv = reinterpret_cast<const u32x4*>(p);
-    int i = tid;
-    for (; i + 7 * 256 < nvec; i += 8 * 256) {
-        u32x4 xs[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) xs[u] = __builtin_nontemporal_load(pv + i + 256 * u);
-#pragma unroll
-        for (int u = 0; u < 8; ++u) scan_chunk(s, xs[u], (i + 256 * u) << 4);
-    }
-    for (; i + 3 * 256 < nvec; i += 4 * 256) {
-        u32x4 xs[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) xs[u] = __builtin_nontemporal_load(pv + i + 256 * u);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) scan_chunk(s, xs[u], (i + 256 * u) << 4);
-    }
-    for (; i < nvec; i += 256) scan_chunk(s, pv[i], i << 4);
-    for (int c = (nvec << 4) + tid; c < cols; c += 256) s.byte(p[c], c);
-    s.wave_reduce();
-    if (lane == 0) {
-        s_sum[wave] = s.sum;
-        s_m1[wave] = s.m1;
-        s_m2[wave] = s.m2;
-        s_first[wave] = s.first;
-        s_last[wave] = s.last;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        RowScan t;
-        t.init();
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            t.sum += s_sum[w];
-            const int n1 = min(t.m1, s_m1[w]);
-            const int n2 = min(max(t.m1, s_m1[w]), min(t.m2, s_m2[w]));
-            t.m1 = n1;
-            t.m2 = n2;
-            t.first = min(t.first, s_first[w]);
-            t.last = max(t.last, s_last[w]);
-        }
-        finish_row(t, row, cols, dTos_lin, dTos_trans, sTod_lin, sTod_trans, nnz_out, row_first, row_last);
-    }
-}
-
-// Long rows, one wavefront per row: a wavefront takes its rows one after the other (consecutive wavefronts hold
-// consecutive rows at any time), each row in batches of eight 16-byte chunks per lane with the next batch requested
-// before the current one is scanned; no cross-wavefront reduction, no barrier, no LDS.
-__global__ __launch_bounds__(256) void acsr_rows_stream_kernel(const uint8_t* __restrict__ mask, int rows, int cols,
-                                                               int64_t ld, float* __restrict__ dTos_lin,
-                                                               float* __restrict__ dTos_trans, float* __restrict__ sTod_lin,
-                                                               float* __restrict__ sTod_trans, float* __restrict__ nnz_out,
-                                                               int32_t* __restrict__ row_first,
-                                                               int32_t* __restrict__ row_last, int32_t* __restrict__ summary) {
-    init_summary(summary);
-    const int lane = threadIdx.x & 63;
-    const int n_waves = gridDim.x * 4;
-    const int nvec = cols >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n_waves = blockDim.x >> 6;
+    const int r_end = min(rows, ((int)blockIdx.x + 1) * per_block);
     constexpr int NB = 8;
-    auto load_batch = [&](u32x4 (&xs)[NB], const u32x4* pv, int i0) {
-#pragma unroll
-        for (int u = 0; u < NB; ++u) {
-            const int i = i0 + 64 * u;
-            xs[u] = i < nvec ? __builtin_nontemporal_load(pv + i) : u32x4{0, 0, 0, 0};
-        }
-    };
-    for (int row = blockIdx.x * 4 + (threadIdx.x >> 6); row < rows; row += n_waves) {
+    BlockFold f;
+    f.init(cols);
+    for (int row = blockIdx.x * per_block + wave; row < r_end; row += n_waves) {
         const uint8_t* p = mask + (int64_t)row * ld;
-        const u32x4* pv = reinterpret_cast<const u32x4*>(p);
+        const int head = min(cols, (int)(-reinterpret_cast<uintptr_t>(p) & 15));
+        const int nvec = (cols - head) >> 4;
+        const u32x4* pv = reinterpret_cast<const u32x4*>(p + head);
         RowScan s;
         s.init();
-        u32x4 cur[NB], nxt[NB];
-        load_batch(cur, pv, lane);
+        const int tail0 = head + (nvec << 4);  // fewer than 16 bytes before `head` and fewer than 16 from `tail0` on
+        uint32_t edge = 0;
+        const int edge_col = lane < 16 ? lane : tail0 + lane - 16;
+        if (lane < 16 ? lane < head : (lane < 32 && edge_col < cols)) edge = p[edge_col];
         for (int i0 = lane; i0 < nvec; i0 += 64 * NB) {
-            const bool more = i0 + 64 * NB < nvec;
-            if (more) load_batch(nxt, pv, i0 + 64 * NB);
+            u32x4 xs[NB];
 #pragma unroll
-            for (int u = 0; u < NB; ++u) scan_chunk(s, cur[u], (i0 + 64 * u) << 4);
-            if (more) {
+            for (int u = 0; u < NB; ++u) xs[u] = i0 + 64 * u < nvec ? __builtin_nontemporal_load(pv + i0 + 64 * u) : u32x4{0, 0, 0, 0};
 #pragma unroll
-                for (int u = 0; u < NB; ++u) cur[u] = nxt[u];
+            for (int u = 0; u < NB; ++u) scan_chunk(s, xs[u], head + ((i0 + 64 * u) << 4));
+        }
+        s.byte(edge, edge_col);
+        s.wave_reduce();
+        if (lane == 0) {
+            float lin, trans;
+            const bool failed = finish_row(s, row, cols, o, FOLD ? 1.0f : kUnpackFailed, &lin, &trans);
+            if constexpr (FOLD) {
+                f.failed += failed;
+                f.row(row, lin, trans, (int)s.sum);
             }
         }
-        for (int c = (nvec << 4) + lane; c < cols; c += 64) s.byte(p[c], c);
-        s.wave_reduce();
-        if (lane == 0) finish_row(s, row, cols, dTos_lin, dTos_trans, sTod_lin, sTod_trans, nnz_out, row_first, row_last);
+    }
+    if constexpr (FOLD) {
+        if (lane == 0) s_fold[wave] = f;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (int w = 1; w < n_waves; ++w) f.merge(s_fold[w]);
+            o.put(o.span_start, blockIdx.x, (float)f.lo);
+            o.put(o.span_end, blockIdx.x, (float)f.hi);
+            int4* const mine = reinterpret_cast<int4*>(shares) + 2 * blockIdx.x;
+            mine[0] = make_int4(f.t_max, f.failed, f.step_min, f.step_max);
+            mine[1] = make_int4(f.off_phase, 0, 0, 0);
+        }
     }
 }
 
-// One thread per row block: span_start = min(cols, min_r trans_r), span_end = max(-1, max_r nnz_r*lin_r + trans_r)
-// evaluated in double from the exact integers (a, lin, nnz) and rounded once to float32.  The same pass reduces
-// the summary: T = max nnz, smallest / largest column step over rows with nnz > 1, and how many rows with
-// nnz > 1 have a first column that is not congruent to the row index modulo their step.
+// One thread per row block: spans and summary (BlockFold) of rows that are in memory.
 __global__ __launch_bounds__(256) void acsr_spans_kernel(float* __restrict__ sTod_lin,
                                                          const float* __restrict__ sTod_trans,
                                                          const float* __restrict__ nnz, int rows, int cols,
@@ -261,38 +239,27 @@ __global__ __launch_bounds__(256) void acsr_spans_kernel(float* __restrict__ sTo
                                                          float* __restrict__ span_end, int32_t* __restrict__ summary) {
     const int g = blockIdx.x * blockDim.x + threadIdx.x;
     const int n_blocks = (rows + block_height - 1) / block_height;
-    int t_max = 0, step_min = 0x7fffffff, step_max = 0, off_phase = 0, failed = 0;
+    BlockFold f;
+    f.init(cols);
     if (g < n_blocks) {
-        double lo = (double)cols, hi = -1.0;
         const int r1 = min(rows, (g + 1) * block_height);
         for (int r = g * block_height; r < r1; ++r) {
             float linf = sTod_lin[r];
             if (linf == kUnpackFailed) {  // a row the reference would have asserted on: counted, then stored as (1, 0) like
-                ++failed;                 // the rows with at most one live column
+                ++f.failed;               // the rows with at most one live column
                 linf = 1.0f;
                 sTod_lin[r] = linf;
             }
-            const int lin = (int)linf;
-            const int a = (int)rintf(linf * sTod_trans[r]);
-            const int cnt = (int)nnz[r];
-            const double t = (double)a / (double)lin;
-            lo = fmin(lo, t);
-            hi = fmax(hi, (double)((int64_t)cnt * lin) + t);
-            t_max = max(t_max, cnt);
-            if (cnt > 1) {
-                step_min = min(step_min, lin);
-                step_max = max(step_max, lin);
-                off_phase += ((a - r) % lin) != 0;
-            }
+            f.row(r, linf, sTod_trans[r], (int)nnz[r]);
         }
-        span_start[g] = (float)lo;
-        span_end[g] = (float)hi;
+        span_start[g] = (float)f.lo;
+        span_end[g] = (float)f.hi;
     }
-    t_max = wave_max_i(t_max);
-    step_min = wave_min_i(step_min);
-    step_max = wave_max_i(step_max);
-    off_phase = (int)wave_sum((float)off_phase);  // at most 64 * block_height per wavefront: exact in float
-    failed = (int)wave_sum((float)failed);
+    const int t_max = wave_max_i(f.t_max);
+    const int step_min = wave_min_i(f.step_min);
+    const int step_max = wave_max_i(f.step_max);
+    const int off_phase = (int)wave_sum((float)f.off_phase);  // at most 64 * block_height per wavefront: exact in float
+    const int failed = (int)wave_sum((float)f.failed);
     if ((threadIdx.x & 63) == 0) {
         if (failed) atomicAdd(&summary[1], failed);
         atomicMax(&summary[0], t_max);
@@ -422,16 +389,13 @@ __device__ __forceinline__ RowScan pattern_row(int pattern, int64_t i, int64_t s
     return r;
 }
 
-__global__ __launch_bounds__(256) void acsr_rows_pattern_kernel(int pattern, int s, int64_t p0, int64_t p1,
-                                                                float* __restrict__ dTos_lin, float* __restrict__ dTos_trans,
-                                                                float* __restrict__ sTod_lin, float* __restrict__ sTod_trans,
-                                                                float* __restrict__ nnz_out, int32_t* __restrict__ row_first,
-                                                                int32_t* __restrict__ row_last, int32_t* __restrict__ summary) {
+__global__ __launch_bounds__(256) void acsr_rows_pattern_kernel(int pattern, int s, int64_t p0, int64_t p1, RowOut o,
+                                                                int32_t* __restrict__ summary) {
     init_summary(summary);
     const int row = blockIdx.x * blockDim.x + threadIdx.x;
     if (row >= s) return;
-    finish_row(pattern_row(pattern, row, s, p0, p1), row, s, dTos_lin, dTos_trans, sTod_lin, sTod_trans, nnz_out, row_first,
-               row_last);
+    float lin, trans;
+    finish_row(pattern_row(pattern, row, s, p0, p1), row, s, o, kUnpackFailed, &lin, &trans);
 }
 
 __global__ __launch_bounds__(256) void mask_generate_kernel(uint8_t* __restrict__ mask, int rows, int cols,
@@ -474,23 +438,36 @@ extern "C" int splat_acsr_build(const uint8_t* mask, int64_t rows, int64_t cols,
     if (rows > (1 << 23) || cols > (1 << 23))
         return fail(SPLAT_E_SHAPE, "splat_acsr_build: rows and cols are limited to 2^23 (got %lld, %lld)", (long long)rows, (long long)cols);
     hipStream_t st = (hipStream_t)stream;
-    const int vec_ok = ((reinterpret_cast<uintptr_t>(mask) & 15) == 0 && (ld & 15) == 0) ? 1 : 0;
-    // rows of 16 KiB and more: a workgroup per row; 4 to 16 KiB: a wavefront per row, each wavefront taking several rows
-    // (at 8 KiB rows 0.028 against 0.038 ms with caches flushed; at 16 KiB the two are equal and the workgroup form is
-    // 5 % faster on a mask that is found in the caches)
-    if (vec_ok && cols >= 4096 && cols < 16384)
-        acsr_rows_stream_kernel<<<(unsigned)min((int64_t)1024, (rows + 3) / 4), 256, 0, st>>>(mask, (int)rows, (int)cols, ld, dTos_lin, dTos_trans, sTod_lin,
-                                                              sTod_trans, nnz, row_first, row_last, summary);
-    else if (vec_ok && cols >= 4096)
-        acsr_rows_wide_kernel<<<(unsigned)rows, 256, 0, st>>>(mask, (int)rows, (int)cols, ld, dTos_lin, dTos_trans, sTod_lin,
-                                                              sTod_trans, nnz, row_first, row_last, summary);
-    else
-        acsr_rows_kernel<<<(unsigned)((rows + 3) / 4), 256, 0, st>>>(mask, (int)rows, (int)cols, ld, vec_ok, dTos_lin, dTos_trans,
-                                                                     sTod_lin, sTod_trans, nnz, row_first, row_last, summary);
+    const RowOut out{dTos_lin, dTos_trans, sTod_lin, sTod_trans, nnz, row_first, row_last, nullptr, nullptr, 0};
+    acsr_rows_kernel<false><<<(unsigned)((rows + kRowWaves - 1) / kRowWaves), 64 * kRowWaves, 0, st>>>(mask, (int)rows, (int)cols, ld,
+                                                                                                      kRowWaves, out, summary, nullptr);
     const int n_blocks = (int)((rows + block_height - 1) / block_height);
     acsr_spans_kernel<<<(n_blocks + 255) / 256, 256, 0, st>>>(sTod_lin, sTod_trans, nnz, (int)rows, (int)cols, block_height,
                                                                span_start, span_end, summary);
     return check_launch("splat_acsr_build");
+}
+
+extern "C" int splat_acsr_build_record(const uint8_t* mask, int64_t rows, int64_t cols, int64_t ld, int32_t block_height, void* record,
+                                       int64_t twin, int32_t* shares, void* stream) {
+    begin_launch();
+    if (!mask || !record || !shares) return fail(SPLAT_E_NULL, "splat_acsr_build_record: null pointer argument");
+    if (rows <= 0 || cols <= 0 || ld < cols || block_height <= 0 || rows > (1 << 23) || cols > (1 << 23))
+        return fail(SPLAT_E_SHAPE, "splat_acsr_build_record: need 0 < rows, cols <= 2^23, ld >= cols, block_height > 0 (got %lld, %lld, %lld, %d)",
+                    (long long)rows, (long long)cols, (long long)ld, block_height);
+    const int64_t n_blocks = (rows + block_height - 1) / block_height;
+    const int64_t row_step = (rows + 63) & ~(int64_t)63, span_step = (n_blocks + 63) & ~(int64_t)63;
+    if (twin != 0 && twin < 7 * row_step + 2 * span_step)
+        return fail(SPLAT_E_SHAPE, "splat_acsr_build_record: the duplicate at %lld overlaps the record", (long long)twin);
+    if ((reinterpret_cast<uintptr_t>(record) & 3) != 0 || (reinterpret_cast<uintptr_t>(shares) & 15) != 0)
+        return fail(SPLAT_E_ALIGN, "splat_acsr_build_record: misaligned record or shares");
+    float* const f = static_cast<float*>(record);
+    const RowOut out{f, f + row_step, f + 2 * row_step, f + 3 * row_step, f + 4 * row_step,
+                     reinterpret_cast<int32_t*>(f + 5 * row_step), reinterpret_cast<int32_t*>(f + 6 * row_step),
+                     f + 7 * row_step, f + 7 * row_step + span_step, twin};
+    const int waves = (int)min((int64_t)kRowWaves, min((int64_t)block_height, rows));
+    acsr_rows_kernel<true><<<(unsigned)n_blocks, 64 * waves, 0, (hipStream_t)stream>>>(mask, (int)rows, (int)cols, ld, block_height, out,
+                                                                                       nullptr, shares);
+    return check_launch("splat_acsr_build_record");
 }
 
 static int check_pattern(const char* who, int64_t s, int32_t pattern, int64_t p0, int64_t p1) {
@@ -516,8 +493,8 @@ extern "C" int splat_acsr_build_pattern(int32_t pattern, int64_t s, int64_t p0, 
     if (int rc = check_pattern(who, s, pattern, p0, p1)) return rc;
     if (p0 > (1 << 23) || p1 > (1 << 23)) return fail(SPLAT_E_SHAPE, "%s: pattern parameters are limited to 2^23", who);
     hipStream_t st = (hipStream_t)stream;
-    acsr_rows_pattern_kernel<<<(unsigned)((s + 255) / 256), 256, 0, st>>>(pattern, (int)s, p0, p1, dTos_lin, dTos_trans, sTod_lin,
-                                                                         sTod_trans, nnz, row_first, row_last, summary);
+    const RowOut out{dTos_lin, dTos_trans, sTod_lin, sTod_trans, nnz, row_first, row_last, nullptr, nullptr, 0};
+    acsr_rows_pattern_kernel<<<(unsigned)((s + 255) / 256), 256, 0, st>>>(pattern, (int)s, p0, p1, out, summary);
     const int n_blocks = (int)((s + block_height - 1) / block_height);
     acsr_spans_kernel<<<(n_blocks + 255) / 256, 256, 0, st>>>(sTod_lin, sTod_trans, nnz, (int)s, (int)s, block_height, span_start,
                                                                span_end, summary);

@@ -17,7 +17,9 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/custom_class.h>
 
+#include <algorithm>
 #include <cstring>
+#include <mutex>
 #include <vector>
 
 #include "../../include/splat_hip.h"
@@ -38,6 +40,7 @@ struct Api {
     decltype(&splat_softmax) softmax;
     decltype(&splat_spmm) spmm;
     decltype(&splat_spmm_planned) spmm_planned;
+    decltype(&splat_acsr_build_record) build_record;
 } api;
 PyObject* g_error = nullptr;  // SplatError
 
@@ -418,6 +421,106 @@ PyObject* py_spmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
 }
 
+// ---- the ACSR of a mask ---------------------------------------------------------------------------------------------------------
+constexpr int64_t kShareBlocks = 1024;  // row blocks whose shares of the summary a buffer holds
+
+// Pinned buffers for the shares of the builds under way: one per build between its launch and its end (the call waits for the
+// stream before it gives the buffer back), at most kKeep of them kept for the next ones.
+class ShareBuffers {
+  public:
+    at::Tensor take() {
+        {
+            std::lock_guard<std::mutex> hold(m_);
+            if (!free_.empty()) {
+                at::Tensor t = std::move(free_.back());
+                free_.pop_back();
+                return t;
+            }
+        }
+        return at::empty({kShareBlocks * 8}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+    }
+    void give(at::Tensor t) {
+        std::lock_guard<std::mutex> hold(m_);
+        if (free_.size() < kKeep) free_.push_back(std::move(t));
+    }
+
+  private:
+    static constexpr size_t kKeep = 4;
+    std::mutex m_;
+    std::vector<at::Tensor> free_;
+};
+ShareBuffers* share_buffers() {
+    static ShareBuffers* b = new ShareBuffers;  // (never destroyed: the allocator may be gone at the process's end)
+    return b;
+}
+
+// One array of a record, as a tensor of its own on the record's storage.
+at::Tensor part_of(const at::Tensor& record, int64_t offset, int64_t n, caffe2::TypeMeta type) {
+    at::Tensor t = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(record.storage()), record.key_set(), type);
+    t.unsafeGetTensorImpl()->set_storage_offset(record.storage_offset() + offset);
+    t.unsafeGetTensorImpl()->set_sizes_contiguous({n});
+    return t;
+}
+
+// build(mask, block_height) -> ((9 tensors), (9 tensors), T, failed rows, smallest step, largest step, rows off phase): the arrays
+// of a record and of its duplicate, dTos_lin, dTos_trans, sTod_lin, sTod_trans, nnz, row_first, row_last, span_start, span_end.
+// Waits for the stream (T comes back as a number).  None when the case is not an ordinary one.
+PyObject* py_build(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 2) return PyErr_Format(PyExc_TypeError, "build takes 2 arguments");
+    try {
+        if (!THPVariable_Check(a[0])) Py_RETURN_NONE;
+        const at::Tensor& mask = THPVariable_Unpack(a[0]);
+        const long long bh = PyLong_AsLongLong(a[1]);
+        if (bh == -1 && PyErr_Occurred()) return nullptr;
+        if (!mask.is_cuda() || mask.scalar_type() != at::kByte || mask.dim() != 2 || mask.get_device() != c10::hip::current_device() ||
+            mask.numel() == 0 || mask.stride(1) != 1 || mask.stride(0) < mask.size(1) || bh < 1 || bh > (1 << 23))
+            Py_RETURN_NONE;
+        const int64_t rows = mask.size(0), cols = mask.size(1), blocks = (rows + bh - 1) / bh;
+        // the one-kernel build gives a row block to a workgroup: short blocks and very tall ones leave wavefronts or CUs idle
+        if (blocks > kShareBlocks || bh < 4 || bh > 64) Py_RETURN_NONE;
+        const auto stream = c10::hip::getCurrentHIPStream(mask.get_device());
+        const int64_t row_step = (rows + 63) / 64 * 64, span_step = (blocks + 63) / 64 * 64, twin = 7 * row_step + 2 * span_step;
+        const at::Tensor kept = at::empty({2 * twin}, mask.options().dtype(at::kFloat));
+        at::Tensor shares = share_buffers()->take();
+        const int32_t* const sh = shares.data_ptr<int32_t>();
+        const int rc = api.build_record(mask.data_ptr<uint8_t>(), rows, cols, mask.stride(0), (int32_t)bh, kept.data_ptr(), twin,
+                                        shares.data_ptr<int32_t>(), stream.stream());
+        if (rc) return raise_rc("splat_acsr_build_record", rc);
+        PyThreadState* const released = PyEval_SaveThread();
+        std::string failed_wait;
+        try {
+            c10::hip::stream_synchronize(stream.stream());
+        } catch (const std::exception& e) {
+            failed_wait = e.what();
+        }
+        PyEval_RestoreThread(released);
+        if (!failed_wait.empty()) {  // (the buffer is not given back: the kernel may still write to it)
+            new at::Tensor(std::move(shares));
+            PyErr_SetString(PyExc_RuntimeError, failed_wait.c_str());
+            return nullptr;
+        }
+        int32_t t_max = 0, bad = 0, step_min = 0x7fffffff, step_max = 0, off = 0;
+        for (int64_t b = 0; b < blocks; ++b) {
+            const int32_t* s = sh + 8 * b;
+            t_max = std::max(t_max, s[0]), bad += s[1], step_min = std::min(step_min, s[2]), step_max = std::max(step_max, s[3]), off += s[4];
+        }
+        share_buffers()->give(std::move(shares));
+        PyObject* sets[2];
+        for (int k = 0; k < 2; ++k) {
+            sets[k] = PyTuple_New(9);
+            if (!sets[k]) return nullptr;
+            for (int i = 0; i < 9; ++i) {
+                const int64_t at = k * twin + (i < 7 ? i * row_step : 7 * row_step + (i - 7) * span_step);
+                PyTuple_SET_ITEM(sets[k], i, THPVariable_Wrap(part_of(kept, at, i < 7 ? rows : blocks,
+                                                                      caffe2::TypeMeta::fromScalarType(i == 5 || i == 6 ? at::kInt : at::kFloat))));
+            }
+        }
+        return Py_BuildValue("NNiiiii", sets[0], sets[1], t_max, bad, step_min, step_max, off);
+    } catch (const std::exception& e) {
+        return raise_std(e);
+    }
+}
+
 // bind({entry point: address}, SplatError)
 PyObject* py_bind(PyObject*, PyObject* args) {
     PyObject *table, *err;
@@ -435,7 +538,7 @@ PyObject* py_bind(PyObject*, PyObject* args) {
         !take("splat_attention_fwd_stats", api.fwd_stats) || !take("splat_transpose_keys", api.transpose_keys) ||
         !take("splat_attention_bwd", api.bwd) || !take("splat_attention_bwd_keys", api.bwd_keys) || !take("splat_sddmm", api.sddmm) ||
         !take("splat_sddmm_probs", api.sddmm_probs) || !take("splat_sddmm_planned", api.sddmm_planned) ||
-        !take("splat_softmax", api.softmax) || !take("splat_spmm", api.spmm) || !take("splat_spmm_planned", api.spmm_planned))
+        !take("splat_softmax", api.softmax) || !take("splat_spmm", api.spmm) || !take("splat_spmm_planned", api.spmm_planned) || !take("splat_acsr_build_record", api.build_record))
         return nullptr;
     Py_INCREF(err);
     Py_XSETREF(g_error, err);
@@ -448,6 +551,7 @@ PyMethodDef methods[] = {
     {"forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_forward)), METH_FASTCALL, "fused forward"},
     {"grad_state", py_grad_state, METH_VARARGS, "what the differentiable attention keeps"},
     {"attend", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_attend)), METH_FASTCALL, "differentiable attention"},
+    {"build", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_build)), METH_FASTCALL, "the ACSR of a mask tensor"},
     {"sddmm", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_sddmm)), METH_FASTCALL, "sampled product"},
     {"softmax", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_softmax)), METH_FASTCALL, "softmax of compressed rows"},
     {"spmm", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_spmm)), METH_FASTCALL, "compressed rows times dense"},
