@@ -1,0 +1,48 @@
+"""The float32 attention kernels (16 rows a wavefront, 64 a workgroup, tiles of 32 or 16 positions) against float64 where their
+tiles can go wrong: lengths around the edges of rows, workgroups and row blocks, windows that begin and end inside a subtile,
+gathered and two-segment walks, rows without entries, K stored either way."""
+import pytest
+import torch
+
+import acsr_helpers as A
+from r_attention import RegularAttention, attention_with_grad
+
+pytestmark = pytest.mark.gpu
+
+MASKS = {
+    "diagonal": lambda L: [A.causal_windowed_pattern(L, 0)],
+    "causal": lambda L: [A.causal_windowed_pattern(L, 16)],
+    "windowed": lambda L: [A.windowed_pattern(L, 23)],
+    "dilated": lambda L: [A.dilated_pattern(L, 11, 3)],
+    "strided": lambda L: A.strided_patterns(L, 9, 7),
+    "far only": lambda L: A.strided_patterns(L, 9, 7)[1:],  # the first rows hold nothing
+}
+CASES = [(m, L, d) for m in MASKS for L in (17, 64, 257) for d in (64, 128)] + \
+    [("causal", L, 64) for L in (1, 15, 16, 63, 65, 127, 128, 129, 700)] + [("dilated", L, 128) for L in (33, 130, 700)]
+
+
+@pytest.mark.parametrize("name,L,d", CASES)
+def test_forward_and_gradients_against_float64(dev, name, L, d):
+    masks = MASKS[name](L)
+    if L < 8 and name == "far only":
+        pytest.skip("no entries")
+    B, H = 2, 2
+    g = torch.Generator().manual_seed(L + d)
+    q, k, v, go = (torch.randn(B, H, L, d, generator=g) for _ in range(4))
+    live = sum(m.device_mask(dev) for m in masks).cpu() > 0
+    wide = [t.double().requires_grad_(True) for t in (q, k, v)]
+    s = (wide[0] @ wide[1].transpose(2, 3) * d ** -0.5).masked_fill(~live, float("-inf"))
+    p = torch.where(live.any(1)[:, None], torch.softmax(s, -1), torch.zeros_like(s)).masked_fill(~live, 0.0)
+    want = p @ wide[2]
+    grads = torch.autograd.grad(want, wide, go.double())
+    attn = RegularAttention(B, L, H, d, masks, 16, 16, dev, torch.float32, scale=d ** -0.5)
+    on = [t.to(dev) for t in (q, k, v)]
+    for kT in (on[1].transpose(2, 3), on[1].transpose(2, 3).contiguous()):
+        got = attn([on[0], kT, on[2]]).cpu()
+        assert float((got - want).detach().abs().max()) <= 1e-5
+    on = [t.requires_grad_(True) for t in on]
+    out = attention_with_grad(*on, attn)
+    assert float((out.cpu() - want).detach().abs().max()) <= 1e-5
+    for a, b in zip(torch.autograd.grad(out, on, go.to(dev)), grads):
+        b = torch.nan_to_num(b)
+        assert float((a.cpu() - b).abs().max()) <= 2e-5 * max(1.0, float(b.abs().max()))

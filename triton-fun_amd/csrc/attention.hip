@@ -26,28 +26,6 @@
 
 namespace splat {
 
-struct AttnParams {
-    const void* q;
-    const void* k;
-    const void* v;
-    void* o;
-    int64_t q_sb, q_sh, q_sl;
-    int64_t k_sb, k_sh, k_sd, k_sl;
-    int64_t v_sb, v_sh, v_sl;
-    int64_t o_sb, o_sh, o_sl;
-    int B, H, L;
-    float scale_log2e;
-    int n_seg;
-    SegPtrs seg[SPLAT_MAX_SEGMENTS];
-    int n_row_blocks;
-    int total;
-    int row_stride;
-    const PlanRec* plan;  // plan table of this mask (PLANNED kernels), variant already selected
-    float* lse;           // optional [B*H, L]: log of every row's sum of exponentials (natural log, scaled scores)
-};
-
-constexpr float kRescaleThreshold = 8.0f;  // in log2 units: exponentials stay below 2^8 before the reference moves
-
 // Exponentials of one tile of scores against the rows' references (mb = reference * c2), as MFMA B fragments; returns
 // the lane's sum.
 template <int NT, typename T>
@@ -100,9 +78,10 @@ __device__ __forceinline__ bool softmax_tile(f32x16 (&s)[NT], Frag<T> (&pf)[NT][
 }
 
 template <typename T, int D, bool KT, int BN, int NSTAGE, bool PLANNED>
-__global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void attn_fwd_kernel(const AttnParams p) {
+__global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnParams p) {
     using G = TileGeom<T, D, KT, BN>;
     constexpr int ES = G::ES;
+    static_assert(ES == 2, "16-bit element types (float32: attention_f32.hip)");
     constexpr int BM = 128;
     constexpr int KS = D / 16;  // contraction steps of the score product
     constexpr int DT = D / 32;  // 32-row tiles of O^T
@@ -110,7 +89,6 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void attn_fwd_kernel(c
     constexpr int PD = NSTAGE - 1;  // tiles whose copies run ahead of the tile being computed
     static_assert(NT == 1 || NT == 2, "tiles of 32 or 64 keys");
     static_assert(PD == 1 || PD == 3, "the wait ladder below covers 2 and 4 stages");
-    constexpr bool FAST_DMA = (ES == 2);  // lane offsets of the LDS-DMA do not depend on the instruction index
 
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     __shared__ SegPlan s_plan[SPLAT_MAX_SEGMENTS];
@@ -172,9 +150,9 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void attn_fwd_kernel(c
     // ---- tile walker: asynchronous global -> LDS copies of a tile into a stage -------------------------
     // A tile is copied as 1 KiB blocks, one wavefront instruction each; block q holds tile rows q*RPI.. and
     // wavefront w issues blocks w, w+4, ...  Lane i of a block supplies physical chunk i, i.e. (row i / CPR,
-    // chunk position i % CPR), and loads the logical chunk the tile's swizzle assigns to that position.  For
-    // 16-bit types that assignment does not depend on the block, so a lane's source offset within a block is
-    // a per-segment constant and the block's base is wavefront-uniform.
+    // chunk position i % CPR), and loads the logical chunk the tile's swizzle assigns to that position.  That
+    // assignment does not depend on the block, so a lane's source offset within a block is a per-segment
+    // constant and the block's base is wavefront-uniform.
     constexpr int V_CPR = G::V_ROWB / 16, V_RPI = 1024 / G::V_ROWB;
     constexpr int K_CPR = G::K_ROWB / 16, K_RPI = 1024 / G::K_ROWB;
     constexpr int V_NI = BN * G::V_ROWB / 4096, K_NI = G::K_ROWS * G::K_ROWB / 4096;  // blocks per wavefront
@@ -185,7 +163,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void attn_fwd_kernel(c
         char* ks_w = smem + stage * G::STAGE;
         char* vs_w = ks_w + G::K_BYTES;
         auto key_row = [&](int row) { return min(max(pl.c0 + pl.cs * (j0 + row), 0), L - 1); };
-        dma_tile<T, G::V_ROWB, BN, (ES == 2 ? 2 : 0)>(vs_w, wave, lane, [&](int row) { return vb + (int64_t)key_row(row) * p.v_sl; });
+        dma_tile<T, G::V_ROWB, BN, 2>(vs_w, wave, lane, [&](int row) { return vb + (int64_t)key_row(row) * p.v_sl; });
         if constexpr (KT) {
             // rows = contraction index, BN consecutive keys per row (dense walk); a chunk that would run past
             // the last key is replaced by the last whole chunk (those positions are never live)
@@ -194,7 +172,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void attn_fwd_kernel(c
                 const int q = wave + 4 * i;
                 const int flat = q * 64 + lane;
                 const int row = flat / K_CPR, pc = flat % K_CPR;
-                const int lc = logical_chunk<G::K_ROWB, (ES == 2 ? 2 : 0)>(row, pc);
+                const int lc = logical_chunk<G::K_ROWB, 2>(row, pc);
                 const int c = min(pl.c0 + j0 + lc * G::EPC, L - G::EPC);
                 dma16(kb + (int64_t)row * p.k_sd + c, ks_w + q * 1024);
             }
@@ -202,7 +180,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void attn_fwd_kernel(c
             dma_tile<T, G::K_ROWB, BN, 1>(ks_w, wave, lane, [&](int row) { return kb + (int64_t)key_row(row) * p.k_sl; });
         }
     };
-    // FAST_DMA state for the segment being fetched: per-lane byte offsets inside a block, wavefront-uniform
+    // State of the fast copies for the segment being fetched: per-lane byte offsets inside a block, wavefront-uniform
     // running pointers to block `wave` of the next tile, and the byte distance between tile positions.
     uint32_t v_lane_off = 0, k_lane_off = 0;
     bool lane_off_fits = true;  // the copy instruction takes a 32-bit per-lane offset: wider ones go the general way
@@ -210,33 +188,31 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void attn_fwd_kernel(c
     const char* k_next = nullptr;
     int64_t v_key = 0, k_key = 0;  // bytes from one tile position to the next (K^T layout: from one d row to the next)
     auto set_lane_offsets = [&](const SegPlan& pl) {
-        if constexpr (FAST_DMA) {
-            const int vr = lane / V_CPR, vpc = lane % V_CPR;
-            // the largest offsets of the segment: the last row of a block, with gathered rows pl.cs keys apart
-            const int64_t v_far = (int64_t)pl.cs * (V_RPI - 1) * p.v_sl * ES + G::V_ROWB;
-            const int64_t k_far = KT ? (int64_t)(K_RPI - 1) * p.k_sd * ES + G::K_ROWB : (int64_t)pl.cs * (K_RPI - 1) * p.k_sl * ES + G::K_ROWB;
-            lane_off_fits = v_far < ((int64_t)1 << 32) && k_far < ((int64_t)1 << 32);
-            v_lane_off = (uint32_t)((int64_t)pl.cs * vr * p.v_sl * ES) + logical_chunk<G::V_ROWB, 2>(vr, vpc) * 16;
-            v_key = (int64_t)p.v_sl * ES * pl.cs;
-            v_next = reinterpret_cast<const char*>(vb) + (int64_t)pl.c0 * p.v_sl * ES + (int64_t)wave * V_RPI * v_key;
-            const int kr = lane / K_CPR, kpc = lane % K_CPR;
-            if constexpr (KT) {
-                k_lane_off = (uint32_t)((int64_t)kr * p.k_sd * ES) + logical_chunk<G::K_ROWB, 2>(kr, kpc) * 16;
-                k_key = (int64_t)p.k_sd * ES;
-                k_next = reinterpret_cast<const char*>(kb) + (int64_t)pl.c0 * ES + (int64_t)wave * K_RPI * k_key;
-            } else {
-                k_lane_off = (uint32_t)((int64_t)pl.cs * kr * p.k_sl * ES) +
-                             logical_chunk<G::K_ROWB, 1>(wave * K_RPI + kr, kpc) * 16;
-                k_key = (int64_t)p.k_sl * ES * pl.cs;
-                k_next = reinterpret_cast<const char*>(kb) + (int64_t)pl.c0 * p.k_sl * ES + (int64_t)wave * K_RPI * k_key;
-            }
+        const int vr = lane / V_CPR, vpc = lane % V_CPR;
+        // the largest offsets of the segment: the last row of a block, with gathered rows pl.cs keys apart
+        const int64_t v_far = (int64_t)pl.cs * (V_RPI - 1) * p.v_sl * ES + G::V_ROWB;
+        const int64_t k_far = KT ? (int64_t)(K_RPI - 1) * p.k_sd * ES + G::K_ROWB : (int64_t)pl.cs * (K_RPI - 1) * p.k_sl * ES + G::K_ROWB;
+        lane_off_fits = v_far < ((int64_t)1 << 32) && k_far < ((int64_t)1 << 32);
+        v_lane_off = (uint32_t)((int64_t)pl.cs * vr * p.v_sl * ES) + logical_chunk<G::V_ROWB, 2>(vr, vpc) * 16;
+        v_key = (int64_t)p.v_sl * ES * pl.cs;
+        v_next = reinterpret_cast<const char*>(vb) + (int64_t)pl.c0 * p.v_sl * ES + (int64_t)wave * V_RPI * v_key;
+        const int kr = lane / K_CPR, kpc = lane % K_CPR;
+        if constexpr (KT) {
+            k_lane_off = (uint32_t)((int64_t)kr * p.k_sd * ES) + logical_chunk<G::K_ROWB, 2>(kr, kpc) * 16;
+            k_key = (int64_t)p.k_sd * ES;
+            k_next = reinterpret_cast<const char*>(kb) + (int64_t)pl.c0 * ES + (int64_t)wave * K_RPI * k_key;
+        } else {
+            k_lane_off = (uint32_t)((int64_t)pl.cs * kr * p.k_sl * ES) +
+                         logical_chunk<G::K_ROWB, 1>(wave * K_RPI + kr, kpc) * 16;
+            k_key = (int64_t)p.k_sl * ES * pl.cs;
+            k_next = reinterpret_cast<const char*>(kb) + (int64_t)pl.c0 * p.k_sl * ES + (int64_t)wave * K_RPI * k_key;
         }
     };
     // whether every key of the tile exists, so that the running pointers can be used as they are
     auto tile_is_fast = [&](const SegPlan& pl, int tile) {
         const int j0 = tile * BN;
         const int key_first = pl.c0 + pl.cs * j0, key_last = pl.c0 + pl.cs * (j0 + BN - 1);
-        bool fast = FAST_DMA && lane_off_fits && key_last < L;
+        bool fast = lane_off_fits && key_last < L;
         if constexpr (KT) fast = fast && (key_first + BN <= L);
         return fast;
     };
@@ -283,24 +259,17 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void attn_fwd_kernel(c
     const int tr_col = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
     uint32_t k_addr[KT ? NT : KS];  // K tile: row-major: (row lm, swizzled chunk of step ks); K^T: (row 8g + tr_row, block nt)
     uint32_t v_addr[DT];            // V tile: (row 4g + tr_row, swizzled 64-byte block dt, column tr_col)
-    if constexpr (ES == 2) {
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-            v_addr[dt] = smem_base + G::K_BYTES + (4 * g + tr_row) * G::V_ROWB +
-                         ((dt ^ swz64<G::V_ROWB>(4 * g + tr_row)) * 64) + tr_col * 2;
-        if constexpr (KT) {
+    for (int dt = 0; dt < DT; ++dt)
+        v_addr[dt] = smem_base + G::K_BYTES + (4 * g + tr_row) * G::V_ROWB +
+                     ((dt ^ swz64<G::V_ROWB>(4 * g + tr_row)) * 64) + tr_col * 2;
+    if constexpr (KT) {
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-                k_addr[nt] = smem_base + (8 * g + tr_row) * G::K_ROWB + ((nt ^ swz64<G::K_ROWB>(8 * g + tr_row)) * 64) + tr_col * 2;
-        } else {
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) k_addr[ks] = smem_base + lds_off<G::K_ROWB, true>(lm, (16 * ks + 8 * g) * ES);
-        }
+        for (int nt = 0; nt < NT; ++nt)
+            k_addr[nt] = smem_base + (8 * g + tr_row) * G::K_ROWB + ((nt ^ swz64<G::K_ROWB>(8 * g + tr_row)) * 64) + tr_col * 2;
     } else {
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) v_addr[dt] = smem_base + G::K_BYTES + (32 * dt + lm) * 4;
-#pragma unroll
-        for (int i = 0; i < (KT ? NT : KS); ++i) k_addr[i] = smem_base;
+        for (int ks = 0; ks < KS; ++ks) k_addr[ks] = smem_base + lds_off<G::K_ROWB, true>(lm, (16 * ks + 8 * g) * ES);
     }
 
     // Two ways to take a tile's exponentials.  The careful one tracks the row maxima and moves the reference (with a
@@ -435,28 +404,17 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void attn_fwd_kernel(c
                 Frag<T> kfr[NT][KS];
                 auto load_k = [&](int nt, int ks) {
                     Frag<T> kf;
-                    if constexpr (ES == 2) {
-                        if constexpr (KT) {
-                            // rows 16ks + 8g + {0..3} and +4: multiples of 4 rows leave the lane's swizzle term alone
-                            const uint32_t a0 = k_addr[nt] + 16 * ks * G::K_ROWB;
-                            kf = frag_from_tr<T>(lds_load_tr16(a0), lds_load_tr16(a0 + 4 * G::K_ROWB));
-                        } else {
-                            kf.v = __builtin_bit_cast(typename Frag<T>::vec, lds_load128(k_addr[ks] + 32 * nt * G::K_ROWB));
-                        }
+                    if constexpr (KT) {
+                        // rows 16ks + 8g + {0..3} and +4: multiples of 4 rows leave the lane's swizzle term alone
+                        const uint32_t a0 = k_addr[nt] + 16 * ks * G::K_ROWB;
+                        kf = frag_from_tr<T>(lds_load_tr16(a0), lds_load_tr16(a0 + 4 * G::K_ROWB));
                     } else {
-                        const char* ks_l = smem + stage_it * G::STAGE;
-                        if constexpr (KT) {
-#pragma unroll
-                            for (int e = 0; e < 8; ++e)
-                                kf.v[e] = *reinterpret_cast<const float*>(ks_l + (16 * ks + 8 * g + e) * G::K_ROWB + (32 * nt + lm) * 4);
-                        } else {
-                            kf = lds_frag_row_swz<T, G::K_ROWB>(ks_l, 32 * nt + lm, 16 * ks + 8 * g);
-                        }
+                        kf.v = __builtin_bit_cast(typename Frag<T>::vec, lds_load128(k_addr[ks] + 32 * nt * G::K_ROWB));
                     }
                     return kf;
                 };
                 constexpr int NMMA = NT * KS;
-                constexpr int K_AHEAD = (ES != 2) ? NMMA : ((KT ? 6 : 12) < NMMA ? (KT ? 6 : 12) : NMMA);  // fragments
+                constexpr int K_AHEAD = (KT ? 6 : 12) < NMMA ? (KT ? 6 : 12) : NMMA;  // fragments
 #pragma unroll
                 for (int i = 0; i < K_AHEAD; ++i) kfr[i / KS][i % KS] = load_k(i / KS, i % KS);
                 __builtin_amdgcn_sched_barrier(0);  // keep the requests above the matrix work
@@ -470,14 +428,12 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void attn_fwd_kernel(c
                         kfr[(i + K_AHEAD) / KS][(i + K_AHEAD) % KS] = load_k((i + K_AHEAD) / KS, (i + K_AHEAD) % KS);
                         __builtin_amdgcn_sched_barrier(0);
                     }
-                    if constexpr (FAST_DMA) {
-                        if ((i + 1) % MMA_PER_DMA == 0 && (i + 1) / MMA_PER_DMA <= NDMA) {
-                            if (spread) issue_step((i + 1) / MMA_PER_DMA - 1, stage_pf);
-                            __builtin_amdgcn_sched_barrier(0);
-                        }
+                    if ((i + 1) % MMA_PER_DMA == 0 && (i + 1) / MMA_PER_DMA <= NDMA) {
+                        if (spread) issue_step((i + 1) / MMA_PER_DMA - 1, stage_pf);
+                        __builtin_amdgcn_sched_barrier(0);
                     }
                 }
-                if constexpr (FAST_DMA && (NMMA / MMA_PER_DMA < NDMA)) {
+                if constexpr (NMMA / MMA_PER_DMA < NDMA) {
                     if (spread) {
 #pragma unroll
                         for (int s = NMMA / MMA_PER_DMA; s < NDMA; ++s) issue_step(s, stage_pf);
@@ -495,17 +451,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void attn_fwd_kernel(c
                 // V fragments are requested one 16-key step (DT fragments) ahead of the MFMAs that consume them.
                 auto load_v = [&](int nt, int t, int dt) {
                     Frag<T> vf;
-                    if constexpr (ES == 2) {
-                        const uint32_t a0 = v_addr[dt] + (32 * nt + 16 * t) * G::V_ROWB;
-                        vf = frag_from_tr<T>(lds_load_tr16(a0), lds_load_tr16(a0 + 8 * G::V_ROWB));
-                    } else {
-                        const int rbase = 32 * nt + 16 * t + 4 * g;
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            vf.v[e] = lds_load_f32(v_addr[dt] + (rbase + e) * G::V_ROWB);
-                            vf.v[4 + e] = lds_load_f32(v_addr[dt] + (rbase + 8 + e) * G::V_ROWB);
-                        }
-                    }
+                    const uint32_t a0 = v_addr[dt] + (32 * nt + 16 * t) * G::V_ROWB;
+                    vf = frag_from_tr<T>(lds_load_tr16(a0), lds_load_tr16(a0 + 8 * G::V_ROWB));
                     return vf;
                 };
                 Frag<T> vfr[2][DT];
@@ -709,7 +656,7 @@ static int attention_fwd_common(const char* who, const void* q, int64_t q_sb, in
     }
     hipStream_t st = (hipStream_t)stream;
     switch (dtype) {
-        case SPLAT_F32: return dispatch_attn<float>(p, d, kt, st);
+        case SPLAT_F32: return launch_attn_f32(p, d, kt, st);
         case SPLAT_F16: return dispatch_attn<f16>(p, d, kt, st);
         default: return dispatch_attn<bf16>(p, d, kt, st);
     }

@@ -6,6 +6,31 @@ namespace splat {
 
 constexpr float kNegBigA = -1.0e30f;
 
+struct AttnParams {
+    const void* q;
+    const void* k;
+    const void* v;
+    void* o;
+    int64_t q_sb, q_sh, q_sl;
+    int64_t k_sb, k_sh, k_sd, k_sl;
+    int64_t v_sb, v_sh, v_sl;
+    int64_t o_sb, o_sh, o_sl;
+    int B, H, L;
+    float scale_log2e;
+    int n_seg;
+    SegPtrs seg[SPLAT_MAX_SEGMENTS];
+    int n_row_blocks;
+    int total;
+    int row_stride;
+    const PlanRec* plan;  // plan table of this mask (PLANNED kernels), variant already selected
+    float* lse;           // optional [B*H, L]: log of every row's sum of exponentials (natural log, scaled scores)
+};
+
+constexpr float kRescaleThreshold = 8.0f;  // in log2 units: exponentials stay below 2^8 before the reference moves
+
+// the float32 forward (attention_f32.hip); p.n_row_blocks and p.total are filled in by the launch
+int launch_attn_f32(const AttnParams& p, int d, bool kt, hipStream_t st);
+
 // Live positions of one row in the tile that starts at position j0, one bit per position (bit b = position j0 + b):
 // the row's span [lo, lo + cnt) intersected with its periodic pattern.  `first` is the smallest offset >= 0 in the tile
 // whose position is congruent to the row's first one modulo its step (0 for unit step) and `pat` has a bit at every
