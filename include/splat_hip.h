@@ -36,7 +36,7 @@
 extern "C" {
 #endif
 
-#define SPLAT_VERSION 1000 /* major*10000 + minor*100 + patch; 0.2.0 added the planned forward, 0.3.0 splat_spmm_t, 0.4.0 splat_attention_fwd_stats, splat_sddmm_probs, 0.5.0 splat_attention_fwd_noalloc, 0.6.0 moved the two measurement aids out (libsplat_bench.so, splat_bench.h), 0.7.0 added splat_sddmm_planned, splat_spmm_planned, 0.8.0 splat_spmm_t_planned, 0.9.0 splat_attention_bwd_keys, 0.10.0 splat_acsr_build_record */
+#define SPLAT_VERSION 1000 /* major*10000 + minor*100 + patch; 0.2.0 added the planned forward, 0.3.0 splat_spmm_t, 0.4.0 splat_attention_fwd_stats, splat_sddmm_probs, 0.5.0 splat_attention_fwd_noalloc, 0.6.0 moved the two measurement aids out (libsplat_bench.so, splat_bench.h), 0.7.0 added splat_sddmm_planned, splat_spmm_planned, 0.8.0 splat_spmm_t_planned, 0.9.0 splat_attention_bwd_keys, 0.10.0 splat_acsr_build_record, splat_attention_bwd_f32, splat_attention_bwd_keys_f32 */
 
 /* element types of q/k/v/score/output buffers */
 #define SPLAT_F32 0
@@ -333,6 +333,15 @@ int splat_attention_bwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl,
                         int64_t plan_t_bytes, int32_t B, int32_t H, int32_t L, int32_t d, float scale, int32_t dtype,
                         void* stream);
 
+/* The same in float32, in two launches (dq; dk and dv together), with the arithmetic of the float32 forward. */
+int splat_attention_bwd_f32(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* k, int64_t k_sb,
+                        int64_t k_sh, int64_t k_sl, const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sl,
+                        const void* out, int64_t o_sb, int64_t o_sh, int64_t o_sl, const void* dout, int64_t g_sb,
+                        int64_t g_sh, int64_t g_sl, const float* lse, float* delta, void* dq, void* dk, void* dv,
+                        const splat_acsr_seg* segs /* host */, int32_t n_seg, const void* plan, int64_t plan_bytes,
+                        const splat_acsr_seg* segs_t /* host */, int32_t n_seg_t, const void* plan_t,
+                        int64_t plan_t_bytes, int32_t B, int32_t H, int32_t L, int32_t d, float scale, void* stream);
+
 /* The keys' side of that pass for a list of rows of the transposed mask (no counterpart in the reference, which is forward
  * only: r_attention.py:77-100).  For transposed masks that keep a few keys with very long columns (a strided pattern's far
  * field: one key in 128 with up to L queries), whose walk by 128 consecutive keys runs almost empty tiles: the caller
@@ -353,6 +362,15 @@ int splat_attention_bwd_keys(const void* q, int64_t q_sb, int64_t q_sh, int64_t 
                              const splat_acsr_seg* segs_t /* host */, int32_t n_seg_t, const void* plan_t,
                              int64_t plan_t_bytes, int32_t B, int32_t H, int32_t L, int32_t n_rows, int32_t d, float scale,
                              int32_t dtype, void* dk, void* dv, int32_t rows_per_stretch, void* stream);
+
+/* The same in float32. */
+int splat_attention_bwd_keys_f32(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* k, int64_t k_sb,
+                             int64_t k_sh, int64_t k_sl, const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sl,
+                             const void* dout, int64_t g_sb, int64_t g_sh, int64_t g_sl, const float* lse,
+                             const float* delta, const int32_t* key_of_row, void* dk_rows, void* dv_rows,
+                             const splat_acsr_seg* segs_t /* host */, int32_t n_seg_t, const void* plan_t,
+                             int64_t plan_t_bytes, int32_t B, int32_t H, int32_t L, int32_t n_rows, int32_t d, float scale,
+                             void* dk, void* dv, int32_t rows_per_stretch, void* stream);
 
 #ifdef __cplusplus
 }

@@ -46,3 +46,18 @@ def test_forward_and_gradients_against_float64(dev, name, L, d):
     for a, b in zip(torch.autograd.grad(out, on, go.to(dev)), grads):
         b = torch.nan_to_num(b)
         assert float((a.cpu() - b).abs().max()) <= 2e-5 * max(1.0, float(b.abs().max()))
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_listed_rows_of_the_transposed_mask(dev, d):
+    """The keys of a strided far field row by row (rows cut into stretches of queries, their shares added up) against the walk
+    by blocks of keys."""
+    B, H, L = 1, 2, 1500
+    attn = RegularAttention(B, L, H, d, A.strided_patterns(L, 64, 50), 16, 16, dev, torch.float32, scale=d ** -0.5)
+    g = torch.Generator(device=dev).manual_seed(d)
+    q, k, v, go = (torch.randn(B, H, L, d, generator=g, device=dev) for _ in range(4))
+    x = [q, k.transpose(2, 3), v]
+    one = attn.backward_pass(x, go, sparse_rows=False)
+    two = attn.backward_pass(x, go, sparse_rows=True)
+    for a, b in zip(one, two):
+        assert float((a - b).abs().max()) <= 2e-5 * float(b.abs().max())

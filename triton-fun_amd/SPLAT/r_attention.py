@@ -253,18 +253,18 @@ class RegularAttention(nn.Module):
         """Gradients (dq, dk, dv), each [B, H, L, d], of ``forward(x)`` for x = [q, kT, v] and the upstream gradient
         ``grad_out`` [B, H, L, d].  The ACSR of the transposed mask is built on first use; see ``r_backward``.  ``lse``
         and ``out``: the rows' statistic and the output of ``forward_with_stats`` for the same x.  Where the fused
-        forward applies (16-bit dtype, d in {64, 128}) the gradients come from the fused backward kernel, which needs both
+        forward applies (one dtype, d in {64, 128}) the gradients come from the fused backward kernel, which needs both
         (a forward is run here when one is missing); otherwise, or with ``fused=False``, from the operators composed over
         compressed matrices, which ``lse`` spares the softmax pass.  ``sparse_rows``: how the fused kernel takes segments
         of the transposed mask that keep few keys with long columns (``r_backward.attention_backward_fused``)."""
         from r_backward import attention_backward, attention_backward_fused
         q, kT, v = x
         self._ensure_transposed()
-        fusable = (self.fused and q.shape[-1] in (64, 128) and q.dtype in (torch.float16, torch.bfloat16) and
+        fusable = (self.fused and q.shape[-1] in (64, 128) and
                    q.dtype == kT.dtype == v.dtype == grad_out.dtype == self._out_dtype)
         if fused is None:
             fused = fusable
-        elif fused and not fusable:
+        elif fused and not (fusable and q.dtype in (torch.float16, torch.bfloat16)):
             raise _hip.SplatError("the fused backward needs a 16-bit dtype shared by all tensors and d in {64, 128}")
         if not fused:
             return attention_backward(q, kT, v, grad_out, self.segments, self._segments_t, self.scale, lse)
@@ -285,7 +285,7 @@ class RegularAttention(nn.Module):
 
     def _grad_state(self):
         """What the native differentiable path (csrc/host_ext.cpp) keeps for this module: the mask and the transposed mask
-        with their plans and the row-sparse segments' schedule.  None where it does not apply (float32, other head
+        with their plans and the row-sparse segments' schedule.  None where it does not apply (other head
         dimensions, ``fused=False``, a mask without a transposed ACSR, a first call under stream capture)."""
         if self._native_grad is None:
             from r_backward import keys_side_schedule
@@ -293,7 +293,7 @@ class RegularAttention(nn.Module):
             if torch.cuda.is_current_stream_capturing():
                 return None
             self._native_grad = False
-            if d in (64, 128) and self._out_dtype in (torch.float16, torch.bfloat16):
+            if d in (64, 128):
                 try:
                     self._ensure_transposed()
                 except _hip.SplatError:

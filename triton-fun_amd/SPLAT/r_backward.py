@@ -311,14 +311,16 @@ def attention_backward_fused(q: torch.Tensor, kT: torch.Tensor, v: torch.Tensor,
     """(dq, dk, dv) as ``attention_backward`` gives them, from three launches of one kernel and without a compressed
     matrix: ``out`` and ``lse`` are the output and the row statistic of the fused forward for the same inputs
     (``RegularAttention.forward_with_stats``), ``plan`` / ``plan_t`` the fused kernel's plans (``attention_plan``) of the
-    mask's segments and of the transposed mask's.  16-bit dtypes, d in {64, 128}; operands whose rows are not contiguous
+    mask's segments and of the transposed mask's.  One dtype, d in {64, 128}; operands whose rows are not contiguous
     16-byte pieces (K^T-contiguous keys among them) are copied first.  Segments of the transposed mask that keep few keys
     with long columns are taken row by row (``keys_side_schedule``; ``plan_t`` then goes unused) where that pays (``sparse_rows`` None), wherever
     there are such segments (True) or never (False)."""
     B, H, L, d = q.shape
     dt, dev = q.dtype, q.device
-    if dt not in (torch.float16, torch.bfloat16) or d not in (64, 128):
-        raise _hip.SplatError("the fused backward takes fp16 / bf16 tensors with d in {64, 128}")
+    if d not in (64, 128):
+        raise _hip.SplatError("the fused backward takes tensors with d in {64, 128}")
+    code = _hip.dtype_code(dt)
+    epc, f32 = 16 // q.element_size(), code == _hip.SPLAT_F32
     # K^T with the keys contiguous (the reference's layout): one streaming transpose instead of a strided copy
     k = transpose_keys(kT) if (kT.dim() == 4 and kT.stride(3) == 1 and kT.stride(2) != 1) else kT.transpose(2, 3)
 
@@ -326,7 +328,7 @@ def attention_backward_fused(q: torch.Tensor, kT: torch.Tensor, v: torch.Tensor,
         _hip.require_device_tensor(t, name)
         if t.dtype != dt or tuple(t.shape) != (B, H, L, d):
             raise _hip.SplatError(f"{name} must be a {dt} tensor of shape {(B, H, L, d)}, got {t.dtype} {tuple(t.shape)}")
-        if t.stride(3) != 1 or t.data_ptr() % 16 != 0 or any(t.stride(i) % 8 != 0 for i in (0, 1, 2)):
+        if t.stride(3) != 1 or t.data_ptr() % 16 != 0 or any(t.stride(i) % epc != 0 for i in (0, 1, 2)):
             t = t.contiguous()
         return t
     q, k, v, out, grad_out = rows(q, "q"), rows(k, "k"), rows(v, "v"), rows(out, "out"), rows(grad_out, "grad_out")
@@ -351,9 +353,10 @@ def attention_backward_fused(q: torch.Tensor, kT: torch.Tensor, v: torch.Tensor,
     args += [lse.data_ptr(), delta.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
              arr, len(segments), plan.data_ptr(), plan.numel() * plan.element_size(),
              arr_t, len(segments_t), plan_t.data_ptr(), plan_t.numel() * plan_t.element_size(),
-             B, H, L, d, float(scale), _hip.dtype_code(dt)]
+             B, H, L, d, float(scale)]
     with torch.cuda.device(dev):
-        rc = _hip.lib().splat_attention_bwd(*args, _hip.stream_ptr(dev))
+        rc = _hip.lib().splat_attention_bwd_f32(*args, _hip.stream_ptr(dev)) if f32 else \
+            _hip.lib().splat_attention_bwd(*args, code, _hip.stream_ptr(dev))
         _hip.check(rc, "splat_attention_bwd")
         if sched is not None:
             R = sched.n_rows
@@ -363,7 +366,9 @@ def attention_backward_fused(q: torch.Tensor, kT: torch.Tensor, v: torch.Tensor,
             # (the call's second kernel adds a key's shares, one per stretch, onto what the other segments gave it)
             args += [lse.data_ptr(), delta.data_ptr(), sched.key_of_row.data_ptr(), part[0].data_ptr(), part[1].data_ptr(),
                      sched.rows.seg_array(R), 1, plan_r.data_ptr(), plan_r.numel() * plan_r.element_size(),
-                     B, H, L, R, d, float(scale), _hip.dtype_code(dt), dk.data_ptr(), dv.data_ptr(), sched.per_stretch]
-            rc = _hip.lib().splat_attention_bwd_keys(*args, _hip.stream_ptr(dev))
+                     B, H, L, R, d, float(scale)]
+            to = [dk.data_ptr(), dv.data_ptr(), sched.per_stretch, _hip.stream_ptr(dev)]
+            rc = _hip.lib().splat_attention_bwd_keys_f32(*args, *to) if f32 else \
+                _hip.lib().splat_attention_bwd_keys(*args, code, *to)
             _hip.check(rc, "splat_attention_bwd_keys")
     return dq, dk, dv

@@ -22,34 +22,11 @@
 // contiguous.
 #include <initializer_list>
 
-#include "attn_tile.hpp"
+#include "attn_bwd.hpp"
 
 namespace splat {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-enum { kBwdDQ = 0, kBwdDK = 1, kBwdDV = 2, kBwdDKV = 3 };
-
-struct BwdParams {
-    const void* a;  // register operand A, one row per lane: Q (dQ), K (dK, dV)
-    const void* b;  // register operand B: dO (dQ), V (dK); unused (dV)
-    const void* x;  // tile operand X: K (dQ), Q (dK, dV)
-    const void* y;  // tile operand Y: V (dQ), dO (dK, dV)
-    void* out;      // dQ, dK, dV
-    void* out2;     // dK + dV in one launch: dV (same strides as out)
-    int64_t a_sb, a_sh, a_sl, b_sb, b_sh, b_sl, x_sb, x_sh, x_sl, y_sb, y_sh, y_sl, o_sb, o_sh, o_sl;
-    const float* lse;    // [B*H, L], natural log, per query
-    const float* delta;  // [B*H, L], D per query (dK, dV: written by the dQ launch before them on the stream)
-    const void* o;       // dQ only: the forward's output, from which that launch computes D = rowsum(dO * O) ...
-    int64_t oo_sb, oo_sh, oo_sl;
-    float* delta_w;      // ... and where it stores it
-    int B, H, L;
-    int Lr;               // rows of the launch: L, or the number of rows of a rectangular keys' side (dK, dV of selected keys)
-    const int* row_map;   // [Lr] or null: the row of A / B that row r of the mask stands for (r itself when null)
-    float scale, scale_log2e;
-    int n_seg, n_row_blocks, total, row_stride;
-    const PlanRec* plan;  // plan table of the mask (dQ) or of its transpose (dK, dV), first variant
-};
 
 template <typename T, int D, int MODE>
 __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(const BwdParams p) {
@@ -667,18 +644,20 @@ struct Rows3 {
 };
 
 // Checks shared by the two entry points; `who` names the caller in messages.
-static int check_bwd_common(const char* who, int B, int H, int L, int d, float scale, int dtype, std::initializer_list<Rows3> rows,
+static int check_bwd_common(const char* who, bool f32, int B, int H, int L, int d, float scale, int dtype, std::initializer_list<Rows3> rows,
                             std::initializer_list<const void*> aligned16) {
     if (B <= 0 || H <= 0 || L <= 0) return fail(SPLAT_E_SHAPE, "%s: need B, H, L > 0 (got %d, %d, %d)", who, B, H, L);
     if (L > (1 << 23)) return fail(SPLAT_E_SHAPE, "%s: L is limited to 2^23 (got %d)", who, L);
     if (d != 64 && d != 128) return fail(SPLAT_E_UNSUPPORTED, "%s: head dim must be 64 or 128 (got %d)", who, d);
-    if (dtype != SPLAT_F16 && dtype != SPLAT_BF16) return fail(SPLAT_E_UNSUPPORTED, "%s: 16-bit element types only (got dtype %d)", who, dtype);
+    if (!f32 && dtype != SPLAT_F16 && dtype != SPLAT_BF16)
+        return fail(SPLAT_E_UNSUPPORTED, "%s: 16-bit element types only (got dtype %d)", who, dtype);
+    const int epc = f32 ? 4 : 8;
     if (!(scale > 0.f)) return fail(SPLAT_E_UNSUPPORTED, "%s: scale must be > 0 (got %g)", who, (double)scale);
     auto mis = [&](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) != 0; };
     for (const Rows3& r : rows) {
         if (mis(r.ptr)) return fail(SPLAT_E_ALIGN, "%s: every tensor of rows must be 16-byte aligned", who);
-        if ((r.sb % 8) != 0 || (r.sh % 8) != 0 || (r.sl % 8) != 0)
-            return fail(SPLAT_E_ALIGN, "%s: every batch/head/row stride must be a multiple of 8 elements (16 bytes)", who);
+        if ((r.sb % epc) != 0 || (r.sh % epc) != 0 || (r.sl % epc) != 0)
+            return fail(SPLAT_E_ALIGN, "%s: every batch/head/row stride must be a multiple of %d elements (16 bytes)", who, epc);
         if (r.sl < d) return fail(SPLAT_E_SHAPE, "%s: row strides must be >= d", who);
     }
     for (const void* ptr : aligned16)
@@ -716,18 +695,17 @@ static BwdParams bwd_keys_params(const BwdParams& base, Rows3 q, Rows3 k, Rows3 
 
 using namespace splat;
 
-extern "C" int splat_attention_bwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* k, int64_t k_sb,
+static int bwd_impl(const char* who, bool f32, const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* k, int64_t k_sb,
                                    int64_t k_sh, int64_t k_sl, const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sl,
                                    const void* out, int64_t o_sb, int64_t o_sh, int64_t o_sl, const void* dout, int64_t g_sb,
                                    int64_t g_sh, int64_t g_sl, const float* lse, float* delta, void* dq, void* dk, void* dv,
                                    const splat_acsr_seg* segs, int32_t n_seg, const void* plan, int64_t plan_bytes,
                                    const splat_acsr_seg* segs_t, int32_t n_seg_t, const void* plan_t, int64_t plan_t_bytes,
                                    int32_t B, int32_t H, int32_t L, int32_t d, float scale, int32_t dtype, void* stream) {
-    const char* who = "splat_attention_bwd";
     if (!q || !k || !v || !out || !dout || !lse || !delta || !dq || !dk || !dv || !segs || !segs_t || !plan || !plan_t)
         return fail(SPLAT_E_NULL, "%s: null pointer argument", who);
     const Rows3 rq{q, q_sb, q_sh, q_sl}, rk{k, k_sb, k_sh, k_sl}, rv{v, v_sb, v_sh, v_sl}, ro{out, o_sb, o_sh, o_sl}, rg{dout, g_sb, g_sh, g_sl};
-    if (int rc = check_bwd_common(who, B, H, L, d, scale, dtype, {rq, rk, rv, ro, rg}, {dq, dk, dv, plan, plan_t})) return rc;
+    if (int rc = check_bwd_common(who, f32, B, H, L, d, scale, dtype, {rq, rk, rv, ro, rg}, {dq, dk, dv, plan, plan_t})) return rc;
     if ((reinterpret_cast<uintptr_t>(lse) & 3) != 0 || (reinterpret_cast<uintptr_t>(delta) & 3) != 0)
         return fail(SPLAT_E_ALIGN, "%s: lse and delta must be 4-byte aligned", who);
     SegPtrs tmp[SPLAT_MAX_SEGMENTS];
@@ -755,24 +733,30 @@ extern "C" int splat_attention_bwd(const void* q, int64_t q_sb, int64_t q_sh, in
     pq.o = out; pq.oo_sb = o_sb; pq.oo_sh = o_sh; pq.oo_sl = o_sl; pq.delta_w = delta;  // D = rowsum(dO * O): computed and stored by this launch
     // dK, dV: rows = keys, the transposed mask's plan
     const BwdParams pk = bwd_keys_params(base, rq, rk, rv, rg, dk, segs_t, n_seg_t, plan_t, L, nullptr, d);
+    if (f32) {
+        BwdParams pkv = pk;
+        pkv.out2 = dv;
+        if (int rc = launch_bwd_dq_f32(pq, d, st)) return rc;
+        return launch_bwd_dkv_f32(pkv, d, st);
+    }
     BwdParams pv = pk;
     pv.b = nullptr;
     pv.out = dv;
     return dtype == SPLAT_F16 ? run_bwd<f16>(pq, pk, pv, d, st) : run_bwd<bf16>(pq, pk, pv, d, st);
 }
 
-extern "C" int splat_attention_bwd_keys(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* k, int64_t k_sb,
+
+static int bwd_keys_impl(const char* who, bool f32, const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* k, int64_t k_sb,
                                         int64_t k_sh, int64_t k_sl, const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sl,
                                         const void* dout, int64_t g_sb, int64_t g_sh, int64_t g_sl, const float* lse,
                                         const float* delta, const int32_t* key_of_row, void* dk_rows, void* dv_rows,
                                         const splat_acsr_seg* segs_t, int32_t n_seg_t, const void* plan_t, int64_t plan_t_bytes,
                                         int32_t B, int32_t H, int32_t L, int32_t n_rows, int32_t d, float scale, int32_t dtype,
                                         void* dk, void* dv, int32_t rows_per_stretch, void* stream) {
-    const char* who = "splat_attention_bwd_keys";
     if (!q || !k || !v || !dout || !lse || !delta || !key_of_row || !dk_rows || !dv_rows || !segs_t || !plan_t)
         return fail(SPLAT_E_NULL, "%s: null pointer argument", who);
     const Rows3 rq{q, q_sb, q_sh, q_sl}, rk{k, k_sb, k_sh, k_sl}, rv{v, v_sb, v_sh, v_sl}, rg{dout, g_sb, g_sh, g_sl};
-    if (int rc = check_bwd_common(who, B, H, L, d, scale, dtype, {rq, rk, rv, rg}, {dk_rows, dv_rows, plan_t})) return rc;
+    if (int rc = check_bwd_common(who, f32, B, H, L, d, scale, dtype, {rq, rk, rv, rg}, {dk_rows, dv_rows, plan_t})) return rc;
     if (n_rows <= 0 || n_rows > (1 << 23)) return fail(SPLAT_E_SHAPE, "%s: need 0 < n_rows <= 2^23 (got %d)", who, n_rows);
     if ((dk == nullptr) != (dv == nullptr)) return fail(SPLAT_E_NULL, "%s: dk and dv go together (both or neither)", who);
     if (dk) {
@@ -793,12 +777,66 @@ extern "C" int splat_attention_bwd_keys(const void* q, int64_t q_sb, int64_t q_s
         return fail(SPLAT_E_SHAPE, "%s: too many row blocks", who);
     const BwdParams base = bwd_base(lse, delta, B, H, L, scale);
     const BwdParams pk = bwd_keys_params(base, rq, rk, rv, rg, dk_rows, segs_t, n_seg_t, plan_t, n_rows, key_of_row, d);
+    hipStream_t st = (hipStream_t)stream;
+    if (f32) {
+        BwdParams pkv = pk;
+        pkv.out2 = dv_rows;
+        if (int rc = launch_bwd_dkv_f32(pkv, d, st)) return rc;
+        return dk ? launch_rows_add<float>(dk_rows, dv_rows, dk, dv, key_of_row, B, H, L, n_rows, rows_per_stretch, d, st) : 0;
+    }
     BwdParams pv = pk;
     pv.b = nullptr;
     pv.out = dv_rows;
-    hipStream_t st = (hipStream_t)stream;
     if (int rc = dtype == SPLAT_F16 ? run_bwd_keys<f16>(pk, pv, d, st) : run_bwd_keys<bf16>(pk, pv, d, st)) return rc;
     if (!dk) return 0;
     return dtype == SPLAT_F16 ? launch_rows_add<f16>(dk_rows, dv_rows, dk, dv, key_of_row, B, H, L, n_rows, rows_per_stretch, d, st)
                               : launch_rows_add<bf16>(dk_rows, dv_rows, dk, dv, key_of_row, B, H, L, n_rows, rows_per_stretch, d, st);
+}
+
+extern "C" int splat_attention_bwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* k, int64_t k_sb,
+                                   int64_t k_sh, int64_t k_sl, const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sl,
+                                   const void* out, int64_t o_sb, int64_t o_sh, int64_t o_sl, const void* dout, int64_t g_sb,
+                                   int64_t g_sh, int64_t g_sl, const float* lse, float* delta, void* dq, void* dk, void* dv,
+                                   const splat_acsr_seg* segs, int32_t n_seg, const void* plan, int64_t plan_bytes,
+                                   const splat_acsr_seg* segs_t, int32_t n_seg_t, const void* plan_t, int64_t plan_t_bytes,
+                                   int32_t B, int32_t H, int32_t L, int32_t d, float scale, int32_t dtype, void* stream) {
+    return bwd_impl("splat_attention_bwd", false, q, q_sb, q_sh, q_sl, k, k_sb, k_sh, k_sl, v, v_sb, v_sh, v_sl, out, o_sb, o_sh, o_sl,
+        dout, g_sb, g_sh, g_sl, lse, delta, dq, dk, dv, segs, n_seg, plan, plan_bytes, segs_t, n_seg_t, plan_t, plan_t_bytes, B, H, L,
+        d, scale, dtype, stream);
+}
+
+extern "C" int splat_attention_bwd_f32(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* k, int64_t k_sb,
+                                   int64_t k_sh, int64_t k_sl, const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sl,
+                                   const void* out, int64_t o_sb, int64_t o_sh, int64_t o_sl, const void* dout, int64_t g_sb,
+                                   int64_t g_sh, int64_t g_sl, const float* lse, float* delta, void* dq, void* dk, void* dv,
+                                   const splat_acsr_seg* segs, int32_t n_seg, const void* plan, int64_t plan_bytes,
+                                   const splat_acsr_seg* segs_t, int32_t n_seg_t, const void* plan_t, int64_t plan_t_bytes,
+                                   int32_t B, int32_t H, int32_t L, int32_t d, float scale, void* stream) {
+    return bwd_impl("splat_attention_bwd_f32", true, q, q_sb, q_sh, q_sl, k, k_sb, k_sh, k_sl, v, v_sb, v_sh, v_sl, out, o_sb, o_sh,
+        o_sl, dout, g_sb, g_sh, g_sl, lse, delta, dq, dk, dv, segs, n_seg, plan, plan_bytes, segs_t, n_seg_t, plan_t, plan_t_bytes, B,
+        H, L, d, scale, SPLAT_F32, stream);
+}
+
+extern "C" int splat_attention_bwd_keys(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* k, int64_t k_sb,
+                                        int64_t k_sh, int64_t k_sl, const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sl,
+                                        const void* dout, int64_t g_sb, int64_t g_sh, int64_t g_sl, const float* lse,
+                                        const float* delta, const int32_t* key_of_row, void* dk_rows, void* dv_rows,
+                                        const splat_acsr_seg* segs_t, int32_t n_seg_t, const void* plan_t, int64_t plan_t_bytes,
+                                        int32_t B, int32_t H, int32_t L, int32_t n_rows, int32_t d, float scale, int32_t dtype,
+                                        void* dk, void* dv, int32_t rows_per_stretch, void* stream) {
+    return bwd_keys_impl("splat_attention_bwd_keys", false, q, q_sb, q_sh, q_sl, k, k_sb, k_sh, k_sl, v, v_sb, v_sh, v_sl, dout, g_sb,
+        g_sh, g_sl, lse, delta, key_of_row, dk_rows, dv_rows, segs_t, n_seg_t, plan_t, plan_t_bytes, B, H, L, n_rows, d, scale, dtype,
+        dk, dv, rows_per_stretch, stream);
+}
+
+extern "C" int splat_attention_bwd_keys_f32(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* k, int64_t k_sb,
+                                        int64_t k_sh, int64_t k_sl, const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sl,
+                                        const void* dout, int64_t g_sb, int64_t g_sh, int64_t g_sl, const float* lse,
+                                        const float* delta, const int32_t* key_of_row, void* dk_rows, void* dv_rows,
+                                        const splat_acsr_seg* segs_t, int32_t n_seg_t, const void* plan_t, int64_t plan_t_bytes,
+                                        int32_t B, int32_t H, int32_t L, int32_t n_rows, int32_t d, float scale, void* dk, void* dv,
+                                   int32_t rows_per_stretch, void* stream) {
+    return bwd_keys_impl("splat_attention_bwd_keys_f32", true, q, q_sb, q_sh, q_sl, k, k_sb, k_sh, k_sl, v, v_sb, v_sh, v_sl, dout,
+        g_sb, g_sh, g_sl, lse, delta, key_of_row, dk_rows, dv_rows, segs_t, n_seg_t, plan_t, plan_t_bytes, B, H, L, n_rows, d, scale,
+        SPLAT_F32, dk, dv, rows_per_stretch, stream);
 }

@@ -19,7 +19,6 @@
 namespace splat {
 
 constexpr int kF32Stages = 2;
-constexpr int f32_tile(int d) { return d == 64 ? 32 : 16; }  // positions per tile
 
 template <int D, bool KT, bool PLANNED>
 __global__ __launch_bounds__(256, 3) void attn_fwd_f32_kernel(const AttnParams p) {
@@ -83,13 +82,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_f32_kernel(const AttnParams p
         WalkF32 w;
         w.seg = sg;
         if constexpr (PLANNED) {
-            const PlanRec r = plan_uniform_load(pt + plan_seg_at(p.n_seg, rb, sg));
-            w.pl.c0 = r.x, w.pl.cs = r.y, w.pl.n_tiles = r.z, w.pl.uniform = r.w;
-            const PlanRec s0 = plan_uniform_load(pt + plan_span_at(n_rb, p.n_seg, rb, sg, 2 * half));
-            const PlanRec s1 = plan_uniform_load(pt + plan_span_at(n_rb, p.n_seg, rb, sg, 2 * half + 1));
-            w.tile = max(min(s0.x, s1.x), 0) / BN;
-            w.end = min((max(max(s0.w, s1.w), 0) + BN - 1) / BN, r.z * (kBN / BN));
-            w.end = max(w.end, w.tile);
+            w = walk_f32<BN>(pt, n_rb, p.n_seg, rb, half, sg);
         } else {
             const SegPlan l = s_plan[sg];
             w.pl.c0 = __builtin_amdgcn_readfirstlane(l.c0);

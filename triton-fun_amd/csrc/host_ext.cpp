@@ -34,6 +34,8 @@ struct Api {
     decltype(&splat_transpose_keys) transpose_keys;
     decltype(&splat_attention_bwd) bwd;
     decltype(&splat_attention_bwd_keys) bwd_keys;
+    decltype(&splat_attention_bwd_f32) bwd_f32;
+    decltype(&splat_attention_bwd_keys_f32) bwd_keys_f32;
     decltype(&splat_sddmm) sddmm;
     decltype(&splat_sddmm_probs) sddmm_probs;
     decltype(&splat_sddmm_planned) sddmm_planned;
@@ -257,21 +259,27 @@ struct Attend : public torch::autograd::Function<Attend> {
         at::Tensor delta = at::empty({B, H, L}, lse.options());
         void* stream = stream_of(q);
         const Mask &m = *st.fwd, &mt = *st.keys;
-        int rc = api.bwd(q.data_ptr(), q.stride(0), q.stride(1), q.stride(2), k.data_ptr(), k.stride(0), k.stride(1), k.stride(2), v.data_ptr(),
-                         v.stride(0), v.stride(1), v.stride(2), out.data_ptr(), out.stride(0), out.stride(1), out.stride(2), g.data_ptr(),
-                         g.stride(0), g.stride(1), g.stride(2), lse.data_ptr<float>(), delta.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(),
-                         dv.data_ptr(), m.segs, m.n_seg, m.plan_ptr(), m.plan_bytes(), mt.segs, mt.n_seg, mt.plan_ptr(), mt.plan_bytes(), B, H,
-                         L, d, scale, code, stream);
+#define SPLAT_ARGS                                                                                                                        \
+    q.data_ptr(), q.stride(0), q.stride(1), q.stride(2), k.data_ptr(), k.stride(0), k.stride(1), k.stride(2), v.data_ptr(), v.stride(0), \
+        v.stride(1), v.stride(2), out.data_ptr(), out.stride(0), out.stride(1), out.stride(2), g.data_ptr(), g.stride(0), g.stride(1),   \
+        g.stride(2), lse.data_ptr<float>(), delta.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), m.segs, m.n_seg,       \
+        m.plan_ptr(), m.plan_bytes(), mt.segs, mt.n_seg, mt.plan_ptr(), mt.plan_bytes(), B, H, L, d, scale
+        int rc = code == SPLAT_F32 ? api.bwd_f32(SPLAT_ARGS, stream) : api.bwd(SPLAT_ARGS, code, stream);
+#undef SPLAT_ARGS
         TORCH_CHECK(rc == 0, failure("splat_attention_bwd", rc));
         if (st.rows) {  // the row-sparse segments of the transposed mask, row by row, onto what the others gave
             const Mask& r = *st.rows;
             at::Tensor part = at::empty({2, B, H, r.rows, d}, contiguous);
             char* half = static_cast<char*>(part.data_ptr()) + part.nbytes() / 2;
-            rc = api.bwd_keys(q.data_ptr(), q.stride(0), q.stride(1), q.stride(2), k.data_ptr(), k.stride(0), k.stride(1), k.stride(2),
-                              v.data_ptr(), v.stride(0), v.stride(1), v.stride(2), g.data_ptr(), g.stride(0), g.stride(1), g.stride(2),
-                              lse.data_ptr<float>(), delta.data_ptr<float>(), st.key_of_row.data_ptr<int32_t>(), part.data_ptr(), half, r.segs,
-                              r.n_seg, r.plan_ptr(), r.plan_bytes(), B, H, L, r.rows, d, scale, code, dk.data_ptr(), dv.data_ptr(),
-                              st.per_stretch, stream);
+#define SPLAT_ARGS                                                                                                                        \
+    q.data_ptr(), q.stride(0), q.stride(1), q.stride(2), k.data_ptr(), k.stride(0), k.stride(1), k.stride(2), v.data_ptr(), v.stride(0), \
+        v.stride(1), v.stride(2), g.data_ptr(), g.stride(0), g.stride(1), g.stride(2), lse.data_ptr<float>(), delta.data_ptr<float>(),   \
+        st.key_of_row.data_ptr<int32_t>(), part.data_ptr(), half, r.segs, r.n_seg, r.plan_ptr(), r.plan_bytes(), B, H, L, r.rows, d, scale
+            if (code == SPLAT_F32)
+                rc = api.bwd_keys_f32(SPLAT_ARGS, dk.data_ptr(), dv.data_ptr(), st.per_stretch, stream);
+            else
+                rc = api.bwd_keys(SPLAT_ARGS, code, dk.data_ptr(), dv.data_ptr(), st.per_stretch, stream);
+#undef SPLAT_ARGS
             TORCH_CHECK(rc == 0, failure("splat_attention_bwd_keys", rc));
         }
         return {dq, dk, dv, at::Tensor(), at::Tensor()};
@@ -536,7 +544,8 @@ PyObject* py_bind(PyObject*, PyObject* args) {
     };
     if (!take("splat_last_error", api.last_error) || !take("splat_attention_fwd_planned", api.fwd_planned) ||
         !take("splat_attention_fwd_stats", api.fwd_stats) || !take("splat_transpose_keys", api.transpose_keys) ||
-        !take("splat_attention_bwd", api.bwd) || !take("splat_attention_bwd_keys", api.bwd_keys) || !take("splat_sddmm", api.sddmm) ||
+        !take("splat_attention_bwd", api.bwd) || !take("splat_attention_bwd_keys", api.bwd_keys) ||
+        !take("splat_attention_bwd_f32", api.bwd_f32) || !take("splat_attention_bwd_keys_f32", api.bwd_keys_f32) || !take("splat_sddmm", api.sddmm) ||
         !take("splat_sddmm_probs", api.sddmm_probs) || !take("splat_sddmm_planned", api.sddmm_planned) ||
         !take("splat_softmax", api.softmax) || !take("splat_spmm", api.spmm) || !take("splat_spmm_planned", api.spmm_planned) || !take("splat_acsr_build_record", api.build_record))
         return nullptr;

@@ -15,6 +15,7 @@
 namespace splat {
 
 constexpr int kF32Rows = 64;  // rows of a workgroup: 4 wavefronts of 16, half a row block of the plan
+constexpr int f32_tile(int d) { return d == 64 ? 32 : 16; }  // positions per tile: 8 KB an operand
 
 __device__ __forceinline__ void mma4(f32x4& acc, float a, float b) { acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc, 0, 0, 0); }
 
@@ -45,6 +46,20 @@ struct WalkF32 {
     int seg, tile, end;
     SegPlan pl;
 };
+
+// Segment sg of row block rb in the plan table, cut down to the tiles that the given half of the block's rows sees
+template <int BN>
+__device__ __forceinline__ WalkF32 walk_f32(const PlanRec* pt, int n_rb, int n_seg, int rb, int half, int sg) {
+    WalkF32 w;
+    w.seg = sg;
+    const PlanRec r = plan_uniform_load(pt + plan_seg_at(n_seg, rb, sg));
+    w.pl.c0 = r.x, w.pl.cs = r.y, w.pl.n_tiles = r.z, w.pl.uniform = r.w;
+    const PlanRec s0 = plan_uniform_load(pt + plan_span_at(n_rb, n_seg, rb, sg, 2 * half));
+    const PlanRec s1 = plan_uniform_load(pt + plan_span_at(n_rb, n_seg, rb, sg, 2 * half + 1));
+    w.tile = max(min(s0.x, s1.x), 0) / BN;
+    w.end = max(min((max(max(s0.w, s1.w), 0) + BN - 1) / BN, r.z * (kBN / BN)), w.tile);
+    return w;
+}
 
 // The window of one row in the walk of the current segment, the periodic part of its live positions, and the extent of the
 // wavefront's 16 rows: subtiles before lo_min / from hi_max on hold nothing for it, from lo_max to hi_min they need no mask.
