@@ -559,6 +559,11 @@ static int launch_attn(const AttnParams& p0, hipStream_t st) {
 // kernel also supports 32-key tiles in a ring of 4 stages; it measured slower at d = 128 and equal at d = 64).
 template <typename T>
 static int dispatch_attn(const AttnParams& p, int d, bool kt, hipStream_t st) {
+    // few row blocks: the kernel of 16 rows a wavefront (attention_rows16.hip).  Its workgroups, two per row block, take 32 KB
+    // (d = 64) or 64 KB of LDS; the line lies where it stops being faster over windows of 32 to 512: three workgroups a CU at
+    // d = 64 (384 row blocks: 9.5 -> 8.6, 10.8 -> 10.1, 17.8 -> 17.5 us; 448: 9.5 -> 9.9, 17.8 -> 20.4), one and a half at d = 128
+    // (192: 9.8 -> 8.6, 10.9 -> 10.1, 18.0 -> 18.7 us; 320: 12.0 -> 13.9)
+    if ((int64_t)p.B * p.H * count_row_blocks(p.L, kPlanBM, p.row_stride) <= (d == 64 ? 384 : 192)) return launch_attn_rows16<T>(p, d, kt, st);
     if (p.plan) {
         if (d == 64) return kt ? launch_attn<T, 64, true, 64, 2, true>(p, st) : launch_attn<T, 64, false, 64, 2, true>(p, st);
         return kt ? launch_attn<T, 128, true, 64, 2, true>(p, st) : launch_attn<T, 128, false, 64, 2, true>(p, st);

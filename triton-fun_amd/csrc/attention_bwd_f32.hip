@@ -40,7 +40,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_f32_kernel(cons
     const int rb = at >> 1, half = at & 1;
     const int b = bh / p.H, h = bh % p.H;
     const int rs = p.row_stride, L = p.L, Lr = p.Lr;
-    const int k0 = half * kF32Rows;
+    const int k0 = half * kHalfRows;
     const int r0 = block_first_row(rb, kPlanBM, rs) + rs * k0;
     if (r0 >= Lr) return;
 
@@ -82,8 +82,8 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_f32_kernel(cons
     // ---- plan: the row block's walk, cut down to the tiles that this half of it sees ----
     const PlanRec* const pt = p.plan;
     const int n_rb = p.n_row_blocks;
-    auto walk_of = [&](int sg) { return walk_f32<BN>(pt, n_rb, p.n_seg, rb, half, sg); };
-    auto next_segment = [&](WalkF32& w) {  // the first segment from w.seg on that has tiles
+    auto walk_of = [&](int sg) { return half_walk<BN>(pt, n_rb, p.n_seg, rb, half, sg); };
+    auto next_segment = [&](HalfWalk& w) {  // the first segment from w.seg on that has tiles
         for (int sg = w.seg; sg < p.n_seg; ++sg) {
             w = walk_of(sg);
             if (w.end > w.tile) return;
@@ -92,18 +92,18 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_f32_kernel(cons
     };
     int total = 0;
     for (int sg = 0; sg < p.n_seg; ++sg) {
-        const WalkF32 w = walk_of(sg);
+        const HalfWalk w = walk_of(sg);
         total += w.end - w.tile;
     }
     total = __builtin_amdgcn_readfirstlane(total);
 
     // ---- asynchronous copies of one tile (see attention_f32.hip) ----
-    auto position_row = [&](const WalkF32& w, int j) { return min(max(w.pl.c0 + w.pl.cs * j, 0), L - 1); };
+    auto position_row = [&](const HalfWalk& w, int j) { return min(max(w.pl.c0 + w.pl.cs * j, 0), L - 1); };
     uint32_t x_off[NI], y_off[NI];
     const char *x_next = nullptr, *y_next = nullptr;
     int64_t x_row = 0, y_row = 0;  // bytes from one tile row to the next
     bool off_fits = true;
-    auto set_offsets = [&](const WalkF32& w) {
+    auto set_offsets = [&](const HalfWalk& w) {
         x_row = (int64_t)p.x_sl * 4 * w.pl.cs;
         y_row = (int64_t)p.y_sl * 4 * w.pl.cs;
         off_fits = x_row * RPI < ((int64_t)1 << 31) && y_row * RPI < ((int64_t)1 << 31);
@@ -117,7 +117,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_f32_kernel(cons
         x_next = reinterpret_cast<const char*>(xb) + first * p.x_sl * 4 + wave * RPI * x_row;
         y_next = reinterpret_cast<const char*>(yb) + first * p.y_sl * 4 + wave * RPI * y_row;
     };
-    auto issue_next = [&](WalkF32& w, int stage) {
+    auto issue_next = [&](HalfWalk& w, int stage) {
         char* xs_w = smem + RING + stage * STAGE;
         const int j0 = w.tile * BN;
         if (off_fits && w.pl.c0 + w.pl.cs * (j0 + BN - 1) < L && w.pl.c0 + w.pl.cs * j0 >= 0) {
@@ -154,7 +154,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_f32_kernel(cons
     for (int j = 0; j < 4; ++j) c_addr[j] = smem_base + RING + lds_off<ROWB, true>(4 * g + j, 16 * n);
     uint32_t st_addr = smem_base + 16 * g;
 
-    WalkF32 fetch, cur;
+    HalfWalk fetch, cur;
     fetch.seg = 0;
     next_segment(fetch);
     if (fetch.seg < p.n_seg) set_offsets(fetch);
@@ -170,7 +170,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_f32_kernel(cons
         if constexpr (KEYS) acc2[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
     const float c2 = p.scale_log2e;
-    RowStateF32 rows;
+    RowState rows;
     bool entered = false;
     int stage = 0;
 #if defined(__HIP_DEVICE_COMPILE__)

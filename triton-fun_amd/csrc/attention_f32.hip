@@ -29,7 +29,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_f32_kernel(const AttnParams p
     constexpr int TILE = BN * D * 4, STAGE = 2 * TILE;
     constexpr int NDMA = STAGE / 4096;  // copy instructions per wavefront and tile
     constexpr int K_SWZ = KT ? (K_ROWB == 128 ? 2 : 0) : 1;
-    static_assert(kPlanBM == 2 * kF32Rows && kBN % BN == 0, "half a row block of the plan per workgroup");
+    static_assert(kPlanBM == 2 * kHalfRows && kBN % BN == 0, "half a row block of the plan per workgroup");
 
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     __shared__ SegPlan s_plan[SPLAT_MAX_SEGMENTS];
@@ -47,7 +47,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_f32_kernel(const AttnParams p
     const int rb = at >> 1, half = at & 1;
     const int b = bh / p.H, h = bh % p.H;
     const int rs = p.row_stride, L = p.L;
-    const int k0 = half * kF32Rows;                    // the workgroup's first row within its row block
+    const int k0 = half * kHalfRows;                    // the workgroup's first row within its row block
     const int r0 = block_first_row(rb, kPlanBM, rs) + rs * k0;
     if (r0 >= L) return;
 
@@ -79,10 +79,10 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_f32_kernel(const AttnParams p
     const int n_rb = p.n_row_blocks;
     if constexpr (!PLANNED) plan_segments<kPlanBM, kBN>(p.seg, p.n_seg, block_first_row(rb, kPlanBM, rs), rs, L, !KT, s_plan, &s_ps, tid);
     auto walk_of = [&](int sg) {
-        WalkF32 w;
+        HalfWalk w;
         w.seg = sg;
         if constexpr (PLANNED) {
-            w = walk_f32<BN>(pt, n_rb, p.n_seg, rb, half, sg);
+            w = half_walk<BN>(pt, n_rb, p.n_seg, rb, half, sg);
         } else {
             const SegPlan l = s_plan[sg];
             w.pl.c0 = __builtin_amdgcn_readfirstlane(l.c0);
@@ -93,7 +93,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_f32_kernel(const AttnParams p
         }
         return w;
     };
-    auto next_segment = [&](WalkF32& w) {  // the first segment from w.seg on that has tiles
+    auto next_segment = [&](HalfWalk& w) {  // the first segment from w.seg on that has tiles
         for (int sg = w.seg; sg < p.n_seg; ++sg) {
             w = walk_of(sg);
             if (w.end > w.tile) return;
@@ -102,7 +102,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_f32_kernel(const AttnParams p
     };
     int total = 0;
     for (int sg = 0; sg < p.n_seg; ++sg) {
-        const WalkF32 w = walk_of(sg);
+        const HalfWalk w = walk_of(sg);
         total += w.end - w.tile;
     }
     total = __builtin_amdgcn_readfirstlane(total);
@@ -112,7 +112,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_f32_kernel(const AttnParams p
     // uniform pointers and per-lane offsets that stay the same for the whole segment ----
     constexpr int NI = TILE / 4096;  // blocks per wavefront and operand
     constexpr int V_CPR = V_ROWB / 16, V_RPI = 1024 / V_ROWB, K_CPR = K_ROWB / 16, K_RPI = 1024 / K_ROWB;
-    auto issue_general = [&](const WalkF32& w, int stage) {
+    auto issue_general = [&](const HalfWalk& w, int stage) {
         const int j0 = w.tile * BN;
         char* ks_w = smem + stage * STAGE;
         auto key_row = [&](int row) { return min(max(w.pl.c0 + w.pl.cs * (j0 + row), 0), L - 1); };
@@ -134,7 +134,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_f32_kernel(const AttnParams p
     const char *v_next = nullptr, *k_next = nullptr;
     int64_t v_row = 0, k_row = 0;  // bytes from one tile row to the next
     bool off_fits = true;          // the copy instruction takes a 32-bit offset
-    auto set_offsets = [&](const WalkF32& w) {
+    auto set_offsets = [&](const HalfWalk& w) {
         v_row = (int64_t)p.v_sl * 4 * w.pl.cs;
         k_row = KT ? (int64_t)p.k_sd * 4 : (int64_t)p.k_sl * 4 * w.pl.cs;
         off_fits = v_row * V_RPI < ((int64_t)1 << 31) && k_row * K_RPI < ((int64_t)1 << 31);
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_f32_kernel(const AttnParams p
         k_next = reinterpret_cast<const char*>(kb) + (KT ? first * 4 : first * p.k_sl * 4) + wave * K_RPI * k_row;
     };
     // copy tile `w.tile` into the stage and move on (w: the fetching walk; its pointers stand at that tile)
-    auto issue_next = [&](WalkF32& w, int stage) {
+    auto issue_next = [&](HalfWalk& w, int stage) {
         const int last = w.pl.c0 + w.pl.cs * (w.tile * BN + BN - 1);
         if (off_fits && last < L && w.pl.c0 + w.pl.cs * w.tile * BN >= 0) {
             char* ks_w = smem + stage * STAGE;
@@ -179,7 +179,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_f32_kernel(const AttnParams p
         for (int t = 0; t < KQ; ++t) k_addr[t] = smem_base + lds_off<K_ROWB, true>(n, (16 * t + 4 * g) * 4);
     uint32_t v_addr = smem_base + TILE + 4 * g * V_ROWB + n * 16;
 
-    WalkF32 fetch, cur;
+    HalfWalk fetch, cur;
     fetch.seg = 0;
     next_segment(fetch);
     if (fetch.seg < p.n_seg) set_offsets(fetch);
@@ -200,7 +200,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_f32_kernel(const AttnParams p
     for (int i = 0; i < 4 * DH; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m_ref = kNegBigA, l_run = 0.f;
     const float c2 = p.scale_log2e;
-    RowStateF32 rows;
+    RowState rows;
     bool entered = false;
     int stage = 0, stage_pf = PD;
 

@@ -30,6 +30,9 @@ constexpr float kRescaleThreshold = 8.0f;  // in log2 units: exponentials stay b
 
 // the float32 forward (attention_f32.hip); p.n_row_blocks and p.total are filled in by the launch
 int launch_attn_f32(const AttnParams& p, int d, bool kt, hipStream_t st);
+// the 16-bit forward for launches of few row blocks (attention_rows16.hip)
+template <typename T>
+int launch_attn_rows16(const AttnParams& p, int d, bool kt, hipStream_t st);
 
 // Live positions of one row in the tile that starts at position j0, one bit per position (bit b = position j0 + b):
 // the row's span [lo, lo + cnt) intersected with its periodic pattern.  `first` is the smallest offset >= 0 in the tile

@@ -40,6 +40,14 @@ template <int ROWB>
 __device__ __forceinline__ constexpr int swz64(int row) {
     return ROWB >= 256 ? (row & 3) : ((row >> 1) & 1);
 }
+// The same for transposing reads 16 columns (32 bytes) wide, whose 64 lanes touch 16 rows: four groups of 4 consecutive rows, 4
+// apart (rows = positions) or 8 apart (rows = d); the 32-byte blocks of any 8 of them that come together fill the 256-byte
+// bank space.
+template <int ROWB>
+__device__ __forceinline__ constexpr int swz32(int row) {
+    static_assert(ROWB == 64 || ROWB == 128 || ROWB == 256, "row pitch");
+    return ROWB == 256 ? (row & 7) : ROWB == 128 ? (((row >> 1) & 1) | (((row >> 3) & 1) << 1)) : ((row >> 3) & 1);
+}
 // Swizzle for tiles that are read both ways: the 64-byte block index is rotated as for the transposing read, and the
 // chunk inside the block by the next two row bits, so that the 16 rows a row-wise 16-byte read touches at once land on
 // 16 different chunk positions of the 256-byte bank space (rows 16 apart share their pattern; rows 8 apart differ in
@@ -49,12 +57,13 @@ __device__ __forceinline__ constexpr int dual_chunk(int row, int c) {
     return (((c >> 2) ^ swz64<ROWB>(row)) << 2) | ((c & 3) ^ ((row >> 2) & 3));
 }
 // logical 16-byte chunk held at physical chunk position pc of `row`; MODE 0: none, 1: chunk XOR (b128 row reads),
-// 2: 64-byte block XOR (transposing reads), 3: both kinds of read (dual_chunk)
+// 2: 64-byte block XOR (transposing reads), 3: both kinds of read (dual_chunk), 4: 32-byte block XOR (narrow transposing reads)
 template <int ROWB, int MODE>
 __device__ __forceinline__ int logical_chunk(int row, int pc) {
     if constexpr (MODE == 1) return pc ^ swz<ROWB>(row);
     if constexpr (MODE == 2) return (((pc >> 2) ^ swz64<ROWB>(row)) << 2) | (pc & 3);
     if constexpr (MODE == 3) return dual_chunk<ROWB>(row, pc);
+    if constexpr (MODE == 4) return (((pc >> 1) ^ swz32<ROWB>(row)) << 1) | (pc & 1);
     return pc;
 }
 
