@@ -65,7 +65,7 @@ def _host_ext() -> None:
     inc = [*include_paths(), os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]
     cmd = ["g++", "-O2", "-fPIC", "-shared", "-std=c++17", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
            *(f"-I{p}" for p in inc), os.path.join(CSRC, "host_ext.cpp"), "-o", HOST_EXT,
-           *(f"-L{p}" for p in library_paths()), "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+           *(f"-L{p}" for p in library_paths()), "-ltorch_python", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"g++ failed on host_ext.cpp:\n{r.stderr}")
