@@ -1,0 +1,94 @@
+"""The operators' kernels for head dimensions that pad their tiles and for rows of the compressed matrix that start anywhere,
+against float64: 16-bit types, d in whole 16-byte pieces, odd row lengths, few and many row blocks."""
+import pytest
+import torch
+
+import acsr_helpers as A
+import r_sddmm
+import r_spmm
+from r_attention import RegularAttention
+
+pytestmark = pytest.mark.gpu
+
+SENTINEL = -77.0
+MASKS = {
+    "one": lambda L: [A.causal_windowed_pattern(L, 0)],
+    "causal17": lambda L: [A.causal_windowed_pattern(L, 16)],
+    "windowed129": lambda L: [A.windowed_pattern(L, 64)],
+    "windowed301": lambda L: [A.windowed_pattern(L, 150)],
+    "dilated": lambda L: [A.dilated_pattern(L, 41, 3)],
+    "strided": lambda L: A.strided_patterns(L, 13, 7),
+}
+HALF_ULP = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}  # of a value, rounded once from float32
+
+
+def case(dev, name, B, H, L, d, dtype):
+    masks = MASKS[name](L)
+    g = torch.Generator().manual_seed(L + d)
+    q, k, v = (torch.randn(B, H, L, d, generator=g).to(dtype) for _ in range(3))
+    attn = RegularAttention(B, L, H, d, masks, 16, 16, dev, dtype, scale=d ** -0.5, fused=False)
+    return masks, attn, q, k, v
+
+
+def slots(attn, L):
+    """(columns [L, T], live [L, T]) of the compressed rows."""
+    cols, live = zip(*(r_sddmm.live_slot_columns(t[2].cpu(), t[3].cpu(), t[4].cpu(), int(t[5]), None if fc is None else fc.cpu())
+                       for t, fc in zip(attn.segments.tuples, attn.segments.first_cols)))
+    return torch.cat(cols, 1).clamp(0, L - 1), torch.cat(live, 1)
+
+
+@pytest.mark.parametrize("name", MASKS)
+@pytest.mark.parametrize("B,H,L", [(1, 2, 130), (1, 3, 333), (4, 16, 530)])
+@pytest.mark.parametrize("dtype,d", [(torch.float16, 8), (torch.bfloat16, 24), (torch.float16, 32), (torch.float16, 64),
+                                     (torch.bfloat16, 72), (torch.float16, 80), (torch.bfloat16, 96), (torch.bfloat16, 120),
+                                     (torch.float16, 128)])
+def test_operators_against_float64(dev, name, B, H, L, d, dtype):
+    masks, attn, q, k, v = case(dev, name, B, H, L, d, dtype)
+    T = attn.acsr_trailing_dim if len(masks) == 1 else attn.segments.T
+    cols, live = slots(attn, L)
+    scores = q.double() @ k.double().transpose(2, 3) * d ** -0.5
+    want = scores.gather(3, cols.expand(B, H, L, T))
+    lse = torch.logsumexp(scores.masked_fill(~(sum(m.device_mask(dev) for m in masks).cpu() > 0), float("-inf")), -1)
+    qd, kd, vd = q.to(dev), k.to(dev).transpose(2, 3), v.to(dev)
+    none = [None] * 4
+
+    def sddmm(**kw):
+        out = torch.full((B, H, L, T), SENTINEL, dtype=dtype, device=dev)
+        r_sddmm.rsddmm_launcher(qd, kd, out, *none, T, None, None, None, None, 16, 16, scale=d ** -0.5, segments=attn.segments, **kw)
+        return out
+    got = sddmm()
+    assert torch.all(got.cpu()[..., ~live] == SENTINEL), "dead slots must not be written"
+    # float32 sums of d products of 16-bit values, then one rounding
+    err = (got.double().cpu() - want).abs()[..., live]
+    assert bool((err <= 1.01 * HALF_ULP[dtype] * want.abs()[..., live] + 1e-5).all())
+    assert torch.equal(got, sddmm(plan=False))
+    probs = sddmm(lse=lse.float().to(dev).contiguous())
+    pw = torch.exp(want - lse[..., None])
+    perr = (probs.double().cpu() - pw).abs()[..., live]
+    assert bool((perr <= 1.01 * HALF_ULP[dtype] * pw[..., live] + 1e-5).all())
+    # the product of the stored probabilities; dead slots hold anything
+    given = torch.where(live.to(dev), probs, torch.full_like(probs, float("nan")))
+    dense = torch.zeros(B, H, L, L, dtype=torch.float64)
+    dense.scatter_add_(3, cols.expand(B, H, L, T), torch.where(live, probs.double().cpu(), torch.zeros(()).double()))
+    ref = dense @ v.double()
+    out = torch.full((B, H, L, d), SENTINEL, dtype=dtype, device=dev)
+    r_spmm.rspmm_launcher(given, vd, out, *none, None, None, T, None, None, 16, 16, segments=attn.segments)
+    oerr = (out.double().cpu() - ref).abs()
+    assert bool((oerr <= 1.01 * HALF_ULP[dtype] * ref.abs() + 1e-5).all())
+
+
+@pytest.mark.parametrize("d", [24, 80])
+def test_padding_meets_no_infinity(dev, d):
+    """An infinite key gives infinite scores at its column and leaves every other one finite: the padded part of the tiles
+    multiplies nothing of it."""
+    B, H, L = 1, 2, 200
+    masks, attn, q, k, v = case(dev, "windowed129", B, H, L, d, torch.float16)
+    k[:, :, 60] = float("inf")
+    T = attn.acsr_trailing_dim
+    cols, live = slots(attn, L)
+    out = torch.zeros(B, H, L, T, dtype=torch.float16, device=dev)
+    r_sddmm.rsddmm_launcher(q.abs().to(dev) + 1, k.to(dev).transpose(2, 3), out, *[None] * 4, T, None, None, None, None, 16, 16,
+                            segments=attn.segments)
+    got = out.cpu()
+    hit = (cols == 60) & live
+    assert bool((got[..., hit] == float("inf")).all()) and bool(torch.isfinite(got[..., live & ~hit]).all())

@@ -69,11 +69,11 @@ _HALF = (torch.float16, torch.bfloat16)
 
 def _takes_a_plan(x, output, y, B: int, H: int, L: int, d: int, T: int, segs: ACSRSegments) -> bool:
     """Whether this launch runs the kernel that reads a plan table (the library decides by the same rules and ignores the
-    plan otherwise): 16-bit types, d = 64 / 128, rows of K contiguous, 16-byte alignment, and at least 256 row blocks or rows
-    of at most 256 slots (fewer blocks of longer rows are better off with the general kernel's split of the key range)."""
-    if x.dtype not in (torch.float16, torch.bfloat16) or output.dtype != x.dtype or d not in (64, 128):
+    plan otherwise): 16-bit types, d up to 128 in whole 16-byte pieces, rows of K contiguous, and at least 256 row blocks or
+    rows of at most 256 slots (fewer blocks of longer rows are better off with the general kernel's split of the key range)."""
+    if x.dtype not in (torch.float16, torch.bfloat16) or output.dtype != x.dtype or d % 8 != 0 or d > 128:
         return False
-    if y.stride(2) != 1 or T % 8 != 0 or any(off % 8 for off in segs.offsets):
+    if y.stride(2) != 1:
         return False
     return B * H * ((L + 127) // 128) >= 256 or T <= 256
 
@@ -92,8 +92,8 @@ def rsddmm_launcher(x: torch.Tensor, y: torch.Tensor, output: torch.Tensor,
     geometry and are accepted unchanged; the HIP kernel tiles by itself from the row maps.  With ``lse`` (float32
     [B, H, L], contiguous: every row's log of its sum of exp(scale * score), as the fused forward hands it out) the
     stored value is exp(scale * score - lse[row]), the row's softmax probability, instead of the score.
-    ``plan``: the mask's plan table (``ACSRSegments.plan``); by default the launches that use one (16-bit types, d = 64 or
-    128, at least 256 row blocks of 128 rows or rows of at most 256 slots) build it on their first call and keep it with the metadata, ``False``
+    ``plan``: the mask's plan table (``ACSRSegments.plan``); by default the launches that use one (16-bit types, d a multiple
+    of 8 up to 128, at least 256 row blocks of 128 rows or rows of at most 256 slots) build it on their first call and keep it with the metadata, ``False``
     launches without one.  The results are the same bit for bit.
     Returns (output, sTod_linear_transformations, sTod_translations, nnzs)."""
     for name, t in (("x", x), ("y", y), ("output", output)):
@@ -103,8 +103,8 @@ def rsddmm_launcher(x: torch.Tensor, y: torch.Tensor, output: torch.Tensor,
     segs = segments or ACSRSegments.single(dTos_linear_transformations, dTos_translations,
                                            sTod_linear_transformations, sTod_translations, nnzs, trailing_dim)
     if plan is None and x.dim() == 4 and output.shape[-1] == trailing_dim:
-        # (the library uses the table where it has a kernel that reads one: 16-bit types at d = 64 / 128)
-        mask = segs.native(x.shape[2], x.device, x.shape[3] in (64, 128) and x.dtype in _HALF)
+        # (the library uses the table where it has a kernel that reads one: 16-bit types, d in whole 16-byte pieces up to 128)
+        mask = segs.native(x.shape[2], x.device, x.shape[3] % 8 == 0 and x.shape[3] <= 128 and x.dtype in _HALF)
         if mask is not None and _hip.host().sddmm(mask, x, y, output, 1.0 if scale is None else scale, lse):
             return (output, sTod_linear_transformations, sTod_translations, nnzs)
     B, H, L, d = x.shape

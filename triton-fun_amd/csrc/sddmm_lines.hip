@@ -1,5 +1,6 @@
-// SDDMM on ACSR for the common fast shape: 16-bit inputs and outputs of one type, d = 64 or 128, rows of K contiguous,
-// 16-byte alignment everywhere, at least 256 row blocks in the launch or rows of at most 256 slots.
+// SDDMM on ACSR for the common fast shape: 16-bit inputs and outputs of one type, rows of Q and K contiguous in whole 16-byte
+// pieces, d at most 128, at least 256 row blocks in the launch or rows of at most 256 slots.  d = 64 and 128 with output rows
+// on 16-byte boundaries have instantiations of their own; the others (PART) pad the contraction to 64 or 128 in LDS.
 //
 // A workgroup of 8 wavefronts owns 128 rows of one (batch, head); wavefront w owns rows 16w..16w+15 and computes
 // S^T = K Q^T with 16x16x32 MFMAs (rows = keys, columns = queries: a lane owns one query row and, per 16-key block, 4
@@ -21,6 +22,14 @@
 // a lane reads the 24 aligned bytes around its 8 slots and shifts (a 16-byte LDS read at a 2-byte offset costs several
 // times an aligned one).  Other plans (rows with differing steps) walk dense columns and store element by element under
 // the row's affine test.
+//
+// PART: a key row fills d / 8 of the stage row's chunks; the lanes of a copy whose chunk lies past it sit the copy out (every
+// copy instruction covers a whole stage row, so it always has lanes), and those chunks hold the zeros written once at the
+// start, so that an infinity in K meets no padding.  Contraction steps past d are skipped.  Rows of the compressed matrix
+// that start anywhere are stored through the cache, which joins the lines that two units share.  The bound is as above;
+// 16 heads of 2000 rows, 129 slots, d = 80, float16: 23.4 us in the general kernel (256 workgroups of four wavefronts,
+// one step in flight), 12.4 here; the shapes below the
+// block limit gain as much (4 heads of 1000 rows, 255 slots, d = 96, the three operators: 51 -> 31 us).
 #include <algorithm>
 #include <type_traits>
 
@@ -45,7 +54,7 @@ struct LinesGeom {
     static constexpr int LDS_BYTES = PLANNED ? PLAN_AT : PLAN_AT + (int)sizeof(PlanScratch<BM>) + SPLAT_MAX_SEGMENTS * ((int)sizeof(SegPlan) + 4);
 };
 
-template <typename T, int D, int NST, int KEYS, int HL, int BM_, bool PROBS, bool PLANNED>
+template <typename T, int D, int NST, int KEYS, int HL, int BM_, bool PROBS, bool PLANNED, bool PART>
 __global__ __launch_bounds__(BM_ * 4, 4) void sddmm_lines_kernel(const SddmmParams p) {
     using G = LinesGeom<D, NST, KEYS, HL, BM_, PLANNED>;
     static_assert(!PLANNED || BM_ == kPlanBM, "the plan table is laid out for 128-row blocks");
@@ -91,7 +100,18 @@ __global__ __launch_bounds__(BM_ * 4, 4) void sddmm_lines_kernel(const SddmmPara
     const T* qr = qb + (int64_t)min(my_r, L - 1) * p.q_sl;
     Frag<T> qf[KS];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qf[ks] = global_frag<T>(qr + 32 * ks + 8 * g4);
+    for (int ks = 0; ks < KS; ++ks) {
+        if (!PART || 32 * ks + 8 * g4 < p.d)
+            qf[ks] = global_frag<T>(qr + 32 * ks + 8 * g4);
+        else
+            qf[ks].v = __builtin_bit_cast(typename Frag<T>::vec, u32x4{0u, 0u, 0u, 0u});
+    }
+    if constexpr (PART) {  // the padding of the key rows: what no copy writes
+        if (p.d < D) {     // workgroup-uniform
+            for (int at = tid * 16; at < NST * STAGE; at += BM_ * 64) *reinterpret_cast<u32x4*>(s_kring + at) = u32x4{0u, 0u, 0u, 0u};
+            lds_barrier();
+        }
+    }
     const float out_scale = PROBS ? 1.0f : p.scale;
     const float exp_mul = p.scale * 1.4426950408889634f;
     float exp_sub = 0.f;
@@ -194,13 +214,13 @@ __global__ __launch_bounds__(BM_ * 4, 4) void sddmm_lines_kernel(const SddmmPara
                 const char* base = kbytes + key_first * k_rowb;
 #pragma unroll
                 for (int i = 0; i < NI; ++i)
-                    dma16_uniform(base, d_off[i], s_kring + stage * STAGE + (wave + NW * i) * 1024);
+                    if (!PART || d_col[i] < p.d * 2) dma16_uniform(base, d_off[i], s_kring + stage * STAGE + (wave + NW * i) * 1024);
                 return;
             }
 #pragma unroll
             for (int i = 0; i < NI; ++i) {
                 const int n = min(max(pl.c0 + pl.cs * (s * KEYS + d_row[i]), 0), p.n_keys - 1);
-                dma16(kbytes + n * k_rowb + d_col[i], s_kring + stage * STAGE + (wave + NW * i) * 1024);
+                if (!PART || d_col[i] < p.d * 2) dma16(kbytes + n * k_rowb + d_col[i], s_kring + stage * STAGE + (wave + NW * i) * 1024);
             }
         };
 
@@ -231,7 +251,7 @@ __global__ __launch_bounds__(BM_ * 4, 4) void sddmm_lines_kernel(const SddmmPara
                 for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
                     for (int kt = 0; kt < 2; ++kt)
-                        fr[half][2 * ks + kt].v = __builtin_bit_cast(
+                        if (!PART || 32 * ks < p.d) fr[half][2 * ks + kt].v = __builtin_bit_cast(
                             typename Frag<T>::vec, *reinterpret_cast<const u32x4*>(s_kring + a_off[ks] + (stage * STAGE + (32 * half + 16 * kt) * ROWB)));
             };
             f32x4v acc[2][2];
@@ -244,7 +264,7 @@ __global__ __launch_bounds__(BM_ * 4, 4) void sddmm_lines_kernel(const SddmmPara
                 for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
                     for (int kt = 0; kt < 2; ++kt) {
-                        mma16(acc[half][kt], fr[half][2 * ks + kt], qf[ks]);
+                        if (!PART || 32 * ks < p.d) mma16(acc[half][kt], fr[half][2 * ks + kt], qf[ks]);
                     }
             };
             // scores of 32 positions into the rows' rings (uniform plans) or straight to their slots (other plans)
@@ -294,6 +314,13 @@ __global__ __launch_bounds__(BM_ * 4, 4) void sddmm_lines_kernel(const SddmmPara
                 r[3] = __builtin_amdgcn_alignbit(x4, x3, sh);
                 return r;
             };
+            // 8 slots: around the cache where rows start on 16-byte boundaries, through it at any other alignment
+            auto store8 = [&](T* dst, const u32x4& val) {
+                if (!PART || p.out_vec)
+                    __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(dst));
+                else
+                    __builtin_memcpy(dst, &val, 16);
+            };
             // store the units that the positions from pos0 up to pos1 (the first HL of them since the last call) have
             // completed
             auto flush = [&](int pos0, int pos1) {
@@ -305,7 +332,7 @@ __global__ __launch_bounds__(BM_ * 4, 4) void sddmm_lines_kernel(const SddmmPara
                     for (int c = 0; c < NC; ++c) {
                         const int s0 = HL * f_done[c] + 8 * f_piece;
                         const u32x4 val = take(c, s0);
-                        __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>((T*)p.out + f_base[c] + s0));
+                        store8((T*)p.out + f_base[c] + s0, val);
                         f_done[c] += 1;
                     }
                     return;
@@ -324,7 +351,7 @@ __global__ __launch_bounds__(BM_ * 4, 4) void sddmm_lines_kernel(const SddmmPara
                             T* const dst = (T*)p.out + f_base[c] + s0;
                             const int n = f_cnt[c] - s0;
                             if (n >= 8) {
-                                __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(dst));
+                                store8(dst, val);
                             } else {
                                 typedef T v8 __attribute__((ext_vector_type(8)));
                                 const v8 e8 = __builtin_bit_cast(v8, val);
@@ -359,7 +386,7 @@ __global__ __launch_bounds__(BM_ * 4, 4) void sddmm_lines_kernel(const SddmmPara
     }
 }
 
-template <typename T, int D, int NST, int KEYS, int HL, int BM, bool PROBS, bool PLANNED>
+template <typename T, int D, int NST, int KEYS, int HL, int BM, bool PROBS, bool PLANNED, bool PART>
 static int launch_lines_variant(const char* who, SddmmParams p, hipStream_t st) {
     using G = LinesGeom<D, NST, KEYS, HL, BM, PLANNED>;
     static_assert(G::LDS_BYTES * (256 / BM) <= 160 * 1024, "16 wavefronts per compute unit");
@@ -369,7 +396,7 @@ static int launch_lines_variant(const char* who, SddmmParams p, hipStream_t st) 
     p.key_split = 1;
     p.total = (int)blocks;
     static uint64_t reserved = 0;
-    auto kern = sddmm_lines_kernel<T, D, NST, KEYS, HL, BM, PROBS, PLANNED>;
+    auto kern = sddmm_lines_kernel<T, D, NST, KEYS, HL, BM, PROBS, PLANNED, PART>;
     if (int rc = reserve_dynamic_lds(&reserved, reinterpret_cast<const void*>(kern), G::LDS_BYTES, who)) return rc;
     const int grid = ((p.total + 7) / 8) * 8;
     kern<<<grid, BM * 4, G::LDS_BYTES, st>>>(p);
@@ -379,31 +406,31 @@ static int launch_lines_variant(const char* who, SddmmParams p, hipStream_t st) 
 // Whole 128-byte lines are what the memory system likes best (a blocked mask at d = 128: 0.25 ms against 0.34 ms with
 // halves), but their rings take 34 KiB of LDS, which at d = 128 leaves room for steps of 32 keys only (two barriers per
 // 64 keys).  Short rows (one or two lines) are better off with halves and steps of 64 keys.
-template <typename T, bool PROBS, bool PLANNED>
+template <typename T, bool PROBS, bool PLANNED, bool PART>
 static int launch_lines_typed(const char* who, const SddmmParams& p, hipStream_t st) {
-    if (p.d == 128) {
-        if (p.T >= 256) return launch_lines_variant<T, 128, PLANNED ? 5 : 4, 32, 64, 128, PROBS, PLANNED>(who, p, st);
-        return launch_lines_variant<T, 128, 3, 64, 32, 128, PROBS, PLANNED>(who, p, st);
+    if (p.d > 64) {
+        if (p.T >= 256) return launch_lines_variant<T, 128, PLANNED ? 5 : 4, 32, 64, 128, PROBS, PLANNED, PART>(who, p, st);
+        return launch_lines_variant<T, 128, 3, 64, 32, 128, PROBS, PLANNED, PART>(who, p, st);
     }
-    if (p.T >= 128) return launch_lines_variant<T, 64, 4, 64, 64, 128, PROBS, PLANNED>(who, p, st);
-    return launch_lines_variant<T, 64, 4, 64, 32, 128, PROBS, PLANNED>(who, p, st);
+    if (p.T >= 128) return launch_lines_variant<T, 64, 4, 64, 64, 128, PROBS, PLANNED, PART>(who, p, st);
+    return launch_lines_variant<T, 64, 4, 64, 32, 128, PROBS, PLANNED, PART>(who, p, st);
 }
 
-int launch_sddmm_lines(const char* who, const SddmmParams& p_in, int in_dtype, hipStream_t st) {
-    if (in_dtype == SPLAT_F32 || p_in.out_dtype != in_dtype) return 0;
-    if (p_in.d != 64 && p_in.d != 128) return 0;
-    if (p_in.k_sd != 1 || !p_in.q_vec || !p_in.k_vec || !p_in.out_vec) return 0;
-    const SddmmParams& p = p_in;
+int launch_sddmm_lines(const char* who, const SddmmParams& p, int in_dtype, hipStream_t st) {
+    if (in_dtype == SPLAT_F32 || p.out_dtype != in_dtype) return 0;
+    if (p.d % 8 != 0 || p.d > 128) return 0;
+    if (p.k_sd != 1 || !p.q_vec || !p.k_vec) return 0;
     // Few row blocks with long rows are better off with the general kernel, which splits a block's key range over several
     // workgroups (64 blocks of 1024 slots: 0.021 against 0.029 ms; of 256 slots: 0.016 against 0.013).
     if ((int64_t)p.B * p.H * count_row_blocks(p.L, 128, p.row_stride) < 256 && p.T > 256) return 0;
-    const bool probs = p.row_lse != nullptr;
-    const SddmmParams& pp = p;
+    const bool part = (p.d != 64 && p.d != 128) || !p.out_vec;
     auto go = [&](auto t, auto probs_c, auto planned_c) {
-        return launch_lines_typed<decltype(t), decltype(probs_c)::value, decltype(planned_c)::value>(who, pp, st);
+        constexpr bool PROBS = decltype(probs_c)::value, PLANNED = decltype(planned_c)::value;
+        return part ? launch_lines_typed<decltype(t), PROBS, PLANNED, true>(who, p, st)
+                    : launch_lines_typed<decltype(t), PROBS, PLANNED, false>(who, p, st);
     };
-    auto by_plan = [&](auto t, auto probs_c) { return pp.plan ? go(t, probs_c, std::true_type{}) : go(t, probs_c, std::false_type{}); };
-    auto by_probs = [&](auto t) { return probs ? by_plan(t, std::true_type{}) : by_plan(t, std::false_type{}); };
+    auto by_plan = [&](auto t, auto probs_c) { return p.plan ? go(t, probs_c, std::true_type{}) : go(t, probs_c, std::false_type{}); };
+    auto by_probs = [&](auto t) { return p.row_lse ? by_plan(t, std::true_type{}) : by_plan(t, std::false_type{}); };
     return in_dtype == SPLAT_BF16 ? by_probs(bf16{}) : by_probs(f16{});
 }
 

@@ -1,4 +1,4 @@
-// Kernel arguments of the SpMM kernels (spmm.hip: every shape; spmm_thin.hip, spmm_tile.hip, spmm_t_thin.hip: 16-bit types, 64 / 128
+// Kernel arguments of the SpMM kernels (spmm.hip: every shape; spmm_thin.hip, spmm_tile.hip: 16-bit types, up to 128 output columns; spmm_t_thin.hip: 64 / 128
 // output columns).
 #pragma once
 #include "acsr_plan.hpp"

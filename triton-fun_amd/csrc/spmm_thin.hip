@@ -373,7 +373,7 @@ static int launch_thin_variant(const char* who, SpmmParams p, hipStream_t st) {
 int launch_spmm_thin(const char* who, const SpmmParams& p, int in_dtype, hipStream_t st) {
     if (!p.plan) return 0;  // this kernel starts from the mask's plan table
     if (in_dtype == SPLAT_F32 || p.out_dtype != in_dtype) return 0;
-    if (p.n_out != 64 && p.n_out != 128) return 0;
+    if (p.n_out != 64 && p.n_out != 128) return launch_spmm_tile(who, p, in_dtype, st);
     if (!p.v_vec || !p.out_vec) return 0;
     // a lane reads 16 bytes at a time from inside its row's share of a segment
     for (int k = 0; k < p.n_seg; ++k)

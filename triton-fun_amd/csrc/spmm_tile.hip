@@ -1,6 +1,6 @@
 // SpMM on ACSR for 16-bit launches with the mask's plan table, except those that spmm_thin.hip's rings take (long rows on
-// 16-byte boundaries in a compressed matrix larger than the last-level cache): probabilities, V and output of one type, 64 or
-// 128 output columns.
+// 16-byte boundaries in a compressed matrix larger than the last-level cache): probabilities, V and output of one type, at
+// most 128 output columns in whole 16-byte pieces (64 and 128 have instantiations of their own; PART takes the others).
 //
 // A workgroup of 8 wavefronts owns 128 rows of one (batch, head) and walks their key positions in steps of 64 as the
 // table lists them.  Per step the whole workgroup loads every row's 64 entries (8 pieces of 8 consecutive slots, 16 bytes
@@ -11,6 +11,11 @@
 // (chunks permuted by the row so that a read covers all banks), the A operands transposing reads of the V tile (layout of
 // spmm_thin.hip).  Plans whose rows step differently walk dense columns and gather element by element under the row's
 // affine test.  The output leaves through an LDS turn-around as whole rows, non-temporal.
+//
+// PART: V rows fill n_out / 8 chunks of a tile row padded to 64 or 128 columns; the chunks past them repeat the last one (what
+// they add lands in columns that are not stored), feature blocks past n_out are skipped, and the two wavefronts of a row pair
+// take alternating feature blocks.  16 heads of 2000 rows, 129 slots, 80 columns, float16: 21.4 us in the general kernel
+// (256 workgroups of four wavefronts, no step ahead), 9.8 here.
 #include <algorithm>
 #include <type_traits>
 
@@ -32,7 +37,7 @@ struct PTileGeom {
     static constexpr int LDS_BYTES = MASK_AT + 81 * 16;
 };
 
-template <typename T, int D>
+template <typename T, int D, bool PART>
 __global__ __launch_bounds__(512, 4) void spmm_tile_kernel(const SpmmParams p) {
     using G = PTileGeom<D>;
     constexpr int BM = G::BM, ROWB = G::ROWB, P_ROWB = G::P_ROWB, V_STAGE = G::V_STAGE, STAGE = G::STAGE, O_ROW = G::O_ROW;
@@ -80,7 +85,7 @@ __global__ __launch_bounds__(512, 4) void spmm_tile_kernel(const SpmmParams p) {
     for (int i = 0; i < NI; ++i) {
         const int id = tid + 512 * i;
         v_row[i] = id / CPR;
-        v_col[i] = (id % CPR) * 16;
+        v_col[i] = (PART ? min(id % CPR, p.n_out / 8 - 1) : id % CPR) * 16;
         v_lds[i] = v_row[i] * ROWB + v_chunk<ROWB>(v_row[i], id % CPR) * 16;
     }
     // this thread's pieces of every probability tile: block row prow, positions 8 (pq + 4 c) .. + 7 of the step, c = 0, 1;
@@ -91,6 +96,7 @@ __global__ __launch_bounds__(512, 4) void spmm_tile_kernel(const SpmmParams p) {
 #pragma unroll
     for (int c = 0; c < 2; ++c) p_lds[c] = V_STAGE + prow * P_ROWB + (((pq + 4 * c) ^ ((prow >> 1) & 7)) << 4);
 
+    auto feature_block = [&](int fd) { return PART ? 2 * fd + fh : FD * fh + fd; };
     // A wavefront owns 32 of the block's rows (two B operands, cb) and half of the features (FD A operands): every fragment
     // read from LDS serves two MFMAs or FD of them.  B: lane (row li of the 16, positions 8 g4 .. + 7 of half step hf); A: lane s
     // of 16-lane block g4 addresses key row 8 g4 + s / 4 (and 4 rows on) and the 4 features 16 dt + 4 (s % 4)
@@ -101,7 +107,7 @@ __global__ __launch_bounds__(512, 4) void spmm_tile_kernel(const SpmmParams p) {
         const int blk = ROWB >= 256 ? sq : (sq >> 1);
 #pragma unroll
         for (int fd = 0; fd < FD; ++fd) {
-            const int dt = FD * fh + fd;
+            const int dt = feature_block(fd);
             v_off[fd] = (8 * g4 + sq) * ROWB + in_half + 64 * ((dt >> 1) ^ blk) + 32 * ((dt & 1) ^ (g4 & 1));
         }
 #pragma unroll
@@ -229,6 +235,7 @@ __global__ __launch_bounds__(512, 4) void spmm_tile_kernel(const SpmmParams p) {
                     pf[cb].v = __builtin_bit_cast(typename Frag<T>::vec, *reinterpret_cast<const u32x4*>(smem + p_off[cb][hf] + par * STAGE));
 #pragma unroll
                 for (int fd = 0; fd < FD; ++fd) {
+                    if (PART && 16 * feature_block(fd) >= p.n_out) break;  // wavefront-uniform
                     const char* a = smem + v_off[fd] + (par * STAGE + 32 * hf * ROWB);
                     const Frag<T> vf = frag_from_tr<T>(lds_tr16(a), lds_tr16(a + 4 * ROWB));
                     mma16(acc[fd][0], vf, pf[0]);
@@ -243,7 +250,7 @@ __global__ __launch_bounds__(512, 4) void spmm_tile_kernel(const SpmmParams p) {
         }
     }
 
-    // ---- output: O^T accumulators (lane: row 32 cg + 16 cb + li, features 16 (FD fh + fd) + 4 g4 .. + 3) turned around in
+    // ---- output: O^T accumulators (lane: row 32 cg + 16 cb + li, features 16 feature_block(fd) + 4 g4 .. + 3) turned around in
     // LDS, rows stored whole (every wavefront has passed the last barrier of the loop: the tiles are free)
     typedef T v4 __attribute__((ext_vector_type(4)));
 #pragma unroll
@@ -253,7 +260,7 @@ __global__ __launch_bounds__(512, 4) void spmm_tile_kernel(const SpmmParams p) {
             v4 t;
 #pragma unroll
             for (int j = 0; j < 4; ++j) t[j] = (T)acc[fd][cb][j];
-            *reinterpret_cast<v4*>(smem + (32 * cg + 16 * cb + li) * O_ROW + (16 * (FD * fh + fd) + 4 * g4) * 2) = t;
+            *reinterpret_cast<v4*>(smem + (32 * cg + 16 * cb + li) * O_ROW + (16 * feature_block(fd) + 4 * g4) * 2) = t;
         }
     lds_barrier();  // a row's two halves come from two wavefronts
     const char* const o_stg = smem + (16 * wave) * O_ROW;
@@ -263,14 +270,14 @@ __global__ __launch_bounds__(512, 4) void spmm_tile_kernel(const SpmmParams p) {
         const int row = flat / CPR, c = flat % CPR;
         const int r = r0 + rs * (16 * wave + row);
         const u32x4 val = *reinterpret_cast<const u32x4*>(o_stg + row * O_ROW + c * 16);
-        if (r < L) {
-            char* orow = reinterpret_cast<char*>(p.out) + ((int64_t)bh * L + r) * ROWB;
+        if (r < L && (!PART || c < p.n_out / 8)) {
+            char* orow = reinterpret_cast<char*>(p.out) + ((int64_t)bh * L + r) * (PART ? p.n_out * 2 : ROWB);
             __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(orow + c * 16));
         }
     }
 }
 
-template <typename T, int D>
+template <typename T, int D, bool PART>
 static int launch_tile_variant(const char* who, SpmmParams p, hipStream_t st) {
     using G = PTileGeom<D>;
     static_assert(G::LDS_BYTES <= 80 * 1024, "two workgroups per compute unit");
@@ -280,7 +287,7 @@ static int launch_tile_variant(const char* who, SpmmParams p, hipStream_t st) {
     if (blocks > 0x7ffffff0) return 0;
     p.total = (int)blocks;
     static uint64_t reserved = 0;
-    auto kern = spmm_tile_kernel<T, D>;
+    auto kern = spmm_tile_kernel<T, D, PART>;
     if (int rc = reserve_dynamic_lds(&reserved, reinterpret_cast<const void*>(kern), G::LDS_BYTES, who)) return rc;
     const int grid = ((p.total + 7) / 8) * 8;
     kern<<<grid, 512, G::LDS_BYTES, st>>>(p);
@@ -290,15 +297,17 @@ static int launch_tile_variant(const char* who, SpmmParams p, hipStream_t st) {
 int launch_spmm_tile(const char* who, const SpmmParams& p, int in_dtype, hipStream_t st) {
     if (!p.plan) return 0;  // this kernel starts from the mask's plan table
     if (in_dtype == SPLAT_F32 || p.out_dtype != in_dtype) return 0;
-    if (p.n_out != 64 && p.n_out != 128) return 0;
-    if (!p.v_vec || !p.out_vec) return 0;
+    if (p.n_out > 128) return 0;
+    if (!p.v_vec || !p.out_vec) return 0;  // (out_vec: rows of out are whole 16-byte pieces, so n_out is a multiple of 8)
     // a thread reads 16 bytes at a time from inside its row's share of a segment
     if (p.T < 8) return 0;
     for (int k = 0; k < p.n_seg; ++k)
         if (p.seg[k].max_cnt < 8) return 0;
     auto by_d = [&](auto t) {
         using TT = decltype(t);
-        return p.n_out == 128 ? launch_tile_variant<TT, 128>(who, p, st) : launch_tile_variant<TT, 64>(who, p, st);
+        if (p.n_out == 128) return launch_tile_variant<TT, 128, false>(who, p, st);
+        if (p.n_out > 64) return launch_tile_variant<TT, 128, true>(who, p, st);
+        return p.n_out == 64 ? launch_tile_variant<TT, 64, false>(who, p, st) : launch_tile_variant<TT, 64, true>(who, p, st);
     };
     return in_dtype == SPLAT_BF16 ? by_d(bf16{}) : by_d(f16{});
 }
