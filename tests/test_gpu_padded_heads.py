@@ -92,3 +92,12 @@ def test_padding_meets_no_infinity(dev, d):
     got = out.cpu()
     hit = (cols == 60) & live
     assert bool((got[..., hit] == float("inf")).all()) and bool(torch.isfinite(got[..., live & ~hit]).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("L,d", [(1, 8), (63, 64), (64, 80), (65, 33), (131, 128)])
+@pytest.mark.parametrize("lead", [0, 1, 3])
+def test_transposed_keys_from_any_alignment(dev, L, d, lead, dtype):
+    """K^T whose rows start ``lead`` elements into longer ones, whole pieces and remainders: the copy holds the same bits."""
+    kT = torch.randn(2, 3, d, L + lead, generator=torch.Generator().manual_seed(L + d)).to(dtype).to(dev)[..., lead:]
+    assert torch.equal(A.transpose_keys(kT), kT.transpose(2, 3).contiguous())
