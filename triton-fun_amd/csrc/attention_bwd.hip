@@ -3,7 +3,8 @@
 // With S = scale * Q K^T on the live columns, P = exp(S - lse) (lse: the forward's row statistic), O = P V and the
 // upstream gradient dO:  D = rowsum(dO * O),  dP = dO V^T,  dS = P * (dP - D),
 //     dQ = scale * dS K        dK = scale * dS^T Q        dV = P^T dO.
-// One kernel, four modes (d = 128: dQ, dK, dV, 8 products; d = 64: dQ, dK+dV, 7), built like the forward (attention.hip): a workgroup of 4 wavefronts owns 128 "rows", one
+// One kernel, four modes (d = 128: dQ, dK, dV, 8 products, or in smaller launches dQ here and the rest in attention_bwd_pair.hip, 7;
+// d = 64: dQ, dK+dV, 7), built like the forward (attention.hip): a workgroup of 4 wavefronts owns 128 "rows", one
 // lane one row (two lanes share it), and walks 64-position tiles of the rows' spans as the mask's plan table lists
 // them; per tile two operand tiles X and Y arrive in LDS through the asynchronous copy ring.
 //
@@ -627,6 +628,16 @@ static int run_bwd_keys(const BwdParams& dk, const BwdParams& dv, int d, hipStre
         BwdParams dkv = dk;
         dkv.out2 = dv.out;
         return launch_bwd<T, 64, kBwdDKV>(dkv, st);
+    }
+    if (dk.total <= 1024) {
+        // Launches of at most four row blocks a CU: one walk by pairs of wavefronts (attention_bwd_pair.hip), which puts eight
+        // wavefronts on a row block where the two launches below put four.  Training steps, bfloat16: 128 row blocks, window 512:
+        // 82 -> 69 us; 512 blocks, two segments: 128 -> 114; 1024 blocks, window 32: 135 -> 133.  Beyond, the beginnings and ends
+        // of its workgroups, which nothing else on the CU covers, cost what the fifth product does: 2048 blocks, window 128:
+        // 279 against 295 us, window 512: 491 against 491; 4096 blocks, dilated 512 / 2: 986 against 972.
+        BwdParams dkv = dk;
+        dkv.out2 = dv.out;
+        return launch_bwd_pair<T>(dkv, st);
     }
     if (int rc = launch_bwd<T, 128, kBwdDK>(dk, st)) return rc;
     return launch_bwd<T, 128, kBwdDV>(dv, st);

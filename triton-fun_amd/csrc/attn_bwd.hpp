@@ -27,6 +27,10 @@ struct BwdParams {
     const PlanRec* plan;  // plan table of the mask (dQ) or of its transpose (dK, dV), first variant
 };
 
+// dK + dV at d = 128, 16-bit types (attention_bwd_pair.hip)
+template <typename T>
+int launch_bwd_pair(const BwdParams& dkv, hipStream_t st);
+
 // float32: dQ (which also computes and stores D), and dK + dV of the rows that `dkv` describes
 int launch_bwd_dq_f32(const BwdParams& dq, int d, hipStream_t st);
 int launch_bwd_dkv_f32(const BwdParams& dkv, int d, hipStream_t st);
