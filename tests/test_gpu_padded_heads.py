@@ -101,3 +101,38 @@ def test_transposed_keys_from_any_alignment(dev, L, d, lead, dtype):
     """K^T whose rows start ``lead`` elements into longer ones, whole pieces and remainders: the copy holds the same bits."""
     kT = torch.randn(2, 3, d, L + lead, generator=torch.Generator().manual_seed(L + d)).to(dtype).to(dev)[..., lead:]
     assert torch.equal(A.transpose_keys(kT), kT.transpose(2, 3).contiguous())
+
+
+@pytest.mark.parametrize("in_place", [False, True])
+@pytest.mark.parametrize("in_dt,out_dt", [(torch.float16, torch.float16), (torch.bfloat16, torch.float32), (torch.float32, torch.bfloat16),
+                                          (torch.float32, torch.float32)])
+@pytest.mark.parametrize("L,T", [(1, 3), (5, 3), (21, 7), (16, 7), (21, 9), (13, 11), (40, 15), (100, 33), (65, 111), (67, 113), (203, 129), (259, 239), (300, 241)])
+def test_softmax_of_rows_at_every_alignment(dev, L, T, in_dt, out_dt, in_place):
+    """Rows of every chunk alignment up to the end of the buffer (the tensors fill their allocation's last chunk or not), with live rows, short ones, empty ones and one that is the type's
+    lowest value throughout, against float64; dead slots keep what they held."""
+    import r_softmax
+    if in_place and in_dt != out_dt:
+        pytest.skip("in place: one type")
+    B, H = 1, 3
+    g = torch.Generator().manual_seed(L + T)
+    counts = torch.full((L,), float(T))
+    counts[torch.rand(L, generator=g) < 0.3] = float(T // 2)
+    counts[3::8], counts[5::11] = 0.0, 1.0
+    x = (2 * torch.randn(B, H, L, T, generator=g)).to(in_dt)
+    x[:, 1, 4 % L] = torch.finfo(in_dt).min
+    live = torch.arange(T)[None, :] < counts[:, None]
+    x = torch.where(live, x, torch.full_like(x, 55.0))
+    want = torch.softmax(x.double().masked_fill(~live, float("-inf")), -1)
+    cnt = counts.to(dev)
+    xd = x.to(dev)
+    out = xd if in_place else torch.full((B, H, L, T), 55.0, dtype=out_dt, device=dev)
+    z = torch.zeros(L, device=dev)
+    r_softmax.rsoftmax_launcher(xd, out, z, z, z, z, T, 256, cnt, (1, 1), 16)
+    got = out.double().cpu()
+    assert torch.all(got[..., ~live] == 55.0)
+    keep = live.expand(B, H, L, T).clone()
+    if in_dt != torch.float16:
+        keep[:, 1, 4 % L] = False  # (a row below the kernel's -1e30 has no defined result; its neighbours do)
+    tol = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 0.0}[out_dt] * 1.01
+    bad = keep & ~((got - want).abs() <= tol * want + 1e-6)
+    assert not bool(bad.any()), [(*i, float(got[tuple(i)]), float(want[tuple(i)])) for i in bad.nonzero().tolist()[:8]]
