@@ -1,5 +1,5 @@
-// Kernel arguments of the SpMM kernels (spmm.hip: every shape; spmm_thin.hip, spmm_tile.hip: 16-bit types, up to 128 output columns; spmm_t_thin.hip: 64 / 128
-// output columns).
+// Kernel arguments of the SpMM kernels (spmm.hip: every shape; spmm_thin.hip: 16-bit types, 64 / 128 output columns; spmm_tile.hip:
+// 16-bit types, up to 128; spmm_t_thin.hip, the transposed product: 64 / 128).
 #pragma once
 #include "acsr_plan.hpp"
 
