@@ -136,3 +136,18 @@ def test_softmax_of_rows_at_every_alignment(dev, L, T, in_dt, out_dt, in_place):
     tol = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 0.0}[out_dt] * 1.01
     bad = keep & ~((got - want).abs() <= tol * want + 1e-6)
     assert not bool(bad.any()), [(*i, float(got[tuple(i)]), float(want[tuple(i)])) for i in bad.nonzero().tolist()[:8]]
+
+
+@pytest.mark.parametrize("d", [8, 64, 80, 96])
+@pytest.mark.parametrize("B,H,L", [(1, 2, 130), (4, 16, 131), (2, 16, 256)])
+def test_operators_with_the_keys_contiguous(dev, d, B, H, L):
+    """K^T stored along the keys, on both sides of the lines at which it is turned first: as with K's rows contiguous, up to the
+    order of the float32 additions (one ulp of the 16-bit scores)."""
+    masks, attn, q, k, v = case(dev, "windowed129", B, H, L, d, torch.float16)
+    outs = []
+    for kT in (k.to(dev).transpose(2, 3), k.to(dev).transpose(2, 3).contiguous()):
+        out = torch.full((B, H, L, attn.acsr_trailing_dim), SENTINEL, dtype=torch.float16, device=dev)
+        r_sddmm.rsddmm_launcher(q.to(dev), kT, out, *[None] * 4, attn.acsr_trailing_dim, None, None, None, None, 16, 16, scale=d ** -0.5,
+                                segments=attn.segments)
+        outs.append(out.double().cpu())
+    assert bool(((outs[0] - outs[1]).abs() <= 2.02 * HALF_ULP[torch.float16] * outs[0].abs() + 1e-5).all())

@@ -384,7 +384,13 @@ PyObject* py_sddmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const double scale = PyFloat_AsDouble(a[4]);
         if (scale == -1.0 && PyErr_Occurred()) return nullptr;
         int rc = 0;
-        if (m->max_step >= 2 && y.stride(3) == 1 && y.stride(2) != 1) {
+        // K^T with the keys contiguous is read in place by the general kernel only.  Up to d = 64 a pass that turns it and the kernel of
+        // thin wavefronts on the copy take less (the three operators, bfloat16: 64 heads of 4096 rows, 33 slots, d = 32: 114 -> 92 us;
+        // 512 slots, d = 64: 300 -> 263; 4 heads of 4001 rows, 301 slots, d = 64: 49 -> 43), beyond it the copy costs as much as it
+        // gives (64 heads of 2048 rows, 255 slots: d = 80 122 -> 125, d = 96 126 -> 129), and so does its launch below 64 row blocks
+        // (one head of 200 rows: 21 -> 25).
+        const bool turned = code != SPLAT_F32 && out_code == code && d % 8 == 0 && d <= 64 && B * H * ((L + 127) / 128) >= 64;
+        if ((m->max_step >= 2 || turned) && y.stride(3) == 1 && y.stride(2) != 1) {
             if (y.stride(2) < keys) Py_RETURN_FALSE;
             y = transposed_keys(y, &rc).transpose(2, 3);
             if (rc) return raise_rc("splat_transpose_keys", rc);
