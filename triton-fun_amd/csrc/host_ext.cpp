@@ -237,6 +237,10 @@ PyObject* py_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
 using torch::autograd::SavedVariable;
 using torch::autograd::variable_list;
 
+// Forward-mode differentiation has no rule here: an output without a tangent would read as a derivative of zero, so such a call
+// is left to the Python function, which refuses it.
+bool has_tangent(const at::Tensor& t) { return t._fw_grad(/*level=*/0).defined(); }
+
 at::Tensor in_pieces(const at::Tensor& t) { return rows_in_pieces(t, 16 / t.element_size()) ? t : t.contiguous(); }
 
 // The gradients of one call.  A node of its own rather than torch::autograd::Function: the engine runs it on its device thread,
@@ -346,7 +350,8 @@ PyObject* py_attend(PyObject*, PyObject* const* a, Py_ssize_t n) {
         if (!q || !k || !v || st->fwd->device != dev) Py_RETURN_NONE;
         const int64_t epc = 16 / q->element_size();
         for (const at::Tensor* t : {q, k, v})
-            if (t->scalar_type() != st->dtype || !is_shape(*t, st->B, st->H, st->L, st->d) || !rows_in_pieces(*t, epc) || t->stride(2) < st->d)
+            if (has_tangent(*t) || t->scalar_type() != st->dtype || !is_shape(*t, st->B, st->H, st->L, st->d) || !rows_in_pieces(*t, epc) ||
+                t->stride(2) < st->d)
                 Py_RETURN_NONE;
         const double scale = PyFloat_AsDouble(a[4]);
         if (scale == -1.0 && PyErr_Occurred()) return nullptr;
