@@ -30,3 +30,21 @@ def test_a_tangent_is_refused_and_not_dropped(dev, which):
             attention_with_grad(*x, attn)
     with forward_ad.dual_level():  # the level alone is nothing to refuse
         assert attention_with_grad(*_operands(dev), attn).grad_fn.name() == "AttendBackward"
+
+
+@pytest.mark.filterwarnings("ignore::torch.jit.TracerWarning", "ignore::DeprecationWarning")
+def test_a_trace_follows_its_inputs(dev):
+    attn = _module(dev)
+    attention_with_grad(*_operands(dev), attn)  # (the plan's kernels are not for the trace)
+    traced = torch.jit.trace(lambda q, k, v: attention_with_grad(q, k, v, attn), tuple(_operands(dev)), check_trace=False)
+    other = [(2 * t).detach().requires_grad_(True) for t in _operands(dev)]
+    assert torch.equal(traced(*other), attention_with_grad(*other, attn))
+
+
+def test_functorch_transforms_get_the_message_that_names_them(dev):
+    attn = _module(dev)
+    q, k, v = _operands(dev)
+    with pytest.raises(RuntimeError, match="functorch transforms"):
+        torch.vmap(lambda a: attention_with_grad(a, k, v, attn))(q[None])
+    with pytest.raises(RuntimeError, match="functorch transforms"):
+        torch.func.grad(lambda a: attention_with_grad(a, k, v, attn).float().sum())(q.detach())

@@ -11,6 +11,7 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/TracerMode.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
@@ -237,9 +238,11 @@ PyObject* py_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
 using torch::autograd::SavedVariable;
 using torch::autograd::variable_list;
 
-// Forward-mode differentiation has no rule here: an output without a tangent would read as a derivative of zero, so such a call
-// is left to the Python function, which refuses it.
-bool has_tangent(const at::Tensor& t) { return t._fw_grad(/*level=*/0).defined(); }
+// What the Python function handles or refuses, and a plain node would get silently or obscurely wrong: wrappers without memory of
+// their own (functorch, fake tensors), and forward-mode tangents (an output without one would read as a derivative of zero).
+bool is_wrapped(const at::Tensor& t) {
+    return !t.has_storage() || t.unsafeGetTensorImpl()->is_python_dispatch() || t._fw_grad(/*level=*/0).defined();
+}
 
 at::Tensor in_pieces(const at::Tensor& t) { return rows_in_pieces(t, 16 / t.element_size()) ? t : t.contiguous(); }
 
@@ -347,10 +350,11 @@ PyObject* py_attend(PyObject*, PyObject* const* a, Py_ssize_t n) {
         if (!st) return nullptr;
         const int dev = c10::hip::current_device();
         const at::Tensor *q = tensor4(a[1], dev), *k = tensor4(a[2], dev), *v = tensor4(a[3], dev);
-        if (!q || !k || !v || st->fwd->device != dev) Py_RETURN_NONE;
+        // (under torch.jit.trace the Python function is recorded as an operation that runs again, a node would be a constant)
+        if (!q || !k || !v || st->fwd->device != dev || at::tracer::impl::is_dispatch_enabled()) Py_RETURN_NONE;
         const int64_t epc = 16 / q->element_size();
         for (const at::Tensor* t : {q, k, v})
-            if (has_tangent(*t) || t->scalar_type() != st->dtype || !is_shape(*t, st->B, st->H, st->L, st->d) || !rows_in_pieces(*t, epc) ||
+            if (is_wrapped(*t) || t->scalar_type() != st->dtype || !is_shape(*t, st->B, st->H, st->L, st->d) || !rows_in_pieces(*t, epc) ||
                 t->stride(2) < st->d)
                 Py_RETURN_NONE;
         const double scale = PyFloat_AsDouble(a[4]);
