@@ -5,6 +5,7 @@ import torch
 import torch.autograd.forward_ad as forward_ad
 
 import acsr_helpers as A
+import _splat_hip as hip
 from r_attention import RegularAttention, attention_with_grad
 
 pytestmark = pytest.mark.gpu
@@ -48,3 +49,9 @@ def test_functorch_transforms_get_the_message_that_names_them(dev):
         torch.vmap(lambda a: attention_with_grad(a, k, v, attn))(q[None])
     with pytest.raises(RuntimeError, match="functorch transforms"):
         torch.func.grad(lambda a: attention_with_grad(a, k, v, attn).float().sum())(q.detach())
+
+
+def test_a_scale_the_kernels_refuse_is_a_splat_error(dev):
+    attn = _module(dev, scale=-1.0)
+    with pytest.raises(hip.SplatError, match=r"^splat_attention_fwd_stats failed \(code -5\): .*scale must be > 0"):
+        attention_with_grad(*_operands(dev), attn)

@@ -15,6 +15,7 @@
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -24,6 +25,8 @@
 #include <algorithm>
 #include <cstring>
 #include <mutex>
+#include <stdexcept>
+#include <string>
 #include <vector>
 
 #include "../../include/splat_hip.h"
@@ -123,6 +126,19 @@ c10::intrusive_ptr<H> held(PyObject* cap, const char* name) {
     return p ? c10::intrusive_ptr<H>::reclaim_copy(p) : c10::intrusive_ptr<H>();
 }
 Mask* mask_of(PyObject* cap) { return static_cast<Mask*>(PyCapsule_GetPointer(cap, kMaskName)); }
+
+// A call of the library that failed: SplatError in the program, as from the Python launchers.
+struct Failure : std::runtime_error {
+    using std::runtime_error::runtime_error;
+};
+// The same from the autograd engine's thread: the engine carries a persisted Python error over to the thread that called backward.
+[[noreturn]] void raise_on_engine_thread(const std::string& what) {
+    pybind11::gil_scoped_acquire gil;
+    PyErr_SetString(g_error, what.c_str());
+    python_error e;
+    e.persist();
+    throw e;
+}
 
 // A 4-dimensional device tensor on the current device, or null.
 const at::Tensor* tensor4(PyObject* o, int device) {
@@ -283,7 +299,7 @@ struct AttendBackward : public torch::autograd::Node {
         m.plan_ptr(), m.plan_bytes(), mt.segs, mt.n_seg, mt.plan_ptr(), mt.plan_bytes(), B, H, L, d, scale
         int rc = code == SPLAT_F32 ? api.bwd_f32(SPLAT_ARGS, stream) : api.bwd(SPLAT_ARGS, code, stream);
 #undef SPLAT_ARGS
-        TORCH_CHECK(rc == 0, failure("splat_attention_bwd", rc));
+        if (rc) raise_on_engine_thread(failure("splat_attention_bwd", rc));
         if (st.rows) {  // the row-sparse segments of the transposed mask, row by row, onto what the others gave
             const Mask& r = *st.rows;
             at::Tensor part = fresh({2, B, H, r.rows, d}, st.dtype);
@@ -297,13 +313,13 @@ struct AttendBackward : public torch::autograd::Node {
             else
                 rc = api.bwd_keys(SPLAT_ARGS, code, dk.data_ptr(), dv.data_ptr(), st.per_stretch, stream);
 #undef SPLAT_ARGS
-            TORCH_CHECK(rc == 0, failure("splat_attention_bwd_keys", rc));
+            if (rc) raise_on_engine_thread(failure("splat_attention_bwd_keys", rc));
         }
         return {dq, dk, dv};
     }
 };
 
-// The output, with the node that gives the gradients as its history.
+// The output, with the node that gives the gradients as its history; undefined when the forward leaves the case to the launcher.
 at::Tensor attend(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const c10::intrusive_ptr<GradState>& st, double scale) {
     at::Tensor out, lse;
     {
@@ -312,7 +328,8 @@ at::Tensor attend(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
         lse = fresh({st->B, st->H, st->L}, at::kFloat);
         int rc = 0;
         const Did did = forward(*st->fwd, q, k.transpose(2, 3), v, out, scale, lse.data_ptr<float>(), &rc);
-        TORCH_CHECK(did == Did::kYes, rc ? failure("splat_attention_fwd_stats", rc) : std::string("attention: unusual operands"));
+        if (did == Did::kFailed) throw Failure(failure("splat_attention_fwd_stats", rc));
+        if (did == Did::kNo) return at::Tensor();
     }
     std::shared_ptr<AttendBackward> node(new AttendBackward(), torch::autograd::deleteNode);
     node->set_next_edges(torch::autograd::collect_next_edges(q, k, v));
@@ -359,7 +376,12 @@ PyObject* py_attend(PyObject*, PyObject* const* a, Py_ssize_t n) {
                 Py_RETURN_NONE;
         const double scale = PyFloat_AsDouble(a[4]);
         if (scale == -1.0 && PyErr_Occurred()) return nullptr;
-        return THPVariable_Wrap(attend(*q, *k, *v, st, scale));
+        const at::Tensor out = attend(*q, *k, *v, st, scale);
+        if (!out.defined()) Py_RETURN_NONE;
+        return THPVariable_Wrap(out);
+    } catch (const Failure& e) {
+        PyErr_SetString(g_error, e.what());
+        return nullptr;
     } catch (const std::exception& e) {
         return raise_std(e);
     }
