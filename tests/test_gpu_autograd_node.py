@@ -6,7 +6,7 @@ import torch.autograd.forward_ad as forward_ad
 
 import acsr_helpers as A
 import _splat_hip as hip
-from r_attention import RegularAttention, attention_with_grad
+from r_attention import RegularAttention, _AttentionFunction, attention_with_grad
 
 pytestmark = pytest.mark.gpu
 
@@ -55,3 +55,47 @@ def test_a_scale_the_kernels_refuse_is_a_splat_error(dev):
     attn = _module(dev, scale=-1.0)
     with pytest.raises(hip.SplatError, match=r"^splat_attention_fwd_stats failed \(code -5\): .*scale must be > 0"):
         attention_with_grad(*_operands(dev), attn)
+
+
+def _gradients(f, x):
+    out = f(*x)
+    return [out, *torch.autograd.grad(out, x, torch.linspace(-1, 1, out.numel(), device=out.device).view(out.shape).to(out.dtype))]
+
+
+def test_saved_tensor_hooks_see_what_the_python_function_saves(dev):
+    """The same tensors in the same order go through the hooks, and what they hand back is what the backward reads."""
+    attn, x = _module(dev), _operands(dev)
+    want = _gradients(lambda q, k, v: attention_with_grad(q, k, v, attn), x)
+    seen = {}
+    for name, f in (("node", attention_with_grad), ("function", _AttentionFunction.apply)):
+        packed = seen[name] = []
+
+        def pack(t):
+            packed.append((t.dtype, tuple(t.shape)))
+            return t.cpu()
+        with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.to(dev)):
+            got = _gradients(lambda q, k, v: f(q, k, v, attn), x)
+        assert all(torch.equal(a, b) for a, b in zip(got, want)), name
+    assert seen["node"] == seen["function"] and len(seen["node"]) == 5
+
+
+@pytest.mark.parametrize("swap", [lambda t: t.float() if t.dim() == 4 else t, lambda t: t[:, :, :-1], lambda t: t.cpu(),
+                                  lambda t: t.double() if t.dim() == 3 else t])
+def test_a_saved_tensor_that_came_back_as_another_is_refused(dev, swap):
+    attn, x = _module(dev), _operands(dev)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, swap):
+        out = attention_with_grad(*x, attn)
+        with pytest.raises(hip.SplatError, match="came back with another type, shape or device"):
+            torch.autograd.grad(out.sum(), x)
+
+
+def test_a_saved_tensor_that_came_back_on_odd_rows_is_copied(dev):
+    attn, x = _module(dev), _operands(dev)
+    want = _gradients(lambda q, k, v: attention_with_grad(q, k, v, attn), x)
+
+    def odd(t):
+        wide = torch.empty(*t.shape[:-1], t.shape[-1] + 1, dtype=t.dtype, device=t.device)[..., 1:]
+        return wide.copy_(t)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, odd):
+        got = _gradients(lambda q, k, v: attention_with_grad(q, k, v, attn), x)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))

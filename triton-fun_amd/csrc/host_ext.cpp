@@ -267,24 +267,36 @@ at::Tensor in_pieces(const at::Tensor& t) { return rows_in_pieces(t, 16 / t.elem
 // dispatch through the autograd keys for every workspace) took longer than the launches (B = 2, H = 4, L = 777, d = 64, float16:
 // 74 us a step, here 62).
 struct AttendBackward : public torch::autograd::Node {
-    SavedVariable q_, k_, v_, out_;
-    at::Tensor lse_;
+    SavedVariable q_, k_, v_, lse_, out_;
     c10::intrusive_ptr<GradState> state;
     float scale = 1.f;
 
     std::string name() const override { return "AttendBackward"; }
     void release_variables() override {
         std::lock_guard<std::mutex> lock(mutex_);
-        q_.reset_data(), k_.reset_data(), v_.reset_data(), out_.reset_data();
-        lse_.reset();
+        q_.reset_data(), k_.reset_data(), v_.reset_data(), lse_.reset_data(), out_.reset_data();
+    }
+    // A saved tensor as the kernels read it.  Hooks of the program may have packed it and unpacked another one: what would be read
+    // out of bounds is refused, rows that are not whole pieces are copied.
+    at::Tensor checked(const char* name, const at::Tensor& t) const {
+        const GradState& st = *state;
+        if (!t.defined() || !t.is_cuda() || t.layout() != at::kStrided || t.get_device() != st.fwd->device || t.scalar_type() != st.dtype ||
+            t.dim() != 4 || !is_shape(t, st.B, st.H, st.L, st.d))
+            raise_on_engine_thread(std::string("the saved tensor ") + name + " came back with another type, shape or device");
+        return in_pieces(t);
     }
     variable_list apply(variable_list&& grads) override {
         std::lock_guard<std::mutex> lock(mutex_);
         if (!grads[0].defined()) return variable_list(3);
-        const at::Tensor q = q_.unpack(), k = k_.unpack(), v = v_.unpack(), out = out_.unpack(shared_from_this());
-        const at::Tensor &lse = lse_, &grad = grads[0];
+        const at::Tensor q0 = q_.unpack(), k0 = k_.unpack(), v0 = v_.unpack(), lse0 = lse_.unpack(), out0 = out_.unpack(shared_from_this());
+        const at::Tensor& grad = grads[0];
         at::AutoDispatchBelowADInplaceOrView below;
         const GradState& st = *state;
+        const at::Tensor q = checked("q", q0), k = checked("k", k0), v = checked("v", v0), out = checked("out", out0);
+        if (!lse0.defined() || !lse0.is_cuda() || lse0.get_device() != st.fwd->device || lse0.scalar_type() != at::kFloat ||
+            lse0.sizes() != at::IntArrayRef({st.B, st.H, st.L}))
+            raise_on_engine_thread("the saved row statistic came back with another type, shape or device");
+        const at::Tensor lse = lse0.contiguous();
         const at::Tensor g = in_pieces(grad.scalar_type() == st.dtype ? grad : grad.to(st.dtype));
         const int64_t B = st.B, H = st.H, L = st.L, d = st.d;
         const int code = dtype_code(st.dtype);
@@ -334,9 +346,10 @@ at::Tensor attend(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
     std::shared_ptr<AttendBackward> node(new AttendBackward(), torch::autograd::deleteNode);
     node->set_next_edges(torch::autograd::collect_next_edges(q, k, v));
     torch::autograd::set_history(out, node);
+    // (the order of the Python function's save_for_backward, which saved-tensor hooks see)
     node->q_ = SavedVariable(q, false), node->k_ = SavedVariable(k, false), node->v_ = SavedVariable(v, false);
-    node->out_ = SavedVariable(out, true);
-    node->lse_ = lse, node->state = st, node->scale = (float)scale;
+    node->lse_ = SavedVariable(lse, false), node->out_ = SavedVariable(out, true);
+    node->state = st, node->scale = (float)scale;
     return out;
 }
 
