@@ -99,3 +99,19 @@ def test_a_saved_tensor_that_came_back_on_odd_rows_is_copied(dev):
     with torch.autograd.graph.saved_tensors_hooks(lambda t: t, odd):
         got = _gradients(lambda q, k, v: attention_with_grad(q, k, v, attn), x)
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+class _NoGradient(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x):
+        return x.clone()
+
+    @staticmethod
+    def backward(ctx, grad):
+        return None
+
+
+def test_zeros_where_no_gradient_arrives(dev):
+    attn, x = _module(dev), _operands(dev)
+    got = torch.autograd.grad(_NoGradient.apply(attention_with_grad(*x, attn)).sum(), x)
+    assert all(g.shape == t.shape and not g.any() for g, t in zip(got, x))

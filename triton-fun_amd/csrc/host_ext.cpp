@@ -287,7 +287,6 @@ struct AttendBackward : public torch::autograd::Node {
     }
     variable_list apply(variable_list&& grads) override {
         std::lock_guard<std::mutex> lock(mutex_);
-        if (!grads[0].defined()) return variable_list(3);
         const at::Tensor q0 = q_.unpack(), k0 = k_.unpack(), v0 = v_.unpack(), lse0 = lse_.unpack(), out0 = out_.unpack(shared_from_this());
         const at::Tensor& grad = grads[0];
         at::AutoDispatchBelowADInplaceOrView below;
@@ -297,8 +296,11 @@ struct AttendBackward : public torch::autograd::Node {
             lse0.sizes() != at::IntArrayRef({st.B, st.H, st.L}))
             raise_on_engine_thread("the saved row statistic came back with another type, shape or device");
         const at::Tensor lse = lse0.contiguous();
-        const at::Tensor g = in_pieces(grad.scalar_type() == st.dtype ? grad : grad.to(st.dtype));
         const int64_t B = st.B, H = st.H, L = st.L, d = st.d;
+        // (no gradient arrived: zeros, as the Python function gets them)
+        const at::Tensor g = !grad.defined()                  ? at::zeros({B, H, L, d}, q.options())
+                             : grad.scalar_type() == st.dtype ? in_pieces(grad)
+                                                              : in_pieces(grad.to(st.dtype));
         const int code = dtype_code(st.dtype);
         at::Tensor dq = fresh({B, H, L, d}, st.dtype), dk = fresh({B, H, L, d}, st.dtype), dv = fresh({B, H, L, d}, st.dtype);
         at::Tensor delta = fresh({B, H, L}, at::kFloat);
