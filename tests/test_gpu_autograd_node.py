@@ -115,3 +115,18 @@ def test_zeros_where_no_gradient_arrives(dev):
     attn, x = _module(dev), _operands(dev)
     got = torch.autograd.grad(_NoGradient.apply(attention_with_grad(*x, attn)).sum(), x)
     assert all(g.shape == t.shape and not g.any() for g, t in zip(got, x))
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 64), (torch.float16, 128), (torch.float32, 64), (torch.bfloat16, 80)])
+@pytest.mark.parametrize("dims", [(2,), (0, 1), (0, 1, 2), (3,)])
+def test_gradients_of_sums_arrive_with_strides_of_zero(dev, dtype, d, dims):
+    """The gradient of a sum is one tensor expanded along the summed dimensions: the same as its copy in memory."""
+    attn = RegularAttention(B, L, H, d, A.causal_windowed_pattern(L, 70), 16, 16, dev, dtype, scale=d ** -0.5)
+    g = torch.Generator(device="cpu").manual_seed(6)
+    x = [torch.randn(B, H, L, d, generator=g).to(dtype).to(dev).requires_grad_(True) for _ in range(3)]
+    up = torch.randn(B, H, L, d, generator=g).to(dtype).to(dev).sum(dim=dims, keepdim=True)
+    for f in (attention_with_grad, _AttentionFunction.apply):
+        out = f(*x, attn)
+        got = torch.autograd.grad(out.sum(dim=dims, keepdim=True), x, up, retain_graph=True)
+        want = torch.autograd.grad(out, x, up.expand_as(out).contiguous())
+        assert all(torch.equal(a, b) for a, b in zip(got, want))

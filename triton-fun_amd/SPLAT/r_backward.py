@@ -183,7 +183,8 @@ def attention_backward(q: torch.Tensor, kT: torch.Tensor, v: torch.Tensor, grad_
     k = kT.transpose(2, 3)
     if k.stride(3) != 1:
         k = k.contiguous()
-    grad_out = grad_out.contiguous() if grad_out.stride(3) != 1 else grad_out
+    if grad_out.stride(3) != 1 or grad_out.stride(2) < d:  # (the gradient of a sum over the rows has row stride 0)
+        grad_out = grad_out.contiguous()
     T = segments.T
     probs = torch.empty((B, H, L, T), dtype=dt, device=dev)
     _sddmm(q, kT, probs, segments, scale, lse)
@@ -328,7 +329,8 @@ def attention_backward_fused(q: torch.Tensor, kT: torch.Tensor, v: torch.Tensor,
         _hip.require_device_tensor(t, name)
         if t.dtype != dt or tuple(t.shape) != (B, H, L, d):
             raise _hip.SplatError(f"{name} must be a {dt} tensor of shape {(B, H, L, d)}, got {t.dtype} {tuple(t.shape)}")
-        if t.stride(3) != 1 or t.data_ptr() % 16 != 0 or any(t.stride(i) % epc != 0 for i in (0, 1, 2)):
+        # (rows apart from each other too: the gradient of a sum over the rows has row stride 0)
+        if t.stride(3) != 1 or t.stride(2) < d or t.data_ptr() % 16 != 0 or any(t.stride(i) % epc != 0 for i in (0, 1, 2)):
             t = t.contiguous()
         return t
     q, k, v, out, grad_out = rows(q, "q"), rows(k, "k"), rows(v, "v"), rows(out, "out"), rows(grad_out, "grad_out")

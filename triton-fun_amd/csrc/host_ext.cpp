@@ -260,7 +260,11 @@ bool is_wrapped(const at::Tensor& t) {
     return !t.has_storage() || t.unsafeGetTensorImpl()->is_python_dispatch() || t._fw_grad(/*level=*/0).defined();
 }
 
-at::Tensor in_pieces(const at::Tensor& t) { return rows_in_pieces(t, 16 / t.element_size()) ? t : t.contiguous(); }
+// t itself where the kernels can read it (rows apart from each other: not the gradient of a sum over the rows, whose row stride is
+// 0), else a copy
+at::Tensor in_pieces(const at::Tensor& t) {
+    return rows_in_pieces(t, 16 / t.element_size()) && t.stride(2) >= t.size(3) ? t : t.contiguous();
+}
 
 // The gradients of one call.  A node of its own rather than torch::autograd::Function: the engine runs it on its device thread,
 // and what the generic one does there around two launches (a dictionary of saved values, an output saved with its history, a
