@@ -162,3 +162,34 @@ def test_product_does_not_import_the_oracle():
             if f.endswith((".py", ".hip", ".hpp", ".cpp", ".h")):
                 text = open(os.path.join(base, f)).read()
                 assert "oracle" not in text, os.path.join(base, f)
+
+
+def test_the_plans_alignment_is_not_looked_at_under_stream_capture(monkeypatch):
+    """The look reads the table back, which waits for the stream: under capture it is left out, with a plan that an earlier
+    launcher call built as without one, and SpMM takes the launch for one without a table; outside it is made once."""
+    import r_spmm
+    from acsr_helpers import ACSRSegments
+    L, T = 200, 300
+    looks = []
+
+    class Table(torch.Tensor):
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            looks.append(func)
+            return super().__torch_function__(func, types, args, kwargs or {})
+    n_rb = -(-L // 128)
+    table = torch.zeros(2 * n_rb * (5 + 128) * 16, dtype=torch.uint8).as_subclass(Table)
+    segs = ACSRSegments([(None,) * 5 + (T, None, None)], [None])
+    monkeypatch.setattr(hip, "resolve_device", lambda d: torch.device("cuda", 0))
+    capturing = True
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
+    x, out = torch.empty(1, 1, L, T, dtype=torch.bfloat16), torch.empty(1, 1, L, 64, dtype=torch.bfloat16)
+    assert segs.plan_is_aligned(L, 0) is None and not r_spmm._takes_a_plan(x, out, 64, segs)
+    segs.splat_plans = {(L, 1, (0,), 0): [table, None]}
+    looks.clear()
+    assert segs.plan_is_aligned(L, 0) is None and not r_spmm._takes_a_plan(x, out, 64, segs) and not looks
+    capturing = False
+    assert segs.plan_is_aligned(L, 0) is True and looks
+    capturing = True
+    looks.clear()
+    assert segs.plan_is_aligned(L, 0) is True and not looks

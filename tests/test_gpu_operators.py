@@ -381,6 +381,44 @@ def test_the_unfused_launchers_under_stream_capture(dev):
         assert float((got.float().cpu() - want).abs().max()) <= 2 * TOL[torch.bfloat16]
 
 
+@pytest.mark.parametrize("width", [255, 100])
+def test_spmm_captured_first_after_another_operator_built_the_plan(dev, width):
+    """SpMM's first call of all is the captured one, the plan is there already (SDDMM built it): nothing is read back while
+    capturing, and every replay equals the eager call up to the order of the additions."""
+    L, d, B, H = 1024, 64, 4, 4
+    acsr = A.create_acsr(O.create_causal_windowed_mask(L, width), 16, dev)
+    T = acsr[5]
+    q, k, v = O.make_inputs(48, B, H, L, d, torch.bfloat16)
+    qd, kT, vd = q.to(dev), k.to(dev).transpose(2, 3), v.to(dev)
+    scores = torch.full((B, H, L, T), SENTINEL, dtype=torch.bfloat16, device=dev)
+    o = torch.zeros(B, H, L, d, dtype=torch.bfloat16, device=dev)
+    r_sddmm.rsddmm_launcher(qd, kT, scores, acsr[0], acsr[1], acsr[2], acsr[3], T, acsr[4], (1, 1), None, None, 16, 16, scale=d ** -0.5)
+    r_softmax.rsoftmax_launcher(scores, scores, acsr[0], acsr[1], acsr[2], acsr[3], T, 256, acsr[4], (1, 1), 16)
+    assert hasattr(acsr[3], "splat_plans")
+
+    def run():
+        r_spmm.rspmm_launcher(scores, vd, o, acsr[0], acsr[1], acsr[2], acsr[3], acsr[6], acsr[7], T, acsr[4], (1, 1, 1), 16, 16)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream(device=dev)
+    side.wait_stream(torch.cuda.current_stream(dev))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side):
+        with torch.cuda.graph(graph, stream=side):
+            run()
+    torch.cuda.current_stream(dev).wait_stream(side)
+    got = []
+    for _ in range(3):
+        o.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        got.append(o.clone())
+        run()
+    want = o.float()
+    # the two kernels add float32 in another order and round once: at most one ulp apart, 2^-7 of a value
+    for g in got:
+        assert float((g.float() - want).abs().max()) <= 2 ** -7 * float(want.abs().max())
+
+
 def test_sddmm_two_aligned_segments_in_a_launch_of_many_row_blocks(dev):
     """Two segments per row whose slots both start on 16-byte boundaries (local window 384 + every 8th earlier column: the
     second segment's slots start at offset 384 of a row of 464): the thin-wavefront kernel walks one segment after the

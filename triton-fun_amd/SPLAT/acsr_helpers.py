@@ -497,15 +497,20 @@ class ACSRSegments:
         holder = self._plan_holder if self._plan_holder is not None else self
         return (int(L), len(self), tuple(self.offsets), dev.index) in getattr(holder, "splat_plans", {})
 
-    def plan_is_aligned(self, L: int, device) -> bool:
+    def plan_is_aligned(self, L: int, device) -> bool | None:
         """Whether every live row starts on a multiple of 8 positions of its block's walk in the plan for ``L`` rows (blocked
         masks): one look at the rows' records of the first variant (gathered walks), which follow its 5 records per block
-        and segment: [lo, cnt, lin, phase] each."""
+        and segment: [lo, cnt, lin, phase] each.  The first look waits for the stream, so under stream capture a plan that has
+        not been looked at is left alone: None."""
+        if torch.cuda.is_current_stream_capturing() and not self.has_plan(L, device):
+            return None
         table = self.plan(L, device)
         holder = self._plan_holder if self._plan_holder is not None else self
         dev = _hip.resolve_device(device)
         entry = holder.splat_plans[(int(L), len(self), tuple(self.offsets), dev.index)]
         if entry[1] is None:
+            if torch.cuda.is_current_stream_capturing():
+                return None
             n_rb = table.numel() // (2 * len(self) * (5 + 128) * 16)
             recs = table.view(torch.int32).view(-1, 4)
             rows = recs[n_rb * len(self) * 5:n_rb * len(self) * (5 + 128)]

@@ -18,6 +18,15 @@ from r_sddmm import live_slot_columns
 _HALF = (torch.float16, torch.bfloat16)
 
 
+def _takes_a_plan(x, output, n_out: int, segs: ACSRSegments) -> bool:
+    """Whether this launch is faster with the mask's plan table: 16-bit types, a multiple of 8 output columns up to 128, and
+    not rows of at least 256 slots that all start on a multiple of 8 positions (blocked masks with large blocks).  What is not
+    known (under stream capture, before any eager call has looked) counts as such rows: the general kernel needs no table."""
+    if x.dtype not in _HALF or output.dtype != x.dtype or n_out % 8 != 0 or n_out > 128:
+        return False
+    return x.shape[3] < 256 or segs.plan_is_aligned(x.shape[2], x.device) is False
+
+
 def rspmm_preamble(mask, output_shape: tuple[int], BLOCK_SIZE_X: int, BLOCK_SIZE_Y: int, GPU_ID: Any,
                    output_dtype: torch.dtype) -> tuple[torch.Tensor, tuple[int], int]:
     """-> (output [B, H, L, n] uninitialised, grid_dim = (ceil(n / BSX), ceil(L / BSY), B*H), T = max row nnz)."""
@@ -63,18 +72,14 @@ def rspmm_launcher(x: torch.Tensor, y: torch.Tensor, output: torch.Tensor,
                                            sTod_linear_transformations, sTod_translations, nnzs, acsr_trailing_dim)
     vs = y.stride()
     dev = x.device
+    tabled = plan is None and _takes_a_plan(x, output, n_out, segs)
     if plan is None:
-        capturing = torch.cuda.is_current_stream_capturing()
-        tabled = x.dtype in _HALF and output.dtype == x.dtype and n_out % 8 == 0 and n_out <= 128 \
-            and not (T >= 256 and (segs.has_plan(L, dev) or not capturing) and segs.plan_is_aligned(L, dev))
         mask = segs.native(L, dev, tabled)
         if mask is not None and _hip.host().spmm(mask, x, y, output):
             return (output, sTod_linear_transformations, sTod_translations, nnzs)
     arr = segs.seg_array(L, T)
-    if plan is None and x.dtype in (torch.float16, torch.bfloat16) and output.dtype == x.dtype and n_out % 8 == 0 and n_out <= 128 \
-            and (segs.has_plan(L, dev) or not torch.cuda.is_current_stream_capturing()) \
-            and not (T >= 256 and segs.plan_is_aligned(L, dev)):  # (no table is built under stream capture: building synchronises)
-        plan = segs.plan(L, dev)
+    if tabled and (segs.has_plan(L, dev) or not torch.cuda.is_current_stream_capturing()):
+        plan = segs.plan(L, dev)  # (no table is built under stream capture: building synchronises)
     if plan is not None and plan is not False:
         _hip.require_device_tensor(plan, "plan")
         if plan.device != dev:
