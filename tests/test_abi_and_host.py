@@ -193,3 +193,28 @@ def test_the_plans_alignment_is_not_looked_at_under_stream_capture(monkeypatch):
     capturing = True
     looks.clear()
     assert segs.plan_is_aligned(L, 0) is True and not looks
+
+
+def test_metadata_with_native_handles_copies_and_saves(monkeypatch):
+    """The handles that a launcher call leaves with ``sTod_translations`` stay with it: a deep copy and a saved file hold the
+    tensor and its plain attributes, load without executing anything, and are given handles of their own by the next call."""
+    import copy
+    import io
+    from acsr_helpers import ACSRSegments
+    t = torch.arange(4.0)
+    t.splat_row_stride = 1
+    arrays = [torch.zeros(4), torch.zeros(4), torch.ones(4), t, torch.ones(4)]
+    monkeypatch.setattr(hip, "require_device_tensor", lambda *a: None)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+
+    def native(on):
+        return ACSRSegments.single(*arrays[:3], on, arrays[4], 1).native(4, torch.device("cuda", 0), False)
+    handle = native(t)
+    assert type(handle).__name__ == "PyCapsule" and native(t) is handle
+    file = io.BytesIO()
+    torch.save(t, file)
+    file.seek(0)
+    for other in (copy.deepcopy(t), copy.copy(t), torch.load(file, weights_only=True)):
+        assert torch.equal(other, t) and other.splat_row_stride == 1
+        own = native(other)
+        assert type(own).__name__ == "PyCapsule" and (own is not handle or other.data_ptr() == t.data_ptr())

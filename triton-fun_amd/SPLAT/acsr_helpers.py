@@ -13,6 +13,7 @@ Additions that keep the reference behaviour as the default:
 """
 from __future__ import annotations
 
+from collections import OrderedDict
 from dataclasses import dataclass
 from math import ceil
 from typing import Any, Sequence, Type
@@ -422,6 +423,14 @@ def transpose_keys(kT: torch.Tensor) -> torch.Tensor:
     return out
 
 
+class _NativeMasks(dict):
+    """What ``ACSRSegments.native`` has built, by key: handles of this process that point into the metadata's memory.  A copy or a
+    saved file of the tensor that carries them has other memory and gets none (an empty mapping that every loader takes)."""
+
+    def __reduce__(self):
+        return OrderedDict, ()
+
+
 class ACSRSegments:
     """Several disjoint affine segments per row.  Segment k owns compressed slots
     [offsets[k], offsets[k] + T_k); ``T`` is the total trailing dimension."""
@@ -523,8 +532,8 @@ class ACSRSegments:
         (building synchronises).  The metadata is taken to be immutable from then on."""
         holder = self._plan_holder if self._plan_holder is not None else self
         kept = holder.__dict__.get("splat_native")
-        if kept is None:
-            kept = holder.__dict__["splat_native"] = {}
+        if type(kept) is not _NativeMasks:
+            kept = holder.__dict__["splat_native"] = _NativeMasks()
         # (the tensors' addresses: separate tensors may come with one sTod_translations and other companions)
         key = (L, device.index, with_plan) if holder is self else \
             (L, device.index, with_plan, *(t.data_ptr() for t in self.tuples[0][:5]))
