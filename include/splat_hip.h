@@ -36,7 +36,7 @@
 extern "C" {
 #endif
 
-#define SPLAT_VERSION 1000 /* major*10000 + minor*100 + patch; 0.2.0 added the planned forward, 0.3.0 splat_spmm_t, 0.4.0 splat_attention_fwd_stats, splat_sddmm_probs, 0.5.0 splat_attention_fwd_noalloc, 0.6.0 moved the two measurement aids out (libsplat_bench.so, splat_bench.h), 0.7.0 added splat_sddmm_planned, splat_spmm_planned, 0.8.0 splat_spmm_t_planned, 0.9.0 splat_attention_bwd_keys, 0.10.0 splat_acsr_build_record, splat_attention_bwd_f32, splat_attention_bwd_keys_f32 */
+#define SPLAT_VERSION 1100 /* major*10000 + minor*100 + patch; 0.2.0 added the planned forward, 0.3.0 splat_spmm_t, 0.4.0 splat_attention_fwd_stats, splat_sddmm_probs, 0.5.0 splat_attention_fwd_noalloc, 0.6.0 moved the two measurement aids out (libsplat_bench.so, splat_bench.h), 0.7.0 added splat_sddmm_planned, splat_spmm_planned, 0.8.0 splat_spmm_t_planned, 0.9.0 splat_attention_bwd_keys, 0.10.0 splat_acsr_build_record, splat_attention_bwd_f32, splat_attention_bwd_keys_f32, 0.11.0 gave splat_acsr_build_record's int32 arrays a buffer of their own */
 
 /* element types of q/k/v/score/output buffers */
 #define SPLAT_F32 0
@@ -102,16 +102,17 @@ int splat_acsr_build(const uint8_t* mask, int64_t rows, int64_t cols, int64_t ld
                      float* sTod_trans, float* nnz, float* span_start, float* span_end,
                      int32_t* row_first, int32_t* row_last, int32_t* summary, void* stream);
 
-/* The same build in one kernel, for callers that wait for it: the arrays in one buffer, the summary in shares.
- *   record   device: dTos_lin, dTos_trans, sTod_lin, sTod_trans, nnz (float32), row_first, row_last (int32), each starting a
- *            multiple of 64 elements (rows rounded up to one) after the one before, then span_start, span_end (float32),
- *            ceil(rows/block_height) rounded up to a multiple of 64 elements each
- *   twin     0, or the distance in 4-byte elements to a duplicate of the record, written as well
- *   shares   [ceil(rows/block_height)][8] int32, device-accessible memory that the host can read (pinned): per row block
- *            the five figures of `summary` above, in its order, over the block's rows alone; complete once the stream
- *            has been waited for */
-int splat_acsr_build_record(const uint8_t* mask, int64_t rows, int64_t cols, int64_t ld, int32_t block_height, void* record,
-                            int64_t twin, int32_t* shares, void* stream);
+/* The same build in one kernel, for callers that wait for it: the arrays in two buffers, the summary in shares.
+ *   record    device: dTos_lin, dTos_trans, sTod_lin, sTod_trans, nnz, each starting rows rounded up to a multiple of 64
+ *             elements after the one before, then span_start, span_end, ceil(rows/block_height) rounded up to a multiple
+ *             of 64 elements each
+ *   extents   device: row_first, row_last, with the rows' distance
+ *   duplicate not 0: both buffers are twice as long and the same arrays are written again behind the first ones
+ *   shares    [ceil(rows/block_height)][8] int32, device-accessible memory that the host can read (pinned): per row block
+ *             the five figures of `summary` above, in its order, over the block's rows alone; complete once the stream
+ *             has been waited for */
+int splat_acsr_build_record(const uint8_t* mask, int64_t rows, int64_t cols, int64_t ld, int32_t block_height, float* record,
+                            int32_t* extents, int32_t duplicate, int32_t* shares, void* stream);
 
 /* Fill a rows x cols byte mask (row pitch ld) with one of the SPLAT_MASK_* patterns.
  * Device-side equivalent of the O(s^2) Python loops at acsr_helpers.py:18-55. */

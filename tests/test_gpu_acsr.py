@@ -244,3 +244,23 @@ def test_mask_tensors_of_any_pitch_in_one_kernel(dev, rows, cols, pitch, offset,
     assert np.array_equal(A.row_extents(mask, dev)[1].cpu().numpy(), O.row_extents(mask.cpu().numpy())[1])
     got[0].fill_(7.0)
     check_acsr(mask, BH, dev)
+
+
+def test_the_returned_metadata_saves_and_copies(dev):
+    """Every tensor of a build by the one-kernel path, alone and all together, with the attributes the launchers read, through
+    torch.save (which takes no tensors of two types on one storage) and copy.deepcopy."""
+    import copy
+    import io
+    mask = torch.from_numpy(np.asarray(O.create_causal_windowed_mask(300, 70), dtype=np.uint8)).to(dev)
+    acsr = A.create_acsr(mask, 16, dev)
+    tensors = [t for t in acsr if isinstance(t, torch.Tensor)]
+
+    def through_file(x):
+        f = io.BytesIO()
+        torch.save(x, f)
+        f.seek(0)
+        return torch.load(f, weights_only=True)
+    for t, got, twin in zip(tensors, through_file(tensors), copy.deepcopy(tensors)):
+        assert torch.equal(got, t) and torch.equal(twin, t) and torch.equal(through_file(t), t)
+    for other in (through_file(acsr[3]), copy.deepcopy(acsr[3])):
+        assert torch.equal(other.splat_first_col, acsr[3].splat_first_col) and other.splat_max_step == acsr[3].splat_max_step

@@ -46,7 +46,7 @@ _SIGNATURES = {
     "splat_version": (ctypes.c_int, []),
     "splat_last_error": (ctypes.c_char_p, []),
     "splat_acsr_build": (ctypes.c_int, [_vp, _i64, _i64, _i64, _i32] + [_vp] * 10 + [_vp]),
-    "splat_acsr_build_record": (ctypes.c_int, [_vp, _i64, _i64, _i64, _i32, _vp, _i64, _vp, _vp]),
+    "splat_acsr_build_record": (ctypes.c_int, [_vp, _i64, _i64, _i64, _i32, _vp, _vp, _i32, _vp, _vp]),
     "splat_mask_generate": (ctypes.c_int, [_vp, _i64, _i64, _i64, _i32, _i64, _i64, _vp]),
     "splat_acsr_build_pattern": (ctypes.c_int, [_i32, _i64, _i64, _i64, _i32] + [_vp] * 10 + [_vp]),
     "splat_sddmm": (ctypes.c_int, [_vp, _i64, _i64, _i64, _vp, _i64, _i64, _i64, _i64, _vp, ctypes.POINTER(AcsrSeg), _i32,

@@ -293,8 +293,8 @@ def _checked_summary(b: AcsrBuild, t_max: int, failed: int, step_min: int, step_
 
 def _build_and_wait(entry: _MaskEntry, dm: torch.Tensor, BLOCK_HEIGHT: int):
     """The build in one kernel that is waited for, kept with the mask's entry: a duplicate of its arrays for the caller, or
-    None where the native host path leaves the case to ``build_acsr``."""
-    found = None if torch.cuda.is_current_stream_capturing() else _hip.host().build(dm, BLOCK_HEIGHT)
+    None where the native host path leaves the case to ``build_acsr`` (stream capture among them)."""
+    found = _hip.host().build(dm, BLOCK_HEIGHT)
     if found is None:
         return None
     b = AcsrBuild()

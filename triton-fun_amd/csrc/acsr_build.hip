@@ -81,17 +81,20 @@ __device__ __forceinline__ void init_summary(int32_t* summary) {
 }
 constexpr float kUnpackFailed = 0.0f;  // stored as a row's sTod_lin (a real step is >= 1) until the span kernel has counted it
 
-// Where a build's arrays go.  `twin`, when not 0, is the distance in elements from every array to its duplicate: a caller
-// that keeps a build and hands out another copy gets both from one kernel.
+// Where a build's arrays go.  `twin` / `twin_i`, when not 0, are the distances in elements from every float32 / int32 array to its
+// duplicate: a caller that keeps a build and hands out another copy gets both from one kernel.
 struct RowOut {
     float *dTos_lin, *dTos_trans, *sTod_lin, *sTod_trans, *nnz;
     int32_t *row_first, *row_last;
     float *span_start, *span_end;
-    int64_t twin;
-    template <typename T>
-    __device__ __forceinline__ void put(T* p, int i, T x) const {
+    int64_t twin, twin_i;
+    __device__ __forceinline__ void put(float* p, int i, float x) const {
         p[i] = x;
         if (twin) p[i + twin] = x;
+    }
+    __device__ __forceinline__ void put(int32_t* p, int i, int32_t x) const {
+        p[i] = x;
+        if (twin_i) p[i + twin_i] = x;
     }
 };
 
@@ -438,7 +441,7 @@ extern "C" int splat_acsr_build(const uint8_t* mask, int64_t rows, int64_t cols,
     if (rows > (1 << 23) || cols > (1 << 23))
         return fail(SPLAT_E_SHAPE, "splat_acsr_build: rows and cols are limited to 2^23 (got %lld, %lld)", (long long)rows, (long long)cols);
     hipStream_t st = (hipStream_t)stream;
-    const RowOut out{dTos_lin, dTos_trans, sTod_lin, sTod_trans, nnz, row_first, row_last, nullptr, nullptr, 0};
+    const RowOut out{dTos_lin, dTos_trans, sTod_lin, sTod_trans, nnz, row_first, row_last, nullptr, nullptr, 0, 0};
     acsr_rows_kernel<false><<<(unsigned)((rows + kRowWaves - 1) / kRowWaves), 64 * kRowWaves, 0, st>>>(mask, (int)rows, (int)cols, ld,
                                                                                                       kRowWaves, out, summary, nullptr);
     const int n_blocks = (int)((rows + block_height - 1) / block_height);
@@ -447,23 +450,22 @@ extern "C" int splat_acsr_build(const uint8_t* mask, int64_t rows, int64_t cols,
     return check_launch("splat_acsr_build");
 }
 
-extern "C" int splat_acsr_build_record(const uint8_t* mask, int64_t rows, int64_t cols, int64_t ld, int32_t block_height, void* record,
-                                       int64_t twin, int32_t* shares, void* stream) {
+extern "C" int splat_acsr_build_record(const uint8_t* mask, int64_t rows, int64_t cols, int64_t ld, int32_t block_height, float* record,
+                                       int32_t* extents, int32_t duplicate, int32_t* shares, void* stream) {
     begin_launch();
-    if (!mask || !record || !shares) return fail(SPLAT_E_NULL, "splat_acsr_build_record: null pointer argument");
+    if (!mask || !record || !extents || !shares) return fail(SPLAT_E_NULL, "splat_acsr_build_record: null pointer argument");
     if (rows <= 0 || cols <= 0 || ld < cols || block_height <= 0 || rows > (1 << 23) || cols > (1 << 23))
         return fail(SPLAT_E_SHAPE, "splat_acsr_build_record: need 0 < rows, cols <= 2^23, ld >= cols, block_height > 0 (got %lld, %lld, %lld, %d)",
                     (long long)rows, (long long)cols, (long long)ld, block_height);
     const int64_t n_blocks = (rows + block_height - 1) / block_height;
     const int64_t row_step = (rows + 63) & ~(int64_t)63, span_step = (n_blocks + 63) & ~(int64_t)63;
-    if (twin != 0 && twin < 7 * row_step + 2 * span_step)
-        return fail(SPLAT_E_SHAPE, "splat_acsr_build_record: the duplicate at %lld overlaps the record", (long long)twin);
-    if ((reinterpret_cast<uintptr_t>(record) & 3) != 0 || (reinterpret_cast<uintptr_t>(shares) & 15) != 0)
-        return fail(SPLAT_E_ALIGN, "splat_acsr_build_record: misaligned record or shares");
-    float* const f = static_cast<float*>(record);
-    const RowOut out{f, f + row_step, f + 2 * row_step, f + 3 * row_step, f + 4 * row_step,
-                     reinterpret_cast<int32_t*>(f + 5 * row_step), reinterpret_cast<int32_t*>(f + 6 * row_step),
-                     f + 7 * row_step, f + 7 * row_step + span_step, twin};
+    if ((reinterpret_cast<uintptr_t>(record) & 3) != 0 || (reinterpret_cast<uintptr_t>(extents) & 3) != 0 ||
+        (reinterpret_cast<uintptr_t>(shares) & 15) != 0)
+        return fail(SPLAT_E_ALIGN, "splat_acsr_build_record: misaligned record, extents or shares");
+    float* const f = record;
+    const RowOut out{f, f + row_step, f + 2 * row_step, f + 3 * row_step, f + 4 * row_step, extents, extents + row_step,
+                     f + 5 * row_step, f + 5 * row_step + span_step, duplicate ? 5 * row_step + 2 * span_step : 0,
+                     duplicate ? 2 * row_step : 0};
     const int waves = (int)min((int64_t)kRowWaves, min((int64_t)block_height, rows));
     acsr_rows_kernel<true><<<(unsigned)n_blocks, 64 * waves, 0, (hipStream_t)stream>>>(mask, (int)rows, (int)cols, ld, block_height, out,
                                                                                        nullptr, shares);
@@ -493,7 +495,7 @@ extern "C" int splat_acsr_build_pattern(int32_t pattern, int64_t s, int64_t p0, 
     if (int rc = check_pattern(who, s, pattern, p0, p1)) return rc;
     if (p0 > (1 << 23) || p1 > (1 << 23)) return fail(SPLAT_E_SHAPE, "%s: pattern parameters are limited to 2^23", who);
     hipStream_t st = (hipStream_t)stream;
-    const RowOut out{dTos_lin, dTos_trans, sTod_lin, sTod_trans, nnz, row_first, row_last, nullptr, nullptr, 0};
+    const RowOut out{dTos_lin, dTos_trans, sTod_lin, sTod_trans, nnz, row_first, row_last, nullptr, nullptr, 0, 0};
     acsr_rows_pattern_kernel<<<(unsigned)((s + 255) / 256), 256, 0, st>>>(pattern, (int)s, p0, p1, out, summary);
     const int n_blocks = (int)((s + block_height - 1) / block_height);
     acsr_spans_kernel<<<(n_blocks + 255) / 256, 256, 0, st>>>(sTod_lin, sTod_trans, nnz, (int)s, (int)s, block_height, span_start,

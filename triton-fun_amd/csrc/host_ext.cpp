@@ -14,6 +14,7 @@
 #include <ATen/TracerMode.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/function.h>
@@ -549,8 +550,8 @@ ShareBuffers* share_buffers() {
 }
 
 // One array of a record, as a tensor of its own on the record's storage.
-at::Tensor part_of(const at::Tensor& record, int64_t offset, int64_t n, caffe2::TypeMeta type) {
-    at::Tensor t = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(record.storage()), record.key_set(), type);
+at::Tensor part_of(const at::Tensor& record, int64_t offset, int64_t n) {
+    at::Tensor t = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(record.storage()), record.key_set(), record.dtype());
     t.unsafeGetTensorImpl()->set_storage_offset(record.storage_offset() + offset);
     t.unsafeGetTensorImpl()->set_sizes_contiguous({n});
     return t;
@@ -572,13 +573,15 @@ PyObject* py_build(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const int64_t rows = mask.size(0), cols = mask.size(1), blocks = (rows + bh - 1) / bh;
         // the one-kernel build gives a row block to a workgroup: short blocks and very tall ones leave wavefronts or CUs idle
         if (blocks > kShareBlocks || bh < 4 || bh > 64) Py_RETURN_NONE;
+        if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) Py_RETURN_NONE;  // (it waits)
         const auto stream = c10::hip::getCurrentHIPStream(mask.get_device());
-        const int64_t row_step = (rows + 63) / 64 * 64, span_step = (blocks + 63) / 64 * 64, twin = 7 * row_step + 2 * span_step;
-        const at::Tensor kept = fresh({2 * twin}, at::kFloat);
+        const int64_t row_step = (rows + 63) / 64 * 64, span_step = (blocks + 63) / 64 * 64, twin = 5 * row_step + 2 * span_step;
+        // (a storage per type: torch.save takes no tensors of two types on one)
+        const at::Tensor record = fresh({2 * twin}, at::kFloat), extents = fresh({4 * row_step}, at::kInt);
         at::Tensor shares = share_buffers()->take();
         const int32_t* const sh = shares.data_ptr<int32_t>();
-        const int rc = api.build_record(mask.data_ptr<uint8_t>(), rows, cols, mask.stride(0), (int32_t)bh, kept.data_ptr(), twin,
-                                        shares.data_ptr<int32_t>(), stream.stream());
+        const int rc = api.build_record(mask.data_ptr<uint8_t>(), rows, cols, mask.stride(0), (int32_t)bh, record.data_ptr<float>(),
+                                        extents.data_ptr<int32_t>(), 1, shares.data_ptr<int32_t>(), stream.stream());
         if (rc) return raise_rc("splat_acsr_build_record", rc);
         PyThreadState* const released = PyEval_SaveThread();
         std::string failed_wait;
@@ -604,9 +607,14 @@ PyObject* py_build(PyObject*, PyObject* const* a, Py_ssize_t n) {
             sets[k] = PyTuple_New(9);
             if (!sets[k]) return nullptr;
             for (int i = 0; i < 9; ++i) {
-                const int64_t at = k * twin + (i < 7 ? i * row_step : 7 * row_step + (i - 7) * span_step);
-                PyTuple_SET_ITEM(sets[k], i, THPVariable_Wrap(part_of(kept, at, i < 7 ? rows : blocks,
-                                                                      caffe2::TypeMeta::fromScalarType(i == 5 || i == 6 ? at::kInt : at::kFloat))));
+                at::Tensor t;
+                if (i == 5 || i == 6)
+                    t = part_of(extents, (2 * k + i - 5) * row_step, rows);
+                else if (i < 5)
+                    t = part_of(record, k * twin + i * row_step, rows);
+                else
+                    t = part_of(record, k * twin + 5 * row_step + (i - 7) * span_step, blocks);
+                PyTuple_SET_ITEM(sets[k], i, THPVariable_Wrap(std::move(t)));
             }
         }
         return Py_BuildValue("NNiiiii", sets[0], sets[1], t_max, bad, step_min, step_max, off);
