@@ -381,6 +381,34 @@ def test_the_unfused_launchers_under_stream_capture(dev):
         assert float((got.float().cpu() - want).abs().max()) <= 2 * TOL[torch.bfloat16]
 
 
+@pytest.mark.parametrize("dtype,d,heads,L,window,layout,builds", [
+    (torch.float16, 80, 2, 300, 129, "rows", True),      # short rows: the kernel that reads the table
+    (torch.float16, 80, 2, 700, 513, "rows", False),     # few row blocks of long rows: the general kernel
+    (torch.bfloat16, 64, 2, 700, 513, "rows", False),
+    (torch.bfloat16, 32, 44, 700, 513, "rows", True),    # 264 row blocks
+    (torch.bfloat16, 80, 2, 300, 129, "keys", False),    # K^T along the keys is read in place by the general kernel
+    (torch.bfloat16, 64, 2, 300, 129, "keys", False),
+    (torch.bfloat16, 64, 22, 300, 129, "keys", True),    # 66 row blocks: K turned first
+    (torch.float32, 64, 2, 300, 129, "rows", False)])
+def test_sddmm_builds_a_plan_only_for_the_kernel_that_reads_one(dev, dtype, d, heads, L, window, layout, builds):
+    acsr = A.create_acsr(A.windowed_pattern(L, window // 2), 16, dev)
+    T = acsr[5]
+    q, k, _ = O.make_inputs(49, 1, heads, L, d, dtype)
+    kT = k.to(dev).transpose(2, 3)
+    out = torch.zeros(1, heads, L, T, dtype=dtype, device=dev)
+
+    def run(plan):
+        r_sddmm.rsddmm_launcher(q.to(dev), kT.contiguous() if layout == "keys" else kT, out, acsr[0], acsr[1], acsr[2], acsr[3], T,
+                                acsr[4], (1, 1), None, None, 16, 16, scale=d ** -0.5, plan=plan)
+        return out.clone()
+    got = run(None)
+    assert hasattr(acsr[3], "splat_plans") == builds
+    want = run(False)
+    # (the same bits where both read K alike; one ulp where one of them turned it: another order of the float32 sums)
+    ulp = {torch.float16: 2 ** -10, torch.bfloat16: 2 ** -7, torch.float32: 0}[dtype]
+    assert torch.equal(got, want) or float((got.float() - want.float()).abs().max()) <= ulp * float(want.float().abs().max())
+
+
 @pytest.mark.parametrize("width", [255, 100])
 def test_spmm_captured_first_after_another_operator_built_the_plan(dev, width):
     """SpMM's first call of all is the captured one, the plan is there already (SDDMM built it): nothing is read back while
