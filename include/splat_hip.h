@@ -36,7 +36,7 @@
 extern "C" {
 #endif
 
-#define SPLAT_VERSION 1100 /* major*10000 + minor*100 + patch; 0.2.0 added the planned forward, 0.3.0 splat_spmm_t, 0.4.0 splat_attention_fwd_stats, splat_sddmm_probs, 0.5.0 splat_attention_fwd_noalloc, 0.6.0 moved the two measurement aids out (libsplat_bench.so, splat_bench.h), 0.7.0 added splat_sddmm_planned, splat_spmm_planned, 0.8.0 splat_spmm_t_planned, 0.9.0 splat_attention_bwd_keys, 0.10.0 splat_acsr_build_record, splat_attention_bwd_f32, splat_attention_bwd_keys_f32, 0.11.0 gave splat_acsr_build_record's int32 arrays a buffer of their own */
+#define SPLAT_VERSION 1100 /* major*10000 + minor*100 + patch; 0.2.0 added the planned forward, 0.3.0 splat_spmm_t, 0.4.0 splat_attention_fwd_stats, splat_sddmm_probs, 0.5.0 splat_attention_fwd_noalloc, 0.6.0 moved the two measurement aids out (libsplat_bench.so, splat_bench.h), 0.7.0 added splat_sddmm_planned, splat_spmm_planned, 0.8.0 splat_spmm_t_planned, 0.9.0 splat_attention_bwd_keys, 0.10.0 splat_acsr_build_record, splat_attention_bwd_f32, splat_attention_bwd_keys_f32, 0.11.0 gave splat_acsr_build_record's int32 arrays a buffer of their own and added splat_attention_plan_report */
 
 /* element types of q/k/v/score/output buffers */
 #define SPLAT_F32 0
@@ -187,7 +187,7 @@ int splat_spmm(const void* p, const void* v, int64_t v_sb, int64_t v_sh, int64_t
  * rows of at least 256 slots on 16-byte boundaries in compressed matrices of more than 192 MB (64 or 128 columns) through per-row rings of
  * aligned lines, everything else through a workgroup-wide tile: -20 % at B=2 H=32 L=8192 d=128 T=512, -23 % at B=4 H=16 L=4096 d=64 T=256, -40 % on rows
  * of 64 slots; masks of at least 256 slots per row whose rows all start on multiples of 8 positions of their block's walk
- * (blocked masks with large blocks) are better served by splat_spmm (the Python launcher looks that up in the table once
+ * (blocked masks with large blocks) are better served by splat_spmm (the Python launcher learns that from the plan's report
  * and picks).  Other shapes ignore the plan.  Same results as
  * splat_spmm up to the order of the float32 additions.  Replaces the same reference code (rspmm_launcher,
  * r_spmm.py:128-190). */
@@ -219,12 +219,19 @@ int splat_attention_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl,
  *   host-only arithmetic, reads nothing on the device.
  * splat_attention_plan: fill `plan` (device memory, 16-byte aligned, plan_bytes >= the size above); the
  *   work is enqueued on `stream`, and forwards that use the plan must be ordered after it.
+ * splat_attention_plan_report: the same, and per row block four int32 into `report` (device-accessible memory that the host
+ *   can read, 16-byte aligned; as many blocks as plan_bytes / (2*133*16*n_seg)), complete once the stream has been waited
+ *   for: [0] whether some live row starts off a multiple of 8 positions of the block's walk (0 in every block: masks of large
+ *   blocks, for which splat_spmm beats splat_spmm_planned), [1] tiles of 64 positions that the block walks, [2] its
+ *   live positions, [3] 0.
  * splat_attention_fwd_planned: as splat_attention_fwd, with the plan of the same segments and L; results
  *   are bit-identical to splat_attention_fwd.  A plan built from other segments or another L gives
  *   undefined results (only its size is checked). */
 int64_t splat_attention_plan_bytes(const splat_acsr_seg* segs /* host */, int32_t n_seg, int32_t L);
 int splat_attention_plan(const splat_acsr_seg* segs /* host */, int32_t n_seg, int32_t L, void* plan,
                          int64_t plan_bytes, void* stream);
+int splat_attention_plan_report(const splat_acsr_seg* segs /* host */, int32_t n_seg, int32_t L, void* plan,
+                                int64_t plan_bytes, int32_t* report, int64_t report_bytes, void* stream);
 int splat_attention_fwd_planned(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* kT,
                                 int64_t k_sb, int64_t k_sh, int64_t k_sd, int64_t k_sl, const void* v,
                                 int64_t v_sb, int64_t v_sh, int64_t v_sl, void* out, int64_t o_sb,

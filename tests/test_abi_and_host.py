@@ -164,35 +164,35 @@ def test_product_does_not_import_the_oracle():
                 assert "oracle" not in text, os.path.join(base, f)
 
 
-def test_the_plans_alignment_is_not_looked_at_under_stream_capture(monkeypatch):
-    """The look reads the table back, which waits for the stream: under capture it is left out, with a plan that an earlier
-    launcher call built as without one, and SpMM takes the launch for one without a table; outside it is made once."""
+def test_spmm_looks_at_nothing_on_the_device_under_stream_capture(monkeypatch):
+    """Which kernel a launch of long rows takes hangs on the plan's alignment, which comes with the plan's report: under
+    capture it is taken from a plan that is there (SDDMM or the fused forward may have built it), and without one the launch
+    counts as one without a table.  Neither builds a plan nor reads one back: both would wait for the stream."""
     import r_spmm
     from acsr_helpers import ACSRSegments
     L, T = 200, 300
-    looks = []
 
     class Table(torch.Tensor):
         @classmethod
         def __torch_function__(cls, func, types, args=(), kwargs=None):
-            looks.append(func)
-            return super().__torch_function__(func, types, args, kwargs or {})
-    n_rb = -(-L // 128)
-    table = torch.zeros(2 * n_rb * (5 + 128) * 16, dtype=torch.uint8).as_subclass(Table)
+            raise AssertionError(f"{func} on the plan table")
     segs = ACSRSegments([(None,) * 5 + (T, None, None)], [None])
     monkeypatch.setattr(hip, "resolve_device", lambda d: torch.device("cuda", 0))
-    capturing = True
-    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
     x, out = torch.empty(1, 1, L, T, dtype=torch.bfloat16), torch.empty(1, 1, L, 64, dtype=torch.bfloat16)
     assert segs.plan_is_aligned(L, 0) is None and not r_spmm._takes_a_plan(x, out, 64, segs)
-    segs.splat_plans = {(L, 1, (0,), 0): [table, None]}
-    looks.clear()
-    assert segs.plan_is_aligned(L, 0) is None and not r_spmm._takes_a_plan(x, out, 64, segs) and not looks
-    capturing = False
-    assert segs.plan_is_aligned(L, 0) is True and looks
-    capturing = True
-    looks.clear()
-    assert segs.plan_is_aligned(L, 0) is True and not looks
+    for aligned in (True, False, None):  # (None: a table from a file that an earlier version saved)
+        segs.splat_plans = {(L, 1, (0,), 0): [torch.zeros(16, dtype=torch.uint8).as_subclass(Table), aligned]}
+        assert segs.plan_is_aligned(L, 0) is aligned and r_spmm._takes_a_plan(x, out, 64, segs) == (aligned is False)
+
+
+def test_the_plans_report_is_checked_before_anything_is_launched():
+    lib = hip.lib()
+    seg = (hip.AcsrSeg * 1)()
+    assert lib.splat_attention_plan_report(seg, 1, 300, 16, 1 << 20, None, 64, None) == -1 and b"report" in lib.splat_last_error()
+    assert lib.splat_attention_plan_report(seg, 1, 300, 16, 1 << 20, 24, 64, None) == -4 and b"report" in lib.splat_last_error()
+    assert lib.splat_attention_plan_report(seg, 1, 300, 16, 1 << 20, 16, 47, None) == -2 and b"report needs 48" in lib.splat_last_error()
+    assert lib.splat_attention_plan_report(None, 1, 300, 16, 1 << 20, 16, 48, None) == -1
 
 
 def test_metadata_with_native_handles_copies_and_saves(monkeypatch):

@@ -411,7 +411,7 @@ def test_sddmm_builds_a_plan_only_for_the_kernel_that_reads_one(dev, dtype, d, h
 
 @pytest.mark.parametrize("width", [255, 100])
 def test_spmm_captured_first_after_another_operator_built_the_plan(dev, width):
-    """SpMM's first call of all is the captured one, the plan is there already (SDDMM built it): nothing is read back while
+    """SpMM's first call of all is the captured one, the plan is there already (SDDMM built it): nothing is built or read back while
     capturing, and every replay equals the eager call up to the order of the additions."""
     L, d, B, H = 1024, 64, 4, 4
     acsr = A.create_acsr(O.create_causal_windowed_mask(L, width), 16, dev)

@@ -76,6 +76,7 @@ _SIGNATURES = {
                                                   _i32, _i32, _i32, _i32, _vp]),
     "splat_attention_plan_bytes": (ctypes.c_int64, [ctypes.POINTER(AcsrSeg), _i32, _i32]),
     "splat_attention_plan": (ctypes.c_int, [ctypes.POINTER(AcsrSeg), _i32, _i32, _vp, _i64, _vp]),
+    "splat_attention_plan_report": (ctypes.c_int, [ctypes.POINTER(AcsrSeg), _i32, _i32, _vp, _i64, _vp, _i64, _vp]),
     "splat_attention_fwd_planned": (ctypes.c_int, [_vp, _i64, _i64, _i64, _vp, _i64, _i64, _i64, _i64, _vp, _i64, _i64, _i64,
                                                    _vp, _i64, _i64, _i64, ctypes.POINTER(AcsrSeg), _i32, _i32, _i32, _i32,
                                                    _i32, _f32, _i32, _vp, _i64, _vp]),

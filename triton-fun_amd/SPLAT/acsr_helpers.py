@@ -492,38 +492,29 @@ class ACSRSegments:
             if nbytes <= 0:
                 raise _hip.SplatError(f"no plan for {len(self)} segments and L={L}")
             table = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-            with torch.cuda.device(dev):
-                rc = _hip.lib().splat_attention_plan(arr, len(self), L, table.data_ptr(), nbytes, _hip.stream_ptr(dev))
-                _hip.check(rc, "splat_attention_plan")
-                # once, so that later launches may run on any stream without ordering themselves after the plan kernel
-                torch.cuda.current_stream(dev).synchronize()
-            plans[key] = [table, None]
+            with torch.cuda.device(dev):  # (waits once, so that later launches may run on any stream without ordering themselves after it)
+                aligned = _hip.host().plan(ctypes.addressof(arr), len(self), L, table)
+            plans[key] = [table, aligned]
         return plans[key][0]
+
+    def _plan_entry(self, L: int, device):
+        holder = self._plan_holder if self._plan_holder is not None else self
+        return getattr(holder, "splat_plans", {}).get((int(L), len(self), tuple(self.offsets), _hip.resolve_device(device).index))
 
     def has_plan(self, L: int, device) -> bool:
         """Whether ``plan`` would return a table it already holds (no kernel, no synchronisation)."""
-        dev = _hip.resolve_device(device)
-        holder = self._plan_holder if self._plan_holder is not None else self
-        return (int(L), len(self), tuple(self.offsets), dev.index) in getattr(holder, "splat_plans", {})
+        return self._plan_entry(L, device) is not None
 
     def plan_is_aligned(self, L: int, device) -> bool | None:
         """Whether every live row starts on a multiple of 8 positions of its block's walk in the plan for ``L`` rows (blocked
-        masks): one look at the rows' records of the first variant (gathered walks), which follow its 5 records per block
-        and segment: [lo, cnt, lin, phase] each.  The first look waits for the stream, so under stream capture a plan that has
-        not been looked at is left alone: None."""
-        if torch.cuda.is_current_stream_capturing() and not self.has_plan(L, device):
-            return None
-        table = self.plan(L, device)
-        holder = self._plan_holder if self._plan_holder is not None else self
-        dev = _hip.resolve_device(device)
-        entry = holder.splat_plans[(int(L), len(self), tuple(self.offsets), dev.index)]
-        if entry[1] is None:
+        masks), from the report that comes with the plan; None under stream capture where no plan exists (building one waits
+        for the stream)."""
+        entry = self._plan_entry(L, device)
+        if entry is None:
             if torch.cuda.is_current_stream_capturing():
                 return None
-            n_rb = table.numel() // (2 * len(self) * (5 + 128) * 16)
-            recs = table.view(torch.int32).view(-1, 4)
-            rows = recs[n_rb * len(self) * 5:n_rb * len(self) * (5 + 128)]
-            entry[1] = bool((((rows[:, 0] & 7) == 0) | (rows[:, 1] <= 0)).all())
+            self.plan(L, device)
+            entry = self._plan_entry(L, device)
         return entry[1]
 
     def native(self, L: int, device, with_plan: bool):

@@ -21,7 +21,7 @@ _HALF = (torch.float16, torch.bfloat16)
 def _takes_a_plan(x, output, n_out: int, segs: ACSRSegments) -> bool:
     """Whether this launch is faster with the mask's plan table: 16-bit types, a multiple of 8 output columns up to 128, and
     not rows of at least 256 slots that all start on a multiple of 8 positions (blocked masks with large blocks).  What is not
-    known (under stream capture, before any eager call has looked) counts as such rows: the general kernel needs no table."""
+    known (under stream capture without a plan) counts as such rows: the general kernel needs no table."""
     if x.dtype not in _HALF or output.dtype != x.dtype or n_out % 8 != 0 or n_out > 128:
         return False
     return x.shape[3] < 256 or segs.plan_is_aligned(x.shape[2], x.device) is False

@@ -576,6 +576,7 @@ static int dispatch_attn(const AttnParams& p, int d, bool kt, hipStream_t st) {
 // the results written to the table.
 struct PlanParams {
     PlanRec* table;
+    int4* report;  // may be null
     SegPtrs seg[SPLAT_MAX_SEGMENTS];
     int n_seg, L, rs, n_rb;
 };
@@ -583,9 +584,11 @@ __global__ __launch_bounds__(256) void attn_plan_kernel(const PlanParams p) {
     constexpr int BM = kPlanBM, BN = 64;
     __shared__ SegPlan s_plan[SPLAT_MAX_SEGMENTS];
     __shared__ PlanScratch<BM> s_ps;
+    __shared__ int s_misaligned, s_live;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lm = lane & 31;
     const int rb = blockIdx.x, variant = blockIdx.y;
     const int n_seg = p.n_seg, n_rb = p.n_rb;
+    if (tid == 0) s_misaligned = 0, s_live = 0;  // (plan_segments has the barriers)
     PlanRec* const pt = p.table + variant * plan_variant_recs(n_rb, n_seg);
     plan_segments<BM, BN>(p.seg, n_seg, block_first_row(rb, BM, p.rs), p.rs, p.L, variant == 0, s_plan, &s_ps, tid);
     for (int sg = 0; sg < n_seg; ++sg) {
@@ -596,6 +599,19 @@ __global__ __launch_bounds__(256) void attn_plan_kernel(const PlanParams p) {
         if (lane == 0) pt[plan_span_at(n_rb, n_seg, rb, sg, wave)] = PlanRec{sp.lo_min, sp.lo_max, sp.hi_min, sp.hi_max};
         if (lane < 32)
             pt[plan_row_at(n_rb, n_seg, rb, sg, wave * 32 + lm)] = PlanRec{win.lo, win.cnt, win.lin, pl.uniform ? 0 : win_phase(win)};
+        if (lane < 32 && win.cnt > 0) {
+            if ((win.lo & 7) != 0) s_misaligned = 1;
+            atomicAdd(&s_live, cached_row_map<BM>(&s_ps, sg, wave * 32 + lm).cnt);
+        }
+    }
+    // what a host that waits for the plan learns with it, from the walks of the first variant
+    if (p.report != nullptr && variant == 0) {
+        __syncthreads();
+        if (tid == 0) {
+            int tiles = 0;
+            for (int sg = 0; sg < n_seg; ++sg) tiles += s_plan[sg].n_tiles;
+            p.report[rb] = make_int4(s_misaligned, tiles, s_live, 0);
+        }
     }
 }
 
@@ -731,10 +747,9 @@ extern "C" int64_t splat_attention_plan_bytes(const splat_acsr_seg* segs, int32_
     return 2 * plan_variant_recs(n_rb, n_seg) * (int64_t)sizeof(PlanRec);
 }
 
-extern "C" int splat_attention_plan(const splat_acsr_seg* segs, int32_t n_seg, int32_t L, void* plan, int64_t plan_bytes,
-                                    void* stream) {
+static int attention_plan_common(const char* who, const splat_acsr_seg* segs, int32_t n_seg, int32_t L, void* plan, int64_t plan_bytes,
+                                 int32_t* report, void* stream) {
     begin_launch();
-    const char* who = "splat_attention_plan";
     if (!segs || !plan) return fail(SPLAT_E_NULL, "%s: null pointer argument", who);
     if (L <= 0 || L > (1 << 23)) return fail(SPLAT_E_SHAPE, "%s: need 0 < L <= 2^23 (got %d)", who, L);
     if ((reinterpret_cast<uintptr_t>(plan) & 15) != 0) return fail(SPLAT_E_ALIGN, "%s: the plan must be 16-byte aligned", who);
@@ -744,12 +759,31 @@ extern "C" int splat_attention_plan(const splat_acsr_seg* segs, int32_t n_seg, i
     if (plan_bytes < need)
         return fail(SPLAT_E_SHAPE, "%s: the plan needs %lld bytes for this mask, got %lld", who, (long long)need, (long long)plan_bytes);
     p.table = static_cast<PlanRec*>(plan);
+    p.report = reinterpret_cast<int4*>(report);
     p.n_seg = n_seg;
     p.L = L;
     p.rs = common_row_stride(segs, n_seg);
     p.n_rb = count_row_blocks(L, kPlanBM, p.rs);
     attn_plan_kernel<<<dim3(p.n_rb, 2), 256, 0, (hipStream_t)stream>>>(p);
     return check_launch(who);
+}
+
+extern "C" int splat_attention_plan(const splat_acsr_seg* segs, int32_t n_seg, int32_t L, void* plan, int64_t plan_bytes,
+                                    void* stream) {
+    return attention_plan_common("splat_attention_plan", segs, n_seg, L, plan, plan_bytes, nullptr, stream);
+}
+
+extern "C" int splat_attention_plan_report(const splat_acsr_seg* segs, int32_t n_seg, int32_t L, void* plan, int64_t plan_bytes,
+                                           int32_t* report, int64_t report_bytes, void* stream) {
+    const char* who = "splat_attention_plan_report";
+    if (!report) return fail(SPLAT_E_NULL, "%s: null report", who);
+    if ((reinterpret_cast<uintptr_t>(report) & 15) != 0) return fail(SPLAT_E_ALIGN, "%s: the report must be 16-byte aligned", who);
+    if (segs && n_seg >= 1 && n_seg <= SPLAT_MAX_SEGMENTS && L > 0 && L <= (1 << 23)) {  // (else refused below)
+        const int64_t need = 16 * (int64_t)count_row_blocks(L, kPlanBM, common_row_stride(segs, n_seg));
+        if (report_bytes < need)
+            return fail(SPLAT_E_SHAPE, "%s: the report needs %lld bytes for this mask, got %lld", who, (long long)need, (long long)report_bytes);
+    }
+    return attention_plan_common(who, segs, n_seg, L, plan, plan_bytes, report, stream);
 }
 
 extern "C" int splat_attention_fwd_noalloc(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* kT,

@@ -51,6 +51,7 @@ struct Api {
     decltype(&splat_spmm) spmm;
     decltype(&splat_spmm_planned) spmm_planned;
     decltype(&splat_acsr_build_record) build_record;
+    decltype(&splat_attention_plan_report) plan_report;
 } api;
 PyObject* g_error = nullptr;  // SplatError
 
@@ -516,15 +517,15 @@ PyObject* py_spmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
 }
 
-// ---- the ACSR of a mask ---------------------------------------------------------------------------------------------------------
-constexpr int64_t kShareBlocks = 1024;  // row blocks whose shares of the summary a buffer holds
+// ---- the ACSR and the plan of a mask ---------------------------------------------------------------------------------------------
+constexpr int64_t kShareBlocks = 1024;  // row blocks of a build whose shares of the summary a kept buffer holds
 
-// Pinned buffers for the shares of the builds under way: one per build between its launch and its end (the call waits for the
-// stream before it gives the buffer back), at most kKeep of them kept for the next ones.
+// Pinned buffers for what builds and plans under way tell the host: one per call between its launch and its end (the call waits for
+// the stream before it gives the buffer back), at most kKeep of them kept for the next ones, longer ones than usual not at all.
 class ShareBuffers {
   public:
-    at::Tensor take() {
-        {
+    at::Tensor take(int64_t n) {
+        if (n <= kShareBlocks * 8) {
             std::lock_guard<std::mutex> hold(m_);
             if (!free_.empty()) {
                 at::Tensor t = std::move(free_.back());
@@ -532,11 +533,11 @@ class ShareBuffers {
                 return t;
             }
         }
-        return at::empty({kShareBlocks * 8}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+        return at::empty({std::max(n, kShareBlocks * 8)}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
     }
     void give(at::Tensor t) {
         std::lock_guard<std::mutex> hold(m_);
-        if (free_.size() < kKeep) free_.push_back(std::move(t));
+        if (t.numel() == kShareBlocks * 8 && free_.size() < kKeep) free_.push_back(std::move(t));
     }
 
   private:
@@ -547,6 +548,60 @@ class ShareBuffers {
 ShareBuffers* share_buffers() {
     static ShareBuffers* b = new ShareBuffers;  // (never destroyed: the allocator may be gone at the process's end)
     return b;
+}
+
+// A call that returned an error: its buffer is given back where the arguments were refused (negative codes), but not where an error of
+// the runtime was found with the launch, which may have happened all the same and write to it later.
+PyObject* refused(const char* what, int rc, at::Tensor& shares) {
+    if (rc < 0)
+        share_buffers()->give(std::move(shares));
+    else
+        new at::Tensor(std::move(shares));
+    return raise_rc(what, rc);
+}
+
+// Waits for the stream without the interpreter's lock; false with a Python error set when that failed, and then the buffer is not
+// given back either.
+bool wait_for(const c10::hip::HIPStream& stream, at::Tensor& shares) {
+    PyThreadState* const released = PyEval_SaveThread();
+    std::string failed_wait;
+    try {
+        c10::hip::stream_synchronize(stream.stream());
+    } catch (const std::exception& e) {
+        failed_wait = e.what();
+    }
+    PyEval_RestoreThread(released);
+    if (failed_wait.empty()) return true;
+    new at::Tensor(std::move(shares));
+    PyErr_SetString(PyExc_RuntimeError, failed_wait.c_str());
+    return false;
+}
+
+// plan(arr_address, n_seg, L, table) -> whether every live row starts on a multiple of 8 positions of its block's walk.  Fills the plan
+// table on the current device and waits for it, so that launches on any stream may use it.
+PyObject* py_plan(PyObject*, PyObject* args) {
+    unsigned long long addr;
+    int n_seg, L;
+    PyObject* o;
+    if (!PyArg_ParseTuple(args, "KiiO", &addr, &n_seg, &L, &o)) return nullptr;
+    if (!THPVariable_Check(o)) return PyErr_Format(PyExc_TypeError, "table must be a tensor");
+    try {
+        const at::Tensor& table = THPVariable_Unpack(o);
+        const auto* segs = reinterpret_cast<const splat_acsr_seg*>(static_cast<uintptr_t>(addr));
+        const int64_t bytes = table.nbytes(), blocks = n_seg > 0 ? bytes / (2 * (5 + 128) * 16 * (int64_t)n_seg) : 0;
+        const auto stream = c10::hip::getCurrentHIPStream(table.get_device());
+        at::Tensor shares = share_buffers()->take(4 * blocks);
+        const int32_t* const sh = shares.data_ptr<int32_t>();
+        const int rc = api.plan_report(segs, n_seg, L, table.data_ptr(), bytes, shares.data_ptr<int32_t>(), shares.nbytes(), stream.stream());
+        if (rc) return refused("splat_attention_plan_report", rc, shares);
+        if (!wait_for(stream, shares)) return nullptr;
+        bool aligned = true;
+        for (int64_t b = 0; b < blocks; ++b) aligned = aligned && sh[4 * b] == 0;
+        share_buffers()->give(std::move(shares));
+        return PyBool_FromLong(aligned);
+    } catch (const std::exception& e) {
+        return raise_std(e);
+    }
 }
 
 // One array of a record, as a tensor of its own on the record's storage.
@@ -578,24 +633,12 @@ PyObject* py_build(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const int64_t row_step = (rows + 63) / 64 * 64, span_step = (blocks + 63) / 64 * 64, twin = 5 * row_step + 2 * span_step;
         // (a storage per type: torch.save takes no tensors of two types on one)
         const at::Tensor record = fresh({2 * twin}, at::kFloat), extents = fresh({4 * row_step}, at::kInt);
-        at::Tensor shares = share_buffers()->take();
+        at::Tensor shares = share_buffers()->take(8 * blocks);
         const int32_t* const sh = shares.data_ptr<int32_t>();
         const int rc = api.build_record(mask.data_ptr<uint8_t>(), rows, cols, mask.stride(0), (int32_t)bh, record.data_ptr<float>(),
                                         extents.data_ptr<int32_t>(), 1, shares.data_ptr<int32_t>(), stream.stream());
-        if (rc) return raise_rc("splat_acsr_build_record", rc);
-        PyThreadState* const released = PyEval_SaveThread();
-        std::string failed_wait;
-        try {
-            c10::hip::stream_synchronize(stream.stream());
-        } catch (const std::exception& e) {
-            failed_wait = e.what();
-        }
-        PyEval_RestoreThread(released);
-        if (!failed_wait.empty()) {  // (the buffer is not given back: the kernel may still write to it)
-            new at::Tensor(std::move(shares));
-            PyErr_SetString(PyExc_RuntimeError, failed_wait.c_str());
-            return nullptr;
-        }
+        if (rc) return refused("splat_acsr_build_record", rc, shares);
+        if (!wait_for(stream, shares)) return nullptr;
         int32_t t_max = 0, bad = 0, step_min = 0x7fffffff, step_max = 0, off = 0;
         for (int64_t b = 0; b < blocks; ++b) {
             const int32_t* s = sh + 8 * b;
@@ -641,7 +684,8 @@ PyObject* py_bind(PyObject*, PyObject* args) {
         !take("splat_attention_bwd", api.bwd) || !take("splat_attention_bwd_keys", api.bwd_keys) ||
         !take("splat_attention_bwd_f32", api.bwd_f32) || !take("splat_attention_bwd_keys_f32", api.bwd_keys_f32) || !take("splat_sddmm", api.sddmm) ||
         !take("splat_sddmm_probs", api.sddmm_probs) || !take("splat_sddmm_planned", api.sddmm_planned) ||
-        !take("splat_softmax", api.softmax) || !take("splat_spmm", api.spmm) || !take("splat_spmm_planned", api.spmm_planned) || !take("splat_acsr_build_record", api.build_record))
+        !take("splat_softmax", api.softmax) || !take("splat_spmm", api.spmm) || !take("splat_spmm_planned", api.spmm_planned) ||
+        !take("splat_acsr_build_record", api.build_record) || !take("splat_attention_plan_report", api.plan_report))
         return nullptr;
     Py_INCREF(err);
     Py_XSETREF(g_error, err);
@@ -654,6 +698,7 @@ PyMethodDef methods[] = {
     {"forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_forward)), METH_FASTCALL, "fused forward"},
     {"grad_state", py_grad_state, METH_VARARGS, "what the differentiable attention keeps"},
     {"attend", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_attend)), METH_FASTCALL, "differentiable attention"},
+    {"plan", py_plan, METH_VARARGS, "the plan table of a mask"},
     {"build", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_build)), METH_FASTCALL, "the ACSR of a mask tensor"},
     {"sddmm", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_sddmm)), METH_FASTCALL, "sampled product"},
     {"softmax", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_softmax)), METH_FASTCALL, "softmax of compressed rows"},
