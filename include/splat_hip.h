@@ -36,7 +36,7 @@
 extern "C" {
 #endif
 
-#define SPLAT_VERSION 1100 /* major*10000 + minor*100 + patch; 0.2.0 added the planned forward, 0.3.0 splat_spmm_t, 0.4.0 splat_attention_fwd_stats, splat_sddmm_probs, 0.5.0 splat_attention_fwd_noalloc, 0.6.0 moved the two measurement aids out (libsplat_bench.so, splat_bench.h), 0.7.0 added splat_sddmm_planned, splat_spmm_planned, 0.8.0 splat_spmm_t_planned, 0.9.0 splat_attention_bwd_keys, 0.10.0 splat_acsr_build_record, splat_attention_bwd_f32, splat_attention_bwd_keys_f32, 0.11.0 gave splat_acsr_build_record's int32 arrays a buffer of their own and added splat_attention_plan_report */
+#define SPLAT_VERSION 1100 /* major*10000 + minor*100 + patch; 0.2.0 added the planned forward, 0.3.0 splat_spmm_t, 0.4.0 splat_attention_fwd_stats, splat_sddmm_probs, 0.5.0 splat_attention_fwd_noalloc, 0.6.0 moved the two measurement aids out (libsplat_bench.so, splat_bench.h), 0.7.0 added splat_sddmm_planned, splat_spmm_planned, 0.8.0 splat_spmm_t_planned, 0.9.0 splat_attention_bwd_keys, 0.10.0 splat_acsr_build_record, splat_attention_bwd_f32, splat_attention_bwd_keys_f32, 0.11.0 gave splat_acsr_build_record's int32 arrays a buffer of their own and added splat_attention_plan_report, splat_attention_fwd_hinted */
 
 /* element types of q/k/v/score/output buffers */
 #define SPLAT_F32 0
@@ -254,6 +254,18 @@ int splat_attention_fwd_stats(const void* q, int64_t q_sb, int64_t q_sh, int64_t
                               int32_t n_seg, int32_t B, int32_t H, int32_t L, int32_t d, float scale,
                               int32_t dtype, const void* plan, int64_t plan_bytes, float* lse,
                               void* stream);
+
+/* The fused forward with everything optional: `plan` and `lse` may be NULL, and live_percent (0: unknown) says how much of what
+ * the plan walks is live: 100 * (sum of [2]) / (sum of [1] * 8192) over the blocks of splat_attention_plan_report, rounded up.
+ * Only affects speed, by the choice of the kernel in launches of few row blocks; with 0 `out` is bit-identical to the other
+ * forwards', else the same up to the order of the float32 additions. */
+int splat_attention_fwd_hinted(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* kT,
+                               int64_t k_sb, int64_t k_sh, int64_t k_sd, int64_t k_sl, const void* v,
+                               int64_t v_sb, int64_t v_sh, int64_t v_sl, void* out, int64_t o_sb,
+                               int64_t o_sh, int64_t o_sl, const splat_acsr_seg* segs /* host */,
+                               int32_t n_seg, int32_t B, int32_t H, int32_t L, int32_t d, float scale,
+                               int32_t dtype, const void* plan, int64_t plan_bytes, float* lse, int32_t live_percent,
+                               void* stream);
 
 /* The fused forward for callers that cannot allocate device memory or hold a plan buffer: code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc.  No counterpart in the reference.  Same arguments and

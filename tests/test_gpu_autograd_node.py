@@ -53,7 +53,7 @@ def test_functorch_transforms_get_the_message_that_names_them(dev):
 
 def test_a_scale_the_kernels_refuse_is_a_splat_error(dev):
     attn = _module(dev, scale=-1.0)
-    with pytest.raises(hip.SplatError, match=r"^splat_attention_fwd_stats failed \(code -5\): .*scale must be > 0"):
+    with pytest.raises(hip.SplatError, match=r"^splat_attention_fwd_hinted failed \(code -5\): .*scale must be > 0"):
         attention_with_grad(*_operands(dev), attn)
 
 

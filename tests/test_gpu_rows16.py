@@ -4,7 +4,7 @@ import pytest
 import torch
 
 import acsr_helpers as A
-from r_attention import RegularAttention
+from r_attention import RegularAttention, attention_launcher
 
 pytestmark = pytest.mark.gpu
 
@@ -40,14 +40,48 @@ def test_against_float64(dev, name, L, dtype, d):
         assert float((got - ref).abs().max()) <= (8e-3 if dtype == torch.float16 else 4e-2)
 
 
-@pytest.mark.parametrize("d,most", [(64, 384), (128, 192)])
-def test_both_sides_of_the_line(dev, d, most):
-    """`most` heads of one row block go to this kernel, one head more to the other: the shared heads agree."""
+@pytest.mark.parametrize("d,most,mask,percent", [(64, 320, A.windowed_pattern(128, 20), 30), (128, 192, A.windowed_pattern(128, 20), 30),
+                                                 (64, 128, A.blocked_pattern(128, 128), 100), (128, 128, A.blocked_pattern(128, 128), 100)])
+def test_both_sides_of_the_line(dev, d, most, mask, percent):
+    """`most` heads of one row block go to this kernel, one head more to the other: the shared heads agree.  The line depends on how
+    much of the walk is live; the module's first call (the launcher) and the next (native) take the same side."""
     L, dtype = 128, torch.bfloat16
     g = torch.Generator(device=dev).manual_seed(d)
     q, k, v = (torch.randn(1, most + 1, L, d, generator=g, device=dev).to(dtype) for _ in range(3))
     outs = []
     for H in (most, most + 1):
-        attn = RegularAttention(1, L, H, d, A.windowed_pattern(L, 20), 16, 16, dev, dtype, scale=d ** -0.5)
-        outs.append(attn([q[:, :H], k[:, :H].transpose(2, 3), v[:, :H]]).float())
+        attn = RegularAttention(1, L, H, d, mask, 16, 16, dev, dtype, scale=d ** -0.5)
+        x = [q[:, :H], k[:, :H].transpose(2, 3), v[:, :H]]
+        first = attn(x).clone()
+        assert attn._live_percent == percent
+        # the kernels differ in the order of their additions: equal bits say which one ran
+        kinds = [attention_launcher(*x, torch.empty_like(first), attn.segments, attn.scale, attn._plan, live_percent=p) for p in (1, 100)]
+        assert torch.equal(first, attn(x)) and torch.equal(first, attn.forward_with_stats(x)[0])
+        assert torch.equal(first, kinds[0] if percent <= 75 else kinds[1])
+        assert torch.equal(*kinds) == (H <= 128 or H > (320 if d == 64 else 192))
+        outs.append(first.float())
     assert float((outs[0] - outs[1][:, :most]).norm() / outs[0].norm()) <= 4e-3
+    assert not torch.equal(outs[0], outs[1][:, :most])
+
+
+@pytest.mark.parametrize("L,masks", [(700, lambda L: [A.causal_windowed_pattern(L, 199)]), (300, lambda L: [A.dilated_pattern(L, 40, 3)]),
+                                     (640, lambda L: [A.blocked_pattern(L, 128)]), (777, lambda L: A.strided_patterns(L, 64, 32))])
+def test_live_percent_is_what_the_masks_say(dev, L, masks):
+    """Live entries over the positions of the tiles that each block of 128 rows walks (64 positions each; dense runs start on a
+    multiple of 64, gathered ones at the block's first column), rounded up."""
+    segs = A.create_acsr_segments(masks(L), 16, dev)
+    assert segs.live_percent(L, dev) == 0
+    segs.plan(L, dev)
+    rs = {int(t[3].splat_row_stride) for t in segs.tuples}
+    rs = rs.pop() if len(rs) == 1 else 1
+    live = walked = 0
+    for m, t in zip(masks(L), segs.tuples):
+        dm, step = m.device_mask(dev).cpu() > 0, int(t[3].splat_max_step)
+        live += int(dm.sum())
+        for b in range(-(-L // (128 * rs)) * rs):
+            r0 = b // rs * 128 * rs + b % rs
+            cols = torch.nonzero(dm[r0:r0 + 128 * rs:rs].any(0)).flatten()
+            if cols.numel():
+                c0 = int(cols[0]) if step > 1 else int(cols[0]) // 64 * 64
+                walked += -(-((int(cols[-1]) - c0) // step + 1) // 64) * 64 * 128
+    assert segs.live_percent(L, dev) == -(-100 * live // walked)

@@ -493,8 +493,7 @@ class ACSRSegments:
                 raise _hip.SplatError(f"no plan for {len(self)} segments and L={L}")
             table = torch.empty(nbytes, dtype=torch.uint8, device=dev)
             with torch.cuda.device(dev):  # (waits once, so that later launches may run on any stream without ordering themselves after it)
-                aligned = _hip.host().plan(ctypes.addressof(arr), len(self), L, table)
-            plans[key] = [table, aligned]
+                plans[key] = [table, *_hip.host().plan(ctypes.addressof(arr), len(self), L, table)]
         return plans[key][0]
 
     def _plan_entry(self, L: int, device):
@@ -517,6 +516,11 @@ class ACSRSegments:
             entry = self._plan_entry(L, device)
         return entry[1]
 
+    def live_percent(self, L: int, device) -> int:
+        """How much of what the plan's blocks walk is live, in percent rounded up (a causal window of 512: 80); 0 without a plan."""
+        entry = self._plan_entry(L, device)
+        return entry[2] if entry is not None and len(entry) > 2 else 0
+
     def native(self, L: int, device, with_plan: bool):
         """The segments as the native host path takes them (``_splat_hip.host().mask``), with the plan table or without, built
         on first use and kept where ``plan`` keeps its tables; None under stream capture when it would have to be built
@@ -535,7 +539,7 @@ class ACSRSegments:
             arr = self.seg_array(L)
             own = [t for seg in self.seg_args() for t in seg[:6] if t is not None and t is not holder]
             mask = kept[key] = _hip.host().mask(ctypes.addressof(arr), len(self), L, self.plan(L, device) if with_plan else None,
-                                                self.max_step, tuple(own))
+                                                self.live_percent(L, device) if with_plan else 0, self.max_step, tuple(own))
         return mask
 
     def seg_args(self) -> list[tuple]:

@@ -41,13 +41,15 @@ _NO_GUARD = contextlib.nullcontext()
 
 def attention_launcher(q: torch.Tensor, kT: torch.Tensor, v: torch.Tensor, output: torch.Tensor,
                        segments: ACSRSegments, scale: float = 1.0, plan: torch.Tensor | None = None,
-                       lse: torch.Tensor | None = None) -> torch.Tensor:
+                       lse: torch.Tensor | None = None, *, live_percent: int = 0) -> torch.Tensor:
     """Fused forward: output[b, h, r, :] = softmax over the live columns of (scale * q.kT)[b, h, r, :] times v.
     q [B, H, L, d], kT [B, H, d, L] (unit stride along d or along L), v [B, H, L, d], output [B, H, L, d];
     d in {64, 128}; one dtype for all four.  ``plan`` (from ``attention_plan`` for the same segments and L) spares
     every workgroup the derivation of its tiles from the ACSR arrays; the results are the same.  ``lse`` (float32
     [B, H, L], contiguous), when given, receives every row's log of the sum of exp(scale * score) over its live
-    columns (+inf for a row without any), so that the row's probabilities are exp(scale * score - lse)."""
+    columns (+inf for a row without any), so that the row's probabilities are exp(scale * score - lse).
+    ``live_percent`` (``ACSRSegments.live_percent``): a hint for the choice of the kernel in launches of few row blocks, where the
+    results then agree up to the order of the float32 additions."""
     for name, t in (("q", q), ("kT", kT), ("v", v), ("output", output)):
         _hip.require_device_tensor(t, name)
         if t.dim() != 4:
@@ -100,18 +102,10 @@ def attention_launcher(q: torch.Tensor, kT: torch.Tensor, v: torch.Tensor, outpu
             raise _hip.SplatError(f"lse must be a contiguous float32 tensor of shape {(B, H, L)} on {dev}")
     # (the device guard costs 3-4 us of the call's 16 on the host: entered only when another device is current)
     with (_NO_GUARD if torch.cuda.current_device() == dev.index else torch.cuda.device(dev)):
-        if lse is not None:
-            rc = _hip.lib().splat_attention_fwd_stats(*args, plan.data_ptr() if plan is not None else None,
-                                                      plan.numel() * plan.element_size() if plan is not None else 0,
-                                                      lse.data_ptr(), _hip.stream_ptr(dev))
-            _hip.check(rc, "splat_attention_fwd_stats")
-        elif plan is None:
-            rc = _hip.lib().splat_attention_fwd(*args, _hip.stream_ptr(dev))
-            _hip.check(rc, "splat_attention_fwd")
-        else:
-            rc = _hip.lib().splat_attention_fwd_planned(*args, plan.data_ptr(), plan.numel() * plan.element_size(),
-                                                        _hip.stream_ptr(dev))
-            _hip.check(rc, "splat_attention_fwd_planned")
+        rc = _hip.lib().splat_attention_fwd_hinted(*args, plan.data_ptr() if plan is not None else None,
+                                                   plan.numel() * plan.element_size() if plan is not None else 0,
+                                                   lse.data_ptr() if lse is not None else None, live_percent, _hip.stream_ptr(dev))
+        _hip.check(rc, "splat_attention_fwd_hinted")
     if target is not output:
         target.copy_(output)
     return target
@@ -159,6 +153,7 @@ class RegularAttention(nn.Module):
         self.rspmm_grid_dim = (-(-head_dim // BLOCK_SIZE_X), -(-seq_length // BLOCK_SIZE_Y), batch * num_heads)
         self._unfused_ready = False
         self._plan = None  # the fused kernel's plan of this mask, built on the first fused forward
+        self._live_percent = 0  # how much of what the plan walks is live
         self._segments_t = None  # ACSR of the transposed mask(s), built on the first backward
         self._plan_t = None  # the fused backward's plan of the transposed mask
         self._lse = None  # the rows' softmax statistics, allocated by the first forward_with_stats
@@ -206,7 +201,7 @@ class RegularAttention(nn.Module):
         fusable = self.fused and q.shape[-1] in (64, 128) and q.dtype == k.dtype == v.dtype == self._out_dtype
         if fusable:
             self._ensure_plan()
-            return attention_launcher(q, k, v, self.rspmm_output, self.segments, self.scale, self._plan)
+            return attention_launcher(q, k, v, self.rspmm_output, self.segments, self.scale, self._plan, live_percent=self._live_percent)
 
         multi = self.segments  # (also for one segment: the object keeps what every call would otherwise rebuild and recheck)
         rsddmm_launcher(q, k, self.rsddmm_output,
@@ -231,6 +226,7 @@ class RegularAttention(nn.Module):
         """The fused kernel's plan of this mask, and the mask as the native host path takes it."""
         if self._plan is None:
             self._plan = attention_plan(self.segments, self._shape[2], self._device)
+            self._live_percent = self.segments.live_percent(self._shape[2], self._device)
         if self._native is None:
             self._native = self.segments.native(self._shape[2], self._device, True)
 
@@ -245,7 +241,8 @@ class RegularAttention(nn.Module):
         self._ensure_plan()
         if self._lse is None:
             self._lse = torch.empty(self._shape[:3], dtype=torch.float32, device=self._device)
-        attention_launcher(q, k, v, self.rspmm_output, self.segments, self.scale, self._plan, self._lse)
+        attention_launcher(q, k, v, self.rspmm_output, self.segments, self.scale, self._plan, self._lse,
+                           live_percent=self._live_percent)
         return self.rspmm_output, self._lse
 
     def backward_pass(self, x, grad_out: torch.Tensor, lse: torch.Tensor | None = None, out: torch.Tensor | None = None,
@@ -319,7 +316,8 @@ class _AttentionFunction(torch.autograd.Function):
             attn._ensure_plan()
             out = torch.empty_like(attn.rspmm_output)
             lse = torch.empty(attn._shape[:3], dtype=torch.float32, device=out.device)
-            attention_launcher(q, k.transpose(2, 3), v, out, attn.segments, attn.scale, attn._plan, lse)
+            attention_launcher(q, k.transpose(2, 3), v, out, attn.segments, attn.scale, attn._plan, lse,
+                               live_percent=attn._live_percent)
             ctx.save_for_backward(q, k, v, lse, out)
             return out
         out = attn([q, k.transpose(2, 3), v])

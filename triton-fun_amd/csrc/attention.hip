@@ -559,11 +559,17 @@ static int launch_attn(const AttnParams& p0, hipStream_t st) {
 // kernel also supports 32-key tiles in a ring of 4 stages; it measured slower at d = 128 and equal at d = 64).
 template <typename T>
 static int dispatch_attn(const AttnParams& p, int d, bool kt, hipStream_t st) {
-    // few row blocks: the kernel of 16 rows a wavefront (attention_rows16.hip).  Its workgroups, two per row block, take 32 KB
-    // (d = 64) or 64 KB of LDS; the line lies where it stops being faster over windows of 32 to 512: three workgroups a CU at
-    // d = 64 (384 row blocks: 9.5 -> 8.6, 10.8 -> 10.1, 17.8 -> 17.5 us; 448: 9.5 -> 9.9, 17.8 -> 20.4), one and a half at d = 128
-    // (192: 9.8 -> 8.6, 10.9 -> 10.1, 18.0 -> 18.7 us; 320: 12.0 -> 13.9)
-    if ((int64_t)p.B * p.H * count_row_blocks(p.L, kPlanBM, p.row_stride) <= (d == 64 ? 384 : 192)) return launch_attn_rows16<T>(p, d, kt, st);
+    // Few row blocks: the kernel of 16 rows a wavefront (attention_rows16.hip), two workgroups per row block.  Up to 128 row blocks
+    // every workgroup has a CU to itself and it is the faster one whatever the mask: bf16, 128 blocks, 32x32x16 kernel -> this one,
+    // window 32 / 512 / blocks of 2048: d = 64 7.4 -> 5.3, 13.8 -> 10.9, 60.5 -> 52.6 us, d = 128 9.1 -> 6.6, 17.4 -> 14.4, 80.4 -> 73.8.
+    // Beyond that workgroups share a CU's LDS, from which this kernel reads every operand for half the rows: it wins where it skips
+    // masked positions and loses where there are none.  The line lies at three quarters of the walked positions live and 320 (192 at
+    // d = 128) blocks: at 192 blocks, d = 64, windows 128 / 320 (half, 72 % live) 8.5 -> 7.7, 11.1 -> 10.5 us, window 512 (80 %)
+    // 13.9 -> 13.4, blocks of 256 (all) 11.4 -> 12.4; d = 128 10.4 -> 9.4, 13.9 -> 13.6, 17.5 -> 17.7, 14.4 -> 16.9; at 384 blocks,
+    // d = 64, window 256 with K^T along the keys 12.1 -> 12.4.
+    const int64_t blocks = (int64_t)p.B * p.H * count_row_blocks(p.L, kPlanBM, p.row_stride);
+    if (blocks <= 128 || (p.live_percent > 0 && p.live_percent <= 75 && blocks <= (d == 64 ? 320 : 192)))
+        return launch_attn_rows16<T>(p, d, kt, st);
     if (p.plan) {
         if (d == 64) return kt ? launch_attn<T, 64, true, 64, 2, true>(p, st) : launch_attn<T, 64, false, 64, 2, true>(p, st);
         return kt ? launch_attn<T, 128, true, 64, 2, true>(p, st) : launch_attn<T, 128, false, 64, 2, true>(p, st);
@@ -624,7 +630,7 @@ static int attention_fwd_common(const char* who, const void* q, int64_t q_sb, in
                                 int64_t v_sh, int64_t v_sl, void* out, int64_t o_sb, int64_t o_sh, int64_t o_sl,
                                 const splat_acsr_seg* segs, int32_t n_seg, int32_t B, int32_t H, int32_t L, int32_t d,
                                 float scale, int32_t dtype, const void* plan, int64_t plan_bytes, bool planned,
-                                float* lse, void* stream) {
+                                float* lse, void* stream, int32_t live_percent = 0) {
     if (!q || !kT || !v || !out || !segs) return fail(SPLAT_E_NULL, "%s: null pointer argument", who);
     if (B <= 0 || H <= 0 || L <= 0) return fail(SPLAT_E_SHAPE, "%s: need B, H, L > 0 (got %d, %d, %d)", who, B, H, L);
     if (L > (1 << 23)) return fail(SPLAT_E_SHAPE, "%s: L is limited to 2^23 (got %d)", who, L);
@@ -667,6 +673,7 @@ static int attention_fwd_common(const char* who, const void* q, int64_t q_sb, in
     p.row_stride = common_row_stride(segs, n_seg);
     p.plan = nullptr;
     p.lse = lse;
+    p.live_percent = live_percent;
     if (planned) {
         if (!plan) return fail(SPLAT_E_NULL, "%s: null plan", who);
         if ((reinterpret_cast<uintptr_t>(plan) & 15) != 0) return fail(SPLAT_E_ALIGN, "%s: the plan must be 16-byte aligned", who);
@@ -714,6 +721,20 @@ extern "C" int splat_attention_fwd_stats(const void* q, int64_t q_sb, int64_t q_
     if ((reinterpret_cast<uintptr_t>(lse) & 3) != 0) return fail(SPLAT_E_ALIGN, "%s: lse must be 4-byte aligned", who);
     return attention_fwd_common(who, q, q_sb, q_sh, q_sl, kT, k_sb, k_sh, k_sd, k_sl, v, v_sb, v_sh, v_sl, out, o_sb, o_sh,
                                 o_sl, segs, n_seg, B, H, L, d, scale, dtype, plan, plan_bytes, plan != nullptr, lse, stream);
+}
+
+extern "C" int splat_attention_fwd_hinted(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* kT,
+                                          int64_t k_sb, int64_t k_sh, int64_t k_sd, int64_t k_sl, const void* v,
+                                          int64_t v_sb, int64_t v_sh, int64_t v_sl, void* out, int64_t o_sb,
+                                          int64_t o_sh, int64_t o_sl, const splat_acsr_seg* segs, int32_t n_seg, int32_t B,
+                                          int32_t H, int32_t L, int32_t d, float scale, int32_t dtype, const void* plan,
+                                          int64_t plan_bytes, float* lse, int32_t live_percent, void* stream) {
+    const char* who = "splat_attention_fwd_hinted";
+    if ((reinterpret_cast<uintptr_t>(lse) & 3) != 0) return fail(SPLAT_E_ALIGN, "%s: lse must be 4-byte aligned", who);
+    if (live_percent < 0 || live_percent > 100) return fail(SPLAT_E_SHAPE, "%s: live_percent is %d", who, live_percent);
+    return attention_fwd_common(who, q, q_sb, q_sh, q_sl, kT, k_sb, k_sh, k_sd, k_sl, v, v_sb, v_sh, v_sl, out, o_sb, o_sh,
+                                o_sl, segs, n_seg, B, H, L, d, scale, dtype, plan, plan_bytes, plan != nullptr, lse, stream,
+                                live_percent);
 }
 
 // ---- the forward for callers that cannot allocate: the plan lives in a file-scope device array ----------------

@@ -6,7 +6,7 @@
 // wavefront 16 of them, so that the same launch spreads over twice the workgroups and each walks fewer tiles, and pairs of
 // subtiles of 16 keys outside a wavefront's rows are skipped.  16x16x32 matrix instructions run at the rate of the 32x32x16 ones,
 // but every operand read from LDS then serves 16 rows instead of 32: in launches that fill the chip the LDS becomes the bound
-// and the other kernel is the faster one (dispatch_attn in attention.hip has the line).  Measured, bf16, 16 heads of 1024 rows,
+// and the other kernel is the faster one unless much of the walk is masked (dispatch_attn in attention.hip has the lines).  Measured, bf16, 16 heads of 1024 rows,
 // that kernel -> this one: d = 64, window 32: 8.3 -> 6.5 us, 128: 9.2 -> 7.3, 512: 14.6 -> 11.9; d = 128: 9.8 -> 7.5, 10.9 -> 9.0,
 // 18.1 -> 15.6 (rings of three stages and tiles of 32 keys: equal at d = 64, up to 12 % slower at d = 128).
 //

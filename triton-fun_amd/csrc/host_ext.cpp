@@ -37,8 +37,7 @@ namespace {
 // ---- the library's entry points -------------------------------------------------------------------------------------
 struct Api {
     decltype(&splat_last_error) last_error;
-    decltype(&splat_attention_fwd_planned) fwd_planned;
-    decltype(&splat_attention_fwd_stats) fwd_stats;
+    decltype(&splat_attention_fwd_hinted) fwd_hinted;
     decltype(&splat_transpose_keys) transpose_keys;
     decltype(&splat_attention_bwd) bwd;
     decltype(&splat_attention_bwd_keys) bwd_keys;
@@ -93,6 +92,7 @@ struct Mask : torch::CustomClassHolder {
     int64_t rows = 0;
     int max_step = 1;
     at::Tensor plan;               // may be undefined
+    int live_percent = 0;          // of the positions that the plan walks, 0: unknown
     std::vector<at::Tensor> keep;  // the arrays that `segs` points into
     int device = 0;
     const void* plan_ptr() const { return plan.data_ptr(); }
@@ -167,20 +167,20 @@ at::Tensor transposed_keys(const at::Tensor& kT, int* rc) {
     return k;
 }
 
-// mask(arr_address, n_seg, rows, plan | None, max_step, (tensors...)) -> capsule
+// mask(arr_address, n_seg, rows, plan | None, live_percent, max_step, (tensors...)) -> capsule
 PyObject* py_mask(PyObject*, PyObject* args) {
     unsigned long long addr;
-    int n_seg, max_step;
+    int n_seg, live, max_step;
     long long rows;
     PyObject *plan, *tensors;
-    if (!PyArg_ParseTuple(args, "KiLOiO!", &addr, &n_seg, &rows, &plan, &max_step, &PyTuple_Type, &tensors)) return nullptr;
+    if (!PyArg_ParseTuple(args, "KiLOiiO!", &addr, &n_seg, &rows, &plan, &live, &max_step, &PyTuple_Type, &tensors)) return nullptr;
     if (n_seg < 1 || n_seg > SPLAT_MAX_SEGMENTS) {
         PyErr_SetString(PyExc_ValueError, "number of segments");
         return nullptr;
     }
     auto m = c10::make_intrusive<Mask>();
     std::memcpy(m->segs, reinterpret_cast<const void*>(static_cast<uintptr_t>(addr)), n_seg * sizeof(splat_acsr_seg));
-    m->n_seg = n_seg, m->rows = rows, m->max_step = max_step;
+    m->n_seg = n_seg, m->rows = rows, m->live_percent = live, m->max_step = max_step;
     for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(tensors); ++i) {
         PyObject* o = PyTuple_GET_ITEM(tensors, i);
         if (!THPVariable_Check(o)) continue;
@@ -219,16 +219,10 @@ Did forward(const Mask& m, const at::Tensor& q, at::Tensor kT, const at::Tensor&
         }
     }
     void* st = stream_of(q);
-    if (lse)
-        *rc = api.fwd_stats(q.data_ptr(), q.stride(0), q.stride(1), q.stride(2), kT.data_ptr(), kT.stride(0), kT.stride(1), kT.stride(2),
-                            kT.stride(3), v.data_ptr(), v.stride(0), v.stride(1), v.stride(2), out.data_ptr(), out.stride(0),
-                            out.stride(1), out.stride(2), m.segs, m.n_seg, B, H, L, d, (float)scale, code, m.plan_ptr(),
-                            m.plan_bytes(), lse, st);
-    else
-        *rc = api.fwd_planned(q.data_ptr(), q.stride(0), q.stride(1), q.stride(2), kT.data_ptr(), kT.stride(0), kT.stride(1),
-                              kT.stride(2), kT.stride(3), v.data_ptr(), v.stride(0), v.stride(1), v.stride(2), out.data_ptr(),
-                              out.stride(0), out.stride(1), out.stride(2), m.segs, m.n_seg, B, H, L, d, (float)scale, code,
-                              m.plan_ptr(), m.plan_bytes(), st);
+    *rc = api.fwd_hinted(q.data_ptr(), q.stride(0), q.stride(1), q.stride(2), kT.data_ptr(), kT.stride(0), kT.stride(1), kT.stride(2),
+                         kT.stride(3), v.data_ptr(), v.stride(0), v.stride(1), v.stride(2), out.data_ptr(), out.stride(0), out.stride(1),
+                         out.stride(2), m.segs, m.n_seg, B, H, L, d, (float)scale, code, m.plan_ptr(), m.plan_bytes(), lse, m.live_percent,
+                         st);
     return *rc ? Did::kFailed : Did::kYes;
 }
 
@@ -245,7 +239,7 @@ PyObject* py_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
         if (scale == -1.0 && PyErr_Occurred()) return nullptr;
         int rc = 0;
         const Did did = forward(*m, *q, *kT, *v, *out, scale, nullptr, &rc);
-        if (did == Did::kFailed) return raise_rc("splat_attention_fwd_planned", rc);
+        if (did == Did::kFailed) return raise_rc("splat_attention_fwd_hinted", rc);
         return PyBool_FromLong(did == Did::kYes);
     } catch (const std::exception& e) {
         return raise_std(e);
@@ -348,7 +342,7 @@ at::Tensor attend(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
         lse = fresh({st->B, st->H, st->L}, at::kFloat);
         int rc = 0;
         const Did did = forward(*st->fwd, q, k.transpose(2, 3), v, out, scale, lse.data_ptr<float>(), &rc);
-        if (did == Did::kFailed) throw Failure(failure("splat_attention_fwd_stats", rc));
+        if (did == Did::kFailed) throw Failure(failure("splat_attention_fwd_hinted", rc));
         if (did == Did::kNo) return at::Tensor();
     }
     std::shared_ptr<AttendBackward> node(new AttendBackward(), torch::autograd::deleteNode);
@@ -577,8 +571,9 @@ bool wait_for(const c10::hip::HIPStream& stream, at::Tensor& shares) {
     return false;
 }
 
-// plan(arr_address, n_seg, L, table) -> whether every live row starts on a multiple of 8 positions of its block's walk.  Fills the plan
-// table on the current device and waits for it, so that launches on any stream may use it.
+// plan(arr_address, n_seg, L, table) -> (whether every live row starts on a multiple of 8 positions of its block's walk, how much of what
+// the blocks walk is live, in percent).  Fills the plan table on the current device and waits for it, so that launches on any stream
+// may use it.
 PyObject* py_plan(PyObject*, PyObject* args) {
     unsigned long long addr;
     int n_seg, L;
@@ -596,9 +591,11 @@ PyObject* py_plan(PyObject*, PyObject* args) {
         if (rc) return refused("splat_attention_plan_report", rc, shares);
         if (!wait_for(stream, shares)) return nullptr;
         bool aligned = true;
-        for (int64_t b = 0; b < blocks; ++b) aligned = aligned && sh[4 * b] == 0;
+        int64_t walked = 0, live = 0;
+        for (int64_t b = 0; b < blocks; ++b) aligned = aligned && sh[4 * b] == 0, walked += sh[4 * b + 1] * int64_t(64 * 128), live += sh[4 * b + 2];
         share_buffers()->give(std::move(shares));
-        return PyBool_FromLong(aligned);
+        const long percent = walked > 0 ? (long)std::clamp<int64_t>((100 * live + walked - 1) / walked, 1, 100) : 1;
+        return Py_BuildValue("Nl", PyBool_FromLong(aligned), percent);
     } catch (const std::exception& e) {
         return raise_std(e);
     }
@@ -679,8 +676,8 @@ PyObject* py_bind(PyObject*, PyObject* args) {
         fn = reinterpret_cast<std::remove_reference_t<decltype(fn)>>(static_cast<uintptr_t>(PyLong_AsUnsignedLongLong(o)));
         return !PyErr_Occurred();
     };
-    if (!take("splat_last_error", api.last_error) || !take("splat_attention_fwd_planned", api.fwd_planned) ||
-        !take("splat_attention_fwd_stats", api.fwd_stats) || !take("splat_transpose_keys", api.transpose_keys) ||
+    if (!take("splat_last_error", api.last_error) || !take("splat_attention_fwd_hinted", api.fwd_hinted) ||
+        !take("splat_transpose_keys", api.transpose_keys) ||
         !take("splat_attention_bwd", api.bwd) || !take("splat_attention_bwd_keys", api.bwd_keys) ||
         !take("splat_attention_bwd_f32", api.bwd_f32) || !take("splat_attention_bwd_keys_f32", api.bwd_keys_f32) || !take("splat_sddmm", api.sddmm) ||
         !take("splat_sddmm_probs", api.sddmm_probs) || !take("splat_sddmm_planned", api.sddmm_planned) ||
