@@ -100,8 +100,10 @@ def rsddmm_launcher(x: torch.Tensor, y: torch.Tensor, output: torch.Tensor,
     [B, H, L], contiguous: every row's log of its sum of exp(scale * score), as the fused forward hands it out) the
     stored value is exp(scale * score - lse[row]), the row's softmax probability, instead of the score.
     ``plan``: the mask's plan table (``ACSRSegments.plan``); by default the launches that use one (16-bit types, d a multiple
-    of 8 up to 128, at least 256 row blocks of 128 rows or rows of at most 256 slots) build it on their first call and keep it with the metadata, ``False``
-    launches without one.  The results are the same bit for bit.
+    of 8 up to 128, rows of K contiguous, at least 256 row blocks of 128 rows or rows of at most 256 slots) build it on their first
+    call and keep it with the metadata, ``False`` launches without one.  The results are the same bit for bit, but for K^T with
+    unit stride along the keys: by default such a K is turned into rows first where that is faster (16-bit types, d up to 64, at
+    least 64 row blocks), with a plan given or ``False`` it is read in place, and the two differ in the order of the float32 additions.
     Returns (output, sTod_linear_transformations, sTod_translations, nnzs)."""
     for name, t in (("x", x), ("y", y), ("output", output)):
         _hip.require_device_tensor(t, name)

@@ -192,7 +192,7 @@ PyObject* py_mask(PyObject*, PyObject* args) {
 }
 
 // ---- fused forward -------------------------------------------------------------------------------------------------------
-// 1: launched, 0: not an ordinary case, < 0 or > 1 after `rc` was set: failed
+// kNo: not an ordinary case, nothing was done; kYes: launched; kFailed: the library refused, its code is in `rc`
 enum class Did { kNo, kYes, kFailed };
 
 Did forward(const Mask& m, const at::Tensor& q, at::Tensor kT, const at::Tensor& v, const at::Tensor& out, double scale, float* lse,
@@ -430,11 +430,11 @@ PyObject* py_sddmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const double scale = PyFloat_AsDouble(a[4]);
         if (scale == -1.0 && PyErr_Occurred()) return nullptr;
         int rc = 0;
-        // K^T with the keys contiguous is read in place by the general kernel only.  Up to d = 64 a pass that turns it and the kernel of
-        // thin wavefronts on the copy take less (the three operators, bfloat16: 64 heads of 4096 rows, 33 slots, d = 32: 114 -> 92 us;
-        // 512 slots, d = 64: 300 -> 263; 4 heads of 4001 rows, 301 slots, d = 64: 49 -> 43), beyond it the copy costs as much as it
-        // gives (64 heads of 2048 rows, 255 slots: d = 80 122 -> 125, d = 96 126 -> 129), and so does its launch below 64 row blocks
-        // (one head of 200 rows: 21 -> 25).
+        // K^T with the keys contiguous is read in place by the general kernel only.  Up to d = 64 a pass that turns it and a kernel on
+        // the copy take less: the kernel of thin wavefronts where the launch has its shape (the three operators, bfloat16: 64 heads of
+        // 4096 rows, 33 slots, d = 32: 114 -> 92 us; 512 slots, d = 64: 300 -> 263), in launches of fewer than 256 row blocks of more
+        // than 256 slots the general kernel, which is faster on rows of K as well (4 heads of 4001 rows, 301 slots, d = 64: 49 -> 43).  Beyond d = 64 the copy costs as much as it gives (64 heads of 2048 rows, 255 slots: d = 80 122 -> 125,
+        // d = 96 126 -> 129), and so does its launch below 64 row blocks (one head of 200 rows: 21 -> 25).
         const bool turned = code != SPLAT_F32 && out_code == code && d % 8 == 0 && d <= 64 && B * H * ((L + 127) / 128) >= 64;
         if ((m->max_step >= 2 || turned) && y.stride(3) == 1 && y.stride(2) != 1) {
             if (y.stride(2) < keys) Py_RETURN_FALSE;

@@ -33,8 +33,6 @@ int check_launch(const char* what);
 // process that uses several GPUs needs it on each): `done` is a bit mask over device ordinals, one per kernel.
 int reserve_dynamic_lds(uint64_t* done, const void* kernel, size_t bytes, const char* who);
 
-constexpr int kWave = 64;
-
 // f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>)
 template <int N, int I = 0, typename F>
 __host__ __device__ __forceinline__ void static_for(F&& f) {
@@ -94,15 +92,6 @@ __device__ __forceinline__ void mma16(f32x4v& acc, const Frag<f16>& a, const Fra
 __device__ __forceinline__ constexpr int acc_row(int j, int g) { return 8 * (j >> 2) + 4 * g + (j & 3); }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
-
-template <typename T>
-__device__ __forceinline__ T from_float(float x) {
-    return (T)x;
-}
-template <typename T>
-__device__ __forceinline__ float to_float(T x) {
-    return (float)x;
-}
 
 // Store a float as element `idx` of a buffer whose element type is chosen at run time.
 __device__ __forceinline__ void store_as(void* base, int64_t idx, float x, int dtype) {

@@ -103,7 +103,6 @@ __device__ __forceinline__ void dma4(const void* src, char* lds_block) {
                  : "s"(lds_address(lds_block)), "v"(src)
                  : "memory", "m0");
 }
-__device__ __forceinline__ void dma_wait_all() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // Copy a ROWS x ROWB-byte tile into LDS; row r comes from row_ptr(r) (16-byte aligned, ROWB readable bytes).
 // Each wavefront issues ROWS*ROWB/4096 instructions of 1 KiB.
@@ -120,22 +119,6 @@ __device__ __forceinline__ void dma_tile(char* tile, int wave, int lane, RowPtr 
         const int c = logical_chunk<ROWB, SWZ>(row, pc);
         dma16(reinterpret_cast<const char*>(row_ptr(row)) + c * 16, tile + q * 1024);
     }
-}
-
-// K fragment (8 consecutive contraction values of row `row`) from a swizzled row-major tile.
-template <typename T, int ROWB>
-__device__ __forceinline__ Frag<T> lds_frag_row_swz(const char* tile, int row, int elem_col) {
-    Frag<T> f;
-    if constexpr (sizeof(T) == 2) {
-        u32x4 r = *reinterpret_cast<const u32x4*>(tile + lds_off<ROWB, true>(row, elem_col * 2));
-        f.v = __builtin_bit_cast(typename Frag<T>::vec, r);
-    } else {
-        u32x4 r0 = *reinterpret_cast<const u32x4*>(tile + lds_off<ROWB, true>(row, elem_col * 4));
-        u32x4 r1 = *reinterpret_cast<const u32x4*>(tile + lds_off<ROWB, true>(row, elem_col * 4 + 16));
-        u32x8 r = __builtin_shufflevector(r0, r1, 0, 1, 2, 3, 4, 5, 6, 7);
-        f.v = __builtin_bit_cast(typename Frag<T>::vec, r);
-    }
-    return f;
 }
 
 typedef __attribute__((address_space(3))) const u32x4 lds_u32x4;
