@@ -1,5 +1,8 @@
 """The autograd node of the native host path (csrc/host_ext.cpp) where a program does more than call backward: it must do what
 the Python function that it stands in for does."""
+import gc
+import threading
+
 import pytest
 import torch
 import torch.autograd.forward_ad as forward_ad
@@ -130,3 +133,82 @@ def test_gradients_of_sums_arrive_with_strides_of_zero(dev, dtype, d, dims):
         got = torch.autograd.grad(out.sum(dim=dims, keepdim=True), x, up, retain_graph=True)
         want = torch.autograd.grad(out, x, up.expand_as(out).contiguous())
         assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("reentrant", [False, True])
+def test_checkpointing_gives_the_same_gradients(dev, reentrant):
+    from torch.utils.checkpoint import checkpoint
+    attn, x = _module(dev), _operands(dev)
+    want = _gradients(lambda q, k, v: attention_with_grad(q, k, v, attn), x)
+    up = torch.linspace(-1, 1, want[0].numel(), device=dev).view(want[0].shape).to(want[0].dtype)
+    out = checkpoint(lambda q, k, v: attention_with_grad(q, k, v, attn), *x, use_reentrant=reentrant)
+    out.backward(up)
+    assert torch.equal(out, want[0]) and all(torch.equal(t.grad, g) for t, g in zip(x, want[1:]))
+
+
+def test_the_backward_outlives_the_module(dev):
+    """What the backward reads of the mask belongs to the node: metadata and plans of a module that is gone, with their memory
+    written over by whatever is allocated next."""
+    x = _operands(dev)
+    want = _gradients(lambda q, k, v: attention_with_grad(q, k, v, _module(dev)), x)
+    attn = _module(dev)
+    out = attention_with_grad(*x, attn)
+    del attn
+    gc.collect()
+    rubbish = [torch.full((n,), -1, dtype=torch.int32, device=dev) for n in (64, 128, 256, 320, 512, 1024, 4096, 16384) for _ in range(32)]
+    got = torch.autograd.grad(out, x, torch.linspace(-1, 1, out.numel(), device=dev).view(out.shape).to(out.dtype))
+    assert all(torch.equal(a, b) for a, b in zip(got, want[1:])) and len(rubbish) == 256
+
+
+def test_the_graph_is_freed_kept_and_guarded_as_usual(dev):
+    attn, x = _module(dev), _operands(dev)
+    out = attention_with_grad(*x, attn)
+    first = torch.autograd.grad(out.sum(), x, retain_graph=True)
+    again = torch.autograd.grad(out.sum(), x)
+    assert all(torch.equal(a, b) for a, b in zip(first, again))
+    with pytest.raises(RuntimeError, match="second time"):
+        torch.autograd.grad(out.sum(), x)
+    out = attention_with_grad(*x, attn)
+    with torch.no_grad():
+        x[1].mul_(2)
+    with pytest.raises(RuntimeError, match="inplace operation"):
+        torch.autograd.grad(out.sum(), x)
+
+
+@pytest.mark.parametrize("which", [0, 1, 2])
+def test_hooks_and_inputs_that_need_no_gradient(dev, which):
+    attn, x = _module(dev), _operands(dev)
+    want = torch.autograd.grad(attention_with_grad(*x, attn).sum(), x)[which]
+    alone = [t if i == which else t.detach() for i, t in enumerate(x)]
+    out = attention_with_grad(*alone, attn)
+    seen = []
+    out.grad_fn.register_hook(lambda grads_in, grads_out: seen.append((len(grads_in), len(grads_out))))
+    x[which].register_hook(lambda g: 2 * g)
+    got, = torch.autograd.grad(out.sum(), alone[which])
+    assert torch.equal(got, 2 * want) and seen == [(3, 1)]
+
+
+def test_threads_with_streams_of_their_own(dev):
+    """Forward and backward of one module from two threads at once, each on its stream: every call has tensors of its own."""
+    attn = _module(dev)
+    want = _gradients(lambda q, k, v: attention_with_grad(q, k, v, attn), _operands(dev))
+    torch.cuda.synchronize()
+    found, failed = [], []
+
+    def work():
+        try:
+            with torch.cuda.stream(torch.cuda.Stream(device=dev)):
+                x = _operands(dev)
+                for _ in range(20):
+                    found.append(_gradients(lambda q, k, v: attention_with_grad(q, k, v, attn), x))
+                torch.cuda.current_stream(dev).synchronize()
+        except Exception as e:  # noqa: BLE001
+            failed.append(e)
+    threads = [threading.Thread(target=work) for _ in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not failed and len(found) == 40
+    assert all(torch.equal(a, b) for got in found for a, b in zip(got, want))
