@@ -610,7 +610,7 @@ at::Tensor part_of(const at::Tensor& record, int64_t offset, int64_t n) {
 }
 
 // build(mask, block_height) -> ((9 tensors), (9 tensors), T, failed rows, smallest step, largest step, rows off phase): the arrays
-// of a record and of its duplicate, dTos_lin, dTos_trans, sTod_lin, sTod_trans, nnz, row_first, row_last, span_start, span_end.
+// of a record and of its duplicate (without row_last), dTos_lin, dTos_trans, sTod_lin, sTod_trans, nnz, row_first, row_last, span_start, span_end.
 // Waits for the stream (T comes back as a number).  None when the case is not an ordinary one.
 PyObject* py_build(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 2) return PyErr_Format(PyExc_TypeError, "build takes 2 arguments");
@@ -647,6 +647,11 @@ PyObject* py_build(PyObject*, PyObject* const* a, Py_ssize_t n) {
             sets[k] = PyTuple_New(9);
             if (!sets[k]) return nullptr;
             for (int i = 0; i < 9; ++i) {
+                if (k == 1 && i == 6) {  // (the caller's set: nobody reads its row_last)
+                    Py_INCREF(Py_None);
+                    PyTuple_SET_ITEM(sets[k], i, Py_None);
+                    continue;
+                }
                 at::Tensor t;
                 if (i == 5 || i == 6)
                     t = part_of(extents, (2 * k + i - 5) * row_step, rows);
