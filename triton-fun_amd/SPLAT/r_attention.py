@@ -250,9 +250,10 @@ class RegularAttention(nn.Module):
         """Gradients (dq, dk, dv), each [B, H, L, d], of ``forward(x)`` for x = [q, kT, v] and the upstream gradient
         ``grad_out`` [B, H, L, d].  The ACSR of the transposed mask is built on first use; see ``r_backward``.  ``lse``
         and ``out``: the rows' statistic and the output of ``forward_with_stats`` for the same x.  Where the fused
-        forward applies (one dtype, d in {64, 128}) the gradients come from the fused backward kernel, which needs both
+        forward applies (one dtype, d in {64, 128}) the gradients come from the fused backward kernels, which need both
         (a forward is run here when one is missing); otherwise, or with ``fused=False``, from the operators composed over
-        compressed matrices, which ``lse`` spares the softmax pass.  ``sparse_rows``: how the fused kernel takes segments
+        compressed matrices, which ``lse`` spares the softmax pass.  ``fused=True`` insists on the kernels for 16-bit types: it
+        raises for float32, whose fused kernels the default takes.  ``sparse_rows``: how the fused kernel takes segments
         of the transposed mask that keep few keys with long columns (``r_backward.attention_backward_fused``)."""
         from r_backward import attention_backward, attention_backward_fused
         q, kT, v = x
@@ -262,7 +263,7 @@ class RegularAttention(nn.Module):
         if fused is None:
             fused = fusable
         elif fused and not (fusable and q.dtype in (torch.float16, torch.bfloat16)):
-            raise _hip.SplatError("the fused backward needs a 16-bit dtype shared by all tensors and d in {64, 128}")
+            raise _hip.SplatError("fused=True needs a 16-bit dtype shared by all tensors and d in {64, 128}")
         if not fused:
             return attention_backward(q, kT, v, grad_out, self.segments, self._segments_t, self.scale, lse)
         if lse is None or out is None:

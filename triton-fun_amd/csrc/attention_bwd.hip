@@ -633,8 +633,8 @@ static int run_bwd_keys(const BwdParams& dk, const BwdParams& dv, int d, hipStre
         // Launches of at most four row blocks a CU: one walk by pairs of wavefronts (attention_bwd_pair.hip), which puts eight
         // wavefronts on a row block where the two launches below put four.  Training steps, bfloat16: 128 row blocks, window 512:
         // 82 -> 69 us; 512 blocks, two segments: 128 -> 114; 1024 blocks, window 32: 135 -> 133.  Beyond, the beginnings and ends
-        // of its workgroups, which nothing else on the CU covers, cost what the fifth product does: 2048 blocks, window 128:
-        // 279 against 295 us, window 512: 491 against 491; 4096 blocks, dilated 512 / 2: 986 against 972.
+        // of its workgroups, which nothing else on the CU covers, cost what the fifth product does (the two launches -> the pairs):
+        // 2048 blocks, window 128: 279 -> 295 us, window 512: 491 -> 491; 4096 blocks, dilated 512 / 2: 986 -> 972.
         BwdParams dkv = dk;
         dkv.out2 = dv.out;
         return launch_bwd_pair<T>(dkv, st);

@@ -9,7 +9,9 @@
 // dK and the other dV, and what the other one needs (dS of the one half, P of the other: 2 KiB as ready B operands) goes through
 // LDS.  The accumulating products run one tile behind the scores, so that the pair needs no barrier but the tile's own and the
 // exponentials issue between matrix instructions that do not wait for them; the tiles come through a ring of three stages.
-// One workgroup of 133 KiB a CU: two wavefronts a SIMD, as two workgroups of the four-wavefront kernel would give.
+// One workgroup of 133 KiB a CU: two wavefronts a SIMD, as two workgroups of the four-wavefront kernel would give.  A second one
+// would take more than a smaller ring: 64 registers of accumulators and 64 of K and V fragments are all that the 128 registers of
+// a wavefront at four a SIMD hold.
 // Bound: the latency of the walk (its launches leave the chip part idle); where they fill it, what one workgroup a CU leaves
 // uncovered: B = 2, H = 32, L = 8192, dilated 512 / 2, bfloat16: 545 us against 322 + 233 for the two launches.  Measured and not
 // taken there: one role's wavefronts at a higher priority 559, four or three fragments ahead instead of six 549 / 554.

@@ -13,7 +13,10 @@
 //     (Tiles of half or twice the size and rings of three measured equal or slower, up to 10 %.)
 //   * the layouts of tile_f32.hpp: 16-byte LDS reads throughout and no exchange of probabilities between lanes.
 // Measured against the 32x32x2 kernel it replaces (128 rows a workgroup, tiles of 64 keys): B = 32, H = 12, L = 1024, window 257,
-// d = 64: 347 -> 255 us (matrix units busy 63 % of the time); one head of 512 rows, window 64: 20.0 -> 9.8 us.
+// d = 64: 347 -> 255 us (matrix units busy 63 % of the time); one head of 512 rows, window 64: 20.0 -> 9.8 us.  Masks with little or
+// nothing to skip, where a read from LDS serves half the rows it served there, gain less and lose nothing: 64 heads of 4096 rows,
+// blocks of 512 d = 64 571 -> 521 us, d = 128 1197 -> 1039, no mask 2224 -> 2100 and 4972 -> 4112; 32 heads of 2048 rows, blocks of
+// 512 147 -> 143 and 315 -> 308, of 128 45 -> 42 and 94 -> 95; one head of 1024 rows, no mask 82 -> 49 and 156 -> 87.
 #include "tile_f32.hpp"
 
 namespace splat {
