@@ -67,3 +67,29 @@ def test_native_operators_refuse_what_the_launchers_check(dev):
         attn([q[:, :, :128], q[:, :, :128].transpose(2, 3), q[:, :, :128]])
     assert not hip.host().forward(attn._native, q, q.float().transpose(2, 3), q, attn.rspmm_output, 1.0)
     assert not hip.host().softmax(attn.segments.native(L, dev, False), q, q[:, :1])
+
+
+def test_running_out_of_memory_is_the_error_a_program_catches(dev):
+    """Allocations of the native path that the device's limit refuses raise what torch.empty raises, in the forward and in the
+    backward, and the call works again with room."""
+    L, H, d = 8192, 16, 128  # an output of 32 MB
+    attn = RegularAttention(1, L, H, d, A.causal_windowed_pattern(L, 31), 16, 16, dev, torch.bfloat16, scale=d ** -0.5)
+    x = [torch.randn(1, H, L, d, device=dev).to(torch.bfloat16).requires_grad_(True) for _ in range(3)]
+    want = torch.autograd.grad(attention_with_grad(*x, attn).sum(), x)
+    out = attention_with_grad(*x, attn)
+    up = torch.ones_like(out)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    room = torch.cuda.get_device_properties(dev).total_memory
+    fits = []
+    try:
+        torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved(dev) / room, dev)
+        with pytest.raises(torch.OutOfMemoryError):
+            for _ in range(64):  # what is reserved and free
+                fits.append(attention_with_grad(*x, attn))
+        with pytest.raises(torch.OutOfMemoryError):
+            torch.autograd.grad(out, x, up, retain_graph=True)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, dev)
+    got = torch.autograd.grad(out, x, up)
+    assert all(torch.equal(a, b) for a, b in zip(got, want)) and len(fits) < 64

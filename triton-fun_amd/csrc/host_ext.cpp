@@ -25,6 +25,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <stdexcept>
 #include <string>
@@ -154,8 +155,9 @@ PyObject* raise_rc(const char* what, int rc) {
     PyErr_SetString(g_error, failure(what, rc).c_str());
     return nullptr;
 }
-PyObject* raise_std(const std::exception& e) {
-    if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
+// The C++ exception being handled as the Python error that PyTorch's own functions raise for it (out of memory among them).
+PyObject* raise_current() {
+    if (!PyErr_Occurred()) torch::translate_exception_to_python(std::current_exception());
     return nullptr;
 }
 
@@ -241,8 +243,8 @@ PyObject* py_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const Did did = forward(*m, *q, *kT, *v, *out, scale, nullptr, &rc);
         if (did == Did::kFailed) return raise_rc("splat_attention_fwd_hinted", rc);
         return PyBool_FromLong(did == Did::kYes);
-    } catch (const std::exception& e) {
-        return raise_std(e);
+    } catch (...) {
+        return raise_current();
     }
 }
 
@@ -397,8 +399,8 @@ PyObject* py_attend(PyObject*, PyObject* const* a, Py_ssize_t n) {
     } catch (const Failure& e) {
         PyErr_SetString(g_error, e.what());
         return nullptr;
-    } catch (const std::exception& e) {
-        return raise_std(e);
+    } catch (...) {
+        return raise_current();
     }
 }
 
@@ -454,8 +456,8 @@ PyObject* py_sddmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
 #undef SPLAT_ARGS
         if (rc) return raise_rc("splat_sddmm", rc);
         Py_RETURN_TRUE;
-    } catch (const std::exception& e) {
-        return raise_std(e);
+    } catch (...) {
+        return raise_current();
     }
 }
 
@@ -476,8 +478,8 @@ PyObject* py_softmax(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                    code, out_code, stream_of(*x));
         if (rc) return raise_rc("splat_softmax", rc);
         Py_RETURN_TRUE;
-    } catch (const std::exception& e) {
-        return raise_std(e);
+    } catch (...) {
+        return raise_current();
     }
 }
 
@@ -506,8 +508,8 @@ PyObject* py_spmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
                           L, keys, w, T, code, out_code, st);
         if (rc) return raise_rc("splat_spmm", rc);
         Py_RETURN_TRUE;
-    } catch (const std::exception& e) {
-        return raise_std(e);
+    } catch (...) {
+        return raise_current();
     }
 }
 
@@ -558,16 +560,16 @@ PyObject* refused(const char* what, int rc, at::Tensor& shares) {
 // given back either.
 bool wait_for(const c10::hip::HIPStream& stream, at::Tensor& shares) {
     PyThreadState* const released = PyEval_SaveThread();
-    std::string failed_wait;
+    std::exception_ptr failed;
     try {
         c10::hip::stream_synchronize(stream.stream());
-    } catch (const std::exception& e) {
-        failed_wait = e.what();
+    } catch (...) {
+        failed = std::current_exception();
     }
     PyEval_RestoreThread(released);
-    if (failed_wait.empty()) return true;
+    if (!failed) return true;
     new at::Tensor(std::move(shares));
-    PyErr_SetString(PyExc_RuntimeError, failed_wait.c_str());
+    torch::translate_exception_to_python(failed);
     return false;
 }
 
@@ -596,8 +598,8 @@ PyObject* py_plan(PyObject*, PyObject* args) {
         share_buffers()->give(std::move(shares));
         const long percent = walked > 0 ? (long)std::clamp<int64_t>((100 * live + walked - 1) / walked, 1, 100) : 1;
         return Py_BuildValue("Nl", PyBool_FromLong(aligned), percent);
-    } catch (const std::exception& e) {
-        return raise_std(e);
+    } catch (...) {
+        return raise_current();
     }
 }
 
@@ -663,8 +665,8 @@ PyObject* py_build(PyObject*, PyObject* const* a, Py_ssize_t n) {
             }
         }
         return Py_BuildValue("NNiiiii", sets[0], sets[1], t_max, bad, step_min, step_max, off);
-    } catch (const std::exception& e) {
-        return raise_std(e);
+    } catch (...) {
+        return raise_current();
     }
 }
 
