@@ -209,8 +209,10 @@ def test_metadata_with_native_handles_copies_and_saves(monkeypatch):
 
     def native(on):
         return ACSRSegments.single(*arrays[:3], on, arrays[4], 1).native(4, torch.device("cuda", 0), False)
+    without = native(t)
+    t.splat_first_col = torch.zeros(4, dtype=torch.int32)
     handle = native(t)
-    assert type(handle).__name__ == "PyCapsule" and native(t) is handle
+    assert type(handle).__name__ == "PyCapsule" and native(t) is handle and handle is not without
     file = io.BytesIO()
     torch.save(t, file)
     file.seek(0)

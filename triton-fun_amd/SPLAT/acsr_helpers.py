@@ -529,9 +529,11 @@ class ACSRSegments:
         kept = holder.__dict__.get("splat_native")
         if type(kept) is not _NativeMasks:
             kept = holder.__dict__["splat_native"] = _NativeMasks()
-        # (the tensors' addresses: separate tensors may come with one sTod_translations and other companions)
+        # (the tensors' addresses: separate tensors may come with one sTod_translations and other companions, and the first columns
+        # may be attached to it after a call)
+        fc = self.first_cols[0]
         key = (L, device.index, with_plan) if holder is self else \
-            (L, device.index, with_plan, *(t.data_ptr() for t in self.tuples[0][:5]))
+            (L, device.index, with_plan, *(t.data_ptr() for t in self.tuples[0][:5]), fc.data_ptr() if fc is not None else 0)
         mask = kept.get(key)
         if mask is None:
             if torch.cuda.is_current_stream_capturing():
