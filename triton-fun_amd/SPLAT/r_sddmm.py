@@ -67,22 +67,13 @@ def _strides4(t: torch.Tensor, name: str):
 _HALF = (torch.float16, torch.bfloat16)
 
 
-def _takes_a_plan(x, output, k_rows: bool, T: int) -> bool:
+def _takes_a_plan(x, output, blocks: int, d: int, k_rows: bool, T: int) -> bool:
     """Whether this launch runs the kernel that reads a plan table (the library decides by the same rules and ignores the
     plan otherwise, so that building one would be for nothing): 16-bit types, d up to 128 in whole 16-byte pieces, rows of K
     contiguous (``k_rows``), and at least 256 row blocks or rows of at most 256 slots (fewer blocks of longer rows are better off
     with the general kernel's split of the key range)."""
-    B, H, L, d = x.shape
-    if x.dtype not in _HALF or output.dtype != x.dtype or d % 8 != 0 or d > 128 or not k_rows:
-        return False
-    return T <= 256 or B * H * ((L + 127) // 128) >= 256
-
-
-def _keys_become_rows(x, y, segs: ACSRSegments) -> bool:
-    """Whether the native host path hands the kernels rows of K: they are rows already, or it turns K first, which it does for
-    gathered rows and, up to d = 64, in launches of at least 64 row blocks (csrc/host_ext.cpp)."""
-    B, H, L, d = x.shape
-    return y.stride(2) == 1 or (d <= 64 and B * H * ((L + 127) // 128) >= 64) or segs.gathered
+    return (k_rows and d % 8 == 0 and d <= 128 and (T <= 256 or blocks >= 256) and x.dtype in _HALF
+            and output.dtype == x.dtype)
 
 
 def rsddmm_launcher(x: torch.Tensor, y: torch.Tensor, output: torch.Tensor,
@@ -112,7 +103,12 @@ def rsddmm_launcher(x: torch.Tensor, y: torch.Tensor, output: torch.Tensor,
     segs = segments or ACSRSegments.single(dTos_linear_transformations, dTos_translations,
                                            sTod_linear_transformations, sTod_translations, nnzs, trailing_dim)
     if plan is None and x.dim() == 4 and y.dim() == 4 and output.shape[-1] == trailing_dim:
-        mask = segs.native(x.shape[2], x.device, _takes_a_plan(x, output, _keys_become_rows(x, y, segs), trailing_dim))
+        B, H, L, d = x.shape
+        blocks = B * H * ((L + 127) // 128)
+        # (the native path hands the kernels rows of K where they are rows already, where rows are gathered, and, up to d = 64, in launches
+        # of at least 64 row blocks, for which it turns K first: csrc/host_ext.cpp)
+        k_rows = y.stride(2) == 1 or (d <= 64 and blocks >= 64) or segs.gathered
+        mask = segs.native(L, x.device, _takes_a_plan(x, output, blocks, d, k_rows, trailing_dim))
         if mask is not None and _hip.host().sddmm(mask, x, y, output, 1.0 if scale is None else scale, lse):
             return (output, sTod_linear_transformations, sTod_translations, nnzs)
     B, H, L, d = x.shape
@@ -138,7 +134,7 @@ def rsddmm_launcher(x: torch.Tensor, y: torch.Tensor, output: torch.Tensor,
             raise _hip.SplatError(f"lse must be a contiguous float32 tensor of shape {(B, H, L)} on {dev}")
     # (building the table synchronises once, which a stream under capture must not do: such a call uses a table only if an
     # earlier call has left one)
-    if plan is None and _takes_a_plan(x, output, y.stride(2) == 1, trailing_dim) \
+    if plan is None and _takes_a_plan(x, output, B * H * ((L + 127) // 128), d, y.stride(2) == 1, trailing_dim) \
             and (segs.has_plan(L, dev) or not torch.cuda.is_current_stream_capturing()):
         plan = segs.plan(L, dev)
     if plan is not None and plan is not False:
