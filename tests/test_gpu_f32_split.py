@@ -1,0 +1,69 @@
+"""The float32 forward on split operands against float64: what the parts hold, and what they do not (taken again in
+float32 arithmetic)."""
+import pytest
+import torch
+
+import acsr_helpers as A
+from r_attention import RegularAttention
+
+pytestmark = pytest.mark.gpu
+
+
+def case(dev, masks, B, H, L, d, seed, scale_q=1.0, scale_k=1.0, scale_v=1.0):
+    g = torch.Generator().manual_seed(seed)
+    q, k, v = (torch.randn(B, H, L, d, generator=g) * s for s in (scale_q, scale_k, scale_v))
+    live = sum(m.device_mask(dev) for m in masks).cpu() > 0
+    s = (q.double() @ k.double().transpose(2, 3) * d ** -0.5).masked_fill(~live, float("-inf"))
+    want = torch.softmax(s, -1) @ v.double()
+    attn = RegularAttention(B, L, H, d, masks, 16, 16, dev, torch.float32, scale=d ** -0.5)
+    return attn, [q.to(dev), k.to(dev).transpose(2, 3), v.to(dev)], want, live
+
+
+def error(got, want):
+    return float((got.double().cpu() - want).norm() / want.norm())
+
+
+# scores of N(0, 1) operands are rounded to 2^-24 of up to 5 or so, the sums behind them as often as they have terms: 1e-6 is three
+# times what that comes to, and far below what an operand's missing part would give (2^-17)
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("q,k,v", [(1, 1, 1), (1, 1, 1e-30), (1, 1, 1e-36), (1, 1, 1e36), (1e-20, 1e20, 1), (1e-35, 1e35, 1), (1e35, 1e-35, 1), (1e-36, 1, 1)])
+def test_scales_of_the_operands(dev, d, q, k, v):
+    attn, x, want, _ = case(dev, [A.causal_windowed_pattern(401, 149)], 1, 2, 401, d, d, q, k, v)
+    assert error(attn(x), want) <= 1e-6
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_scores_that_rise_along_the_walk(dev, d):
+    """Later keys outrun the references of the first tiles by far more than an exponential holds."""
+    attn, x, want, _ = case(dev, [A.causal_windowed_pattern(300, 199)], 1, 2, 300, d, 3 * d)
+    x[1].mul_(torch.linspace(0.1, 60.0, 300, device=dev))
+    s = (x[0].double() @ x[1].double() * d ** -0.5).cpu()
+    live = A.causal_windowed_pattern(300, 199).device_mask(dev).cpu() > 0
+    want = torch.softmax(s.masked_fill(~live, float("-inf")), -1) @ x[2].double().cpu()
+    assert error(attn(x), want) <= 1e-6 * float(s.abs().max())  # a score's rounding is relative to it
+
+
+@pytest.mark.parametrize("keys_along", [False, True])
+@pytest.mark.parametrize("L,d", [(400, 64), (400, 128), (96, 64)])
+def test_values_that_are_not_finite_reach_the_rows_that_see_them(dev, L, d, keys_along):
+    w = 40
+    attn, x, want, live = case(dev, [A.causal_windowed_pattern(L, w - 1)], 1, 2, L, d, L + d)
+    clean = attn(x).clone()
+    x[2][:, :, 50, 3] = float("inf")
+    x[2][:, :, 50, 7] = 3.4e38  # above what a bfloat16 holds
+    x[1][:, 1, :, 9] = float("nan")
+    x[0][:, 0, 70, 2] = float("inf")
+    if keys_along:
+        x[1] = x[1].contiguous()
+    got = attn(x)
+    sees_v, sees_k = live[:, 50].to(dev), live[:, 9].to(dev)
+    assert bool(torch.isnan(got[:, 1, sees_k]).all()) and bool(torch.isnan(got[:, 0, 70]).all())
+    ok = sees_v.clone()
+    ok[70] = False
+    assert bool((got[:, 0, ok, 3] == float("inf")).all()) and bool((got[:, 0, ok, 7] > 1e35).all())
+    rest = torch.ones_like(got, dtype=torch.bool)
+    rest[:, 1, sees_k] = False
+    rest[:, 0, 70] = False
+    rest[:, :, sees_v, 3] = False
+    rest[:, :, sees_v, 7] = False
+    assert bool(torch.isfinite(got[rest]).all()) and float((got[rest] - clean[rest]).abs().max()) <= 1e-5

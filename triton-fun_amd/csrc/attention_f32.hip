@@ -1,40 +1,38 @@
 // Fused ACSR sparse-attention forward in float32 (online softmax), gfx950.
 //
-// Bound: the float32 matrix instructions (157 TFLOP/s nominal on this chip, 154 measured in a large product: a sixteenth of
-// what the 16-bit ones give), so everything here serves two ends: no matrix work on masked positions, and matrix work on every
-// SIMD at every moment.
-//   * 16x16x4 instructions: a wavefront owns 16 query rows and takes keys in subtiles of 16, skipping the subtiles outside its
-//     rows' spans (a window of 257 costs 272 + 15 positions on average; the 32x32x2 form, with 32 rows and tiles of 64 keys,
-//     346).  Both forms run at the same rate.
-//   * little vector arithmetic: these matrix instructions run on the vector units (a loop of them takes 33 cycles each, with
-//     four v_fma beside each 46), so every address that can be wavefront-uniform is, and masks are built only where needed.
-//   * small tiles: 16 KB a stage (32 keys at d = 64, 16 at d = 128) in a ring of two, so that four workgroups fit a CU (three at
-//     d = 128, by registers) and one computes while another waits; 64 rows a workgroup, so that short problems spread over more CUs.
-//     (Tiles of half or twice the size and rings of three measured equal or slower, up to 10 %.)
-//   * the layouts of tile_f32.hpp: 16-byte LDS reads throughout and no exchange of probabilities between lanes.
-// Measured against the 32x32x2 kernel it replaces (128 rows a workgroup, tiles of 64 keys): B = 32, H = 12, L = 1024, window 257,
-// d = 64: 347 -> 255 us (matrix units busy 63 % of the time); one head of 512 rows, window 64: 20.0 -> 9.8 us.  Masks with little or
-// nothing to skip, where a read from LDS serves half the rows it served there, gain less and lose nothing: 64 heads of 4096 rows,
-// blocks of 512 d = 64 571 -> 521 us, d = 128 1197 -> 1039, no mask 2224 -> 2100 and 4972 -> 4112; 32 heads of 2048 rows, blocks of
-// 512 147 -> 143 and 315 -> 308, of 128 45 -> 42 and 94 -> 95; one head of 1024 rows, no mask 82 -> 49 and 156 -> 87.
-#include "tile_f32.hpp"
+// The float32 matrix instructions run at a sixteenth of the rate of the 16-bit ones (154 TFLOP/s in a large product), so both
+// products are taken on the latter, of operands split into three bfloat16 parts (split3.hpp: six products for one, three eighths
+// of the time, and closer to float64).  Bound: the 16-bit matrix instructions at the clock that the power limit leaves under
+// them, and the vector instructions beside them, 200 a tile and wavefront in about as many cycles, half of them splitting.
+//   * 16 rows a wavefront, 16x16x32 instructions, tiles of 32 positions, the layouts of attention_rows16.hip: 160 registers at
+//     d = 64, three wavefronts a SIMD (two at d = 128), which overlap each other's vector and matrix phases.
+//   * K and V are split once a workgroup: every thread holds its pieces of the next tile in registers, splits them, and writes the
+//     parts between two barriers into the one stage of planes.  A second stage that is written during the products costs the LDS of
+//     the third workgroup a CU (d = 64, 64 heads of 2048 rows, window 256 / 32: 72 / 35.4 us against 68 / 32.7; d = 128, of
+//     the second: 204 / 102 against 127 / 59), 128 rows a workgroup halve the splitting but leave one or two of them a CU
+//     (70 / 35.8 and 143 / 78), 32 rows a wavefront with the scores a tile ahead take 216 registers and run no faster.
+//   * 64 rows a workgroup, so that short problems spread over more CUs, and little that runs once: in a launch of few tiles the
+//     instructions of the beginning and the end come from memory (a barrier and a second pass for references that are left
+//     behind cost 1 of 8.6 us there).  Two groups of wavefronts that share the tiles of 64 rows and add up at the end: 14.4 for 16.3 at
+//     a window of 256 and one workgroup a CU, 8.1 for 7.6 at 32, and other bits for a walk that is planned than for one that is not.
+// Measured against the kernel on the float32 instructions that it replaces: B = 32, H = 12, L = 1024, window 257, d = 64: 252 -> 197 us;
+// 64 heads of 4096 rows, blocks of 512, d = 64 517 -> 376; 64 heads of 2048 rows, d = 128, window 256 180 -> 127, window 32 66 -> 59;
+// one head of 512 rows, window 64: 9.5 -> 8.7.  Relative error against float64 (norms) 2.5e-7 -> 1.6e-7 there, 4.0e-7 -> 3.0e-7 at
+// window 257, 6.6e-7 -> 5.4e-7 at blocks of 1024 and d = 128.
+#include "rows16.hpp"
+#include "split3.hpp"
 
 namespace splat {
 
-constexpr int kF32Stages = 2;
-
 template <int D, bool KT, bool PLANNED>
-__global__ __launch_bounds__(256, 3) void attn_fwd_f32_kernel(const AttnParams p) {
-    constexpr int BN = f32_tile(D), SUB = BN / 16, NSTAGE = kF32Stages, PD = NSTAGE - 1;
-    constexpr int KQ = D / 16;  // groups of 16 contraction values of the score product
-    constexpr int DH = D / 64;  // 64-column halves of the output
-    constexpr int V_ROWB = D * 4, K_ROWB = KT ? BN * 4 : D * 4;
-    constexpr int TILE = BN * D * 4, STAGE = 2 * TILE;
-    constexpr int NDMA = STAGE / 4096;  // copy instructions per wavefront and tile
-    constexpr int K_SWZ = KT ? (K_ROWB == 128 ? 2 : 0) : 1;
+__global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_fwd_f32_kernel(const AttnParams p) {
+    constexpr int BN = 32, ROWB = 2 * D, PLANE = BN * ROWB, TILE = 3 * PLANE;  // positions a tile; bytes of a row, a plane, an operand
+    constexpr int KS = D / 32, DT = D / 16;
+    constexpr int CPR = D / 8;                // 8-value pieces of a row
+    constexpr int NP = 2 * BN * CPR / 256;    // pieces a thread: the first half of them K's, the others V's
     static_assert(kPlanBM == 2 * kHalfRows && kBN % BN == 0, "half a row block of the plan per workgroup");
 
-    extern __shared__ __attribute__((aligned(1024))) char smem[];
+    extern __shared__ __attribute__((aligned(1024))) char smem[];  // three planes of K, three of V
     __shared__ SegPlan s_plan[SPLAT_MAX_SEGMENTS];
     __shared__ PlanScratch<kPlanBM> s_ps;
 
@@ -60,27 +58,18 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_f32_kernel(const AttnParams p
     float* ob = (float*)p.o + b * p.o_sb + h * p.o_sh;
     const int my_row = r0 + rs * (wave * 16 + n);
 
-    // ---- the lane's share of its Q row, resident: B operand of the score product ----
-    float q[D / 4];
+    // ---- Q, resident: B operand of S^T; requested now, split once the first tile is on its way ----
+    Frag<float> q_raw[KS];
     {
         const float* qr = qb + (int64_t)min(my_row, L - 1) * p.q_sl;
 #pragma unroll
-        for (int t = 0; t < KQ; ++t) {
-            if constexpr (KT) {  // instruction s takes d = 4s + g
-#pragma unroll
-                for (int j = 0; j < 4; ++j) q[4 * t + j] = qr[16 * t + 4 * j + g];
-            } else {
-                const f32x4 x = *reinterpret_cast<const f32x4*>(qr + 16 * t + 4 * g);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) q[4 * t + j] = x[j];
-            }
-        }
+        for (int ks = 0; ks < KS; ++ks) q_raw[ks] = global_frag<float>(qr + 32 * ks + 8 * g);
     }
 
     // ---- plan: the row block's walk, cut down to the tiles that this half of it sees ----
     const PlanRec* const pt = p.plan;
     const int n_rb = p.n_row_blocks;
-    if constexpr (!PLANNED) plan_segments<kPlanBM, kBN>(p.seg, p.n_seg, block_first_row(rb, kPlanBM, rs), rs, L, !KT, s_plan, &s_ps, tid);
+    if constexpr (!PLANNED) plan_segments<kPlanBM, kBN>(p.seg, p.n_seg, block_first_row(rb, kPlanBM, rs), rs, L, true, s_plan, &s_ps, tid);
     auto walk_of = [&](int sg) {
         HalfWalk w;
         w.seg = sg;
@@ -103,115 +92,98 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_f32_kernel(const AttnParams p
         }
         w.seg = p.n_seg, w.tile = 0, w.end = 0x7fffffff;
     };
-    int total = 0;
-    for (int sg = 0; sg < p.n_seg; ++sg) {
+    HalfWalk fetch;
+    fetch.seg = 0;
+    next_segment(fetch);
+    int total = fetch.end - fetch.tile;
+    for (int sg = fetch.seg + 1; sg < p.n_seg; ++sg) {
         const HalfWalk w = walk_of(sg);
         total += w.end - w.tile;
     }
-    total = __builtin_amdgcn_readfirstlane(total);
+    total = fetch.seg < p.n_seg ? __builtin_amdgcn_readfirstlane(total) : 0;
 
-    // ---- asynchronous copies of one tile: 1 KiB blocks, wavefront w issues blocks w, w + 4, ...  The vector arithmetic shares
-    // its units with the float32 matrix instructions, so a tile whose positions all exist is copied from running wavefront-
-    // uniform pointers and per-lane offsets that stay the same for the whole segment ----
-    constexpr int NI = TILE / 4096;  // blocks per wavefront and operand
-    constexpr int V_CPR = V_ROWB / 16, V_RPI = 1024 / V_ROWB, K_CPR = K_ROWB / 16, K_RPI = 1024 / K_ROWB;
-    auto issue_general = [&](const HalfWalk& w, int stage) {
-        const int j0 = w.tile * BN;
-        char* ks_w = smem + stage * STAGE;
-        auto key_row = [&](int row) { return min(max(w.pl.c0 + w.pl.cs * (j0 + row), 0), L - 1); };
-        dma_tile<float, V_ROWB, BN, 0>(ks_w + TILE, wave, lane, [&](int row) { return vb + (int64_t)key_row(row) * p.v_sl; });
-        if constexpr (KT) {
-            // rows = d, BN consecutive keys each (dense walk); a chunk past the last key is replaced by the last whole one
+    // ---- a tile's way into LDS: pieces of 8 values, by their position in the tile's rows.  K stored along the keys is turned here:
+    // lanes are keys, a piece is 8 loads, one of each d. ----
+    int pc_row[NP], pc_c[NP];  // tile row and piece of the row
+    uint32_t pc_to[NP];        // LDS address of its first part
+    const uint32_t smem_base = lds_address(smem);
 #pragma unroll
-            for (int i = 0; i < NI; ++i) {
-                const int blk = wave + 4 * i, flat = blk * 64 + lane;
-                const int row = flat / K_CPR;
-                const int c = min(w.pl.c0 + j0 + logical_chunk<K_ROWB, K_SWZ>(row, flat % K_CPR) * 4, L - 4);
-                dma16(kb + (int64_t)row * p.k_sd + c, ks_w + blk * 1024);
+    for (int i = 0; i < NP; ++i) {
+        const int f = (tid + 256 * i) % (BN * CPR);
+        const bool is_k = i < NP / 2;
+        const int row = KT && is_k ? f % BN : f / CPR, c = KT && is_k ? f / BN : f % CPR;
+        const int to = is_k ? c ^ swz<ROWB>(row) : (((c >> 1) ^ swz32<ROWB>(row)) << 1) | (c & 1);
+        pc_row[i] = row, pc_c[i] = c;
+        pc_to[i] = smem_base + (is_k ? 0 : TILE) + row * ROWB + to * 16;
+    }
+    f32x8 raw[NP];
+    // an operand of one head within 32-bit offsets, and strides that 24-bit products take
+    const int64_t k_far = KT ? p.k_sd * D + L : p.k_sl * L, v_far = p.v_sl * L;
+    const bool narrow = max(k_far, v_far) * 4 < ((int64_t)1 << 32) && max(KT ? p.k_sd : p.k_sl, p.v_sl) * 4 < (1 << 24) && p.k_sd >= 0;
+    auto load_next = [&](HalfWalk& w) {  // the tile the walk stands at, which moves on
+        const int c0 = w.pl.c0 + w.pl.cs * w.tile * BN;
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            const bool is_k = i < NP / 2;
+            const char* base = reinterpret_cast<const char*>(is_k ? kb : vb);
+            const int key = min(max(c0 + w.pl.cs * pc_row[i], 0), L - 1);
+            if (KT && is_k) {
+                if (narrow) {
+                    uint32_t off = __umul24(8 * pc_c[i], (uint32_t)p.k_sd * 4) + 4 * key;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e, off += (uint32_t)p.k_sd * 4) raw[i][e] = *reinterpret_cast<const float*>(base + off);
+                } else {
+                    const float* src = kb + (int64_t)(8 * pc_c[i]) * p.k_sd + key;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) raw[i][e] = src[e * p.k_sd];
+                }
+            } else {
+                const int64_t sl = is_k ? p.k_sl : p.v_sl;
+                if (narrow)
+                    raw[i] = global_frag<float>(reinterpret_cast<const float*>(base + (__umul24(key, (uint32_t)sl * 4) + 32 * pc_c[i]))).v;
+                else
+                    raw[i] = global_frag<float>(reinterpret_cast<const float*>(base) + key * sl + 8 * pc_c[i]).v;
             }
-        } else {
-            dma_tile<float, K_ROWB, BN, K_SWZ>(ks_w, wave, lane, [&](int row) { return kb + (int64_t)key_row(row) * p.k_sl; });
         }
-    };
-    uint32_t v_off = 0, k_off[NI];
-    const char *v_next = nullptr, *k_next = nullptr;
-    int64_t v_row = 0, k_row = 0;  // bytes from one tile row to the next
-    bool off_fits = true;          // the copy instruction takes a 32-bit offset
-    auto set_offsets = [&](const HalfWalk& w) {
-        v_row = (int64_t)p.v_sl * 4 * w.pl.cs;
-        k_row = KT ? (int64_t)p.k_sd * 4 : (int64_t)p.k_sl * 4 * w.pl.cs;
-        off_fits = v_row * V_RPI < ((int64_t)1 << 31) && k_row * K_RPI < ((int64_t)1 << 31);
-        v_off = (uint32_t)(v_row * (lane / V_CPR)) + (lane % V_CPR) * 16;
-#pragma unroll
-        for (int i = 0; i < NI; ++i)
-            k_off[i] = (uint32_t)(k_row * (lane / K_CPR)) +
-                       logical_chunk<K_ROWB, K_SWZ>((wave + 4 * i) * K_RPI + lane / K_CPR, lane % K_CPR) * 16;
-        const int64_t first = w.pl.c0 + (int64_t)w.pl.cs * BN * w.tile;
-        v_next = reinterpret_cast<const char*>(vb) + first * p.v_sl * 4 + wave * V_RPI * v_row;
-        k_next = reinterpret_cast<const char*>(kb) + (KT ? first * 4 : first * p.k_sl * 4) + wave * K_RPI * k_row;
-    };
-    // copy tile `w.tile` into the stage and move on (w: the fetching walk; its pointers stand at that tile)
-    auto issue_next = [&](HalfWalk& w, int stage) {
-        const int last = w.pl.c0 + w.pl.cs * (w.tile * BN + BN - 1);
-        if (off_fits && last < L && w.pl.c0 + w.pl.cs * w.tile * BN >= 0) {
-            char* ks_w = smem + stage * STAGE;
-#pragma unroll
-            for (int i = 0; i < NI; ++i) {
-                dma16_uniform(k_next + 4 * i * K_RPI * k_row, k_off[i], ks_w + (wave + 4 * i) * 1024);
-                dma16_uniform(v_next + 4 * i * V_RPI * v_row, v_off, ks_w + TILE + (wave + 4 * i) * 1024);
-            }
-        } else {
-            issue_general(w, stage);
-        }
-        v_next += BN * v_row;
-        k_next += KT ? (int64_t)(BN * 4) : BN * k_row;
         if (++w.tile >= w.end) {
             ++w.seg;
             next_segment(w);
-            if (w.seg < p.n_seg) set_offsets(w);
         }
     };
 
-    // ---- LDS read addresses: of stage 0, moved on once a tile ----
-    const uint32_t smem_base = lds_address(smem);
-    uint32_t k_addr[KT ? 1 : KQ];
-    if constexpr (KT)
-        k_addr[0] = smem_base + g * K_ROWB + n * 4;
-    else
+    // ---- LDS read addresses ----
+    const int tr_row = (lane & 15) >> 2, tr_byte = 8 * (lane & 3);  // transposing reads: lane s of a group reads row s / 4
+    uint32_t k_addr[KS], v_addr[DT];
 #pragma unroll
-        for (int t = 0; t < KQ; ++t) k_addr[t] = smem_base + lds_off<K_ROWB, true>(n, (16 * t + 4 * g) * 4);
-    uint32_t v_addr = smem_base + TILE + 4 * g * V_ROWB + n * 16;
+    for (int ks = 0; ks < KS; ++ks) k_addr[ks] = smem_base + lds_off<ROWB, true>(n, (32 * ks + 8 * g) * 2);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+        v_addr[dt] = smem_base + TILE + (4 * g + tr_row) * ROWB + (dt ^ swz32<ROWB>(4 * g + tr_row)) * 32 + tr_byte;
 
-    HalfWalk fetch, cur;
-    fetch.seg = 0;
-    next_segment(fetch);
-    if (fetch.seg < p.n_seg) set_offsets(fetch);
-    cur = fetch;
+    // the row windows of the first segment with tiles, then the first tile, are requested before Q is looked at
+    HalfWalk cur = fetch;
     PlanRec win_rec = {0, 0, 1, 0};
     if constexpr (PLANNED) {
-        if (cur.seg < p.n_seg) win_rec = pt[plan_row_at(n_rb, p.n_seg, rb, cur.seg, k0 + wave * 16 + n)];
+        if (total > 0) win_rec = pt[plan_row_at(n_rb, p.n_seg, rb, cur.seg, k0 + wave * 16 + n)];
     }
+    if (total > 0) load_next(fetch);
+    Split3 qf[KS];
+    float q_most = 0.f;
 #pragma unroll
-    for (int i = 0; i < PD; ++i) {
-        if (i < total) {
-            issue_next(fetch, i);
-        }
+    for (int ks = 0; ks < KS; ++ks) {
+        qf[ks] = split3(q_raw[ks].v);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) q_most = fmaxf(q_most, fabsf(q_raw[ks].v[e]));
     }
+    bool beyond = out_of_split(q_most);  // something that the split operands do not hold
 
-    f32x4 o[4 * DH];
+    f32x4 o[DT];
 #pragma unroll
-    for (int i = 0; i < 4 * DH; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int dt = 0; dt < DT; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const float c2 = p.scale_log2e, slack = kRescaleThreshold / c2;
     float m_ref = kNegBigA, l_run = 0.f;
-    const float c2 = p.scale_log2e;
-    RowState rows;
     bool entered = false;
-    int stage = 0, stage_pf = PD;
-
-#if defined(__HIP_DEVICE_COMPILE__)
-    // Q is in its registers before the loop, so that no wait of the compiler's for it holds up the copies in flight there
-#pragma unroll
-    for (int i = 0; i < D / 4; ++i) asm volatile("" ::"v"(q[i]));
-#endif
+    RowState rows;
 
     for (int it = 0; it < total; ++it) {
         if (!entered) {
@@ -228,105 +200,82 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_f32_kernel(const AttnParams p
             entered = true;
         }
         const int j0 = cur.tile * BN;
-
-        // this wavefront's copies of tile `it` have landed once only those of the later tiles are outstanding; after the
-        // barrier everybody's have, and everybody is done with tile it - 1, whose stage the next fetch overwrites
-        if (total - 1 - it >= PD - 1)
-            wait_loads<NDMA*(PD - 1)>();
-        else
-            wait_loads<0>();
-        __builtin_amdgcn_s_barrier();
-        if (it + PD < total) {
-            issue_next(fetch, stage_pf);
-            stage_pf = stage_pf + 1 == NSTAGE ? 0 : stage_pf + 1;
+        lds_barrier();  // everybody is done with tile it - 1
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            const Split3 s = split3(raw[i]);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) lds_store128(pc_to[i] + k * PLANE, __builtin_bit_cast(u32x4, s.p[k].v));
         }
+        if (it + 1 < total) load_next(fetch);
+        lds_barrier();  // tile `it` is there
 
         if (j0 + BN > rows.lo_min && j0 < rows.hi_max) {
-            auto sub_live = [&](int s) { return SUB == 1 || (j0 + 16 * s + 16 > rows.lo_min && j0 + 16 * s < rows.hi_max); };
-            const bool full = j0 >= rows.lo_max && j0 + BN <= rows.hi_min;
-            // Fragments are requested a phase ahead of their use (all of the tile's K now, V before the exponentials), outside
-            // the branches of the subtiles; the barriers to scheduling keep the compiler from moving the requests down again.
-            f32x4 kf[SUB][KQ];
+            // ---- S^T = K . Q^T, of two subtiles of 16 positions.  Fragments are requested ahead of their products, part k of a
+            // step as the one of the step before is done with ----
+            Frag<bf16> kf[2][3];
+            auto load_kf = [&](int ks, int k) {
 #pragma unroll
-            for (int u = 0; u < SUB; ++u)
-#pragma unroll
-                for (int t = 0; t < KQ; ++t) {
-                    if constexpr (KT) {
-                        const uint32_t blk = K_ROWB == 128 ? (u ^ ((g >> 1) & 1)) * 64 : 0;
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) kf[u][t][j] = lds_load_f32(k_addr[0] + blk + (16 * t + 4 * j) * K_ROWB);
-                    } else {
-                        kf[u][t] = lds_load_f32x4(k_addr[t] + 16 * u * K_ROWB);
-                    }
-                }
-            __builtin_amdgcn_sched_barrier(0);
-            f32x4 s[SUB];
-#pragma unroll
-            for (int u = 0; u < SUB; ++u) {
-                if (!sub_live(u)) {
-                    s[u] = f32x4{kNegBigA, kNegBigA, kNegBigA, kNegBigA};
-                    continue;
-                }
-                s[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int t = 0; t < KQ; ++t)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) mma4(s[u], kf[u][t][j], q[4 * t + j]);
-            }
-            f32x4 vf[2][4][DH];
-            auto load_v = [&](int u) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-#pragma unroll
-                    for (int hh = 0; hh < DH; ++hh) vf[u & 1][j][hh] = lds_load_f32x4(v_addr + (16 * u + j) * V_ROWB + 256 * hh);
+                for (int u = 0; u < 2; ++u) kf[u][k].v = __builtin_bit_cast(bf16x8, lds_load128(k_addr[ks] + k * PLANE + 16 * u * ROWB));
             };
-            load_v(0);
-            __builtin_amdgcn_sched_barrier(0);
-            if (!full) rows.mask_tile(s, j0, g, cur.pl.uniform != 0);
-            float mx = s[0][0];
 #pragma unroll
-            for (int u = 0; u < SUB; ++u)
+            for (int k = 2; k >= 0; --k) load_kf(0, k);
+            __builtin_amdgcn_sched_barrier(0);
+            f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+            for (int m = 0; m < 12 * KS; ++m) {
+                const int ks = m / 12, i = (m % 12) / 2, u = m % 2;
+                mma16(s[u], kf[u][kSplitA[i]], qf[ks].p[kSplitB[i]]);
+                if (u == 1 && kSplitLast[kSplitA[i]] == i && ks + 1 < KS) load_kf(ks + 1, kSplitA[i]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (!(j0 >= rows.lo_max && j0 + BN <= rows.hi_min)) rows.mask_tile(s, j0, g, cur.pl.uniform != 0);
+            // ---- online softmax against a lazily moved reference (see attention.hip): the row's maximum is only taken over its four
+            // lanes where one of them has outrun the reference ----
+            float mx = m_ref;
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) mx = fmaxf(mx, s[u][j]);
-            // ---- online softmax against a lazily moved reference (see attention.hip) ----
-            mx = over_groups(mx, [](float x, float y) { return fmaxf(x, y); });
-            if (__any((mx - m_ref) * c2 > kRescaleThreshold)) {
-                const float m_new = ((mx - m_ref) * c2 > kRescaleThreshold) ? mx : m_ref;
+            if (__any(mx - m_ref > slack)) {
+                mx = over_groups(mx, [](float x, float y) { return fmaxf(x, y); });
+                const float m_new = mx - m_ref > slack ? mx : m_ref;
                 const float alpha = fast_exp2((m_ref - m_new) * c2);
                 m_ref = m_new;
                 l_run *= alpha;
 #pragma unroll
-                for (int i = 0; i < 4 * DH; ++i) o[i] *= alpha;
+                for (int dt = 0; dt < DT; ++dt) o[dt] *= alpha;
             }
             // a row that has seen no live score keeps offset 0, so that its (all masked) entries map to 0
             const float mb = m_ref > 0.5f * kNegBigA ? m_ref * c2 : 0.f;
+            Frag<bf16> vf[2][3];
+            auto load_vf = [&](int d2, int k) {
 #pragma unroll
-            for (int u = 0; u < SUB; ++u) {
-                if (u + 1 < SUB) {
-                    load_v(u + 1);
-                    __builtin_amdgcn_sched_barrier(0);
+                for (int y = 0; y < 2; ++y) {
+                    const uint32_t a0 = v_addr[2 * d2 + y] + k * PLANE;
+                    vf[y][k] = frag_from_tr<bf16>(lds_load_tr16(a0), lds_load_tr16(a0 + 16 * ROWB));
                 }
-                if (!sub_live(u)) continue;
+            };
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    s[u][j] = fast_exp2(fmaf(s[u][j], c2, -mb));
-                    l_run += s[u][j];
-                }
-                // ---- O^T += V^T . P^T ----
+            for (int k = 2; k >= 0; --k) load_vf(0, k);
+            __builtin_amdgcn_sched_barrier(0);
+            f32x8 e;
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
+            for (int j = 0; j < 8; ++j) {
+                e[j] = fast_exp2(fmaf(s[j >> 2][j & 3], c2, -mb));
+                l_run += e[j];
+            }
+            const Split3 pf = split3(e);
+            // ---- O^T += V^T . P^T, of two tiles of 16 columns at a time ----
 #pragma unroll
-                    for (int hh = 0; hh < DH; ++hh)
-#pragma unroll
-                        for (int dt = 0; dt < 4; ++dt) mma4(o[4 * hh + dt], vf[u & 1][j][hh][dt], s[u][j]);
+            for (int m = 0; m < 6 * DT; ++m) {
+                const int d2 = m / 12, i = (m % 12) / 2, y = m % 2;
+                mma16(o[2 * d2 + y], vf[y][kSplitA[i]], pf.p[kSplitB[i]]);
+                if (y == 1 && kSplitLast[kSplitA[i]] == i && 2 * d2 + 2 < DT) load_vf(d2 + 1, kSplitA[i]);
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
         if (!cur.pl.uniform) rows.next_tile();
-        stage = stage + 1 == NSTAGE ? 0 : stage + 1;
-        const int delta = stage == 0 ? -(NSTAGE - 1) * STAGE : STAGE;
-        v_addr += delta;
-#pragma unroll
-        for (int t = 0; t < (KT ? 1 : KQ); ++t) k_addr[t] += delta;
         if (++cur.tile >= cur.end) {
             ++cur.seg;
             next_segment(cur);
@@ -334,20 +283,76 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_f32_kernel(const AttnParams p
         }
     }
 
-    // ---- epilogue: a lane holds 16 consecutive columns (per 64) of its row ----
     const float l_tot = over_groups(l_run, [](float x, float y) { return x + y; });
+    // What is not finite anywhere stays so in a row's sum or outputs; outputs that are subnormal by far mean a V that is.
+    float chk = l_tot * 0.f, most = 0.f;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            chk = fmaf(o[dt][j], 0.f, chk);
+            most = fmaxf(most, fabsf(o[dt][j]));
+        }
+    beyond |= chk != 0.f || (most > 0.f && most < 0x1p-96f * l_tot);  // (NaN compares unequal)
+    if (__any(beyond)) {
+        // ---- this wavefront's rows once more in float32 arithmetic, position by position, each lane a quarter of a row's columns,
+        // live positions only ----
+        constexpr int QD = D / 4;
+        const float* qr = qb + (int64_t)min(my_row, L - 1) * p.q_sl + g * QD;
+        float q[QD], acc[QD];
+#pragma unroll
+        for (int i = 0; i < QD; ++i) q[i] = qr[i], acc[i] = 0.f;
+        float m = -__builtin_inff(), l = 0.f;
+        for (int sg = 0; sg < p.n_seg; ++sg) {
+            const HalfWalk w = walk_of(sg);
+            RowWin win;
+            if constexpr (PLANNED) {
+                const PlanRec wr = pt[plan_row_at(n_rb, p.n_seg, rb, sg, k0 + wave * 16 + n)];
+                win.lo = wr.x, win.cnt = wr.y, win.lin = wr.z;
+            } else {
+                win = make_row_win(cached_row_map<kPlanBM>(&s_ps, sg, k0 + wave * 16 + n), w.pl);
+            }
+            for (int j = w.tile * BN; j < w.end * BN; ++j) {
+                const bool live = win_live(win, j);
+                if (!__any(live)) continue;
+                const int64_t key = min(max(w.pl.c0 + w.pl.cs * j, 0), L - 1);
+                const float* kr = KT ? kb + (int64_t)(g * QD) * p.k_sd + key : kb + key * p.k_sl + g * QD;
+                float s = 0.f;
+#pragma unroll
+                for (int i = 0; i < QD; ++i) s = fmaf(q[i], kr[KT ? i * p.k_sd : i], s);
+                s = over_groups(s, [](float x, float y) { return x + y; }) * c2;
+                if (live) {
+                    const float m_new = fmaxf(m, s);
+                    const float off = m_new > -__builtin_inff() ? m_new : 0.f;
+                    const float alpha = m > -__builtin_inff() ? fast_exp2(m - off) : 1.f;
+                    const float e = fast_exp2(s - off);
+                    m = m_new;
+                    l = fmaf(l, alpha, e);
+                    const float* vr = vb + key * p.v_sl + g * QD;
+#pragma unroll
+                    for (int i = 0; i < QD; ++i) acc[i] = fmaf(acc[i], alpha, e * vr[i]);
+                }
+            }
+        }
+        const float inv = l > 0.f ? 1.0f / l : 0.f;
+        if (my_row < L) {
+            if (p.lse != nullptr && g == 0)
+                p.lse[(int64_t)bh * L + my_row] = l > 0.f ? (m + __log2f(l)) * 0.6931471805599453f : __builtin_inff();
+            float* orow = ob + (int64_t)my_row * p.o_sl + g * QD;
+#pragma unroll
+            for (int i = 0; i < QD; ++i) orow[i] = acc[i] * inv;
+        }
+        return;
+    }
+
+    // ---- epilogue: a lane holds columns 16 dt + 4g .. + 3 of its row ----
     const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
     if (my_row < L) {
         if (p.lse != nullptr && g == 0)
             p.lse[(int64_t)bh * L + my_row] = l_tot > 0.f ? (m_ref * c2 + __log2f(l_tot)) * 0.6931471805599453f : __builtin_inff();
         float* orow = ob + (int64_t)my_row * p.o_sl;
 #pragma unroll
-        for (int hh = 0; hh < DH; ++hh)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const f32x4 x = {o[4 * hh][i] * inv, o[4 * hh + 1][i] * inv, o[4 * hh + 2][i] * inv, o[4 * hh + 3][i] * inv};
-                *reinterpret_cast<f32x4*>(orow + 64 * hh + 16 * g + 4 * i) = x;
-            }
+        for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<f32x4*>(orow + 16 * dt + 4 * g) = o[dt] * inv;
     }
 }
 
@@ -357,8 +362,7 @@ static int launch(const AttnParams& p0, hipStream_t st) {
     AttnParams p = p0;
     p.n_row_blocks = count_row_blocks(p.L, kPlanBM, p.row_stride);
     p.total = p.B * p.H * 2 * p.n_row_blocks;
-    if (PLANNED && KT) p.plan += plan_variant_recs(p.n_row_blocks, p.n_seg);  // the dense-walk variant
-    const size_t lds = kF32Stages * 2 * f32_tile(D) * D * 4;
+    const size_t lds = 6 * 32 * D * 2;
     auto kern = attn_fwd_f32_kernel<D, KT, PLANNED>;
     static uint64_t lds_reserved = 0;
     if (int rc = reserve_dynamic_lds(&lds_reserved, reinterpret_cast<const void*>(kern), lds, "splat_attention_fwd")) return rc;

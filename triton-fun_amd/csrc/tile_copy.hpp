@@ -128,6 +128,9 @@ __device__ __forceinline__ u32x4 lds_load128(uint32_t addr) { return *reinterpre
 __device__ __forceinline__ s16x4 lds_load_tr16(uint32_t addr) {
     return __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>((uintptr_t)addr));
 }
+__device__ __forceinline__ void lds_store128(uint32_t addr, u32x4 x) {
+    *reinterpret_cast<__attribute__((address_space(3))) u32x4*>((uintptr_t)addr) = x;
+}
 __device__ __forceinline__ float lds_load_f32(uint32_t addr) { return *reinterpret_cast<lds_f32*>((uintptr_t)addr); }
 
 // Wait until at most N of this wavefront's global loads (LDS-DMA copies included) are outstanding.

@@ -1,5 +1,4 @@
-// Pieces of the fused float32 attention kernels (forward and backward): 16x16 tiles of scores on the float32 matrix
-// instruction.
+// Pieces of the fused float32 backward kernels: 16x16 tiles of scores on the float32 matrix instruction.
 //
 // Operand layouts of acc[16x16] += A[16x4] * B[4x16] (v_mfma_f32_16x16x4_f32): lane (n = lane % 16, g = lane / 16) feeds row n
 // of A and column n of B at contraction slot g, and holds rows 4g .. 4g + 3 of column n of the result.  Which index of the
