@@ -1,10 +1,10 @@
-"""The float32 forward on split operands against float64: what the parts hold, and what they do not (taken again in
+"""The float32 forward and backward on split operands against float64: what the parts hold, and what they do not (taken again in
 float32 arithmetic)."""
 import pytest
 import torch
 
 import acsr_helpers as A
-from r_attention import RegularAttention
+from r_attention import RegularAttention, attention_with_grad
 
 pytestmark = pytest.mark.gpu
 
@@ -67,3 +67,47 @@ def test_values_that_are_not_finite_reach_the_rows_that_see_them(dev, L, d, keys
     rest[:, :, sees_v, 3] = False
     rest[:, :, sees_v, 7] = False
     assert bool(torch.isfinite(got[rest]).all()) and float((got[rest] - clean[rest]).abs().max()) <= 1e-5
+
+
+def gradients(dev, d, L, scale_q, scale_k, scale_v, scale_g, seed=0, change=None):
+    masks = [A.causal_windowed_pattern(L, 69)]
+    g = torch.Generator().manual_seed(seed + d)
+    q, k, v, go = (torch.randn(1, 2, L, d, generator=g) * s for s in (scale_q, scale_k, scale_v, scale_g))
+    if change is not None:
+        change(q, k, v, go)
+    live = masks[0].device_mask(dev).cpu() > 0
+    wide = [t.double().requires_grad_(True) for t in (q, k, v)]
+    p = torch.softmax((wide[0] @ wide[1].transpose(2, 3) * d ** -0.5).masked_fill(~live, float("-inf")), -1)
+    want = torch.autograd.grad(p @ wide[2], wide, go.double())
+    attn = RegularAttention(1, L, 2, d, masks, 16, 16, dev, torch.float32, scale=d ** -0.5)
+    on = [t.to(dev).requires_grad_(True) for t in (q, k, v)]
+    got = torch.autograd.grad(attention_with_grad(*on, attn), on, go.to(dev))
+    return got, want, live
+
+
+# as above, through one more product and a difference that may cancel
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("q,k,v,g", [(1, 1, 1, 1), (1, 1, 1, 1e-30), (1, 1, 1, 1e-36), (1, 1, 1e-34, 1), (1, 1, 1e-20, 1e20),
+                                     (1e-34, 1, 1, 1), (1, 1e-34, 1, 1), (1e30, 1e-30, 1, 1), (1, 1, 1e15, 1e15)])
+def test_gradients_at_scales_of_the_operands(dev, d, q, k, v, g):
+    got, want, _ = gradients(dev, d, 211, q, k, v, g)
+    for a, b in zip(got, want):
+        if float(b.abs().max()) > 1e-35:  # (below, float32 itself is subnormal)
+            assert error(a, b) <= 3e-6
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_gradients_that_are_not_finite_stay_where_they_belong(dev, d):
+    def spoil(q, k, v, go):
+        go[0, 0, 100, 5] = float("inf")
+        v[0, 1, 20, 3] = float("nan")
+    clean, _, live = gradients(dev, d, 211, 1, 1, 1, 1)
+    got, _, _ = gradients(dev, d, 211, 1, 1, 1, 1, change=spoil)
+    sees, seen = live[:, 20].to(dev), live[100].to(dev)  # the rows that see key 20, the keys that row 100 sees
+    assert not bool(torch.isfinite(got[0][0, 0, 100]).any()) and not bool(torch.isfinite(got[2][0, 0, seen, 5]).any())
+    assert not bool(torch.isfinite(got[0][0, 1, sees]).any())
+    rows = torch.arange(211, device=dev) != 100
+    assert torch.allclose(got[0][0, 0, rows], clean[0][0, 0, rows], rtol=0, atol=1e-5)
+    assert torch.allclose(got[0][0, 1, ~sees], clean[0][0, 1, ~sees], rtol=0, atol=1e-5)
+    for i in (1, 2) if d == 64 else ():  # (at d = 128 dK and dV are float32 products, where 0 * inf of a tile's masked positions is NaN)
+        assert torch.allclose(got[i][0, 0, ~seen], clean[i][0, 0, ~seen], rtol=0, atol=1e-5)

@@ -1,32 +1,33 @@
 // Fused backward of the ACSR attention in float32: dQ, and dK + dV, without any compressed [B, H, L, T] matrix in memory.
 //
 // The products, the roles of the operands and the plans are those of attention_bwd.hip (dQ: rows are queries, positions keys, X = K,
-// Y = V; dK + dV: rows are keys, positions queries, X = Q, Y = dO), the tiles those of attention_f32.hip: a wavefront owns 16
-// rows and takes positions in subtiles of 16, four wavefronts share tiles of 32 (d = 64) or 16 (d = 128) positions:
+// Y = V; dK + dV: rows are keys, positions queries, X = Q, Y = dO):
 //     S^T = X A^T;  P;  dP^T = Y B^T;  dS = P (dP - D);  acc^T += X^T dS^T;  dK + dV also acc2^T += Y^T P^T
-// Bound, as there: the float32 matrix instructions and the vector arithmetic that shares their units.  Seven products a live
-// entry, where the operators composed over compressed matrices took eight launches, five of them over [B, H, L, T] matrices
-// in memory: forward and backward of B = 2, H = 8, L = 2048, causal window 128, d = 64, 211 -> 79 us.
-// A and B stay in registers, X and Y come through the asynchronous copy ring; their tiles are read row-wise for the products over d and
-// column-wise for those over positions, both as 16-byte pieces without bank conflicts (pieces of a row are permuted among the
-// row's own 256 bytes).
+// They run, as in attention_f32.hip, on the 16-bit matrix instructions, of operands split into three parts (split3.hpp): a wavefront
+// owns 16 rows, four of them share tiles of 32 positions, whose pieces every thread loads a tile ahead, splits, and writes between two
+// barriers.  A and B are split once and stay in registers.  dK + dV at d = 128 does not fit them and is a kernel of its own
+// (attention_bwd_f32_keys.hip).
+// Measured against the kernel on the float32 instructions, us: 64 heads of 2048 rows, d = 64, window 256: dQ 140 -> 97, dK + dV 181 ->
+// 135; 128 heads, window 32: 99 -> 81 and 116 -> 107; 32 heads, d = 128, window 256 / 32: dQ 142 -> 110 and 59 -> 51; one head, window 32,
+// d = 64: 11.0 -> 9.7 and 10.8 -> 9.6.  Two workgroups of dQ a CU instead of three at d = 64: 110.  Relative error of dq, dk, dv
+// against float64 (norms), window 257: 5.1e-7, 5.1e-7, 4.9e-7 -> 4.3e-7, 4.3e-7, 4.2e-7.
 #include "attn_bwd.hpp"
-#include "tile_f32.hpp"
+#include "rows16.hpp"
+#include "split3.hpp"
 
 namespace splat {
 
 template <int D, bool KEYS>
-__global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_f32_kernel(const BwdParams p) {
-    constexpr int BN = f32_tile(D), SUB = BN / 16;
-    constexpr int KQ = D / 16, DH = D / 64;
-    constexpr int ROWB = D * 4, TILE = BN * ROWB, STAGE = 2 * TILE;
-    constexpr int STATS = 512;       // lse and D of a tile's positions: 64 floats each, the first BN in use
-    constexpr int RING = 2 * STATS;  // both stages' statistics come first
-    constexpr int NI = TILE / 4096;  // copy blocks per wavefront and operand
-    constexpr int CPR = ROWB / 16, RPI = 1024 / ROWB;
+__global__ __launch_bounds__(256, D == 64 && !KEYS ? 3 : 2) void attn_bwd_f32_kernel(const BwdParams p) {
+    constexpr int BN = 32, ROWB = 2 * D, PLANE = BN * ROWB, TILE = 3 * PLANE;  // positions a tile; bytes of a row, a plane, an operand
+    constexpr int STATS = 2 * TILE;           // lse and D of the tile's positions (dK + dV)
+    constexpr int KS = D / 32, DT = D / 16;
+    constexpr int CPR = D / 8;                // 8-value pieces of a row
+    constexpr int NP = 2 * BN * CPR / 256;    // pieces a thread: the first half of them X's, the others Y's
+    constexpr int AHEAD = D == 64 ? 2 : 1;    // parts of fragments requested ahead of their products (as many as registers are left)
     constexpr float kLog2e = 1.4426950408889634f;
 
-    extern __shared__ __attribute__((aligned(1024))) char smem[];
+    extern __shared__ __attribute__((aligned(1024))) char smem[];  // three planes of X, three of Y, the statistics
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -51,33 +52,24 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_f32_kernel(cons
     const float* lse_b = p.lse + (int64_t)bh * L;
     const float* del_b = p.delta + (int64_t)bh * L;
 
-    // ---- the lane's share of its rows of A and B, resident: B operands of the products over d ----
+    // ---- the lane's share of its rows of A and B: B operands of the products over d ----
     const int out_row = r0 + rs * (wave * 16 + n);
     int my_row = min(out_row, Lr - 1);
     if constexpr (KEYS) {
         if (p.row_map) my_row = min(max(p.row_map[my_row], 0), L - 1);
     }
-    float ar[D / 4], br[D / 4];
-    auto load_row = [&](const float* row, float (&to)[D / 4]) {
+    const float* const a_row = ab + (int64_t)my_row * p.a_sl;
+    const float* const b_row = bb + (int64_t)my_row * p.b_sl;
+    f32x8 a_raw[KS], b_raw[KS], o_raw[KEYS ? 1 : KS];
 #pragma unroll
-        for (int t = 0; t < KQ; ++t) {
-            const f32x4 x = *reinterpret_cast<const f32x4*>(row + 16 * t + 4 * g);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) to[4 * t + j] = x[j];
-        }
-    };
-    load_row(ab + (int64_t)my_row * p.a_sl, ar);
-    load_row(bb + (int64_t)my_row * p.b_sl, br);
-    float row_lse2 = 0.f, row_delta = 0.f;  // dQ: the lane's own query
-    if constexpr (!KEYS) {
-        row_lse2 = lse_b[my_row] * kLog2e;
-        float orow[D / 4];
-        load_row((const float*)p.o + b * p.oo_sb + h * p.oo_sh + (int64_t)my_row * p.oo_sl, orow);
-        float s = 0.f;
-#pragma unroll
-        for (int i = 0; i < D / 4; ++i) s = fmaf(br[i], orow[i], s);
-        row_delta = over_groups(s, [](float x, float y) { return x + y; });  // D = rowsum(dO * O); stored after the tile loop
+    for (int ks = 0; ks < KS; ++ks) {
+        a_raw[ks] = global_frag<float>(a_row + 32 * ks + 8 * g).v;
+        b_raw[ks] = global_frag<float>(b_row + 32 * ks + 8 * g).v;
+        if constexpr (!KEYS)
+            o_raw[ks] = global_frag<float>((const float*)p.o + b * p.oo_sb + h * p.oo_sh + (int64_t)my_row * p.oo_sl + 32 * ks + 8 * g).v;
     }
+    float row_lse2 = 0.f, row_delta = 0.f;  // dQ: the lane's own query
+    if constexpr (!KEYS) row_lse2 = lse_b[my_row] * kLog2e;
 
     // ---- plan: the row block's walk, cut down to the tiles that this half of it sees ----
     const PlanRec* const pt = p.plan;
@@ -90,96 +82,96 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_f32_kernel(cons
         }
         w.seg = p.n_seg, w.tile = 0, w.end = 0x7fffffff;
     };
-    int total = 0;
-    for (int sg = 0; sg < p.n_seg; ++sg) {
+    HalfWalk fetch;
+    fetch.seg = 0;
+    next_segment(fetch);
+    int total = fetch.end - fetch.tile;
+    for (int sg = fetch.seg + 1; sg < p.n_seg; ++sg) {
         const HalfWalk w = walk_of(sg);
         total += w.end - w.tile;
     }
-    total = __builtin_amdgcn_readfirstlane(total);
+    total = fetch.seg < p.n_seg ? __builtin_amdgcn_readfirstlane(total) : 0;
 
-    // ---- asynchronous copies of one tile (see attention_f32.hip) ----
-    auto position_row = [&](const HalfWalk& w, int j) { return min(max(w.pl.c0 + w.pl.cs * j, 0), L - 1); };
-    uint32_t x_off[NI], y_off[NI];
-    const char *x_next = nullptr, *y_next = nullptr;
-    int64_t x_row = 0, y_row = 0;  // bytes from one tile row to the next
-    bool off_fits = true;
-    auto set_offsets = [&](const HalfWalk& w) {
-        x_row = (int64_t)p.x_sl * 4 * w.pl.cs;
-        y_row = (int64_t)p.y_sl * 4 * w.pl.cs;
-        off_fits = x_row * RPI < ((int64_t)1 << 31) && y_row * RPI < ((int64_t)1 << 31);
+    // ---- a tile's way into LDS: pieces of 8 values, by their position in the tile's rows ----
+    const uint32_t smem_base = lds_address(smem);
+    int pc_row[NP], pc_c[NP];
+    uint32_t pc_to[NP];  // LDS address of its first part
 #pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            const int c = logical_chunk<ROWB, 1>((wave + 4 * i) * RPI + lane / CPR, lane % CPR) * 16;
-            x_off[i] = (uint32_t)(x_row * (lane / CPR)) + c;
-            y_off[i] = (uint32_t)(y_row * (lane / CPR)) + c;
-        }
-        const int64_t first = w.pl.c0 + (int64_t)w.pl.cs * BN * w.tile;
-        x_next = reinterpret_cast<const char*>(xb) + first * p.x_sl * 4 + wave * RPI * x_row;
-        y_next = reinterpret_cast<const char*>(yb) + first * p.y_sl * 4 + wave * RPI * y_row;
-    };
-    auto issue_next = [&](HalfWalk& w, int stage) {
-        char* xs_w = smem + RING + stage * STAGE;
-        const int j0 = w.tile * BN;
-        if (off_fits && w.pl.c0 + w.pl.cs * (j0 + BN - 1) < L && w.pl.c0 + w.pl.cs * j0 >= 0) {
+    for (int i = 0; i < NP; ++i) {
+        const int f = (tid + 256 * i) % (BN * CPR);
+        pc_row[i] = f / CPR, pc_c[i] = f % CPR;
+        pc_to[i] = smem_base + (i < NP / 2 ? 0 : TILE) + pc_row[i] * ROWB + ((pc_c[i] ^ swz_both16<ROWB>(pc_row[i])) << 4);
+    }
+    f32x8 raw[NP];
+    float raw_stat = 0.f;  // dK + dV: wavefront 0 carries lse (lanes 0..31) and D
+    // operands of one head within 32-bit offsets, and strides that 24-bit products take
+    const bool narrow = max(p.x_sl, p.y_sl) * 4 * L < ((int64_t)1 << 32) && max(p.x_sl, p.y_sl) * 4 < (1 << 24);
+    auto load_next = [&](HalfWalk& w) {  // the tile the walk stands at, which moves on
+        const int c0 = w.pl.c0 + w.pl.cs * w.tile * BN;
+        auto position = [&](int row) { return min(max(c0 + w.pl.cs * row, 0), L - 1); };
 #pragma unroll
-            for (int i = 0; i < NI; ++i) {
-                dma16_uniform(x_next + 4 * i * RPI * x_row, x_off[i], xs_w + (wave + 4 * i) * 1024);
-                dma16_uniform(y_next + 4 * i * RPI * y_row, y_off[i], xs_w + TILE + (wave + 4 * i) * 1024);
-            }
-        } else {
-            dma_tile<float, ROWB, BN, 1>(xs_w, wave, lane, [&](int row) { return xb + (int64_t)position_row(w, j0 + row) * p.x_sl; });
-            dma_tile<float, ROWB, BN, 1>(xs_w + TILE, wave, lane, [&](int row) { return yb + (int64_t)position_row(w, j0 + row) * p.y_sl; });
+        for (int i = 0; i < NP; ++i) {
+            const char* base = reinterpret_cast<const char*>(i < NP / 2 ? xb : yb);
+            const int64_t sl = i < NP / 2 ? p.x_sl : p.y_sl;
+            const int row = position(pc_row[i]);
+            if (narrow)
+                raw[i] = global_frag<float>(reinterpret_cast<const float*>(base + (__umul24(row, (uint32_t)sl * 4) + 32 * pc_c[i]))).v;
+            else
+                raw[i] = global_frag<float>(reinterpret_cast<const float*>(base) + row * sl + 8 * pc_c[i]).v;
         }
         if constexpr (KEYS) {
-            const int q = position_row(w, j0 + (lane & (BN - 1)));
-            if (wave == 0) dma4(lse_b + q, smem + stage * STATS);
-            if (wave == 1) dma4(del_b + q, smem + stage * STATS + 256);
+            if (wave == 0) raw_stat = (lane < BN ? lse_b : del_b)[position(lane & (BN - 1))];
         }
-        x_next += BN * x_row;
-        y_next += BN * y_row;
         if (++w.tile >= w.end) {
             ++w.seg;
             next_segment(w);
-            if (w.seg < p.n_seg) set_offsets(w);
         }
     };
 
-    // ---- LDS read addresses: of stage 0, moved on once a tile ----
-    const uint32_t smem_base = lds_address(smem);
-    uint32_t x_addr[KQ];  // row-wise: row n of a subtile, piece 4t + g (Y: TILE further)
-    uint32_t c_addr[4];   // column-wise: row 4g + j, piece n
-#pragma unroll
-    for (int t = 0; t < KQ; ++t) x_addr[t] = smem_base + RING + lds_off<ROWB, true>(n, (16 * t + 4 * g) * 4);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) c_addr[j] = smem_base + RING + lds_off<ROWB, true>(4 * g + j, 16 * n);
-    uint32_t st_addr = smem_base + 16 * g;
+    // ---- LDS read addresses of X (Y: TILE further) ----
+    const int tr_row = (lane & 15) >> 2, tr_chunk = (lane >> 1) & 1, tr_byte = 8 * (lane & 1);  // transposing reads: 4 rows x 32 bytes
+    // (pieces of a row are permuted by an exclusive or, so that the addresses of one row differ by one)
+    uint32_t r_base = smem_base + n * ROWB + ((g ^ swz_both16<ROWB>(n)) << 4);
+    uint32_t c_base = smem_base + (4 * g + tr_row) * ROWB + ((tr_chunk ^ swz_both16<ROWB>(4 * g + tr_row)) << 4) + tr_byte;
 
-    HalfWalk fetch, cur;
-    fetch.seg = 0;
-    next_segment(fetch);
-    if (fetch.seg < p.n_seg) set_offsets(fetch);
-    cur = fetch;
+    HalfWalk cur = fetch;
     PlanRec win_rec = {0, 0, 1, 0};
-    if (cur.seg < p.n_seg) win_rec = pt[plan_row_at(n_rb, p.n_seg, rb, cur.seg, k0 + wave * 16 + n)];
-    if (total > 0) issue_next(fetch, 0);
+    if (total > 0) win_rec = pt[plan_row_at(n_rb, p.n_seg, rb, cur.seg, k0 + wave * 16 + n)];
+    if (total > 0) load_next(fetch);
 
-    f32x4 acc[4 * DH], acc2[KEYS ? 4 * DH : 1];
+    // (one operand after the other: their raw and split forms together would not fit the registers at d = 128)
+    Split3 af[KS], bf[KS];
+    float a_most = 0.f, b_most = 0.f;
 #pragma unroll
-    for (int i = 0; i < 4 * DH; ++i) {
-        acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if constexpr (KEYS) acc2[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int ks = 0; ks < KS; ++ks) {
+        bf[ks] = split3(b_raw[ks]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            b_most = fmaxf(b_most, fabsf(b_raw[ks][e]));
+            if constexpr (!KEYS) row_delta = fmaf(b_raw[ks][e], o_raw[ks][e], row_delta);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+        af[ks] = split3(a_raw[ks]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) a_most = fmaxf(a_most, fabsf(a_raw[ks][e]));
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (!KEYS) row_delta = over_groups(row_delta, [](float x, float y) { return x + y; });  // D = rowsum(dO * O)
+    bool beyond = out_of_split(a_most) || out_of_split(b_most);  // something that the split operands do not hold
+    float x_most = 0.f, y_most = 0.f;                            // of the thread's pieces of the tiles
+
+    f32x4 acc[DT], acc2[KEYS ? DT : 1];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+        acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if constexpr (KEYS) acc2[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
     const float c2 = p.scale_log2e;
     RowState rows;
     bool entered = false;
-    int stage = 0;
-#if defined(__HIP_DEVICE_COMPILE__)
-    // the register operands are in their registers before the loop, so that no wait of the compiler's for them holds up the
-    // copies in flight there
-#pragma unroll
-    for (int i = 0; i < D / 4; ++i) asm volatile("" ::"v"(ar[i]), "v"(br[i]));
-    asm volatile("" ::"v"(row_lse2), "v"(row_delta));
-#endif
 
     for (int it = 0; it < total; ++it) {
         if (!entered) {
@@ -189,101 +181,97 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_f32_kernel(cons
             entered = true;
         }
         const int j0 = cur.tile * BN;
-        // this wavefront's copies of tile `it` have landed; after the barrier everybody's have, and everybody is done with
-        // tile it - 1, whose stage the next fetch overwrites
-        wait_loads<0>();
-        __builtin_amdgcn_s_barrier();
-        if (it + 1 < total) issue_next(fetch, stage ^ 1);
+        lds_barrier();  // everybody is done with tile it - 1
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            const Split3 s = split3(raw[i]);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) lds_store128(pc_to[i] + k * PLANE, __builtin_bit_cast(u32x4, s.p[k].v));
+            float& most = i < NP / 2 ? x_most : y_most;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) most = fmaxf(most, fabsf(raw[i][e]));
+        }
+        if constexpr (KEYS) {
+            if (wave == 0) reinterpret_cast<float*>(smem + STATS)[lane] = raw_stat;
+        }
+        if (it + 1 < total) load_next(fetch);
+        lds_barrier();  // tile `it` is there
 
         if (j0 + BN > rows.lo_min && j0 < rows.hi_max) {
-            auto sub_live = [&](int u) { return SUB == 1 || (j0 + 16 * u + 16 > rows.lo_min && j0 + 16 * u < rows.hi_max); };
-            const bool full = j0 >= rows.lo_max && j0 + BN <= rows.hi_min;
-            // fragments are requested a phase ahead of their use, outside the branches of the subtiles
-            f32x4 xf[SUB][KQ], yf[SUB][KQ];
+#if defined(__HIP_DEVICE_COMPILE__)
+            asm volatile("" : "+v"(r_base), "+v"(c_base));  // (the addresses are made here: kept over the loop they would spill)
+#endif
+            auto r_addr = [&](int ks) { return r_base ^ (uint32_t)(ks << 6); };
+            auto c_addr = [&](int dt) { return c_base ^ (uint32_t)(dt << 5); };
+            // ---- S^T = X A^T, then dP^T = Y B^T, of two subtiles of 16 positions; fragments are requested ahead of their products, part k
+            // of a step as the one of the step before is done with ----
+            Frag<bf16> rf[2][3];
+            auto load_rf = [&](int x) {  // part 2 - x % 3 of step x / 3
+                const int st = x / 3, k = 2 - x % 3;
 #pragma unroll
-            for (int u = 0; u < SUB; ++u)
-#pragma unroll
-                for (int t = 0; t < KQ; ++t) xf[u][t] = lds_load_f32x4(x_addr[t] + 16 * u * ROWB);
-            __builtin_amdgcn_sched_barrier(0);
-            f32x4 s[SUB], ds[SUB];
-#pragma unroll
-            for (int u = 0; u < SUB; ++u) {
-                if (sub_live(u)) {
-                    s[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                    for (int t = 0; t < KQ; ++t)
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) mma4(s[u], xf[u][t][j], ar[4 * t + j]);
-                } else {
-                    s[u] = f32x4{kNegBigA, kNegBigA, kNegBigA, kNegBigA};
-                }
-#pragma unroll
-                for (int t = 0; t < KQ; ++t) yf[u][t] = lds_load_f32x4(x_addr[t] + TILE + 16 * u * ROWB);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            f32x4 lse4[KEYS ? SUB : 1], del4[KEYS ? SUB : 1];
-            if constexpr (KEYS) {
-#pragma unroll
-                for (int u = 0; u < SUB; ++u) {
-                    lse4[u] = lds_load_f32x4(st_addr + 64 * u);
-                    del4[u] = lds_load_f32x4(st_addr + 256 + 64 * u);
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < SUB; ++u) {
-                if (!sub_live(u)) continue;
-                ds[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int t = 0; t < KQ; ++t)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) mma4(ds[u], yf[u][t][j], br[4 * t + j]);
-            }
-            // ---- P = exp2(S * scale * log2e - lse * log2e); masked scores underflow to exactly 0.  dS = P (dP - D) ----
-            if (!full) rows.mask_tile(s, j0, g, cur.pl.uniform != 0);
-            f32x4 xc[4][DH], yc[KEYS ? 4 : 1][DH];
-            auto load_columns = [&](int u) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-#pragma unroll
-                    for (int hh = 0; hh < DH; ++hh) {
-                        xc[j][hh] = lds_load_f32x4(c_addr[j] + 16 * u * ROWB + 256 * hh);
-                        if constexpr (KEYS) yc[j][hh] = lds_load_f32x4(c_addr[j] + TILE + 16 * u * ROWB + 256 * hh);
-                    }
+                for (int u = 0; u < 2; ++u)
+                    rf[u][k].v = __builtin_bit_cast(bf16x8, lds_load128(r_addr(st % KS) + (st / KS) * TILE + k * PLANE + 16 * u * ROWB));
             };
 #pragma unroll
-            for (int u = 0; u < SUB; ++u) {
-                load_columns(u);
+            for (int x = 0; x < AHEAD; ++x) load_rf(x);
+            __builtin_amdgcn_sched_barrier(0);
+            f32x4 s[2], ds[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) s[u] = ds[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int m = 0; m < 24 * KS; ++m) {
+                const int st = m / 12, i = (m % 12) / 2, u = m % 2, x = 3 * st + 2 - kSplitA[i];
+                if (st < KS)
+                    mma16(s[u], rf[u][kSplitA[i]], af[st % KS].p[kSplitB[i]]);
+                else
+                    mma16(ds[u], rf[u][kSplitA[i]], bf[st % KS].p[kSplitB[i]]);
+                if (u == 1 && kSplitLast[kSplitA[i]] == i && x + AHEAD < 6 * KS) load_rf(x + AHEAD);
                 __builtin_amdgcn_sched_barrier(0);
-                if (!sub_live(u)) continue;
+            }
+            // ---- P = exp2(S * scale * log2e - lse * log2e); masked scores underflow to exactly 0.  dS = P (dP - D) ----
+            if (!(j0 >= rows.lo_max && j0 + BN <= rows.hi_min)) rows.mask_tile(s, j0, g, cur.pl.uniform != 0);
+            Frag<bf16> cf[2][3];
+            auto load_cf = [&](int operand, int x) {
+                const int d2 = x / 3, k = 2 - x % 3;
+#pragma unroll
+                for (int y = 0; y < 2; ++y) {
+                    const uint32_t a0 = c_addr(2 * d2 + y) + operand * TILE + k * PLANE;
+                    cf[y][k] = frag_from_tr<bf16>(lds_load_tr16(a0), lds_load_tr16(a0 + 16 * ROWB));
+                }
+            };
+            f32x8 pr, dsv;
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                f32x4 lse4, del4;
+                if constexpr (KEYS) {
+                    lse4 = __builtin_bit_cast(f32x4, lds_load128(smem_base + STATS + 64 * u + 16 * g));
+                    del4 = __builtin_bit_cast(f32x4, lds_load128(smem_base + STATS + 128 + 64 * u + 16 * g));
+                }
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    if constexpr (KEYS) {
-                        s[u][j] = fast_exp2(fmaf(s[u][j], c2, -kLog2e * lse4[u][j]));
-                        ds[u][j] = s[u][j] * (ds[u][j] - del4[u][j]);
-                    } else {
-                        ds[u][j] = fast_exp2(fmaf(s[u][j], c2, -row_lse2)) * (ds[u][j] - row_delta);
-                    }
+                    const int e = 4 * u + j;
+                    pr[e] = fast_exp2(fmaf(s[u][j], c2, KEYS ? -kLog2e * lse4[j] : -row_lse2));
+                    dsv[e] = pr[e] * (ds[u][j] - (KEYS ? del4[j] : row_delta));
                 }
-                // ---- acc^T += X^T dS^T, acc2^T += Y^T P^T ----
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-#pragma unroll
-                    for (int hh = 0; hh < DH; ++hh)
-#pragma unroll
-                        for (int dt = 0; dt < 4; ++dt) {
-                            mma4(acc[4 * hh + dt], xc[j][hh][dt], ds[u][j]);
-                            if constexpr (KEYS) mma4(acc2[4 * hh + dt], yc[j][hh][dt], s[u][j]);
-                        }
             }
+            // ---- acc2^T += Y^T P^T, acc^T += X^T dS^T, of two tiles of 16 columns at a time ----
+            auto accumulate = [&](f32x4 (&to)[DT], int operand, const f32x8& v) {
+#pragma unroll
+                for (int x = 0; x < AHEAD; ++x) load_cf(operand, x);
+                __builtin_amdgcn_sched_barrier(0);
+                const Split3 vf = split3(v);
+#pragma unroll
+                for (int m = 0; m < 6 * DT; ++m) {
+                    const int d2 = m / 12, i = (m % 12) / 2, y = m % 2, x = 3 * d2 + 2 - kSplitA[i];
+                    mma16(to[2 * d2 + y], cf[y][kSplitA[i]], vf.p[kSplitB[i]]);
+                    if (y == 1 && kSplitLast[kSplitA[i]] == i && x + AHEAD < 3 * DT / 2) load_cf(operand, x + AHEAD);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            };
+            if constexpr (KEYS) accumulate(acc2, 1, pr);
+            accumulate(acc, 0, dsv);
         }
         if (!cur.pl.uniform) rows.next_tile();
-        stage ^= 1;
-        const int delta = stage == 0 ? -STAGE : STAGE;
-#pragma unroll
-        for (int t = 0; t < KQ; ++t) x_addr[t] += delta;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) c_addr[j] += delta;
-        st_addr += stage == 0 ? -STATS : STATS;
         if (++cur.tile >= cur.end) {
             ++cur.seg;
             next_segment(cur);
@@ -291,23 +279,74 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_f32_kernel(cons
         }
     }
 
-    // ---- epilogue: a lane holds 16 consecutive columns (per 64) of its row ----
-    if (out_row < Lr) {
-        if constexpr (!KEYS) {
-            if (g == 0) p.delta_w[(int64_t)bh * L + out_row] = row_delta;
+    // What is not finite anywhere stays so in a row's results (NaN compares unequal).  Operands of the tiles that are all far below
+    // normal matter to results of their own size, whatever those are multiplied with.
+    float chk = 0.f;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            chk = fmaf(acc[dt][j], 0.f, chk);
+            if constexpr (KEYS) chk = fmaf(acc2[dt][j], 0.f, chk);
         }
-        auto store_row = [&](void* base, const f32x4 (&a)[4 * DH], float scale) {
-            float* row = (float*)base + b * p.o_sb + h * p.o_sh + (int64_t)out_row * p.o_sl;
+    auto all_tiny = [](float most) { return __any(most > 0.f) && !__any(most >= 0x1p-96f); };
+    beyond |= chk != 0.f || all_tiny(x_most) || all_tiny(y_most);
+    auto out_at = [&](void* base) { return (float*)base + b * p.o_sb + h * p.o_sh + (int64_t)out_row * p.o_sl; };
+    if constexpr (!KEYS) {
+        if (out_row < Lr && g == 0) p.delta_w[(int64_t)bh * L + out_row] = row_delta;
+    }
+    if (__any(beyond)) {
+        // ---- this wavefront's rows once more in float32 arithmetic, position by position, each lane a quarter of a row's columns,
+        // live positions only ----
+        constexpr int QD = D / 4;
+        float a[QD], bq[QD], r1[QD], r2[KEYS ? QD : 1];
 #pragma unroll
-            for (int hh = 0; hh < DH; ++hh)
+        for (int i = 0; i < QD; ++i) {
+            a[i] = a_row[g * QD + i], bq[i] = b_row[g * QD + i], r1[i] = 0.f;
+            if constexpr (KEYS) r2[i] = 0.f;
+        }
+        for (int sg = 0; sg < p.n_seg; ++sg) {
+            const HalfWalk w = walk_of(sg);
+            const PlanRec wr = pt[plan_row_at(n_rb, p.n_seg, rb, sg, k0 + wave * 16 + n)];
+            const RowWin win = {wr.x, wr.y, wr.z};
+            for (int j = w.tile * BN; j < w.end * BN; ++j) {
+                const bool live = win_live(win, j);
+                if (!__any(live)) continue;
+                const int64_t pos = min(max(w.pl.c0 + w.pl.cs * j, 0), L - 1);
+                const float *xr = xb + pos * p.x_sl + g * QD, *yr = yb + pos * p.y_sl + g * QD;
+                float s = 0.f, dp = 0.f;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const f32x4 x = {a[4 * hh][i] * scale, a[4 * hh + 1][i] * scale, a[4 * hh + 2][i] * scale, a[4 * hh + 3][i] * scale};
-                    *reinterpret_cast<f32x4*>(row + 64 * hh + 16 * g + 4 * i) = x;
+                for (int i = 0; i < QD; ++i) s = fmaf(a[i], xr[i], s), dp = fmaf(bq[i], yr[i], dp);
+                s = over_groups(s, [](float x, float y) { return x + y; });
+                dp = over_groups(dp, [](float x, float y) { return x + y; });
+                if (live) {
+                    const float e = fast_exp2(fmaf(s, c2, KEYS ? -kLog2e * lse_b[pos] : -row_lse2));
+                    const float d = e * (dp - (KEYS ? del_b[pos] : row_delta));
+#pragma unroll
+                    for (int i = 0; i < QD; ++i) {
+                        r1[i] = fmaf(d, xr[i], r1[i]);
+                        if constexpr (KEYS) r2[i] = fmaf(e, yr[i], r2[i]);
+                    }
                 }
-        };
-        store_row(p.out, acc, p.scale);
-        if constexpr (KEYS) store_row(p.out2, acc2, 1.0f);
+            }
+        }
+        if (out_row < Lr) {
+#pragma unroll
+            for (int i = 0; i < QD; ++i) {
+                out_at(p.out)[g * QD + i] = r1[i] * p.scale;
+                if constexpr (KEYS) out_at(p.out2)[g * QD + i] = r2[i];
+            }
+        }
+        return;
+    }
+
+    // ---- epilogue: a lane holds columns 16 dt + 4g .. + 3 of its row ----
+    if (out_row < Lr) {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+            *reinterpret_cast<f32x4*>(out_at(p.out) + 16 * dt + 4 * g) = acc[dt] * p.scale;
+            if constexpr (KEYS) *reinterpret_cast<f32x4*>(out_at(p.out2) + 16 * dt + 4 * g) = acc2[dt];
+        }
     }
 }
 
@@ -316,7 +355,7 @@ static int launch(const BwdParams& p0, hipStream_t st) {
     begin_launch();
     BwdParams p = p0;
     p.total = p.B * p.H * 2 * p.n_row_blocks;
-    constexpr size_t lds = 2 * 512 + 2 * 2 * f32_tile(D) * D * 4;
+    constexpr size_t lds = 6 * 32 * D * 2 + 256;
     auto kern = attn_bwd_f32_kernel<D, KEYS>;
     static uint64_t lds_reserved = 0;
     if (int rc = reserve_dynamic_lds(&lds_reserved, reinterpret_cast<const void*>(kern), lds, "splat_attention_bwd_f32")) return rc;
@@ -325,6 +364,6 @@ static int launch(const BwdParams& p0, hipStream_t st) {
 }
 
 int launch_bwd_dq_f32(const BwdParams& dq, int d, hipStream_t st) { return d == 64 ? launch<64, false>(dq, st) : launch<128, false>(dq, st); }
-int launch_bwd_dkv_f32(const BwdParams& dkv, int d, hipStream_t st) { return d == 64 ? launch<64, true>(dkv, st) : launch<128, true>(dkv, st); }
+int launch_bwd_dkv_f32(const BwdParams& dkv, int d, hipStream_t st) { return d == 64 ? launch<64, true>(dkv, st) : launch_bwd_dkv_f32_d128(dkv, st); }
 
 }  // namespace splat

@@ -34,5 +34,6 @@ int launch_bwd_pair(const BwdParams& dkv, hipStream_t st);
 // float32: dQ (which also computes and stores D), and dK + dV of the rows that `dkv` describes
 int launch_bwd_dq_f32(const BwdParams& dq, int d, hipStream_t st);
 int launch_bwd_dkv_f32(const BwdParams& dkv, int d, hipStream_t st);
+int launch_bwd_dkv_f32_d128(const BwdParams& dkv, hipStream_t st);  // attention_bwd_f32_keys.hip
 
 }  // namespace splat

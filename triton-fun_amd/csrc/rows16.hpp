@@ -1,4 +1,4 @@
-// Pieces of the fused attention kernels whose wavefronts own 16 rows (attention_f32.hip, attention_bwd_f32.hip,
+// Pieces of the fused attention kernels whose wavefronts own 16 rows (attention_f32.hip, attention_bwd_f32.hip, attention_bwd_f32_keys.hip,
 // attention_rows16.hip): reductions over the lanes of a row, the walk of half a row block over its tiles, and the rows'
 // windows.  Lane (n = lane % 16, g = lane / 16) holds row n's scores at positions 4g .. 4g + 3 of every subtile of 16.
 #pragma once

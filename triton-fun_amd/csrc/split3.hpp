@@ -48,8 +48,13 @@ __device__ __forceinline__ Split3 split3(const f32x8& x) {
     return s;
 }
 
-// whether the largest magnitude of some values is outside what products of split operands keep float32's precision for
-__device__ __forceinline__ bool out_of_split(float most) { return (most > 0.f && most < 0x1p-96f) || most > 0x1p80f; }
+// Whether the largest magnitude of some values is outside what products of split operands keep float32's precision for.
+__device__ __forceinline__ bool out_of_split(float most) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(most));  // found here, not where the answer is wanted: the values need not be kept until then
+#endif
+    return (most > 0.f && most < 0x1p-96f) || most > 0x1p80f;
+}
 
 // The six products of a split operand pair, in the order they are added: A's parts one after the other, the smallest first, so that
 // the registers of a part that is done with can take the next fragment's.

@@ -56,6 +56,14 @@ template <int ROWB>
 __device__ __forceinline__ constexpr int dual_chunk(int row, int c) {
     return (((c >> 2) ^ swz64<ROWB>(row)) << 2) | ((c & 3) ^ ((row >> 2) & 3));
 }
+// Swizzle of the 16-byte chunk index for tiles that are read row-wise, 16 rows at the same chunk, and by the narrow transposing
+// reads: the 16 rows of either half get 16 different chunk positions of the 256-byte bank space, and any 8 consecutive of them
+// different 32-byte blocks.
+template <int ROWB>
+__device__ __forceinline__ constexpr int swz_both16(int row) {
+    static_assert(ROWB == 128 || ROWB == 256, "row pitch");
+    return ROWB == 256 ? ((row & 7) << 1) | ((row >> 3) & 1) : ((row >> 1) & 3) << 1 | ((row >> 3) & 1);
+}
 // logical 16-byte chunk held at physical chunk position pc of `row`; MODE 0: none, 1: chunk XOR (b128 row reads),
 // 2: 64-byte block XOR (transposing reads), 3: both kinds of read (dual_chunk), 4: 32-byte block XOR (narrow transposing reads)
 template <int ROWB, int MODE>
