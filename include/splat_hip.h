@@ -267,6 +267,18 @@ int splat_attention_fwd_hinted(const void* q, int64_t q_sb, int64_t q_sh, int64_
                                int32_t dtype, const void* plan, int64_t plan_bytes, float* lse, int32_t live_percent,
                                void* stream);
 
+/* splat_attention_fwd_hinted for K^T with the keys contiguous (k_sl == 1) whose rows are not whole 16-byte pieces: any L >= 8, any
+ * strides and any address of its element's alignment.  The plan is needed.  SPLAT_E_UNSUPPORTED, with nothing launched, in launches
+ * that copy K in whole pieces (16-bit types beyond the few row blocks of the kernel that loads K through registers):
+ * splat_transpose_keys turns it for those.  `out` is bit-identical to the other forwards' on rows of K. */
+int splat_attention_fwd_keys(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* kT,
+                             int64_t k_sb, int64_t k_sh, int64_t k_sd, const void* v,
+                             int64_t v_sb, int64_t v_sh, int64_t v_sl, void* out, int64_t o_sb,
+                             int64_t o_sh, int64_t o_sl, const splat_acsr_seg* segs /* host */,
+                             int32_t n_seg, int32_t B, int32_t H, int32_t L, int32_t d, float scale,
+                             int32_t dtype, const void* plan, int64_t plan_bytes, float* lse, int32_t live_percent,
+                             void* stream);
+
 /* The fused forward for callers that cannot allocate device memory or hold a plan buffer: code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc.  No counterpart in the reference.  Same arguments and
  * bit-identical results as splat_attention_fwd_planned, without the plan arguments: the plan is rebuilt by every call

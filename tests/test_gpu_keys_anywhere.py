@@ -1,0 +1,56 @@
+"""K^T with the keys contiguous whose rows start anywhere, read where it lies: bit for bit what rows of the same keys give, at lengths
+around the edges of pieces and tiles, at odd strides and addresses, and up to the last byte of its memory."""
+import ctypes
+
+import pytest
+import torch
+
+import _splat_hip as hip
+import acsr_helpers as A
+from r_attention import RegularAttention
+
+pytestmark = pytest.mark.gpu
+
+TYPES = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}
+
+
+@pytest.mark.parametrize("dtype", TYPES)
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("L", [8, 9, 15, 63, 65, 130, 201, 519])
+def test_equals_rows_of_keys(dev, dtype, d, L):
+    B, H, dt = 2, 3, TYPES[dtype]
+    masks = [A.causal_windowed_pattern(L, 33)] if L % 2 else [A.windowed_pattern(L, 70)]
+    attn = RegularAttention(B, L, H, d, masks, 16, 16, dev, dt, scale=d ** -0.5)
+    g = torch.Generator(device=dev).manual_seed(L + d)
+    q, k, v = (torch.randn(B, H, L, d, generator=g, device=dev).to(dt) for _ in range(3))
+    first = attn([q, k.transpose(2, 3), v]).clone()
+    want = attn([q, k.transpose(2, 3), v]).clone()
+    assert torch.equal(first, want)
+    # as it is stored by a contiguous copy: the last row ends where its memory ends
+    whole = torch.empty(B * H * d * L, dtype=dt, device=dev)
+    exact = whole.view(B, H, d, L)
+    exact.copy_(k.transpose(2, 3))
+    assert torch.equal(attn([q, exact, v]), want)
+    # a part of longer rows, from an odd element on; what lies around it must not matter
+    long = torch.full((B, H, d, L + 7), float("nan"), dtype=dt, device=dev)
+    part = long[..., 3:3 + L]
+    part.copy_(k.transpose(2, 3))
+    assert torch.equal(attn([q, part, v]), want)
+
+
+@pytest.mark.parametrize("blocks,ran", [(128, True), (129, False)])
+def test_launches_that_copy_whole_pieces_refuse(dev, blocks, ran):
+    L, d, dt = 121, 64, torch.bfloat16
+    attn = RegularAttention(1, L, blocks, d, A.windowed_pattern(L, L), 16, 16, dev, dt, scale=1.0)
+    q, v = (torch.randn(1, blocks, L, d, device=dev).to(dt) for _ in range(2))
+    kT = torch.randn(1, blocks, d, L, device=dev).to(dt)
+    want = attn([q, kT.transpose(2, 3).contiguous().transpose(2, 3), v]).clone()
+    assert torch.equal(attn([q, kT, v]), want)  # through the transposing copy where the kernel refuses
+    out, arr, plan = torch.zeros_like(q), attn.segments.seg_array(L), attn._plan
+    rc = hip.lib().splat_attention_fwd_keys(q.data_ptr(), *q.stride()[:3], kT.data_ptr(), *kT.stride()[:3], v.data_ptr(), *v.stride()[:3],
+                                            out.data_ptr(), *out.stride()[:3], arr, 1, 1, blocks, L, d, ctypes.c_float(1.0),
+                                            hip.dtype_code(dt), plan.data_ptr(), plan.numel() * plan.element_size(), None, 0,
+                                            hip.stream_ptr(dev))
+    torch.cuda.synchronize()
+    assert (rc == 0) == ran and bool((out == 0).all()) != ran
+    assert not ran or torch.equal(out, want)

@@ -86,6 +86,9 @@ _SIGNATURES = {
     "splat_attention_fwd_hinted": (ctypes.c_int, [_vp, _i64, _i64, _i64, _vp, _i64, _i64, _i64, _i64, _vp, _i64, _i64, _i64,
                                                  _vp, _i64, _i64, _i64, ctypes.POINTER(AcsrSeg), _i32, _i32, _i32, _i32,
                                                  _i32, _f32, _i32, _vp, _i64, _vp, _i32, _vp]),
+    "splat_attention_fwd_keys": (ctypes.c_int, [_vp, _i64, _i64, _i64, _vp, _i64, _i64, _i64, _vp, _i64, _i64, _i64,
+                                                _vp, _i64, _i64, _i64, ctypes.POINTER(AcsrSeg), _i32, _i32, _i32, _i32,
+                                                _i32, _f32, _i32, _vp, _i64, _vp, _i32, _vp]),
     "splat_attention_bwd": (ctypes.c_int, [_vp, _i64, _i64, _i64] * 5 + [_vp] * 5 +
                             [ctypes.POINTER(AcsrSeg), _i32, _vp, _i64] * 2 + [_i32, _i32, _i32, _i32, _f32, _i32, _vp]),
     "splat_attention_bwd_keys": (ctypes.c_int, [_vp, _i64, _i64, _i64] * 4 + [_vp] * 5 +

@@ -570,6 +570,7 @@ static int dispatch_attn(const AttnParams& p, int d, bool kt, hipStream_t st) {
     const int64_t blocks = (int64_t)p.B * p.H * count_row_blocks(p.L, kPlanBM, p.row_stride);
     if (blocks <= 128 || (p.live_percent > 0 && p.live_percent <= 75 && blocks <= (d == 64 ? 320 : 192)))
         return launch_attn_rows16<T>(p, d, kt, st);
+    if (p.keys_anywhere) return fail(SPLAT_E_UNSUPPORTED, "splat_attention_fwd_keys: this launch copies K in whole 16-byte pieces");
     if (p.plan) {
         if (d == 64) return kt ? launch_attn<T, 64, true, 64, 2, true>(p, st) : launch_attn<T, 64, false, 64, 2, true>(p, st);
         return kt ? launch_attn<T, 128, true, 64, 2, true>(p, st) : launch_attn<T, 128, false, 64, 2, true>(p, st);
@@ -630,7 +631,7 @@ static int attention_fwd_common(const char* who, const void* q, int64_t q_sb, in
                                 int64_t v_sh, int64_t v_sl, void* out, int64_t o_sb, int64_t o_sh, int64_t o_sl,
                                 const splat_acsr_seg* segs, int32_t n_seg, int32_t B, int32_t H, int32_t L, int32_t d,
                                 float scale, int32_t dtype, const void* plan, int64_t plan_bytes, bool planned,
-                                float* lse, void* stream, int32_t live_percent = 0) {
+                                float* lse, void* stream, int32_t live_percent = 0, bool keys_anywhere = false) {
     if (!q || !kT || !v || !out || !segs) return fail(SPLAT_E_NULL, "%s: null pointer argument", who);
     if (B <= 0 || H <= 0 || L <= 0) return fail(SPLAT_E_SHAPE, "%s: need B, H, L > 0 (got %d, %d, %d)", who, B, H, L);
     if (L > (1 << 23)) return fail(SPLAT_E_SHAPE, "%s: L is limited to 2^23 (got %d)", who, L);
@@ -650,13 +651,17 @@ static int attention_fwd_common(const char* who, const void* q, int64_t q_sb, in
     else
         return fail(SPLAT_E_ALIGN, "%s: kT needs unit stride along d (k_sd == 1) or along keys (k_sl == 1); got k_sd=%lld k_sl=%lld", who,
                     (long long)k_sd, (long long)k_sl);
-    if (kt && ((L % epc) != 0 || (k_sd % epc) != 0 || L < epc))
+    if (keys_anywhere) {
+        if (!kt || !planned || L < 8 || k_sd < L) return fail(SPLAT_E_UNSUPPORTED, "%s: needs a plan, at least 8 keys and rows of them", who);
+        if ((reinterpret_cast<uintptr_t>(kT) & (es - 1)) != 0) return fail(SPLAT_E_ALIGN, "%s: kT is not aligned to its element size", who);
+    }
+    if (!keys_anywhere && kt && ((L % epc) != 0 || (k_sd % epc) != 0 || L < epc))
         return fail(SPLAT_E_ALIGN, "%s: with K^T contiguous along keys, L and the d-stride must be multiples of %d (got L=%d, k_sd=%lld)", who,
                     epc, L, (long long)k_sd);
     auto mis = [&](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) != 0; };
     auto bad = [&](int64_t s) { return (s % epc) != 0; };
-    if (mis(q) || mis(kT) || mis(v) || mis(out)) return fail(SPLAT_E_ALIGN, "%s: q, kT, v and out must be 16-byte aligned", who);
-    if (bad(q_sb) || bad(q_sh) || bad(q_sl) || bad(k_sb) || bad(k_sh) || bad(v_sb) || bad(v_sh) || bad(v_sl) || bad(o_sb) || bad(o_sh) || bad(o_sl))
+    if (mis(q) || (mis(kT) && !keys_anywhere) || mis(v) || mis(out)) return fail(SPLAT_E_ALIGN, "%s: q, kT, v and out must be 16-byte aligned", who);
+    if (bad(q_sb) || bad(q_sh) || bad(q_sl) || (!keys_anywhere && (bad(k_sb) || bad(k_sh))) || bad(v_sb) || bad(v_sh) || bad(v_sl) || bad(o_sb) || bad(o_sh) || bad(o_sl))
         return fail(SPLAT_E_ALIGN, "%s: every batch/head/row stride must be a multiple of %d elements (16 bytes)", who, epc);
     if (q_sl < d || v_sl < d || o_sl < d) return fail(SPLAT_E_SHAPE, "%s: row strides must be >= d", who);
 
@@ -673,7 +678,7 @@ static int attention_fwd_common(const char* who, const void* q, int64_t q_sb, in
     p.row_stride = common_row_stride(segs, n_seg);
     p.plan = nullptr;
     p.lse = lse;
-    p.live_percent = live_percent;
+    p.live_percent = live_percent, p.keys_anywhere = keys_anywhere;
     if (planned) {
         if (!plan) return fail(SPLAT_E_NULL, "%s: null plan", who);
         if ((reinterpret_cast<uintptr_t>(plan) & 15) != 0) return fail(SPLAT_E_ALIGN, "%s: the plan must be 16-byte aligned", who);
@@ -735,6 +740,20 @@ extern "C" int splat_attention_fwd_hinted(const void* q, int64_t q_sb, int64_t q
     return attention_fwd_common(who, q, q_sb, q_sh, q_sl, kT, k_sb, k_sh, k_sd, k_sl, v, v_sb, v_sh, v_sl, out, o_sb, o_sh,
                                 o_sl, segs, n_seg, B, H, L, d, scale, dtype, plan, plan_bytes, plan != nullptr, lse, stream,
                                 live_percent);
+}
+
+extern "C" int splat_attention_fwd_keys(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* kT,
+                                        int64_t k_sb, int64_t k_sh, int64_t k_sd, const void* v,
+                                        int64_t v_sb, int64_t v_sh, int64_t v_sl, void* out, int64_t o_sb,
+                                        int64_t o_sh, int64_t o_sl, const splat_acsr_seg* segs, int32_t n_seg, int32_t B,
+                                        int32_t H, int32_t L, int32_t d, float scale, int32_t dtype, const void* plan,
+                                        int64_t plan_bytes, float* lse, int32_t live_percent, void* stream) {
+    const char* who = "splat_attention_fwd_keys";
+    if ((reinterpret_cast<uintptr_t>(lse) & 3) != 0) return fail(SPLAT_E_ALIGN, "%s: lse must be 4-byte aligned", who);
+    if (live_percent < 0 || live_percent > 100) return fail(SPLAT_E_SHAPE, "%s: live_percent is %d", who, live_percent);
+    return attention_fwd_common(who, q, q_sb, q_sh, q_sl, kT, k_sb, k_sh, k_sd, 1, v, v_sb, v_sh, v_sl, out, o_sb, o_sh,
+                                o_sl, segs, n_seg, B, H, L, d, scale, dtype, plan, plan_bytes, plan != nullptr, lse, stream,
+                                live_percent, true);
 }
 
 // ---- the forward for callers that cannot allocate: the plan lives in a file-scope device array ----------------

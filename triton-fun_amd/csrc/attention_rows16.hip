@@ -17,8 +17,16 @@
 
 namespace splat {
 
-template <typename T, int D, bool KT, bool PLANNED>
-__global__ __launch_bounds__(256, 3) void attn_fwd_rows16_kernel(const AttnParams p) {
+// How K is stored: rows of keys, or K^T with the keys contiguous, whose rows are whole 16-byte pieces or start anywhere.  The last
+// cannot take the asynchronous copies, which move aligned words: its pieces come through registers, a tile ahead, instead of a launch
+// that turns K first.  bf16, K^T of 12 heads of 1037 keys, window 201, turned first -> read where it lies: d = 128 15.9 -> 12.1 us (rows
+// of K 11.4; three workgroups' worth of registers would spill 19 of them: 13.0), d = 64 11.8 -> 9.2; 11 heads of 2041, window 101
+// 16.1 -> 12.5 and 12.1 -> 8.4.
+enum { kKeyRows, kKeysWhole, kKeysAnywhere };
+
+template <typename T, int D, int LAYOUT, bool PLANNED>
+__global__ __launch_bounds__(256, LAYOUT == kKeysAnywhere && D == 128 ? 2 : 3) void attn_fwd_rows16_kernel(const AttnParams p) {
+    constexpr bool KT = LAYOUT != kKeyRows, ANY = LAYOUT == kKeysAnywhere;
     constexpr int ES = 2, BN = 64, SUB = BN / 16;
     static_assert(sizeof(T) == ES && kPlanBM == 2 * kHalfRows && kBN % BN == 0, "tile shape");
     constexpr int KS = D / 32;  // contraction steps of the score product
@@ -104,7 +112,8 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_rows16_kernel(const AttnParam
         char* ks_w = smem + stage * STAGE;
         auto key_row = [&](int row) { return min(max(w.pl.c0 + w.pl.cs * (j0 + row), 0), L - 1); };
         dma_tile<T, V_ROWB, BN, V_SWZ>(ks_w + TILE, wave, lane, [&](int row) { return vb + (int64_t)key_row(row) * p.v_sl; });
-        if constexpr (KT) {
+        if constexpr (ANY) {
+        } else if constexpr (KT) {
             // rows = d, BN consecutive keys each (dense walk); a chunk past the last key is replaced by the last whole one
 #pragma unroll
             for (int i = 0; i < NI; ++i) {
@@ -131,13 +140,42 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_rows16_kernel(const AttnParam
         v_next = reinterpret_cast<const char*>(vb) + first * p.v_sl * ES + wave * V_RPI * v_row;
         k_next = reinterpret_cast<const char*>(kb) + (KT ? first * ES : first * p.k_sl * ES) + wave * K_RPI * k_row;
     };
+    // K^T whose rows start anywhere comes through registers: requested with V's copies, written to the stage a tile later
+    u32x4 k_reg[ANY ? NI : 1];
+    auto load_keys = [&](const HalfWalk& w) {
+        const int c0 = w.pl.c0 + w.tile * BN;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int flat = tid + 256 * i, c = c0 + 8 * (flat % K_CPR);
+            const int over = min(max(c + 8 - L, 0), 8);  // keys of the piece that do not exist: the row's last whole piece, moved down
+            u32x4 x;
+            __builtin_memcpy(&x, kb + (int64_t)(flat / K_CPR) * p.k_sd + min(c, L - 8), 16);
+            if (over > 0) {
+                const uint64_t lo = (uint64_t)x[1] << 32 | x[0], hi = (uint64_t)x[3] << 32 | x[2];
+                const int s = 16 * (over & 3);
+                const uint64_t a = over >= 4 ? hi : lo, b = over >= 4 ? 0 : hi;
+                const uint64_t l = s == 0 ? a : (a >> s) | (b << (64 - s)), h = b >> s;
+                x = u32x4{(uint32_t)l, (uint32_t)(l >> 32), (uint32_t)h, (uint32_t)(h >> 32)};
+            }
+            k_reg[i] = x;
+        }
+    };
+    auto store_keys = [&](int stage) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int flat = tid + 256 * i, row = flat / K_CPR, c = flat % K_CPR;
+            const int to = (((c >> 1) ^ swz32<K_ROWB>(row)) << 1) | (c & 1);
+            lds_store128(lds_address(smem) + stage * STAGE + row * K_ROWB + to * 16, k_reg[i]);
+        }
+    };
     auto issue_next = [&](HalfWalk& w, int stage) {
+        if constexpr (ANY) load_keys(w);
         const int last = w.pl.c0 + w.pl.cs * (w.tile * BN + BN - 1);
         if (off_fits && last < L && w.pl.c0 + w.pl.cs * w.tile * BN >= 0) {
             char* ks_w = smem + stage * STAGE;
 #pragma unroll
             for (int i = 0; i < NI; ++i) {
-                dma16_uniform(k_next + 4 * i * K_RPI * k_row, k_off, ks_w + (wave + 4 * i) * 1024);
+                if constexpr (!ANY) dma16_uniform(k_next + 4 * i * K_RPI * k_row, k_off, ks_w + (wave + 4 * i) * 1024);
                 dma16_uniform(v_next + 4 * i * V_RPI * v_row, v_off, ks_w + TILE + (wave + 4 * i) * 1024);
             }
         } else {
@@ -211,6 +249,10 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_rows16_kernel(const AttnParam
         // this wavefront's copies of tile `it` have landed; after the barrier everybody's have, and everybody is done with
         // tile it - 1, whose stage the next fetch overwrites
         wait_loads<0>();
+        if constexpr (ANY) {
+            store_keys(stage);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        }
         __builtin_amdgcn_s_barrier();
         if (it + 1 < total) issue_next(fetch, stage ^ 1);
 
@@ -319,29 +361,30 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_rows16_kernel(const AttnParam
     }
 }
 
-template <typename T, int D, bool KT, bool PLANNED>
+template <typename T, int D, int LAYOUT, bool PLANNED>
 static int launch(const AttnParams& p0, hipStream_t st) {
     begin_launch();
     AttnParams p = p0;
     p.n_row_blocks = count_row_blocks(p.L, kPlanBM, p.row_stride);
     p.total = p.B * p.H * 2 * p.n_row_blocks;
-    if (PLANNED && KT) p.plan += plan_variant_recs(p.n_row_blocks, p.n_seg);  // the dense-walk variant
+    if (PLANNED && LAYOUT != kKeyRows) p.plan += plan_variant_recs(p.n_row_blocks, p.n_seg);  // the dense-walk variant
     constexpr size_t lds = 2 * 2 * 64 * D * 2;  // two stages of two tiles of 64 positions
-    auto kern = attn_fwd_rows16_kernel<T, D, KT, PLANNED>;
+    auto kern = attn_fwd_rows16_kernel<T, D, LAYOUT, PLANNED>;
     static uint64_t lds_reserved = 0;
     if (int rc = reserve_dynamic_lds(&lds_reserved, reinterpret_cast<const void*>(kern), lds, "splat_attention_fwd")) return rc;
     kern<<<((p.total + 7) / 8) * 8, 256, lds, st>>>(p);
     return check_launch("splat_attention_fwd");
 }
 
+template <typename T, int D>
+static int launch_layout(const AttnParams& p, bool kt, hipStream_t st) {
+    if (p.keys_anywhere) return launch<T, D, kKeysAnywhere, true>(p, st);
+    if (p.plan) return kt ? launch<T, D, kKeysWhole, true>(p, st) : launch<T, D, kKeyRows, true>(p, st);
+    return kt ? launch<T, D, kKeysWhole, false>(p, st) : launch<T, D, kKeyRows, false>(p, st);
+}
 template <typename T>
 int launch_attn_rows16(const AttnParams& p, int d, bool kt, hipStream_t st) {
-    if (p.plan) {
-        if (d == 64) return kt ? launch<T, 64, true, true>(p, st) : launch<T, 64, false, true>(p, st);
-        return kt ? launch<T, 128, true, true>(p, st) : launch<T, 128, false, true>(p, st);
-    }
-    if (d == 64) return kt ? launch<T, 64, true, false>(p, st) : launch<T, 64, false, false>(p, st);
-    return kt ? launch<T, 128, true, false>(p, st) : launch<T, 128, false, false>(p, st);
+    return d == 64 ? launch_layout<T, 64>(p, kt, st) : launch_layout<T, 128>(p, kt, st);
 }
 template int launch_attn_rows16<f16>(const AttnParams&, int, bool, hipStream_t);
 template int launch_attn_rows16<bf16>(const AttnParams&, int, bool, hipStream_t);

@@ -25,6 +25,7 @@ struct AttnParams {
     const PlanRec* plan;  // plan table of this mask (PLANNED kernels), variant already selected
     float* lse;           // optional [B*H, L]: log of every row's sum of exponentials (natural log, scaled scores)
     int live_percent;     // host only: share of the walked positions that some row sees, 0 where the caller did not say
+    bool keys_anywhere;   // host only: K^T with the keys contiguous whose rows are not whole 16-byte pieces
 };
 
 constexpr float kRescaleThreshold = 8.0f;  // in log2 units: exponentials stay below 2^8 before the reference moves

@@ -39,6 +39,7 @@ namespace {
 struct Api {
     decltype(&splat_last_error) last_error;
     decltype(&splat_attention_fwd_hinted) fwd_hinted;
+    decltype(&splat_attention_fwd_keys) fwd_keys;
     decltype(&splat_transpose_keys) transpose_keys;
     decltype(&splat_attention_bwd) bwd;
     decltype(&splat_attention_bwd_keys) bwd_keys;
@@ -215,6 +216,15 @@ Did forward(const Mask& m, const at::Tensor& q, at::Tensor kT, const at::Tensor&
         // columns (dense runs are all this layout can be read in), else turned around first
         const bool as_is = m.max_step < 2 && L % epc == 0 && kT.stride(0) % epc == 0 && kT.stride(1) % epc == 0 &&
                            kT.stride(2) % epc == 0 && aligned16(kT);
+        if (!as_is && m.max_step < 2) {  // loaded from where it lies, if the launch can
+            *rc = api.fwd_keys(q.data_ptr(), q.stride(0), q.stride(1), q.stride(2), kT.data_ptr(), kT.stride(0), kT.stride(1), kT.stride(2),
+                               v.data_ptr(), v.stride(0), v.stride(1), v.stride(2), out.data_ptr(), out.stride(0), out.stride(1),
+                               out.stride(2), m.segs, m.n_seg, B, H, L, d, (float)scale, code, m.plan_ptr(), m.plan_bytes(), lse,
+                               m.live_percent, stream_of(q));
+            if (*rc == 0) return Did::kYes;
+            if (*rc != SPLAT_E_UNSUPPORTED) return Did::kFailed;
+            *rc = 0;
+        }
         if (!as_is) {
             kT = transposed_keys(kT, rc).transpose(2, 3);
             if (*rc) return Did::kFailed;
@@ -683,7 +693,7 @@ PyObject* py_bind(PyObject*, PyObject* args) {
         fn = reinterpret_cast<std::remove_reference_t<decltype(fn)>>(static_cast<uintptr_t>(PyLong_AsUnsignedLongLong(o)));
         return !PyErr_Occurred();
     };
-    if (!take("splat_last_error", api.last_error) || !take("splat_attention_fwd_hinted", api.fwd_hinted) ||
+    if (!take("splat_last_error", api.last_error) || !take("splat_attention_fwd_hinted", api.fwd_hinted) || !take("splat_attention_fwd_keys", api.fwd_keys) ||
         !take("splat_transpose_keys", api.transpose_keys) ||
         !take("splat_attention_bwd", api.bwd) || !take("splat_attention_bwd_keys", api.bwd_keys) ||
         !take("splat_attention_bwd_f32", api.bwd_f32) || !take("splat_attention_bwd_keys_f32", api.bwd_keys_f32) || !take("splat_sddmm", api.sddmm) ||
