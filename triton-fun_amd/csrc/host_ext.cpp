@@ -20,6 +20,7 @@
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/object_ptr.h>
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/custom_class.h>
 
@@ -647,21 +648,22 @@ PyObject* py_build(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const int rc = api.build_record(mask.data_ptr<uint8_t>(), rows, cols, mask.stride(0), (int32_t)bh, record.data_ptr<float>(),
                                         extents.data_ptr<int32_t>(), 1, shares.data_ptr<int32_t>(), stream.stream());
         if (rc) return refused("splat_acsr_build_record", rc, shares);
-        if (!wait_for(stream, shares)) return nullptr;
-        int32_t t_max = 0, bad = 0, step_min = 0x7fffffff, step_max = 0, off = 0;
-        for (int64_t b = 0; b < blocks; ++b) {
-            const int32_t* s = sh + 8 * b;
-            t_max = std::max(t_max, s[0]), bad += s[1], step_min = std::min(step_min, s[2]), step_max = std::max(step_max, s[3]), off += s[4];
-        }
-        share_buffers()->give(std::move(shares));
-        PyObject* sets[2];
+        // while the kernel runs: the arrays as tensors of their own (a call over 8192 x 8192: 37.6 -> 36.6 us)
+        struct Written {  // (the kernel writes the shares: a way out before the wait does not give them back)
+            at::Tensor& shares;
+            bool waited = false;
+            ~Written() {
+                if (!waited) new at::Tensor(std::move(shares));
+            }
+        } written{shares};
+        THPObjectPtr sets[2];
         for (int k = 0; k < 2; ++k) {
             sets[k] = PyTuple_New(9);
             if (!sets[k]) return nullptr;
             for (int i = 0; i < 9; ++i) {
                 if (k == 1 && i == 6) {  // (the caller's set: nobody reads its row_last)
                     Py_INCREF(Py_None);
-                    PyTuple_SET_ITEM(sets[k], i, Py_None);
+                    PyTuple_SET_ITEM(sets[k].get(), i, Py_None);
                     continue;
                 }
                 at::Tensor t;
@@ -671,10 +673,20 @@ PyObject* py_build(PyObject*, PyObject* const* a, Py_ssize_t n) {
                     t = part_of(record, k * twin + i * row_step, rows);
                 else
                     t = part_of(record, k * twin + 5 * row_step + (i - 7) * span_step, blocks);
-                PyTuple_SET_ITEM(sets[k], i, THPVariable_Wrap(std::move(t)));
+                PyObject* const wrapped = THPVariable_Wrap(std::move(t));
+                if (!wrapped) return nullptr;
+                PyTuple_SET_ITEM(sets[k].get(), i, wrapped);
             }
         }
-        return Py_BuildValue("NNiiiii", sets[0], sets[1], t_max, bad, step_min, step_max, off);
+        written.waited = true;
+        if (!wait_for(stream, shares)) return nullptr;
+        int32_t t_max = 0, bad = 0, step_min = 0x7fffffff, step_max = 0, off = 0;
+        for (int64_t b = 0; b < blocks; ++b) {
+            const int32_t* s = sh + 8 * b;
+            t_max = std::max(t_max, s[0]), bad += s[1], step_min = std::min(step_min, s[2]), step_max = std::max(step_max, s[3]), off += s[4];
+        }
+        share_buffers()->give(std::move(shares));
+        return Py_BuildValue("NNiiiii", sets[0].release(), sets[1].release(), t_max, bad, step_min, step_max, off);
     } catch (...) {
         return raise_current();
     }
