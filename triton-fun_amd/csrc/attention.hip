@@ -53,7 +53,7 @@ __device__ __forceinline__ bool softmax_tile(f32x16 (&s)[NT], Frag<T> (&pf)[NT][
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
         for (int j = 0; j < 16; ++j) mx = fmaxf(mx, s[nt][j]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32));  // the other half of the row lives in lane ^ 32
+    mx = with_lane_xor<32, 64>(mx, [](float a, float b) { return fmaxf(a, b); });  // the other half of the row lives in lane ^ 32
     // move the reference only when some row's maximum has outrun it by the threshold (always on the first
     // live tile); rows that do not move keep alpha = 1
     if (__any((mx - m_ref) * c2 > kRescaleThreshold)) {
@@ -504,7 +504,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnParams p) {
         constexpr int OROW = D * ES + 16;  // padded row of the staging tile
         static_assert(4 * 32 * OROW <= NSTAGE * G::STAGE, "staging space");
         char* stg = smem + wave * (32 * OROW);
-        const float l_tot = l_run + __shfl_xor(l_run, 32);
+        const float l_tot = with_lane_xor<32, 64>(l_run, [](float a, float b) { return a + b; });
         const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
         if (p.lse != nullptr && g == 0) {
             // probabilities are exp(scale * score - lse); a row without live columns gets +inf (every probability 0)

@@ -102,7 +102,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(const BwdParams p) {
         for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
             for (int e = 0; e < 8; ++e) s = fmaf((float)bf[ks].v[e], (float)of[ks].v[e], s);
-        s += __shfl_xor(s, 32);
+        s = with_lane_xor<32, 64>(s, [](float a, float b) { return a + b; });
         row_delta = s;  // (stored after the tile loop: a store in flight would be waited for with the first tile's copies)
     }
 

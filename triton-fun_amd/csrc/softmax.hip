@@ -159,8 +159,7 @@ __global__ __launch_bounds__(256) void softmax_rows_vec(const Tin* __restrict__ 
                     mx = fmaxf(mx, v[c][e]);
                 }
             }
-#pragma unroll
-            for (int o = LPR / 2; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+            mx = wave_max<LPR>(mx);
             const float mb = mx * kLog2e;
 #pragma unroll
             for (int c = 0; c < NCH; ++c)
@@ -181,8 +180,7 @@ __global__ __launch_bounds__(256) void softmax_rows_vec(const Tin* __restrict__ 
                     }
                 }
             }
-#pragma unroll
-            for (int o = LPR / 2; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+            mx = wave_max<LPR>(mx);
             const float mb = mx * kLog2e;
 #pragma unroll
             for (int c = 0; c < NCH; ++c) {
@@ -198,8 +196,7 @@ __global__ __launch_bounds__(256) void softmax_rows_vec(const Tin* __restrict__ 
                 }
             }
         }
-#pragma unroll
-        for (int o = LPR / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+        sum = wave_sum<LPR>(sum);
         const float inv = sum > 0.f ? 1.0f / sum : 0.f;
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
