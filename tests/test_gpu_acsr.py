@@ -246,6 +246,25 @@ def test_mask_tensors_of_any_pitch_in_one_kernel(dev, rows, cols, pitch, offset,
     check_acsr(mask, BH, dev)
 
 
+@pytest.mark.parametrize("BH", [1, 15, 63, 65, 200])
+def test_rows_solved_together_and_bytes_beyond_one(dev, BH):
+    """Row blocks around the 64 rows that are solved at once; the first two ones at every place of a 16-byte piece and in
+    different pieces, after and before bytes that are live without being one."""
+    rows, cols = 200, 333
+    mask = torch.zeros(rows, cols, dtype=torch.uint8)
+    for r in range(rows):
+        if r % 23 == 22:
+            continue  # an empty row
+        a, b = 10 + r % 40, 11 + r % 40 + r % 37
+        mask[r, a] = 1
+        if r % 29 == 28:
+            continue  # a row of a single column
+        mask[r, b] = 1
+        mask[r, r % 8] = 2 + r % 254 if r % 3 == 0 else 0
+        mask[r, 100 + r % 99: 332 - r % 61: 1 + r % 5] = 1 if r % 2 else 255
+    check_acsr(mask.to(dev), BH, dev)
+
+
 def test_the_returned_metadata_saves_and_copies(dev):
     """Every tensor of a build by the one-kernel path, alone and all together, with the attributes the launchers read, through
     torch.save (which takes no tensors of two types on one storage) and copy.deepcopy."""

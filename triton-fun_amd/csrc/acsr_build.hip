@@ -34,21 +34,34 @@ struct RowScan {
             m2 = col;
         }
     }
-    __device__ __forceinline__ void dword(uint32_t x, int col0) {
-        if (x == 0) return;
-        sum = __builtin_amdgcn_sad_u8(x, 0u, sum);
-        uint32_t nz = ~zero_bytes(x) & 0x80808080u;  // bytes that are nonzero
-        int lo = (__builtin_ctz(nz) >> 3), hi = ((31 - __builtin_clz(nz)) >> 3);
-        first = min(first, col0 + lo);
-        last = max(last, col0 + hi);
-        if (m2 == kInf) {
-            uint32_t eq = zero_bytes(x ^ 0x01010101u);  // bytes equal to 1
-            while (eq) {
-                int b = __builtin_ctz(eq) >> 3;
-                add_one(col0 + b);
-                eq &= eq - 1;
-            }
+    // 16 bytes of columns behind all that this lane has seen: bit c of a 16-bit mask for column col0 + c
+    __device__ __forceinline__ void piece(const u32x4& x, int col0) {
+        const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+        uint32_t nz[4], one[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            sum = __builtin_amdgcn_sad_u8(w[k], 0u, sum);
+            nz[k] = ~zero_bytes(w[k]) & 0x80808080u;
+            one[k] = zero_bytes(w[k] ^ 0x01010101u);
         }
+        const uint32_t live = columns(nz), ones = columns(one);
+        if (live) {
+            first = min(first, col0 + __builtin_ctz(live));
+            last = col0 + 31 - __builtin_clz(live);
+        }
+        if (ones && m2 == kInf) {
+            const int a = col0 + __builtin_ctz(ones);
+            const uint32_t rest = ones & (ones - 1);
+            const int b = rest ? col0 + __builtin_ctz(rest) : kInf;
+            m2 = m1 == kInf ? b : a;
+            m1 = min(m1, a);
+        }
+    }
+    // the 0x80 of 16 bytes as 16 bits: a dot product with the powers of two (sums of at most 128 * 255)
+    static __device__ __forceinline__ uint32_t columns(const uint32_t (&f)[4]) {
+        const uint32_t lo = __builtin_amdgcn_udot4(f[1], 0x80402010u, __builtin_amdgcn_udot4(f[0], 0x08040201u, 0u, false), false);
+        const uint32_t hi = __builtin_amdgcn_udot4(f[3], 0x80402010u, __builtin_amdgcn_udot4(f[2], 0x08040201u, 0u, false), false);
+        return (lo >> 7) | (hi << 1);
     }
     __device__ __forceinline__ void byte(uint32_t x, int col) {
         if (x == 0) return;
@@ -58,19 +71,12 @@ struct RowScan {
         if (x == 1) add_one(col);
     }
     __device__ __forceinline__ void wave_reduce() {
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            uint32_t s2 = __shfl_xor(sum, o);
-            int a1 = __shfl_xor(m1, o), a2 = __shfl_xor(m2, o);
-            int f2 = __shfl_xor(first, o), l2 = __shfl_xor(last, o);
-            sum += s2;
-            int n1 = min(m1, a1);
-            int n2 = min(max(m1, a1), min(m2, a2));
-            m1 = n1;
-            m2 = n2;
-            first = min(first, f2);
-            last = max(last, l2);
-        }
+        sum = (uint32_t)over_lanes<64>((int)sum, [](int a, int b) { return a + b; });
+        const int a = wave_min_i(m1);  // (in one lane, whose second one is the only other candidate it has)
+        m2 = wave_min_i(m1 == a ? m2 : m1);
+        m1 = a;
+        first = wave_min_i(first);
+        last = wave_max_i(last);
     }
 };
 
@@ -134,18 +140,18 @@ __device__ __forceinline__ bool finish_row(const RowScan& s, int row, int cols, 
 // the summary: T = max nnz, smallest / largest column step over rows with nnz > 1, how many rows with nnz > 1 have a first
 // column that is not congruent to the row index modulo their step, and how many the reference would have asserted on.
 struct BlockFold {
-    double lo, hi;
+    float lo, hi;  // (a rounding is monotone: the least of the rounded is the least, rounded)
     int t_max, step_min, step_max, off_phase, failed;
     __device__ __forceinline__ void init(int cols) {
-        lo = (double)cols, hi = -1.0;
+        lo = (float)cols, hi = -1.0f;
         t_max = 0, step_min = 0x7fffffff, step_max = 0, off_phase = 0, failed = 0;
     }
     __device__ __forceinline__ void row(int r, float linf, float trans, int cnt) {
         const int lin = (int)linf;
         const int a = (int)rintf(linf * trans);
         const double t = (double)a / (double)lin;
-        lo = fmin(lo, t);
-        hi = fmax(hi, (double)((int64_t)cnt * lin) + t);
+        lo = fminf(lo, (float)t);
+        hi = fmaxf(hi, (float)((double)((int64_t)cnt * lin) + t));
         t_max = max(t_max, cnt);
         if (cnt > 1) {
             step_min = min(step_min, lin);
@@ -153,83 +159,87 @@ struct BlockFold {
             off_phase += ((a - r) % lin) != 0;
         }
     }
-    __device__ __forceinline__ void merge(const BlockFold& b) {
-        lo = fmin(lo, b.lo), hi = fmax(hi, b.hi);
-        t_max = max(t_max, b.t_max), step_min = min(step_min, b.step_min), step_max = max(step_max, b.step_max);
-        off_phase += b.off_phase, failed += b.failed;
+    __device__ __forceinline__ void wave_reduce() {
+        auto add = [](int a, int b) { return a + b; };
+        lo = over_lanes<64>(lo, [](float a, float b) { return fminf(a, b); }), hi = wave_max(hi);
+        t_max = wave_max_i(t_max), step_min = wave_min_i(step_min), step_max = wave_max_i(step_max);
+        off_phase = over_lanes<64>(off_phase, add), failed = over_lanes<64>(failed, add);
     }
 };
 
-__device__ __forceinline__ void scan_chunk(RowScan& s, const u32x4& x, int c) {
-    if ((x.x | x.y | x.z | x.w) == 0) return;
-    s.dword(x.x, c);
-    s.dword(x.y, c + 4);
-    s.dword(x.z, c + 8);
-    s.dword(x.w, c + 12);
-}
-
 // A workgroup takes `per_block` consecutive rows, a wavefront one row at a time: 16-byte pieces from the row's first aligned
-// address on (rows of any pitch), eight per lane in flight, and single bytes at the two ends.  Sixteen wavefronts and at most
-// 64 registers, so that a CU holds two workgroups and the loads of 32 rows are in flight at once: a mask of 8192 rows is one
-// wave of workgroups over the chip.  No cross-wavefront traffic but the block's fold.
+// address on (rows of any pitch), four per lane in flight, and single bytes at the two ends.  Sixteen wavefronts and at most
+// 64 registers, so that a CU holds two workgroups: a mask of 8192 rows is one wave of workgroups over the chip.  What a
+// wavefront found goes to LDS; the first one solves up to 64 rows at once, a lane each, and stores them side by side.
 //
 // FOLD: the workgroup's rows are one span block; its spans and its share of the summary (5 integers, 8 apart, into memory
 // that the host reads) come from the same kernel.  With a second kernel for the spans, which walks 16 rows a thread with
 // few threads, and the summary read back through a copy, an 8192 x 8192 mask took 23 us on the GPU in two kernels and 95 us
-// for the whole call; in this one kernel 16.7 us (4.0 TB/s) and 37 us.
+// for the whole call.  One kernel in which every wavefront's first lane solved its row and the workgroup's first thread
+// folded the wavefronts' one by one: 16.6 us, 36.1 for the call.  This one, whose pieces are read without a branch per dword:
+// 12.4 us with eight pieces in flight and about 10.7 with four, which need less code and no spills (two pieces + 1.3 us,
+// 8 wavefronts + 0.2, 4 wavefronts + 2.7); 30.7 for the call: the 67 MB at the rate of a large copy.
 constexpr int kRowWaves = 16;
 template <bool FOLD>
 __global__ __launch_bounds__(64 * kRowWaves, 8) void acsr_rows_kernel(const uint8_t* __restrict__ mask, int rows, int cols, int64_t ld,
                                                                       int per_block, RowOut o, int32_t* __restrict__ summary,
                                                                       int32_t* __restrict__ shares) {
-    __shared__ BlockFold s_fold[kRowWaves];
+    __shared__ RowScan s_row[2][64];
     if constexpr (!FOLD) init_summary(summary);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n_waves = blockDim.x >> 6;
     const int r_end = min(rows, ((int)blockIdx.x + 1) * per_block);
-    constexpr int NB = 8;
+    constexpr int NB = 4;
     BlockFold f;
     f.init(cols);
-    for (int row = blockIdx.x * per_block + wave; row < r_end; row += n_waves) {
-        const uint8_t* p = mask + (int64_t)row * ld;
-        const int head = min(cols, (int)(-reinterpret_cast<uintptr_t>(p) & 15));
-        const int nvec = (cols - head) >> 4;
-        const u32x4* pv = reinterpret_cast<const u32x4*>(p + head);
-        RowScan s;
-        s.init();
-        const int tail0 = head + (nvec << 4);  // fewer than 16 bytes before `head` and fewer than 16 from `tail0` on
-        uint32_t edge = 0;
-        const int edge_col = lane < 16 ? lane : tail0 + lane - 16;
-        if (lane < 16 ? lane < head : (lane < 32 && edge_col < cols)) edge = p[edge_col];
-        for (int i0 = lane; i0 < nvec; i0 += 64 * NB) {
-            u32x4 xs[NB];
+    int turn = 0;
+    for (int base = blockIdx.x * per_block; base < r_end; base += 64, turn ^= 1) {
+        const int n = min(64, r_end - base);
+        for (int k = wave; k < n; k += n_waves) {
+            const uint8_t* p = mask + (int64_t)(base + k) * ld;
+            const int head = min(cols, (int)(-reinterpret_cast<uintptr_t>(p) & 15));
+            const int nvec = (cols - head) >> 4;
+            const u32x4* pv = reinterpret_cast<const u32x4*>(p + head);
+            RowScan s;
+            s.init();
+            const int tail0 = head + (nvec << 4);  // fewer than 16 bytes before `head` and fewer than 16 from `tail0` on
+            uint32_t edge = 0;
+            const int edge_col = lane < 16 ? lane : tail0 + lane - 16;
+            if (lane < 16 ? lane < head : (lane < 32 && edge_col < cols)) edge = p[edge_col];
+            for (int i0 = lane; i0 < nvec; i0 += 64 * NB) {
+                u32x4 xs[NB];
 #pragma unroll
-            for (int u = 0; u < NB; ++u) xs[u] = i0 + 64 * u < nvec ? __builtin_nontemporal_load(pv + i0 + 64 * u) : u32x4{0, 0, 0, 0};
+                for (int u = 0; u < NB; ++u) xs[u] = i0 + 64 * u < nvec ? __builtin_nontemporal_load(pv + i0 + 64 * u) : u32x4{0, 0, 0, 0};
 #pragma unroll
-            for (int u = 0; u < NB; ++u) scan_chunk(s, xs[u], head + ((i0 + 64 * u) << 4));
+                for (int u = 0; u < NB; ++u)
+                    if ((xs[u].x | xs[u].y | xs[u].z | xs[u].w) != 0) s.piece(xs[u], head + ((i0 + 64 * u) << 4));
+            }
+            s.byte(edge, edge_col);
+            s.wave_reduce();
+            if (lane == 0) s_row[turn][k] = s;
         }
-        s.byte(edge, edge_col);
-        s.wave_reduce();
-        if (lane == 0) {
+        __syncthreads();  // (one is enough: wavefront 0 has read the half before when it comes to the next one)
+        if (wave == 0 && lane < n) {
             float lin, trans;
-            const bool failed = finish_row(s, row, cols, o, FOLD ? 1.0f : kUnpackFailed, &lin, &trans);
+            const RowScan s = s_row[turn][lane];
+            const bool failed = finish_row(s, base + lane, cols, o, FOLD ? 1.0f : kUnpackFailed, &lin, &trans);
             if constexpr (FOLD) {
                 f.failed += failed;
-                f.row(row, lin, trans, (int)s.sum);
+                f.row(base + lane, lin, trans, (int)s.sum);
             }
         }
     }
     if constexpr (FOLD) {
-        if (lane == 0) s_fold[wave] = f;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            for (int w = 1; w < n_waves; ++w) f.merge(s_fold[w]);
-            o.put(o.span_start, blockIdx.x, (float)f.lo);
-            o.put(o.span_end, blockIdx.x, (float)f.hi);
-            int4* const mine = reinterpret_cast<int4*>(shares) + 2 * blockIdx.x;
-            mine[0] = make_int4(f.t_max, f.failed, f.step_min, f.step_max);
-            mine[1] = make_int4(f.off_phase, 0, 0, 0);
+        if (wave == 0) {
+            f.wave_reduce();
+            if (lane == 0) {
+                o.put(o.span_start, blockIdx.x, f.lo);
+                o.put(o.span_end, blockIdx.x, f.hi);
+                int4* const mine = reinterpret_cast<int4*>(shares) + 2 * blockIdx.x;
+                mine[0] = make_int4(f.t_max, f.failed, f.step_min, f.step_max);
+                mine[1] = make_int4(f.off_phase, 0, 0, 0);
+            }
         }
     }
 }
@@ -255,8 +265,8 @@ __global__ __launch_bounds__(256) void acsr_spans_kernel(float* __restrict__ sTo
             }
             f.row(r, linf, sTod_trans[r], (int)nnz[r]);
         }
-        span_start[g] = (float)f.lo;
-        span_end[g] = (float)f.hi;
+        span_start[g] = f.lo;
+        span_end[g] = f.hi;
     }
     const int t_max = wave_max_i(f.t_max);
     const int step_min = wave_min_i(f.step_min);
