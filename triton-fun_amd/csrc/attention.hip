@@ -18,9 +18,10 @@
 // Which keys a tile holds is decided per workgroup from the rows' (a, lin, cnt) maps: if all rows
 // share the column step and phase, tiles enumerate exactly those columns (key index c0 + cs*j,
 // gathered rows of K/V) and validity is a per-row range test in j; otherwise tiles are dense columns
-// and validity is the full affine test (offset, step divisibility, count).  Each wavefront skips
-// tiles that lie outside all of its rows' spans and drops the mask on tiles inside all of them.
+// and validity is the full affine test (offset, step divisibility, count).  Each wavefront skips tiles (d = 64: halves of tiles)
+// that lie outside all of its rows' spans and drops the mask on tiles inside all of them.
 #include <mutex>
+#include <type_traits>
 
 #include "attn_tile.hpp"
 
@@ -388,32 +389,33 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnParams p) {
                 if (!spread) issue_tile_general(ppl, pf_tile, stage_pf);
             }
 
-            const bool skip = (j0 + BN <= w_lo_min) || (j0 >= w_hi_max);
-            if (!skip) {
+            // NP 32-key halves of the tile, from half `half` on
+            auto compute = [&](auto parts, int half) __attribute__((always_inline)) {
+                constexpr int NP = decltype(parts)::value;
                 const bool full = (j0 >= w_lo_max) && (j0 + BN <= w_hi_min);
-
+                const uint32_t k_half = NP < NT ? half * 32 * G::K_ROWB : 0, v_half = NP < NT ? half * 32 * G::V_ROWB : 0;
                 // ---- S^T = K . Q^T ----
                 // K fragments are requested from LDS a few MFMAs ahead of their use, never more than 12 read
                 // instructions at a time: the counter that tracks them holds 15, and the compiler falls back to
                 // waiting for every outstanding read once it could overflow.
-                f32x16 s_acc[NT];
+                f32x16 s_acc[NP];
 #pragma unroll
-                for (int nt = 0; nt < NT; ++nt)
+                for (int nt = 0; nt < NP; ++nt)
 #pragma unroll
                     for (int j = 0; j < 16; ++j) s_acc[nt][j] = 0.f;
-                Frag<T> kfr[NT][KS];
+                Frag<T> kfr[NP][KS];
                 auto load_k = [&](int nt, int ks) {
                     Frag<T> kf;
                     if constexpr (KT) {
                         // rows 16ks + 8g + {0..3} and +4: multiples of 4 rows leave the lane's swizzle term alone
-                        const uint32_t a0 = k_addr[nt] + 16 * ks * G::K_ROWB;
+                        const uint32_t a0 = (NP < NT && half ? k_addr[NT - 1] : k_addr[nt]) + 16 * ks * G::K_ROWB;
                         kf = frag_from_tr<T>(lds_load_tr16(a0), lds_load_tr16(a0 + 4 * G::K_ROWB));
                     } else {
-                        kf.v = __builtin_bit_cast(typename Frag<T>::vec, lds_load128(k_addr[ks] + 32 * nt * G::K_ROWB));
+                        kf.v = __builtin_bit_cast(typename Frag<T>::vec, lds_load128(k_addr[ks] + k_half + 32 * nt * G::K_ROWB));
                     }
                     return kf;
                 };
-                constexpr int NMMA = NT * KS;
+                constexpr int NMMA = NP * KS;
                 constexpr int K_AHEAD = (KT ? 6 : 12) < NMMA ? (KT ? 6 : 12) : NMMA;  // fragments
 #pragma unroll
                 for (int i = 0; i < K_AHEAD; ++i) kfr[i / KS][i % KS] = load_k(i / KS, i % KS);
@@ -440,18 +442,22 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnParams p) {
                     }
                 }
                 // ---- mask, online softmax against a lazily updated reference ----
-                Frag<T> pf[NT][2];
-                if (!full) mask_tile<NT>(s_acc, row_live_bits(win, j0, first, pat), g);
+                Frag<T> pf[NP][2];
+                if (!full) {
+                    const uint64_t live = row_live_bits(win, j0, first, pat);
+#pragma unroll
+                    for (int nt = 0; nt < NP; ++nt) mask_half(s_acc[nt], (uint32_t)(live >> (32 * (half + nt))) >> (4 * g));
+                }
                 if (settled && !careful_only)
-                    l_run += exp_tile<NT, T>(s_acc, pf, m_ref * c2, c2);
+                    l_run += exp_tile<NP, T>(s_acc, pf, m_ref * c2, c2);
                 else
-                    settled = softmax_tile<NT, T, DT>(s_acc, pf, m_ref, l_run, o_acc, c2);
+                    settled = softmax_tile<NP, T, DT>(s_acc, pf, m_ref, l_run, o_acc, c2);
 
                 // ---- O^T += V^T . P^T ----
                 // V fragments are requested one 16-key step (DT fragments) ahead of the MFMAs that consume them.
                 auto load_v = [&](int nt, int t, int dt) {
                     Frag<T> vf;
-                    const uint32_t a0 = v_addr[dt] + (32 * nt + 16 * t) * G::V_ROWB;
+                    const uint32_t a0 = v_addr[dt] + v_half + (32 * nt + 16 * t) * G::V_ROWB;
                     vf = frag_from_tr<T>(lds_load_tr16(a0), lds_load_tr16(a0 + 8 * G::V_ROWB));
                     return vf;
                 };
@@ -460,17 +466,28 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnParams p) {
                 for (int dt = 0; dt < DT; ++dt) vfr[0][dt] = load_v(0, 0, dt);
                 __builtin_amdgcn_sched_barrier(0);  // keep the requests above the matrix work
 #pragma unroll
-                for (int step = 0; step < 2 * NT; ++step) {
+                for (int step = 0; step < 2 * NP; ++step) {
                     const int nt = step >> 1, t = step & 1;
 #pragma unroll
                     for (int dt = 0; dt < DT; ++dt) {
                         mma32(o_acc[dt], vfr[step & 1][dt], pf[nt][t]);
-                        if (step + 1 < 2 * NT) {
+                        if (step + 1 < 2 * NP) {
                             vfr[(step + 1) & 1][dt] = load_v((step + 1) >> 1, (step + 1) & 1, dt);
                             __builtin_amdgcn_sched_barrier(0);
                         }
                     }
                 }
+            };
+            // A wavefront of 32 rows ends its span in the middle of a tile as often as not.  Where half of a tile holds nothing
+            // for it, that half is left out: 64 heads of 4096, d = 64, window 256, 44.6 -> 43.7 us, 256 keys with step 3
+            // 39.1 -> 38.3, two segments 39.3 -> 38.3; a walk without such tiles takes no more tests than before.  Not at d = 128: the
+            // second path's code costs its first fetch, 1 us of 50 at windows up to 64, against 1 % gained at 512.
+            constexpr bool BY_HALVES = D == 64 && NT == 2;
+            constexpr int NEAR = BY_HALVES ? BN / 2 : BN, FAR = BN - NEAR;
+            if (j0 + NEAR > w_lo_min && j0 + FAR < w_hi_max) {
+                compute(std::integral_constant<int, NT>{}, 0);
+            } else if (BY_HALVES && j0 + BN > w_lo_min && j0 < w_hi_max) {
+                if constexpr (BY_HALVES) compute(std::integral_constant<int, 1>{}, j0 + BN / 2 > w_lo_min ? 0 : 1);
             } else if (spread) {
 #pragma unroll
                 for (int s = 0; s < NDMA; ++s) issue_step(s, stage_pf);

@@ -375,6 +375,16 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(const BwdParams p) {
             } else
 #pragma unroll
             for (int nt = 0; nt < 2; ++nt) {
+                static_assert(!THREE || NDMA <= KS, "the first half issues all copies");
+                // half a tile that holds nothing for this wavefront, as at the ends of most spans (bfloat16, 64 heads of 4096, the
+                // whole step: window 65 at d = 64 131 -> 123 us, 33 at d = 128 257 -> 252; 64 heads of 8192, 512 / 2, 985 -> 977)
+                if (nt == 0 ? j0 + 32 <= w_lo_min : j0 + 32 >= w_hi_max) {
+                    if (nt == 0 && spread) {
+#pragma unroll
+                        for (int s = 0; s < NDMA; ++s) issue_step(s, stage_pf);
+                    }
+                    continue;
+                }
                 // ---- S^T (32 positions x 32 rows) = X rows . A^T ----
                 f32x16 s_acc;
 #pragma unroll
@@ -394,14 +404,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(const BwdParams p) {
                         __builtin_amdgcn_sched_barrier(0);
                     }
                 }
-                if (!full) {
-                    const uint32_t bits = (uint32_t)(live >> (32 * nt)) >> (4 * g);
-#pragma unroll
-                    for (int j = 0; j < 16; ++j) {
-                        const int c = 8 * (j >> 2) + (j & 3);
-                        s_acc[j] = keep_or_mask(s_acc[j], ((int)(bits << (31 - c))) >> 31);
-                    }
-                }
+                if (!(j0 + 32 * nt >= w_lo_max && j0 + 32 * nt + 32 <= w_hi_min)) mask_half(s_acc, (uint32_t)(live >> (32 * nt)) >> (4 * g));
                 // ---- P^T = exp2(S^T * scale*log2e - lse*log2e); masked scores underflow to exactly 0 ----
                 if constexpr (POS_STATS) {
 #pragma unroll

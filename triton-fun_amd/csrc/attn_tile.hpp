@@ -54,18 +54,13 @@ __device__ __forceinline__ float keep_or_mask(float x, int keep) {
     return __builtin_bit_cast(float, (xb & (uint32_t)keep) | (nb & ~(uint32_t)keep));
 }
 
-// Accumulator register j of 32-key half nt of a lane holds position 32*nt + 8*(j/4) + 4*g + j%4 of the tile; its bit
-// of `live` (see row_live_bits) says whether the score is kept.
-template <int NT>
-__device__ __forceinline__ void mask_tile(f32x16 (&s)[NT], uint64_t live, int g) {
+// Accumulator register j of a 32-key half of a tile holds the half's position 8*(j/4) + 4*g + j%4; `bits`, the half's part
+// of `live` (see row_live_bits) moved down by 4*g, says whether the score is kept.
+__device__ __forceinline__ void mask_half(f32x16& s, uint32_t bits) {
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-        const uint32_t bits = (uint32_t)(live >> (32 * nt)) >> (4 * g);
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const int c = 8 * (j >> 2) + (j & 3);
-            s[nt][j] = keep_or_mask(s[nt][j], ((int)(bits << (31 - c))) >> 31);
-        }
+    for (int j = 0; j < 16; ++j) {
+        const int c = 8 * (j >> 2) + (j & 3);
+        s[j] = keep_or_mask(s[j], ((int)(bits << (31 - c))) >> 31);
     }
 }
 
