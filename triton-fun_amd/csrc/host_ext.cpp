@@ -449,7 +449,10 @@ PyObject* py_sddmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
         // than 256 slots the general kernel, which is faster on rows of K as well (4 heads of 4001 rows, 301 slots, d = 64: 49 -> 43).  Beyond d = 64 the copy costs as much as it gives (64 heads of 2048 rows, 255 slots: d = 80 122 -> 125,
         // d = 96 126 -> 129), and so does its launch below 64 row blocks (one head of 200 rows: 21 -> 25).
         const bool turned = code != SPLAT_F32 && out_code == code && d % 8 == 0 && d <= 64 && B * H * ((L + 127) / 128) >= 64;
-        if ((m->max_step >= 2 || turned) && y.stride(3) == 1 && y.stride(2) != 1) {
+        // (float32 of up to 128 inner values turns K on its way into LDS, gathered or not, operators_f32.hip: 16 heads of 1605 rows,
+        // 176 slots with step 2, d = 128, the three operators 76.9 -> 72.3 us without the copy)
+        const bool in_place = code == SPLAT_F32 && out_code == code && d <= 128;
+        if (((m->max_step >= 2 && !in_place) || turned) && y.stride(3) == 1 && y.stride(2) != 1) {
             if (y.stride(2) < keys) Py_RETURN_FALSE;
             y = transposed_keys(y, &rc).transpose(2, 3);
             if (rc) return raise_rc("splat_transpose_keys", rc);

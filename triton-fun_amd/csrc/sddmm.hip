@@ -532,7 +532,9 @@ static int sddmm_common(const char* who, const void* q, int64_t q_sb, int64_t q_
     begin_launch();
     if (const int rc = launch_sddmm_lines(who, p, in_dtype, st)) return rc < 0 ? rc : check_launch(who);
     switch (in_dtype) {
-        case SPLAT_F32: return launch_sddmm<float>(who, p, kt, st);
+        case SPLAT_F32:
+            if (launch_sddmm_f32(p, kt, st)) return check_launch(who);
+            return launch_sddmm<float>(who, p, kt, st);
         case SPLAT_F16: return launch_sddmm<f16>(who, p, kt, st);
         default: return launch_sddmm<bf16>(who, p, kt, st);
     }

@@ -578,7 +578,9 @@ static int spmm_common(const char* who, const void* pp, const void* v, int64_t v
     begin_launch();
     if (const int rc = launch_spmm_thin(who, p, in_dtype, st)) return rc < 0 ? rc : check_launch(who);
     switch (in_dtype) {
-        case SPLAT_F32: return launch_spmm<float>(p, st);
+        case SPLAT_F32:
+            if (launch_spmm_f32(p, st)) return check_launch(who);
+            return launch_spmm<float>(p, st);
         case SPLAT_F16: return launch_spmm<f16>(p, st);
         default: return launch_spmm<bf16>(p, st);
     }

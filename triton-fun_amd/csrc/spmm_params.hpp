@@ -26,6 +26,8 @@ struct SpmmParams {
 int launch_spmm_thin(const char* who, const SpmmParams& p, int in_dtype, hipStream_t st);
 // The same for rows that are short or not aligned (see spmm_tile.hip; launch_spmm_thin hands them over).
 int launch_spmm_tile(const char* who, const SpmmParams& p, int in_dtype, hipStream_t st);
+// The same for float32 (see operators_f32.hip).
+int launch_spmm_f32(const SpmmParams& p, hipStream_t st);
 
 // ---- shared by the kernels of thin wavefronts ----
 // Physical 16-byte chunk of logical chunk c of V tile row `row`: the 64-byte block index is XORed with the row's low bits
