@@ -74,9 +74,9 @@ typedef struct splat_acsr_seg {
                                  row.  Used for rows with exactly one live column, whose stored
                                  translation acsr_helpers.py:126-130 hard-codes to 0.   */
     int32_t slot_offset;     /* first compressed slot of this segment (0 for one segment) */
-    int32_t row_stride_hint; /* 0 or 1: none.  n > 1: every row's column step is n and its first column is
-                                congruent to the row index modulo n (splat_acsr_build reports this in
-                                summary[2..4]); kernels then group rows by phase.  Only affects speed. */
+    int32_t row_stride_hint; /* 0 or 1: none.  n > 1: every row's column step is n and its first column less
+                                the row index has one residue modulo n (splat_acsr_build reports this in
+                                summary[2..6]); kernels then group rows by phase.  Only affects speed. */
 } splat_acsr_seg;
 
 int splat_version(void);
@@ -95,7 +95,8 @@ const char* splat_last_error(void);
  *                      assertion (nnz > 1 but fewer than two entries equal to 1), [2] / [3] smallest / largest column
  *                      step over rows with nnz > 1 (INT32_MAX / 0 when there is none), [4] number of rows with
  *                      nnz > 1 whose first column is not congruent to the row index modulo the row's step,
- *                      [5..7] reserved.
+ *                      [5] / [6] smallest / largest residue of first column - row index modulo the row's step over
+ *                      these rows (INT32_MAX / 0 when there is none), [7] reserved.
  * Reads rows*ld bytes once; the caller reads `summary` back after synchronising the stream. */
 int splat_acsr_build(const uint8_t* mask, int64_t rows, int64_t cols, int64_t ld,
                      int32_t block_height, float* dTos_lin, float* dTos_trans, float* sTod_lin,
@@ -109,7 +110,7 @@ int splat_acsr_build(const uint8_t* mask, int64_t rows, int64_t cols, int64_t ld
  *   extents   device: row_first, row_last, with the rows' distance
  *   duplicate not 0: both buffers are twice as long and the same arrays are written again behind the first ones
  *   shares    [ceil(rows/block_height)][8] int32, device-accessible memory that the host can read (pinned): per row block
- *             the five figures of `summary` above, in its order, over the block's rows alone; complete once the stream
+ *             the first seven figures of `summary` above, in its order, over the block's rows alone; complete once the stream
  *             has been waited for */
 int splat_acsr_build_record(const uint8_t* mask, int64_t rows, int64_t cols, int64_t ld, int32_t block_height, float* record,
                             int32_t* extents, int32_t duplicate, int32_t* shares, void* stream);

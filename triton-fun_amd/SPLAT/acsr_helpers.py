@@ -263,7 +263,8 @@ class AcsrBuild:
     def resolve(self) -> None:
         if self.summary is None:
             return
-        _checked_summary(self, *self.summary.tolist()[:5])  # the one synchronisation: T is returned as a Python int, like the reference
+        t_max, failed, step_min, step_max, _, res_min, res_max = self.summary.tolist()[:7]
+        _checked_summary(self, t_max, failed, step_min, step_max, res_min, res_max)  # the one synchronisation: T is returned as a Python int, like the reference
 
     @property
     def T(self) -> int:
@@ -281,12 +282,18 @@ class AcsrBuild:
         return self._max_step
 
 
-def _checked_summary(b: AcsrBuild, t_max: int, failed: int, step_min: int, step_max: int, off_phase: int) -> None:
+def _checked_summary(b: AcsrBuild, t_max: int, failed: int, step_min: int, step_max: int, res_min: int, res_max: int) -> None:
     b.summary = None
     assert failed == 0, "Incorrect unpacking of affine-indices."
     b._T = t_max
-    # rows whose columns step by n and start in phase with the row index (dilated windows): kernels group them by phase
-    b._row_stride = step_min if (step_min == step_max and step_max > 1 and off_phase == 0) else 1
+    # Rows whose columns step by n and whose first column less the row index has one residue modulo n (dilated windows): kernels group
+    # the rows by phase and walk every n-th column (bfloat16 forward, 64 heads of 8192 rows, 511 slots with step 2: 347 -> 206 us).  With
+    # 32 rows a phase or fewer, row blocks of 128 hold little: 128 heads of 512 rows, 5 slots with step 60, take 16 us on dense
+    # columns and 41 grouped, with step 16 a training step 81 and 103; 128 heads of 160 rows, step 4 (40 a phase) 14.8 and 12.7.  A
+    # single head is faster grouped there too (2 of 512, step 60: 9.4 and 4.7), so rows in phase with their index, residue 0, which
+    # programs of few heads have had grouped all along, stay so at any number.
+    grouped = res_min == res_max and (res_min == 0 or b.nnz.shape[0] > 32 * step_max)
+    b._row_stride = step_min if (step_min == step_max and step_max > 1 and grouped) else 1
     # the largest column step of any row: above 1 some rows are gathered (dilated windows, strided far fields)
     b._max_step = step_max
 

@@ -83,7 +83,7 @@ struct RowScan {
 // The summary's starting values, written by the first workgroup of the rows kernel (no kernel of its own): the rows
 // kernels themselves never touch the summary otherwise, the span kernel that follows them reduces into it.
 __device__ __forceinline__ void init_summary(int32_t* summary) {
-    if (blockIdx.x == 0 && threadIdx.x < 8) summary[threadIdx.x] = (threadIdx.x == 2) ? 0x7fffffff : 0;
+    if (blockIdx.x == 0 && threadIdx.x < 8) summary[threadIdx.x] = (threadIdx.x == 2 || threadIdx.x == 5) ? 0x7fffffff : 0;
 }
 constexpr float kUnpackFailed = 0.0f;  // stored as a row's sTod_lin (a real step is >= 1) until the span kernel has counted it
 
@@ -137,14 +137,15 @@ __device__ __forceinline__ bool finish_row(const RowScan& s, int row, int cols, 
 
 // The rows of one span block folded together: span_start = min(cols, min_r trans_r), span_end = max(-1, max_r nnz_r*lin_r +
 // trans_r), evaluated in double from the exact integers (a, lin, nnz) and rounded once to float32, and the block's share of
-// the summary: T = max nnz, smallest / largest column step over rows with nnz > 1, how many rows with nnz > 1 have a first
-// column that is not congruent to the row index modulo their step, and how many the reference would have asserted on.
+// the summary: T = max nnz, smallest / largest column step over rows with nnz > 1, how many of these have a first column that
+// is not congruent to the row index modulo their step, the smallest / largest residue of the first column less the row index, and how
+// many rows the reference would have asserted on.
 struct BlockFold {
     float lo, hi;  // (a rounding is monotone: the least of the rounded is the least, rounded)
-    int t_max, step_min, step_max, off_phase, failed;
+    int t_max, step_min, step_max, off_phase, res_min, res_max, failed;
     __device__ __forceinline__ void init(int cols) {
         lo = (float)cols, hi = -1.0f;
-        t_max = 0, step_min = 0x7fffffff, step_max = 0, off_phase = 0, failed = 0;
+        t_max = 0, step_min = 0x7fffffff, step_max = 0, off_phase = 0, res_min = 0x7fffffff, res_max = 0, failed = 0;
     }
     __device__ __forceinline__ void row(int r, float linf, float trans, int cnt) {
         const int lin = (int)linf;
@@ -156,13 +157,18 @@ struct BlockFold {
         if (cnt > 1) {
             step_min = min(step_min, lin);
             step_max = max(step_max, lin);
-            off_phase += ((a - r) % lin) != 0;
+            const int rem = (a - r) % lin;
+            const int res = rem < 0 ? rem + lin : rem;
+            off_phase += res != 0;
+            res_min = min(res_min, res);
+            res_max = max(res_max, res);
         }
     }
     __device__ __forceinline__ void wave_reduce() {
         auto add = [](int a, int b) { return a + b; };
         lo = over_lanes<64>(lo, [](float a, float b) { return fminf(a, b); }), hi = wave_max(hi);
         t_max = wave_max_i(t_max), step_min = wave_min_i(step_min), step_max = wave_max_i(step_max);
+        res_min = wave_min_i(res_min), res_max = wave_max_i(res_max);
         off_phase = over_lanes<64>(off_phase, add), failed = over_lanes<64>(failed, add);
     }
 };
@@ -172,7 +178,7 @@ struct BlockFold {
 // 64 registers, so that a CU holds two workgroups: a mask of 8192 rows is one wave of workgroups over the chip.  What a
 // wavefront found goes to LDS; the first one solves up to 64 rows at once, a lane each, and stores them side by side.
 //
-// FOLD: the workgroup's rows are one span block; its spans and its share of the summary (5 integers, 8 apart, into memory
+// FOLD: the workgroup's rows are one span block; its spans and its share of the summary (7 integers, 8 apart, into memory
 // that the host reads) come from the same kernel.  With a second kernel for the spans, which walks 16 rows a thread with
 // few threads, and the summary read back through a copy, an 8192 x 8192 mask took 23 us on the GPU in two kernels and 95 us
 // for the whole call.  One kernel in which every wavefront's first lane solved its row and the workgroup's first thread
@@ -238,7 +244,7 @@ __global__ __launch_bounds__(64 * kRowWaves, 8) void acsr_rows_kernel(const uint
                 o.put(o.span_end, blockIdx.x, f.hi);
                 int4* const mine = reinterpret_cast<int4*>(shares) + 2 * blockIdx.x;
                 mine[0] = make_int4(f.t_max, f.failed, f.step_min, f.step_max);
-                mine[1] = make_int4(f.off_phase, 0, 0, 0);
+                mine[1] = make_int4(f.off_phase, f.res_min, f.res_max, 0);
             }
         }
     }
@@ -271,6 +277,8 @@ __global__ __launch_bounds__(256) void acsr_spans_kernel(float* __restrict__ sTo
     const int t_max = wave_max_i(f.t_max);
     const int step_min = wave_min_i(f.step_min);
     const int step_max = wave_max_i(f.step_max);
+    const int res_min = wave_min_i(f.res_min);
+    const int res_max = wave_max_i(f.res_max);
     const int off_phase = (int)wave_sum((float)f.off_phase);  // at most 64 * block_height per wavefront: exact in float
     const int failed = (int)wave_sum((float)f.failed);
     if ((threadIdx.x & 63) == 0) {
@@ -279,6 +287,8 @@ __global__ __launch_bounds__(256) void acsr_spans_kernel(float* __restrict__ sTo
         atomicMin(&summary[2], step_min);
         atomicMax(&summary[3], step_max);
         if (off_phase) atomicAdd(&summary[4], off_phase);
+        atomicMin(&summary[5], res_min);
+        atomicMax(&summary[6], res_max);
     }
 }
 

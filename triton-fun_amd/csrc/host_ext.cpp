@@ -683,13 +683,14 @@ PyObject* py_build(PyObject*, PyObject* const* a, Py_ssize_t n) {
         }
         written.waited = true;
         if (!wait_for(stream, shares)) return nullptr;
-        int32_t t_max = 0, bad = 0, step_min = 0x7fffffff, step_max = 0, off = 0;
+        int32_t t_max = 0, bad = 0, step_min = 0x7fffffff, step_max = 0, res_min = 0x7fffffff, res_max = 0;
         for (int64_t b = 0; b < blocks; ++b) {
             const int32_t* s = sh + 8 * b;
-            t_max = std::max(t_max, s[0]), bad += s[1], step_min = std::min(step_min, s[2]), step_max = std::max(step_max, s[3]), off += s[4];
+            t_max = std::max(t_max, s[0]), bad += s[1], step_min = std::min(step_min, s[2]), step_max = std::max(step_max, s[3]);
+            res_min = std::min(res_min, s[5]), res_max = std::max(res_max, s[6]);
         }
         share_buffers()->give(std::move(shares));
-        return Py_BuildValue("NNiiiii", sets[0].release(), sets[1].release(), t_max, bad, step_min, step_max, off);
+        return Py_BuildValue("NNiiiiii", sets[0].release(), sets[1].release(), t_max, bad, step_min, step_max, res_min, res_max);
     } catch (...) {
         return raise_current();
     }
