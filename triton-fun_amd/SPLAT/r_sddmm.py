@@ -93,8 +93,8 @@ def rsddmm_launcher(x: torch.Tensor, y: torch.Tensor, output: torch.Tensor,
     ``plan``: the mask's plan table (``ACSRSegments.plan``); by default the launches that use one (16-bit types, d a multiple
     of 8 up to 128, rows of K contiguous, at least 256 row blocks of 128 rows or rows of at most 256 slots) build it on their first
     call and keep it with the metadata, ``False`` launches without one.  The results are the same bit for bit, but for K^T with
-    unit stride along the keys: by default such a K is turned into rows first where that is faster (16-bit types, d up to 64, at
-    least 64 row blocks), with a plan given or ``False`` it is read in place, and the two differ in the order of the float32 additions.
+    unit stride along the keys: by default such a K is turned into rows first where that is faster (16-bit types, d up to 64, more
+    than 256 row blocks), with a plan given or ``False`` it is read in place, and the two differ in the order of the float32 additions.
     Returns (output, sTod_linear_transformations, sTod_translations, nnzs)."""
     for name, t in (("x", x), ("y", y), ("output", output)):
         _hip.require_device_tensor(t, name)
@@ -105,8 +105,8 @@ def rsddmm_launcher(x: torch.Tensor, y: torch.Tensor, output: torch.Tensor,
     if plan is None and x.dim() == 4 and y.dim() == 4 and output.shape[-1] == trailing_dim:
         B, H, L, d = x.shape
         blocks = B * H * ((L + 127) // 128)
-        # (the native path hands the kernels rows of K where they are rows already, where rows are gathered, and, up to d = 64, in launches
-        # of at least 64 row blocks, for which it turns K first: csrc/host_ext.cpp)
+        # (launches that read the table: rows of K, those that gather, and, up to d = 64, those of at least 64 row blocks, for which the
+        # native path turns K first or whose kernel turns it: csrc/host_ext.cpp)
         k_rows = y.stride(2) == 1 or (d <= 64 and blocks >= 64) or segs.gathered
         mask = segs.native(L, x.device, _takes_a_plan(x, output, blocks, d, k_rows, trailing_dim))
         if mask is not None and _hip.host().sddmm(mask, x, y, output, 1.0 if scale is None else scale, lse):

@@ -38,20 +38,6 @@ __device__ __forceinline__ f32x4 row_piece(const float* row, int c, int n, bool 
     return x;
 }
 
-// The extent of a wavefront's 16 rows in tile positions, as wave_span, from lanes that hold the window of row n = lane % 16
-__device__ __forceinline__ WaveSpan span_of_rows16(const RowWin& w, bool uniform) {
-    const bool empty = w.cnt <= 0;
-    auto lo = [](int a, int b) { return min(a, b); };
-    auto hi = [](int a, int b) { return max(a, b); };
-    WaveSpan s;
-    s.lo_min = __builtin_amdgcn_readfirstlane(over_rows16(empty ? 0x3fffffff : w.lo, lo));
-    s.lo_max = __builtin_amdgcn_readfirstlane(over_rows16(empty ? 0x3fffffff : w.lo, hi));
-    s.hi_min = __builtin_amdgcn_readfirstlane(over_rows16(empty ? -0x3fffffff : w.lo + w.cnt, lo));
-    s.hi_max = __builtin_amdgcn_readfirstlane(over_rows16(empty ? -0x3fffffff : w.lo + w.cnt, hi));
-    if (!uniform) s.lo_max = 0x3fffffff;
-    return s;
-}
-
 }  // namespace
 
 // out[bh, r, s] = scale * q[r] . k[column of slot s], or the probability exp(that - lse[r]).  S^T = K Q^T: a lane owns one row and

@@ -1,5 +1,5 @@
-// Pieces of the fused attention kernels whose wavefronts own 16 rows (attention_f32.hip, attention_bwd_f32.hip, attention_bwd_f32_keys.hip,
-// attention_rows16.hip): reductions over the lanes of a row, the walk of half a row block over its tiles, and the rows'
+// Pieces of the kernels whose wavefronts own 16 rows (attention_f32.hip, attention_bwd_f32.hip, attention_bwd_f32_keys.hip,
+// attention_rows16.hip, operators_f32.hip, sddmm_rows16.hip): reductions over the lanes of a row, the walk of half a row block over its tiles, and the rows'
 // windows.  Lane (n = lane % 16, g = lane / 16) holds row n's scores at positions 4g .. 4g + 3 of every subtile of 16.
 #pragma once
 #include "attn_tile.hpp"
@@ -26,6 +26,20 @@ __device__ __forceinline__ int over_rows16(int x, F f) {
     x = f(x, __builtin_amdgcn_update_dpp(0, x, 0x124, 0xf, 0xf, true));
     x = f(x, __builtin_amdgcn_update_dpp(0, x, 0x122, 0xf, 0xf, true));
     return f(x, __builtin_amdgcn_update_dpp(0, x, 0x121, 0xf, 0xf, true));
+}
+
+// The extent of a wavefront's 16 rows in tile positions, as wave_span, from lanes that hold the window of row n = lane % 16
+__device__ __forceinline__ WaveSpan span_of_rows16(const RowWin& w, bool uniform) {
+    const bool empty = w.cnt <= 0;
+    auto lo = [](int a, int b) { return min(a, b); };
+    auto hi = [](int a, int b) { return max(a, b); };
+    WaveSpan s;
+    s.lo_min = __builtin_amdgcn_readfirstlane(over_rows16(empty ? 0x3fffffff : w.lo, lo));
+    s.lo_max = __builtin_amdgcn_readfirstlane(over_rows16(empty ? 0x3fffffff : w.lo, hi));
+    s.hi_min = __builtin_amdgcn_readfirstlane(over_rows16(empty ? -0x3fffffff : w.lo + w.cnt, lo));
+    s.hi_max = __builtin_amdgcn_readfirstlane(over_rows16(empty ? -0x3fffffff : w.lo + w.cnt, hi));
+    if (!uniform) s.lo_max = 0x3fffffff;
+    return s;
 }
 
 // Position of a walk over tiles of BN positions: the segment, its plan, the next tile and the end of the segment's range.

@@ -530,6 +530,7 @@ static int sddmm_common(const char* who, const void* q, int64_t q_sb, int64_t q_
         if (segs[k].slot_offset % 8 != 0) p.out_vec = 0;
     hipStream_t st = (hipStream_t)stream;
     begin_launch();
+    if (in_dtype != SPLAT_F32 && launch_sddmm_rows16(p, in_dtype, kt, st)) return check_launch(who);
     if (const int rc = launch_sddmm_lines(who, p, in_dtype, st)) return rc < 0 ? rc : check_launch(who);
     switch (in_dtype) {
         case SPLAT_F32:

@@ -27,7 +27,9 @@ struct SddmmParams {
 // Launches the line-wise kernel when the problem has its shape (see sddmm_lines.hip); returns 1 when it did, 0 when the
 // general kernel has to run, a negative code on errors.  `p` is complete except for key_split / total.
 int launch_sddmm_lines(const char* who, const SddmmParams& p, int in_dtype, hipStream_t st);
-// The same for float32 inputs (see operators_f32.hip); `kt`: K is stored along the keys.
+// The same for 16-bit launches of few row blocks (see sddmm_rows16.hip); `kt`: K is stored along the keys.
+int launch_sddmm_rows16(const SddmmParams& p, int in_dtype, bool kt, hipStream_t st);
+// The same for float32 inputs (see operators_f32.hip).
 int launch_sddmm_f32(const SddmmParams& p, bool kt, hipStream_t st);
 
 }  // namespace splat

@@ -1,0 +1,204 @@
+// SDDMM on ACSR of 16-bit operands in launches of few row blocks, inner dimension up to 128.
+//
+// Such a launch is one chain of latencies a workgroup, row maps -> plan -> tile -> products -> stores, and what shortens it is
+// little work a workgroup: 64 rows of one (batch, head) in 4 wavefronts of 16, tiles of 64 positions requested a tile ahead through
+// registers, two stages, one barrier a tile, and a row block's tiles shared out over workgroups until there are two a CU (four: 10.4
+// for 9.1 us at 16 heads of 1024 rows, 300 slots, d = 32).  K stored along the keys is turned on its way into LDS, lanes = keys, wherever its
+// rows start and whatever the step.  The kernels that took these launches, bfloat16, heads of 1024 rows, us: rows of K, 4 heads, 129 slots, d = 128
+// (sddmm_lines.hip) 8.9 -> 6.6; 8 heads, 300 slots (sddmm.hip) d = 32 16.7 -> 7.5, d = 128 14.1 -> 8.6; K along the keys (sddmm.hip), 8 heads,
+// 33 slots, d = 80 15.7 -> 6.3, 32 heads 16.5 -> 8.0; where K was turned by a launch of its own first, 16 heads of 1000 rows, 129 slots,
+// d = 64, the three operators 26.5 -> 20.5.  An SpMM of this shape was slower than spmm_tile.hip's at every size (1.04 to 1.26).
+#include <algorithm>
+
+#include "rows16.hpp"
+#include "sddmm_params.hpp"
+
+namespace splat {
+
+namespace {
+
+constexpr int kTile = 64;
+static_assert(kPlanBM == 2 * kHalfRows && kBN == kTile, "half a row block of the plan per workgroup, its tiles");
+
+template <typename T>
+struct Vec4 {
+    typedef T type __attribute__((ext_vector_type(4)));
+};
+
+}  // namespace
+
+// S^T = K Q^T: a lane owns one row and holds four consecutive positions of every 16.  KS: 32-value steps of the contraction.
+template <typename T, int KS, bool KT>
+__global__ __launch_bounds__(256, 4) void sddmm_rows16_kernel(const SddmmParams p) {
+    constexpr int ROWB = KS == 1 ? 64 : KS == 2 ? 128 : 256;  // bytes of an LDS row: a power of two, for the swizzle
+    constexpr int STAGE = kTile * ROWB, CPR = 4 * KS, NP = kTile * CPR / 256;
+    typedef typename Vec4<T>::type vec4;
+
+    __shared__ __attribute__((aligned(1024))) char smem[2 * STAGE];
+    __shared__ SegPlan s_plan[SPLAT_MAX_SEGMENTS];
+    __shared__ PlanScratch<kHalfRows> s_ps;
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 15, g = lane >> 4;
+
+    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    if (logical >= p.total) return;
+    const int share = logical % p.key_split, block = logical / p.key_split;
+    const int per_head = 2 * p.n_row_blocks;  // halves of the plan's row blocks
+    const int bh = block / per_head;
+    const int at_block = per_head - 1 - block % per_head;
+    const int rb = at_block >> 1, half = at_block & 1;
+    const int b = bh / p.H, h = bh % p.H;
+    const int rs = p.row_stride, L = p.L, d = p.d;
+    const int r0 = block_first_row(rb, kPlanBM, rs) + rs * half * kHalfRows;
+    if (r0 >= L) return;
+
+    const T* kb = (const T*)p.k + b * p.k_sb + h * p.k_sh;
+    const int row_in = min(r0 + rs * (wave * 16 + n), L - 1);
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+
+    Frag<T> q[KS];
+    {
+        const T* qr = (const T*)p.q + b * p.q_sb + h * p.q_sh + (int64_t)row_in * p.q_sl;
+#pragma unroll
+        for (int t = 0; t < KS; ++t) {
+            q[t].v = __builtin_bit_cast(typename Frag<T>::vec, zero);
+            if (32 * t + 8 * g < d) q[t] = global_frag<T>(qr + 32 * t + 8 * g);
+        }
+    }
+    if (!p.plan) plan_segments<kHalfRows, kTile>(p.seg, p.n_seg, r0, rs, L, true, s_plan, &s_ps, tid);
+
+    const uint32_t base = lds_address(smem);
+    int pc_row[NP], pc_c[NP];
+    uint32_t pc_to[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+        const int f = tid + 256 * i;
+        pc_row[i] = KT ? f % kTile : f / CPR;
+        pc_c[i] = KT ? f / kTile : f % CPR;
+        pc_to[i] = base + lds_off<ROWB, true>(pc_row[i], pc_c[i] * 16);
+    }
+    uint32_t k_addr[KS];
+#pragma unroll
+    for (int t = 0; t < KS; ++t) k_addr[t] = base + lds_off<ROWB, true>(n, (4 * t + g) * 16);
+
+    T* const out_row = (T*)p.out + ((int64_t)bh * L + row_in) * p.T;
+    const float lse = p.row_lse ? p.row_lse[(int64_t)bh * L + row_in] : 0.f;
+
+    uint32_t stage = 0;
+    for (int sg = 0; sg < p.n_seg; ++sg) {
+        HalfWalk walk;
+        RowWin win;
+        if (p.plan) {
+            const PlanRec rec = p.plan[plan_row_at(p.n_row_blocks, p.n_seg, rb, sg, half * kHalfRows + wave * 16 + n)];
+            walk = half_walk<kTile>(p.plan, p.n_row_blocks, p.n_seg, rb, half, sg);
+            // (the table knows the mask alone: a row's slots are bounded by the buffer's here, as load_row_map does)
+            const int64_t most = walk.pl.uniform ? (int64_t)p.seg[sg].max_cnt : (int64_t)rec.z * (p.seg[sg].max_cnt - 1) + 1;
+            win.lo = rec.x, win.cnt = (int)min((int64_t)rec.y, most), win.lin = rec.z;
+        } else {
+            walk.pl.c0 = __builtin_amdgcn_readfirstlane(s_plan[sg].c0);
+            walk.pl.cs = __builtin_amdgcn_readfirstlane(s_plan[sg].cs);
+            walk.pl.n_tiles = __builtin_amdgcn_readfirstlane(s_plan[sg].n_tiles);
+            walk.pl.uniform = __builtin_amdgcn_readfirstlane(s_plan[sg].uniform);
+            walk.tile = 0, walk.end = walk.pl.n_tiles;
+            win = make_row_win(cached_row_map<kHalfRows>(&s_ps, sg, wave * 16 + n), walk.pl);
+        }
+        const SegPlan pl = walk.pl;
+        const int tiles = walk.end - walk.tile;
+        const int first = walk.tile + tiles * share / p.key_split, end = walk.tile + tiles * (share + 1) / p.key_split;
+        if (first >= end) continue;
+
+        u32x4 raw[NP];
+        auto load_tile = [&](int tile) {
+#pragma unroll
+            for (int i = 0; i < NP; ++i) {
+                const int key = min(max(pl.c0 + pl.cs * (tile * kTile + pc_row[i]), 0), p.n_keys - 1);
+                raw[i] = zero;
+                if (8 * pc_c[i] < d) {
+                    if constexpr (KT) {
+                        const T* src = kb + (int64_t)(8 * pc_c[i]) * p.k_sd + (int64_t)key * p.k_sl;
+                        Frag<T> f;
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) f.v[e] = src[e * p.k_sd];
+                        raw[i] = __builtin_bit_cast(u32x4, f.v);
+                    } else {
+                        raw[i] = *reinterpret_cast<const u32x4*>(kb + (int64_t)key * p.k_sl + 8 * pc_c[i]);
+                    }
+                }
+            }
+        };
+        load_tile(first);
+        const WaveSpan span = span_of_rows16(win, pl.uniform != 0);
+        T* const dst = out_row + p.seg[sg].slot_offset;
+
+        for (int tile = first; tile < end; ++tile) {
+            const int j0 = tile * kTile;
+#pragma unroll
+            for (int i = 0; i < NP; ++i) lds_store128(pc_to[i] + stage, raw[i]);
+            lds_barrier();  // the tile is there, and everybody is done with the one before it, whose stage comes next
+            if (tile + 1 < end) load_tile(tile + 1);
+#pragma unroll
+            for (int u = 0; u < kTile / 16; ++u) {
+                const int ju = j0 + 16 * u;
+                if (ju + 16 <= span.lo_min || ju >= span.hi_max) continue;
+                f32x4 s = {0.f, 0.f, 0.f, 0.f};
+                Frag<T> kf[KS];
+#pragma unroll
+                for (int t = 0; t < KS; ++t)
+                    kf[t].v = __builtin_bit_cast(typename Frag<T>::vec, lds_load128(k_addr[t] + stage + 16 * u * ROWB));
+#pragma unroll
+                for (int t = 0; t < KS; ++t) mma16(s, kf[t], q[t]);
+                s *= p.scale;
+                if (p.row_lse) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) s[j] = fast_exp2((s[j] - lse) * 1.4426950408889634f);
+                }
+                vec4 x;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) x[j] = (T)s[j];
+                const int at = ju + 4 * g - win.lo;  // of the lane's first position, from the row's first
+                if (ju >= span.lo_max && ju + 16 <= span.hi_min) {
+                    __builtin_memcpy(dst + at, &x, 8);  // any alignment
+                } else if (pl.uniform) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        if ((unsigned)(at + j) < (unsigned)win.cnt) dst[at + j] = x[j];
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        if (win_live(win, ju + 4 * g + j)) dst[win_slot(win, ju + 4 * g + j)] = x[j];
+                }
+            }
+            stage ^= STAGE;
+        }
+    }
+}
+
+int launch_sddmm_rows16(const SddmmParams& p0, int in_dtype, bool kt, hipStream_t st) {
+    if (p0.out_dtype != in_dtype || p0.d % 8 != 0 || p0.d > 128 || !p0.q_vec || (!kt && !p0.k_vec)) return 0;
+    SddmmParams p = p0;
+    p.n_row_blocks = count_row_blocks(p.L, kPlanBM, p.row_stride);
+    const int64_t blocks = 2 * (int64_t)p.B * p.H * p.n_row_blocks;
+    // The lines: rows of K, d <= 96: at 256 blocks 0.46 to 0.95 of the other kernels' time, at 512 0.84 to 1.08; d = 128 and short rows 0.65 to 1.01
+    // at 128, 0.89 to 1.03 at 256.  A second segment doubles the prologue: 0.95 to 0.99 at half of that, 1.01 to 1.06 there.  K along the
+    // keys, which the general kernel reads badly: 0.48 to 0.99 at 512, 0.66 to 1.20 at 1024.
+    if (blocks > (kt ? 512 : (p.d > 96 && p.T <= 256 ? 128 : 256) / p.n_seg)) return 0;
+    p.key_split = (int)std::min<int64_t>((p.T + kTile - 1) / kTile + 2, std::max<int64_t>(1, 512 / blocks));
+    p.total = (int)(blocks * p.key_split);
+    const int grid = ((p.total + 7) / 8) * 8;
+    auto go = [&](auto t, auto kt_c) {
+        using T = decltype(t);
+        constexpr bool KT = decltype(kt_c)::value;
+        if (p.d <= 32) sddmm_rows16_kernel<T, 1, KT><<<grid, 256, 0, st>>>(p);
+        else if (p.d <= 64) sddmm_rows16_kernel<T, 2, KT><<<grid, 256, 0, st>>>(p);
+        else if (p.d <= 96) sddmm_rows16_kernel<T, 3, KT><<<grid, 256, 0, st>>>(p);
+        else sddmm_rows16_kernel<T, 4, KT><<<grid, 256, 0, st>>>(p);
+    };
+    auto by_type = [&](auto kt_c) { return in_dtype == SPLAT_BF16 ? go(bf16{}, kt_c) : go(f16{}, kt_c); };
+    if (kt) by_type(std::true_type{});
+    else by_type(std::false_type{});
+    return 1;
+}
+
+}  // namespace splat
