@@ -168,15 +168,29 @@ __global__ __launch_bounds__(512, 4) void spmm_tile_kernel(const SpmmParams p) {
 #pragma unroll
             for (int i = 0; i < NI; ++i) *reinterpret_cast<u32x4*>(smem + stage * STAGE + v_lds[i]) = reg[i];
         };
-        auto write_p = [&](int stage, const u32x4 (&reg)[2]) {
+        // a piece as it was loaded, what it keeps of its place, and by how many entries it was loaded off that
+        struct Pieces {
+            u32x4 raw[2], keep[2];
+            int moved[2];
+        };
+        const bool some_risky = __builtin_amdgcn_readfirstlane(__any(risky)) != 0;
+        // The pieces are shifted and masked here, on their way into LDS: done where they are requested, a step waited for its own requests
+        // before its products.  The three operators, bfloat16: 96 heads of 3712 rows, 143 slots, d = 96 196 -> 187 us; 256 heads of 2048 rows,
+        // 40 slots, d = 32 156 -> 145; float16, 16 heads of 2000 rows, 129 slots, d = 80 26.6 -> 25.6.  What this path holds counts: with the
+        // masks read from LDS here and a test of each piece's own shift they took 204, 149 and 26.7.
+        auto write_p = [&](int stage, const Pieces& pc) {
 #pragma unroll
-            for (int c = 0; c < 2; ++c) *reinterpret_cast<u32x4*>(smem + stage * STAGE + p_lds[c]) = reg[c];
+            for (int c = 0; c < 2; ++c) {
+                u32x4 x = pc.raw[c];
+                if (some_risky) x = shift_elements(x, pc.moved[c]);
+                *reinterpret_cast<u32x4*>(smem + stage * STAGE + p_lds[c]) = x & pc.keep[c];
+            }
         };
         // This thread's two pieces of step s.  A piece that straddles an end of the row's span is loaded like any other, as 16
         // bytes from where its first entry would be, and the entries outside the span are cleared: what lies there (dead slots,
         // the neighbouring row) is readable memory except before the first and after the last row of the buffer, whose pieces
         // are loaded from inside the row and shifted.  (Steps past the last one hold nothing of any row: nothing is read.)
-        auto load_probs = [&](int s, u32x4 (&out)[2]) {
+        auto load_probs = [&](int s, Pieces& out) {
             if (uniform) {
 #pragma unroll
                 for (int c = 0; c < 2; ++c) {
@@ -184,10 +198,9 @@ __global__ __launch_bounds__(512, 4) void spmm_tile_kernel(const SpmmParams p) {
                     const bool touches = u + 8 > 0 && u < mine.cnt;
                     const int u_ld = risky ? min(max(u, -off), p.T - off - 8) : u;
                     const T* src_p = touches ? prow_p + u_ld : pb;  // (the buffer's first 16 bytes: any readable address)
-                    u32x4 raw;
-                    __builtin_memcpy(&raw, src_p, 16);  // any alignment
-                    if (u_ld != u) raw = shift_elements(raw, u_ld - u);
-                    out[c] = raw & s_mask[min(max(-u, 0), 8) * 9 + min(max(u + 8 - mine.cnt, 0), 8)];
+                    __builtin_memcpy(&out.raw[c], src_p, 16);  // any alignment
+                    out.moved[c] = u_ld - u;
+                    out.keep[c] = s_mask[min(max(-u, 0), 8) * 9 + min(max(u + 8 - mine.cnt, 0), 8)];
                 }
             } else {
                 typedef T vec8 __attribute__((ext_vector_type(8)));
@@ -197,7 +210,9 @@ __global__ __launch_bounds__(512, 4) void spmm_tile_kernel(const SpmmParams p) {
 #pragma unroll
                     for (int e = 0; e < 8; ++e) v[e] = (T)0.f;
                     if (mine.cnt > 0) v = gather_affine8<vec8>(prow_p, mine, s * kBN + 8 * (pq + 4 * c));
-                    out[c] = __builtin_bit_cast(u32x4, v);
+                    out.raw[c] = __builtin_bit_cast(u32x4, v);
+                    out.moved[c] = 0;
+                    out.keep[c] = u32x4{~0u, ~0u, ~0u, ~0u};
                 }
             }
         };
@@ -205,7 +220,7 @@ __global__ __launch_bounds__(512, 4) void spmm_tile_kernel(const SpmmParams p) {
         // ---- prologue: tile 0 into stage 0, tile 1 requested (everyone has left both stages at the barrier that ended the
         // segment before)
         u32x4 vreg[NI];
-        u32x4 praw[2];
+        Pieces praw;
         load_v(0, vreg);
         load_probs(0, praw);
         write_v(0, vreg);
