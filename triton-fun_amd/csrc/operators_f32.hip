@@ -170,7 +170,7 @@ __global__ __launch_bounds__(256, 4) void sddmm_f32_kernel(const SddmmParams p) 
 
 // out[bh, r, :] = sum over the live slots s of p[bh, r, s] * v[column of s, :].  O^T = V^T P^T: a lane reads its row's entries at 8 consecutive
 // positions straight from the compressed row, zeros where the row has none, and holds four consecutive columns of every 16.
-// NT: 16-column tiles of the output.
+// NT: 16-column tiles of the output that a workgroup takes.
 template <int NT>
 __global__ __launch_bounds__(256, 4) void spmm_f32_kernel(const SpmmParams p) {
     // 16 bytes of padding: rows 8 apart, which the lanes of one read touch, fall into different halves of the banks
@@ -186,8 +186,9 @@ __global__ __launch_bounds__(256, 4) void spmm_f32_kernel(const SpmmParams p) {
 
     const int logical = xcd_remap(blockIdx.x, gridDim.x);
     if (logical >= p.total) return;
-    const int bh = logical / p.n_row_blocks;
-    const int rb = p.n_row_blocks - 1 - logical % p.n_row_blocks;
+    const int col0 = logical % p.n_col_chunks * (16 * NT), block = logical / p.n_col_chunks;
+    const int bh = block / p.n_row_blocks;
+    const int rb = p.n_row_blocks - 1 - block % p.n_row_blocks;
     const int b = bh / p.H, h = bh % p.H;
     const int rs = p.row_stride, L = p.L;
     const int r0 = block_first_row(rb, kRows, rs);
@@ -227,7 +228,7 @@ __global__ __launch_bounds__(256, 4) void spmm_f32_kernel(const SpmmParams p) {
 #pragma unroll
             for (int i = 0; i < NP; ++i) {
                 const int key = min(max(pl.c0 + pl.cs * (tile * kTile + pc_row[i]), 0), p.n_keys - 1);
-                raw[i] = row_piece(vb + (int64_t)key * p.v_sl, pc_c[i], p.n_out, p.v_vec);
+                raw[i] = row_piece(vb + (int64_t)key * p.v_sl, col0 / 4 + pc_c[i], p.n_out, p.v_vec);
             }
         };
         load_tile(0);
@@ -235,19 +236,18 @@ __global__ __launch_bounds__(256, 4) void spmm_f32_kernel(const SpmmParams p) {
         const WaveSpan span = span_of_rows16(win, pl.uniform != 0);
         const float* const src = p_row + p.seg[sg].slot_offset;
         auto dead = [&](int j0) { return j0 + kTile <= span.lo_min || j0 >= span.hi_max; };
+        auto inside = [&](int j0) { return j0 >= span.lo_max && j0 + kTile <= span.hi_min; };
         f32x8 pr;
         auto load_probs = [&](int tile) {
             const int j0 = tile * kTile;
             if (dead(j0)) return;
             const int at = j0 + 8 * g - win.lo;
-            if (j0 >= span.lo_max && j0 + kTile <= span.hi_min) {
+            if (inside(j0)) {
                 __builtin_memcpy(&pr, src + at, 32);  // any alignment
             } else if (pl.uniform) {
                 const int last = max(win.cnt - 1, 0);
 #pragma unroll
-                for (int e = 0; e < 8; ++e) pr[e] = src[min(max(at + e, 0), last)];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) pr[e] = (unsigned)(at + e) < (unsigned)win.cnt ? pr[e] : 0.f;
+                for (int e = 0; e < 8; ++e) pr[e] = src[min(max(at + e, 0), last)];  // (what is not the row's goes when it is used)
             } else {
                 pr = gather_affine8<f32x8>(src, win, j0 + 8 * g);
             }
@@ -257,13 +257,18 @@ __global__ __launch_bounds__(256, 4) void spmm_f32_kernel(const SpmmParams p) {
         for (int tile = 0; tile < pl.n_tiles; ++tile) {
 #pragma unroll
             for (int i = 0; i < NP; ++i) lds_store128(pc_to[i] + stage, __builtin_bit_cast(u32x4, raw[i]));
-            const f32x8 now = pr;
+            f32x8 now = pr;
             lds_barrier();  // the tile is there, and everybody is done with the one before it, whose stage comes next
             if (tile + 1 < pl.n_tiles) {
                 load_tile(tile + 1);
                 load_probs(tile + 1);
             }
             if (!dead(tile * kTile)) {
+                if (pl.uniform && !inside(tile * kTile)) {
+                    const int at = tile * kTile + 8 * g - win.lo;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) now[e] = (unsigned)(at + e) < (unsigned)win.cnt ? now[e] : 0.f;
+                }
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     float vf[NT];
@@ -281,7 +286,7 @@ __global__ __launch_bounds__(256, 4) void spmm_f32_kernel(const SpmmParams p) {
         float* const orow = (float*)p.out + ((int64_t)bh * L + my_row) * p.n_out;
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            const int c = 16 * t + 4 * g;
+            const int c = col0 + 16 * t + 4 * g;
             if (p.out_vec && c + 4 <= p.n_out) {
                 *reinterpret_cast<f32x4*>(orow + c) = o[t];
             } else {
@@ -323,11 +328,19 @@ int launch_spmm_f32(const SpmmParams& p0, hipStream_t st) {
     p.n_row_blocks = count_row_blocks(p.L, kRows, p.row_stride);
     const int64_t blocks = (int64_t)p.B * p.H * p.n_row_blocks;
     if (blocks > 0x7ffffff0) return 0;
-    p.total = (int)blocks;
+    // Launches of few row blocks share the columns out as well: a wavefront's chain of matrix instructions, 32 cycles each, is what they wait
+    // for.  Times over those of one workgroup a row block, masks of 33 to 300 slots: 32 columns a workgroup, up to 3 workgroups a CU
+    // 0.48 to 0.98 (4 heads of 1024 rows, 300 slots, d = 128: 27.4 -> 13.1 us), at 4 0.84 to 1.07, above 0.95 to 1.48; 64 of 128 columns, up to
+    // 4 a CU 0.67 to 0.95, at 8 1.08 to 1.21.
+    const int tiles = (p.n_out + 15) / 16;
+    const int nt = tiles <= 2 || blocks * ((tiles + 1) / 2) <= 768 ? 2 : tiles <= 4 || (tiles > 6 && blocks * 2 <= 1024) ? 4 : tiles <= 6 ? 6 : 8;
+    p.n_col_chunks = (tiles + nt - 1) / nt;
+    if (blocks * p.n_col_chunks > 0x7ffffff0) return 0;
+    p.total = (int)(blocks * p.n_col_chunks);
     const int grid = ((p.total + 7) / 8) * 8;
-    if (p.n_out <= 32) spmm_f32_kernel<2><<<grid, 256, 0, st>>>(p);
-    else if (p.n_out <= 64) spmm_f32_kernel<4><<<grid, 256, 0, st>>>(p);
-    else if (p.n_out <= 96) spmm_f32_kernel<6><<<grid, 256, 0, st>>>(p);
+    if (nt == 2) spmm_f32_kernel<2><<<grid, 256, 0, st>>>(p);
+    else if (nt == 4) spmm_f32_kernel<4><<<grid, 256, 0, st>>>(p);
+    else if (nt == 6) spmm_f32_kernel<6><<<grid, 256, 0, st>>>(p);
     else spmm_f32_kernel<8><<<grid, 256, 0, st>>>(p);
     return 1;
 }
