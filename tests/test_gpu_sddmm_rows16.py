@@ -40,8 +40,8 @@ def test_scores(dev, name, d, layout, dtype):
         assert torch.all(got[..., ~lv] == SENTINEL)
 
 
-# 512 half row blocks of 64 (K along the keys), 256 (rows), 128 (rows of d > 96): one launch each side of the lines, two segments too
-@pytest.mark.parametrize("layout,heads", [("keys", 128), ("keys", 129), ("rows", 64), ("rows", 65), ("rows", 32), ("rows", 33), ("rows", 16), ("rows", 17)])
+# 4 half row blocks a head; 512 of them (K along the keys), 640 and, d > 96, 256 (rows, with the plan table): both sides of the lines, two segments too
+@pytest.mark.parametrize("layout,heads", [("keys", 128), ("keys", 129), ("rows", 64), ("rows", 65), ("rows", 160), ("rows", 161)])
 @pytest.mark.parametrize("two", [False, True])
 @pytest.mark.parametrize("d", [64, 128])
 def test_launch_sizes(dev, d, two, layout, heads):
