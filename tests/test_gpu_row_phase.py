@@ -46,3 +46,23 @@ def test_forward_and_gradients_of_odd_dilated_windows(dev, L, w, s, d, fused, dt
         got = [out.detach(), *torch.autograd.grad(out, (q, k, v), grad)]
     for a, b in zip(got, want):
         assert float((a.double().cpu() - b).norm() / b.norm()) <= tol
+
+
+def test_a_forward_without_a_plan_buffer_takes_masks_that_fit_only_ungrouped(dev):
+    """985 row blocks fill the library's own buffer; grouped by phase the mask would need 988."""
+    import _splat_hip as hip
+    from r_attention import attention_plan
+    from test_zz_no_alloc import forward_args
+    L, d = 985 * 128, 64
+    segs = A.create_acsr_segments([A.dilated_pattern(L, 9, 4)], 16, dev)
+    arr = hip.seg_array(segs.seg_args(), L)
+    assert arr[0].row_stride_hint == 4 and hip.lib().splat_attention_plan_bytes(arr, 1, L) > hip.STATIC_PLAN_BYTES
+    g = torch.Generator().manual_seed(3)
+    q, k, v = (torch.randn(1, 1, L, d, generator=g).half().to(dev) for _ in range(3))
+    got, want = torch.empty_like(q), torch.empty_like(q)
+    args = lambda out: forward_args(q, k.transpose(2, 3), v, out, arr, 1, d ** -0.5)
+    hip.check(hip.lib().splat_attention_fwd_noalloc(*args(got), hip.stream_ptr(dev)), "splat_attention_fwd_noalloc")
+    plan = attention_plan(segs, L, dev)
+    hip.check(hip.lib().splat_attention_fwd_planned(*args(want), plan.data_ptr(), plan.numel(), hip.stream_ptr(dev)), "splat_attention_fwd_planned")
+    # (float16 probabilities of the two walks are rounded against different references: 2^-11 each)
+    assert float((got.double() - want.double()).norm() / want.double().norm()) <= 1e-3

@@ -851,8 +851,15 @@ extern "C" int splat_attention_fwd_noalloc(const void* q, int64_t q_sb, int64_t 
     const char* who = "splat_attention_fwd_noalloc";
     if (!segs) return fail(SPLAT_E_NULL, "%s: null pointer argument", who);
     if (L <= 0 || L > (1 << 23)) return fail(SPLAT_E_SHAPE, "%s: need 0 < L <= 2^23 (got %d)", who, L);
-    const int64_t need = splat_attention_plan_bytes(segs, n_seg, L);
+    int64_t need = splat_attention_plan_bytes(segs, n_seg, L);
     if (need <= 0) return fail(SPLAT_E_SHAPE, "%s: no plan for n_seg=%d, L=%d", who, n_seg, L);
+    // (rows grouped by phase round the row blocks up to a multiple of the stride: a mask that fits only without the hint goes without)
+    splat_acsr_seg plain[SPLAT_MAX_SEGMENTS];
+    if (need > kStaticPlanBytes && common_row_stride(segs, n_seg) > 1) {
+        for (int k = 0; k < n_seg; ++k) plain[k] = segs[k], plain[k].row_stride_hint = 1;
+        segs = plain;
+        need = splat_attention_plan_bytes(segs, n_seg, L);
+    }
     if (need > kStaticPlanBytes)
         return fail(SPLAT_E_SHAPE,
                     "%s: this mask's plan needs %lld bytes, the built-in buffer holds %lld (about %lld row blocks of 128 rows "
