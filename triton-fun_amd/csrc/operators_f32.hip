@@ -304,8 +304,12 @@ int launch_sddmm_f32(const SddmmParams& p0, bool kt, hipStream_t st) {
     p.n_row_blocks = count_row_blocks(p.L, kRows, p.row_stride);
     const int64_t blocks = (int64_t)p.B * p.H * p.n_row_blocks;
     if (blocks > 0x7ffffff0) return 0;
-    // few row blocks: their tiles are shared out, as the general kernel does
-    p.key_split = blocks >= 1024 ? 1 : (int)std::min<int64_t>(32, (1024 + blocks - 1) / blocks);
+    // Few row blocks: their tiles are shared out over up to three workgroups a CU, to no more than there are tiles (every further one has
+    // the prologue and nothing to do).  Over 168 launches of 16 to 640 blocks 0.87 of the time that up to four and 32 a block take (4 heads
+    // of 1024 rows, two segments of 94 slots, d = 128 17.7 -> 10.6 us); from 512 blocks on two a block pay for short contractions of longer rows
+    // (129 and 300 slots: d = 32, 64 0.87 to 0.93 of one, d = 96, 128 1.01 to 1.17).
+    p.key_split = (int)std::min<int64_t>((p.T + kTile - 1) / kTile + 3, std::max<int64_t>(1, 768 / blocks));
+    if (p.key_split == 1 && blocks < 1024 && p.d <= 64 && p.T > 64) p.key_split = 2;
     p.total = (int)(blocks * p.key_split);
     const int grid = ((p.total + 7) / 8) * 8;
     auto go = [&](auto kq) {
