@@ -70,8 +70,8 @@ _HALF = (torch.float16, torch.bfloat16)
 def _takes_a_plan(x, output, blocks: int, d: int, k_rows: bool, T: int) -> bool:
     """Whether this launch runs the kernel that reads a plan table (the library decides by the same rules and ignores the
     plan otherwise, so that building one would be for nothing): 16-bit types, d up to 128 in whole 16-byte pieces, rows of K
-    contiguous (``k_rows``), and at least 256 row blocks or rows of at most 256 slots (fewer blocks of longer rows are better off
-    with the general kernel's split of the key range)."""
+    contiguous (``k_rows``), and at least 256 row blocks or rows of at most 256 slots (fewer blocks of longer rows go
+    to kernels that split the key range and plan for themselves where no table is handed over)."""
     return (k_rows and d % 8 == 0 and d <= 128 and (T <= 256 or blocks >= 256) and x.dtype in _HALF
             and output.dtype == x.dtype)
 

@@ -1,5 +1,5 @@
 // SDDMM on ACSR for the common fast shape: 16-bit inputs and outputs of one type, rows of Q and K contiguous in whole 16-byte
-// pieces, d at most 128, at least 256 row blocks in the launch or rows of at most 256 slots.  d = 64 and 128 with output rows
+// pieces, d at most 128, at least 256 row blocks in the launch or rows of at most 256 slots, beyond the launch sizes of sddmm_rows16.hip.  d = 64 and 128 with output rows
 // on 16-byte boundaries have instantiations of their own; the others (PART) pad the contraction to 64 or 128 in LDS.
 //
 // A workgroup of 8 wavefronts owns 128 rows of one (batch, head); wavefront w owns rows 16w..16w+15 and computes
@@ -420,8 +420,8 @@ int launch_sddmm_lines(const char* who, const SddmmParams& p, int in_dtype, hipS
     if (in_dtype == SPLAT_F32 || p.out_dtype != in_dtype) return 0;
     if (p.d % 8 != 0 || p.d > 128) return 0;
     if (p.k_sd != 1 || !p.q_vec || !p.k_vec) return 0;
-    // Few row blocks with long rows are better off with the general kernel, which splits a block's key range over several
-    // workgroups (64 blocks of 1024 slots: 0.021 against 0.029 ms; of 256 slots: 0.016 against 0.013).
+    // Few row blocks with long rows that sddmm_rows16.hip leaves are better off with the general kernel, which splits a block's key
+    // range over several workgroups too (64 blocks of 1024 slots: 0.021 against 0.029 ms; of 256 slots: 0.016 against 0.013).
     if ((int64_t)p.B * p.H * count_row_blocks(p.L, 128, p.row_stride) < 256 && p.T > 256) return 0;
     const bool part = (p.d != 64 && p.d != 128) || !p.out_vec;
     auto go = [&](auto t, auto probs_c, auto planned_c) {

@@ -1,4 +1,5 @@
-// Kernel arguments of the SDDMM kernels (sddmm.hip: every shape; sddmm_lines.hip: 16-bit types, d = 64 / 128).
+// Kernel arguments of the SDDMM kernels (sddmm.hip: every shape; sddmm_lines.hip, sddmm_rows16.hip: 16-bit types, operators_f32.hip: float32,
+// up to 128 inner values).
 #pragma once
 #include "acsr_plan.hpp"
 
