@@ -40,10 +40,10 @@ def test_scores(dev, name, d, layout, dtype):
         assert torch.all(got[..., ~lv] == SENTINEL)
 
 
-# 4 half row blocks a head; 512 of them (K along the keys), 640 and, d > 96, 256 (rows, with the plan table): both sides of the lines, two segments too
-@pytest.mark.parametrize("layout,heads", [("keys", 128), ("keys", 129), ("rows", 64), ("rows", 65), ("rows", 160), ("rows", 161)])
+# 4 half row blocks a head; 512 of them (K along the keys; 1024 where 64 < d <= 96), 640 and, d > 96, 256 (rows, with the plan table): both sides of the lines, two segments too
+@pytest.mark.parametrize("layout,heads", [("keys", 128), ("keys", 129), ("keys", 256), ("keys", 257), ("rows", 64), ("rows", 65), ("rows", 160), ("rows", 161)])
 @pytest.mark.parametrize("two", [False, True])
-@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("d", [64, 80, 128])
 def test_launch_sizes(dev, d, two, layout, heads):
     L = 250
     pats = A.strided_patterns(L, 40, 16) if two else [A.causal_windowed_pattern(L, 69)]

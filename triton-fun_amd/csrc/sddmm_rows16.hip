@@ -181,12 +181,12 @@ int launch_sddmm_rows16(const SddmmParams& p0, int in_dtype, bool kt, hipStream_
     p.n_row_blocks = count_row_blocks(p.L, kPlanBM, p.row_stride);
     const int64_t blocks = 2 * (int64_t)p.B * p.H * p.n_row_blocks;
     // The lines, as shares of the other kernels' time.  K along the keys, which the general kernel reads badly: 0.34 to 0.85 up to 512 blocks,
-    // 0.66 to 1.20 at 1024.  Rows of K with the plan table, masks of 33 to 129 slots: d <= 96 0.62 to 1.04 up to 640 blocks, 0.83 to 1.21 at 1024;
+    // at 1024 0.66 to 0.89 for d = 80 and rows of 33 to 129 slots, 0.82 to 1.20 for d = 128 or 300 slots.  Rows of K with the plan table, masks of 33 to 129 slots: d <= 96 0.62 to 1.04 up to 640 blocks, 0.83 to 1.21 at 1024;
     // d = 128 0.60 to 0.91 up to 256, 0.84 to 1.07 from 384 to 640; 300 slots 0.43 to 0.97 up to 512, 0.82 to 1.03 at 640.  Without the
     // table the prologue is longer, and once more for every segment: d <= 96 0.42 to 0.98 at 256 blocks, 0.84 to 1.08 at 512, d = 128 0.65 to 1.01
     // at 128, 0.89 to 1.03 at 256; two segments 0.90 to 0.99 at half of that, 1.01 to 1.06 there.
     const bool wide = p.d > 96 && p.T <= 256;
-    const int most = kt ? 512 : p.plan ? (wide ? 256 : p.T <= 256 ? 640 : 512) : (wide ? 128 : 256) / p.n_seg;
+    const int most = kt ? (p.d > 64 && p.d <= 96 && p.T <= 256 ? 1024 : 512) : p.plan ? (wide ? 256 : p.T <= 256 ? 640 : 512) : (wide ? 128 : 256) / p.n_seg;
     if (blocks > most) return 0;
     p.key_split = (int)std::min<int64_t>((p.T + kTile - 1) / kTile + 2, std::max<int64_t>(1, 512 / blocks));
     p.total = (int)(blocks * p.key_split);
