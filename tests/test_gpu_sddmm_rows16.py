@@ -40,8 +40,8 @@ def test_scores(dev, name, d, layout, dtype):
         assert torch.all(got[..., ~lv] == SENTINEL)
 
 
-# 4 half row blocks a head; 512 of them (K along the keys; 1024 where 64 < d <= 96), 640 and, d > 96, 256 (rows, with the plan table): both sides of the lines, two segments too
-@pytest.mark.parametrize("layout,heads", [("keys", 128), ("keys", 129), ("keys", 256), ("keys", 257), ("rows", 64), ("rows", 65), ("rows", 160), ("rows", 161)])
+# 4 half row blocks a head; 512 of them (K along the keys; 1024 where 64 < d <= 96), 640 and, d > 96, 256 (rows, with the plan table), 1024 to 4096 (the same, 70 or 55 slots): both sides of the lines, two segments too
+@pytest.mark.parametrize("layout,heads", [("keys", 128), ("keys", 129), ("keys", 256), ("keys", 257), ("rows", 64), ("rows", 65), ("rows", 160), ("rows", 161), ("rows", 256), ("rows", 257), ("rows", 1024), ("rows", 1025)])
 @pytest.mark.parametrize("two", [False, True])
 @pytest.mark.parametrize("d", [64, 80, 128])
 def test_launch_sizes(dev, d, two, layout, heads):
@@ -57,3 +57,15 @@ def test_launch_sizes(dev, d, two, layout, heads):
     masks = O.create_strided_segment_masks(L, 40, 16) if two else [O.create_causal_windowed_mask(L, 69)]
     want = torch.cat([O.compress(dense, O.create_acsr(m, 16), first_col=O.row_extents(m)[0], fill=SENTINEL) for m in masks], -1)
     assert torch.equal(out.float().cpu(), want)
+
+
+@pytest.mark.parametrize("width", [17, 40, 41])
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_short_rows_in_launches_that_fill_the_chip(dev, d, width):
+    L, heads = 250, 300
+    acsr, acsr_np = acsr_pair(O.create_causal_windowed_mask(L, width - 1), 16, dev)
+    q, k = signs((1, heads, L, d), heads, torch.float16), signs((1, heads, L, d), d, torch.float16)
+    out = torch.full((1, heads, L, acsr[5]), SENTINEL, dtype=torch.float16, device=dev)
+    r_sddmm.rsddmm_launcher(q.to(dev), k.to(dev).transpose(2, 3), out, acsr[0], acsr[1], acsr[2], acsr[3], acsr[5], acsr[4], (1, 1), None, None, 16, 16)
+    want, lv, got = O.sddmm(q.float(), k.float().transpose(2, 3), acsr_np, first_col=[0] * L), live(acsr_np), out.float().cpu()
+    assert torch.equal(got[..., lv], want[..., lv]) and torch.all(got[..., ~lv] == SENTINEL)

@@ -1,5 +1,6 @@
 // SDDMM on ACSR for the common fast shape: 16-bit inputs and outputs of one type, rows of Q and K contiguous in whole 16-byte
-// pieces, d at most 128, at least 256 row blocks in the launch or rows of at most 256 slots, beyond the launch sizes of sddmm_rows16.hip.  d = 64 and 128 with output rows
+// pieces, d at most 128, at least 256 row blocks in the launch or rows of at most 256 slots, where sddmm_rows16.hip does not
+// take the launch.  d = 64 and 128 with output rows
 // on 16-byte boundaries have instantiations of their own; the others (PART) pad the contraction to 64 or 128 in LDS.
 //
 // A workgroup of 8 wavefronts owns 128 rows of one (batch, head); wavefront w owns rows 16w..16w+15 and computes

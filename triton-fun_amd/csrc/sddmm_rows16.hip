@@ -1,4 +1,4 @@
-// SDDMM on ACSR of 16-bit operands in launches of few row blocks, inner dimension up to 128.
+// SDDMM on ACSR of 16-bit operands in launches of few row blocks, and of short rows in larger ones, inner dimension up to 128.
 //
 // Such a launch is one chain of latencies a workgroup, row maps -> plan -> tile -> products -> stores, and what shortens it is
 // little work a workgroup: 64 rows of one (batch, head) in 4 wavefronts of 16, tiles of 64 positions requested a tile ahead through
@@ -187,7 +187,13 @@ int launch_sddmm_rows16(const SddmmParams& p0, int in_dtype, bool kt, hipStream_
     // at 128, 0.89 to 1.03 at 256; two segments 0.90 to 0.99 at half of that, 1.01 to 1.06 there.
     const bool wide = p.d > 96 && p.T <= 256;
     const int most = kt ? (p.d > 64 && p.d <= 96 && p.T <= 256 ? 1024 : 512) : p.plan ? (wide ? 256 : p.T <= 256 ? 640 : 512) : (wide ? 128 : 256) / p.n_seg;
-    if (blocks > most) return 0;
+    // And with the table, launches that fill the chip, rows of K: rows of at most 40 slots at 0.70 to 0.95 (one of 40 launches 1.03) up to 16384
+    // blocks; longer ones that are no whole 64-byte pieces, which the line-wise kernel stores in most, from where that has more than its one
+    // round of workgroups (at 1024 blocks 0.83 to 1.10) to 4096: d <= 32 0.57 to 0.95, d = 64 from 129 slots on 0.63 to 0.99, d = 80 to 128 up
+    // to 240 slots 0.55 to 0.96 (whole pieces, 128 slots, 1.05 to 1.32; 251 slots at d = 128 1.06 to 1.12).
+    const bool ragged = p.T % 32 != 0 && p.T <= (p.d > 64 ? 240 : 255) && (p.d <= 32 || p.d > 64 || p.T >= 120);
+    const bool fills = !kt && p.plan && (p.T <= 40 ? blocks <= 16384 : ragged && blocks > 1024 && blocks <= 4096);
+    if (blocks > most && !fills) return 0;
     p.key_split = (int)std::min<int64_t>((p.T + kTile - 1) / kTile + 2, std::max<int64_t>(1, 512 / blocks));
     p.total = (int)(blocks * p.key_split);
     const int grid = ((p.total + 7) / 8) * 8;
