@@ -246,6 +246,23 @@ def test_mask_tensors_of_any_pitch_in_one_kernel(dev, rows, cols, pitch, offset,
     check_acsr(mask, BH, dev)
 
 
+@pytest.mark.parametrize("rows,cols,pitch,offset", [(40, 12288, 12288, 0), (40, 12289, 12289, 1), (33, 16384, 16400, 7), (70, 20011, 20011, 0)])
+def test_rows_around_the_length_that_keeps_more_pieces_in_flight(dev, rows, cols, pitch, offset):
+    """The build that leaves its summary on the device, against the one that is waited for (held to the oracle above)."""
+    g = torch.Generator().manual_seed(cols)
+    flat = torch.zeros(offset + rows * pitch, dtype=torch.uint8, device=dev)
+    mask = flat[offset:].view(rows, pitch)[:, :cols]
+    mask.copy_(torch.rand(rows, cols, generator=g) < 0.3)
+    mask[: rows // 2, : cols - 20] = 0  # first columns in the last pieces
+    want = check_acsr(mask, 16, dev)
+    first, last = A.row_extents(mask, dev)
+    got = A.build_acsr(mask.clone(), 16, torch.device(dev))
+    for name, w in zip(("dTos_lin", "dTos_trans", "sTod_lin", "sTod_trans", "nnz", "T", "span_start", "span_end"), want):
+        assert got.T == w if name == "T" else np.array_equal(bits(getattr(got, name)), bits(w)), name
+    assert torch.equal(got.row_first.cpu(), first.cpu()) and torch.equal(got.row_last.cpu(), last.cpu())
+    assert int(got.row_stride) == int(want[3].splat_row_stride) and int(got.max_step) == int(want[3].splat_max_step)
+
+
 @pytest.mark.parametrize("BH", [1, 15, 63, 65, 200])
 def test_rows_solved_together_and_bytes_beyond_one(dev, BH):
     """Row blocks around the 64 rows that are solved at once; the first two ones at every place of a 16-byte piece and in

@@ -174,7 +174,7 @@ struct BlockFold {
 };
 
 // A workgroup takes `per_block` consecutive rows, a wavefront one row at a time: 16-byte pieces from the row's first aligned
-// address on (rows of any pitch), four per lane in flight, and single bytes at the two ends.  Sixteen wavefronts and at most
+// address on (rows of any pitch), NB per lane in flight, and single bytes at the two ends.  Sixteen wavefronts and at most
 // 64 registers, so that a CU holds two workgroups: a mask of 8192 rows is one wave of workgroups over the chip.  What a
 // wavefront found goes to LDS; the first one solves up to 64 rows at once, a lane each, and stores them side by side.
 //
@@ -182,11 +182,15 @@ struct BlockFold {
 // that the host reads) come from the same kernel.  With a second kernel for the spans, which walks 16 rows a thread with
 // few threads, and the summary read back through a copy, an 8192 x 8192 mask took 23 us on the GPU in two kernels and 95 us
 // for the whole call.  One kernel in which every wavefront's first lane solved its row and the workgroup's first thread
-// folded the wavefronts' one by one: 16.6 us, 36.1 for the call.  This one, whose pieces are read without a branch per dword:
-// 12.4 us with eight pieces in flight and about 10.7 with four, which need less code and no spills (two pieces + 1.3 us,
-// 8 wavefronts + 0.2, 4 wavefronts + 2.7); 30.7 for the call: the 67 MB at the rate of a large copy.
+// folded the wavefronts' one by one: 17.4 us.  This one, whose pieces are read without a branch per dword: 12.7 us with
+// four pieces in flight and 15.1 with eight, whose code and spills (with the fold) cost more than they hide; the 67 MB of that mask come
+// from the last-level cache, with caches flushed it takes 16.3 (23.7 before, 21.3 with eight).
+// Rows of 16384 bytes, 268 MB, bound by HBM: with the fold four pieces 49.7 / 52.5 flushed, eight 50.3 / 55.0; without the fold and its
+// registers (splat_acsr_build, both kernels) eight do not spill, and win where the cache does not hold the mask: 55.1 / 57.4
+// against 59.5 / 62.6, at rows of 12288 bytes 35.5 / 37.8 against 35.2 / 37.9, of 8192 23.3 / 26.5 against 22.7 / 26.3.
 constexpr int kRowWaves = 16;
-template <bool FOLD>
+constexpr int kLongRow = 12288;  // bytes a row from which on eight pieces are in flight, without FOLD
+template <bool FOLD, int NB = 4>
 __global__ __launch_bounds__(64 * kRowWaves, 8) void acsr_rows_kernel(const uint8_t* __restrict__ mask, int rows, int cols, int64_t ld,
                                                                       int per_block, RowOut o, int32_t* __restrict__ summary,
                                                                       int32_t* __restrict__ shares) {
@@ -196,7 +200,6 @@ __global__ __launch_bounds__(64 * kRowWaves, 8) void acsr_rows_kernel(const uint
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n_waves = blockDim.x >> 6;
     const int r_end = min(rows, ((int)blockIdx.x + 1) * per_block);
-    constexpr int NB = 4;
     BlockFold f;
     f.init(cols);
     int turn = 0;
@@ -462,8 +465,8 @@ extern "C" int splat_acsr_build(const uint8_t* mask, int64_t rows, int64_t cols,
         return fail(SPLAT_E_SHAPE, "splat_acsr_build: rows and cols are limited to 2^23 (got %lld, %lld)", (long long)rows, (long long)cols);
     hipStream_t st = (hipStream_t)stream;
     const RowOut out{dTos_lin, dTos_trans, sTod_lin, sTod_trans, nnz, row_first, row_last, nullptr, nullptr, 0, 0};
-    acsr_rows_kernel<false><<<(unsigned)((rows + kRowWaves - 1) / kRowWaves), 64 * kRowWaves, 0, st>>>(mask, (int)rows, (int)cols, ld,
-                                                                                                      kRowWaves, out, summary, nullptr);
+    const auto kern = cols > kLongRow ? acsr_rows_kernel<false, 8> : acsr_rows_kernel<false>;
+    kern<<<(unsigned)((rows + kRowWaves - 1) / kRowWaves), 64 * kRowWaves, 0, st>>>(mask, (int)rows, (int)cols, ld, kRowWaves, out, summary, nullptr);
     const int n_blocks = (int)((rows + block_height - 1) / block_height);
     acsr_spans_kernel<<<(n_blocks + 255) / 256, 256, 0, st>>>(sTod_lin, sTod_trans, nnz, (int)rows, (int)cols, block_height,
                                                                span_start, span_end, summary);
