@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import acsr_helpers as A
-from r_attention import RegularAttention, attention_with_grad
+from r_attention import RegularAttention, attention_launcher, attention_with_grad
 
 pytestmark = pytest.mark.gpu
 
@@ -46,6 +46,33 @@ def test_forward_and_gradients_against_float64(dev, name, L, d):
     for a, b in zip(torch.autograd.grad(out, on, go.to(dev)), grads):
         b = torch.nan_to_num(b)
         assert float((a.cpu() - b).abs().max()) <= 2e-5 * max(1.0, float(b.abs().max()))
+
+
+# windows that start at, before and behind the middle of a tile of the row block's walk, and save the workgroup's own one or not
+STARTS = {"16 to both sides": lambda L: [A.windowed_pattern(L, 16)], "17": lambda L: [A.windowed_pattern(L, 17)],
+          "3": lambda L: [A.windowed_pattern(L, 3)], "40": lambda L: [A.windowed_pattern(L, 40)],
+          "gathered": lambda L: [A.dilated_pattern(L, 17, 2)], "residue": lambda L: [A.dilated_pattern(L, 21, 3)],
+          "two segments": lambda L: A.strided_patterns(L, 20, 18), "steps on dense columns": lambda L: A.strided_patterns(L, 30, 7)[1:]}
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("L", [130, 515])
+@pytest.mark.parametrize("name", STARTS)
+def test_walks_that_start_inside_a_tile(dev, name, L, d):
+    masks, B, H = STARTS[name](L), 1, 2
+    g = torch.Generator().manual_seed(L + d)
+    q, k, v = (torch.randn(B, H, L, d, generator=g) for _ in range(3))
+    live = sum(m.device_mask(dev) for m in masks).cpu() > 0
+    s = (q.double() @ k.double().transpose(2, 3) * d ** -0.5).masked_fill(~live, float("-inf"))
+    want = torch.where(live.any(1)[:, None], torch.softmax(s, -1), torch.zeros_like(s)) @ v.double()
+    attn = RegularAttention(B, L, H, d, masks, 16, 16, dev, torch.float32, scale=d ** -0.5)
+    on = [t.to(dev) for t in (q, k, v)]
+    got = attn([on[0], on[1].transpose(2, 3), on[2]]).clone()
+    assert float((got.cpu() - want).abs().max()) <= 1e-5
+    assert torch.equal(attn([on[0], on[1].transpose(2, 3).contiguous(), on[2]]), got)
+    out = torch.empty_like(got)  # without a plan table
+    attention_launcher(on[0], on[1].transpose(2, 3), on[2], out, attn.segments, d ** -0.5)
+    assert torch.equal(out, got)
 
 
 @pytest.mark.parametrize("d", [64, 128])

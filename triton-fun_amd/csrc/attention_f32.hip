@@ -24,6 +24,17 @@
 
 namespace splat {
 
+// The walk of a workgroup's own 64 rows.  It starts `at0` positions into the row block's (the plan's c0 moves along; the windows in the
+// plan table are relative to the row block's): at the row block's tile that holds the first position that one of the rows sees, or,
+// where that saves a tile, at that position, as for windows to both sides, which start in the middle of a tile (d = 128, window 33,
+// 4 heads of 512 rows 12.4 -> 10.6 us, 64 of 2048 66.8 -> 57.6; the kernel on the float32 instructions, which skipped positions 16 at a
+// time, took 12.0 for the former).  Dense walks start at a multiple of 16, and only there, since K stored along the keys is
+// read in runs of 32 keys: causal windows of 8 to 128, from wherever they start, took 2 to 3 % longer with it at 64 heads of 2048.
+struct OwnWalk {
+    int seg, tile, end, at0;
+    SegPlan pl;
+};
+
 template <int D, bool KT, bool PLANNED>
 __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_fwd_f32_kernel(const AttnParams p) {
     constexpr int BN = 32, ROWB = 2 * D, PLANE = BN * ROWB, TILE = 3 * PLANE;  // positions a tile; bytes of a row, a plane, an operand
@@ -71,35 +82,47 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_fwd_f32_kernel(cons
     const int n_rb = p.n_row_blocks;
     if constexpr (!PLANNED) plan_segments<kPlanBM, kBN>(p.seg, p.n_seg, block_first_row(rb, kPlanBM, rs), rs, L, true, s_plan, &s_ps, tid);
     auto walk_of = [&](int sg) {
-        HalfWalk w;
+        OwnWalk w;
         w.seg = sg;
+        int lo, hi;
         if constexpr (PLANNED) {
-            w = half_walk<BN>(pt, n_rb, p.n_seg, rb, half, sg);
+            const PlanRec r = plan_uniform_load(pt + plan_seg_at(p.n_seg, rb, sg));
+            w.pl.c0 = r.x, w.pl.cs = r.y, w.pl.n_tiles = r.z, w.pl.uniform = r.w;
+            const PlanRec s0 = plan_uniform_load(pt + plan_span_at(n_rb, p.n_seg, rb, sg, 2 * half));
+            const PlanRec s1 = plan_uniform_load(pt + plan_span_at(n_rb, p.n_seg, rb, sg, 2 * half + 1));
+            lo = min(s0.x, s1.x), hi = max(s0.w, s1.w);
         } else {
             const SegPlan l = s_plan[sg];
             w.pl.c0 = __builtin_amdgcn_readfirstlane(l.c0);
             w.pl.cs = __builtin_amdgcn_readfirstlane(l.cs);
             w.pl.n_tiles = __builtin_amdgcn_readfirstlane(l.n_tiles);
             w.pl.uniform = __builtin_amdgcn_readfirstlane(l.uniform);
-            w.tile = 0, w.end = w.pl.n_tiles * (kBN / BN);
+            const RowWin win = make_row_win(cached_row_map<kPlanBM>(&s_ps, sg, k0 + lane), w.pl);
+            lo = __builtin_amdgcn_readfirstlane(wave_min_i(win.cnt > 0 ? win.lo : 0x3fffffff));
+            hi = __builtin_amdgcn_readfirstlane(wave_max_i(win.cnt > 0 ? win.lo + win.cnt : 0));
+        }
+        hi = min(hi, w.pl.n_tiles * kBN);
+        w.at0 = 0, w.tile = 0, w.end = 0;
+        if (lo < hi) {
+            const int tiled = max(lo, 0) & ~(BN - 1), own = max(lo, 0) & (w.pl.cs == 1 ? ~15 : ~0);
+            w.end = (hi - own + BN - 1) / BN;
+            w.at0 = (hi - tiled + BN - 1) / BN > w.end ? own : tiled;
+            w.pl.c0 += w.pl.cs * w.at0;
         }
         return w;
     };
-    auto next_segment = [&](HalfWalk& w) {  // the first segment from w.seg on that has tiles
+    auto next_segment = [&](OwnWalk& w) {  // the first segment from w.seg on that has tiles
         for (int sg = w.seg; sg < p.n_seg; ++sg) {
             w = walk_of(sg);
             if (w.end > w.tile) return;
         }
         w.seg = p.n_seg, w.tile = 0, w.end = 0x7fffffff;
     };
-    HalfWalk fetch;
+    OwnWalk fetch;
     fetch.seg = 0;
     next_segment(fetch);
     int total = fetch.end - fetch.tile;
-    for (int sg = fetch.seg + 1; sg < p.n_seg; ++sg) {
-        const HalfWalk w = walk_of(sg);
-        total += w.end - w.tile;
-    }
+    for (int sg = fetch.seg + 1; sg < p.n_seg; ++sg) total += walk_of(sg).end;
     total = fetch.seg < p.n_seg ? __builtin_amdgcn_readfirstlane(total) : 0;
 
     // ---- a tile's way into LDS: pieces of 8 values, by their position in the tile's rows.  K stored along the keys is turned here:
@@ -121,7 +144,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_fwd_f32_kernel(cons
     // an operand of one head within 32-bit offsets, and strides that 24-bit products take
     const int64_t k_far = KT ? p.k_sd * D + L : p.k_sl * L, v_far = p.v_sl * L;
     const bool narrow = max(k_far, v_far) * 4 < ((int64_t)1 << 32) && max(KT ? p.k_sd : p.k_sl, p.v_sl) * 4 < (1 << 24) && p.k_sd >= 0;
-    auto load_next = [&](HalfWalk& w) {  // the tile the walk stands at, which moves on
+    auto load_next = [&](OwnWalk& w) {  // the tile the walk stands at, which moves on
         const int c0 = w.pl.c0 + w.pl.cs * w.tile * BN;
 #pragma unroll
         for (int i = 0; i < NP; ++i) {
@@ -162,7 +185,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_fwd_f32_kernel(cons
         v_addr[dt] = smem_base + TILE + (4 * g + tr_row) * ROWB + (dt ^ swz32<ROWB>(4 * g + tr_row)) * 32 + tr_byte;
 
     // the row windows of the first segment with tiles, then the first tile, are requested before Q is looked at
-    HalfWalk cur = fetch;
+    OwnWalk cur = fetch;
     PlanRec win_rec = {0, 0, 1, 0};
     if constexpr (PLANNED) {
         if (total > 0) win_rec = pt[plan_row_at(n_rb, p.n_seg, rb, cur.seg, k0 + wave * 16 + n)];
@@ -192,7 +215,11 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_fwd_f32_kernel(cons
             int phase;
             if constexpr (PLANNED) {
                 if (it > 0) win_rec = pt[plan_row_at(n_rb, p.n_seg, rb, cur.seg, k0 + wave * 16 + n)];
-                w.lo = win_rec.x, w.cnt = win_rec.y, w.lin = win_rec.z, phase = win_rec.w;
+                w.lo = win_rec.x - cur.at0, w.cnt = win_rec.y, w.lin = win_rec.z, phase = win_rec.w;
+                if (!cur.pl.uniform) {
+                    phase -= cur.at0 % w.lin;
+                    if (phase < 0) phase += w.lin;
+                }
             } else {
                 w = make_row_win(cached_row_map<kPlanBM>(&s_ps, cur.seg, k0 + wave * 16 + n), cur.pl);
                 phase = cur.pl.uniform ? 0 : win_phase(w);
@@ -305,15 +332,15 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_fwd_f32_kernel(cons
         for (int i = 0; i < QD; ++i) q[i] = qr[i], acc[i] = 0.f;
         float m = -__builtin_inff(), l = 0.f;
         for (int sg = 0; sg < p.n_seg; ++sg) {
-            const HalfWalk w = walk_of(sg);
+            const OwnWalk w = walk_of(sg);
             RowWin win;
             if constexpr (PLANNED) {
                 const PlanRec wr = pt[plan_row_at(n_rb, p.n_seg, rb, sg, k0 + wave * 16 + n)];
-                win.lo = wr.x, win.cnt = wr.y, win.lin = wr.z;
+                win.lo = wr.x - w.at0, win.cnt = wr.y, win.lin = wr.z;
             } else {
                 win = make_row_win(cached_row_map<kPlanBM>(&s_ps, sg, k0 + wave * 16 + n), w.pl);
             }
-            for (int j = w.tile * BN; j < w.end * BN; ++j) {
+            for (int j = 0; j < w.end * BN; ++j) {
                 const bool live = win_live(win, j);
                 if (!__any(live)) continue;
                 const int64_t key = min(max(w.pl.c0 + w.pl.cs * j, 0), L - 1);
