@@ -111,3 +111,50 @@ def test_gradients_that_are_not_finite_stay_where_they_belong(dev, d):
     assert torch.allclose(got[0][0, 1, ~sees], clean[0][0, 1, ~sees], rtol=0, atol=1e-5)
     for i in (1, 2) if d == 64 else ():  # (at d = 128 dK and dV are float32 products, where 0 * inf of a tile's masked positions is NaN)
         assert torch.allclose(got[i][0, 0, ~seen], clean[i][0, 0, ~seen], rtol=0, atol=1e-5)
+
+
+def small(at):
+    """Column 5 of one operand far below the others."""
+    def change(*x):
+        x[at][..., 5] *= 1e-36
+    return change
+
+
+def column_error(got, want):
+    return float((got[..., 5].double().cpu() - want[..., 5]).norm() / want[..., 5].norm())
+
+
+# what the kernel splits itself, dS, is small where dO and V are so together, and Q or K may make up for it.  (The bounds here are those of
+# test_gradients_at_scales_of_the_operands: nothing below is smaller than float32's normal values.)
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("q,k,v,g", [(1, 1, 1e-16, 1e-17), (1, 1, 1e-17, 1e-17), (1e-20, 1e20, 1e-17, 1e-18), (1e20, 1e-20, 1e-18, 1e-17), (1, 1, 1e-19, 1e-17)])
+def test_gradients_of_small_inner_values(dev, d, q, k, v, g):
+    got, want, _ = gradients(dev, d, 211, q, k, v, g)
+    for a, b in zip(got, want):
+        if float(b.abs().max()) > 1e-36:
+            assert error(a, b) <= 3e-6
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("operand,gradient", [(1, 0), (0, 1), (3, 2)])  # K and dQ, Q and dK, dO and dV
+def test_gradients_of_a_small_column(dev, d, operand, gradient):
+    got, want, _ = gradients(dev, d, 211, 1, 1, 1, 1, change=small(operand))
+    assert column_error(got[gradient], want[gradient]) <= 3e-6
+
+
+def unlikely_key(q, k, *_):
+    """Key 30 scores -80 with every row: probabilities of about 2^-122.  The rounding of such a score, 2^-25 of it a term or so, is one of its
+    probability 80 times as large: 2e-5 is four times that."""
+    q[..., 0] = 8.0
+    k[..., 0] = 0.0
+    k[..., 30, :] = 0.0
+    k[..., 30, 0] = -80.0 / 8.0 * q.shape[-1] ** 0.5
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_gradients_of_an_unlikely_key(dev, d):
+    got, want, _ = gradients(dev, d, 211, 1, 1, 1, 1, change=unlikely_key)
+    for i in (1, 2):
+        a, b = got[i][:, :, 30].double().cpu(), want[i][:, :, 30]
+        assert float(b.abs().max()) > 1e-37
+        assert float((a - b).norm() / b.norm()) <= 2e-5

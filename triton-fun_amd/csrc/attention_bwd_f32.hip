@@ -161,7 +161,6 @@ __global__ __launch_bounds__(256, D == 64 && !KEYS ? 3 : 2) void attn_bwd_f32_ke
     }
     if constexpr (!KEYS) row_delta = over_groups(row_delta, [](float x, float y) { return x + y; });  // D = rowsum(dO * O)
     bool beyond = out_of_split(a_most) || out_of_split(b_most);  // something that the split operands do not hold
-    float x_most = 0.f, y_most = 0.f;                            // of the thread's pieces of the tiles
 
     f32x4 acc[DT], acc2[KEYS ? DT : 1];
 #pragma unroll
@@ -169,7 +168,9 @@ __global__ __launch_bounds__(256, D == 64 && !KEYS ? 3 : 2) void attn_bwd_f32_ke
         acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
         if constexpr (KEYS) acc2[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    const float c2 = p.scale_log2e;
+    // X and Y are lifted, and with them S, dP and dS, so that what the kernel itself splits holds its parts as well: dS is small where
+    // dO and V are so together.  P is lifted for its product with Y; the results are so twice.
+    const float c2 = p.scale_log2e * (1.f / kSplitLift), lift_delta = row_delta * kSplitLift;
     RowState rows;
     bool entered = false;
 
@@ -184,15 +185,12 @@ __global__ __launch_bounds__(256, D == 64 && !KEYS ? 3 : 2) void attn_bwd_f32_ke
         lds_barrier();  // everybody is done with tile it - 1
 #pragma unroll
         for (int i = 0; i < NP; ++i) {
-            const Split3 s = split3(raw[i]);
+            const Split3 s = split3(raw[i] * kSplitLift);
 #pragma unroll
             for (int k = 0; k < 3; ++k) lds_store128(pc_to[i] + k * PLANE, __builtin_bit_cast(u32x4, s.p[k].v));
-            float& most = i < NP / 2 ? x_most : y_most;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) most = fmaxf(most, fabsf(raw[i][e]));
         }
         if constexpr (KEYS) {
-            if (wave == 0) reinterpret_cast<float*>(smem + STATS)[lane] = raw_stat;
+            if (wave == 0) reinterpret_cast<float*>(smem + STATS)[lane] = lane < BN ? raw_stat : raw_stat * kSplitLift;
         }
         if (it + 1 < total) load_next(fetch);
         lds_barrier();  // tile `it` is there
@@ -229,7 +227,7 @@ __global__ __launch_bounds__(256, D == 64 && !KEYS ? 3 : 2) void attn_bwd_f32_ke
                 __builtin_amdgcn_sched_barrier(0);
             }
             // ---- P = exp2(S * scale * log2e - lse * log2e); masked scores underflow to exactly 0.  dS = P (dP - D) ----
-            if (!(j0 >= rows.lo_max && j0 + BN <= rows.hi_min)) rows.mask_tile(s, j0, g, cur.pl.uniform != 0);
+            if (!(j0 >= rows.lo_max && j0 + BN <= rows.hi_min)) rows.mask_tile(s, j0, g, cur.pl.uniform != 0, kNegBigA * kSplitLift);
             Frag<bf16> cf[2][3];
             auto load_cf = [&](int operand, int x) {
                 const int d2 = x / 3, k = 2 - x % 3;
@@ -251,7 +249,7 @@ __global__ __launch_bounds__(256, D == 64 && !KEYS ? 3 : 2) void attn_bwd_f32_ke
                 for (int j = 0; j < 4; ++j) {
                     const int e = 4 * u + j;
                     pr[e] = fast_exp2(fmaf(s[u][j], c2, KEYS ? -kLog2e * lse4[j] : -row_lse2));
-                    dsv[e] = pr[e] * (ds[u][j] - (KEYS ? del4[j] : row_delta));
+                    dsv[e] = pr[e] * (ds[u][j] - (KEYS ? del4[j] : lift_delta));
                 }
             }
             // ---- acc2^T += Y^T P^T, acc^T += X^T dS^T, of two tiles of 16 columns at a time ----
@@ -268,7 +266,7 @@ __global__ __launch_bounds__(256, D == 64 && !KEYS ? 3 : 2) void attn_bwd_f32_ke
                     __builtin_amdgcn_sched_barrier(0);
                 }
             };
-            if constexpr (KEYS) accumulate(acc2, 1, pr);
+            if constexpr (KEYS) accumulate(acc2, 1, pr * kSplitLift);
             accumulate(acc, 0, dsv);
         }
         if (!cur.pl.uniform) rows.next_tile();
@@ -279,8 +277,7 @@ __global__ __launch_bounds__(256, D == 64 && !KEYS ? 3 : 2) void attn_bwd_f32_ke
         }
     }
 
-    // What is not finite anywhere stays so in a row's results (NaN compares unequal).  Operands of the tiles that are all far below
-    // normal matter to results of their own size, whatever those are multiplied with.
+    // What is not finite anywhere, the lift's overflow included, stays so in a row's results (NaN compares unequal).
     float chk = 0.f;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
@@ -289,8 +286,7 @@ __global__ __launch_bounds__(256, D == 64 && !KEYS ? 3 : 2) void attn_bwd_f32_ke
             chk = fmaf(acc[dt][j], 0.f, chk);
             if constexpr (KEYS) chk = fmaf(acc2[dt][j], 0.f, chk);
         }
-    auto all_tiny = [](float most) { return __any(most > 0.f) && !__any(most >= 0x1p-96f); };
-    beyond |= chk != 0.f || all_tiny(x_most) || all_tiny(y_most);
+    beyond |= chk != 0.f;
     auto out_at = [&](void* base) { return (float*)base + b * p.o_sb + h * p.o_sh + (int64_t)out_row * p.o_sl; };
     if constexpr (!KEYS) {
         if (out_row < Lr && g == 0) p.delta_w[(int64_t)bh * L + out_row] = row_delta;
@@ -320,7 +316,7 @@ __global__ __launch_bounds__(256, D == 64 && !KEYS ? 3 : 2) void attn_bwd_f32_ke
                 s = over_groups(s, [](float x, float y) { return x + y; });
                 dp = over_groups(dp, [](float x, float y) { return x + y; });
                 if (live) {
-                    const float e = fast_exp2(fmaf(s, c2, KEYS ? -kLog2e * lse_b[pos] : -row_lse2));
+                    const float e = fast_exp2(fmaf(s, p.scale_log2e, KEYS ? -kLog2e * lse_b[pos] : -row_lse2));
                     const float d = e * (dp - (KEYS ? del_b[pos] : row_delta));
 #pragma unroll
                     for (int i = 0; i < QD; ++i) {
@@ -344,8 +340,8 @@ __global__ __launch_bounds__(256, D == 64 && !KEYS ? 3 : 2) void attn_bwd_f32_ke
     if (out_row < Lr) {
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
-            *reinterpret_cast<f32x4*>(out_at(p.out) + 16 * dt + 4 * g) = acc[dt] * p.scale;
-            if constexpr (KEYS) *reinterpret_cast<f32x4*>(out_at(p.out2) + 16 * dt + 4 * g) = acc2[dt];
+            *reinterpret_cast<f32x4*>(out_at(p.out) + 16 * dt + 4 * g) = acc[dt] * (1.f / (kSplitLift * kSplitLift)) * p.scale;
+            if constexpr (KEYS) *reinterpret_cast<f32x4*>(out_at(p.out2) + 16 * dt + 4 * g) = acc2[dt] * (1.f / (kSplitLift * kSplitLift));
         }
     }
 }

@@ -49,8 +49,8 @@ __device__ __forceinline__ uint64_t row_live_bits(const RowWin& w, int j0, int f
 }
 
 // x where keep is -1, the masked score -1e30 where keep is 0 (one bit-field insert)
-__device__ __forceinline__ float keep_or_mask(float x, int keep) {
-    const uint32_t xb = __builtin_bit_cast(uint32_t, x), nb = __builtin_bit_cast(uint32_t, kNegBigA);
+__device__ __forceinline__ float keep_or_mask(float x, int keep, float masked = kNegBigA) {
+    const uint32_t xb = __builtin_bit_cast(uint32_t, x), nb = __builtin_bit_cast(uint32_t, masked);
     return __builtin_bit_cast(float, (xb & (uint32_t)keep) | (nb & ~(uint32_t)keep));
 }
 

@@ -94,22 +94,22 @@ struct RowState {
         const int f = first - dec;
         first = f < 0 ? f + win.lin : f;
     }
-    // the scores of a tile (register j of subtile u: position j0 + 16u + 4g + j), masked where the row has no entry
+    // the scores of a tile (register j of subtile u: position j0 + 16u + 4g + j), `masked` where the row has no entry
     template <int SUB>
-    __device__ __forceinline__ void mask_tile(f32x4 (&s)[SUB], int j0, int g, bool uniform) const {
+    __device__ __forceinline__ void mask_tile(f32x4 (&s)[SUB], int j0, int g, bool uniform, float masked = kNegBigA) const {
         if (uniform) {  // every position of the span
             const int at = j0 + 4 * g - win.lo;
 #pragma unroll
             for (int u = 0; u < SUB; ++u)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) s[u][j] = (unsigned)(at + 16 * u + j) < (unsigned)win.cnt ? s[u][j] : kNegBigA;
+                for (int j = 0; j < 4; ++j) s[u][j] = (unsigned)(at + 16 * u + j) < (unsigned)win.cnt ? s[u][j] : masked;
         } else {
             asm volatile("");  // (keeps the bit masks below out of the paths that do not need them)
             const uint64_t bits = row_live_bits(win, j0, first, pat) >> (4 * g);
 #pragma unroll
             for (int u = 0; u < SUB; ++u)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) s[u][j] = keep_or_mask(s[u][j], ((int)((uint32_t)(bits >> (16 * u)) << (31 - j))) >> 31);
+                for (int j = 0; j < 4; ++j) s[u][j] = keep_or_mask(s[u][j], ((int)((uint32_t)(bits >> (16 * u)) << (31 - j))) >> 31, masked);
         }
     }
 };

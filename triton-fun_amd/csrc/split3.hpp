@@ -6,11 +6,16 @@
 // sixteen times the float32 ones' rate, so six of them cost three eighths of one float32 product, and they add sixteen products
 // with one rounding where the float32 ones round after each: against float64, 32 x 32 results over 64 / 128 / 512 N(0, 1) products
 // are off by 1.1e-7 / 1.6e-7 / 3.4e-7 of their norm (float32 instructions: 1.4e-7 / 2.1e-7 / 4.1e-7).
-// What the parts cannot hold is found in the operands or the results, and taken again in float32 arithmetic:
+// What the parts cannot hold:
 //   * an infinity, a NaN or a value above bfloat16's largest (3.39e38) turns its remainders into NaN, and with them every result it
-//     enters;
-//   * the last part of a value below 2^-108 is subnormal, which these instructions take as zero.  In a sum that matters where the
-//     whole result is as small (out_of_split's lower line), in a score where the other factor makes up for it (its upper line).
+//     enters, which is then taken again in float32 arithmetic;
+//   * bfloat16 ends at 2^-133 (the matrix instructions take and give subnormal values as they are), so a value below 2^-110 loses what
+//     it has below that.  The backward multiplies what it splits in the loop by kSplitLift, which puts the last bit of any float32 value
+//     there; results that overflow for it are taken again in float32 arithmetic.  The forward takes a row again
+//     where all outputs that a lane has of it are below 2^-96.  A row's own operand (Q; K and
+//     V in dK + dV) is not lifted, and the row is taken again where all that a lane has of it is small (out_of_split's lower line) or some
+//     of it so large (its upper line) that the other factor's lost bits show.  What is left: single values below 2^-110 among larger
+//     ones of a row, where the other factor is above 2^80.
 #pragma once
 #include "tile_copy.hpp"
 
@@ -47,6 +52,8 @@ __device__ __forceinline__ Split3 split3(const f32x8& x) {
     }
     return s;
 }
+
+constexpr float kSplitLift = 0x1p16f;
 
 // Whether the largest magnitude of some values is outside what products of split operands keep float32's precision for.
 __device__ __forceinline__ bool out_of_split(float most) {
