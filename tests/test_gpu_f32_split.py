@@ -158,3 +158,27 @@ def test_gradients_of_an_unlikely_key(dev, d):
         a, b = got[i][:, :, 30].double().cpu(), want[i][:, :, 30]
         assert float(b.abs().max()) > 1e-37
         assert float((a - b).norm() / b.norm()) <= 2e-5
+
+
+@pytest.mark.parametrize("keys_along", [False, True])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("unlikely", [False, True])
+def test_forward_of_a_small_column(dev, d, unlikely, keys_along):
+    """A column of V that is small, or that only an unlikely key has."""
+    L, masks = 211, [A.causal_windowed_pattern(211, 69)]
+    g = torch.Generator().manual_seed(d)
+    q, k, v = (torch.randn(1, 2, L, d, generator=g) for _ in range(3))
+    if unlikely:
+        unlikely_key(q, k)
+        v[..., 5] = 0.0
+        v[..., 30, 5] = 1.0
+    else:
+        small(2)(q, k, v)
+    live = masks[0].device_mask(dev).cpu() > 0
+    want = torch.softmax((q.double() @ k.double().transpose(2, 3) * d ** -0.5).masked_fill(~live, float("-inf")), -1) @ v.double()
+    attn = RegularAttention(1, L, 2, d, masks, 16, 16, dev, torch.float32, scale=d ** -0.5)
+    kT = k.to(dev).transpose(2, 3)
+    got = attn([q.to(dev), kT.contiguous() if keys_along else kT, v.to(dev)])
+    assert error(got, want) <= 1e-6 * (20 if unlikely else 1)
+    rows = live[:, 30] if unlikely else torch.ones(L, dtype=torch.bool)
+    assert column_error(got[:, :, rows.to(dev)], want[:, :, rows]) <= (2e-5 if unlikely else 1e-6)

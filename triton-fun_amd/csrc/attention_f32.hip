@@ -312,16 +312,19 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_fwd_f32_kernel(cons
     }
 
     const float l_tot = over_groups(l_run, [](float x, float y) { return x + y; });
-    // What is not finite anywhere stays so in a row's sum or outputs; outputs that are subnormal by far mean a V that is.
-    float chk = l_tot * 0.f, most = 0.f;
+    // What is not finite anywhere stays so in a row's sum or outputs.  An output far below normal is one whose probabilities or values
+    // are (one less than twice its bits: the smallest magnitude but zero).
+    float chk = l_tot * 0.f;
+    uint32_t least = ~0u;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            chk = fmaf(o[dt][j], 0.f, chk);
-            most = fmaxf(most, fabsf(o[dt][j]));
+            const float x = o[dt][j];  // (a bit cast of the element itself takes the vector's first)
+            chk = fmaf(x, 0.f, chk);
+            least = min(least, (__builtin_bit_cast(uint32_t, x) << 1) - 1);
         }
-    beyond |= chk != 0.f || (most > 0.f && most < 0x1p-96f * l_tot);  // (NaN compares unequal)
+    beyond |= chk != 0.f || least < __builtin_bit_cast(uint32_t, 0x1p-104f * l_tot) << 1;  // (NaN compares unequal)
     if (__any(beyond)) {
         // ---- this wavefront's rows once more in float32 arithmetic, position by position, each lane a quarter of a row's columns,
         // live positions only ----

@@ -11,8 +11,8 @@
 //     enters, which is then taken again in float32 arithmetic;
 //   * bfloat16 ends at 2^-133 (the matrix instructions take and give subnormal values as they are), so a value below 2^-110 loses what
 //     it has below that.  The backward multiplies what it splits in the loop by kSplitLift, which puts the last bit of any float32 value
-//     there; results that overflow for it are taken again in float32 arithmetic.  The forward takes a row again
-//     where all outputs that a lane has of it are below 2^-96.  A row's own operand (Q; K and
+//     there; results that overflow for it are taken again in float32 arithmetic.  The forward, whose probabilities are at most 2^8, takes a row again
+//     where an output is below 2^-104: a small column of V, or one that only keys of small probability have.  A row's own operand (Q; K and
 //     V in dK + dV) is not lifted, and the row is taken again where all that a lane has of it is small (out_of_split's lower line) or some
 //     of it so large (its upper line) that the other factor's lost bits show.  What is left: single values below 2^-110 among larger
 //     ones of a row, where the other factor is above 2^80.
