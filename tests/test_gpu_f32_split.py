@@ -4,7 +4,7 @@ import pytest
 import torch
 
 import acsr_helpers as A
-from r_attention import RegularAttention, attention_with_grad
+from r_attention import RegularAttention, attention_launcher, attention_with_grad
 
 pytestmark = pytest.mark.gpu
 
@@ -182,3 +182,58 @@ def test_forward_of_a_small_column(dev, d, unlikely, keys_along):
     assert error(got, want) <= 1e-6 * (20 if unlikely else 1)
     rows = live[:, 30] if unlikely else torch.ones(L, dtype=torch.bool)
     assert column_error(got[:, :, rows.to(dev)], want[:, :, rows]) <= (2e-5 if unlikely else 1e-6)
+
+
+WALKS = {"windowed": lambda L: [A.windowed_pattern(L, 23)], "gathered": lambda L: [A.dilated_pattern(L, 11, 3)],
+         "two segments": lambda L: A.strided_patterns(L, 20, 18), "steps on dense columns": lambda L: A.strided_patterns(L, 30, 7)[1:]}
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("L", [130, 257])
+@pytest.mark.parametrize("name", list(WALKS))
+def test_rows_taken_again_on_every_walk(dev, name, L, d):
+    """Column 0 of Q and V beyond what the parts hold, of K and dO zero: the same scores, every row in float32 arithmetic."""
+    masks, B, H = WALKS[name](L), 1, 2
+    g = torch.Generator().manual_seed(L + d)
+    q, k, v, go = (torch.randn(B, H, L, d, generator=g) for _ in range(4))
+    q[..., 0] = v[..., 0] = 2.0 ** 90
+    k[..., 0] = go[..., 0] = 0.0
+    live = sum(m.device_mask(dev) for m in masks).cpu() > 0
+    wide = [t.double().requires_grad_(True) for t in (q, k, v)]
+    s = (wide[0] @ wide[1].transpose(2, 3) * d ** -0.5).masked_fill(~live, float("-inf"))
+    p = torch.where(live.any(1)[:, None], torch.softmax(s, -1), torch.zeros_like(s)).masked_fill(~live, 0.0)
+    want = p @ wide[2]
+    grads = [torch.nan_to_num(t) for t in torch.autograd.grad(want, wide, go.double())]
+    want = want.detach()
+
+    def close(got, want):  # N(0, 1) columns, and column 0, which may be 2^90 times as large
+        for part in (slice(0, 1), slice(1, None)):
+            a, b = got[..., part].double().cpu(), want[..., part]
+            assert float((a - b).abs().max()) <= 2e-5 * max(1.0, float(b.abs().max()))
+
+    attn = RegularAttention(B, L, H, d, masks, 16, 16, dev, torch.float32, scale=d ** -0.5)
+    on = [t.to(dev) for t in (q, k, v)]
+    for kT in (on[1].transpose(2, 3), on[1].transpose(2, 3).contiguous()):
+        close(attn([on[0], kT, on[2]]), want)
+        out = torch.empty_like(on[0])  # without a plan table
+        attention_launcher(on[0], kT, on[2], out, attn.segments, d ** -0.5)
+        close(out, want)
+    on = [t.requires_grad_(True) for t in on]
+    for a, b in zip(torch.autograd.grad(attention_with_grad(*on, attn), on, go.to(dev)), grads):
+        close(a, b)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_listed_rows_taken_again(dev, d):
+    B, H, L = 1, 2, 700
+    attn = RegularAttention(B, L, H, d, A.strided_patterns(L, 64, 50), 16, 16, dev, torch.float32, scale=d ** -0.5)
+    g = torch.Generator(device=dev).manual_seed(d)
+    q, k, v, go = (torch.randn(B, H, L, d, generator=g, device=dev) for _ in range(4))
+    k[..., 0] = go[..., 0] = 0.0
+    far = [t.clone() for t in (q, v)]
+    for t in far:
+        t[..., 0] = 2.0 ** 90
+    clean = attn.backward_pass([q, k.transpose(2, 3), v], go, sparse_rows=True)
+    again = attn.backward_pass([far[0], k.transpose(2, 3), far[1]], go, sparse_rows=True)
+    for a, b in zip(again, clean):
+        assert float((a - b)[..., 1:].abs().max()) <= 2e-5 * float(b.abs().max())

@@ -38,6 +38,29 @@ def test_equals_rows_of_keys(dev, dtype, d, L):
     assert torch.equal(attn([q, part, v]), want)
 
 
+@pytest.mark.parametrize("dtype", TYPES)
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("L", [201, 519])
+def test_two_segments(dev, dtype, d, L):
+    """A window and a band 60 to 80 keys before it: walks that change segments, the second of which begins with rows of nothing."""
+    B, H, dt = 2, 3, TYPES[dtype]
+    at = torch.arange(L)
+    back = at[:, None] - at[None, :]
+    masks = [((back >= lo) & (back <= hi)).to(torch.uint8).to(dev) for lo, hi in ((0, 33), (60, 80))]
+    attn = RegularAttention(B, L, H, d, masks, 16, 16, dev, dt, scale=d ** -0.5)
+    g = torch.Generator(device=dev).manual_seed(L + d)
+    q, k, v = (torch.randn(B, H, L, d, generator=g, device=dev).to(dt) for _ in range(3))
+    want = attn([q, k.transpose(2, 3), v]).clone()
+    live = sum(masks).cpu() > 0
+    s = (q.double() @ k.double().transpose(2, 3) * d ** -0.5).cpu().masked_fill(~live, float("-inf"))
+    assert float((want.double().cpu() - torch.softmax(s, -1) @ v.double().cpu()).abs().max()) <= (1e-5 if dt == torch.float32 else 0.04)
+    assert torch.equal(attn([q, k.transpose(2, 3).contiguous(), v]), want)
+    long = torch.full((B, H, d, L + 7), float("nan"), dtype=dt, device=dev)
+    part = long[..., 3:3 + L]
+    part.copy_(k.transpose(2, 3))
+    assert torch.equal(attn([q, part, v]), want)
+
+
 @pytest.mark.parametrize("blocks,ran", [(128, True), (129, False)])
 def test_launches_that_copy_whole_pieces_refuse(dev, blocks, ran):
     L, d, dt = 121, 64, torch.bfloat16
