@@ -154,10 +154,10 @@ int splat_sddmm_probs(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, c
 
 /* splat_sddmm (lse == NULL) or splat_sddmm_probs (lse != NULL) with the mask's plan table: `plan` is what
  * splat_attention_plan wrote for the same segments and L (its per-block column ranges and per-row windows are those of
- * every tiled kernel here, not only the fused one).  The kernel for 16-bit types, d a multiple of 8 up to 128 and
- * launches of at least 256 row blocks (or rows of at most 256 slots) then starts its copies after two scalar loads instead of deriving the plan from the ACSR arrays
- * (-7 % at B=2 H=32 L=8192 d=128 T=512, -18 % at B=4 H=16 L=4096 d=64 T=256); other shapes ignore the plan.  Same
- * results bit for bit.  A plan built from other metadata gives wrong scores but no access outside the buffers.
+ * every tiled kernel here, not only the fused one).  The kernels for 16-bit types and d a multiple of 8 up to 128 then start their
+ * copies after a few scalar loads instead of deriving the plan from the ACSR arrays (-7 % at B=2 H=32 L=8192 d=128 T=512,
+ * -18 % at B=4 H=16 L=4096 d=64 T=256); the general kernel, which takes other shapes and rows of more than 256 slots in some
+ * launches of fewer than 256 row blocks, ignores the plan.  Same results bit for bit.  A plan built from other metadata gives wrong scores but no access outside the buffers.
  * Replaces the same reference code as splat_sddmm (rsddmm_launcher, r_sddmm.py:153-188). */
 int splat_sddmm_planned(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* kT,
                         int64_t k_sb, int64_t k_sh, int64_t k_sd, int64_t k_sl, void* out,

@@ -69,3 +69,26 @@ def test_short_rows_in_launches_that_fill_the_chip(dev, d, width):
     r_sddmm.rsddmm_launcher(q.to(dev), k.to(dev).transpose(2, 3), out, acsr[0], acsr[1], acsr[2], acsr[3], acsr[5], acsr[4], (1, 1), None, None, 16, 16)
     want, lv, got = O.sddmm(q.float(), k.float().transpose(2, 3), acsr_np, first_col=[0] * L), live(acsr_np), out.float().cpu()
     assert torch.equal(got[..., lv], want[..., lv]) and torch.all(got[..., ~lv] == SENTINEL)
+
+
+# half row blocks on both sides of every line of the launcher: rows of up to 256 slots, 300 (512 of one segment) and 450 (128 at d = 64, 256, 512 of two segments)
+@pytest.mark.parametrize("probabilities", [False, True])
+@pytest.mark.parametrize("two", [False, True])
+@pytest.mark.parametrize("d", [64, 96, 128])
+@pytest.mark.parametrize("width,heads", [(39, 3), (39, 40), (70, 12), (70, 30), (70, 75), (70, 82), (300, 10), (300, 17), (300, 37), (300, 64), (300, 65),
+                                         (450, 15), (450, 17), (450, 37), (450, 65)])
+def test_the_plan_table_changes_no_bit(dev, width, heads, d, two, probabilities):
+    """Rows of K, operands whose sums round, scores and probabilities."""
+    L = 500
+    pats = A.strided_patterns(L, width - 20, 32) if two else [A.causal_windowed_pattern(L, width - 1)]
+    segs = A.create_acsr_segments(pats, 16, dev)
+    g = torch.Generator(device=dev).manual_seed(width + heads)
+    q, k = (torch.randn(1, heads, L, d, generator=g, device=dev).to(torch.bfloat16) for _ in range(2))
+    lse = torch.randn(1, heads, L, generator=g, device=dev) + 20.0 if probabilities else None
+    got = []
+    for plan in (segs.plan(L, dev), False, None):
+        out = torch.full((1, heads, L, segs.T), SENTINEL, dtype=torch.bfloat16, device=dev)
+        r_sddmm.rsddmm_launcher(q, k.transpose(2, 3), out, None, None, None, None, segs.T, None, None, None, None, 16, 16, scale=0.3, segments=segs,
+                                lse=lse, plan=plan)
+        got.append(out)
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])

@@ -84,7 +84,8 @@ __global__ __launch_bounds__(256, 4) void sddmm_rows16_kernel(const SddmmParams 
     for (int t = 0; t < KS; ++t) k_addr[t] = base + lds_off<ROWB, true>(n, (4 * t + g) * 16);
 
     T* const out_row = (T*)p.out + ((int64_t)bh * L + row_in) * p.T;
-    const float lse = p.row_lse ? p.row_lse[(int64_t)bh * L + row_in] : 0.f;
+    // (one rounding as in sddmm_lines.hip, which takes the launches without a plan table: the same bits)
+    const float exp_mul = p.scale * 1.4426950408889634f, exp_sub = p.row_lse ? p.row_lse[(int64_t)bh * L + row_in] * 1.4426950408889634f : 0.f;
 
     uint32_t stage = 0;
     for (int sg = 0; sg < p.n_seg; ++sg) {
@@ -149,10 +150,11 @@ __global__ __launch_bounds__(256, 4) void sddmm_rows16_kernel(const SddmmParams 
                     kf[t].v = __builtin_bit_cast(typename Frag<T>::vec, lds_load128(k_addr[t] + stage + 16 * u * ROWB));
 #pragma unroll
                 for (int t = 0; t < KS; ++t) mma16(s, kf[t], q[t]);
-                s *= p.scale;
                 if (p.row_lse) {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) s[j] = fast_exp2((s[j] - lse) * 1.4426950408889634f);
+                    for (int j = 0; j < 4; ++j) s[j] = fast_exp2(fmaf(s[j], exp_mul, -exp_sub));
+                } else {
+                    s *= p.scale;
                 }
                 vec4 x;
 #pragma unroll
@@ -181,12 +183,18 @@ int launch_sddmm_rows16(const SddmmParams& p0, int in_dtype, bool kt, hipStream_
     p.n_row_blocks = count_row_blocks(p.L, kPlanBM, p.row_stride);
     const int64_t blocks = 2 * (int64_t)p.B * p.H * p.n_row_blocks;
     // The lines, as shares of the other kernels' time.  K along the keys, which the general kernel reads badly: 0.34 to 0.85 up to 512 blocks,
-    // at 1024 0.66 to 0.89 for d = 80 and rows of 33 to 129 slots, 0.82 to 1.20 for d = 128 or 300 slots.  Rows of K with the plan table, masks of 33 to 129 slots: d <= 96 0.62 to 1.04 up to 640 blocks, 0.83 to 1.21 at 1024;
-    // d = 128 0.60 to 0.91 up to 256, 0.84 to 1.07 from 384 to 640; 300 slots 0.43 to 0.97 up to 512, 0.82 to 1.03 at 640.  Without the
-    // table the prologue is longer, and once more for every segment: d <= 96 0.42 to 0.98 at 256 blocks, 0.84 to 1.08 at 512, d = 128 0.65 to 1.01
-    // at 128, 0.89 to 1.03 at 256; two segments 0.90 to 0.99 at half of that, 1.01 to 1.06 there.
-    const bool wide = p.d > 96 && p.T <= 256;
-    const int most = kt ? (p.d > 64 && p.d <= 96 && p.T <= 256 ? 1024 : 512) : p.plan ? (wide ? 256 : p.T <= 256 ? 640 : 512) : (wide ? 128 : 256) / p.n_seg;
+    // at 1024 0.66 to 0.89 for d = 80 and rows of 33 to 129 slots, 0.82 to 1.20 for d = 128 or 300 slots.
+    // Rows of K of up to 256 slots with the plan table, masks of 33 to 129 slots: d <= 96 0.62 to 1.04 up to 640 blocks, 0.83 to 1.21 at 1024;
+    // d = 128 0.60 to 0.91 up to 256, 0.84 to 1.07 from 384 to 640.  Without the table the prologue is longer, and once more for every segment:
+    // d <= 96 0.42 to 0.98 at 256 blocks, 0.84 to 1.08 at 512, d = 128 0.65 to 1.01 at 128, 0.89 to 1.03 at 256; two segments 0.90 to 0.99 at
+    // half of that, 1.01 to 1.06 there.  (sddmm_lines.hip, which takes the others, adds in the same order: the table changes no bit.)
+    // Longer rows: the others are the general kernel's up to 511, which adds in another order, so the line is one for both.  With the table and
+    // without, one segment of up to 400 slots 0.34 to 1.11 up to 512 blocks, two of up to 700 0.28 to 1.06; beyond, 0.35 to 1.00 up to 256
+    // (320 to 512: 0.73 to 1.42) but for one segment at d = 64, 0.55 to 0.85 up to 128, 0.84 to 1.20 at 192 and 256.
+    const bool d64 = p.d > 32 && p.d <= 64, wide = p.d > 96;
+    const int long_rows = p.T <= (p.n_seg > 1 ? 700 : 400) ? 512 : d64 && p.n_seg == 1 ? 128 : 256;
+    const int rows = p.T > 256 ? long_rows : p.plan ? (wide ? 256 : 640) : (wide ? 128 : 256) / p.n_seg;
+    const int most = kt ? (p.d > 64 && p.d <= 96 && p.T <= 256 ? 1024 : 512) : rows;
     // And with the table, launches that fill the chip, rows of K: rows of at most 40 slots at 0.70 to 0.95 (one of 40 launches 1.03) up to 16384
     // blocks; longer ones that are no whole 64-byte pieces, which the line-wise kernel stores in most, from where that has more than its one
     // round of workgroups (at 1024 blocks 0.83 to 1.10) to 4096: d <= 32 0.57 to 0.95, d = 64 from 129 slots on 0.63 to 0.99, d = 80 to 128 up
