@@ -36,7 +36,7 @@
 extern "C" {
 #endif
 
-#define SPLAT_VERSION 1100 /* major*10000 + minor*100 + patch; 0.2.0 added the planned forward, 0.3.0 splat_spmm_t, 0.4.0 splat_attention_fwd_stats, splat_sddmm_probs, 0.5.0 splat_attention_fwd_noalloc, 0.6.0 moved the two measurement aids out (libsplat_bench.so, splat_bench.h), 0.7.0 added splat_sddmm_planned, splat_spmm_planned, 0.8.0 splat_spmm_t_planned, 0.9.0 splat_attention_bwd_keys, 0.10.0 splat_acsr_build_record, splat_attention_bwd_f32, splat_attention_bwd_keys_f32, 0.11.0 gave splat_acsr_build_record's int32 arrays a buffer of their own and added splat_attention_plan_report, splat_attention_fwd_hinted */
+#define SPLAT_VERSION 1200 /* major*10000 + minor*100 + patch; 0.2.0 added the planned forward, 0.3.0 splat_spmm_t, 0.4.0 splat_attention_fwd_stats, splat_sddmm_probs, 0.5.0 splat_attention_fwd_noalloc, 0.6.0 moved the two measurement aids out (libsplat_bench.so, splat_bench.h), 0.7.0 added splat_sddmm_planned, splat_spmm_planned, 0.8.0 splat_spmm_t_planned, 0.9.0 splat_attention_bwd_keys, 0.10.0 splat_acsr_build_record, splat_attention_bwd_f32, splat_attention_bwd_keys_f32, 0.11.0 gave splat_acsr_build_record's int32 arrays a buffer of their own and added splat_attention_plan_report, splat_attention_fwd_hinted, 0.12.0 added splat_attention_fwd_keys and summary[5..6] of splat_acsr_build, which a row_stride_hint may come from */
 
 /* element types of q/k/v/score/output buffers */
 #define SPLAT_F32 0
@@ -286,7 +286,8 @@ int splat_attention_fwd_keys(const void* q, int64_t q_sb, int64_t q_sh, int64_t 
  * into a buffer of SPLAT_STATIC_PLAN_BYTES that is part of the library's device image (each GPU the library runs on
  * holds one until the process ends), then the forward runs from it on the same stream.  The call allocates and frees
  * nothing.  Masks whose plan is larger (splat_attention_plan_bytes; 4256 bytes per 128-row block and segment) are
- * rejected with SPLAT_E_SHAPE.  All calls on one GPU share that one buffer: two calls whose work may overlap on a
+ * rejected with SPLAT_E_SHAPE, but for those whose plan is larger only for a row_stride_hint (rows grouped by phase fill their last
+ * blocks less): they are planned without it, which walks other tiles, so their results agree with the planned forward's to rounding.  All calls on one GPU share that one buffer: two calls whose work may overlap on a
  * GPU (different streams, different threads) race; order them.  The first call on a GPU for a given element type, head
  * size and K layout also looks up the buffer's address and raises its kernel's LDS limit, which are not stream
  * operations: make that call outside any stream capture (one eager warm-up call per configuration is enough; every

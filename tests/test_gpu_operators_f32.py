@@ -82,3 +82,23 @@ def test_two_segments_in_launches_that_share_tiles_out_and_ones_that_do_not(dev)
         res = torch.empty(B, H, L, d, device=dev)
         r_spmm.rspmm_launcher(out.remainder(7.0), vd, res, None, None, None, None, None, None, segs.T, None, None, 16, 16, segments=segs)
         assert torch.equal(res.cpu(), want.expand(B, H, L, d))
+
+
+# 1024 row blocks of 64 rows of more than 600 slots at d <= 64 (450 for 33 to 56 values) go to the general kernel: both sides of each line
+@pytest.mark.parametrize("layout", ["rows", "keys"])
+@pytest.mark.parametrize("d,width,heads", [(32, 600, 64), (32, 601, 64), (64, 601, 63), (40, 450, 64), (40, 451, 64), (56, 451, 64), (57, 451, 64), (80, 601, 64)])
+@pytest.mark.parametrize("step", [1, 2])
+def test_sddmm_on_both_sides_of_the_general_kernel(dev, step, d, width, heads, layout):
+    """Through the launcher's own path, which turns K along the keys for gathered masks where the general kernel runs."""
+    L = 1024
+    mask = O.create_dilated_mask(L, width, 2) if step == 2 else O.create_causal_windowed_mask(L, width - 1)
+    acsr, acsr_np = acsr_pair(mask, 16, dev)
+    q, k = whole((1, heads, L, d), heads).to(dev), whole((1, heads, L, d), d).to(dev)
+    out = torch.full((1, heads, L, acsr[5]), SENTINEL, device=dev)
+    kT = k.transpose(2, 3)
+    r_sddmm.rsddmm_launcher(q, kT.contiguous() if layout == "keys" else kT, out, acsr[0], acsr[1], acsr[2], acsr[3], acsr[5], acsr[4], (1, 1), None, None, 16, 16)
+    lv = live(acsr_np)
+    for h in (0, heads // 2, heads - 1):
+        want = O.sddmm(q[:, h:h + 1].cpu(), k[:, h:h + 1].cpu().transpose(2, 3), acsr_np, first_col=O.row_extents(mask)[0])
+        got = out[:, h:h + 1].cpu()
+        assert torch.equal(got[..., lv], want[..., lv]) and torch.all(got[..., ~lv] == SENTINEL)

@@ -1,8 +1,8 @@
 // ACSR builder and mask generators.
 //
 // splat_acsr_build, splat_acsr_build_record: one wavefront per mask row streams the row once (16-byte loads), reducing the byte sum (nnz), the first two columns whose byte equals 1 (the affine map's anchors a < b) and the
-// first/last nonzero column.  Lane 0 then evaluates the 2x2 solve of acsr_helpers.py:122 in closed
-// form in double precision and rounds to float32, which is what the reference's
+// first/last nonzero column.  The first wavefront of a workgroup then evaluates the 2x2 solve of acsr_helpers.py:122 for up to 64 of its rows,
+// a lane each, in closed form in double precision and rounds to float32, which is what the reference's
 // float64 -> torch.FloatTensor conversion stores.  The per-row-block span pairs (acsr_helpers.py:135-140) come from the
 // same kernel, or, with the summary on the device, from a second, tiny one.  HBM-bound: rows*ld bytes in, 28*rows out.
 #include "splat_common.hpp"

@@ -377,7 +377,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(const BwdParams p) {
             for (int nt = 0; nt < 2; ++nt) {
                 static_assert(!THREE || NDMA <= KS, "the first half issues all copies");
                 // half a tile that holds nothing for this wavefront, as at the ends of most spans (bfloat16, 64 heads of 4096, the
-                // whole step: window 65 at d = 64 131 -> 123 us, 33 at d = 128 257 -> 252; 64 heads of 8192, 512 / 2, 985 -> 977)
+                // whole step: window 65 at d = 64 131 -> 123 us, 33 at d = 128 257 -> 252)
                 if (nt == 0 ? j0 + 32 <= w_lo_min : j0 + 32 >= w_hi_max) {
                     if (nt == 0 && spread) {
 #pragma unroll

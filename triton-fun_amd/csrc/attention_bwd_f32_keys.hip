@@ -13,7 +13,7 @@
 
 namespace splat {
 
-// Operand layouts of acc[16x16] += A[16x4] * B[4x16] (v_mfma_f32_16x16x4_f32): lane (n = lane % 16, g = lane / 16) feeds row n
+// Operand layouts of mma4 (acc[16x16] += A[16x4] * B[4x16], v_mfma_f32_16x16x4_f32): lane (n = lane % 16, g = lane / 16) feeds row n
 // of A and column n of B at contraction slot g, and holds rows 4g .. 4g + 3 of column n of the result.  Which index of the
 // contraction a slot stands for is free as long as A and B agree:
 //   * products over d take d = 16t + 4g + j in instruction 4t + j, so that one 16-byte read of a row feeds four instructions;
@@ -22,8 +22,6 @@ namespace splat {
 //   * of the output of those, row m of tile dt stands for d = 4m + dt (+ 64h), so that one 16-byte read of a row of the other
 //     operand feeds four tiles, and a lane's 16 results of one row are 16 consecutive columns.
 constexpr int kF32D = 128, kF32Tile = 16;  // positions per tile: 8 KB an operand
-
-__device__ __forceinline__ void mma4(f32x4& acc, float a, float b) { acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc, 0, 0, 0); }
 
 __device__ __forceinline__ f32x4 lds_load_f32x4(uint32_t addr) { return __builtin_bit_cast(f32x4, lds_load128(addr)); }
 
@@ -96,7 +94,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_keys_f32_kernel(const BwdPara
     }
     total = __builtin_amdgcn_readfirstlane(total);
 
-    // ---- asynchronous copies of one tile (see attention_f32.hip) ----
+    // ---- asynchronous copies of one tile (see tile_copy.hpp) ----
     auto position_row = [&](const HalfWalk& w, int j) { return min(max(w.pl.c0 + w.pl.cs * j, 0), L - 1); };
     uint32_t x_off[NI], y_off[NI];
     const char *x_next = nullptr, *y_next = nullptr;

@@ -449,13 +449,14 @@ PyObject* py_sddmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
         // than 256 slots the general kernel, which is faster on rows of K as well (4 heads of 4001 rows, 301 slots, d = 64: 49 -> 43).  Beyond d = 64 the copy costs as much as it gives (64 heads of 2048 rows, 255 slots: d = 80 122 -> 125,
         // d = 96 126 -> 129), and so does its launch below 64 row blocks (one head of 200 rows: 21 -> 25).
         const bool turned = code != SPLAT_F32 && out_code == code && d % 8 == 0 && d <= 64 && B * H * ((L + 127) / 128) >= 64;
-        // Up to 128 inner values float32 (operators_f32.hip) and 16-bit launches of few row blocks (sddmm_rows16.hip, whose conditions are these;
+        // Up to 128 inner values float32 (operators_f32.hip, but for the launches that its launcher leaves to the general kernel) and 16-bit launches of few row blocks (sddmm_rows16.hip, whose conditions are these;
         // a stride of n between a block's rows adds at most n - 1 blocks) turn K on its way into LDS, gathered or not: the three
         // operators, float32, 16 heads of 1605 rows, 176 slots with step 2, d = 128, 76.9 -> 72.3 us without the copy.
         const bool few = d % 8 == 0 && B * H * 2 * ((L + 127) / 128 + std::max(m->max_step - 1, 0)) <= 512 &&
                          (reinterpret_cast<uintptr_t>(x->data_ptr()) & 15) == 0 && x->stride(0) % 8 == 0 && x->stride(1) % 8 == 0 &&
                          x->stride(2) % 8 == 0;
-        const bool in_place = out_code == code && d <= 128 && (code == SPLAT_F32 || few);
+        const bool general_f32 = d <= 64 && T > (d > 32 && d <= 56 ? 450 : 600) && B * H * ((L + 63) / 64 + std::max(m->max_step - 1, 0)) >= 1024;
+        const bool in_place = out_code == code && d <= 128 && (code == SPLAT_F32 ? !general_f32 : few);
         if ((m->max_step >= 2 || turned) && !in_place && y.stride(3) == 1 && y.stride(2) != 1) {
             if (y.stride(2) < keys) Py_RETURN_FALSE;
             y = transposed_keys(y, &rc).transpose(2, 3);

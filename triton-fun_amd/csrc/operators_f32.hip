@@ -9,7 +9,10 @@
 // The three operators against the kernels of 128 rows a workgroup and tiles of 64 that took these launches before (sddmm.hip, spmm.hip, which
 // keep the longer rows and 16-bit outputs): 2 heads of 2048 rows, blocks of 64, d = 80 58 -> 22 us; 2 heads of 3001 rows, 501 slots, d = 96
 // 135 -> 60; 16 heads of 2048, 256 slots, d = 64 87 -> 61, 128 heads 465 -> 361; 64 heads of 2048, 129 slots, d = 128 267 -> 185; where the
-// matrix instructions bound both (64 heads of 4096, blocks of 512) 586 -> 577.  Nowhere slower, so there is no lower or upper size.
+// matrix instructions bound both (64 heads of 4096, blocks of 512) 586 -> 577.  Over 900 launches of 1 to 128 heads of 200 to 2048 rows, 9 to
+// 513 slots, d = 16 to 128, causal, windowed, strided and blocked masks: SDDMM 0.26 to 1.24 of the time, 0.58 in the mean, SpMM 0.20 to 1.06,
+// 0.45.  Large launches of longer rows at d <= 64 are at the upper end; where SDDMM leaves them stands at its launcher.  SpMM keeps them: of 192 to
+// 1024 slots and 512 to 2048 row blocks of d = 16 to 128 0.51 to 1.18, 16 of 864 above 1.02, all of blocked masks at d = 32 and 64.
 #include <algorithm>
 
 #include "rows16.hpp"
@@ -21,9 +24,6 @@ namespace splat {
 namespace {
 
 constexpr int kRows = 64, kTile = 32;
-
-// acc[16x16] += A[16x4] . B[4x16]; lane (n, g) holds value g of row n (A), of column n (B), rows 4g .. 4g + 3 of column n (acc)
-__device__ __forceinline__ void mma4(f32x4& acc, float a, float b) { acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc, 0, 0, 0); }
 
 // values 4c .. 4c + 3 of a row of n values, zeros past its end; `vec`: the row starts on a 16-byte boundary
 __device__ __forceinline__ f32x4 row_piece(const float* row, int c, int n, bool vec) {
@@ -304,6 +304,13 @@ int launch_sddmm_f32(const SddmmParams& p0, bool kt, hipStream_t st) {
     p.n_row_blocks = count_row_blocks(p.L, kRows, p.row_stride);
     const int64_t blocks = (int64_t)p.B * p.H * p.n_row_blocks;
     if (blocks > 0x7ffffff0) return 0;
+    // Launches that fill the chip several times over are bound by the matrix instructions, and the general kernel, whose rows leave in whole
+    // lines, catches up as rows get longer, first where this one pads the contraction (33 to 56 values to 64).  Means over five kinds of masks
+    // and four such launches, rows of K / K along the keys: 384, 512, 768, 1024 slots, d = 16 0.92 / 0.95, 0.98 / 1.03, 1.11 / 1.15, 1.18 / 1.23;
+    // d = 32 0.80 / 0.83, 0.87 / 0.92, 0.99 / 1.04, 1.09 / 1.13; d = 48 0.99 / 1.01, 1.07 / 1.11, 1.11 / 1.15, 1.16 / 1.19; d = 64 0.86 / 0.89,
+    // 0.94 / 0.98, 0.97 / 1.01, 1.02 / 1.06 (blocked masks, which skip nothing, up to 0.3 above these); d = 80 and 128 0.54 to 0.97 throughout.
+    // (host_ext.cpp turns K along the keys for gathered masks where these go to the general kernel: the same line stands there.)
+    if (blocks >= 1024 && p.d <= 64 && p.T > (p.d > 32 && p.d <= 56 ? 450 : 600)) return 0;
     // Few row blocks: their tiles are shared out over up to three workgroups a CU, to no more than there are tiles (every further one has
     // the prologue and nothing to do).  Over 168 launches of 16 to 640 blocks 0.87 of the time that up to four and 32 a block take (4 heads
     // of 1024 rows, two segments of 94 slots, d = 128 17.7 -> 10.6 us); from 512 blocks on two a block pay for short contractions of longer rows

@@ -42,6 +42,9 @@ __device__ __forceinline__ WaveSpan span_of_rows16(const RowWin& w, bool uniform
     return s;
 }
 
+// acc[16x16] += A[16x4] . B[4x16] in float32; lane (n, g) holds value g of row n (A), of column n (B), rows 4g .. 4g + 3 of column n (acc)
+__device__ __forceinline__ void mma4(f32x4& acc, float a, float b) { acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc, 0, 0, 0); }
+
 // Position of a walk over tiles of BN positions: the segment, its plan, the next tile and the end of the segment's range.
 struct HalfWalk {
     int seg, tile, end;

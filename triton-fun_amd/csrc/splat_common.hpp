@@ -105,8 +105,8 @@ __device__ __forceinline__ void store_as(void* base, int64_t idx, float x, int d
 
 // f(v of this lane, v of lane ^ O) for a commutative f, O a power of two, by the vector unit's own exchanges.  Through
 // __shfl_xor, which is a permute through LDS, every step of a reduction waits some 130 cycles for the one before it.
-// Same pairs, same bits: fused forward, 64 heads of 4096 (d = 64, window 256) 44.9 -> 44.6 us and 64 heads of 16384 (d = 128,
-// window 512) 408 -> 406; SDDMM, softmax and SpMM of 64 heads of 8192, 512 slots, 562 -> 559.
+// Same pairs, same bits.  Where a kernel has other work to hide the wait behind, it gives no more than two runs differ by (fused forward,
+// 64 heads of 4096, d = 64, window 256, 44.9 -> 44.6 us).
 // N: the lanes 2 * O apart hold the same already, which an exchange of 4 lanes in groups of 16 or of 2 * O may rely on.
 template <int O, int N, typename V, typename F>
 __device__ __forceinline__ V with_lane_xor(V v, F f) {

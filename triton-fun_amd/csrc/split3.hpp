@@ -1,6 +1,7 @@
 // float32 products on the 16-bit matrix instructions.
 //
-// A float32 value is the sum of three bfloat16 values, its rounding and the roundings of the two remainders (8 + 8 + 8 bits of
+// The published splitting of Henry, Tang and Heinecke ("Leveraging the bfloat16 Artificial Intelligence Datatype For
+// Higher-Precision Computations", 2019): a float32 value is the sum of three bfloat16 values, its rounding and the roundings of the two remainders (8 + 8 + 8 bits of
 // significand; bfloat16 has float32's exponents, so nothing has to be scaled).  Of the nine products of two such sums the six
 // largest are taken, the smallest first; the three left out are below 2^-24 of the product.  The 16-bit instructions run at
 // sixteen times the float32 ones' rate, so six of them cost three eighths of one float32 product, and they add sixteen products
