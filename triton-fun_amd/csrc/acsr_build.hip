@@ -138,8 +138,8 @@ __device__ __forceinline__ bool finish_row(const RowScan& s, int row, int cols, 
 // The rows of one span block folded together: span_start = min(cols, min_r trans_r), span_end = max(-1, max_r nnz_r*lin_r +
 // trans_r), evaluated in double from the exact integers (a, lin, nnz) and rounded once to float32, and the block's share of
 // the summary: T = max nnz, smallest / largest column step over rows with nnz > 1, how many of these have a first column that
-// is not congruent to the row index modulo their step, the smallest / largest residue of the first column less the row index, and how
-// many rows the reference would have asserted on.
+// is not congruent to the row index modulo their step (for callers of the C interface: the grouping here asks the residues), the
+// smallest / largest residue of the first column less the row index, and how many rows the reference would have asserted on.
 struct BlockFold {
     float lo, hi;  // (a rounding is monotone: the least of the rounded is the least, rounded)
     int t_max, step_min, step_max, off_phase, res_min, res_max, failed;

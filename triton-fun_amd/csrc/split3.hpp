@@ -16,7 +16,7 @@
 //     where an output is below 2^-104: a small column of V, or one that only keys of small probability have.  A row's own operand (Q; K and
 //     V in dK + dV) is not lifted, and the row is taken again where all that a lane has of it is small (out_of_split's lower line) or some
 //     of it so large (its upper line) that the other factor's lost bits show.  What is left: single values below 2^-110 among larger
-//     ones of a row, where the other factor is above 2^80.
+//     ones of a row, where the other factor is above 2^80, and, in the forward, a column of V with nothing above 2^-134, which comes out as zero.
 #pragma once
 #include "tile_copy.hpp"
 
