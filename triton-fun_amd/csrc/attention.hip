@@ -99,12 +99,14 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnParams p) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lm = lane & 31, g = lane >> 5;
 
-    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    load_args(p.total, p.n_row_blocks, p.by_blocks.m, p.by_blocks.shift, p.by_h.m, p.by_h.shift, p.H, p.row_stride, p.L, p.n_seg, p.plan, p.scale_log2e,
+              p.q, p.q_sb, p.q_sh, p.q_sl, p.k, p.k_sb, p.k_sh, p.k_sd, p.k_sl, p.v, p.v_sb, p.v_sh, p.v_sl);
+    const int logical = xcd_remap(blockIdx.x, p.total);
     if (logical >= p.total) return;
-    const int bh = logical / p.n_row_blocks;
+    const int bh = quotient(logical, p.by_blocks);
     // later row blocks of causal patterns carry the most keys: hand them out first
-    const int rb = p.n_row_blocks - 1 - (logical % p.n_row_blocks);
-    const int b = bh / p.H, h = bh % p.H;
+    const int rb = p.n_row_blocks - 1 - (logical - bh * p.n_row_blocks);
+    const int b = quotient(bh, p.by_h), h = bh - b * p.H;
     const int rs = p.row_stride;
     const int r0 = block_first_row(rb, BM, rs);
     const int L = p.L;
@@ -561,6 +563,7 @@ static int launch_attn(const AttnParams& p0, hipStream_t st) {
     constexpr int BM = 128;
     p.n_row_blocks = count_row_blocks(p.L, BM, p.row_stride);
     p.total = p.B * p.H * p.n_row_blocks;
+    p.by_blocks = divisor(p.n_row_blocks), p.by_h = divisor(p.H);
     if (PLANNED && KT) p.plan += plan_variant_recs(p.n_row_blocks, p.n_seg);  // the dense-walk variant
     const int grid = ((p.total + 7) / 8) * 8;
     const size_t lds = NSTAGE * (size_t)G::STAGE;

@@ -41,13 +41,15 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_keys_f32_kernel(const BwdPara
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, g = lane >> 4;
 
-    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    load_args(p.total, p.n_row_blocks, p.by_blocks.m, p.by_blocks.shift, p.by_h.m, p.by_h.shift, p.H, p.row_stride, p.L, p.n_seg, p.plan, p.scale_log2e,
+              p.a, p.a_sb, p.a_sh, p.a_sl, p.b, p.b_sb, p.b_sh, p.b_sl, p.x, p.x_sb, p.x_sh, p.x_sl, p.y, p.y_sb, p.y_sh, p.y_sl, p.lse, p.delta);
+    const int logical = xcd_remap(blockIdx.x, p.total);
     if (logical >= p.total) return;
     const int per_head = 2 * p.n_row_blocks;
-    const int bh = logical / per_head;
-    const int at = per_head - 1 - logical % per_head;
+    const int bh = quotient(logical, p.by_blocks);
+    const int at = per_head - 1 - (logical - bh * per_head);
     const int rb = at >> 1, half = at & 1;
-    const int b = bh / p.H, h = bh % p.H;
+    const int b = quotient(bh, p.by_h), h = bh - b * p.H;
     const int rs = p.row_stride, L = p.L, Lr = p.Lr;
     const int k0 = half * kHalfRows;
     const int r0 = block_first_row(rb, kPlanBM, rs) + rs * k0;
@@ -271,6 +273,7 @@ int launch_bwd_dkv_f32_d128(const BwdParams& p0, hipStream_t st) {
     begin_launch();
     BwdParams p = p0;
     p.total = p.B * p.H * 2 * p.n_row_blocks;
+    p.by_blocks = divisor(2 * p.n_row_blocks), p.by_h = divisor(p.H);
     constexpr size_t lds = 2 * 512 + 2 * 2 * kF32Tile * kF32D * 4;
     auto kern = attn_bwd_keys_f32_kernel;
     static uint64_t lds_reserved = 0;

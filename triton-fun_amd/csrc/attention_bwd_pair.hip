@@ -42,11 +42,13 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_pair_kernel(const BwdParams p
     const int pair = wave & 3, role = wave >> 2;  // role 0: positions 0 .. 31 of a tile and dK, 1: positions 32 .. 63 and dV
     const int lm = lane & 31, g = lane >> 5;
 
-    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    load_args(p.total, p.n_row_blocks, p.by_blocks.m, p.by_blocks.shift, p.by_h.m, p.by_h.shift, p.H, p.row_stride, p.L, p.n_seg, p.plan, p.scale_log2e,
+              p.a, p.a_sb, p.a_sh, p.a_sl, p.b, p.b_sb, p.b_sh, p.b_sl, p.x, p.x_sb, p.x_sh, p.x_sl, p.y, p.y_sb, p.y_sh, p.y_sl, p.lse, p.delta);
+    const int logical = xcd_remap(blockIdx.x, p.total);
     if (logical >= p.total) return;
-    const int bh = logical / p.n_row_blocks;
-    const int rb = p.n_row_blocks - 1 - (logical % p.n_row_blocks);
-    const int b = bh / p.H, h = bh % p.H;
+    const int bh = quotient(logical, p.by_blocks);
+    const int rb = p.n_row_blocks - 1 - (logical - bh * p.n_row_blocks);
+    const int b = quotient(bh, p.by_h), h = bh - b * p.H;
     const int rs = p.row_stride;
     const int r0 = block_first_row(rb, BM, rs);
     const int L = p.L, Lr = p.Lr;

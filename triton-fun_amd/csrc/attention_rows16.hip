@@ -45,13 +45,15 @@ __global__ __launch_bounds__(256, LAYOUT == kKeysAnywhere && D == 128 ? 2 : 3) v
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, g = lane >> 4;
 
-    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    load_args(p.total, p.n_row_blocks, p.by_blocks.m, p.by_blocks.shift, p.by_h.m, p.by_h.shift, p.H, p.row_stride, p.L, p.n_seg, p.plan, p.scale_log2e,
+              p.q, p.q_sb, p.q_sh, p.q_sl, p.k, p.k_sb, p.k_sh, p.k_sd, p.k_sl, p.v, p.v_sb, p.v_sh, p.v_sl);
+    const int logical = xcd_remap(blockIdx.x, p.total);
     if (logical >= p.total) return;
     const int per_head = 2 * p.n_row_blocks;
-    const int bh = logical / per_head;
-    const int at = per_head - 1 - logical % per_head;
+    const int bh = quotient(logical, p.by_blocks);
+    const int at = per_head - 1 - (logical - bh * per_head);
     const int rb = at >> 1, half = at & 1;
-    const int b = bh / p.H, h = bh % p.H;
+    const int b = quotient(bh, p.by_h), h = bh - b * p.H;
     const int rs = p.row_stride, L = p.L;
     const int k0 = half * kHalfRows;
     const int r0 = block_first_row(rb, kPlanBM, rs) + rs * k0;
@@ -367,6 +369,7 @@ static int launch(const AttnParams& p0, hipStream_t st) {
     AttnParams p = p0;
     p.n_row_blocks = count_row_blocks(p.L, kPlanBM, p.row_stride);
     p.total = p.B * p.H * 2 * p.n_row_blocks;
+    p.by_blocks = divisor(2 * p.n_row_blocks), p.by_h = divisor(p.H);
     if (PLANNED && LAYOUT != kKeyRows) p.plan += plan_variant_recs(p.n_row_blocks, p.n_seg);  // the dense-walk variant
     constexpr size_t lds = 2 * 2 * 64 * D * 2;  // two stages of two tiles of 64 positions
     auto kern = attn_fwd_rows16_kernel<T, D, LAYOUT, PLANNED>;

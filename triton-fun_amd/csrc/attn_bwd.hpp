@@ -24,6 +24,7 @@ struct BwdParams {
     const int* row_map;   // [Lr] or null: the row of A / B that row r of the mask stands for (r itself when null)
     float scale, scale_log2e;
     int n_seg, n_row_blocks, total, row_stride;
+    Divisor by_blocks, by_h;  // workgroups per head and H, filled in by the launch
     const PlanRec* plan;  // plan table of the mask (dQ) or of its transpose (dK, dV), first variant
 };
 

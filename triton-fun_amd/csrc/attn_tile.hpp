@@ -25,6 +25,7 @@ struct AttnParams {
     const PlanRec* plan;  // plan table of this mask (PLANNED kernels), variant already selected
     float* lse;           // optional [B*H, L]: log of every row's sum of exponentials (natural log, scaled scores)
     int live_percent;     // host only: share of the walked positions that some row sees, 0 where the caller did not say
+    Divisor by_blocks, by_h;  // workgroups per head and H, filled in by the launch
     bool keys_anywhere;   // host only: K^T with the keys contiguous whose rows are not whole 16-byte pieces
 };
 

@@ -56,12 +56,14 @@ __global__ __launch_bounds__(256, 4) void sddmm_f32_kernel(const SddmmParams p) 
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, g = lane >> 4;
 
-    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    load_args(p.total, p.key_split, p.by_split.m, p.by_split.shift, p.by_blocks.m, p.by_blocks.shift, p.by_h.m, p.by_h.shift, p.n_row_blocks, p.H, p.row_stride, p.L,
+              p.n_keys, p.d, p.T, p.n_seg, p.plan, p.q, p.q_sb, p.q_sh, p.q_sl, p.k, p.k_sb, p.k_sh, p.k_sd, p.k_sl, p.out);
+    const int logical = xcd_remap(blockIdx.x, p.total);
     if (logical >= p.total) return;
-    const int share = logical % p.key_split, block = logical / p.key_split;
-    const int bh = block / p.n_row_blocks;
-    const int rb = p.n_row_blocks - 1 - block % p.n_row_blocks;
-    const int b = bh / p.H, h = bh % p.H;
+    const int block = quotient(logical, p.by_split), share = logical - block * p.key_split;
+    const int bh = quotient(block, p.by_blocks);
+    const int rb = p.n_row_blocks - 1 - (block - bh * p.n_row_blocks);
+    const int b = quotient(bh, p.by_h), h = bh - b * p.H;
     const int rs = p.row_stride, L = p.L, d = p.d;
     const int r0 = block_first_row(rb, kRows, rs);
 
@@ -101,8 +103,8 @@ __global__ __launch_bounds__(256, 4) void sddmm_f32_kernel(const SddmmParams p) 
         pl.cs = __builtin_amdgcn_readfirstlane(pl.cs);
         pl.n_tiles = __builtin_amdgcn_readfirstlane(pl.n_tiles);
         pl.uniform = __builtin_amdgcn_readfirstlane(pl.uniform);
-        const int first = (int)((int64_t)pl.n_tiles * share / p.key_split);
-        const int end = (int)((int64_t)pl.n_tiles * (share + 1) / p.key_split);
+        const int first = quotient(pl.n_tiles * share, p.by_split);
+        const int end = quotient(pl.n_tiles * (share + 1), p.by_split);
         if (first >= end) continue;
 
         f32x4 raw[NP];
@@ -184,12 +186,14 @@ __global__ __launch_bounds__(256, 4) void spmm_f32_kernel(const SpmmParams p) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, g = lane >> 4;
 
-    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    load_args(p.total, p.by_chunks.m, p.by_chunks.shift, p.by_blocks.m, p.by_blocks.shift, p.by_h.m, p.by_h.shift, p.n_row_blocks, p.H, p.row_stride, p.L,
+              p.n_keys, p.n_out, p.T, p.n_seg, p.plan, p.v, p.v_sb, p.v_sh, p.v_sl, p.p);
+    const int logical = xcd_remap(blockIdx.x, p.total);
     if (logical >= p.total) return;
-    const int col0 = logical % p.n_col_chunks * (16 * NT), block = logical / p.n_col_chunks;
-    const int bh = block / p.n_row_blocks;
-    const int rb = p.n_row_blocks - 1 - block % p.n_row_blocks;
-    const int b = bh / p.H, h = bh % p.H;
+    const int block = quotient(logical, p.by_chunks), col0 = (logical - block * p.n_col_chunks) * (16 * NT);
+    const int bh = quotient(block, p.by_blocks);
+    const int rb = p.n_row_blocks - 1 - (block - bh * p.n_row_blocks);
+    const int b = quotient(bh, p.by_h), h = bh - b * p.H;
     const int rs = p.row_stride, L = p.L;
     const int r0 = block_first_row(rb, kRows, rs);
 
@@ -318,6 +322,7 @@ int launch_sddmm_f32(const SddmmParams& p0, bool kt, hipStream_t st) {
     p.key_split = (int)std::min<int64_t>((p.T + kTile - 1) / kTile + 3, std::max<int64_t>(1, 768 / blocks));
     if (p.key_split == 1 && blocks < 1024 && p.d <= 64 && p.T > 64) p.key_split = 2;
     p.total = (int)(blocks * p.key_split);
+    p.by_split = divisor(p.key_split), p.by_blocks = divisor(p.n_row_blocks), p.by_h = divisor(p.H);
     const int grid = ((p.total + 7) / 8) * 8;
     auto go = [&](auto kq) {
         constexpr int KQ = decltype(kq)::value;
@@ -348,6 +353,7 @@ int launch_spmm_f32(const SpmmParams& p0, hipStream_t st) {
     p.n_col_chunks = (tiles + nt - 1) / nt;
     if (blocks * p.n_col_chunks > 0x7ffffff0) return 0;
     p.total = (int)(blocks * p.n_col_chunks);
+    p.by_chunks = divisor(p.n_col_chunks), p.by_blocks = divisor(p.n_row_blocks), p.by_h = divisor(p.H);
     const int grid = ((p.total + 7) / 8) * 8;
     if (nt == 2) spmm_f32_kernel<2><<<grid, 256, 0, st>>>(p);
     else if (nt == 4) spmm_f32_kernel<4><<<grid, 256, 0, st>>>(p);

@@ -91,7 +91,7 @@ __global__ __launch_bounds__(256, (KSU > 0 && KSU * 16 < SddmmGeom<T>::DC && !KT
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lm = lane & 31, g = lane >> 5;
 
-    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    const int logical = xcd_remap(blockIdx.x, p.total);
     if (logical >= p.total) return;
     const int ksp = logical % p.key_split;  // this workgroup's share of the row block's tiles
     const int bh = (logical / p.key_split) / p.n_row_blocks;

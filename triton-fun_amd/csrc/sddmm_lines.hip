@@ -81,11 +81,13 @@ __global__ __launch_bounds__(BM_ * 4, 4) void sddmm_lines_kernel(const SddmmPara
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, g4 = lane >> 4;
 
-    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    load_args(p.total, p.key_split, p.by_split.m, p.by_split.shift, p.by_blocks.m, p.by_blocks.shift, p.by_h.m, p.by_h.shift, p.n_row_blocks, p.H, p.row_stride, p.L,
+              p.n_keys, p.d, p.T, p.n_seg, p.plan, p.q, p.q_sb, p.q_sh, p.q_sl, p.k, p.k_sb, p.k_sh, p.k_sd, p.k_sl, p.out);
+    const int logical = xcd_remap(blockIdx.x, p.total);
     if (logical >= p.total) return;
-    const int bh = logical / p.n_row_blocks;
-    const int rb = logical % p.n_row_blocks;
-    const int b = bh / p.H, h = bh % p.H;
+    const int bh = quotient(logical, p.by_blocks);
+    const int rb = logical - bh * p.n_row_blocks;
+    const int b = quotient(bh, p.by_h), h = bh - b * p.H;
     const int rs = p.row_stride;
     const int r0 = block_first_row(rb, BM, rs);
     const int L = p.L;
@@ -396,6 +398,7 @@ static int launch_lines_variant(const char* who, SddmmParams p, hipStream_t st) 
     if (blocks > 0x7ffffff0) return 0;
     p.key_split = 1;
     p.total = (int)blocks;
+    p.by_split = divisor(1), p.by_blocks = divisor(p.n_row_blocks), p.by_h = divisor(p.H);
     static uint64_t reserved = 0;
     auto kern = sddmm_lines_kernel<T, D, NST, KEYS, HL, BM, PROBS, PLANNED, PART>;
     if (int rc = reserve_dynamic_lds(&reserved, reinterpret_cast<const void*>(kern), G::LDS_BYTES, who)) return rc;

@@ -21,6 +21,7 @@ struct SddmmParams {
     int q_vec, k_vec;  // 16-byte loads are legal for q / k
     int out_vec;       // 16-bit outputs: every row's segment starts on a 16-byte boundary
     int row_stride;
+    Divisor by_split, by_blocks, by_h;  // key_split, row blocks (or halves) per head, H: filled in by the launches that read them
     int key_split;  // workgroups per row block: each takes a contiguous share of every segment's tiles
     const PlanRec* plan;  // optional: the mask's plan table for 128-row blocks (variant for row-major K), else nullptr
 };

@@ -42,14 +42,16 @@ __global__ __launch_bounds__(256, 4) void sddmm_rows16_kernel(const SddmmParams 
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, g = lane >> 4;
 
-    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    load_args(p.total, p.key_split, p.by_split.m, p.by_split.shift, p.by_blocks.m, p.by_blocks.shift, p.by_h.m, p.by_h.shift, p.n_row_blocks, p.H, p.row_stride, p.L,
+              p.n_keys, p.d, p.T, p.n_seg, p.plan, p.q, p.q_sb, p.q_sh, p.q_sl, p.k, p.k_sb, p.k_sh, p.k_sd, p.k_sl, p.out);
+    const int logical = xcd_remap(blockIdx.x, p.total);
     if (logical >= p.total) return;
-    const int share = logical % p.key_split, block = logical / p.key_split;
+    const int block = quotient(logical, p.by_split), share = logical - block * p.key_split;
     const int per_head = 2 * p.n_row_blocks;  // halves of the plan's row blocks
-    const int bh = block / per_head;
-    const int at_block = per_head - 1 - block % per_head;
+    const int bh = quotient(block, p.by_blocks);
+    const int at_block = per_head - 1 - (block - bh * per_head);
     const int rb = at_block >> 1, half = at_block & 1;
-    const int b = bh / p.H, h = bh % p.H;
+    const int b = quotient(bh, p.by_h), h = bh - b * p.H;
     const int rs = p.row_stride, L = p.L, d = p.d;
     const int r0 = block_first_row(rb, kPlanBM, rs) + rs * half * kHalfRows;
     if (r0 >= L) return;
@@ -107,7 +109,7 @@ __global__ __launch_bounds__(256, 4) void sddmm_rows16_kernel(const SddmmParams 
         }
         const SegPlan pl = walk.pl;
         const int tiles = walk.end - walk.tile;
-        const int first = walk.tile + tiles * share / p.key_split, end = walk.tile + tiles * (share + 1) / p.key_split;
+        const int first = walk.tile + quotient(tiles * share, p.by_split), end = walk.tile + quotient(tiles * (share + 1), p.by_split);
         if (first >= end) continue;
 
         u32x4 raw[NP];
@@ -204,6 +206,7 @@ int launch_sddmm_rows16(const SddmmParams& p0, int in_dtype, bool kt, hipStream_
     if (blocks > most && !fills) return 0;
     p.key_split = (int)std::min<int64_t>((p.T + kTile - 1) / kTile + 2, std::max<int64_t>(1, 512 / blocks));
     p.total = (int)(blocks * p.key_split);
+    p.by_split = divisor(p.key_split), p.by_blocks = divisor(2 * p.n_row_blocks), p.by_h = divisor(p.H);
     const int grid = ((p.total + 7) / 8) * 8;
     auto go = [&](auto t, auto kt_c) {
         using T = decltype(t);

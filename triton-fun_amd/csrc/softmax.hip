@@ -77,7 +77,8 @@ constexpr float kNegBig = -1.0e30f;
 // SHIFT: T is not a multiple of 8, so row r begins (r * T) % 8 elements into an aligned chunk.
 template <typename Tin, typename Tout, int NCH, int LPR, int RIF, bool SHIFT>
 __global__ __launch_bounds__(256) void softmax_rows_vec(const Tin* __restrict__ x, Tout* __restrict__ y, SoftmaxSegs segs,
-                                                        int64_t n_rows, int L, int T) {
+                                                        int64_t n_rows, int L, int T, Divisor by_l) {
+    load_args(x, y, n_rows, L, T, by_l.m, by_l.shift, segs.n, segs.nnz[0], segs.off[0]);
     typedef typename Vec8<Tin>::type vin;
     typedef typename Vec8<Tout>::type vout;
     constexpr int RPW = 64 / LPR;  // rows per wavefront and group
@@ -131,7 +132,7 @@ __global__ __launch_bounds__(256) void softmax_rows_vec(const Tin* __restrict__ 
     LiveRanges lr[RIF];
 #pragma unroll
     for (int i = 0; i < RIF; ++i)
-        lr[i].request(segs, n_rows < ((int64_t)1 << 32) ? (int)((uint32_t)row[i] % (uint32_t)L) : (int)(row[i] % L));
+        lr[i].request(segs, n_rows < ((int64_t)1 << 31) ? (int)row[i] - quotient((int)row[i], by_l) * L : (int)(row[i] % L));
 #pragma unroll
     for (int i = 0; i < RIF; ++i) {
         lr[i].set(segs, T);
@@ -252,38 +253,39 @@ static int launch_softmax(const void* x, void* y, const SoftmaxSegs& segs, int64
     const bool aligned = ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 31) == 0;
     const Tin* xi = (const Tin*)x;
     Tout* yo = (Tout*)y;
+    const Divisor by_l = divisor(L);
     if (aligned && (T & 7) != 0 && T <= 2032) {
         // rows that start anywhere in a chunk: up to T/8 + 2 chunks cover one
         const int chunks = T / 8 + 2;
         auto groups = [&](int rows_per_wave) { return (unsigned)((n_rows + 4 * rows_per_wave - 1) / (4 * rows_per_wave)); };
         if (chunks <= 16)
-            softmax_rows_vec<Tin, Tout, 1, 16, 1, true><<<groups(4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T);
+            softmax_rows_vec<Tin, Tout, 1, 16, 1, true><<<groups(4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
         else if (chunks <= 32)
             // 8 lanes and four chunks per row, eight rows per wavefront: the per-row work (live counts, masks, two
             // reductions, the element-wise stores at a row's ends) is what such short rows cost, and eight rows share
             // every instruction of it (+46 % over 32 lanes per row at T = 191)
-            softmax_rows_vec<Tin, Tout, 4, 8, 1, true><<<groups(8), 256, 0, st>>>(xi, yo, segs, n_rows, L, T);
+            softmax_rows_vec<Tin, Tout, 4, 8, 1, true><<<groups(8), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
         else if (chunks <= 64)
-            softmax_rows_vec<Tin, Tout, 1, 64, 4, true><<<groups(4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T);
+            softmax_rows_vec<Tin, Tout, 1, 64, 4, true><<<groups(4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
         else if (chunks <= 128)
-            softmax_rows_vec<Tin, Tout, 2, 64, 1, true><<<groups(1), 256, 0, st>>>(xi, yo, segs, n_rows, L, T);
+            softmax_rows_vec<Tin, Tout, 2, 64, 1, true><<<groups(1), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
         else
-            softmax_rows_vec<Tin, Tout, 4, 64, 1, true><<<groups(1), 256, 0, st>>>(xi, yo, segs, n_rows, L, T);
+            softmax_rows_vec<Tin, Tout, 4, 64, 1, true><<<groups(1), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
     } else if (aligned && (T & 7) == 0 && T <= 2048) {
         const int nch = (T / 8 + 63) / 64;
         // row groups in flight per wavefront: 4 where a row is 512 bytes or more (+7 % at T = 512, +4 % at T = 256 over
         // one group, measured), one for shorter rows (more was slower there)
         auto groups = [&](int rows_per_wave) { return (unsigned)((n_rows + 4 * rows_per_wave - 1) / (4 * rows_per_wave)); };
         if (T <= 128)
-            softmax_rows_vec<Tin, Tout, 1, 16, 1, false><<<groups(4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T);
+            softmax_rows_vec<Tin, Tout, 1, 16, 1, false><<<groups(4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
         else if (T <= 256)
-            softmax_rows_vec<Tin, Tout, 1, 32, 4, false><<<groups(2 * 4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T);
+            softmax_rows_vec<Tin, Tout, 1, 32, 4, false><<<groups(2 * 4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
         else if (nch <= 1)
-            softmax_rows_vec<Tin, Tout, 1, 64, 4, false><<<groups(4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T);
+            softmax_rows_vec<Tin, Tout, 1, 64, 4, false><<<groups(4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
         else if (nch <= 2)
-            softmax_rows_vec<Tin, Tout, 2, 64, 1, false><<<groups(1), 256, 0, st>>>(xi, yo, segs, n_rows, L, T);
+            softmax_rows_vec<Tin, Tout, 2, 64, 1, false><<<groups(1), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
         else
-            softmax_rows_vec<Tin, Tout, 4, 64, 1, false><<<groups(1), 256, 0, st>>>(xi, yo, segs, n_rows, L, T);
+            softmax_rows_vec<Tin, Tout, 4, 64, 1, false><<<groups(1), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
     } else {
         softmax_rows_any<Tin, Tout><<<grid, 256, 0, st>>>(xi, yo, segs, n_rows, L, T);
     }

@@ -176,6 +176,35 @@ __device__ __forceinline__ RowMap load_row_map(const float* sTod_lin, const floa
     return m;
 }
 
+// Division by a number that the host knows: n / d is the high part of one product, for every 0 <= n < 2^31 (Granlund and Montgomery,
+// "Division by Invariant Integers using Multiplication", 1994).  A kernel's own division by one of its arguments takes some forty
+// instructions, two of them at the beginning of every workgroup; with load_args below, 16-bit forward of 16 heads of 576 rows, d = 128, window 64
+// 6.85 -> 6.40 us, 12 heads of 1037 12.05 -> 11.57, 64 of 4096 at d = 64 44.2 -> 42.9; one float32 head of 512 rows 8.74 -> 8.34; the three
+// operators, 128 heads of 958 rows of 39 slots, 43.6 -> 41.3 (whose softmax divides once a row in every lane).
+struct Divisor {
+    uint32_t m;
+    int32_t shift;
+};
+inline Divisor divisor(int64_t d) {
+    int l = 0;
+    while (((int64_t)1 << l) < d) ++l;
+    return Divisor{(uint32_t)((((uint64_t)1 << (31 + l)) + d - 1) / d), 31 + l};
+}
+__device__ __forceinline__ int quotient(int n, Divisor d) { return (int)(((uint64_t)(uint32_t)n * d.m) >> d.shift); }
+
+// Kernel arguments that are wanted now, in one round of loads.  Left to itself the compiler loads them where they are used, and a
+// workgroup that has a CU to itself waits some 400 cycles for each of four or five rounds before its first operand is requested.
+template <typename A>
+__device__ __forceinline__ void load_arg(A a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" ::"s"(a));
+#endif
+}
+template <typename... A>
+__device__ __forceinline__ void load_args(A... a) {
+    (load_arg(a), ...);
+}
+
 // Workgroup barrier that hands LDS contents over and nothing else: it waits for this wavefront's LDS traffic, not for
 // its global loads and stores.  __syncthreads() waits for both counters, which serialises a kernel whose loads of the
 // next tile or stores of the previous one are meant to stay in flight across the barrier.  (The empty statements keep
@@ -188,9 +217,9 @@ __device__ __forceinline__ void lds_barrier() {
 
 // Map a launch-order workgroup id onto a logical id so that logically consecutive ids run on the
 // same XCD (hardware deals consecutive workgroup ids round-robin over the 8 XCDs, each with its own
-// L2).  gridDim.x must be 8 * chunk; ids >= total are idle.
-__device__ __forceinline__ int xcd_remap(int wg, int grid) {
-    const int chunk = grid >> 3;
+// L2).  The grid is `total` rounded up to a multiple of 8; ids >= total are idle.
+__device__ __forceinline__ int xcd_remap(int wg, int total) {
+    const int chunk = (total + 7) >> 3;
     return (wg & 7) * chunk + (wg >> 3);
 }
 

@@ -122,7 +122,7 @@ __global__ __launch_bounds__(256, 2) void spmm_kernel(const SpmmParams p) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lm = lane & 31, g = lane >> 5;
 
-    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    const int logical = xcd_remap(blockIdx.x, p.total);
     if (logical >= p.total) return;
     const int cchunk = logical % p.n_col_chunks;
     const int rest = logical / p.n_col_chunks;
@@ -354,7 +354,7 @@ __global__ __launch_bounds__(256, 2) void spmm_t_kernel(const SpmmTParams p) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lm = lane & 31, g = lane >> 5;
 
-    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    const int logical = xcd_remap(blockIdx.x, p.total);
     if (logical >= p.total) return;
     const int cchunk = logical % p.n_col_chunks;
     const int rest = logical / p.n_col_chunks;

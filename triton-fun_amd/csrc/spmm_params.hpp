@@ -16,6 +16,7 @@ struct SpmmParams {
     int n_seg;
     SegPtrs seg[SPLAT_MAX_SEGMENTS];
     int n_row_blocks, total, n_col_chunks;
+    Divisor by_chunks, by_blocks, by_h;  // column chunks, row blocks per head, H: filled in by the launches that read them
     int v_vec;
     int row_stride;
     const PlanRec* plan;  // optional: the mask's plan table for 128-row blocks (gathered walks), else nullptr

@@ -60,7 +60,7 @@ __global__ __launch_bounds__(512, 4) void spmm_t_thin_kernel(const SpmmTParams p
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, g4 = lane >> 4;
 
-    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    const int logical = xcd_remap(blockIdx.x, p.total);
     if (logical >= p.total) return;
     const int bh = logical / p.n_row_blocks;
     const int rb = logical % p.n_row_blocks;
