@@ -1,0 +1,74 @@
+"""The 16-bit forward whose wavefronts share the keys of 32 rows (launches of few row blocks), against float64 around the numbers of tiles
+at which its wavefronts run out of work, get a second tile, or leave the end to fewer of them; with a plan and without."""
+import pytest
+import torch
+
+import acsr_helpers as A
+from r_attention import RegularAttention, attention_launcher
+
+pytestmark = pytest.mark.gpu
+
+
+def band(L, lo, hi, dev):
+    back = torch.arange(L)[:, None] - torch.arange(L)[None, :]
+    return ((back >= lo) & (back <= hi)).to(torch.uint8).to(dev)
+
+
+# 32 rows of a causal window of w see w + 31 positions, of which the walk may begin 7 early: 1, 2, 3, 4, 5, 8, 9, 16, 17 tiles of 32
+MASKS = {f"causal {w}": (lambda w: lambda L, dev: [A.causal_windowed_pattern(L, w - 1)])(w) for w in (1, 2, 34, 65, 90, 98, 130, 218, 226, 474, 490)}
+MASKS |= {
+    "dilated": lambda L, dev: [A.dilated_pattern(L, 50, 3)],
+    "strided": lambda L, dev: A.strided_patterns(L, 40, 16),             # a second segment of periodic columns
+    "bands": lambda L, dev: [band(L, 0, 40, dev), band(L, 200, 330, dev)],  # a second segment that begins with rows of nothing
+    "far only": lambda L, dev: A.strided_patterns(L, 9, 7)[1:],           # the first rows hold nothing
+}
+
+
+@pytest.mark.parametrize("name", MASKS)
+@pytest.mark.parametrize("H", [3, 12])  # eight and four wavefronts a workgroup
+@pytest.mark.parametrize("dtype,d", [(torch.float16, 64), (torch.bfloat16, 64), (torch.float16, 128), (torch.bfloat16, 128)])
+def test_against_float64(dev, name, H, dtype, d):
+    L, B = 1001, 1
+    masks = MASKS[name](L, dev)
+    g = torch.Generator().manual_seed(d + H)
+    q, k, v = (torch.randn(B, H, L, d, generator=g).to(dtype).to(dev) for _ in range(3))
+    live = sum(m if torch.is_tensor(m) else m.device_mask(dev) for m in masks) > 0
+    s = (q.double() @ k.double().transpose(2, 3) * d ** -0.5).masked_fill(~live, float("-inf"))
+    p = torch.where(live.any(1)[:, None], torch.softmax(s, -1), torch.zeros_like(s))
+    ref = p @ v.double()
+    attn = RegularAttention(B, L, H, d, masks, 16, 16, dev, dtype, scale=d ** -0.5)
+    first = attn([q, k.transpose(2, 3), v]).clone()
+    for kT in (k.transpose(2, 3), k.transpose(2, 3).contiguous()):
+        got, lse = attn.forward_with_stats([q, kT, v])
+        # probabilities are rounded to the type once: half an ulp of it (2^-11, 2^-8), relative
+        assert float((got.double() - ref).norm() / ref.norm()) <= (5e-4 if dtype == torch.float16 else 4e-3)
+        assert torch.allclose(lse.double().view(B, H, L), torch.logsumexp(s, -1).nan_to_num(neginf=float("inf")), atol=2e-6 * d, rtol=1e-6)
+    # without a plan the workgroups find the same walks
+    bare = attention_launcher(q, k.transpose(2, 3), v, torch.empty_like(q), attn.segments, attn.scale)
+    assert torch.equal(bare, first)
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.float16, 64), (torch.bfloat16, 128)])
+def test_values_that_no_row_sees_do_not_matter(dev, dtype, d):
+    """A cache that is filled up to row n, NaN behind: the rows up to there are what they are without it."""
+    L, n, B, H = 512, 320, 1, 2
+    g = torch.Generator(device=dev).manual_seed(d)
+    q, k, v = (torch.randn(B, H, L, d, generator=g, device=dev).to(dtype) for _ in range(3))
+    attn = RegularAttention(B, L, H, d, A.causal_windowed_pattern(L, 99), 16, 16, dev, dtype, scale=d ** -0.5)
+    want = attn([q, k.transpose(2, 3), v])[:, :, :n].clone()
+    k[:, :, n:], v[:, :, n:] = float("nan"), float("nan")
+    assert torch.equal(attn([q, k.transpose(2, 3), v])[:, :, :n], want)
+
+
+@pytest.mark.parametrize("H,kt,same", [(224, False, True), (225, False, False), (192, True, True), (193, True, False)])
+def test_the_line_at_d64(dev, H, kt, same):
+    """Launches of 129 row blocks and more come here where some of the walk is dead; equal bits say which kernel ran."""
+    L, d, dtype = 128, 64, torch.bfloat16
+    g = torch.Generator(device=dev).manual_seed(H)
+    q, k, v = (torch.randn(1, H, L, d, generator=g, device=dev).to(dtype) for _ in range(3))
+    attn = RegularAttention(1, L, H, d, A.causal_windowed_pattern(L, 99), 16, 16, dev, dtype, scale=d ** -0.5)
+    whole = attn([q, k.transpose(2, 3).contiguous() if kt else k.transpose(2, 3), v]).clone()
+    few = RegularAttention(1, L, 100, d, A.causal_windowed_pattern(L, 99), 16, 16, dev, dtype, scale=d ** -0.5)
+    part = few([q[:, :100], k[:, :100].transpose(2, 3), v[:, :100]])
+    assert torch.equal(whole[:, :100], part) == same
+    assert float((whole[:, :100].float() - part.float()).norm() / part.float().norm()) <= 4e-3

@@ -20,63 +20,13 @@
 // gathered rows of K/V) and validity is a per-row range test in j; otherwise tiles are dense columns
 // and validity is the full affine test (offset, step divisibility, count).  Each wavefront skips tiles (d = 64: halves of tiles)
 // that lie outside all of its rows' spans and drops the mask on tiles inside all of them.
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
 #include "attn_tile.hpp"
 
 namespace splat {
-
-// Exponentials of one tile of scores against the rows' references (mb = reference * c2), as MFMA B fragments; returns
-// the lane's sum.
-template <int NT, typename T>
-__device__ __forceinline__ float exp_tile(const f32x16 (&s)[NT], Frag<T> (&pf)[NT][2], float mb, float c2) {
-    float rs = 0.f;
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const float pv = fast_exp2(fmaf(s[nt][j], c2, -mb));
-            rs += pv;
-            pf[nt][j >> 3].v[j & 7] = (T)pv;
-        }
-    return rs;
-}
-
-// Fold one tile of 32*NT keys of (masked) scores of one 32-row tile into the running softmax state and emit the
-// exponentials.  One lane owns one query row (half of its positions).  Returns whether every row of the wavefront
-// has a real reference afterwards.
-template <int NT, typename T, int DT>
-__device__ __forceinline__ bool softmax_tile(f32x16 (&s)[NT], Frag<T> (&pf)[NT][2], float& m_ref, float& l_run,
-                                             f32x16 (&o)[DT], float c2) {
-    float mx = s[0][0];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) mx = fmaxf(mx, s[nt][j]);
-    mx = with_lane_xor<32, 64>(mx, [](float a, float b) { return fmaxf(a, b); });  // the other half of the row lives in lane ^ 32
-    // move the reference only when some row's maximum has outrun it by the threshold (always on the first
-    // live tile); rows that do not move keep alpha = 1
-    if (__any((mx - m_ref) * c2 > kRescaleThreshold)) {
-        const float m_new = ((mx - m_ref) * c2 > kRescaleThreshold) ? mx : m_ref;
-        const float alpha = fast_exp2((m_ref - m_new) * c2);
-        const bool had_data = __any(m_ref > 0.5f * kNegBigA);  // otherwise O and l are still all zero
-        m_ref = m_new;
-        if (had_data) {
-            l_run *= alpha;
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-                for (int j = 0; j < 16; ++j) o[dt][j] *= alpha;
-        }
-    }
-    // Masked scores are -1e30: their exponential underflows to exactly 0 as long as the reference is a real
-    // score.  A row that has seen no live score yet keeps the -1e30 reference; give it offset 0 so that its
-    // (all masked) entries still map to 0 instead of exp2(0).
-    const bool real = m_ref > 0.5f * kNegBigA;
-    l_run += exp_tile<NT, T>(s, pf, real ? m_ref * c2 : 0.f, c2);
-    return !__any(!real);
-}
 
 template <typename T, int D, bool KT, int BN, int NSTAGE, bool PLANNED>
 __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnParams p) {
@@ -579,15 +529,24 @@ static int launch_attn(const AttnParams& p0, hipStream_t st) {
 // kernel also supports 32-key tiles in a ring of 4 stages; it measured slower at d = 128 and equal at d = 64).
 template <typename T>
 static int dispatch_attn(const AttnParams& p, int d, bool kt, hipStream_t st) {
-    // Few row blocks: the kernel of 16 rows a wavefront (attention_rows16.hip), two workgroups per row block.  Up to 128 row blocks
-    // every workgroup has a CU to itself and it is the faster one whatever the mask: bf16, 128 blocks, 32x32x16 kernel -> this one,
-    // window 32 / 512 / blocks of 2048: d = 64 7.4 -> 5.3, 13.8 -> 10.9, 60.5 -> 52.6 us, d = 128 9.1 -> 6.6, 17.4 -> 14.4, 80.4 -> 73.8.
-    // Beyond that workgroups share a CU's LDS, from which this kernel reads every operand for half the rows: it wins where it skips
-    // masked positions and loses where there are none.  The line lies at three quarters of the walked positions live and 320 (192 at
-    // d = 128) blocks: at 192 blocks, d = 64, windows 128 / 320 (half, 72 % live) 8.5 -> 7.7, 11.1 -> 10.5 us, window 512 (80 %)
-    // 13.9 -> 13.4, blocks of 256 (all) 11.4 -> 12.4; d = 128 10.4 -> 9.4, 13.9 -> 13.6, 17.5 -> 17.7, 14.4 -> 16.9; at 384 blocks,
-    // d = 64, window 256 with K^T along the keys 12.1 -> 12.4.
+    // Few row blocks: the kernel whose wavefronts share the keys of 32 rows (attention_shared.hip), eight of them where every workgroup
+    // has a CU to itself anyway, else four, two or four workgroups a CU.  It wins as long as its workgroups are on the chip together: 128
+    // blocks at d = 128 (at 192 and window 200 11.9 -> 13.0 us), at d = 64 some 256, less for K^T and for walks that are live throughout.  bf16,
+    // causal windows of 40 / 200 / 800, before -> with it: d = 64, 64 blocks 5.6 -> 4.6, 8.0 -> 5.1, 15.5 -> 6.7, 128 blocks 5.6 -> 4.9, 8.0 -> 5.7,
+    // 15.5 -> 9.6, 192 blocks 6.7 -> 5.7, 9.9 -> 7.0, 17.6 -> 12.5, 256 blocks 6.8 -> 6.4, 10.1 -> 8.2, 17.7 -> 15.6 (blocks of 256 keys 7.8 -> 8.1, K^T and
+    // window 101 8.0 -> 9.3); d = 128, 64 blocks 6.5 -> 5.2, 9.7 -> 6.4, 19.6 -> 8.9, 128 blocks 6.8 -> 6.3, 10.0 -> 7.9, 19.9 -> 13.7.  Eight
+    // against four wavefronts, 64 blocks, windows 200 / 400 / 800: d = 64 5.1 / 5.9 / 6.7 against 4.9 / 6.2 / 8.0, d = 128 6.4 / 7.3 / 8.9 against
+    // 6.3 / 8.1 / 10.5.
     const int64_t blocks = (int64_t)p.B * p.H * count_row_blocks(p.L, kPlanBM, p.row_stride);
+    const bool narrow = std::max(p.v_sl, kt ? 0 : p.k_sl) * 2 < (1 << 24) && std::max(p.v_sl, kt ? 0 : p.k_sl) * 2 * p.L < ((int64_t)1 << 32);
+    if (narrow && (blocks <= 128 || (d == 64 && p.live_percent > 0 && p.live_percent <= 90 && blocks <= (kt ? 192 : 224))))
+        return launch_attn_shared<T>(p, d, kt, blocks <= 64 ? 8 : 4, st);
+    // Some more: the kernel of 16 rows a wavefront (attention_rows16.hip), two workgroups per row block, which reads every operand from
+    // LDS for half the rows: it wins where it skips masked positions and loses where there are none.  The line lies at three quarters of the
+    // walked positions live and 320 (192 at d = 128) blocks: at 192 blocks, d = 64, windows 128 / 320 (half, 72 % live) 8.5 -> 7.7, 11.1 -> 10.5
+    // us, window 512 (80 %) 13.9 -> 13.4, blocks of 256 (all) 11.4 -> 12.4; d = 128 10.4 -> 9.4, 13.9 -> 13.6, 17.5 -> 17.7, 14.4 -> 16.9; at 384
+    // blocks, d = 64, window 256 with K^T along the keys 12.1 -> 12.4.  (Up to 128 blocks it is the faster one of the two whatever the mask,
+    // for rows too far apart for the other's offsets.)
     if (blocks <= 128 || (p.live_percent > 0 && p.live_percent <= 75 && blocks <= (d == 64 ? 320 : 192)))
         return launch_attn_rows16<T>(p, d, kt, st);
     if (p.keys_anywhere) return fail(SPLAT_E_UNSUPPORTED, "splat_attention_fwd_keys: this launch copies K in whole 16-byte pieces");

@@ -1,4 +1,5 @@
-// Fused ACSR sparse-attention forward for 16-bit types in launches of few row blocks, gfx950.
+// Fused ACSR sparse-attention forward for 16-bit types in launches of too many row blocks for attention_shared.hip that still leave the
+// chip part idle, gfx950.
 //
 // Bound: latency.  A launch of the kernel in attention.hip (128 rows a workgroup, 32 a wavefront, tiles of 64 keys one ahead)
 // that does not fill the chip takes as long as one of its workgroups: the chain kernel arguments -> plan -> first tile, then
@@ -148,18 +149,8 @@ __global__ __launch_bounds__(256, LAYOUT == kKeysAnywhere && D == 128 ? 2 : 3) v
         const int c0 = w.pl.c0 + w.tile * BN;
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
-            const int flat = tid + 256 * i, c = c0 + 8 * (flat % K_CPR);
-            const int over = min(max(c + 8 - L, 0), 8);  // keys of the piece that do not exist: the row's last whole piece, moved down
-            u32x4 x;
-            __builtin_memcpy(&x, kb + (int64_t)(flat / K_CPR) * p.k_sd + min(c, L - 8), 16);
-            if (over > 0) {
-                const uint64_t lo = (uint64_t)x[1] << 32 | x[0], hi = (uint64_t)x[3] << 32 | x[2];
-                const int s = 16 * (over & 3);
-                const uint64_t a = over >= 4 ? hi : lo, b = over >= 4 ? 0 : hi;
-                const uint64_t l = s == 0 ? a : (a >> s) | (b << (64 - s)), h = b >> s;
-                x = u32x4{(uint32_t)l, (uint32_t)(l >> 32), (uint32_t)h, (uint32_t)(h >> 32)};
-            }
-            k_reg[i] = x;
+            const int flat = tid + 256 * i;
+            k_reg[i] = keys_piece(kb + (int64_t)(flat / K_CPR) * p.k_sd, c0 + 8 * (flat % K_CPR), L);
         }
     };
     auto store_keys = [&](int stage) {
