@@ -1,4 +1,4 @@
-"""The 16-bit forward whose wavefronts share the keys of 32 rows (launches of few row blocks), against float64 around the numbers of tiles
+"""The forwards whose wavefronts share the keys of their rows (launches of few row blocks), against float64 around the numbers of tiles
 at which its wavefronts run out of work, get a second tile, or leave the end to fewer of them; with a plan and without."""
 import pytest
 import torch
@@ -7,6 +7,11 @@ import acsr_helpers as A
 from r_attention import RegularAttention, attention_launcher
 
 pytestmark = pytest.mark.gpu
+
+
+# 16-bit types: probabilities are rounded to the type once, half an ulp of it (2^-11, 2^-8), relative.  float32: products are off by
+# less than 2^-24 of theirs, and so is every addition; four times what five of them in a row leave
+BOUNDS = {torch.float16: 5e-4, torch.bfloat16: 4e-3, torch.float32: 1.2e-6}
 
 
 def band(L, lo, hi, dev):
@@ -25,10 +30,12 @@ MASKS |= {
 
 
 @pytest.mark.parametrize("name", MASKS)
-@pytest.mark.parametrize("H", [3, 12])  # eight and four wavefronts a workgroup
-@pytest.mark.parametrize("dtype,d", [(torch.float16, 64), (torch.bfloat16, 64), (torch.float16, 128), (torch.bfloat16, 128)])
-def test_against_float64(dev, name, H, dtype, d):
+@pytest.mark.parametrize("few", [True, False])  # eight and four wavefronts of 32 rows (16-bit types), four of 16 and of 32 (float32)
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("dtype", BOUNDS)
+def test_against_float64(dev, name, few, dtype, d):
     L, B = 1001, 1
+    H = 3 if few else 6 if dtype == torch.float32 else 12
     masks = MASKS[name](L, dev)
     g = torch.Generator().manual_seed(d + H)
     q, k, v = (torch.randn(B, H, L, d, generator=g).to(dtype).to(dev) for _ in range(3))
@@ -40,15 +47,14 @@ def test_against_float64(dev, name, H, dtype, d):
     first = attn([q, k.transpose(2, 3), v]).clone()
     for kT in (k.transpose(2, 3), k.transpose(2, 3).contiguous()):
         got, lse = attn.forward_with_stats([q, kT, v])
-        # probabilities are rounded to the type once: half an ulp of it (2^-11, 2^-8), relative
-        assert float((got.double() - ref).norm() / ref.norm()) <= (5e-4 if dtype == torch.float16 else 4e-3)
+        assert float((got.double() - ref).norm() / ref.norm()) <= BOUNDS[dtype]
         assert torch.allclose(lse.double().view(B, H, L), torch.logsumexp(s, -1).nan_to_num(neginf=float("inf")), atol=2e-6 * d, rtol=1e-6)
-    # without a plan the workgroups find the same walks
-    bare = attention_launcher(q, k.transpose(2, 3), v, torch.empty_like(q), attn.segments, attn.scale)
+    # without a plan the workgroups find the same walks (the hint chooses the kernel in either)
+    bare = attention_launcher(q, k.transpose(2, 3), v, torch.empty_like(q), attn.segments, attn.scale, live_percent=attn._live_percent)
     assert torch.equal(bare, first)
 
 
-@pytest.mark.parametrize("dtype,d", [(torch.float16, 64), (torch.bfloat16, 128)])
+@pytest.mark.parametrize("dtype,d", [(torch.float16, 64), (torch.bfloat16, 128), (torch.float32, 64), (torch.float32, 128)])
 def test_values_that_no_row_sees_do_not_matter(dev, dtype, d):
     """A cache that is filled up to row n, NaN behind: the rows up to there are what they are without it."""
     L, n, B, H = 512, 320, 1, 2

@@ -11,14 +11,14 @@
 //     the third workgroup a CU (d = 64, 64 heads of 2048 rows, window 256 / 32: 72 / 35.4 us against 68 / 32.7; d = 128, of
 //     the second: 204 / 102 against 127 / 59), 128 rows a workgroup halve the splitting but leave one or two of them a CU
 //     (70 / 35.8 and 143 / 78), 32 rows a wavefront with the scores a tile ahead take 216 registers and run no faster.
-//   * 64 rows a workgroup, so that short problems spread over more CUs, and little that runs once: in a launch of few tiles the
-//     instructions of the beginning and the end come from memory (a barrier and a second pass for references that are left
-//     behind cost 1 of 8.6 us there).  Two groups of wavefronts that share the tiles of 64 rows and add up at the end: 14.4 for 16.3 at
-//     a window of 256 and one workgroup a CU, 8.1 for 7.6 at 32, and other bits for a walk that is planned than for one that is not.
+//   * 64 rows a workgroup, so that launches that fill the chip once or twice spread over more CUs (those that do not:
+//     attention_shared_f32.hip), and little that runs once: the instructions of the beginning and the end come from memory.
 // Measured against the kernel on the float32 instructions that it replaces: B = 32, H = 12, L = 1024, window 257, d = 64: 252 -> 197 us;
 // 64 heads of 4096 rows, blocks of 512, d = 64 517 -> 376; 64 heads of 2048 rows, d = 128, window 256 180 -> 127, window 32 66 -> 59;
 // one head of 512 rows, window 64: 9.5 -> 8.7.  Relative error against float64 (norms) 2.5e-7 -> 1.6e-7 there, 4.0e-7 -> 3.0e-7 at
 // window 257, 6.6e-7 -> 5.4e-7 at blocks of 1024 and d = 128.
+#include <algorithm>
+
 #include "rows16.hpp"
 #include "split3.hpp"
 
@@ -406,6 +406,17 @@ static int launch(const AttnParams& p0, hipStream_t st) {
 }
 
 int launch_attn_f32(const AttnParams& p, int d, bool kt, hipStream_t st) {
+    // Few row blocks: the kernel whose wavefronts share the keys (attention_shared_f32.hip), of 16 rows up to 32 blocks, of 32 up to 64: as
+    // long as its workgroups, one a CU or two at d = 64, are on the chip together.  This kernel -> that one, causal windows of 16 / 64 / 200 / 400:
+    // d = 64, 4 heads of 1024 rows 7.3 -> 5.6, 8.5 -> 6.0, 14.9 -> 7.8, 22.2 -> 10.6 us, 8 heads 7.4 -> 7.2, 8.6 -> 7.7, 15.0 -> 10.0, 22.0 -> 13.7, 10 heads
+    // 7.5 -> 9.8, 8.7 -> 10.3, 15.1 -> 14.4, 22.2 -> 20.5; d = 128, 4 heads 10.6 -> 8.0, 12.6 -> 8.8, 22.8 -> 12.2, 34.7 -> 17.4, 8 heads 10.8 -> 11.4 (a
+    // twelfth of the walk live: those stay), 12.8 -> 12.3, 23.1 -> 16.7, 34.7 -> 23.5.
+    const int64_t blocks = (int64_t)p.B * p.H * count_row_blocks(p.L, kPlanBM, p.row_stride);
+    const int64_t row_bytes = 4 * std::max(p.v_sl, kt ? 0 : p.k_sl);  // (that kernel's offsets)
+    if (row_bytes < (1 << 24) && row_bytes * p.L < ((int64_t)1 << 32)) {
+        if (blocks <= 32) return launch_attn_shared_f32(p, d, kt, 16, st);
+        if (blocks <= 64 && (d == 64 || p.live_percent == 0 || p.live_percent >= 20)) return launch_attn_shared_f32(p, d, kt, 32, st);
+    }
     if (p.plan) {
         if (d == 64) return kt ? launch<64, true, true>(p, st) : launch<64, false, true>(p, st);
         return kt ? launch<128, true, true>(p, st) : launch<128, false, true>(p, st);

@@ -33,6 +33,8 @@ constexpr float kRescaleThreshold = 8.0f;  // in log2 units: exponentials stay b
 
 // the float32 forward (attention_f32.hip); p.n_row_blocks and p.total are filled in by the launch
 int launch_attn_f32(const AttnParams& p, int d, bool kt, hipStream_t st);
+// the float32 forward whose wavefronts share the keys of 16 or 32 rows (attention_shared_f32.hip)
+int launch_attn_shared_f32(const AttnParams& p, int d, bool kt, int rows, hipStream_t st);
 // the 16-bit forward of 16 rows a wavefront (attention_rows16.hip)
 template <typename T>
 int launch_attn_rows16(const AttnParams& p, int d, bool kt, hipStream_t st);
