@@ -93,3 +93,30 @@ def test_running_out_of_memory_is_the_error_a_program_catches(dev):
         torch.cuda.set_per_process_memory_fraction(1.0, dev)
     got = torch.autograd.grad(out, x, up)
     assert all(torch.equal(a, b) for a, b in zip(got, want)) and len(fits) < 64
+
+
+@pytest.mark.parametrize("layout", ["rows", "tokens", "keys", "odd rows"])
+@pytest.mark.parametrize("L,masks", [(520, lambda L: A.causal_windowed_pattern(L, 99)), (384, lambda L: A.strided_patterns(L, 32, 16)),
+                                     (301, lambda L: A.dilated_pattern(L, 20, 3))])
+@pytest.mark.parametrize("dtype,d", [(torch.float32, 64), (torch.bfloat16, 64), (torch.float16, 80)])
+def test_native_operators_equal_the_launchers(dev, layout, L, masks, dtype, d):
+    """The first forward goes through the three launchers, the next ones through one native call; a layout that comes later goes
+    through the launchers first again, and other types are theirs to refuse."""
+    B, H = 2, 3
+    attn = RegularAttention(B, L, H, d, masks(L), 16, 16, dev, dtype, scale=d ** -0.5, fused=False)
+    q, _, kT, v = _operands(dev, B, H, L, d, dtype, layout)
+    want = [t.clone() for t in (attn([q, kT, v]), attn.rsddmm_output, attn.rsoftmax_output)]
+    kept = attn._operator_masks
+    taken = hip.host().operators(*kept, q, kT, v, attn._rsddmm_output, attn._rsoftmax_output, attn.rspmm_output.zero_(), attn.scale)
+    assert taken and torch.equal(attn.rspmm_output, want[0])
+    live = (torch.arange(attn.acsr_trailing_dim, device=dev) < sum(t[4] for t in attn.segments.tuples)[:, None]) if len(attn.segments) == 1 else None
+    assert torch.equal(attn([q, kT, v]), want[0])
+    if live is not None:
+        for got, w in zip((attn.rsddmm_output, attn.rsoftmax_output), want[1:]):
+            assert torch.equal(got[:, :, live], w[:, :, live])
+    other = kT.contiguous() if layout != "keys" else kT.transpose(2, 3).contiguous().transpose(2, 3)
+    assert None in attn._operator_masks[:2]
+    assert float((attn([q, other, v]).float() - want[0].float()).abs().max()) <= 0.04
+    assert None not in attn._operator_masks[:2] and torch.equal(attn([q, kT, v]), want[0])
+    with pytest.raises(hip.SplatError):
+        attn([q.double(), kT.double(), v.double()])

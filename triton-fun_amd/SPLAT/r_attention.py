@@ -21,9 +21,9 @@ import torch.nn as nn
 import _splat_hip as _hip
 from acsr_helpers import (ACSRSegments, MaskPattern, create_acsr, create_acsr_segments, create_blocked_mask,  # noqa: F401
                           create_causal_windowed_mask, create_windowed_mask, mask_shape, transpose_keys)
-from r_sddmm import rsddmm_launcher, rsddmm_preamble
+from r_sddmm import native_mask as sddmm_mask, rsddmm_launcher, rsddmm_preamble
 from r_softmax import rsoftmax_launcher, rsoftmax_preamble
-from r_spmm import rspmm_launcher, rspmm_preamble
+from r_spmm import native_mask as spmm_mask, rspmm_launcher, rspmm_preamble
 
 
 def _is_segment_list(mask) -> bool:
@@ -112,6 +112,7 @@ def attention_launcher(q: torch.Tensor, kT: torch.Tensor, v: torch.Tensor, outpu
 
 
 class RegularAttention(nn.Module):
+    _operator_masks = None  # as the native call of all three operators takes them: kept by the first forward through the launchers
 
     def __init__(self, batch: int, seq_length: int, num_heads: int, head_dim: int, mask,
                  BLOCK_SIZE_Y: int, BLOCK_SIZE_X: int, GPU_ID: Any, out_dtype: torch.dtype,
@@ -203,6 +204,10 @@ class RegularAttention(nn.Module):
             self._ensure_plan()
             return attention_launcher(q, k, v, self.rspmm_output, self.segments, self.scale, self._plan, live_percent=self._live_percent)
 
+        masks = self._operator_masks
+        if masks is not None and _hip.host().operators(*masks, q, k, v, self._rsddmm_output, self._rsoftmax_output, self.rspmm_output,
+                                                       self.scale):
+            return self.rspmm_output
         multi = self.segments  # (also for one segment: the object keeps what every call would otherwise rebuild and recheck)
         rsddmm_launcher(q, k, self.rsddmm_output,
                         self.dTos_linear_transformations, self.dTos_translations,
@@ -220,7 +225,18 @@ class RegularAttention(nn.Module):
                        self.sTod_linear_transformations, self.sTod_translations,
                        self.span_loop_start, self.span_loop_end, self.acsr_trailing_dim,
                        self.nnzs, self.rspmm_grid_dim, self.BLOCK_SIZE_Y, self.BLOCK_SIZE_X, segments=multi)
+        self._keep_operators(q, k)
         return self.rspmm_output
+
+    def _keep_operators(self, q, k):
+        """The masks that the launchers of a forward like this one have used, for the native call of all three."""
+        if q.dtype != self._out_dtype or q.shape[3] != self._shape[3] or torch.cuda.is_current_stream_capturing():
+            return
+        segs, rows = self.segments, k.stride(2) == 1
+        mask = sddmm_mask(segs, q, k, self._rsddmm_output)
+        of_rows, of_keys, *_ = self._operator_masks or (None, None)
+        self._operator_masks = (mask if rows else of_rows, of_keys if rows else mask, segs.native(self._shape[2], self._device, False),
+                                spmm_mask(segs, self._rsoftmax_output, self.rspmm_output))
 
     def _ensure_plan(self):
         """The fused kernel's plan of this mask, and the mask as the native host path takes it."""

@@ -76,6 +76,16 @@ def _takes_a_plan(x, output, blocks: int, d: int, k_rows: bool, T: int) -> bool:
             and output.dtype == x.dtype)
 
 
+def native_mask(segs: ACSRSegments, x: torch.Tensor, y: torch.Tensor, output: torch.Tensor):
+    """The mask as the native host path takes it for this launch, with the plan table where the launch reads it."""
+    B, H, L, d = x.shape
+    blocks = B * H * ((L + 127) // 128)
+    # (launches that read the table: rows of K, those that gather, and, up to d = 64, those of at least 64 row blocks, for which the
+    # native path turns K first or whose kernel turns it: csrc/host_ext.cpp)
+    k_rows = y.stride(2) == 1 or (d <= 64 and blocks >= 64) or segs.gathered
+    return segs.native(L, x.device, _takes_a_plan(x, output, blocks, d, k_rows, output.shape[-1]))
+
+
 def rsddmm_launcher(x: torch.Tensor, y: torch.Tensor, output: torch.Tensor,
                     dTos_linear_transformations: torch.Tensor, dTos_translations: torch.Tensor,
                     sTod_linear_transformations: torch.Tensor, sTod_translations: torch.Tensor,
@@ -103,12 +113,7 @@ def rsddmm_launcher(x: torch.Tensor, y: torch.Tensor, output: torch.Tensor,
     segs = segments or ACSRSegments.single(dTos_linear_transformations, dTos_translations,
                                            sTod_linear_transformations, sTod_translations, nnzs, trailing_dim)
     if plan is None and x.dim() == 4 and y.dim() == 4 and output.shape[-1] == trailing_dim:
-        B, H, L, d = x.shape
-        blocks = B * H * ((L + 127) // 128)
-        # (launches that read the table: rows of K, those that gather, and, up to d = 64, those of at least 64 row blocks, for which the
-        # native path turns K first or whose kernel turns it: csrc/host_ext.cpp)
-        k_rows = y.stride(2) == 1 or (d <= 64 and blocks >= 64) or segs.gathered
-        mask = segs.native(L, x.device, _takes_a_plan(x, output, blocks, d, k_rows, trailing_dim))
+        mask = native_mask(segs, x, y, output)
         if mask is not None and _hip.host().sddmm(mask, x, y, output, 1.0 if scale is None else scale, lse):
             return (output, sTod_linear_transformations, sTod_translations, nnzs)
     B, H, L, d = x.shape

@@ -27,6 +27,11 @@ def _takes_a_plan(x, output, n_out: int, segs: ACSRSegments) -> bool:
     return x.shape[3] < 256 or segs.plan_is_aligned(x.shape[2], x.device) is False
 
 
+def native_mask(segs: ACSRSegments, x: torch.Tensor, output: torch.Tensor):
+    """The mask as the native host path takes it for this launch, with the plan table where the launch is faster with it."""
+    return segs.native(x.shape[2], x.device, _takes_a_plan(x, output, output.shape[3], segs))
+
+
 def rspmm_preamble(mask, output_shape: tuple[int], BLOCK_SIZE_X: int, BLOCK_SIZE_Y: int, GPU_ID: Any,
                    output_dtype: torch.dtype) -> tuple[torch.Tensor, tuple[int], int]:
     """-> (output [B, H, L, n] uninitialised, grid_dim = (ceil(n / BSX), ceil(L / BSY), B*H), T = max row nnz)."""
@@ -72,13 +77,12 @@ def rspmm_launcher(x: torch.Tensor, y: torch.Tensor, output: torch.Tensor,
                                            sTod_linear_transformations, sTod_translations, nnzs, acsr_trailing_dim)
     vs = y.stride()
     dev = x.device
-    tabled = plan is None and _takes_a_plan(x, output, n_out, segs)
     if plan is None:
-        mask = segs.native(L, dev, tabled)
+        mask = native_mask(segs, x, output)
         if mask is not None and _hip.host().spmm(mask, x, y, output):
             return (output, sTod_linear_transformations, sTod_translations, nnzs)
     arr = segs.seg_array(L, T)
-    if tabled and (segs.has_plan(L, dev) or not torch.cuda.is_current_stream_capturing()):
+    if plan is None and _takes_a_plan(x, output, n_out, segs) and (segs.has_plan(L, dev) or not torch.cuda.is_current_stream_capturing()):
         plan = segs.plan(L, dev)  # (no table is built under stream capture: building synchronises)
     if plan is not None and plan is not False:
         _hip.require_device_tensor(plan, "plan")

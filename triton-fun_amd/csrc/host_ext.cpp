@@ -532,6 +532,29 @@ PyObject* py_spmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
 }
 
+// operators(mask | None, mask | None, mask, mask, q, kT, v, scores, probabilities, out, scale) -> bool: the three operators of one forward.  The
+// masks are those of the sampled product, for rows of K and for K along the keys, of the softmax and of the last product.  What the
+// interpreter does between three calls costs more than the launches (22 -> 12.6 us on the host), and than the kernels of a few row
+// blocks (40 heads of 256 rows, 62 slots, bfloat16, d = 64: 20.1 -> 13.6 us a forward).  False: some
+// operand is not an ordinary one, and the launchers take the whole forward (what has been launched is computed again).
+PyObject* py_operators(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 11) return PyErr_Format(PyExc_TypeError, "operators takes 11 arguments");
+    const int dev = c10::hip::current_device();
+    const at::Tensor *q = tensor4(a[4], dev), *kT = tensor4(a[5], dev), *out = tensor4(a[9], dev);
+    // (the masks were chosen for the output's type and head dimension)
+    if (!q || !kT || !out || q->scalar_type() != out->scalar_type() || q->size(3) != out->size(3)) Py_RETURN_FALSE;
+    PyObject* const mask = a[kT->stride(2) == 1 ? 0 : 1];
+    if (mask == Py_None) Py_RETURN_FALSE;
+    PyObject* const first[] = {mask, a[4], a[5], a[7], a[10], Py_None};
+    PyObject* const second[] = {a[2], a[7], a[8]};
+    PyObject* const third[] = {a[3], a[8], a[6], a[9]};
+    PyObject* did = py_sddmm(nullptr, first, 6);
+    if (did != Py_True) return did;
+    did = py_softmax(nullptr, second, 3);
+    if (did != Py_True) return did;
+    return py_spmm(nullptr, third, 4);
+}
+
 // ---- the ACSR and the plan of a mask ---------------------------------------------------------------------------------------------
 constexpr int64_t kShareBlocks = 1024;  // row blocks of a build whose shares of the summary a kept buffer holds
 
@@ -738,6 +761,7 @@ PyMethodDef methods[] = {
     {"sddmm", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_sddmm)), METH_FASTCALL, "sampled product"},
     {"softmax", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_softmax)), METH_FASTCALL, "softmax of compressed rows"},
     {"spmm", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_spmm)), METH_FASTCALL, "compressed rows times dense"},
+    {"operators", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_operators)), METH_FASTCALL, "the three of them"},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_splat_host", nullptr, -1, methods};
 
