@@ -1,5 +1,5 @@
-"""The backward's keys' side by pairs of wavefronts (d = 128, launches of at most 1024 row blocks) against float64 where its
-halves, stages and exchange can go wrong, and the two sides of the line at which the dispatch changes kernels."""
+"""The backward's keys' side by pairs of wavefronts against float64 where its halves, stages and exchange can go wrong, and large
+launches of it against larger ones."""
 import pytest
 import torch
 
@@ -28,8 +28,9 @@ def step(masks, q, k, v, grad, dev, dtype):
 @pytest.mark.parametrize("name", MASKS)
 @pytest.mark.parametrize("L", [17, 33, 64, 65, 129, 200, 520])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_against_float64(dev, name, L, dtype):
-    masks, B, H, d = MASKS[name](L), 1, 2, 128
+@pytest.mark.parametrize("d", [128, 64])
+def test_against_float64(dev, name, L, dtype, d):
+    masks, B, H = MASKS[name](L), 1, 2
     g = torch.Generator().manual_seed(L)
     q, k, v, grad = (torch.randn(B, H, L, d, generator=g).to(dtype) for _ in range(4))
     live = sum(m.device_mask(dev) for m in masks).cpu() > 0
@@ -46,7 +47,7 @@ def test_against_float64(dev, name, L, dtype):
 
 
 def test_both_sides_of_the_line(dev):
-    """1024 heads of one row block go to this kernel, one head more to the other two: the shared heads agree."""
+    """1024 heads of one row block, and one head more: the shared heads agree."""
     most, L, d, dtype = 1024, 128, 128, torch.bfloat16
     g = torch.Generator(device=dev).manual_seed(5)
     q, k, v, grad = (torch.randn(1, most + 1, L, d, generator=g, device=dev).to(dtype) for _ in range(4))

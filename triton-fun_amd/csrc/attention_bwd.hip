@@ -3,33 +3,24 @@
 // With S = scale * Q K^T on the live columns, P = exp(S - lse) (lse: the forward's row statistic), O = P V and the
 // upstream gradient dO:  D = rowsum(dO * O),  dP = dO V^T,  dS = P * (dP - D),
 //     dQ = scale * dS K        dK = scale * dS^T Q        dV = P^T dO.
-// One kernel, four modes (d = 128: dQ, dK, dV, 8 products, or in smaller launches dQ here and the rest in attention_bwd_pair.hip, 7;
-// d = 64: dQ, dK+dV, 7), built like the forward (attention.hip): a workgroup of 4 wavefronts owns 128 "rows", one
-// lane one row (two lanes share it), and walks 64-position tiles of the rows' spans as the mask's plan table lists
-// them; per tile two operand tiles X and Y arrive in LDS through the asynchronous copy ring.
-//
-//   mode  rows     positions  registers A, B   tile X   tile Y   per 32-position half
-//   dQ    queries  keys       Q, dO            K        V        S^T = X A^T; P; dP^T = Y B^T; dS; acc^T += X^T dS^T
-//   dK    keys     queries    K, V             Q        dO       the same with the mask's transpose
-//   dV    keys     queries    K                Q        dO       S^T = X A^T; P;                 acc^T += Y^T P^T
-//   dK+dV keys     queries    K, V             Q        dO       as dK, and acc2^T += Y^T P^T    (d = 64: both accumulators fit)
-//
-// dQ walks the mask's own plan, dK and dV the plan of the transposed mask (keys as rows).  The dQ launch comes first: its
-// lanes hold their dO rows, so it also computes D (one more read of the lane's O row) and stores it for the other two.  lse
-// and D belong to the queries: one value per lane in dQ, one per tile position otherwise (64 floats each per tile, copied into LDS beside
-// the tiles).  The X tile of dQ / dK is read row-wise (16-byte fragments for S^T) and through the transposing read
+// dQ here: rows are queries, positions keys, X = K, Y = V, the register operands A = Q, B = dO; dK + dV in attention_bwd_pair.hip.  Per
+// half of a tile, 32 positions:    S^T = X A^T; P; dP^T = Y B^T; dS; acc^T += X^T dS^T
+// Built like the forward (attention.hip): a workgroup of 4 wavefronts owns 128 rows, one lane one row (two lanes share it), and walks
+// 64-position tiles of the rows' spans as the mask's plan table lists them; per tile X and Y arrive in LDS through the
+// asynchronous copy ring.  The dQ launch comes first: its lanes hold their dO rows, so it also computes D (one more read of the
+// lane's O row) and stores it for the other.  The X tile is read row-wise (16-byte fragments for S^T) and through the transposing read
 // (for acc^T), hence the swizzle that serves both (tile_copy.hpp: dual_chunk).  Probabilities come straight from the
 // statistic: no running maximum, no rescale, no second pass.  16-bit types, d = 64 or 128, rows of every operand
 // contiguous.
+// Bound: as the forward, matrix pipe, LDS reads and the power limit together.  dP's products come right after the scores', with the
+// exponentials between them and dP's fragments in the registers of the scores' (64 heads of 8192, dilated 512 / 2, d = 128, dQ: 1 to 3 %).
 #include <initializer_list>
 
 #include "attn_bwd.hpp"
 
 namespace splat {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-template <typename T, int D, int MODE>
+template <typename T, int D>
 __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(const BwdParams p) {
     constexpr int ES = 2, BM = 128, BN = 64;
     static_assert(sizeof(T) == ES, "16-bit element types");
@@ -38,14 +29,9 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(const BwdParams p) {
     constexpr int ROWB = D * ES;
     constexpr int TILE = BN * ROWB;             // bytes of one operand tile
     constexpr int STAGE = 2 * TILE;               // X, Y
-    constexpr int STATS = 2 * BN * 4;             // lse[64], D[64] of one stage
-    constexpr int RING = 2 * STATS;               // both stages' statistics come first, then the ring of tiles
     constexpr int CPR = ROWB / 16, RPI = 1024 / ROWB;  // chunks per row, rows per 1 KiB copy block
     constexpr int NI = TILE / 4096;                   // copy blocks per wavefront and tile
     constexpr int NDMA = 2 * NI;
-    constexpr bool POS_STATS = MODE != kBwdDQ;  // lse / D per tile position instead of per lane
-    constexpr bool THREE = MODE != kBwdDV;      // the dP and dS steps
-    constexpr bool BOTH = MODE == kBwdDKV;      // dK and dV from one walk: a second accumulator, fed with P^T and Y^T
 
     extern __shared__ __attribute__((aligned(1024))) char smem[];
 
@@ -64,49 +50,38 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(const BwdParams p) {
     const int r0 = block_first_row(rb, BM, rs);
     const int L = p.L;
 
-    const T* ab = (const T*)p.a + b * p.a_sb + h * p.a_sh;
-    const T* bb = THREE ? (const T*)p.b + b * p.b_sb + h * p.b_sh : nullptr;
     const T* xb = (const T*)p.x + b * p.x_sb + h * p.x_sh;
     const T* yb = (const T*)p.y + b * p.y_sb + h * p.y_sh;
     T* ob = (T*)p.out + b * p.o_sb + h * p.o_sh;
-    const float* lse_b = p.lse + (int64_t)bh * L;
-    const float* del_b = p.delta + (int64_t)bh * L;
 
-    // ---- register operands: fragments of this lane's row, resident for the whole kernel ----
-    const int Lr = p.Lr;
-    int my_row = min(r0 + rs * (wave * 32 + lm), Lr - 1);
-    if constexpr (MODE != kBwdDQ) {
-        if (p.row_map) my_row = min(max(p.row_map[my_row], 0), L - 1);
-    }
-    Frag<T> af[KS], bf[THREE ? KS : 1];
+    // ---- register operands: fragments of this lane's row, resident for the whole kernel (through LDS, as in attention_bwd_pair.hip, they come
+    // no sooner: a stage holds one operand's 128 rows, so that the first tile has to wait for them) ----
+    const int my_row = min(r0 + rs * (wave * 32 + lm), L - 1);
+    Frag<T> af[KS], bf[KS];
+    auto load_row = [&](Frag<T> (&f)[KS], const void* base, int64_t sb, int64_t sh, int64_t sl) {
+        const T* const from = (const T*)base + b * sb + h * sh + (int64_t)my_row * sl + 8 * g;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) af[ks] = global_frag<T>(ab + (int64_t)my_row * p.a_sl + 16 * ks + 8 * g);
-    if constexpr (THREE) {
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) bf[ks] = global_frag<T>(bb + (int64_t)my_row * p.b_sl + 16 * ks + 8 * g);
-    }
+        for (int ks = 0; ks < KS; ++ks) f[ks] = global_frag<T>(from + 16 * ks);
+    };
+    load_row(af, p.a, p.a_sb, p.a_sh, p.a_sl);
+    load_row(bf, p.b, p.b_sb, p.b_sh, p.b_sl);
     const float c2 = p.scale_log2e;
-    float row_lse2 = 0.f, row_delta = 0.f;  // dQ: the lane's own query
-    if constexpr (!POS_STATS) {
-        row_lse2 = lse_b[my_row] * 1.4426950408889634f;
-        // D = rowsum(dO * O) of the lane's row (the two lanes of a row hold half of it each), kept for this launch and stored
-        // for the dK and dV launches that follow it on the stream
-        const T* orow = (const T*)p.o + b * p.oo_sb + h * p.oo_sh + (int64_t)my_row * p.oo_sl;
-        Frag<T> of[KS];  // (all requested before any is used: the accumulators' registers are still free here)
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) of[ks] = global_frag<T>(orow + 16 * ks + 8 * g);
+    const float row_lse2 = p.lse[(int64_t)bh * L + my_row] * 1.4426950408889634f;
+    // D = rowsum(dO * O) of the lane's row (the two lanes of a row hold half of it each), kept for this launch and stored
+    // for the keys' side that follows it on the stream
+    Frag<T> of[KS];  // (all requested before any is used: the accumulators' registers are still free here)
+    load_row(of, p.o, p.oo_sb, p.oo_sh, p.oo_sl);
 #if defined(__HIP_DEVICE_COMPILE__)
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) asm volatile("" ::"v"(of[ks].v));
+    for (int ks = 0; ks < KS; ++ks) asm volatile("" ::"v"(of[ks].v));
 #endif
-        float s = 0.f;
+    float s = 0.f;
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks)
+    for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) s = fmaf((float)bf[ks].v[e], (float)of[ks].v[e], s);
-        s = with_lane_xor<32, 64>(s, [](float a, float b) { return a + b; });
-        row_delta = s;  // (stored after the tile loop: a store in flight would be waited for with the first tile's copies)
-    }
+        for (int e = 0; e < 8; ++e) s = fmaf((float)bf[ks].v[e], (float)of[ks].v[e], s);
+    // (stored after the tile loop: a store in flight would be waited for with the first tile's copies)
+    const float row_delta = with_lane_xor<32, 64>(s, [](float a, float b) { return a + b; });
 
     // ---- plan ----
     const PlanRec* const pt = p.plan;
@@ -126,18 +101,10 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(const BwdParams p) {
     auto position_row = [&](const SegPlan& pl, int j) { return min(max(pl.c0 + pl.cs * j, 0), L - 1); };
     auto issue_tile_general = [&](const SegPlan& pl, int tile, int stage) {
         const int j0 = tile * BN;
-        char* xs_w = smem + RING + stage * STAGE;
+        char* xs_w = smem + stage * STAGE;
         char* ys_w = xs_w + TILE;
         dma_tile<T, ROWB, BN, 3>(xs_w, wave, lane, [&](int row) { return xb + (int64_t)position_row(pl, j0 + row) * p.x_sl; });
         dma_tile<T, ROWB, BN, 3>(ys_w, wave, lane, [&](int row) { return yb + (int64_t)position_row(pl, j0 + row) * p.y_sl; });
-    };
-    auto issue_stats = [&](const SegPlan& pl, int tile, int stage) {
-        if constexpr (POS_STATS) {
-            char* st_w = smem + stage * STATS;
-            const int q = position_row(pl, tile * BN + lane);
-            if (wave == 0) dma4(lse_b + q, st_w);
-            if (wave == 1) dma4(del_b + q, st_w + BN * 4);
-        }
     };
     uint32_t x_lane_off = 0, y_lane_off = 0;
     bool lane_off_fits = true;
@@ -162,7 +129,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(const BwdParams p) {
         return lane_off_fits && pl.c0 + pl.cs * j0 >= 0 && pl.c0 + pl.cs * (j0 + BN - 1) < L;
     };
     auto issue_step = [&](int i, int stage) {
-        char* xs_w = smem + RING + stage * STAGE;
+        char* xs_w = smem + stage * STAGE;
         char* ys_w = xs_w + TILE;
         if (i < NI)
             dma16_uniform(x_next + (int64_t)(4 * RPI * i) * x_key, x_lane_off, xs_w + (wave + 4 * i) * 1024);
@@ -193,28 +160,22 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(const BwdParams p) {
     const uint32_t smem_base = lds_address(smem);
     const int tr_row = (lane & 15) >> 2;
     const int tr_col = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);  // element column inside a 32-element block
-    // row-wise fragments: row lm (+32 for the second half: the swizzle repeats every 16 rows), logical chunk 2*ks + g
-    uint32_t xr_addr[KS], yr_addr[THREE ? KS : 1];
-    // transposing reads: rows 4g + tr_row and 8 rows further (whose swizzle differs), 64-byte block dt
-    uint32_t tr_addr[DT], tr_addr8[DT];
+    // One register each: the swizzle XORs the chunk with bits of the row, so that contraction step ks flips bits 5 .. of the address,
+    // feature block dt bits 6 .., and 8 rows on bit 5 (rows 32 on, in the second half of a tile, have the same pattern); Y lies TILE further.
     auto dual_off = [&](int row, int byte_col) { return row * ROWB + dual_chunk<ROWB>(row, byte_col >> 4) * 16 + (byte_col & 15); };
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-        xr_addr[ks] = smem_base + RING + dual_off(lm, (16 * ks + 8 * g) * ES);
-        if constexpr (THREE) yr_addr[ks] = smem_base + RING + TILE + dual_off(lm, (16 * ks + 8 * g) * ES);
-    }
-    constexpr int TR_BASE = RING + (THREE ? 0 : TILE);  // dQ, dK: transposed reads of X; dV: of Y; dK + dV: of both
-    uint32_t ty_addr[BOTH ? DT : 1], ty_addr8[BOTH ? DT : 1];
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-        tr_addr[dt] = smem_base + TR_BASE + dual_off(4 * g + tr_row, (32 * dt + tr_col) * ES);
-        tr_addr8[dt] = smem_base + TR_BASE + dual_off(4 * g + tr_row + 8, (32 * dt + tr_col) * ES);
-        if constexpr (BOTH) {
-            ty_addr[dt] = tr_addr[dt] + TILE;
-            ty_addr8[dt] = tr_addr8[dt] + TILE;
-        }
-    }
-    uint32_t st_addr = smem_base + 16 * g;  // lse of positions 4g.. of the stage; D is BN*4 bytes further
+    uint32_t xr_addr = smem_base + dual_off(lm, 8 * g * ES);
+    uint32_t tr_addr = smem_base + dual_off(4 * g + tr_row, tr_col * ES);
+    // fragment ks of the tile's rows 32 nt .. (row lm of them): of X at `from` = 0, of Y at TILE
+    auto row_frag = [&](int ks, int nt, int from) {
+        Frag<T> f;
+        f.v = __builtin_bit_cast(typename Frag<T>::vec, lds_load128((xr_addr ^ (32u * ks)) + (from + 32 * nt * ROWB)));
+        return f;
+    };
+    // X's transpose: 16 positions from 16 * step on, features 32 dt ..
+    auto tr_frag = [&](int step, int dt) {
+        const uint32_t at = tr_addr ^ (64u * dt);
+        return frag_from_tr<T>(lds_load_tr16(at + 16 * step * ROWB), lds_load_tr16((at ^ 32u) + (16 * step + 8) * ROWB));
+    };
 
     // ---- first tile's copies, accumulators ----
     pf_seg = 0;
@@ -228,16 +189,14 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(const BwdParams p) {
         } else {
             issue_tile_general(ppl, pf_tile, 0);
         }
-        issue_stats(ppl, pf_tile, 0);
         advance_fetch();
     }
-    f32x16 acc[DT], acc2[BOTH ? DT : 1];
+    f32x16 acc[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
             acc[dt][j] = 0.f;
-            if constexpr (BOTH) acc2[dt][j] = 0.f;
         }
 
     int cur_seg = -1, cur_tile = 0;
@@ -251,11 +210,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(const BwdParams p) {
     // the register operands are in their registers before the loop, so that no wait of the compiler's for them ends up
     // inside it, where it would also wait for the copies in flight
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) asm volatile("" ::"v"(af[ks].v));
-    if constexpr (THREE) {
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) asm volatile("" ::"v"(bf[ks].v));
-    }
+    for (int ks = 0; ks < KS; ++ks) asm volatile("" ::"v"(af[ks].v), "v"(bf[ks].v));
     asm volatile("" ::"v"(row_lse2), "v"(row_delta));
 #endif
 
@@ -297,87 +252,15 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(const BwdParams p) {
         if (fetch) {
             spread = tile_is_fast(ppl, pf_tile);
             if (!spread) issue_tile_general(ppl, pf_tile, stage_pf);
-            issue_stats(ppl, pf_tile, stage_pf);
         }
 
         const bool skip = (j0 + BN <= w_lo_min) || (j0 >= w_hi_max);
         if (!skip) {
             const bool full = (j0 >= w_lo_max) && (j0 + BN <= w_hi_min);
             const uint64_t live = full ? ~0ull : row_live_bits(win, j0, first, pat);
-            if constexpr (!THREE) {
-                // ---- dV: two products only, so the whole 64-position tile fits the registers at once, as in the forward:
-                // all score MFMAs with the fragments requested well ahead, then the exponentials, then the output MFMAs ----
-                constexpr int NMMA = 2 * KS, AHEAD = NMMA < 12 ? NMMA : 12;
-                f32x16 s2[2];
-#pragma unroll
-                for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-                    for (int j = 0; j < 16; ++j) s2[nt][j] = 0.f;
-                Frag<T> xfr[NMMA];
-                auto load_x = [&](int i) {
-                    Frag<T> f;
-                    f.v = __builtin_bit_cast(typename Frag<T>::vec, lds_load128(xr_addr[i % KS] + 32 * (i / KS) * ROWB));
-                    return f;
-                };
-#pragma unroll
-                for (int i = 0; i < AHEAD; ++i) xfr[i] = load_x(i);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int i = 0; i < NMMA; ++i) {
-                    mma32(s2[i / KS], xfr[i], af[i % KS]);
-                    if (i + AHEAD < NMMA) {
-                        xfr[i + AHEAD] = load_x(i + AHEAD);
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
-                    if (i < NDMA) {
-                        if (spread) issue_step(i, stage_pf);
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
-                }
-                Frag<T> pf2[2][2];
-#pragma unroll
-                for (int nt = 0; nt < 2; ++nt) {
-                    if (!full) {
-                        const uint32_t bits = (uint32_t)(live >> (32 * nt)) >> (4 * g);
-#pragma unroll
-                        for (int j = 0; j < 16; ++j) {
-                            const int c = 8 * (j >> 2) + (j & 3);
-                            s2[nt][j] = keep_or_mask(s2[nt][j], ((int)(bits << (31 - c))) >> 31);
-                        }
-                    }
-#pragma unroll
-                    for (int k4 = 0; k4 < 4; ++k4) {
-                        const f32x4 lse4 = __builtin_bit_cast(f32x4, lds_load128(st_addr + (32 * nt + 8 * k4) * 4));
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const int j = 4 * k4 + i;
-                            pf2[nt][j >> 3].v[j & 7] = (T)fast_exp2(fmaf(s2[nt][j], c2, -1.4426950408889634f * lse4[i]));
-                        }
-                    }
-                }
-                auto load_t = [&](int step, int dt) {
-                    const int roff = 16 * step * ROWB;
-                    return frag_from_tr<T>(lds_load_tr16(tr_addr[dt] + roff), lds_load_tr16(tr_addr8[dt] + roff));
-                };
-                Frag<T> tf2[2][DT];
-#pragma unroll
-                for (int dt = 0; dt < DT; ++dt) tf2[0][dt] = load_t(0, dt);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int step = 0; step < 4; ++step) {
-#pragma unroll
-                    for (int dt = 0; dt < DT; ++dt) {
-                        mma32(acc[dt], tf2[step & 1][dt], pf2[step >> 1][step & 1]);
-                        if (step + 1 < 4) {
-                            tf2[(step + 1) & 1][dt] = load_t(step + 1, dt);
-                            __builtin_amdgcn_sched_barrier(0);
-                        }
-                    }
-                }
-            } else
 #pragma unroll
             for (int nt = 0; nt < 2; ++nt) {
-                static_assert(!THREE || NDMA <= KS, "the first half issues all copies");
+                static_assert(NDMA <= KS, "the first half issues all copies");
                 // half a tile that holds nothing for this wavefront, as at the ends of most spans (bfloat16, 64 heads of 4096, the
                 // whole step: window 65 at d = 64 131 -> 123 us, 33 at d = 128 257 -> 252)
                 if (nt == 0 ? j0 + 32 <= w_lo_min : j0 + 32 >= w_hi_max) {
@@ -387,105 +270,57 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(const BwdParams p) {
                     }
                     continue;
                 }
-                // ---- S^T (32 positions x 32 rows) = X rows . A^T ----
-                f32x16 s_acc;
+                // ---- S^T (32 positions x 32 rows) = X rows . A^T; Y's fragments take the places of X's ----
+                f32x16 s_acc, dp;
 #pragma unroll
-                for (int j = 0; j < 16; ++j) s_acc[j] = 0.f;
-                Frag<T> xfr[KS];
+                for (int j = 0; j < 16; ++j) s_acc[j] = 0.f, dp[j] = 0.f;
+                Frag<T> xfr[KS], yfr[KS];
 #pragma unroll
-                for (int ks = 0; ks < KS; ++ks)
-                    xfr[ks].v = __builtin_bit_cast(typename Frag<T>::vec, lds_load128(xr_addr[ks] + 32 * nt * ROWB));
+                for (int ks = 0; ks < KS; ++ks) xfr[ks] = row_frag(ks, nt, 0);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks) {
                     mma32(s_acc, xfr[ks], af[ks]);
+                    yfr[ks] = row_frag(ks, nt, TILE);
                     // the copy instructions of the next tile go between these MFMAs
                     const int step = nt * KS + ks;  // 0 .. 2*KS - 1
-                    if (step < NDMA) {
-                        if (spread) issue_step(step, stage_pf);
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
+                    if (step < NDMA && spread) issue_step(step, stage_pf);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
                 if (!(j0 + 32 * nt >= w_lo_max && j0 + 32 * nt + 32 <= w_hi_min)) mask_half(s_acc, (uint32_t)(live >> (32 * nt)) >> (4 * g));
-                // ---- P^T = exp2(S^T * scale*log2e - lse*log2e); masked scores underflow to exactly 0 ----
-                if constexpr (POS_STATS) {
+                // ---- dP^T = Y rows . B^T, and between its matrix instructions P^T = exp2(S^T * scale*log2e - lse*log2e); masked scores
+                // underflow to exactly 0 ----
+                constexpr int EPM = 16 / KS;  // elements per matrix instruction
+                Frag<T> tf[2][DT];
 #pragma unroll
-                    for (int k4 = 0; k4 < 4; ++k4) {
-                        // (the whole vector is reinterpreted: a bit cast of one element of an integer vector reads element 0)
-                        const f32x4 lse4 = __builtin_bit_cast(f32x4, lds_load128(st_addr + (32 * nt + 8 * k4) * 4));
+                for (int ks = 0; ks < KS; ++ks) {
+                    mma32(dp, yfr[ks], bf[ks]);
 #pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            s_acc[4 * k4 + i] = fast_exp2(fmaf(s_acc[4 * k4 + i], c2, -1.4426950408889634f * lse4[i]));
+                    for (int i = 0; i < EPM; ++i) {
+                        const int j = EPM * ks + i;
+                        s_acc[j] = fast_exp2(fmaf(s_acc[j], c2, -row_lse2));
                     }
-                } else {
-#pragma unroll
-                    for (int j = 0; j < 16; ++j) s_acc[j] = fast_exp2(fmaf(s_acc[j], c2, -row_lse2));
-                }
-                Frag<T> pf[2];  // the second product's B operand: 16 positions each
-                Frag<T> pp[BOTH ? 2 : 1];  // dK + dV: the probabilities themselves, dV's B operand
-                if constexpr (THREE) {
-                    // ---- dP^T = Y rows . B^T ----
-                    f32x16 dp;
-#pragma unroll
-                    for (int j = 0; j < 16; ++j) dp[j] = 0.f;
-                    Frag<T> yfr[KS];
-#pragma unroll
-                    for (int ks = 0; ks < KS; ++ks)
-                        yfr[ks].v = __builtin_bit_cast(typename Frag<T>::vec, lds_load128(yr_addr[ks] + 32 * nt * ROWB));
+                    if (ks >= KS - DT) tf[0][ks - (KS - DT)] = tr_frag(2 * nt, ks - (KS - DT));
                     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int ks = 0; ks < KS; ++ks) mma32(dp, yfr[ks], bf[ks]);
-                    // ---- dS^T = P^T * (dP^T - D) * scale ----
-                    if constexpr (POS_STATS) {
-#pragma unroll
-                        for (int k4 = 0; k4 < 4; ++k4) {
-                            const f32x4 d4 = __builtin_bit_cast(f32x4, lds_load128(st_addr + BN * 4 + (32 * nt + 8 * k4) * 4));
-#pragma unroll
-                            for (int i = 0; i < 4; ++i) {
-                                const int j = 4 * k4 + i;
-                                pf[j >> 3].v[j & 7] = (T)(s_acc[j] * (dp[j] - d4[i]) * p.scale);
-                            }
-                        }
-                    } else {
-#pragma unroll
-                        for (int j = 0; j < 16; ++j) pf[j >> 3].v[j & 7] = (T)(s_acc[j] * (dp[j] - row_delta) * p.scale);
-                    }
-                    if constexpr (BOTH) {
-#pragma unroll
-                        for (int j = 0; j < 16; ++j) pp[j >> 3].v[j & 7] = (T)s_acc[j];
-                    }
-                } else {
-#pragma unroll
-                    for (int j = 0; j < 16; ++j) pf[j >> 3].v[j & 7] = (T)s_acc[j];
                 }
-                // ---- acc^T (d x 32 rows) += tile^T . pf: two steps of 16 positions ----
+                // ---- dS^T = P^T * (dP^T - D) * scale, eight positions' worth of registers ahead of acc^T (d x 32 rows) += X^T . dS^T ----
+                Frag<T> pf[2];  // the second product's B operand: 16 positions each
+                auto d_score = [&](int j) { pf[j >> 3].v[j & 7] = (T)(s_acc[j] * (dp[j] - row_delta) * p.scale); };
+#pragma unroll
+                for (int j = 0; j < 8; ++j) d_score(j);
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
-                    Frag<T> tf[DT];
 #pragma unroll
                     for (int dt = 0; dt < DT; ++dt) {
-                        const int roff = (32 * nt + 16 * t) * ROWB;
-                        tf[dt] = frag_from_tr<T>(lds_load_tr16(tr_addr[dt] + roff), lds_load_tr16(tr_addr8[dt] + roff));
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
+                        mma32(acc[dt], tf[t][dt], pf[t]);
+                        if (t == 0) {
+                            tf[1][dt] = tr_frag(2 * nt + 1, dt);
 #pragma unroll
-                    for (int dt = 0; dt < DT; ++dt) mma32(acc[dt], tf[dt], pf[t]);
-                    if constexpr (BOTH) {
-                        // ---- acc2^T += Y^T . P^T ----
-#pragma unroll
-                        for (int dt = 0; dt < DT; ++dt) {
-                            const int roff = (32 * nt + 16 * t) * ROWB;
-                            tf[dt] = frag_from_tr<T>(lds_load_tr16(ty_addr[dt] + roff), lds_load_tr16(ty_addr8[dt] + roff));
+                            for (int i = 0; i < 8 / DT; ++i) d_score(8 + 8 / DT * dt + i);
                         }
                         __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                        for (int dt = 0; dt < DT; ++dt) mma32(acc2[dt], tf[dt], pp[t]);
                     }
                 }
-            }
-            if (2 * KS < NDMA && spread) {
-#pragma unroll
-                for (int s = 2 * KS; s < NDMA; ++s) issue_step(s, stage_pf);
             }
         } else if (spread) {
 #pragma unroll
@@ -502,34 +337,19 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(const BwdParams p) {
         }
         stage_it ^= 1;
         const int delta_b = stage_it == 0 ? -STAGE : STAGE;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            xr_addr[ks] += delta_b;
-            if constexpr (THREE) yr_addr[ks] += delta_b;
-        }
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-            tr_addr[dt] += delta_b;
-            tr_addr8[dt] += delta_b;
-            if constexpr (BOTH) {
-                ty_addr[dt] += delta_b;
-                ty_addr8[dt] += delta_b;
-            }
-        }
-        st_addr += stage_it == 0 ? -STATS : STATS;
+        xr_addr += delta_b;
+        tr_addr += delta_b;
     }
     // every wavefront has finished reading the last tile before the stages are reused for the output
     wait_loads<0>();
     __syncthreads();
 
-    if constexpr (!POS_STATS) {
-        if (g == 0 && r0 + rs * (wave * 32 + lm) < Lr) p.delta_w[(int64_t)bh * L + my_row] = row_delta;
-    }
+    if (g == 0 && r0 + rs * (wave * 32 + lm) < L) p.delta_w[(int64_t)bh * L + my_row] = row_delta;
 
     // ---- epilogue: out = acc^T transposed through LDS, whole rows per store (each wavefront through a stretch of its own) ----
     {
         constexpr int OROW = D * ES + 16;
-        static_assert(4 * 32 * OROW <= RING + 2 * STAGE, "staging space");
+        static_assert(4 * 32 * OROW <= 2 * STAGE, "staging space");
         char* stg = smem + wave * (32 * OROW);
         auto store_rows = [&](const f32x16 (&a)[DT], T* dst) {
 #pragma unroll
@@ -550,21 +370,20 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(const BwdParams p) {
                 const int row = flat / OCPR, c = flat % OCPR;
                 const int r = r0 + rs * (wave * 32 + row);
                 const u32x4 val = *reinterpret_cast<const u32x4*>(stg + row * OROW + c * 16);
-                if (r < Lr) __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(reinterpret_cast<char*>(dst + (int64_t)r * p.o_sl) + c * 16));
+                if (r < L) __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(reinterpret_cast<char*>(dst + (int64_t)r * p.o_sl) + c * 16));
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (read out before the stretch is written again)
         };
         store_rows(acc, ob);
-        if constexpr (BOTH) store_rows(acc2, (T*)p.out2 + b * p.o_sb + h * p.o_sh);
     }
 }
 
-template <typename T, int D, int MODE>
+template <typename T, int D>
 static int launch_bwd(BwdParams p, hipStream_t st) {
     begin_launch();
-    constexpr int LDS_BYTES = 2 * (2 * 64 * D * 2) + 2 * (2 * 64 * 4);  // two stages of two tiles, two of statistics
+    constexpr int LDS_BYTES = 2 * (2 * 64 * D * 2);  // two stages of two tiles
     const int grid = ((p.total + 7) / 8) * 8;
-    auto kern = attn_bwd_kernel<T, D, MODE>;
+    auto kern = attn_bwd_kernel<T, D>;
     static uint64_t lds_reserved = 0;
     if (int rc = reserve_dynamic_lds(&lds_reserved, reinterpret_cast<const void*>(kern), LDS_BYTES, "splat_attention_bwd")) return rc;
     kern<<<grid, 256, LDS_BYTES, st>>>(p);
@@ -624,34 +443,10 @@ static int launch_rows_add(const void* dk_rows, const void* dv_rows, void* dk, v
     return check_launch("splat_attention_bwd_keys");
 }
 
-// The keys' side: dK and dV of the rows of the transposed mask that `dk` describes (dv: the same launch geometry).
 template <typename T>
-static int run_bwd_keys(const BwdParams& dk, const BwdParams& dv, int d, hipStream_t st) {
-    if (d == 64) {
-        // both accumulators of the keys' side fit the registers at d = 64 (204 of 256; at d = 128 they would need over 300):
-        // one walk, 4 products instead of 3 + 2, the scores and the exponentials once (config 2: 0.160 -> 0.133 ms)
-        BwdParams dkv = dk;
-        dkv.out2 = dv.out;
-        return launch_bwd<T, 64, kBwdDKV>(dkv, st);
-    }
-    if (dk.total <= 1024) {
-        // Launches of at most four row blocks a CU: one walk by pairs of wavefronts (attention_bwd_pair.hip), which puts eight
-        // wavefronts on a row block where the two launches below put four.  Training steps, bfloat16: 128 row blocks, window 512:
-        // 82 -> 69 us; 512 blocks, two segments: 128 -> 114; 1024 blocks, window 32: 135 -> 133.  Beyond, the beginnings and ends
-        // of its workgroups, which nothing else on the CU covers, cost what the fifth product does (the two launches -> the pairs):
-        // 2048 blocks, window 128: 279 -> 295 us, window 512: 491 -> 491; 4096 blocks, dilated 512 / 2: 986 -> 972.
-        BwdParams dkv = dk;
-        dkv.out2 = dv.out;
-        return launch_bwd_pair<T>(dkv, st);
-    }
-    if (int rc = launch_bwd<T, 128, kBwdDK>(dk, st)) return rc;
-    return launch_bwd<T, 128, kBwdDV>(dv, st);
-}
-
-template <typename T>
-static int run_bwd(const BwdParams& dq, const BwdParams& dk, const BwdParams& dv, int d, hipStream_t st) {
-    if (int rc = d == 64 ? launch_bwd<T, 64, kBwdDQ>(dq, st) : launch_bwd<T, 128, kBwdDQ>(dq, st)) return rc;
-    return run_bwd_keys<T>(dk, dv, d, st);
+static int run_bwd(const BwdParams& dq, const BwdParams& dkv, int d, hipStream_t st) {
+    if (int rc = d == 64 ? launch_bwd<T, 64>(dq, st) : launch_bwd<T, 128>(dq, st)) return rc;
+    return launch_bwd_pair<T>(dkv, d, st);
 }
 
 struct Rows3 {
@@ -690,16 +485,16 @@ static BwdParams bwd_base(const float* lse, const float* delta, int B, int H, in
     return base;
 }
 
-// dK (and, as a copy with b = null and out = dV, dV): rows = `Lk` keys, the plan of the (transposed) mask's `n_seg_t` segments
+// dK and dV (out2): rows = `Lk` keys, the plan of the (transposed) mask's `n_seg_t` segments
 // for those rows; outputs contiguous [B, H, Lk, d]
-static BwdParams bwd_keys_params(const BwdParams& base, Rows3 q, Rows3 k, Rows3 v, Rows3 g, void* dk, const splat_acsr_seg* segs_t,
+static BwdParams bwd_keys_params(const BwdParams& base, Rows3 q, Rows3 k, Rows3 v, Rows3 g, void* dk, void* dv, const splat_acsr_seg* segs_t,
                                  int n_seg_t, const void* plan_t, int Lk, const int* row_map, int d) {
     BwdParams pk = base;
     pk.a = k.ptr; pk.a_sb = k.sb; pk.a_sh = k.sh; pk.a_sl = k.sl;
     pk.b = v.ptr; pk.b_sb = v.sb; pk.b_sh = v.sh; pk.b_sl = v.sl;
     pk.x = q.ptr; pk.x_sb = q.sb; pk.x_sh = q.sh; pk.x_sl = q.sl;
     pk.y = g.ptr; pk.y_sb = g.sb; pk.y_sh = g.sh; pk.y_sl = g.sl;
-    pk.out = dk; pk.o_sb = (int64_t)base.H * Lk * d; pk.o_sh = (int64_t)Lk * d; pk.o_sl = d;
+    pk.out = dk; pk.out2 = dv; pk.o_sb = (int64_t)base.H * Lk * d; pk.o_sh = (int64_t)Lk * d; pk.o_sl = d;
     pk.Lr = Lk; pk.row_map = row_map;
     pk.n_seg = n_seg_t; pk.row_stride = common_row_stride(segs_t, n_seg_t);
     pk.n_row_blocks = count_row_blocks(Lk, kPlanBM, pk.row_stride); pk.total = base.B * base.H * pk.n_row_blocks;
@@ -750,17 +545,12 @@ static int bwd_impl(const char* who, bool f32, const void* q, int64_t q_sb, int6
     pq.plan = static_cast<const PlanRec*>(plan);
     pq.o = out; pq.oo_sb = o_sb; pq.oo_sh = o_sh; pq.oo_sl = o_sl; pq.delta_w = delta;  // D = rowsum(dO * O): computed and stored by this launch
     // dK, dV: rows = keys, the transposed mask's plan
-    const BwdParams pk = bwd_keys_params(base, rq, rk, rv, rg, dk, segs_t, n_seg_t, plan_t, L, nullptr, d);
+    const BwdParams pk = bwd_keys_params(base, rq, rk, rv, rg, dk, dv, segs_t, n_seg_t, plan_t, L, nullptr, d);
     if (f32) {
-        BwdParams pkv = pk;
-        pkv.out2 = dv;
         if (int rc = launch_bwd_dq_f32(pq, d, st)) return rc;
-        return launch_bwd_dkv_f32(pkv, d, st);
+        return launch_bwd_dkv_f32(pk, d, st);
     }
-    BwdParams pv = pk;
-    pv.b = nullptr;
-    pv.out = dv;
-    return dtype == SPLAT_F16 ? run_bwd<f16>(pq, pk, pv, d, st) : run_bwd<bf16>(pq, pk, pv, d, st);
+    return dtype == SPLAT_F16 ? run_bwd<f16>(pq, pk, d, st) : run_bwd<bf16>(pq, pk, d, st);
 }
 
 
@@ -794,18 +584,13 @@ static int bwd_keys_impl(const char* who, bool f32, const void* q, int64_t q_sb,
     if ((int64_t)B * H * count_row_blocks(n_rows, kPlanBM, common_row_stride(segs_t, n_seg_t)) > 0x7ffffff0)
         return fail(SPLAT_E_SHAPE, "%s: too many row blocks", who);
     const BwdParams base = bwd_base(lse, delta, B, H, L, scale);
-    const BwdParams pk = bwd_keys_params(base, rq, rk, rv, rg, dk_rows, segs_t, n_seg_t, plan_t, n_rows, key_of_row, d);
+    const BwdParams pk = bwd_keys_params(base, rq, rk, rv, rg, dk_rows, dv_rows, segs_t, n_seg_t, plan_t, n_rows, key_of_row, d);
     hipStream_t st = (hipStream_t)stream;
     if (f32) {
-        BwdParams pkv = pk;
-        pkv.out2 = dv_rows;
-        if (int rc = launch_bwd_dkv_f32(pkv, d, st)) return rc;
+        if (int rc = launch_bwd_dkv_f32(pk, d, st)) return rc;
         return dk ? launch_rows_add<float>(dk_rows, dv_rows, dk, dv, key_of_row, B, H, L, n_rows, rows_per_stretch, d, st) : 0;
     }
-    BwdParams pv = pk;
-    pv.b = nullptr;
-    pv.out = dv_rows;
-    if (int rc = dtype == SPLAT_F16 ? run_bwd_keys<f16>(pk, pv, d, st) : run_bwd_keys<bf16>(pk, pv, d, st)) return rc;
+    if (int rc = dtype == SPLAT_F16 ? launch_bwd_pair<f16>(pk, d, st) : launch_bwd_pair<bf16>(pk, d, st)) return rc;
     if (!dk) return 0;
     return dtype == SPLAT_F16 ? launch_rows_add<f16>(dk_rows, dv_rows, dk, dv, key_of_row, B, H, L, n_rows, rows_per_stretch, d, st)
                               : launch_rows_add<bf16>(dk_rows, dv_rows, dk, dv, key_of_row, B, H, L, n_rows, rows_per_stretch, d, st);
