@@ -36,7 +36,7 @@
 extern "C" {
 #endif
 
-#define SPLAT_VERSION 1200 /* major*10000 + minor*100 + patch; 0.2.0 added the planned forward, 0.3.0 splat_spmm_t, 0.4.0 splat_attention_fwd_stats, splat_sddmm_probs, 0.5.0 splat_attention_fwd_noalloc, 0.6.0 moved the two measurement aids out (libsplat_bench.so, splat_bench.h), 0.7.0 added splat_sddmm_planned, splat_spmm_planned, 0.8.0 splat_spmm_t_planned, 0.9.0 splat_attention_bwd_keys, 0.10.0 splat_acsr_build_record, splat_attention_bwd_f32, splat_attention_bwd_keys_f32, 0.11.0 gave splat_acsr_build_record's int32 arrays a buffer of their own and added splat_attention_plan_report, splat_attention_fwd_hinted, 0.12.0 added splat_attention_fwd_keys and summary[5..6] of splat_acsr_build, which a row_stride_hint may come from */
+#define SPLAT_VERSION 1300 /* major*10000 + minor*100 + patch; 0.2.0 added the planned forward, 0.3.0 splat_spmm_t, 0.4.0 splat_attention_fwd_stats, splat_sddmm_probs, 0.5.0 splat_attention_fwd_noalloc, 0.6.0 moved the two measurement aids out (libsplat_bench.so, splat_bench.h), 0.7.0 added splat_sddmm_planned, splat_spmm_planned, 0.8.0 splat_spmm_t_planned, 0.9.0 splat_attention_bwd_keys, 0.10.0 splat_acsr_build_record, splat_attention_bwd_f32, splat_attention_bwd_keys_f32, 0.11.0 gave splat_acsr_build_record's int32 arrays a buffer of their own and added splat_attention_plan_report, splat_attention_fwd_hinted, 0.12.0 added splat_attention_fwd_keys and summary[5..6] of splat_acsr_build, which a row_stride_hint may come from, 0.13.0 added splat_sddmm_softmax */
 
 /* element types of q/k/v/score/output buffers */
 #define SPLAT_F32 0
@@ -172,6 +172,18 @@ int splat_sddmm_planned(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl,
 int splat_softmax(const void* x, void* y, const splat_acsr_seg* segs /* host */, int32_t n_seg,
                   int64_t BH, int32_t L, int32_t T, int32_t in_dtype, int32_t out_dtype,
                   void* stream);
+
+/* splat_sddmm_planned without statistics (plan may be NULL), then splat_softmax of its output into `probs` ([B,H,L,T]
+ * contiguous, dtype out_dtype, not overlapping out; rows without live slots and dead slots stay as they are in both).
+ * Where the wavefronts of the sampled product own whole rows of at most 256 slots (enough row blocks for the chip, and no
+ * more scores than the caches hold), they take their softmax as well, and a launch and a pass over memory are spared
+ * (float16, 16 heads of 2000 rows, 129 slots, d = 80, with splat_spmm: 26.7 -> 21 us); elsewhere the second launch
+ * follows.  Both results are those of the two calls, bit for bit.  Replaces r_sddmm.py:153-188 and r_softmax.py:126-150. */
+int splat_sddmm_softmax(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* kT, int64_t k_sb,
+                        int64_t k_sh, int64_t k_sd, int64_t k_sl, void* out, void* probs,
+                        const splat_acsr_seg* segs /* host */, int32_t n_seg, int32_t B, int32_t H, int32_t L,
+                        int32_t n_keys, int32_t d, int32_t T, float scale, int32_t in_dtype, int32_t out_dtype,
+                        const void* plan, int64_t plan_bytes, void* stream);
 
 /* SpMM: out[b,h,r,:] = sum_{s<nnz[r]} p[b,h,r,off+s] * v[b,h,c(r,s),:], summed over segments.
  * Replaces rspmm_launcher / r_spmm_kernel_row_maj_row_comp, r_spmm.py:13-126,148-164.

@@ -1,0 +1,81 @@
+"""The sampled product and the softmax of its rows in one call against the two calls, bit for bit: rows at the edges of the softmax's splits and
+beyond the longest that the sampled product takes along, masks whose row blocks interleave, two segments, with the plan table and
+without, launches on both sides of the line from which a workgroup owns whole rows."""
+import ctypes
+
+import pytest
+import torch
+
+import acsr_helpers as A
+import _splat_hip as hip
+from test_gpu_operators import SENTINEL
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 64), (torch.float16, 104), (torch.float32, 40), (torch.float32, 128)])
+@pytest.mark.parametrize("heads", [1, 64, 100])  # (4 half row blocks a head; few, the line's, and what the line-wise kernel takes of the widest)
+@pytest.mark.parametrize("pattern", [lambda L: A.causal_windowed_pattern(L, 5), lambda L: A.causal_windowed_pattern(L, 128),
+                                     lambda L: A.causal_windowed_pattern(L, 129), lambda L: A.dilated_pattern(L, 77, 3),
+                                     lambda L: A.strided_patterns(L, 40, 16), lambda L: A.causal_windowed_pattern(L, 201),
+                                     lambda L: A.blocked_pattern(L, 200), lambda L: A.causal_windowed_pattern(L + 51, 257)],
+                         ids=["5", "128", "129", "dilated 77", "strided", "201", "blocked 200", "257"])
+@pytest.mark.parametrize("layout", ["rows", "keys"])
+def test_equals_the_two_calls(dev, layout, pattern, heads, dtype, d):
+    L = 250
+    masks = pattern(L)
+    segs = A.create_acsr_segments(masks if isinstance(masks, list) else [masks], 16, dev)
+    L, T = segs.tuples[0][0].shape[0], segs.T
+    g = torch.Generator(device=dev).manual_seed(T + d)
+    q, k = (torch.randn(1, heads, L, d, generator=g, device=dev).to(dtype) for _ in range(2))
+    kT = k.transpose(2, 3)
+    if layout == "keys":
+        kT = kT.contiguous()
+    arr, code, stream = segs.seg_array(L, T), hip.dtype_code(dtype), hip.stream_ptr(dev)
+    plan = segs.plan(L, dev)
+    for table, nbytes in ((plan.data_ptr(), plan.numel() * plan.element_size()), (None, 0)):
+        buffers = [torch.full((heads * L * T + 8,), SENTINEL, dtype=dtype, device=dev) for _ in range(4)]
+        want, want_p, got, got_p = (b.data_ptr() for b in buffers)
+        x = (q.data_ptr(), *q.stride()[:3], kT.data_ptr(), *kT.stride()[:4])
+        shape = (arr, len(segs), 1, heads, L, L, d, T, ctypes.c_float(0.2), code, code)
+        if table is None:
+            hip.check(hip.lib().splat_sddmm(*x, want, *shape, stream), "splat_sddmm")
+        else:
+            hip.check(hip.lib().splat_sddmm_planned(*x, want, *shape, None, table, nbytes, stream), "splat_sddmm_planned")
+        hip.check(hip.lib().splat_softmax(want, want_p, arr, len(segs), heads, L, T, code, code, stream), "splat_softmax")
+        hip.check(hip.lib().splat_sddmm_softmax(*x, got, got_p, *shape, table, nbytes, stream), "splat_sddmm_softmax")
+        assert torch.equal(buffers[0], buffers[2]) and torch.equal(buffers[1], buffers[3])
+        rows = buffers[3][:-8].view(heads, L, T).double()
+        sums = torch.where(rows == SENTINEL, 0.0, rows).sum(-1)
+        # (a row of n slots sums to 1 within the roundings of its entries, at most half a unit of the type each, and of its float32 sum)
+        assert float((sums - 1).abs().max()) <= torch.finfo(dtype).eps + 256 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows", [300, 41000, 140000])  # (as many row groups a wavefront as the chip has room for, and more)
+@pytest.mark.parametrize("T", [7, 9, 128, 136, 249, 256, 257, 504, 511, 1023])
+def test_softmax_of_few_and_many_rows(dev, T, rows, dtype):
+    """Every row's live slots against float64, a float32 evaluation of an exponential and a quotient apart, then rounded."""
+    g = torch.Generator(device=dev).manual_seed(T)
+    L = 50
+    nnz = torch.randint(0, T + 1, (L,), generator=g, device=dev).float()
+    nnz[::2] = T
+    zeros = torch.zeros(L, device=dev)
+    seg = (hip.AcsrSeg * 1)()
+    seg[0].sTod_lin, seg[0].sTod_trans, seg[0].nnz, seg[0].slot_offset = zeros.data_ptr(), zeros.data_ptr(), nnz.data_ptr(), 0
+    BH = rows // L
+    x = (torch.randn(BH, L, T, generator=g, device=dev) * 3).to(dtype)
+    buf = torch.full((BH * L * T + 9,), SENTINEL, dtype=dtype, device=dev)
+    for shift in (0, 1):  # (a buffer that starts anywhere, too)
+        buf.fill_(SENTINEL)
+        out = buf[shift:shift + BH * L * T]
+        hip.check(hip.lib().splat_softmax(x.data_ptr(), out.data_ptr(), seg, 1, BH, L, T, hip.dtype_code(dtype), hip.dtype_code(dtype),
+                                          hip.stream_ptr(dev)), "splat_softmax")
+        live = torch.arange(T, device=dev)[None] < nnz[:, None]
+        want = torch.softmax(x[:64].double().masked_fill(~live, float("-inf")), -1)
+        for part, ref in ((out.view(BH, L, T)[:64], want), (out.view(BH, L, T)[-1:], torch.softmax(x[-1:].double().masked_fill(~live, float("-inf")), -1))):
+            err = (part.double() - ref).abs() / ref.clamp_min(1e-30)
+            # (exp2 of a float32 product of up to 40: 40 * 2^-24 of it; the sum and the quotient a few units; one rounding to the type)
+            assert float(torch.where(live & (ref > 1e-4), err, 0.0).max()) <= 128 * 2.0 ** -24 + torch.finfo(dtype).eps / 2 * 1.01
+            assert torch.all(part.double()[~live.expand_as(part)] == SENTINEL)
+        assert torch.all(buf[:shift] == SENTINEL) and torch.all(buf[shift + BH * L * T:] == SENTINEL)

@@ -50,6 +50,7 @@ struct Api {
     decltype(&splat_sddmm_probs) sddmm_probs;
     decltype(&splat_sddmm_planned) sddmm_planned;
     decltype(&splat_softmax) softmax;
+    decltype(&splat_sddmm_softmax) sddmm_softmax;
     decltype(&splat_spmm) spmm;
     decltype(&splat_spmm_planned) spmm_planned;
     decltype(&splat_acsr_build_record) build_record;
@@ -416,9 +417,8 @@ PyObject* py_attend(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // ---- the three operators ------------------------------------------------------------------------------------------------------
-// sddmm(mask, x, y, output, scale, lse | None) -> bool; a plan in the mask is handed on
-PyObject* py_sddmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
-    if (n != 6) return PyErr_Format(PyExc_TypeError, "sddmm takes 6 arguments");
+// sddmm(mask, x, y, output, scale, lse | None) -> bool; a plan in the mask is handed on.  `probs`: the softmax of the output goes there.
+PyObject* sddmm_of(PyObject* const* a, const at::Tensor* probs) {
     Mask* m = mask_of(a[0]);
     if (!m) return nullptr;
     try {
@@ -466,7 +466,11 @@ PyObject* py_sddmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
 #define SPLAT_ARGS                                                                                                                     \
     x->data_ptr(), x->stride(0), x->stride(1), x->stride(2), y.data_ptr(), y.stride(0), y.stride(1), y.stride(2), y.stride(3),        \
         out->data_ptr(), m->segs, m->n_seg, B, H, L, keys, d, T, (float)scale, code, out_code
-        if (m->plan.defined())
+        if (probs)
+            rc = api.sddmm_softmax(x->data_ptr(), x->stride(0), x->stride(1), x->stride(2), y.data_ptr(), y.stride(0), y.stride(1), y.stride(2),
+                                   y.stride(3), out->data_ptr(), probs->data_ptr(), m->segs, m->n_seg, B, H, L, keys, d, T, (float)scale, code,
+                                   out_code, m->plan.defined() ? m->plan_ptr() : nullptr, m->plan.defined() ? m->plan_bytes() : 0, st);
+        else if (m->plan.defined())
             rc = api.sddmm_planned(SPLAT_ARGS, lse, m->plan_ptr(), m->plan_bytes(), st);
         else if (lse)
             rc = api.sddmm_probs(SPLAT_ARGS, lse, st);
@@ -478,6 +482,11 @@ PyObject* py_sddmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     } catch (...) {
         return raise_current();
     }
+}
+
+PyObject* py_sddmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 6) return PyErr_Format(PyExc_TypeError, "sddmm takes 6 arguments");
+    return sddmm_of(a, nullptr);
 }
 
 // softmax(mask, x, output) -> bool
@@ -548,10 +557,15 @@ PyObject* py_operators(PyObject*, PyObject* const* a, Py_ssize_t n) {
     PyObject* const first[] = {mask, a[4], a[5], a[7], a[10], Py_None};
     PyObject* const second[] = {a[2], a[7], a[8]};
     PyObject* const third[] = {a[3], a[8], a[6], a[9]};
-    PyObject* did = py_sddmm(nullptr, first, 6);
+    const at::Tensor *scores = tensor4(a[7], dev), *probs = tensor4(a[8], dev);
+    const bool both = scores && probs && scores->scalar_type() == probs->scalar_type() && scores->sizes() == probs->sizes() &&
+                      probs->is_contiguous() && scores->data_ptr() != probs->data_ptr();
+    PyObject* did = sddmm_of(first, both ? probs : nullptr);
     if (did != Py_True) return did;
-    did = py_softmax(nullptr, second, 3);
-    if (did != Py_True) return did;
+    if (!both) {
+        did = py_softmax(nullptr, second, 3);
+        if (did != Py_True) return did;
+    }
     return py_spmm(nullptr, third, 4);
 }
 
@@ -742,7 +756,7 @@ PyObject* py_bind(PyObject*, PyObject* args) {
         !take("splat_attention_bwd", api.bwd) || !take("splat_attention_bwd_keys", api.bwd_keys) ||
         !take("splat_attention_bwd_f32", api.bwd_f32) || !take("splat_attention_bwd_keys_f32", api.bwd_keys_f32) || !take("splat_sddmm", api.sddmm) ||
         !take("splat_sddmm_probs", api.sddmm_probs) || !take("splat_sddmm_planned", api.sddmm_planned) ||
-        !take("splat_softmax", api.softmax) || !take("splat_spmm", api.spmm) || !take("splat_spmm_planned", api.spmm_planned) ||
+        !take("splat_softmax", api.softmax) || !take("splat_sddmm_softmax", api.sddmm_softmax) || !take("splat_spmm", api.spmm) || !take("splat_spmm_planned", api.spmm_planned) ||
         !take("splat_acsr_build_record", api.build_record) || !take("splat_attention_plan_report", api.plan_report))
         return nullptr;
     Py_INCREF(err);

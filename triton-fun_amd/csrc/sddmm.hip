@@ -486,7 +486,7 @@ using namespace splat;
 static int sddmm_common(const char* who, const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* kT, int64_t k_sb,
                         int64_t k_sh, int64_t k_sd, int64_t k_sl, void* out, const splat_acsr_seg* segs, int32_t n_seg, int32_t B,
                         int32_t H, int32_t L, int32_t n_keys, int32_t d, int32_t T, float scale, int32_t in_dtype,
-                        int32_t out_dtype, const float* row_lse, const void* plan, int64_t plan_bytes, void* stream) {
+                        int32_t out_dtype, const float* row_lse, const void* plan, int64_t plan_bytes, void* probs, void* stream) {
     if (!q || !kT || !out || !segs) return fail(SPLAT_E_NULL, "%s: null pointer argument", who);
     if (B <= 0 || H <= 0 || L <= 0 || n_keys <= 0 || d <= 0 || T <= 0)
         return fail(SPLAT_E_SHAPE, "%s: need B, H, L, n_keys, d, T > 0 (got %d, %d, %d, %d, %d, %d)", who, B, H, L, n_keys, d, T);
@@ -506,6 +506,8 @@ static int sddmm_common(const char* who, const void* q, int64_t q_sb, int64_t q_
     p.scale = scale;
     p.row_lse = row_lse;
     p.plan = nullptr;
+    p.probs = probs;
+    p.probs_vec = T % 8 == 0 && ((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(probs)) & 31) == 0;
     if (plan) {
         if ((reinterpret_cast<uintptr_t>(plan) & 15) != 0) return fail(SPLAT_E_ALIGN, "%s: the plan must be 16-byte aligned", who);
         const int64_t need = splat_attention_plan_bytes(segs, n_seg, L);
@@ -530,15 +532,17 @@ static int sddmm_common(const char* who, const void* q, int64_t q_sb, int64_t q_
         if (segs[k].slot_offset % 8 != 0) p.out_vec = 0;
     hipStream_t st = (hipStream_t)stream;
     begin_launch();
-    if (in_dtype != SPLAT_F32 && launch_sddmm_rows16(p, in_dtype, kt, st)) return check_launch(who);
-    if (const int rc = launch_sddmm_lines(who, p, in_dtype, st)) return rc < 0 ? rc : check_launch(who);
-    switch (in_dtype) {
-        case SPLAT_F32:
-            if (launch_sddmm_f32(p, kt, st)) return check_launch(who);
-            return launch_sddmm<float>(who, p, kt, st);
-        case SPLAT_F16: return launch_sddmm<f16>(who, p, kt, st);
-        default: return launch_sddmm<bf16>(who, p, kt, st);
-    }
+    int took = in_dtype != SPLAT_F32 ? launch_sddmm_rows16(p, in_dtype, kt, st) : launch_sddmm_f32(p, kt, st);
+    if (!took) took = launch_sddmm_lines(who, p, in_dtype, st);
+    int rc;
+    if (took)
+        rc = took < 0 ? took : check_launch(who);
+    else if (in_dtype == SPLAT_F32)
+        rc = launch_sddmm<float>(who, p, kt, st);
+    else
+        rc = in_dtype == SPLAT_F16 ? launch_sddmm<f16>(who, p, kt, st) : launch_sddmm<bf16>(who, p, kt, st);
+    if (rc || !probs || took == 2) return rc;
+    return splat_softmax(out, probs, segs, n_seg, (int64_t)B * H, L, T, out_dtype, out_dtype, stream);
 }
 
 extern "C" int splat_sddmm(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* kT, int64_t k_sb, int64_t k_sh,
@@ -546,7 +550,7 @@ extern "C" int splat_sddmm(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_
                            int32_t L, int32_t n_keys, int32_t d, int32_t T, float scale, int32_t in_dtype, int32_t out_dtype,
                            void* stream) {
     return sddmm_common("splat_sddmm", q, q_sb, q_sh, q_sl, kT, k_sb, k_sh, k_sd, k_sl, out, segs, n_seg, B, H, L, n_keys, d, T,
-                        scale, in_dtype, out_dtype, nullptr, nullptr, 0, stream);
+                        scale, in_dtype, out_dtype, nullptr, nullptr, 0, nullptr, stream);
 }
 
 extern "C" int splat_sddmm_probs(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* kT, int64_t k_sb,
@@ -557,7 +561,7 @@ extern "C" int splat_sddmm_probs(const void* q, int64_t q_sb, int64_t q_sh, int6
     if (!lse) return fail(SPLAT_E_NULL, "%s: null lse", who);
     if ((reinterpret_cast<uintptr_t>(lse) & 3) != 0) return fail(SPLAT_E_ALIGN, "%s: lse must be 4-byte aligned", who);
     return sddmm_common(who, q, q_sb, q_sh, q_sl, kT, k_sb, k_sh, k_sd, k_sl, out, segs, n_seg, B, H, L, n_keys, d, T, scale,
-                        in_dtype, out_dtype, lse, nullptr, 0, stream);
+                        in_dtype, out_dtype, lse, nullptr, 0, nullptr, stream);
 }
 
 extern "C" int splat_sddmm_planned(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* kT, int64_t k_sb,
@@ -569,5 +573,15 @@ extern "C" int splat_sddmm_planned(const void* q, int64_t q_sb, int64_t q_sh, in
     if (!plan) return fail(SPLAT_E_NULL, "%s: null plan", who);
     if (lse && (reinterpret_cast<uintptr_t>(lse) & 3) != 0) return fail(SPLAT_E_ALIGN, "%s: lse must be 4-byte aligned", who);
     return sddmm_common(who, q, q_sb, q_sh, q_sl, kT, k_sb, k_sh, k_sd, k_sl, out, segs, n_seg, B, H, L, n_keys, d, T, scale,
-                        in_dtype, out_dtype, lse, plan, plan_bytes, stream);
+                        in_dtype, out_dtype, lse, plan, plan_bytes, nullptr, stream);
+}
+
+extern "C" int splat_sddmm_softmax(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* kT, int64_t k_sb,
+                                   int64_t k_sh, int64_t k_sd, int64_t k_sl, void* out, void* probs, const splat_acsr_seg* segs,
+                                   int32_t n_seg, int32_t B, int32_t H, int32_t L, int32_t n_keys, int32_t d, int32_t T, float scale,
+                                   int32_t in_dtype, int32_t out_dtype, const void* plan, int64_t plan_bytes, void* stream) {
+    const char* who = "splat_sddmm_softmax";
+    if (!probs) return fail(SPLAT_E_NULL, "%s: null probs", who);
+    return sddmm_common(who, q, q_sb, q_sh, q_sl, kT, k_sb, k_sh, k_sd, k_sl, out, segs, n_seg, B, H, L, n_keys, d, T, scale,
+                        in_dtype, out_dtype, nullptr, plan, plan_bytes, probs, stream);
 }

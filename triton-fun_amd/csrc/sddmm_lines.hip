@@ -317,9 +317,9 @@ __global__ __launch_bounds__(BM_ * 4, 4) void sddmm_lines_kernel(const SddmmPara
                 r[3] = __builtin_amdgcn_alignbit(x4, x3, sh);
                 return r;
             };
-            // 8 slots: around the cache where rows start on 16-byte boundaries, through it at any other alignment
+            // 8 slots: around the cache where rows start on 16-byte boundaries and nobody here reads them again, through it otherwise
             auto store8 = [&](T* dst, const u32x4& val) {
-                if (!PART || p.out_vec)
+                if (!p.probs && (!PART || p.out_vec))
                     __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(dst));
                 else
                     __builtin_memcpy(dst, &val, 16);
@@ -387,6 +387,9 @@ __global__ __launch_bounds__(BM_ * 4, 4) void sddmm_lines_kernel(const SddmmPara
             });
         }
     }
+    if constexpr (PLANNED && !PROBS) {
+        if (p.probs) softmax_own_rows<T>(p, bh, r0 + rs * 16 * wave, rs);
+    }
 }
 
 template <typename T, int D, int NST, int KEYS, int HL, int BM, bool PROBS, bool PLANNED, bool PART>
@@ -398,13 +401,14 @@ static int launch_lines_variant(const char* who, SddmmParams p, hipStream_t st) 
     if (blocks > 0x7ffffff0) return 0;
     p.key_split = 1;
     p.total = (int)blocks;
+    if (!PLANNED || !own_rows_fit(p)) p.probs = nullptr;
     p.by_split = divisor(1), p.by_blocks = divisor(p.n_row_blocks), p.by_h = divisor(p.H);
     static uint64_t reserved = 0;
     auto kern = sddmm_lines_kernel<T, D, NST, KEYS, HL, BM, PROBS, PLANNED, PART>;
     if (int rc = reserve_dynamic_lds(&reserved, reinterpret_cast<const void*>(kern), G::LDS_BYTES, who)) return rc;
     const int grid = ((p.total + 7) / 8) * 8;
     kern<<<grid, BM * 4, G::LDS_BYTES, st>>>(p);
-    return 1;
+    return p.probs ? 2 : 1;
 }
 
 // Whole 128-byte lines are what the memory system likes best (a blocked mask at d = 128: 0.25 ms against 0.34 ms with

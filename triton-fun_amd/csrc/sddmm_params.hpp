@@ -1,7 +1,10 @@
 // Kernel arguments of the SDDMM kernels (sddmm.hip: every shape; sddmm_lines.hip, sddmm_rows16.hip: 16-bit types, operators_f32.hip: float32,
 // up to 128 inner values).
 #pragma once
+#include <type_traits>
+
 #include "acsr_plan.hpp"
+#include "softmax_rows.hpp"
 
 namespace splat {
 
@@ -24,10 +27,57 @@ struct SddmmParams {
     Divisor by_split, by_blocks, by_h;  // key_split, row blocks (or halves) per head, H: filled in by the launches that read them
     int key_split;  // workgroups per row block: each takes a contiguous share of every segment's tiles
     const PlanRec* plan;  // optional: the mask's plan table for 128-row blocks (variant for row-major K), else nullptr
+    void* probs;  // optional, like out: the softmax of its rows as well, by the wavefronts that have stored them
+    int probs_vec;  // T % 8 == 0, and out and probs start on 32-byte boundaries
 };
 
-// Launches the line-wise kernel when the problem has its shape (see sddmm_lines.hip); returns 1 when it did, 0 when the
-// general kernel has to run, a negative code on errors.  `p` is complete except for key_split / total.
+// Whether softmax_own_rows pays: rows of up to 256 slots (of 300 1.05 of the time of a launch for each, of 512 1.03 to 1.13), and 16-bit
+// scores that the caches hold: the three operators, causal masks of 33 to 256 slots, d = 64 and 128: up to 64 MB of scores 0.68 to 0.97
+// of the time, from 90 to 134 MB 0.97 to 1.12.  (Scores and probabilities are stored through the caches then: 4096 rows of 200 slots, 16 heads,
+// d = 128 60 -> 41 us, of which 53 around them.)  Not where a stride between a block's rows leaves most of them empty (224 heads of
+// 128 rows, 21 slots with step 3: 18.7 -> 20.6).
+inline bool own_rows_fit(const SddmmParams& p) {
+    return p.probs && !p.row_lse && p.T <= 256 && (p.row_stride == 1 || p.L >= 128 * p.row_stride) && (p.out_dtype == SPLAT_F32 || (int64_t)p.B * p.H * p.L * p.T <= (int64_t)1 << 25);
+}
+
+// The softmax of the 16 rows r0 + rs * k of head bh that this wavefront, and nobody else, has stored: they come from the cache, and a launch
+// of their own is spared.  The splits of a row over lanes are launch_softmax's: the same bits.
+// float16, 16 heads of 2000 rows, 129 slots, d = 80, the three operators: 26.7 -> 21 us; bfloat16, 208 heads of 128 rows, 64 slots: 16.7 -> 13.6.
+template <typename T>
+__device__ __forceinline__ void softmax_own_rows(const SddmmParams& p, int bh, int r0, int rs) {
+    if (r0 >= p.L) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // stores and the loads that follow them are not ordered otherwise
+    SoftmaxSegs segs;
+    segs.n = p.n_seg;
+#pragma unroll
+    for (int k = 0; k < SPLAT_MAX_SEGMENTS; ++k) segs.nnz[k] = k < p.n_seg ? p.seg[k].nnz : p.seg[0].nnz, segs.off[k] = p.seg[k].slot_offset;
+    const int lane = threadIdx.x & 63, T_ = p.T;
+    const int64_t first = (int64_t)bh * p.L;
+    auto go = [&](auto nch, auto lpr, auto aligned) {
+        constexpr int NCH = decltype(nch)::value, LPR = decltype(lpr)::value, RPW = 64 / LPR, RIF = 16 / RPW < 4 ? 16 / RPW : 4;
+        for (int k0 = 0; k0 < 16; k0 += RPW * RIF) {
+            if (r0 + rs * k0 >= p.L) break;
+            softmax_rows<T, T, NCH, LPR, RIF, decltype(aligned)::value, false>((const T*)p.out, (T*)p.probs, segs, T_, [&](int i, int64_t& row, int& in_head) {
+                const int at = r0 + rs * (k0 + RPW * i + lane / LPR);
+                in_head = at < p.L ? at : r0;
+                row = first + in_head;
+                return at < p.L;
+            });
+        }
+    };
+    using std::integral_constant;
+    if (p.probs_vec) {
+        if (T_ <= 128) go(integral_constant<int, 1>{}, integral_constant<int, 16>{}, std::true_type{});
+        else go(integral_constant<int, 1>{}, integral_constant<int, 32>{}, std::true_type{});
+    } else {
+        if (T_ <= 128) go(integral_constant<int, 1>{}, integral_constant<int, 16>{}, std::false_type{});
+        else if (sizeof(T) == 2) go(integral_constant<int, 4>{}, integral_constant<int, 8>{}, std::false_type{});
+        else go(integral_constant<int, 1>{}, integral_constant<int, 32>{}, std::false_type{});
+    }
+}
+
+// Launches the line-wise kernel when the problem has its shape (see sddmm_lines.hip); returns 1 when it did, 2 when it took the
+// softmax as well, 0 when the general kernel has to run, a negative code on errors.  `p` is complete except for key_split / total.
 int launch_sddmm_lines(const char* who, const SddmmParams& p, int in_dtype, hipStream_t st);
 // The same for 16-bit launches of few row blocks (see sddmm_rows16.hip); `kt`: K is stored along the keys.
 int launch_sddmm_rows16(const SddmmParams& p, int in_dtype, bool kt, hipStream_t st);

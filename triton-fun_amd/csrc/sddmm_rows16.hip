@@ -177,6 +177,7 @@ __global__ __launch_bounds__(256, 4) void sddmm_rows16_kernel(const SddmmParams 
             stage ^= STAGE;
         }
     }
+    if (p.probs) softmax_own_rows<T>(p, bh, r0 + rs * 16 * wave, rs);
 }
 
 int launch_sddmm_rows16(const SddmmParams& p0, int in_dtype, bool kt, hipStream_t st) {
@@ -205,6 +206,10 @@ int launch_sddmm_rows16(const SddmmParams& p0, int in_dtype, bool kt, hipStream_
     const bool fills = !kt && p.plan && (p.T <= 40 ? blocks <= 16384 : ragged && blocks > 1024 && blocks <= 4096);
     if (blocks > most && !fills) return 0;
     p.key_split = (int)std::min<int64_t>((p.T + kTile - 1) / kTile + 2, std::max<int64_t>(1, 512 / blocks));
+    // Whole rows where their softmax follows here: at 256 blocks 0.80 to 0.97 of the three launches' time (33 to 256 slots, d = 64 and 128)
+    // against those with two workgroups a block; at 192 0.92 to 1.14, and below, where more share a block, up to 1.25.
+    if (blocks >= 256 && own_rows_fit(p)) p.key_split = 1;
+    if (p.key_split != 1 || !own_rows_fit(p)) p.probs = nullptr;
     p.total = (int)(blocks * p.key_split);
     p.by_split = divisor(p.key_split), p.by_blocks = divisor(2 * p.n_row_blocks), p.by_h = divisor(p.H);
     const int grid = ((p.total + 7) / 8) * 8;
@@ -219,7 +224,7 @@ int launch_sddmm_rows16(const SddmmParams& p0, int in_dtype, bool kt, hipStream_
     auto by_type = [&](auto kt_c) { return in_dtype == SPLAT_BF16 ? go(bf16{}, kt_c) : go(f16{}, kt_c); };
     if (kt) by_type(std::true_type{});
     else by_type(std::false_type{});
-    return 1;
+    return p.probs ? 2 : 1;
 }
 
 }  // namespace splat
