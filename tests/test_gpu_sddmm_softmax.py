@@ -79,3 +79,29 @@ def test_softmax_of_few_and_many_rows(dev, T, rows, dtype):
             assert float(torch.where(live & (ref > 1e-4), err, 0.0).max()) <= 128 * 2.0 ** -24 + torch.finfo(dtype).eps / 2 * 1.01
             assert torch.all(part.double()[~live.expand_as(part)] == SENTINEL)
         assert torch.all(buf[:shift] == SENTINEL) and torch.all(buf[shift + BH * L * T:] == SENTINEL)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T", [304, 320])
+@pytest.mark.parametrize("planned", [True, False])
+def test_large_matrices_equal_their_halves(dev, planned, T, dtype):
+    """Scores and probabilities that the caches do not hold are stored around them; the halves of the same heads are not: the same bits."""
+    L, d, heads = 2048, 32, 68
+    segs = A.create_acsr_segments([A.causal_windowed_pattern(L, T - 1)], 16, dev)
+    assert segs.T == T
+    g = torch.Generator(device=dev).manual_seed(T)
+    q, k = (torch.randn(1, heads, L, d, generator=g, device=dev).to(dtype) for _ in range(2))
+    arr, code, stream, plan = segs.seg_array(L, T), hip.dtype_code(dtype), hip.stream_ptr(dev), segs.plan(L, dev)
+
+    def both(h0, n):
+        s, p = (torch.full((n, L, T), SENTINEL, dtype=dtype, device=dev) for _ in range(2))
+        a, b = q[:, h0:h0 + n], k[:, h0:h0 + n].transpose(2, 3)
+        table = (None, plan.data_ptr(), plan.numel() * plan.element_size()) if planned else ()
+        hip.check((hip.lib().splat_sddmm_planned if planned else hip.lib().splat_sddmm)(
+            a.data_ptr(), *a.stride()[:3], b.data_ptr(), *b.stride()[:4], s.data_ptr(), arr, 1, 1, n, L, L, d, T, ctypes.c_float(0.2), code,
+            code, *table, stream), "splat_sddmm")
+        hip.check(hip.lib().splat_softmax(s.data_ptr(), p.data_ptr(), arr, 1, n, L, T, code, code, stream), "splat_softmax")
+        return s, p
+    whole, parts = both(0, heads), [both(0, heads // 2), both(heads // 2, heads // 2)]
+    for i in range(2):
+        assert torch.equal(whole[i], torch.cat([x[i] for x in parts]))

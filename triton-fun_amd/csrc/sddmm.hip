@@ -213,7 +213,7 @@ __global__ __launch_bounds__(256, (KSU > 0 && KSU * 16 < SddmmGeom<T>::DC && !KT
         // untested: a position outside the row's span lands on ring entries that are not waiting to be stored.  After each
         // tile every row stores the 64-slot lines that have become complete (and, once its last position has passed,
         // the rest), 8 lanes x 16 bytes per line: whole aligned lines instead of pieces that straddle them, which is
-        // what lets them bypass the L2's write combining (non-temporal stores).
+        // what lets those of large outputs bypass the L2 (non-temporal stores).
         // (measured: rows of four or five lines gain 13 % in launches of 4096 row blocks and lose 5 % in one of 2048)
         const bool use_ring = pl.uniform && p.key_split == 1 && p.out_dtype != SPLAT_F32 &&
                               (p.T >= 384 || (p.T >= 256 && p.total >= 4096));
@@ -385,7 +385,7 @@ __global__ __launch_bounds__(256, (KSU > 0 && KSU * 16 < SddmmGeom<T>::DC && !KT
                         v8 val;
                         __builtin_memcpy(&val, stg + (8 * c + (lane >> 3)) * R_ROW + rix * 2, 16);
                         TO* const dst = (TO*)p.out + f_base[c] + s0;
-                        if (p.out_vec) {
+                        if (p.out_stream) {
                             __builtin_nontemporal_store(val, reinterpret_cast<v8*>(dst));
                         } else {
                             __builtin_memcpy(dst, &val, 16);
@@ -410,7 +410,7 @@ __global__ __launch_bounds__(256, (KSU > 0 && KSU * 16 < SddmmGeom<T>::DC && !KT
                             TO* const dst = (TO*)p.out + f_base[c] + s0;
                             const int n = f_cnt[c] - s0;
                             if (n >= 8) {
-                                if (p.out_vec) {
+                                if (p.out_stream) {
                                     __builtin_nontemporal_store(val, reinterpret_cast<v8*>(dst));
                                 } else {
                                     __builtin_memcpy(dst, &val, 16);
@@ -530,6 +530,13 @@ static int sddmm_common(const char* who, const void* q, int64_t q_sb, int64_t q_
     p.out_vec = (al(out) && T % 8 == 0) ? 1 : 0;
     for (int k = 0; k < n_seg; ++k)
         if (segs[k].slot_offset % 8 != 0) p.out_vec = 0;
+    // Stores around the caches pay for large outputs of whole 64-byte pieces.  The three operators, bfloat16, causal masks, d = 64 and 128, share
+    // of the time with them: 150 to 540 MB of 288 to 512 slots, a multiple of 32, 0.85 to 0.99; of 200 or 304 slots, whose rows share such
+    // pieces, 1.05 to 1.31, of 1000 1.25 to 1.44; and up to 80 MB, which the next operator finds in the caches, 1.02 to 1.17 (from 88 to
+    // 134 MB 0.88 to 1.17).
+    p.out_stream = p.out_vec && T % 32 == 0 && (int64_t)B * H * L * T * 2 > kCachedBytes;
+    for (int k = 0; k < n_seg; ++k)
+        if (segs[k].slot_offset % 32 != 0) p.out_stream = 0;
     hipStream_t st = (hipStream_t)stream;
     begin_launch();
     int took = in_dtype != SPLAT_F32 ? launch_sddmm_rows16(p, in_dtype, kt, st) : launch_sddmm_f32(p, kt, st);

@@ -18,7 +18,7 @@
 // Output, uniform plans (every row of the block has the plan's column step and phase, so tile positions are slots): per
 // 32 positions the scores go from the accumulators into a per-row ring of 64 slots in LDS (four consecutive slots per
 // write, no tests: a position outside the row's span lands on ring entries that are not waiting to be stored), and each
-// row stores the 32-slot half lines that have become complete -- 4 lanes x 16 bytes, aligned, non-temporal -- and its
+// row stores the 32-slot half lines that have become complete -- 4 lanes x 16 bytes -- and its
 // remainder once its last position has passed.  The ring is filled at position granularity and read at slot granularity:
 // a lane reads the 24 aligned bytes around its 8 slots and shifts (a 16-byte LDS read at a 2-byte offset costs several
 // times an aligned one).  Other plans (rows with differing steps) walk dense columns and store element by element under
@@ -27,7 +27,7 @@
 // PART: a key row fills d / 8 of the stage row's chunks; the lanes of a copy whose chunk lies past it sit the copy out (every
 // copy instruction covers a whole stage row, so it always has lanes), and those chunks hold the zeros written once at the
 // start, so that an infinity in K meets no padding.  Contraction steps past d are skipped.  Rows of the compressed matrix
-// that start anywhere are stored through the cache, which joins the lines that two units share.  The bound is as above;
+// that start anywhere, or that the caches hold, are stored through the cache, which joins the lines that two units share.  The bound is as above;
 // 16 heads of 2000 rows, 129 slots, d = 80, float16: 23.4 us in the general kernel (256 workgroups of four wavefronts,
 // one step in flight), 12.4 here; the shapes below the
 // block limit gain as much (4 heads of 1000 rows, 255 slots, d = 96, the three operators: 51 -> 31 us).
@@ -317,9 +317,9 @@ __global__ __launch_bounds__(BM_ * 4, 4) void sddmm_lines_kernel(const SddmmPara
                 r[3] = __builtin_amdgcn_alignbit(x4, x3, sh);
                 return r;
             };
-            // 8 slots: around the cache where rows start on 16-byte boundaries and nobody here reads them again, through it otherwise
+            // 8 slots, at any alignment where they go through the cache
             auto store8 = [&](T* dst, const u32x4& val) {
-                if (!p.probs && (!PART || p.out_vec))
+                if (p.out_stream)
                     __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(dst));
                 else
                     __builtin_memcpy(dst, &val, 16);
@@ -402,6 +402,7 @@ static int launch_lines_variant(const char* who, SddmmParams p, hipStream_t st) 
     p.key_split = 1;
     p.total = (int)blocks;
     if (!PLANNED || !own_rows_fit(p)) p.probs = nullptr;
+    if (p.probs) p.out_stream = 0;
     p.by_split = divisor(1), p.by_blocks = divisor(p.n_row_blocks), p.by_h = divisor(p.H);
     static uint64_t reserved = 0;
     auto kern = sddmm_lines_kernel<T, D, NST, KEYS, HL, BM, PROBS, PLANNED, PART>;

@@ -23,6 +23,7 @@ struct SddmmParams {
     int n_row_blocks, total;
     int q_vec, k_vec;  // 16-byte loads are legal for q / k
     int out_vec;       // 16-bit outputs: every row's segment starts on a 16-byte boundary
+    int out_stream;    // they are stored around the caches, in whole lines
     int row_stride;
     Divisor by_split, by_blocks, by_h;  // key_split, row blocks (or halves) per head, H: filled in by the launches that read them
     int key_split;  // workgroups per row block: each takes a contiguous share of every segment's tiles

@@ -13,14 +13,14 @@
 
 namespace splat {
 
-template <typename Tin, typename Tout, int NCH, int LPR, int RIF, bool ALIGNED>
+template <typename Tin, typename Tout, int NCH, int LPR, int RIF, bool ALIGNED, bool AROUND>
 __global__ __launch_bounds__(256) void softmax_rows_vec(const Tin* __restrict__ x, Tout* __restrict__ y, SoftmaxSegs segs,
                                                         int64_t n_rows, int L, int T, Divisor by_l) {
     load_args(x, y, n_rows, L, T, by_l.m, by_l.shift, segs.n, segs.nnz[0], segs.off[0]);
     constexpr int RPW = 64 / LPR;  // rows per wavefront and group
     const int64_t row0 = (((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * RIF) * RPW + ((threadIdx.x & 63) / LPR);
     if (RPW == 1 && row0 >= n_rows) return;
-    softmax_rows<Tin, Tout, NCH, LPR, RIF, ALIGNED, true>(x, y, segs, T, [&](int i, int64_t& row, int& in_head) {
+    softmax_rows<Tin, Tout, NCH, LPR, RIF, ALIGNED, AROUND>(x, y, segs, T, [&](int i, int64_t& row, int& in_head) {
         const int64_t at = row0 + (int64_t)i * RPW;
         row = at < n_rows ? at : n_rows - 1;
         in_head = n_rows < ((int64_t)1 << 31) ? (int)row - quotient((int)row, by_l) * L : (int)(row % L);
@@ -63,35 +63,39 @@ static int launch_softmax(const void* x, void* y, const SoftmaxSegs& segs, int64
     const Divisor by_l = divisor(L);
     if (T <= 2048) {
         auto groups = [&](int rows_per_wave) { return (unsigned)((n_rows + 4 * rows_per_wave - 1) / (4 * rows_per_wave)); };
-        auto go = [&](auto aligned_c) {
-            constexpr bool ALIGNED = decltype(aligned_c)::value;
+        auto go = [&](auto aligned_c, auto around_c) {
+            constexpr bool ALIGNED = decltype(aligned_c)::value, AROUND = decltype(around_c)::value;
             // Row groups in flight per wavefront: one for short rows and where that leaves fewer wavefronts than the chip has room for
             // (1024 rows of 256 slots 5.7 -> 3.0 us, 16384 of 512, float32, 16.6 -> 14.0), four for 16-bit rows in large launches (131072
             // rows: 256 slots 27.1 -> 26.4, 512 slots 50.6 -> 43.6; float32 56.1 and 103.7 against 51.1 and 99.3 with one).
             const bool few = n_rows <= (sizeof(Tin) == 4 ? 1 << 17 : 20000);
             if (T <= 128)
-                softmax_rows_vec<Tin, Tout, 1, 16, 1, ALIGNED><<<groups(4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
+                softmax_rows_vec<Tin, Tout, 1, 16, 1, ALIGNED, AROUND><<<groups(4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
             else if (T <= 256 && !ALIGNED && sizeof(Tin) == 2)
                 // eight rows of odd lengths share a wavefront's instructions: 262144 rows, 129 slots 37.3 -> 26.7 us over 32 lanes a row, 191 38.8
                 // -> 32.9 (float32 is better off with those: 191 slots 99 against 79)
-                softmax_rows_vec<Tin, Tout, 4, 8, 1, ALIGNED><<<groups(8), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
+                softmax_rows_vec<Tin, Tout, 4, 8, 1, ALIGNED, AROUND><<<groups(8), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
             else if (T <= 256 && few)
-                softmax_rows_vec<Tin, Tout, 1, 32, 1, ALIGNED><<<groups(2), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
+                softmax_rows_vec<Tin, Tout, 1, 32, 1, ALIGNED, AROUND><<<groups(2), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
             else if (T <= 256)
-                softmax_rows_vec<Tin, Tout, 1, 32, 4, ALIGNED><<<groups(2 * 4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
+                softmax_rows_vec<Tin, Tout, 1, 32, 4, ALIGNED, AROUND><<<groups(2 * 4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
             else if (T <= 512 && few)
-                softmax_rows_vec<Tin, Tout, 1, 64, 1, ALIGNED><<<groups(1), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
+                softmax_rows_vec<Tin, Tout, 1, 64, 1, ALIGNED, AROUND><<<groups(1), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
             else if (T <= 512)
-                softmax_rows_vec<Tin, Tout, 1, 64, 4, ALIGNED><<<groups(4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
+                softmax_rows_vec<Tin, Tout, 1, 64, 4, ALIGNED, AROUND><<<groups(4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
             else if (T <= 1024)
-                softmax_rows_vec<Tin, Tout, 2, 64, 1, ALIGNED><<<groups(1), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
+                softmax_rows_vec<Tin, Tout, 2, 64, 1, ALIGNED, AROUND><<<groups(1), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
             else
-                softmax_rows_vec<Tin, Tout, 4, 64, 1, ALIGNED><<<groups(1), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
+                softmax_rows_vec<Tin, Tout, 4, 64, 1, ALIGNED, AROUND><<<groups(1), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
         };
-        if (aligned && T % 8 == 0)
-            go(std::true_type{});
+        if (!aligned || T % 8 != 0)
+            go(std::false_type{}, std::false_type{});
+        // (through the caches where the rows are there and where the next operator finds them there: the three operators, bfloat16 and float32,
+        // d = 64 and 128, 300 to 1000 slots, up to 80 MB 0.86 to 0.97 of the time around them; 134 to 270 MB 1.00 to 1.10)
+        else if (n_rows * T * (int64_t)sizeof(Tin) <= kCachedBytes)
+            go(std::true_type{}, std::false_type{});
         else
-            go(std::false_type{});
+            go(std::true_type{}, std::true_type{});
     } else {
         softmax_rows_any<Tin, Tout><<<grid, 256, 0, st>>>(xi, yo, segs, n_rows, L, T);
     }

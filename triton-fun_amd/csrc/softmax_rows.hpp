@@ -62,6 +62,9 @@ struct Vec8 {
     typedef T type __attribute__((ext_vector_type(8)));
 };
 
+// Bytes of a compressed matrix that the next kernel still finds in the last-level cache (256 MB, with its operands and results).
+constexpr int64_t kCachedBytes = (int64_t)80 << 20;
+
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kNegBig = -1.0e30f;
 
