@@ -874,3 +874,17 @@ def test_key_transpose(dev, L, d, dtype):
         got = A.transpose_keys(kT)
         assert got.is_contiguous() and tuple(got.shape) == (B, H, L, d)
         assert torch.equal(got, kT.transpose(2, 3).contiguous())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("L", [7, 8, 9, 127, 128, 129, 135, 263])
+@pytest.mark.parametrize("d", [8, 60, 64, 72, 136])
+def test_key_transpose_16_bit_edges(dev, L, d, dtype):
+    """Edges of the 16-bit turn's tiles (128 keys, 64 values of d, pieces of 8): rows cut inside a piece, rows shorter than one, tiles
+    of d that are partly there, rows that start on any 2-byte boundary, every bit pattern."""
+    g = torch.Generator().manual_seed(L * 137 + d)
+    wide = torch.randint(-32768, 32768, (3, 2, d, L + 5), generator=g, dtype=torch.int16).view(dtype).to(dev)
+    for off in (0, 1, 5):
+        kT = wide[..., off:off + L]
+        got = A.transpose_keys(kT)
+        assert got.is_contiguous() and torch.equal(got.view(torch.int16), kT.transpose(2, 3).contiguous().view(torch.int16))
