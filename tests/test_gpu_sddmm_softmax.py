@@ -105,3 +105,32 @@ def test_large_matrices_equal_their_halves(dev, planned, T, dtype):
     whole, parts = both(0, heads), [both(0, heads // 2), both(heads // 2, heads // 2)]
     for i in range(2):
         assert torch.equal(whole[i], torch.cat([x[i] for x in parts]))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [300, 140000])  # (small, and beyond what the caches hold)
+@pytest.mark.parametrize("T", [130, 192, 264, 376, 384, 385, 392, 440, 448, 449, 456, 505, 512])
+def test_softmax_16_bit_rows_over_lanes(dev, T, rows, dtype):
+    """Edges of the splits of a 16-bit row over lanes, two segments with dead slots between and after them, in place, against float64."""
+    g = torch.Generator(device=dev).manual_seed(T)
+    L, off = 50, T * 2 // 3 - 1
+    cnt = [torch.randint(0, n + 1, (L,), generator=g, device=dev).float() for n in (off, T - off)]
+    cnt[0][::3], cnt[1][::3] = off, T - off
+    cnt[0][1], cnt[1][1] = 0, 0
+    seg = (hip.AcsrSeg * 2)()
+    for k in range(2):
+        seg[k].sTod_lin = seg[k].sTod_trans = seg[k].nnz = cnt[k].data_ptr()
+        seg[k].slot_offset = (0, off)[k]
+    BH = rows // L
+    x = (torch.randn(BH, L, T, generator=g, device=dev) * 3).to(dtype)
+    slot = torch.arange(T, device=dev)[None]
+    live = (slot < cnt[0][:, None]) | ((slot >= off) & (slot < off + cnt[1][:, None]))
+    want = torch.softmax(torch.cat([x[:32], x[-1:]]).double().masked_fill(~live, float("-inf")), -1)
+    dead = torch.cat([x[:32], x[-1:]])
+    hip.check(hip.lib().splat_softmax(x.data_ptr(), x.data_ptr(), seg, 2, BH, L, T, hip.dtype_code(dtype), hip.dtype_code(dtype),
+                                      hip.stream_ptr(dev)), "splat_softmax")
+    got = torch.cat([x[:32], x[-1:]])
+    err = (got.double() - want).abs() / want.clamp_min(1e-30)
+    # (as above; probabilities above 1e-4 are normal numbers of both types)
+    assert float(torch.where(live & (want > 1e-4), err, 0.0).max()) <= 128 * 2.0 ** -24 + torch.finfo(dtype).eps / 2 * 1.01
+    assert torch.equal(got[~live.expand_as(got)], dead[~live.expand_as(got)])

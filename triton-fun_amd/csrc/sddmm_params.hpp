@@ -55,7 +55,7 @@ __device__ __forceinline__ void softmax_own_rows(const SddmmParams& p, int bh, i
     const int lane = threadIdx.x & 63, T_ = p.T;
     const int64_t first = (int64_t)bh * p.L;
     auto go = [&](auto nch, auto lpr, auto aligned) {
-        constexpr int NCH = decltype(nch)::value, LPR = decltype(lpr)::value, RPW = 64 / LPR, RIF = 16 / RPW < 4 ? 16 / RPW : 4;
+        constexpr int NCH = decltype(nch)::value, LPR = decltype(lpr)::value, RPW = 64 / LPR, RIF = NCH == 1 ? 4 : 2;
         for (int k0 = 0; k0 < 16; k0 += RPW * RIF) {
             if (r0 + rs * k0 >= p.L) break;
             softmax_rows<T, T, NCH, LPR, RIF, decltype(aligned)::value, false>((const T*)p.out, (T*)p.probs, segs, T_, [&](int i, int64_t& row, int& in_head) {
@@ -69,6 +69,7 @@ __device__ __forceinline__ void softmax_own_rows(const SddmmParams& p, int bh, i
     using std::integral_constant;
     if (p.probs_vec) {
         if (T_ <= 128) go(integral_constant<int, 1>{}, integral_constant<int, 16>{}, std::true_type{});
+        else if (sizeof(T) == 2) go(integral_constant<int, 2>{}, integral_constant<int, 16>{}, std::true_type{});
         else go(integral_constant<int, 1>{}, integral_constant<int, 32>{}, std::true_type{});
     } else {
         if (T_ <= 128) go(integral_constant<int, 1>{}, integral_constant<int, 16>{}, std::false_type{});

@@ -65,25 +65,56 @@ static int launch_softmax(const void* x, void* y, const SoftmaxSegs& segs, int64
         auto groups = [&](int rows_per_wave) { return (unsigned)((n_rows + 4 * rows_per_wave - 1) / (4 * rows_per_wave)); };
         auto go = [&](auto aligned_c, auto around_c) {
             constexpr bool ALIGNED = decltype(aligned_c)::value, AROUND = decltype(around_c)::value;
-            // Row groups in flight per wavefront: one for short rows and where that leaves fewer wavefronts than the chip has room for
-            // (1024 rows of 256 slots 5.7 -> 3.0 us, 16384 of 512, float32, 16.6 -> 14.0), four for 16-bit rows in large launches (131072
-            // rows: 256 slots 27.1 -> 26.4, 512 slots 50.6 -> 43.6; float32 56.1 and 103.7 against 51.1 and 99.3 with one).
-            const bool few = n_rows <= (sizeof(Tin) == 4 ? 1 << 17 : 20000);
-            if (T <= 128)
+            // 16-bit rows of 129 to 512 slots: 16 lanes a row, one to four chunks each, so that four rows share a wavefront's instructions and lanes
+            // idle for less than a chunk in 128 slots.  Against 32 or 64 lanes a row and four row groups in flight (one up to 20000 rows),
+            // us, bfloat16, 32000 / 72000 / 240000 rows: 136 slots 8.1 / 13.1 / 30.2 -> 5.9 / 10.5 / 27.7, 256 8.7 / 14.2 -> 6.4 / 13.4, 301 14.1 / 22.6 /
+            // 66.3 -> 8.9 / 16.4 / 49.5, 384 in two segments 16.1 / 28.5 / 85.3 -> 10.3 / 21.3 / 61.3, 448 14.1 / 23.2 / 70.5 -> 11.9 / 22.7 / 67.3.  Around
+            // the caches 32 lanes are as fast up to 256 slots (256: 40.9 both) or faster (200: 35.7 against 40.5), and so are 64 where they
+            // have a chunk each (512 slots, 524288 rows: 165.6 against 168.7).
+            if (T <= 128) {
                 softmax_rows_vec<Tin, Tout, 1, 16, 1, ALIGNED, AROUND><<<groups(4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
-            else if (T <= 256 && !ALIGNED && sizeof(Tin) == 2)
-                // eight rows of odd lengths share a wavefront's instructions: 262144 rows, 129 slots 37.3 -> 26.7 us over 32 lanes a row, 191 38.8
-                // -> 32.9 (float32 is better off with those: 191 slots 99 against 79)
-                softmax_rows_vec<Tin, Tout, 4, 8, 1, ALIGNED, AROUND><<<groups(8), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
-            else if (T <= 256 && few)
-                softmax_rows_vec<Tin, Tout, 1, 32, 1, ALIGNED, AROUND><<<groups(2), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
-            else if (T <= 256)
-                softmax_rows_vec<Tin, Tout, 1, 32, 4, ALIGNED, AROUND><<<groups(2 * 4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
-            else if (T <= 512 && few)
-                softmax_rows_vec<Tin, Tout, 1, 64, 1, ALIGNED, AROUND><<<groups(1), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
-            else if (T <= 512)
-                softmax_rows_vec<Tin, Tout, 1, 64, 4, ALIGNED, AROUND><<<groups(4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
-            else if (T <= 1024)
+                return;
+            }
+            if constexpr (sizeof(Tin) == 2) {
+                if (T <= 256) {
+                    if constexpr (!ALIGNED)
+                        // eight rows of odd lengths share a wavefront's instructions: 262144 rows, 129 slots 37.3 -> 26.7 us over 32 lanes a row, 191
+                        // 38.8 -> 32.9 (float32 is better off with those: 191 slots 99 against 79)
+                        softmax_rows_vec<Tin, Tout, 4, 8, 1, ALIGNED, AROUND><<<groups(8), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
+                    else if constexpr (!AROUND)
+                        softmax_rows_vec<Tin, Tout, 2, 16, 1, ALIGNED, AROUND><<<groups(4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
+                    else
+                        softmax_rows_vec<Tin, Tout, 1, 32, 4, ALIGNED, AROUND><<<groups(2 * 4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
+                    return;
+                }
+                if constexpr (AROUND) {
+                    if (T > 448 && T <= 512) {
+                        softmax_rows_vec<Tin, Tout, 1, 64, 4, ALIGNED, AROUND><<<groups(4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
+                        return;
+                    }
+                }
+                if (T <= 512) {
+                    if (T <= 384)
+                        softmax_rows_vec<Tin, Tout, 3, 16, 1, ALIGNED, AROUND><<<groups(4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
+                    else
+                        softmax_rows_vec<Tin, Tout, 4, 16, 1, ALIGNED, AROUND><<<groups(4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
+                    return;
+                }
+            } else if (T <= 512) {
+                // float32: one row group a wavefront, two of up to 256 slots, and four in flight in large launches (16384 rows of 512 slots 16.6 -> 14.0
+                // with one, 131072 56.1 and 103.7 against 51.1 and 99.3; 16 lanes a row 2 to 12 % slower up to 72000 rows)
+                const bool few = n_rows <= 1 << 17;
+                if (T <= 256 && few)
+                    softmax_rows_vec<Tin, Tout, 1, 32, 1, ALIGNED, AROUND><<<groups(2), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
+                else if (T <= 256)
+                    softmax_rows_vec<Tin, Tout, 1, 32, 4, ALIGNED, AROUND><<<groups(2 * 4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
+                else if (few)
+                    softmax_rows_vec<Tin, Tout, 1, 64, 1, ALIGNED, AROUND><<<groups(1), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
+                else
+                    softmax_rows_vec<Tin, Tout, 1, 64, 4, ALIGNED, AROUND><<<groups(4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
+                return;
+            }
+            if (T <= 1024)
                 softmax_rows_vec<Tin, Tout, 2, 64, 1, ALIGNED, AROUND><<<groups(1), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
             else
                 softmax_rows_vec<Tin, Tout, 4, 64, 1, ALIGNED, AROUND><<<groups(1), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
