@@ -175,7 +175,7 @@ int splat_softmax(const void* x, void* y, const splat_acsr_seg* segs /* host */,
 
 /* splat_sddmm_planned without statistics (plan may be NULL), then splat_softmax of its output into `probs` ([B,H,L,T]
  * contiguous, dtype out_dtype, not overlapping out; rows without live slots and dead slots stay as they are in both).
- * Where the wavefronts of the sampled product own whole rows of at most 256 slots (enough row blocks for the chip, and no
+ * Where the wavefronts of the sampled product own whole rows of at most 512 slots (float32: 256; enough row blocks for the chip, and no
  * more scores than the caches hold), they take their softmax as well, and a launch and a pass over memory are spared
  * (float16, 16 heads of 2000 rows, 129 slots, d = 80, with splat_spmm: 26.7 -> 21 us); elsewhere the second launch
  * follows.  Both results are those of the two calls, bit for bit.  Replaces r_sddmm.py:153-188 and r_softmax.py:126-150. */

@@ -134,3 +134,15 @@ def test_softmax_16_bit_rows_over_lanes(dev, T, rows, dtype):
     # (as above; probabilities above 1e-4 are normal numbers of both types)
     assert float(torch.where(live & (want > 1e-4), err, 0.0).max()) <= 128 * 2.0 ** -24 + torch.finfo(dtype).eps / 2 * 1.01
     assert torch.equal(got[~live.expand_as(got)], dead[~live.expand_as(got)])
+
+
+@pytest.mark.parametrize("T", [264, 301, 384, 385, 392, 441, 512, 513])
+@pytest.mark.parametrize("heads", [30, 60, 110])  # (half row blocks; a round of row blocks that is not full; one more, of which little is left)
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 64), (torch.float16, 128)])
+def test_long_rows_equal_the_two_calls(dev, dtype, d, heads, T):
+    """Rows of more than 256 slots, to the longest that the sampled product takes along and beyond."""
+    test_equals_the_two_calls(dev, "rows", lambda L: A.causal_windowed_pattern(520, T - 1), heads, dtype, d)
+
+
+def test_long_rows_of_two_segments_equal_the_two_calls(dev):
+    test_equals_the_two_calls(dev, "rows", lambda L: A.strided_patterns(700, 256, 16), 50, torch.bfloat16, 64)

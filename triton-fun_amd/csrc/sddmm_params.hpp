@@ -32,13 +32,20 @@ struct SddmmParams {
     int probs_vec;  // T % 8 == 0, and out and probs start on 32-byte boundaries
 };
 
-// Whether softmax_own_rows pays: rows of up to 256 slots (of 300 1.05 of the time of a launch for each, of 512 1.03 to 1.13), and 16-bit
-// scores that the caches hold: the three operators, causal masks of 33 to 256 slots, d = 64 and 128: up to 64 MB of scores 0.68 to 0.97
-// of the time, from 90 to 134 MB 0.97 to 1.12.  (Scores and probabilities are stored through the caches then: 4096 rows of 200 slots, 16 heads,
-// d = 128 60 -> 41 us, of which 53 around them.)  Not where a stride between a block's rows leaves most of them empty (224 heads of
-// 128 rows, 21 slots with step 3: 18.7 -> 20.6).
+// Whether softmax_own_rows pays.  Float32: rows of up to 256 slots (of 300 1.05 of the time of a launch for each, of 512 1.03 to 1.13).  16-bit
+// types: rows of up to 512 slots and scores that the caches hold: causal masks of 33 to 256 slots, d = 64 and 128, the three operators 0.68 to 0.99 of
+// the time up to 80 MB of scores, the two alone 0.82 to 1.25 from 100 to 170 MB.  (Scores and probabilities are stored through the caches
+// then: 4096 rows of 200 slots, 16 heads, d = 128 60 -> 41 us, of which 53 around them.)  Of rows of more than 256 slots the workgroups that have
+// the chip to themselves at a launch's end take longer than the other kernel's, so that their round (512 row blocks) has to be filled, to nine
+// sixteenths, or to three quarters where rows end inside pieces: 283 slots, 520 / 640 / 720 / 1024 row blocks 1.06 / 1.03 / 1.03 / 0.98 of the time
+// at d = 64, 1.04 / 1.02 / 1.00 / 0.96 at 128; 384 slots, 480 / 528 / 576 / 768 blocks 0.91 / 1.00 / 0.97 / 0.91 and 0.87 / 0.97 / 0.95 / 0.92.
+// Not where a stride between a block's rows leaves most of them empty (224 heads of 128 rows, 21 slots with step 3: 18.7 -> 20.6).
 inline bool own_rows_fit(const SddmmParams& p) {
-    return p.probs && !p.row_lse && p.T <= 256 && (p.row_stride == 1 || p.L >= 128 * p.row_stride) && (p.out_dtype == SPLAT_F32 || (int64_t)p.B * p.H * p.L * p.T <= (int64_t)1 << 25);
+    if (!p.probs || p.row_lse || (p.row_stride > 1 && p.L < 128 * p.row_stride)) return false;
+    if (p.out_dtype == SPLAT_F32) return p.T <= 256;
+    if (p.T > 512 || (int64_t)p.B * p.H * p.L * p.T * 2 > kCachedBytes) return false;
+    const int64_t blocks = (int64_t)p.B * p.H * count_row_blocks(p.L, 128, p.row_stride), room = (blocks + 511) / 512 * 512;
+    return p.T <= 256 || blocks <= 512 || blocks * 16 >= room * (p.probs_vec ? 9 : 12);
 }
 
 // The softmax of the 16 rows r0 + rs * k of head bh that this wavefront, and nobody else, has stored: they come from the cache, and a launch
@@ -69,10 +76,14 @@ __device__ __forceinline__ void softmax_own_rows(const SddmmParams& p, int bh, i
     using std::integral_constant;
     if (p.probs_vec) {
         if (T_ <= 128) go(integral_constant<int, 1>{}, integral_constant<int, 16>{}, std::true_type{});
+        else if (sizeof(T) == 2 && T_ > 384) go(integral_constant<int, 4>{}, integral_constant<int, 16>{}, std::true_type{});
+        else if (sizeof(T) == 2 && T_ > 256) go(integral_constant<int, 3>{}, integral_constant<int, 16>{}, std::true_type{});
         else if (sizeof(T) == 2) go(integral_constant<int, 2>{}, integral_constant<int, 16>{}, std::true_type{});
         else go(integral_constant<int, 1>{}, integral_constant<int, 32>{}, std::true_type{});
     } else {
         if (T_ <= 128) go(integral_constant<int, 1>{}, integral_constant<int, 16>{}, std::false_type{});
+        else if (sizeof(T) == 2 && T_ > 384) go(integral_constant<int, 4>{}, integral_constant<int, 16>{}, std::false_type{});
+        else if (sizeof(T) == 2 && T_ > 256) go(integral_constant<int, 3>{}, integral_constant<int, 16>{}, std::false_type{});
         else if (sizeof(T) == 2) go(integral_constant<int, 4>{}, integral_constant<int, 8>{}, std::false_type{});
         else go(integral_constant<int, 1>{}, integral_constant<int, 32>{}, std::false_type{});
     }
