@@ -107,11 +107,11 @@ def test_large_matrices_equal_their_halves(dev, planned, T, dtype):
         assert torch.equal(whole[i], torch.cat([x[i] for x in parts]))
 
 
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("rows", [300, 140000])  # (small, and beyond what the caches hold)
-@pytest.mark.parametrize("T", [130, 192, 264, 376, 384, 385, 392, 440, 448, 449, 456, 505, 512])
-def test_softmax_16_bit_rows_over_lanes(dev, T, rows, dtype):
-    """Edges of the splits of a 16-bit row over lanes, two segments with dead slots between and after them, in place, against float64."""
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows", [300, 140000, 450000])  # (small, and beyond what the caches hold)
+@pytest.mark.parametrize("T", [9, 31, 32, 33, 48, 49, 63, 64, 65, 104, 112, 113, 127, 128, 130, 192, 264, 376, 384, 385, 392, 440, 448, 449, 456, 505, 512])
+def test_softmax_rows_over_lanes(dev, T, rows, dtype):
+    """Edges of the splits of a row over lanes, two segments with dead slots between and after them, in place, against float64."""
     g = torch.Generator(device=dev).manual_seed(T)
     L, off = 50, T * 2 // 3 - 1
     cnt = [torch.randint(0, n + 1, (L,), generator=g, device=dev).float() for n in (off, T - off)]

@@ -1,6 +1,7 @@
 // Kernel arguments of the SDDMM kernels (sddmm.hip: every shape; sddmm_lines.hip, sddmm_rows16.hip: 16-bit types, operators_f32.hip: float32,
 // up to 128 inner values).
 #pragma once
+#include <algorithm>
 #include <type_traits>
 
 #include "acsr_plan.hpp"
@@ -62,7 +63,7 @@ __device__ __forceinline__ void softmax_own_rows(const SddmmParams& p, int bh, i
     const int lane = threadIdx.x & 63, T_ = p.T;
     const int64_t first = (int64_t)bh * p.L;
     auto go = [&](auto nch, auto lpr, auto aligned) {
-        constexpr int NCH = decltype(nch)::value, LPR = decltype(lpr)::value, RPW = 64 / LPR, RIF = NCH == 1 ? 4 : 2;
+        constexpr int NCH = decltype(nch)::value, LPR = decltype(lpr)::value, RPW = 64 / LPR, RIF = std::min(16 / RPW, NCH == 1 ? 4 : 2);
         for (int k0 = 0; k0 < 16; k0 += RPW * RIF) {
             if (r0 + rs * k0 >= p.L) break;
             softmax_rows<T, T, NCH, LPR, RIF, decltype(aligned)::value, false>((const T*)p.out, (T*)p.probs, segs, T_, [&](int i, int64_t& row, int& in_head) {
@@ -73,20 +74,21 @@ __device__ __forceinline__ void softmax_own_rows(const SddmmParams& p, int bh, i
             });
         }
     };
-    using std::integral_constant;
-    if (p.probs_vec) {
-        if (T_ <= 128) go(integral_constant<int, 1>{}, integral_constant<int, 16>{}, std::true_type{});
-        else if (sizeof(T) == 2 && T_ > 384) go(integral_constant<int, 4>{}, integral_constant<int, 16>{}, std::true_type{});
-        else if (sizeof(T) == 2 && T_ > 256) go(integral_constant<int, 3>{}, integral_constant<int, 16>{}, std::true_type{});
-        else if (sizeof(T) == 2) go(integral_constant<int, 2>{}, integral_constant<int, 16>{}, std::true_type{});
-        else go(integral_constant<int, 1>{}, integral_constant<int, 32>{}, std::true_type{});
-    } else {
-        if (T_ <= 128) go(integral_constant<int, 1>{}, integral_constant<int, 16>{}, std::false_type{});
-        else if (sizeof(T) == 2 && T_ > 384) go(integral_constant<int, 4>{}, integral_constant<int, 16>{}, std::false_type{});
-        else if (sizeof(T) == 2 && T_ > 256) go(integral_constant<int, 3>{}, integral_constant<int, 16>{}, std::false_type{});
-        else if (sizeof(T) == 2) go(integral_constant<int, 4>{}, integral_constant<int, 8>{}, std::false_type{});
-        else go(integral_constant<int, 1>{}, integral_constant<int, 32>{}, std::false_type{});
-    }
+    auto split = [&](auto aligned) {
+        constexpr bool ALIGNED = decltype(aligned)::value, F32 = sizeof(T) == 4;
+        auto over = [&](auto nch, auto lpr) { go(nch, lpr, aligned); };
+        using std::integral_constant;
+        if (T_ <= 32) over(integral_constant<int, 1>{}, integral_constant<int, 4>{});
+        else if (T_ <= (F32 ? 48 : 64)) over(integral_constant<int, 1>{}, integral_constant<int, 8>{});
+        else if (F32 && T_ <= 128) over(integral_constant<int, 1>{}, integral_constant<int, 16>{});
+        else if (F32) over(integral_constant<int, 1>{}, integral_constant<int, 32>{});
+        else if (T_ <= 128) over(integral_constant<int, 2>{}, integral_constant<int, 8>{});
+        else if (T_ <= 256) over(integral_constant<int, ALIGNED ? 2 : 4>{}, integral_constant<int, ALIGNED ? 16 : 8>{});
+        else if (T_ <= 384) over(integral_constant<int, 3>{}, integral_constant<int, 16>{});
+        else over(integral_constant<int, 4>{}, integral_constant<int, 16>{});
+    };
+    if (p.probs_vec) split(std::true_type{});
+    else split(std::false_type{});
 }
 
 // Launches the line-wise kernel when the problem has its shape (see sddmm_lines.hip); returns 1 when it did, 2 when it took the

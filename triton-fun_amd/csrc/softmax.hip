@@ -71,8 +71,29 @@ static int launch_softmax(const void* x, void* y, const SoftmaxSegs& segs, int64
             // 66.3 -> 8.9 / 16.4 / 49.5, 384 in two segments 16.1 / 28.5 / 85.3 -> 10.3 / 21.3 / 61.3, 448 14.1 / 23.2 / 70.5 -> 11.9 / 22.7 / 67.3.  Around
             // the caches 32 lanes are as fast up to 256 slots (256: 40.9 both) or faster (200: 35.7 against 40.5), and so are 64 where they
             // have a chunk each (512 slots, 524288 rows: 165.6 against 168.7).
+            // Short rows: four lanes up to 32 slots, eight up to 64 (float32: 48) or, 16-bit types and two chunks each, 128; against 16, bfloat16, 480000 /
+            // 1600000 rows, us: 21 slots 34.5 / 108 -> 11.1 / 29.2, 40 33.7 / 123 -> 17.8 / 52.9, 64 35.1 / 128 -> 20.3 / 65.9, 100 36.0 / 130 -> 29.6 / 112 (32000
+            // rows, 21, 40 and 100 slots 10.8 -> 4.6, 10.5 -> 6.6, 11.8 -> 10.0); float32, 21 slots 32.3 / 101 -> 13.8 / 39.7, 40 30.7 / 111 -> 23.5 / 99.5, 64 slots
+            // of 32000 rows 11.5 -> 12.3.  Matrices that the caches do not hold: 104 slots around them 43.4 / 138 -> 46.6 / 151 with two chunks,
+            // 37.9 / 119 with two row groups of 16 lanes; 127 slots in two segments 229 -> 244.
+            if (T <= 32) {
+                softmax_rows_vec<Tin, Tout, 1, 4, 1, ALIGNED, AROUND><<<groups(16), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
+                return;
+            }
+            if (T <= (sizeof(Tin) == 4 ? 48 : 64)) {
+                constexpr int RIF = sizeof(Tin) == 4 ? 1 : 2;
+                softmax_rows_vec<Tin, Tout, 1, 8, RIF, ALIGNED, AROUND><<<groups(8 * RIF), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
+                return;
+            }
+            if constexpr (sizeof(Tin) == 2 && !AROUND) {
+                if (T <= (n_rows * T * (int64_t)sizeof(Tin) <= kCachedBytes ? 128 : 112)) {
+                    softmax_rows_vec<Tin, Tout, 2, 8, 1, ALIGNED, AROUND><<<groups(8), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
+                    return;
+                }
+            }
             if (T <= 128) {
-                softmax_rows_vec<Tin, Tout, 1, 16, 1, ALIGNED, AROUND><<<groups(4), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
+                constexpr int RIF = sizeof(Tin) == 2 && AROUND ? 2 : 1;
+                softmax_rows_vec<Tin, Tout, 1, 16, RIF, ALIGNED, AROUND><<<groups(4 * RIF), 256, 0, st>>>(xi, yo, segs, n_rows, L, T, by_l);
                 return;
             }
             if constexpr (sizeof(Tin) == 2) {
