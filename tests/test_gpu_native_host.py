@@ -120,3 +120,18 @@ def test_native_operators_equal_the_launchers(dev, layout, L, masks, dtype, d):
     assert None not in attn._operator_masks[:2] and torch.equal(attn([q, kT, v]), want[0])
     with pytest.raises(hip.SplatError):
         attn([q.double(), kT.double(), v.double()])
+
+
+def test_the_operators_follow_the_module_s_segments(dev):
+    """Another mask put in a module's place after a forward is what the next forward computes, in both layouts of K."""
+    L, d, dtype = 300, 64, torch.bfloat16
+    first, other = A.causal_windowed_pattern(L, 20), A.dilated_pattern(L, 21, 2)  # (rows of 21 slots, both)
+    attn, want = (RegularAttention(1, L, 2, d, m, 16, 16, dev, dtype, scale=d ** -0.5, fused=False) for m in (first, other))
+    q, _, kT, v = _operands(dev, 1, 2, L, d, dtype, "rows")
+    for keys in (kT, kT.contiguous()):
+        attn([q, keys, v])
+        attn([q, keys, v])
+    attn.segments = want.segments
+    for keys in (kT, kT.contiguous()):
+        for _ in range(2):
+            assert torch.equal(attn([q, keys, v]), want([q, keys, v]))

@@ -112,7 +112,8 @@ def attention_launcher(q: torch.Tensor, kT: torch.Tensor, v: torch.Tensor, outpu
 
 
 class RegularAttention(nn.Module):
-    _operator_masks = None  # as the native call of all three operators takes them: kept by the first forward through the launchers
+    _operator_masks = None  # as the native call of all three operators takes them: kept by the first forward through the launchers ...
+    _operator_segments = None  # ... and the segments that they stand for
 
     def __init__(self, batch: int, seq_length: int, num_heads: int, head_dim: int, mask,
                  BLOCK_SIZE_Y: int, BLOCK_SIZE_X: int, GPU_ID: Any, out_dtype: torch.dtype,
@@ -205,7 +206,7 @@ class RegularAttention(nn.Module):
             return attention_launcher(q, k, v, self.rspmm_output, self.segments, self.scale, self._plan, live_percent=self._live_percent)
 
         masks = self._operator_masks
-        if masks is not None and _hip.host().operators(*masks, q, k, v, self._rsddmm_output, self._rsoftmax_output, self.rspmm_output,
+        if masks is not None and self._operator_segments is self.segments and _hip.host().operators(*masks, q, k, v, self._rsddmm_output, self._rsoftmax_output, self.rspmm_output,
                                                        self.scale):
             return self.rspmm_output
         multi = self.segments  # (also for one segment: the object keeps what every call would otherwise rebuild and recheck)
@@ -234,7 +235,8 @@ class RegularAttention(nn.Module):
             return
         segs, rows = self.segments, k.stride(2) == 1
         mask = sddmm_mask(segs, q, k, self._rsddmm_output)
-        of_rows, of_keys, *_ = self._operator_masks or (None, None)
+        of_rows, of_keys, *_ = (self._operator_masks if self._operator_segments is segs else None) or (None, None)
+        self._operator_segments = segs
         self._operator_masks = (mask if rows else of_rows, of_keys if rows else mask, segs.native(self._shape[2], self._device, False),
                                 spmm_mask(segs, self._rsoftmax_output, self.rspmm_output))
 
