@@ -78,3 +78,20 @@ def test_the_line_at_d64(dev, H, kt, same):
     part = few([q[:, :100], k[:, :100].transpose(2, 3), v[:, :100]])
     assert torch.equal(whole[:, :100], part) == same
     assert float((whole[:, :100].float() - part.float()).norm() / part.float().norm()) <= 4e-3
+
+
+@pytest.mark.parametrize("kt", [False, True])
+@pytest.mark.parametrize("d", [64, 128])
+def test_float32_scores_have_the_bits_of_larger_launches(dev, d, kt):
+    """The statistic of a row of one key is its score (the scale makes the exponents' factor 1: no other rounding), which the backward
+    takes again: the same bits whichever kernel computed it."""
+    L, H, ln2 = 300, 70, 0.6931471824645996
+    g = torch.Generator(device=dev).manual_seed(d)
+    q, k, v = (torch.randn(1, H, L, d, generator=g, device=dev) for _ in range(3))
+
+    def statistic(heads):
+        attn = RegularAttention(1, L, heads, d, A.causal_windowed_pattern(L, 0), 16, 16, dev, torch.float32, scale=ln2)
+        kT = k[:, :heads].transpose(2, 3)
+        return attn.forward_with_stats([q[:, :heads], kT.contiguous() if kt else kT, v[:, :heads]])[1].clone()
+    want = statistic(H)  # (210 row blocks; then 9 and 36: workgroups of 16 and of 32 rows)
+    assert torch.equal(statistic(3), want[:, :3]) and torch.equal(statistic(12), want[:, :12])

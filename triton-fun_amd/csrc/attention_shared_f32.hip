@@ -3,9 +3,11 @@
 // Bound: latency, as in attention_shared.hip, whose division of the work this is: four wavefronts hold the same rows, 16 or 32, tile k
 // of 32 positions goes to wavefront k % 4, and the parts meet in LDS at the end.  Products and their precision are those of
 // attention_f32.hip (operands split into three bfloat16 parts, 16x16x32).  A wavefront is the only one to read its tiles, so that
-// they go from memory into registers and are split there: no LDS, no barrier.  For that the columns of an operand take the places that
-// make whole pieces of 16 bytes of a lane's loads:
-//   * scores: lane (n, g) holds columns 16i + 4g .. + 3 of key n for every i, of Q's row n the same;
+// they go from memory into registers and are split there: no LDS, no barrier.
+//   * scores: lane (n, g) holds columns 32 ks + 8g .. + 7 of key n and of Q's row n, which are the places they have in the other float32
+//     kernels: a score has the same bits here, in a larger launch, and where the backward takes it again.  (With other columns in those
+//     places, P of the backward was off from the statistic by both roundings: dQ of small training steps, windows 8 to 90, 3.7e-7 instead of 3.1e-7
+//     against float64.)
 //   * output: row r of tile dt of V^T is column (D / 16) r + dt, so that one position's columns of all tiles lie side by side in
 //     memory, and a lane ends with D / 4 consecutive columns of its row.
 // 32 rows (RG = 2) share every split of a tile, at twice the products of a wavefront: they come in where workgroups of 16 would run in
@@ -147,15 +149,15 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_fwd_shared_f32_kern
         for (int u = 0; u < 2; ++u) {
             const uint32_t key = key_at(w, 16 * u + n);
             if constexpr (KT) {
-                const float* from = kb + (int64_t)(4 * g) * p.k_sd + key;
+                const float* from = kb + (int64_t)(8 * g) * p.k_sd + key;
 #pragma unroll
                 for (int i = 0; i < 2 * KS; ++i)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) kr[u][i][e] = from[(16 * i + e) * p.k_sd];
+                    for (int e = 0; e < 4; ++e) kr[u][i][e] = from[(16 * (i & ~1) + 4 * (i & 1) + e) * p.k_sd];
             } else {
-                const uint32_t off = __umul24(key, k_row) + 16 * g;
+                const uint32_t off = __umul24(key, k_row) + 32 * g;
 #pragma unroll
-                for (int i = 0; i < 2 * KS; ++i) kr[u][i] = load4(kb, off + 64 * i);
+                for (int i = 0; i < 2 * KS; ++i) kr[u][i] = load4(kb, off + 64 * (i & ~1) + 16 * (i & 1));
             }
         }
     };
@@ -170,9 +172,9 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_fwd_shared_f32_kern
     f32x4 q_raw[RG][2 * KS];
 #pragma unroll
     for (int rg = 0; rg < RG; ++rg) {
-        const float* qr = qb + (int64_t)min(r0 + rs * (16 * rg + n), L - 1) * p.q_sl + 4 * g;
+        const float* qr = qb + (int64_t)min(r0 + rs * (16 * rg + n), L - 1) * p.q_sl + 8 * g;
 #pragma unroll
-        for (int i = 0; i < 2 * KS; ++i) q_raw[rg][i] = *reinterpret_cast<const f32x4*>(qr + 16 * i);
+        for (int i = 0; i < 2 * KS; ++i) q_raw[rg][i] = *reinterpret_cast<const f32x4*>(qr + 16 * (i & ~1) + 4 * (i & 1));
     }
     if (cur.seg < p.n_seg) request_k(cur), request_v(cur);
 
