@@ -6,7 +6,7 @@
 // they go from memory into registers and are split there: no LDS, no barrier.
 //   * scores: lane (n, g) holds columns 32 ks + 8g .. + 7 of key n and of Q's row n, which are the places they have in the other float32
 //     kernels: a score has the same bits here, in a larger launch, and where the backward takes it again.  (With other columns in those
-//     places, P of the backward was off from the statistic by both roundings: dQ of small training steps, windows 8 to 90, 3.7e-7 instead of 3.1e-7
+//     places, P of the backward was off from the statistic by both roundings: dQ of small training steps, windows 8 to 90, 3.6e-7 instead of 3.2e-7
 //     against float64.)
 //   * output: row r of tile dt of V^T is column (D / 16) r + dt, so that one position's columns of all tiles lie side by side in
 //     memory, and a lane ends with D / 4 consecutive columns of its row.
