@@ -4,6 +4,8 @@ without a HIP device (there is no host fallback)."""
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -220,3 +222,22 @@ def test_metadata_with_native_handles_copies_and_saves(monkeypatch):
         assert torch.equal(other, t) and other.splat_row_stride == 1
         own = native(other)
         assert type(own).__name__ == "PyCapsule" and (own is not handle or other.data_ptr() == t.data_ptr())
+
+
+def test_native_entry_points_raise_what_is_thrown_in_them():
+    """No C++ exception leaves an entry point of the native host path: without a device, finding the current one throws, and a call of
+    any of them has to be a Python error, not the end of the process (in a process of its own for that)."""
+    code = """
+import os, sys
+sys.path.insert(0, sys.argv[1])
+import _splat_hip as hip
+for name, n in (("forward", 6), ("attend", 5), ("sddmm", 6), ("softmax", 3), ("spmm", 4), ("operators", 11)):
+    try:
+        getattr(hip.host(), name)(*[None] * n)
+        print(name, "returned")
+    except Exception as e:
+        print(name, "raised")
+"""
+    r = subprocess.run([sys.executable, "-c", code, os.path.join(ROOT, "triton-fun_amd", "SPLAT")], capture_output=True, text=True,
+                       timeout=300, env={**os.environ, "HIP_VISIBLE_DEVICES": "-1"})
+    assert r.returncode == 0 and r.stdout.count("raised") == 6, r.stdout + r.stderr

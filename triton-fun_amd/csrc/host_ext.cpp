@@ -548,25 +548,29 @@ PyObject* py_spmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // operand is not an ordinary one, and the launchers take the whole forward (what has been launched is computed again).
 PyObject* py_operators(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 11) return PyErr_Format(PyExc_TypeError, "operators takes 11 arguments");
-    const int dev = c10::hip::current_device();
-    const at::Tensor *q = tensor4(a[4], dev), *kT = tensor4(a[5], dev), *out = tensor4(a[9], dev);
-    // (the masks were chosen for the output's type and head dimension)
-    if (!q || !kT || !out || q->scalar_type() != out->scalar_type() || q->size(3) != out->size(3)) Py_RETURN_FALSE;
-    PyObject* const mask = a[kT->stride(2) == 1 ? 0 : 1];
-    if (mask == Py_None) Py_RETURN_FALSE;
-    PyObject* const first[] = {mask, a[4], a[5], a[7], a[10], Py_None};
-    PyObject* const second[] = {a[2], a[7], a[8]};
-    PyObject* const third[] = {a[3], a[8], a[6], a[9]};
-    const at::Tensor *scores = tensor4(a[7], dev), *probs = tensor4(a[8], dev);
-    const bool both = scores && probs && scores->scalar_type() == probs->scalar_type() && scores->sizes() == probs->sizes() &&
-                      probs->is_contiguous() && scores->data_ptr() != probs->data_ptr();
-    PyObject* did = sddmm_of(first, both ? probs : nullptr);
-    if (did != Py_True) return did;
-    if (!both) {
-        did = py_softmax(nullptr, second, 3);
-        if (did != Py_True) return did;
+    try {
+        const int dev = c10::hip::current_device();
+        const at::Tensor *q = tensor4(a[4], dev), *kT = tensor4(a[5], dev), *out = tensor4(a[9], dev);
+        // (the masks were chosen for the output's type and head dimension)
+        if (!q || !kT || !out || q->scalar_type() != out->scalar_type() || q->size(3) != out->size(3)) Py_RETURN_FALSE;
+        PyObject* const mask = a[kT->stride(2) == 1 ? 0 : 1];
+        if (mask == Py_None) Py_RETURN_FALSE;
+        PyObject* const first[] = {mask, a[4], a[5], a[7], a[10], Py_None};
+        PyObject* const second[] = {a[2], a[7], a[8]};
+        PyObject* const third[] = {a[3], a[8], a[6], a[9]};
+        const at::Tensor *scores = tensor4(a[7], dev), *probs = tensor4(a[8], dev);
+        const bool both = scores && probs && scores->scalar_type() == probs->scalar_type() && scores->sizes() == probs->sizes() &&
+                          probs->is_contiguous() && scores->data_ptr() != probs->data_ptr();
+        THPObjectPtr did(sddmm_of(first, both ? probs : nullptr));
+        if (did.get() != Py_True) return did.release();
+        if (!both) {
+            did = py_softmax(nullptr, second, 3);
+            if (did.get() != Py_True) return did.release();
+        }
+        return py_spmm(nullptr, third, 4);
+    } catch (...) {
+        return raise_current();
     }
-    return py_spmm(nullptr, third, 4);
 }
 
 // ---- the ACSR and the plan of a mask ---------------------------------------------------------------------------------------------
