@@ -135,3 +135,22 @@ def test_the_operators_follow_the_module_s_segments(dev):
     for keys in (kT, kT.contiguous()):
         for _ in range(2):
             assert torch.equal(attn([q, keys, v]), want([q, keys, v]))
+
+
+@pytest.mark.parametrize("kind", ["along the keys", "of another type", "on the host"])
+def test_the_operators_refuse_before_they_launch(dev, kind):
+    """A V that is not an ordinary one leaves the native call with nothing done: the launchers run each operator, once."""
+    L, d, dtype = 300, 80, torch.float16
+    attn = RegularAttention(1, L, 2, d, A.causal_windowed_pattern(L, 20), 16, 16, dev, dtype, scale=d ** -0.5, fused=False)
+    q, _, kT, v = _operands(dev, 1, 2, L, d, dtype, "rows")
+    want = attn([q, kT, v]).clone()
+    odd = {"along the keys": v.transpose(2, 3).contiguous().transpose(2, 3), "of another type": v.float(), "on the host": v.cpu()}[kind]
+    attn._rsddmm_output.fill_(7.0)
+    attn._rsoftmax_output.fill_(7.0)
+    assert not hip.host().operators(*attn._operator_masks, q, kT, odd, attn._rsddmm_output, attn._rsoftmax_output, attn.rspmm_output, attn.scale)
+    assert torch.all(attn._rsddmm_output == 7.0) and torch.all(attn._rsoftmax_output == 7.0)
+    if kind == "along the keys":
+        assert torch.equal(attn([q, kT, odd]), want)
+    else:
+        with pytest.raises(hip.SplatError):
+            attn([q, kT, odd])

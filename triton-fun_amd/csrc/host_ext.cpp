@@ -417,76 +417,124 @@ PyObject* py_attend(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // ---- the three operators ------------------------------------------------------------------------------------------------------
-// sddmm(mask, x, y, output, scale, lse | None) -> bool; a plan in the mask is handed on.  `probs`: the softmax of the output goes there.
-PyObject* sddmm_of(PyObject* const* a, const at::Tensor* probs) {
+// Each operator in two halves: whether its operands are ordinary ones, and the launch.  An operand that is none is found before anything runs.
+struct Sampled {  // out = scale * x y on the mask's slots; `turn`: y is turned to rows first
+    const at::Tensor *x, *y, *out;
+    float* lse = nullptr;
+    bool turn = false;
+    bool find(const Mask& m, PyObject* x_, PyObject* y_, PyObject* out_, PyObject* lse_, int dev);
+    int launch(const Mask& m, double scale, const at::Tensor* probs, const char** what) const;  // `probs`: the softmax of the output goes there
+};
+
+bool Sampled::find(const Mask& m, PyObject* x_, PyObject* y_, PyObject* out_, PyObject* lse_, int dev) {
+    x = tensor4(x_, dev), y = tensor4(y_, dev), out = tensor4(out_, dev);
+    if (!x || !y || !out || m.device != dev) return false;
+    const int code = dtype_code(x->scalar_type()), out_code = dtype_code(out->scalar_type());
+    const int64_t B = x->size(0), H = x->size(1), L = x->size(2), d = x->size(3), keys = y->size(3), T = out->size(3);
+    if (code < 0 || out_code < 0 || y->scalar_type() != x->scalar_type() || L != m.rows || x->stride(3) != 1 || B * H * L * d * T == 0 ||
+        !is_shape(*y, B, H, d, keys) || !is_shape(*out, B, H, L, T) || !out->is_contiguous() || (y->stride(2) != 1 && y->stride(3) != 1))
+        return false;
+    if (lse_ != Py_None) {
+        if (!THPVariable_Check(lse_)) return false;
+        const at::Tensor& t = THPVariable_Unpack(lse_);
+        if (!t.is_cuda() || t.get_device() != dev || t.scalar_type() != at::kFloat || !t.is_contiguous() || t.dim() != 3 ||
+            t.size(0) != B || t.size(1) != H || t.size(2) != L)
+            return false;
+        lse = t.data_ptr<float>();
+    }
+    // K^T with the keys contiguous is read in place by the general kernel and by the two named below.  Up to d = 64 a pass that turns it and a kernel on
+    // the copy take less: the kernel of thin wavefronts where the launch has its shape (the three operators, bfloat16: 64 heads of
+    // 4096 rows, 33 slots, d = 32: 114 -> 92 us; 512 slots, d = 64: 300 -> 263), in launches of fewer than 256 row blocks of more
+    // than 256 slots the general kernel, which is faster on rows of K as well (4 heads of 4001 rows, 301 slots, d = 64: 49 -> 43).  Beyond d = 64 the copy costs as much as it gives (64 heads of 2048 rows, 255 slots: d = 80 122 -> 125,
+    // d = 96 126 -> 129), and so does its launch below 64 row blocks (one head of 200 rows: 21 -> 25).
+    const bool turned = code != SPLAT_F32 && out_code == code && d % 8 == 0 && d <= 64 && B * H * ((L + 127) / 128) >= 64;
+    // Up to 128 inner values float32 (operators_f32.hip, but for the launches that its launcher leaves to the general kernel) and 16-bit launches of few row blocks (sddmm_rows16.hip, whose conditions are these;
+    // a stride of n between a block's rows adds at most n - 1 blocks) turn K on its way into LDS, gathered or not: the three
+    // operators, float32, 16 heads of 1605 rows, 176 slots with step 2, d = 128, 76.9 -> 72.3 us without the copy.
+    const bool few = d % 8 == 0 && B * H * 2 * ((L + 127) / 128 + std::max(m.max_step - 1, 0)) <= 512 &&
+                     (reinterpret_cast<uintptr_t>(x->data_ptr()) & 15) == 0 && x->stride(0) % 8 == 0 && x->stride(1) % 8 == 0 &&
+                     x->stride(2) % 8 == 0;
+    const bool general_f32 = d <= 64 && T > (d > 32 && d <= 56 ? 450 : 600) && B * H * ((L + 63) / 64 + std::max(m.max_step - 1, 0)) >= 1024;
+    const bool in_place = out_code == code && d <= 128 && (code == SPLAT_F32 ? !general_f32 : few);
+    turn = (m.max_step >= 2 || turned) && !in_place && y->stride(3) == 1 && y->stride(2) != 1;
+    return !turn || y->stride(2) >= keys;
+}
+
+int Sampled::launch(const Mask& m, double scale, const at::Tensor* probs, const char** what) const {
+    int rc = 0;
+    at::Tensor k = *y;
+    if (turn) {
+        k = transposed_keys(k, &rc).transpose(2, 3);
+        *what = "splat_transpose_keys";
+        if (rc) return rc;
+    }
+    *what = "splat_sddmm";
+    void* st = stream_of(*x);
+    const void* plan = m.plan.defined() ? m.plan_ptr() : nullptr;
+    const int64_t plan_bytes = plan ? m.plan_bytes() : 0;
+#define SPLAT_K x->data_ptr(), x->stride(0), x->stride(1), x->stride(2), k.data_ptr(), k.stride(0), k.stride(1), k.stride(2), k.stride(3), out->data_ptr()
+#define SPLAT_SIZES                                                                                                                   \
+    m.segs, m.n_seg, x->size(0), x->size(1), x->size(2), k.size(3), x->size(3), out->size(3), (float)scale, dtype_code(x->scalar_type()), \
+        dtype_code(out->scalar_type())
+    if (probs) return api.sddmm_softmax(SPLAT_K, probs->data_ptr(), SPLAT_SIZES, plan, plan_bytes, st);
+    if (plan) return api.sddmm_planned(SPLAT_K, SPLAT_SIZES, lse, plan, plan_bytes, st);
+    if (lse) return api.sddmm_probs(SPLAT_K, SPLAT_SIZES, lse, st);
+    return api.sddmm(SPLAT_K, SPLAT_SIZES, st);
+#undef SPLAT_SIZES
+#undef SPLAT_K
+}
+
+// y = softmax of x
+struct Softmax {
+    const at::Tensor *x, *out;
+    bool find(const Mask& m, PyObject* x_, PyObject* out_, int dev) {
+        x = tensor4(x_, dev), out = tensor4(out_, dev);
+        return x && out && m.device == dev && x->sizes() == out->sizes() && x->is_contiguous() && out->is_contiguous() &&
+               x->size(2) == m.rows && x->numel() != 0 && dtype_code(x->scalar_type()) >= 0 && dtype_code(out->scalar_type()) >= 0;
+    }
+    int launch(const Mask& m) const {
+        return api.softmax(x->data_ptr(), out->data_ptr(), m.segs, m.n_seg, x->size(0) * x->size(1), x->size(2), x->size(3),
+                           dtype_code(x->scalar_type()), dtype_code(out->scalar_type()), stream_of(*x));
+    }
+};
+
+// out = x y, x on the mask's slots
+struct Spmm {
+    const at::Tensor *x, *y, *out;
+    bool find(const Mask& m, PyObject* x_, PyObject* y_, PyObject* out_, int dev) {
+        x = tensor4(x_, dev), y = tensor4(y_, dev), out = tensor4(out_, dev);
+        if (!x || !y || !out || m.device != dev) return false;
+        const int64_t B = x->size(0), H = x->size(1), L = x->size(2);
+        return dtype_code(x->scalar_type()) >= 0 && dtype_code(out->scalar_type()) >= 0 && y->scalar_type() == x->scalar_type() &&
+               L == m.rows && x->numel() != 0 && y->numel() != 0 && y->size(0) == B && y->size(1) == H &&
+               is_shape(*out, B, H, L, y->size(3)) && x->is_contiguous() && out->is_contiguous() && y->stride(3) == 1;
+    }
+    int launch(const Mask& m) const {
+#define SPLAT_ARGS                                                                                                                     \
+    x->data_ptr(), y->data_ptr(), y->stride(0), y->stride(1), y->stride(2), out->data_ptr(), m.segs, m.n_seg, x->size(0), x->size(1), \
+        x->size(2), y->size(2), y->size(3), x->size(3), dtype_code(x->scalar_type()), dtype_code(out->scalar_type())
+        if (m.plan.defined()) return api.spmm_planned(SPLAT_ARGS, m.plan_ptr(), m.plan_bytes(), stream_of(*x));
+        return api.spmm(SPLAT_ARGS, stream_of(*x));
+#undef SPLAT_ARGS
+    }
+};
+
+// sddmm(mask, x, y, output, scale, lse | None) -> bool; a plan in the mask is handed on
+PyObject* py_sddmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 6) return PyErr_Format(PyExc_TypeError, "sddmm takes 6 arguments");
     Mask* m = mask_of(a[0]);
     if (!m) return nullptr;
     try {
-        const int dev = c10::hip::current_device();
-        const at::Tensor *x = tensor4(a[1], dev), *y0 = tensor4(a[2], dev), *out = tensor4(a[3], dev);
-        if (!x || !y0 || !out || m->device != dev) Py_RETURN_FALSE;
-        at::Tensor y = *y0;
-        const int code = dtype_code(x->scalar_type()), out_code = dtype_code(out->scalar_type());
-        const int64_t B = x->size(0), H = x->size(1), L = x->size(2), d = x->size(3), keys = y.size(3), T = out->size(3);
-        if (code < 0 || out_code < 0 || y.scalar_type() != x->scalar_type() || L != m->rows || x->stride(3) != 1 || B * H * L * d * T == 0 ||
-            !is_shape(y, B, H, d, keys) || !is_shape(*out, B, H, L, T) || !out->is_contiguous() || (y.stride(2) != 1 && y.stride(3) != 1))
-            Py_RETURN_FALSE;
-        float* lse = nullptr;
-        if (a[5] != Py_None) {
-            if (!THPVariable_Check(a[5])) Py_RETURN_FALSE;
-            const at::Tensor& t = THPVariable_Unpack(a[5]);
-            if (!t.is_cuda() || t.get_device() != dev || t.scalar_type() != at::kFloat || !t.is_contiguous() || t.dim() != 3 ||
-                t.size(0) != B || t.size(1) != H || t.size(2) != L)
-                Py_RETURN_FALSE;
-            lse = t.data_ptr<float>();
-        }
+        Sampled s;
+        if (!s.find(*m, a[1], a[2], a[3], a[5], c10::hip::current_device())) Py_RETURN_FALSE;
         const double scale = PyFloat_AsDouble(a[4]);
         if (scale == -1.0 && PyErr_Occurred()) return nullptr;
-        int rc = 0;
-        // K^T with the keys contiguous is read in place by the general kernel and by the two named below.  Up to d = 64 a pass that turns it and a kernel on
-        // the copy take less: the kernel of thin wavefronts where the launch has its shape (the three operators, bfloat16: 64 heads of
-        // 4096 rows, 33 slots, d = 32: 114 -> 92 us; 512 slots, d = 64: 300 -> 263), in launches of fewer than 256 row blocks of more
-        // than 256 slots the general kernel, which is faster on rows of K as well (4 heads of 4001 rows, 301 slots, d = 64: 49 -> 43).  Beyond d = 64 the copy costs as much as it gives (64 heads of 2048 rows, 255 slots: d = 80 122 -> 125,
-        // d = 96 126 -> 129), and so does its launch below 64 row blocks (one head of 200 rows: 21 -> 25).
-        const bool turned = code != SPLAT_F32 && out_code == code && d % 8 == 0 && d <= 64 && B * H * ((L + 127) / 128) >= 64;
-        // Up to 128 inner values float32 (operators_f32.hip, but for the launches that its launcher leaves to the general kernel) and 16-bit launches of few row blocks (sddmm_rows16.hip, whose conditions are these;
-        // a stride of n between a block's rows adds at most n - 1 blocks) turn K on its way into LDS, gathered or not: the three
-        // operators, float32, 16 heads of 1605 rows, 176 slots with step 2, d = 128, 76.9 -> 72.3 us without the copy.
-        const bool few = d % 8 == 0 && B * H * 2 * ((L + 127) / 128 + std::max(m->max_step - 1, 0)) <= 512 &&
-                         (reinterpret_cast<uintptr_t>(x->data_ptr()) & 15) == 0 && x->stride(0) % 8 == 0 && x->stride(1) % 8 == 0 &&
-                         x->stride(2) % 8 == 0;
-        const bool general_f32 = d <= 64 && T > (d > 32 && d <= 56 ? 450 : 600) && B * H * ((L + 63) / 64 + std::max(m->max_step - 1, 0)) >= 1024;
-        const bool in_place = out_code == code && d <= 128 && (code == SPLAT_F32 ? !general_f32 : few);
-        if ((m->max_step >= 2 || turned) && !in_place && y.stride(3) == 1 && y.stride(2) != 1) {
-            if (y.stride(2) < keys) Py_RETURN_FALSE;
-            y = transposed_keys(y, &rc).transpose(2, 3);
-            if (rc) return raise_rc("splat_transpose_keys", rc);
-        }
-        void* st = stream_of(*x);
-#define SPLAT_ARGS                                                                                                                     \
-    x->data_ptr(), x->stride(0), x->stride(1), x->stride(2), y.data_ptr(), y.stride(0), y.stride(1), y.stride(2), y.stride(3),        \
-        out->data_ptr(), m->segs, m->n_seg, B, H, L, keys, d, T, (float)scale, code, out_code
-        if (probs)
-            rc = api.sddmm_softmax(x->data_ptr(), x->stride(0), x->stride(1), x->stride(2), y.data_ptr(), y.stride(0), y.stride(1), y.stride(2),
-                                   y.stride(3), out->data_ptr(), probs->data_ptr(), m->segs, m->n_seg, B, H, L, keys, d, T, (float)scale, code,
-                                   out_code, m->plan.defined() ? m->plan_ptr() : nullptr, m->plan.defined() ? m->plan_bytes() : 0, st);
-        else if (m->plan.defined())
-            rc = api.sddmm_planned(SPLAT_ARGS, lse, m->plan_ptr(), m->plan_bytes(), st);
-        else if (lse)
-            rc = api.sddmm_probs(SPLAT_ARGS, lse, st);
-        else
-            rc = api.sddmm(SPLAT_ARGS, st);
-#undef SPLAT_ARGS
-        if (rc) return raise_rc("splat_sddmm", rc);
+        const char* what;
+        if (const int rc = s.launch(*m, scale, nullptr, &what)) return raise_rc(what, rc);
         Py_RETURN_TRUE;
     } catch (...) {
         return raise_current();
     }
-}
-
-PyObject* py_sddmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
-    if (n != 6) return PyErr_Format(PyExc_TypeError, "sddmm takes 6 arguments");
-    return sddmm_of(a, nullptr);
 }
 
 // softmax(mask, x, output) -> bool
@@ -495,16 +543,9 @@ PyObject* py_softmax(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Mask* m = mask_of(a[0]);
     if (!m) return nullptr;
     try {
-        const int dev = c10::hip::current_device();
-        const at::Tensor *x = tensor4(a[1], dev), *out = tensor4(a[2], dev);
-        if (!x || !out || m->device != dev || x->sizes() != out->sizes() || !x->is_contiguous() || !out->is_contiguous() ||
-            x->size(2) != m->rows || x->numel() == 0)
-            Py_RETURN_FALSE;
-        const int code = dtype_code(x->scalar_type()), out_code = dtype_code(out->scalar_type());
-        if (code < 0 || out_code < 0) Py_RETURN_FALSE;
-        const int rc = api.softmax(x->data_ptr(), out->data_ptr(), m->segs, m->n_seg, x->size(0) * x->size(1), x->size(2), x->size(3),
-                                   code, out_code, stream_of(*x));
-        if (rc) return raise_rc("splat_softmax", rc);
+        Softmax s;
+        if (!s.find(*m, a[1], a[2], c10::hip::current_device())) Py_RETURN_FALSE;
+        if (const int rc = s.launch(*m)) return raise_rc("splat_softmax", rc);
         Py_RETURN_TRUE;
     } catch (...) {
         return raise_current();
@@ -517,24 +558,9 @@ PyObject* py_spmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Mask* m = mask_of(a[0]);
     if (!m) return nullptr;
     try {
-        const int dev = c10::hip::current_device();
-        const at::Tensor *x = tensor4(a[1], dev), *y = tensor4(a[2], dev), *out = tensor4(a[3], dev);
-        if (!x || !y || !out || m->device != dev) Py_RETURN_FALSE;
-        const int code = dtype_code(x->scalar_type()), out_code = dtype_code(out->scalar_type());
-        const int64_t B = x->size(0), H = x->size(1), L = x->size(2), T = x->size(3), keys = y->size(2), w = y->size(3);
-        if (code < 0 || out_code < 0 || y->scalar_type() != x->scalar_type() || L != m->rows || x->numel() == 0 || y->numel() == 0 ||
-            y->size(0) != B || y->size(1) != H || !is_shape(*out, B, H, L, w) || !x->is_contiguous() || !out->is_contiguous() ||
-            y->stride(3) != 1)
-            Py_RETURN_FALSE;
-        void* st = stream_of(*x);
-        int rc;
-        if (m->plan.defined())
-            rc = api.spmm_planned(x->data_ptr(), y->data_ptr(), y->stride(0), y->stride(1), y->stride(2), out->data_ptr(), m->segs, m->n_seg,
-                                  B, H, L, keys, w, T, code, out_code, m->plan_ptr(), m->plan_bytes(), st);
-        else
-            rc = api.spmm(x->data_ptr(), y->data_ptr(), y->stride(0), y->stride(1), y->stride(2), out->data_ptr(), m->segs, m->n_seg, B, H,
-                          L, keys, w, T, code, out_code, st);
-        if (rc) return raise_rc("splat_spmm", rc);
+        Spmm s;
+        if (!s.find(*m, a[1], a[2], a[3], c10::hip::current_device())) Py_RETURN_FALSE;
+        if (const int rc = s.launch(*m)) return raise_rc("splat_spmm", rc);
         Py_RETURN_TRUE;
     } catch (...) {
         return raise_current();
@@ -544,8 +570,7 @@ PyObject* py_spmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // operators(mask | None, mask | None, mask, mask, q, kT, v, scores, probabilities, out, scale) -> bool: the three operators of one forward.  The
 // masks are those of the sampled product, for rows of K and for K along the keys, of the softmax and of the last product.  What the
 // interpreter does between three calls costs more than the launches (22 -> 12.6 us on the host), and than the kernels of a few row
-// blocks (40 heads of 256 rows, 62 slots, bfloat16, d = 64: 20.1 -> 13.6 us a forward).  False: some
-// operand is not an ordinary one, and the launchers take the whole forward (what has been launched is computed again).
+// blocks (40 heads of 256 rows, 62 slots, bfloat16, d = 64: 20.1 -> 13.6 us a forward).
 PyObject* py_operators(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 11) return PyErr_Format(PyExc_TypeError, "operators takes 11 arguments");
     try {
@@ -553,21 +578,26 @@ PyObject* py_operators(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const at::Tensor *q = tensor4(a[4], dev), *kT = tensor4(a[5], dev), *out = tensor4(a[9], dev);
         // (the masks were chosen for the output's type and head dimension)
         if (!q || !kT || !out || q->scalar_type() != out->scalar_type() || q->size(3) != out->size(3)) Py_RETURN_FALSE;
-        PyObject* const mask = a[kT->stride(2) == 1 ? 0 : 1];
-        if (mask == Py_None) Py_RETURN_FALSE;
-        PyObject* const first[] = {mask, a[4], a[5], a[7], a[10], Py_None};
-        PyObject* const second[] = {a[2], a[7], a[8]};
-        PyObject* const third[] = {a[3], a[8], a[6], a[9]};
-        const at::Tensor *scores = tensor4(a[7], dev), *probs = tensor4(a[8], dev);
-        const bool both = scores && probs && scores->scalar_type() == probs->scalar_type() && scores->sizes() == probs->sizes() &&
-                          probs->is_contiguous() && scores->data_ptr() != probs->data_ptr();
-        THPObjectPtr did(sddmm_of(first, both ? probs : nullptr));
-        if (did.get() != Py_True) return did.release();
-        if (!both) {
-            did = py_softmax(nullptr, second, 3);
-            if (did.get() != Py_True) return did.release();
+        PyObject* const masks[] = {a[kT->stride(2) == 1 ? 0 : 1], a[2], a[3]};
+        Mask* m[3];
+        for (int i = 0; i < 3; ++i) {
+            if (masks[i] == Py_None) Py_RETURN_FALSE;
+            if (!(m[i] = mask_of(masks[i]))) return nullptr;
         }
-        return py_spmm(nullptr, third, 4);
+        Sampled first;
+        Softmax second;
+        Spmm third;
+        if (!first.find(*m[0], a[4], a[5], a[7], Py_None, dev) || !second.find(*m[1], a[7], a[8], dev) || !third.find(*m[2], a[8], a[6], a[9], dev))
+            Py_RETURN_FALSE;
+        const double scale = PyFloat_AsDouble(a[10]);
+        if (scale == -1.0 && PyErr_Occurred()) return nullptr;
+        const bool both = second.x->scalar_type() == second.out->scalar_type() && second.x->data_ptr() != second.out->data_ptr();
+        const char* what;
+        if (const int rc = first.launch(*m[0], scale, both ? second.out : nullptr, &what)) return raise_rc(what, rc);
+        if (!both)
+            if (const int rc = second.launch(*m[1])) return raise_rc("splat_softmax", rc);
+        if (const int rc = third.launch(*m[2])) return raise_rc("splat_spmm", rc);
+        Py_RETURN_TRUE;
     } catch (...) {
         return raise_current();
     }
