@@ -5,6 +5,7 @@ import torch
 
 import acsr_helpers as A
 import _splat_hip as hip
+import r_attention
 from r_attention import RegularAttention, _AttentionFunction, attention_launcher, attention_with_grad
 
 pytestmark = pytest.mark.gpu
@@ -100,12 +101,15 @@ def test_running_out_of_memory_is_the_error_a_program_catches(dev):
                                      (301, lambda L: A.dilated_pattern(L, 20, 3))])
 @pytest.mark.parametrize("dtype,d", [(torch.float32, 64), (torch.bfloat16, 64), (torch.float16, 80)])
 def test_native_operators_equal_the_launchers(dev, layout, L, masks, dtype, d):
-    """The first forward goes through the three launchers, the next ones through one native call; a layout that comes later goes
-    through the launchers first again, and other types are theirs to refuse."""
+    """A forward through the three launchers, and through the one native call, which the module's forwards make; the masks of a layout that
+    comes later are chosen by its first forward, and other types are the launchers' to refuse."""
     B, H = 2, 3
     attn = RegularAttention(B, L, H, d, masks(L), 16, 16, dev, dtype, scale=d ** -0.5, fused=False)
     q, _, kT, v = _operands(dev, B, H, L, d, dtype, layout)
+    attn._choose_operators = lambda *_: None
     want = [t.clone() for t in (attn([q, kT, v]), attn.rsddmm_output, attn.rsoftmax_output)]
+    del attn._choose_operators
+    assert attn._operator_masks is None and torch.equal(attn([q, kT, v]), want[0])
     kept = attn._operator_masks
     taken = hip.host().operators(*kept, q, kT, v, attn._rsddmm_output, attn._rsoftmax_output, attn.rspmm_output.zero_(), attn.scale)
     assert taken and torch.equal(attn.rspmm_output, want[0])
@@ -154,3 +158,30 @@ def test_the_operators_refuse_before_they_launch(dev, kind):
     else:
         with pytest.raises(hip.SplatError):
             attn([q, kT, odd])
+
+
+@pytest.mark.parametrize("layout", ["rows", "keys"])
+@pytest.mark.parametrize("dtype,d", [(torch.float16, 80), (torch.float32, 64)])
+def test_the_first_forward_makes_the_one_call(dev, layout, dtype, d, monkeypatch):
+    """A module's first forward makes the native call of the three operators, not the launchers'; the same under stream capture where
+    a forward has been before it."""
+    L, B, H = 700, 2, 9
+    attn = RegularAttention(B, L, H, d, A.causal_windowed_pattern(L, 60), 16, 16, dev, dtype, scale=d ** -0.5, fused=False)
+    q, _, kT, v = _operands(dev, B, H, L, d, dtype, layout)
+    attn._choose_operators = lambda *_: None
+    want = attn([q, kT, v]).clone()
+    del attn._choose_operators
+
+    def launcher(*args, **kwargs):
+        raise AssertionError("a launcher")
+    for name in ("rsddmm_launcher", "rsoftmax_launcher", "rspmm_launcher"):
+        monkeypatch.setattr(r_attention, name, launcher)
+    assert torch.equal(attn([q, kT, v]), want)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        attn([q, kT, v])
+    for _ in range(3):
+        attn.rspmm_output.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(attn.rspmm_output, want)

@@ -112,7 +112,7 @@ def attention_launcher(q: torch.Tensor, kT: torch.Tensor, v: torch.Tensor, outpu
 
 
 class RegularAttention(nn.Module):
-    _operator_masks = None  # as the native call of all three operators takes them: kept by the first forward through the launchers ...
+    _operator_masks = None  # as the native call of all three operators takes them, chosen by the first forward ...
     _operator_segments = None  # ... and the segments that they stand for
 
     def __init__(self, batch: int, seq_length: int, num_heads: int, head_dim: int, mask,
@@ -205,8 +205,12 @@ class RegularAttention(nn.Module):
             self._ensure_plan()
             return attention_launcher(q, k, v, self.rspmm_output, self.segments, self.scale, self._plan, live_percent=self._live_percent)
 
-        masks = self._operator_masks
-        if masks is not None and self._operator_segments is self.segments and _hip.host().operators(*masks, q, k, v, self._rsddmm_output, self._rsoftmax_output, self.rspmm_output,
+        masks = self._operator_masks if self._operator_segments is self.segments else None
+        if masks is not None and _hip.host().operators(*masks, q, k, v, self._rsddmm_output, self._rsoftmax_output, self.rspmm_output,
+                                                       self.scale):
+            return self.rspmm_output
+        masks = self._choose_operators(masks, q, k)
+        if masks is not None and _hip.host().operators(*masks, q, k, v, self._rsddmm_output, self._rsoftmax_output, self.rspmm_output,
                                                        self.scale):
             return self.rspmm_output
         multi = self.segments  # (also for one segment: the object keeps what every call would otherwise rebuild and recheck)
@@ -226,19 +230,25 @@ class RegularAttention(nn.Module):
                        self.sTod_linear_transformations, self.sTod_translations,
                        self.span_loop_start, self.span_loop_end, self.acsr_trailing_dim,
                        self.nnzs, self.rspmm_grid_dim, self.BLOCK_SIZE_Y, self.BLOCK_SIZE_X, segments=multi)
-        self._keep_operators(q, k)
         return self.rspmm_output
 
-    def _keep_operators(self, q, k):
-        """The masks that the launchers of a forward like this one have used, for the native call of all three."""
-        if q.dtype != self._out_dtype or q.shape[3] != self._shape[3] or torch.cuda.is_current_stream_capturing():
-            return
+    def _choose_operators(self, kept, q, k):
+        """The masks that the launchers of this forward would use, for the native call of all three; None where they are what ``kept`` has,
+        which that call has refused, and where q or k is not what this module takes.  What is chosen under stream capture, where no plan can be
+        built, is not kept."""
+        if not (q.dim() == k.dim() == 4 and q.shape == self._shape and q.device == self._device and q.dtype == self._out_dtype):
+            return None
         segs, rows = self.segments, k.stride(2) == 1
+        of_rows, of_keys, *_ = kept or (None, None)
+        if (of_rows if rows else of_keys) is not None:
+            return None
+        self._prepare_unfused()
         mask = sddmm_mask(segs, q, k, self._rsddmm_output)
-        of_rows, of_keys, *_ = (self._operator_masks if self._operator_segments is segs else None) or (None, None)
-        self._operator_segments = segs
-        self._operator_masks = (mask if rows else of_rows, of_keys if rows else mask, segs.native(self._shape[2], self._device, False),
-                                spmm_mask(segs, self._rsoftmax_output, self.rspmm_output))
+        masks = (mask if rows else of_rows, of_keys if rows else mask, segs.native(self._shape[2], self._device, False),
+                 spmm_mask(segs, self._rsoftmax_output, self.rspmm_output))
+        if not torch.cuda.is_current_stream_capturing():
+            self._operator_masks, self._operator_segments = masks, segs
+        return masks
 
     def _ensure_plan(self):
         """The fused kernel's plan of this mask, and the mask as the native host path takes it."""
