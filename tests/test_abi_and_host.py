@@ -104,10 +104,10 @@ def test_the_fused_backward_checks_its_arguments_on_the_host():
     L, d = 256, 64
     need = lib.splat_attention_plan_bytes(seg, 1, L)
 
-    def bwd(q=16, lse=16, d=d, dtype=2, scale=1.0, plan_bytes=need, q_sl=d, seg_t=seg):
+    def bwd(q=16, lse=16, d=d, dtype=2, scale=1.0, plan_bytes=need, q_sl=d, seg_t=seg, B=1):
         t = [16, 0, 0, d]  # pointer, batch / head / row strides
         return lib.splat_attention_bwd(q, 0, 0, q_sl, *t, *t, *t, *t, lse, 16, 16, 16, 16, seg, 1, 16, plan_bytes,
-                                       seg_t, 1, 16, need, 1, 1, L, d, scale, dtype, None)
+                                       seg_t, 1, 16, need, B, 1, L, d, scale, dtype, None)
     assert bwd(q=None) == -1 and bwd(lse=None) == -1 and bwd(seg_t=None) == -1
     assert bwd(d=96) == -5 and b"64 or 128" in lib.splat_last_error()
     assert bwd(dtype=0) == -5 and b"16-bit" in lib.splat_last_error()
@@ -115,6 +115,10 @@ def test_the_fused_backward_checks_its_arguments_on_the_host():
     assert bwd(q=24) == -4 and bwd(q_sl=d + 4) == -4
     assert bwd(q_sl=32) == -2
     assert bwd(plan_bytes=need - 16) == -2 and b"plan" in lib.splat_last_error()
+    assert bwd(B=1 << 29) == -2 and b"too many" in lib.splat_last_error()  # two row blocks a head, two workgroups each: 2^31
+    t = [16, 0, 0, d]
+    assert lib.splat_attention_bwd_keys(*t, *t, *t, *t, 16, 16, 16, 16, 16, seg, 1, 16, need, 1 << 29, 1, L, 256, d, 1.0, 2, None, None, 0,
+                                        None) == -2 and b"too many" in lib.splat_last_error()
 
 
 def test_the_key_transpose_checks_its_arguments_on_the_host():

@@ -476,6 +476,9 @@ static int check_bwd_common(const char* who, bool f32, int B, int H, int L, int 
     return 0;
 }
 
+// The launches count their workgroups in an int: at most two a row block.
+static bool too_many_blocks(int B, int H, int64_t row_blocks) { return 2 * (int64_t)B * H * row_blocks > 0x7ffffff0; }
+
 static BwdParams bwd_base(const float* lse, const float* delta, int B, int H, int L, float scale) {
     BwdParams base;
     base.lse = lse; base.delta = delta;
@@ -526,8 +529,8 @@ static int bwd_impl(const char* who, bool f32, const void* q, int64_t q_sb, int6
     if (plan_bytes < splat_attention_plan_bytes(segs, n_seg, L) || plan_t_bytes < splat_attention_plan_bytes(segs_t, n_seg_t, L))
         return fail(SPLAT_E_SHAPE, "%s: a plan is smaller than its mask needs (%lld and %lld bytes given)", who, (long long)plan_bytes,
                     (long long)plan_t_bytes);
-    if ((int64_t)B * H * std::max(count_row_blocks(L, kPlanBM, common_row_stride(segs, n_seg)),
-                                  count_row_blocks(L, kPlanBM, common_row_stride(segs_t, n_seg_t))) > 0x7ffffff0)
+    if (too_many_blocks(B, H, std::max(count_row_blocks(L, kPlanBM, common_row_stride(segs, n_seg)),
+                                       count_row_blocks(L, kPlanBM, common_row_stride(segs_t, n_seg_t)))))
         return fail(SPLAT_E_SHAPE, "%s: too many row blocks", who);
     hipStream_t st = (hipStream_t)stream;
 
@@ -581,7 +584,7 @@ static int bwd_keys_impl(const char* who, bool f32, const void* q, int64_t q_sb,
     if (plan_t_bytes < splat_attention_plan_bytes(segs_t, n_seg_t, n_rows))
         return fail(SPLAT_E_SHAPE, "%s: the plan is smaller than %d rows of this mask need (%lld bytes given)", who, n_rows,
                     (long long)plan_t_bytes);
-    if ((int64_t)B * H * count_row_blocks(n_rows, kPlanBM, common_row_stride(segs_t, n_seg_t)) > 0x7ffffff0)
+    if (too_many_blocks(B, H, count_row_blocks(n_rows, kPlanBM, common_row_stride(segs_t, n_seg_t))))
         return fail(SPLAT_E_SHAPE, "%s: too many row blocks", who);
     const BwdParams base = bwd_base(lse, delta, B, H, L, scale);
     const BwdParams pk = bwd_keys_params(base, rq, rk, rv, rg, dk_rows, dv_rows, segs_t, n_seg_t, plan_t, n_rows, key_of_row, d);
