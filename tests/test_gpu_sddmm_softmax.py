@@ -82,11 +82,11 @@ def test_softmax_of_few_and_many_rows(dev, T, rows, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("T", [304, 320])
+@pytest.mark.parametrize("T", [104, 128, 200, 256, 304, 320, 456, 512])
 @pytest.mark.parametrize("planned", [True, False])
 def test_large_matrices_equal_their_halves(dev, planned, T, dtype):
     """Scores and probabilities that the caches do not hold are stored around them; the halves of the same heads are not: the same bits."""
-    L, d, heads = 2048, 32, 68
+    L, d, heads = 2048, 32, 2 * -(-(84 << 20) // (4 * 2048 * T))
     segs = A.create_acsr_segments([A.causal_windowed_pattern(L, T - 1)], 16, dev)
     assert segs.T == T
     g = torch.Generator(device=dev).manual_seed(T)
@@ -146,3 +146,32 @@ def test_long_rows_equal_the_two_calls(dev, dtype, d, heads, T):
 
 def test_long_rows_of_two_segments_equal_the_two_calls(dev):
     test_equals_the_two_calls(dev, "rows", lambda L: A.strided_patterns(700, 256, 16), 50, torch.bfloat16, 64)
+
+
+@pytest.mark.parametrize("din,dout", [(torch.bfloat16, torch.float32), (torch.float16, torch.float16), (torch.float32, torch.float32)])
+@pytest.mark.parametrize("T", [7, 20, 32, 33, 40, 48, 49, 64, 65, 72, 104, 112, 113, 128, 129, 136, 200, 255, 256, 257, 301, 384, 385, 448, 456, 504, 511, 512, 1000])
+def test_a_row_s_bits_do_not_depend_on_the_call(dev, T, din, dout):
+    """A few rows, the same rows among as many as the caches do not hold, and in a buffer that starts off every boundary: one sum."""
+    g = torch.Generator(device=dev).manual_seed(T)
+    L, off = 64, T // 3
+    cnt = [torch.randint(0, n + 1, (L,), generator=g, device=dev).float() for n in (off, T - off)]
+    cnt[0][::2], cnt[1][::2] = off, T - off
+    seg = (hip.AcsrSeg * 2)()
+    for k in range(2):
+        seg[k].sTod_lin = seg[k].sTod_trans = seg[k].nnz = cnt[k].data_ptr()
+        seg[k].slot_offset = (0, off)[k]
+    x = (torch.randn(1, L, T, generator=g, device=dev) * 3).to(din)
+
+    def softmax(x, shift):
+        n = x.shape[0]
+        src = torch.empty(x.numel() + shift, dtype=din, device=dev)[shift:].view(x.shape)
+        src.copy_(x)
+        dst = torch.full((x.numel() + shift,), 7.0, dtype=dout, device=dev)[shift:].view(x.shape)
+        hip.check(hip.lib().splat_softmax(src.data_ptr(), dst.data_ptr(), seg, 2, n, L, T, hip.dtype_code(din), hip.dtype_code(dout),
+                                          hip.stream_ptr(dev)), "splat_softmax")
+        return dst
+    want = softmax(x, 0)
+    assert torch.equal(softmax(x, 1), want)
+    many = (90 << 20) // (L * T * x.element_size())
+    for n in (20000 // L, many):
+        assert torch.equal(softmax(x.expand(n, L, T), 0), want.expand(n, L, T))

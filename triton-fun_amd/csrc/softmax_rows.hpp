@@ -74,6 +74,9 @@ constexpr float kNegBig = -1.0e30f;
 // ALIGNED: T is a multiple of 8 and every chunk of 8 slots starts on a 16-byte boundary.  Otherwise a row's chunks start where it does, and the
 // last one ends where the row ends: it repeats slots of the chunk before it, which count once and may be stored twice, by lanes of one
 // wavefront and with one value.  No row's lanes touch another's slots.
+// A row of up to 512 slots is added in one order, whatever the split: each chunk from its first slot on, then the sums of the chunks 32 apart,
+// 16 apart and so on, of which a lane has some and its neighbours the others.  So its bits depend neither on how many rows a call has, on
+// where they start, nor on which kernel takes them.  (Longer rows, which have one split each, add a lane's chunks one after the other.)
 // AROUND: loads and stores go around the cache.  row_at(i, row, in_head): the row that this lane's part of group i takes, among all rows and
 // among its head's, and whether it is to be stored; a surplus lane shadows some other row.
 template <typename Tin, typename Tout, int NCH, int LPR, int RIF, bool ALIGNED, bool AROUND, typename RowAt>
@@ -143,7 +146,10 @@ __device__ __forceinline__ void softmax_rows(const Tin* __restrict__ x, Tout* __
         }
         // the common case, decided for the whole wavefront: no dead slot anywhere in its rows, so no per-slot selects
         const bool all_whole = !__any(!whole);
-        float sum = 0.f;
+        constexpr int NP = LPR == 64 ? 1 : NCH;
+        float part[NP];
+#pragma unroll
+        for (int c = 0; c < NP; ++c) part[c] = 0.f;
         if (all_whole) {
 #pragma unroll
             for (int c = 0; c < NCH; ++c) {
@@ -161,7 +167,7 @@ __device__ __forceinline__ void softmax_rows(const Tin* __restrict__ x, Tout* __
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     v[c][e] = fast_exp2(fmaf(v[c][e], kLog2e, -mb));
-                    sum += ALIGNED || e >= again[c] ? v[c][e] : 0.f;
+                    part[c % NP] += ALIGNED || e >= again[c] ? v[c][e] : 0.f;
                 }
         } else {
 #pragma unroll
@@ -185,11 +191,17 @@ __device__ __forceinline__ void softmax_rows(const Tin* __restrict__ x, Tout* __
                         // dead slots hold -1e30 and underflow to exactly 0 against any real maximum; a row without live
                         // slots stores nothing, so what its lanes compute does not matter
                         v[c][e] = fast_exp2(fmaf(v[c][e], kLog2e, -mb));
-                        sum += ALIGNED || e >= again[c] ? v[c][e] : 0.f;
+                        part[c % NP] += ALIGNED || e >= again[c] ? v[c][e] : 0.f;
                     }
                 }
             }
         }
+        float sum = part[0];
+        if constexpr (NP > 2) sum += part[2];
+        if constexpr (NP > 3)
+            sum += part[1] + part[3];
+        else if constexpr (NP > 1)
+            sum += part[1];
         sum = wave_sum<LPR>(sum);
         const float inv = sum > 0.f ? 1.0f / sum : 0.f;
 #pragma unroll
