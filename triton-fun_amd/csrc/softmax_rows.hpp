@@ -68,6 +68,17 @@ constexpr int64_t kCachedBytes = (int64_t)80 << 20;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kNegBig = -1.0e30f;
 
+// s plus the values of a chunk from slot `again` on (CUT; else all of them), one after the other.  FRESH: s is nothing yet.
+template <bool CUT, bool FRESH>
+__device__ __forceinline__ float add_chunk(float s, const float (&v)[8], int again) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float x = !CUT || e >= again ? v[e] : 0.f;
+        s = FRESH && e == 0 ? x : s + x;
+    }
+    return s;
+}
+
 // LPR lanes share one row (64 / LPR rows per wavefront): rows shorter than 512 slots still fill every lane.  A wavefront
 // takes RIF such row groups at once and requests all of their chunks before it looks at any (bytes in flight per
 // wavefront are what a streaming kernel lives on).
@@ -92,6 +103,7 @@ __device__ __forceinline__ void softmax_rows(const Tin* __restrict__ x, Tout* __
     // 128 slots 16.4 -> 15.2; 64 heads of 8192 rows, 512 slots: 175 -> 172).
     int at[NCH], again[NCH];  // first slot of the lane's chunk; how many of its slots the chunk before it has
     bool mine[NCH];
+    const int cut = !ALIGNED && T % 8 != 0 ? (nchunk - 1) / LPR : -1;  // which chunk of a lane can be a row's last one
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
         const int ch = lane + LPR * c;
@@ -150,6 +162,17 @@ __device__ __forceinline__ void softmax_rows(const Tin* __restrict__ x, Tout* __
         float part[NP];
 #pragma unroll
         for (int c = 0; c < NP; ++c) part[c] = 0.f;
+        auto add = [&](int c) {  // (with a chunk's sum of its own, nothing is added to zero)
+            float& s = part[c % NP];
+            if (!ALIGNED && c == cut) {
+#if defined(__HIP_DEVICE_COMPILE__)
+                asm("" : "+v"(again[c]));  // (compared here: answers found beforehand take two scalar registers a slot until then)
+#endif
+                s = NP > 1 || c == 0 ? add_chunk<true, true>(s, v[c], again[c]) : add_chunk<true, false>(s, v[c], again[c]);
+            } else {
+                s = NP > 1 || c == 0 ? add_chunk<false, true>(s, v[c], again[c]) : add_chunk<false, false>(s, v[c], again[c]);
+            }
+        };
         if (all_whole) {
 #pragma unroll
             for (int c = 0; c < NCH; ++c) {
@@ -165,10 +188,9 @@ __device__ __forceinline__ void softmax_rows(const Tin* __restrict__ x, Tout* __
 #pragma unroll
             for (int c = 0; c < NCH; ++c)
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    v[c][e] = fast_exp2(fmaf(v[c][e], kLog2e, -mb));
-                    part[c % NP] += ALIGNED || e >= again[c] ? v[c][e] : 0.f;
-                }
+                for (int e = 0; e < 8; ++e) v[c][e] = fast_exp2(fmaf(v[c][e], kLog2e, -mb));
+#pragma unroll
+            for (int c = 0; c < NCH; ++c) add(c);
         } else {
 #pragma unroll
             for (int c = 0; c < NCH; ++c) {
@@ -191,8 +213,8 @@ __device__ __forceinline__ void softmax_rows(const Tin* __restrict__ x, Tout* __
                         // dead slots hold -1e30 and underflow to exactly 0 against any real maximum; a row without live
                         // slots stores nothing, so what its lanes compute does not matter
                         v[c][e] = fast_exp2(fmaf(v[c][e], kLog2e, -mb));
-                        part[c % NP] += ALIGNED || e >= again[c] ? v[c][e] : 0.f;
                     }
+                    add(c);
                 }
             }
         }
