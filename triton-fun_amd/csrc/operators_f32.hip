@@ -42,8 +42,8 @@ __device__ __forceinline__ f32x4 row_piece(const float* row, int c, int n, bool 
 
 // out[bh, r, s] = scale * q[r] . k[column of slot s], or the probability exp(that - lse[r]).  S^T = K Q^T: a lane owns one row and
 // holds four consecutive positions of every 16.  KQ: 16-value steps of the contraction.  KT: K stored along the keys; it is turned on its
-// way into LDS, lanes = keys, wherever its rows start.
-template <int KQ, bool KT>
+// way into LDS, lanes = keys, wherever its rows start.  SM: the softmax of its rows that a wavefront takes at the end (sddmm_params.hpp).
+template <int KQ, bool KT, int SM>
 __global__ __launch_bounds__(256, 4) void sddmm_f32_kernel(const SddmmParams p) {
     constexpr int ROWB = KQ <= 2 ? 128 : KQ <= 4 ? 256 : 512;  // bytes of an LDS row: a power of two, for the swizzle
     constexpr int STAGE = kTile * ROWB, CPR = 4 * KQ, NP = kTile * CPR / 256;
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(256, 4) void sddmm_f32_kernel(const SddmmParams p) 
             stage ^= STAGE;
         }
     }
-    if (p.probs) softmax_own_rows<float>(p, bh, r0 + rs * 16 * wave, rs);
+    if constexpr (SM != kNoSoftmax) softmax_own_rows<float, SM, false>(p, bh, r0 + rs * 16 * wave, rs);
 }
 
 // out[bh, r, :] = sum over the live slots s of p[bh, r, s] * v[column of s, :].  O^T = V^T P^T: a lane reads its row's entries at 8 consecutive
@@ -331,10 +331,13 @@ int launch_sddmm_f32(const SddmmParams& p0, bool kt, hipStream_t st) {
     const int grid = ((p.total + 7) / 8) * 8;
     auto go = [&](auto kq) {
         constexpr int KQ = decltype(kq)::value;
-        if (kt)
-            sddmm_f32_kernel<KQ, true><<<grid, 256, 0, st>>>(p);
-        else
-            sddmm_f32_kernel<KQ, false><<<grid, 256, 0, st>>>(p);
+        by_split_of<kSoftmax32, kSoftmax256>(p, [&](auto sm) {
+            constexpr int SM = decltype(sm)::value;
+            if (kt)
+                sddmm_f32_kernel<KQ, true, SM><<<grid, 256, 0, st>>>(p);
+            else
+                sddmm_f32_kernel<KQ, false, SM><<<grid, 256, 0, st>>>(p);
+        });
     };
     if (p.d <= 32) go(std::integral_constant<int, 2>{});
     else if (p.d <= 64) go(std::integral_constant<int, 4>{});

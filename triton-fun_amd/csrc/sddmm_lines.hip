@@ -55,7 +55,8 @@ struct LinesGeom {
     static constexpr int LDS_BYTES = PLANNED ? PLAN_AT : PLAN_AT + (int)sizeof(PlanScratch<BM>) + SPLAT_MAX_SEGMENTS * ((int)sizeof(SegPlan) + 4);
 };
 
-template <typename T, int D, int NST, int KEYS, int HL, int BM_, bool PROBS, bool PLANNED, bool PART>
+// SM: the softmax of its rows that a wavefront takes at the end (sddmm_params.hpp)
+template <typename T, int D, int NST, int KEYS, int HL, int BM_, bool PROBS, bool PLANNED, bool PART, int SM>
 __global__ __launch_bounds__(BM_ * 4, 4) void sddmm_lines_kernel(const SddmmParams p) {
     using G = LinesGeom<D, NST, KEYS, HL, BM_, PLANNED>;
     static_assert(!PLANNED || BM_ == kPlanBM, "the plan table is laid out for 128-row blocks");
@@ -81,7 +82,7 @@ __global__ __launch_bounds__(BM_ * 4, 4) void sddmm_lines_kernel(const SddmmPara
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, g4 = lane >> 4;
 
-    load_args(p.total, p.key_split, p.by_split.m, p.by_split.shift, p.by_blocks.m, p.by_blocks.shift, p.by_h.m, p.by_h.shift, p.n_row_blocks, p.H, p.row_stride, p.L,
+    load_args(p.total, p.by_blocks.m, p.by_blocks.shift, p.by_h.m, p.by_h.shift, p.n_row_blocks, p.H, p.row_stride, p.L,
               p.n_keys, p.d, p.T, p.n_seg, p.plan, p.q, p.q_sb, p.q_sh, p.q_sl, p.k, p.k_sb, p.k_sh, p.k_sd, p.k_sl, p.out);
     const int logical = xcd_remap(blockIdx.x, p.total);
     if (logical >= p.total) return;
@@ -387,29 +388,34 @@ __global__ __launch_bounds__(BM_ * 4, 4) void sddmm_lines_kernel(const SddmmPara
             });
         }
     }
-    if constexpr (PLANNED && !PROBS) {
-        if (p.probs) softmax_own_rows<T>(p, bh, r0 + rs * 16 * wave, rs);
-    }
+    if constexpr (SM != kNoSoftmax) softmax_own_rows<T, SM, !PART>(p, bh, r0 + rs * 16 * wave, rs);
 }
 
-template <typename T, int D, int NST, int KEYS, int HL, int BM, bool PROBS, bool PLANNED, bool PART>
+// SM_LO, SM_HI: the softmax splits that rows of this variant's lengths have
+template <typename T, int D, int NST, int KEYS, int HL, int BM, bool PROBS, bool PLANNED, bool PART, int SM_LO, int SM_HI>
 static int launch_lines_variant(const char* who, SddmmParams p, hipStream_t st) {
     using G = LinesGeom<D, NST, KEYS, HL, BM, PLANNED>;
     static_assert(G::LDS_BYTES * (256 / BM) <= 160 * 1024, "16 wavefronts per compute unit");
     p.n_row_blocks = count_row_blocks(p.L, BM, p.row_stride);
     const int64_t blocks = (int64_t)p.B * p.H * p.n_row_blocks;
     if (blocks > 0x7ffffff0) return 0;
-    p.key_split = 1;
     p.total = (int)blocks;
-    if (!PLANNED || !own_rows_fit(p)) p.probs = nullptr;
+    if (PROBS || !PLANNED || !own_rows_fit(p) || (!PART && (reinterpret_cast<uintptr_t>(p.probs) & 15) != 0)) p.probs = nullptr;
     if (p.probs) p.out_stream = 0;
-    p.by_split = divisor(1), p.by_blocks = divisor(p.n_row_blocks), p.by_h = divisor(p.H);
-    static uint64_t reserved = 0;
-    auto kern = sddmm_lines_kernel<T, D, NST, KEYS, HL, BM, PROBS, PLANNED, PART>;
-    if (int rc = reserve_dynamic_lds(&reserved, reinterpret_cast<const void*>(kern), G::LDS_BYTES, who)) return rc;
-    const int grid = ((p.total + 7) / 8) * 8;
-    kern<<<grid, BM * 4, G::LDS_BYTES, st>>>(p);
-    return p.probs ? 2 : 1;
+    p.by_blocks = divisor(p.n_row_blocks), p.by_h = divisor(p.H);
+    int rc = 0;
+    auto go = [&](auto sm) {
+        static uint64_t reserved = 0;
+        auto kern = sddmm_lines_kernel<T, D, NST, KEYS, HL, BM, PROBS, PLANNED, PART, decltype(sm)::value>;
+        if ((rc = reserve_dynamic_lds(&reserved, reinterpret_cast<const void*>(kern), G::LDS_BYTES, who)) != 0) return;
+        const int grid = ((p.total + 7) / 8) * 8;
+        kern<<<grid, BM * 4, G::LDS_BYTES, st>>>(p);
+    };
+    if constexpr (PROBS || !PLANNED)
+        go(std::integral_constant<int, kNoSoftmax>{});
+    else
+        by_split_of<SM_LO, SM_HI>(p, go);
+    return rc ? rc : p.probs ? 2 : 1;
 }
 
 // Whole 128-byte lines are what the memory system likes best (a blocked mask at d = 128: 0.25 ms against 0.34 ms with
@@ -418,11 +424,11 @@ static int launch_lines_variant(const char* who, SddmmParams p, hipStream_t st) 
 template <typename T, bool PROBS, bool PLANNED, bool PART>
 static int launch_lines_typed(const char* who, const SddmmParams& p, hipStream_t st) {
     if (p.d > 64) {
-        if (p.T >= 256) return launch_lines_variant<T, 128, PLANNED ? 5 : 4, 32, 64, 128, PROBS, PLANNED, PART>(who, p, st);
-        return launch_lines_variant<T, 128, 3, 64, 32, 128, PROBS, PLANNED, PART>(who, p, st);
+        if (p.T >= 256) return launch_lines_variant<T, 128, PLANNED ? 5 : 4, 32, 64, 128, PROBS, PLANNED, PART, kSoftmax256, kSoftmax512>(who, p, st);
+        return launch_lines_variant<T, 128, 3, 64, 32, 128, PROBS, PLANNED, PART, kSoftmax32, kSoftmax256>(who, p, st);
     }
-    if (p.T >= 128) return launch_lines_variant<T, 64, 4, 64, 64, 128, PROBS, PLANNED, PART>(who, p, st);
-    return launch_lines_variant<T, 64, 4, 64, 32, 128, PROBS, PLANNED, PART>(who, p, st);
+    if (p.T >= 128) return launch_lines_variant<T, 64, 4, 64, 64, 128, PROBS, PLANNED, PART, kSoftmax128, kSoftmax512>(who, p, st);
+    return launch_lines_variant<T, 64, 4, 64, 32, 128, PROBS, PLANNED, PART, kSoftmax32, kSoftmax128>(who, p, st);
 }
 
 int launch_sddmm_lines(const char* who, const SddmmParams& p, int in_dtype, hipStream_t st) {

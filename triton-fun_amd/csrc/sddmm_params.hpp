@@ -49,10 +49,32 @@ inline bool own_rows_fit(const SddmmParams& p) {
     return p.T <= 256 || blocks <= 512 || blocks * 16 >= room * (p.probs_vec ? 9 : 12);
 }
 
+// The splits of a row over lanes that softmax_own_rows has, by the longest row of each: a sampled product's kernel is compiled without softmax
+// and with one of them, which its launch chooses.  With all of them in every kernel, chosen there, 128 registers and up to 24 bytes of scratch
+// instead of 68 to 122 and none held back launches with and without a softmax: bfloat16, 128 heads of 4096 rows, d = 64, the sampled product alone at 33
+// slots 37.7 -> 33.0 us, the three operators at 60 slots 157 -> 141; 256 heads of 8192, 40 slots, d = 32 514 -> 459.
+enum { kNoSoftmax, kSoftmax32, kSoftmax64, kSoftmax128, kSoftmax256, kSoftmax384, kSoftmax512 };
+inline int own_rows_split(int T) {
+    return T <= 32 ? kSoftmax32 : T <= 64 ? kSoftmax64 : T <= 128 ? kSoftmax128 : T <= 256 ? kSoftmax256 : T <= 384 ? kSoftmax384 : kSoftmax512;
+}
+
+// f(integral_constant<int, split>) with the split of this launch, of those from LO to HI that its kernel comes with; without softmax where the
+// rows are longer than HI's (p.probs says which).
+template <int LO, int HI, typename F>
+inline void by_split_of(SddmmParams& p, F f) {
+    const int split = std::max<int>(own_rows_split(p.T), LO);
+    if (split > HI) p.probs = nullptr;
+    if (!p.probs) return f(std::integral_constant<int, kNoSoftmax>{});
+    static_for<HI - LO + 1>([&](auto i) {
+        constexpr int S = LO + decltype(i)::value;
+        if (split == S) f(std::integral_constant<int, S>{});
+    });
+}
+
 // The softmax of the 16 rows r0 + rs * k of head bh that this wavefront, and nobody else, has stored: they come from the cache, and a launch
-// of their own is spared.  The splits of a row over lanes are launch_softmax's: the same bits.
+// of their own is spared.  (The bits are launch_softmax's: see softmax_rows.)  ALIGNED: as there; rows of any length go through the other one.
 // float16, 16 heads of 2000 rows, 129 slots, d = 80, the three operators: 26.7 -> 21 us; bfloat16, 208 heads of 128 rows, 64 slots: 16.7 -> 13.6.
-template <typename T>
+template <typename T, int SPLIT, bool ALIGNED>
 __device__ __forceinline__ void softmax_own_rows(const SddmmParams& p, int bh, int r0, int rs) {
     if (r0 >= p.L) return;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // stores and the loads that follow them are not ordered otherwise
@@ -60,35 +82,22 @@ __device__ __forceinline__ void softmax_own_rows(const SddmmParams& p, int bh, i
     segs.n = p.n_seg;
 #pragma unroll
     for (int k = 0; k < SPLAT_MAX_SEGMENTS; ++k) segs.nnz[k] = k < p.n_seg ? p.seg[k].nnz : p.seg[0].nnz, segs.off[k] = p.seg[k].slot_offset;
-    const int lane = threadIdx.x & 63, T_ = p.T;
+    // lanes a row and chunks a lane; float32 a lane for each chunk
+    constexpr bool F32 = sizeof(T) == 4;
+    constexpr int LPR = SPLIT == kSoftmax32 ? 4 : F32 ? (SPLIT == kSoftmax64 ? 8 : SPLIT == kSoftmax128 ? 16 : 32) : SPLIT >= kSoftmax384 || (SPLIT == kSoftmax256 && ALIGNED) ? 16 : 8;
+    constexpr int NCH = F32 || SPLIT <= kSoftmax64 ? 1 : SPLIT == kSoftmax128 || (SPLIT == kSoftmax256 && ALIGNED) ? 2 : SPLIT == kSoftmax384 ? 3 : 4;
+    constexpr int RPW = 64 / LPR, RIF = std::min(16 / RPW, NCH == 1 ? 4 : SPLIT == kSoftmax512 ? 1 : 2);
+    const int lane = threadIdx.x & 63;
     const int64_t first = (int64_t)bh * p.L;
-    auto go = [&](auto nch, auto lpr, auto aligned) {
-        constexpr int NCH = decltype(nch)::value, LPR = decltype(lpr)::value, RPW = 64 / LPR, RIF = std::min(16 / RPW, NCH == 1 ? 4 : 2);
-        for (int k0 = 0; k0 < 16; k0 += RPW * RIF) {
-            if (r0 + rs * k0 >= p.L) break;
-            softmax_rows<T, T, NCH, LPR, RIF, decltype(aligned)::value, false>((const T*)p.out, (T*)p.probs, segs, T_, [&](int i, int64_t& row, int& in_head) {
-                const int at = r0 + rs * (k0 + RPW * i + lane / LPR);
-                in_head = at < p.L ? at : r0;
-                row = first + in_head;
-                return at < p.L;
-            });
-        }
-    };
-    auto split = [&](auto aligned) {
-        constexpr bool ALIGNED = decltype(aligned)::value, F32 = sizeof(T) == 4;
-        auto over = [&](auto nch, auto lpr) { go(nch, lpr, aligned); };
-        using std::integral_constant;
-        if (T_ <= 32) over(integral_constant<int, 1>{}, integral_constant<int, 4>{});
-        else if (T_ <= (F32 ? 48 : 64)) over(integral_constant<int, 1>{}, integral_constant<int, 8>{});
-        else if (F32 && T_ <= 128) over(integral_constant<int, 1>{}, integral_constant<int, 16>{});
-        else if (F32) over(integral_constant<int, 1>{}, integral_constant<int, 32>{});
-        else if (T_ <= 128) over(integral_constant<int, 2>{}, integral_constant<int, 8>{});
-        else if (T_ <= 256) over(integral_constant<int, ALIGNED ? 2 : 4>{}, integral_constant<int, ALIGNED ? 16 : 8>{});
-        else if (T_ <= 384) over(integral_constant<int, 3>{}, integral_constant<int, 16>{});
-        else over(integral_constant<int, 4>{}, integral_constant<int, 16>{});
-    };
-    if (p.probs_vec) split(std::true_type{});
-    else split(std::false_type{});
+    for (int k0 = 0; k0 < 16; k0 += RPW * RIF) {
+        if (r0 + rs * k0 >= p.L) break;
+        softmax_rows<T, T, NCH, LPR, RIF, ALIGNED, false>((const T*)p.out, (T*)p.probs, segs, p.T, [&](int i, int64_t& row, int& in_head) {
+            const int at = r0 + rs * (k0 + RPW * i + lane / LPR);
+            in_head = at < p.L ? at : r0;
+            row = first + in_head;
+            return at < p.L;
+        });
+    }
 }
 
 // Launches the line-wise kernel when the problem has its shape (see sddmm_lines.hip); returns 1 when it did, 2 when it took the

@@ -27,8 +27,9 @@ struct Vec4 {
 
 }  // namespace
 
-// S^T = K Q^T: a lane owns one row and holds four consecutive positions of every 16.  KS: 32-value steps of the contraction.
-template <typename T, int KS, bool KT>
+// S^T = K Q^T: a lane owns one row and holds four consecutive positions of every 16.  KS: 32-value steps of the contraction.  SM: the softmax of
+// its rows that a wavefront takes at the end (sddmm_params.hpp).
+template <typename T, int KS, bool KT, int SM>
 __global__ __launch_bounds__(256, 4) void sddmm_rows16_kernel(const SddmmParams p) {
     constexpr int ROWB = KS == 1 ? 64 : KS == 2 ? 128 : 256;  // bytes of an LDS row: a power of two, for the swizzle
     constexpr int STAGE = kTile * ROWB, CPR = 4 * KS, NP = kTile * CPR / 256;
@@ -177,7 +178,7 @@ __global__ __launch_bounds__(256, 4) void sddmm_rows16_kernel(const SddmmParams 
             stage ^= STAGE;
         }
     }
-    if (p.probs) softmax_own_rows<T>(p, bh, r0 + rs * 16 * wave, rs);
+    if constexpr (SM != kNoSoftmax) softmax_own_rows<T, SM, false>(p, bh, r0 + rs * 16 * wave, rs);
 }
 
 int launch_sddmm_rows16(const SddmmParams& p0, int in_dtype, bool kt, hipStream_t st) {
@@ -216,10 +217,13 @@ int launch_sddmm_rows16(const SddmmParams& p0, int in_dtype, bool kt, hipStream_
     auto go = [&](auto t, auto kt_c) {
         using T = decltype(t);
         constexpr bool KT = decltype(kt_c)::value;
-        if (p.d <= 32) sddmm_rows16_kernel<T, 1, KT><<<grid, 256, 0, st>>>(p);
-        else if (p.d <= 64) sddmm_rows16_kernel<T, 2, KT><<<grid, 256, 0, st>>>(p);
-        else if (p.d <= 96) sddmm_rows16_kernel<T, 3, KT><<<grid, 256, 0, st>>>(p);
-        else sddmm_rows16_kernel<T, 4, KT><<<grid, 256, 0, st>>>(p);
+        by_split_of<kSoftmax32, kSoftmax512>(p, [&](auto sm) {
+            constexpr int SM = decltype(sm)::value;
+            if (p.d <= 32) sddmm_rows16_kernel<T, 1, KT, SM><<<grid, 256, 0, st>>>(p);
+            else if (p.d <= 64) sddmm_rows16_kernel<T, 2, KT, SM><<<grid, 256, 0, st>>>(p);
+            else if (p.d <= 96) sddmm_rows16_kernel<T, 3, KT, SM><<<grid, 256, 0, st>>>(p);
+            else sddmm_rows16_kernel<T, 4, KT, SM><<<grid, 256, 0, st>>>(p);
+        });
     };
     auto by_type = [&](auto kt_c) { return in_dtype == SPLAT_BF16 ? go(bf16{}, kt_c) : go(f16{}, kt_c); };
     if (kt) by_type(std::true_type{});
