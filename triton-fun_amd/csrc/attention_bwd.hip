@@ -40,7 +40,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(const BwdParams p) {
     const int lm = lane & 31, g = lane >> 5;
 
     load_args(p.total, p.n_row_blocks, p.by_blocks.m, p.by_blocks.shift, p.by_h.m, p.by_h.shift, p.H, p.row_stride, p.L, p.n_seg, p.plan, p.scale_log2e,
-              p.a, p.a_sb, p.a_sh, p.a_sl, p.b, p.b_sb, p.b_sh, p.b_sl, p.x, p.x_sb, p.x_sh, p.x_sl, p.y, p.y_sb, p.y_sh, p.y_sl, p.lse, p.delta);
+              p.a, p.a_sb, p.a_sh, p.a_sl, p.b, p.b_sb, p.b_sh, p.b_sl, p.x, p.x_sb, p.x_sh, p.x_sl, p.y, p.y_sb, p.y_sh, p.y_sl, p.lse);
     const int logical = xcd_remap(blockIdx.x, p.total);
     if (logical >= p.total) return;
     const int bh = quotient(logical, p.by_blocks);
@@ -382,6 +382,8 @@ template <typename T, int D>
 static int launch_bwd(BwdParams p, hipStream_t st) {
     begin_launch();
     constexpr int LDS_BYTES = 2 * (2 * 64 * D * 2);  // two stages of two tiles
+    p.total = p.B * p.H * p.n_row_blocks;
+    p.by_blocks = divisor(p.n_row_blocks), p.by_h = divisor(p.H);
     const int grid = ((p.total + 7) / 8) * 8;
     auto kern = attn_bwd_kernel<T, D>;
     static uint64_t lds_reserved = 0;
@@ -500,8 +502,7 @@ static BwdParams bwd_keys_params(const BwdParams& base, Rows3 q, Rows3 k, Rows3 
     pk.out = dk; pk.out2 = dv; pk.o_sb = (int64_t)base.H * Lk * d; pk.o_sh = (int64_t)Lk * d; pk.o_sl = d;
     pk.Lr = Lk; pk.row_map = row_map;
     pk.n_seg = n_seg_t; pk.row_stride = common_row_stride(segs_t, n_seg_t);
-    pk.n_row_blocks = count_row_blocks(Lk, kPlanBM, pk.row_stride); pk.total = base.B * base.H * pk.n_row_blocks;
-    pk.by_blocks = divisor(pk.n_row_blocks), pk.by_h = divisor(pk.H);
+    pk.n_row_blocks = count_row_blocks(Lk, kPlanBM, pk.row_stride);
     pk.plan = static_cast<const PlanRec*>(plan_t);
     return pk;
 }
@@ -543,8 +544,7 @@ static int bwd_impl(const char* who, bool f32, const void* q, int64_t q_sb, int6
     pq.y = v; pq.y_sb = v_sb; pq.y_sh = v_sh; pq.y_sl = v_sl;
     pq.out = dq; pq.o_sb = (int64_t)H * L * d; pq.o_sh = (int64_t)L * d; pq.o_sl = d;  // the gradients are contiguous [B, H, L, d]
     pq.n_seg = n_seg; pq.row_stride = common_row_stride(segs, n_seg);
-    pq.n_row_blocks = count_row_blocks(L, kPlanBM, pq.row_stride); pq.total = B * H * pq.n_row_blocks;
-    pq.by_blocks = divisor(pq.n_row_blocks), pq.by_h = divisor(H);
+    pq.n_row_blocks = count_row_blocks(L, kPlanBM, pq.row_stride);
     pq.plan = static_cast<const PlanRec*>(plan);
     pq.o = out; pq.oo_sb = o_sb; pq.oo_sh = o_sh; pq.oo_sl = o_sl; pq.delta_w = delta;  // D = rowsum(dO * O): computed and stored by this launch
     // dK, dV: rows = keys, the transposed mask's plan

@@ -393,7 +393,7 @@ static int launch(const BwdParams& p0, hipStream_t st) {
     static_assert(LDS_BYTES <= 160 * 1024 / (D == 64 ? 3 : 2), "workgroups per compute unit");
     BwdParams p = p0;
     p.total = p.B * p.H * 2 * p.n_row_blocks;
-    p.by_blocks = divisor(2 * p.n_row_blocks);
+    p.by_blocks = divisor(2 * p.n_row_blocks), p.by_h = divisor(p.H);
     auto kern = attn_bwd_pair_kernel<T, D>;
     static uint64_t lds_reserved = 0;
     if (int rc = reserve_dynamic_lds(&lds_reserved, reinterpret_cast<const void*>(kern), LDS_BYTES, "splat_attention_bwd")) return rc;

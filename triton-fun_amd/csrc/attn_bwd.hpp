@@ -21,8 +21,9 @@ struct BwdParams {
     int Lr;               // rows of the launch: L, or the number of rows of a rectangular keys' side (dK + dV of selected keys)
     const int* row_map;   // [Lr] or null: the row of A / B that row r of the mask stands for (r itself when null)
     float scale, scale_log2e;
-    int n_seg, n_row_blocks, total, row_stride;
-    Divisor by_blocks, by_h;  // workgroups per head and H, filled in by the launch
+    int n_seg, n_row_blocks, row_stride;
+    int total;                // workgroups; with by_blocks (workgroups per head) and by_h (H) filled in by the launch
+    Divisor by_blocks, by_h;
     const PlanRec* plan;  // plan table of the mask (dQ) or of its transpose (dK + dV), first variant
 };
 

@@ -57,7 +57,7 @@ __global__ __launch_bounds__(512, 4) void spmm_thin_kernel(const SpmmParams p) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, g4 = lane >> 4;
 
-    load_args(p.total, p.by_chunks.m, p.by_chunks.shift, p.by_blocks.m, p.by_blocks.shift, p.by_h.m, p.by_h.shift, p.n_row_blocks, p.H, p.row_stride, p.L,
+    load_args(p.total, p.by_blocks.m, p.by_blocks.shift, p.by_h.m, p.by_h.shift, p.n_row_blocks, p.H, p.row_stride, p.L,
               p.n_keys, p.n_out, p.T, p.n_seg, p.plan, p.v, p.v_sb, p.v_sh, p.v_sl, p.p);
     const int logical = xcd_remap(blockIdx.x, p.total);
     if (logical >= p.total) return;
@@ -361,7 +361,7 @@ static int launch_thin_variant(const char* who, SpmmParams p, hipStream_t st) {
     const int64_t blocks = (int64_t)p.B * p.H * p.n_row_blocks;
     if (blocks > 0x7ffffff0) return 0;
     p.total = (int)blocks;
-    p.by_chunks = divisor(1), p.by_blocks = divisor(p.n_row_blocks), p.by_h = divisor(p.H);
+    p.by_blocks = divisor(p.n_row_blocks), p.by_h = divisor(p.H);
     static uint64_t reserved = 0;
     // (two register sets: more request the lines earlier, which buys nothing -- loads return in order, and the wait for a
     // step's V rows covers every line requested before them -- and costs registers: d = 64 with 3 / 4 / 6 sets is 2 / 5 / 20 %

@@ -54,7 +54,7 @@ __global__ __launch_bounds__(512, 4) void spmm_tile_kernel(const SpmmParams p) {
     const int li = lane & 15, g4 = lane >> 4;
     const int cg = wave & 3, fh = wave >> 2;
 
-    load_args(p.total, p.by_chunks.m, p.by_chunks.shift, p.by_blocks.m, p.by_blocks.shift, p.by_h.m, p.by_h.shift, p.n_row_blocks, p.H, p.row_stride, p.L,
+    load_args(p.total, p.by_blocks.m, p.by_blocks.shift, p.by_h.m, p.by_h.shift, p.n_row_blocks, p.H, p.row_stride, p.L,
               p.n_keys, p.n_out, p.T, p.n_seg, p.plan, p.v, p.v_sb, p.v_sh, p.v_sl, p.p);
     const int logical = xcd_remap(blockIdx.x, p.total);
     if (logical >= p.total) return;
@@ -303,7 +303,7 @@ static int launch_tile_variant(const char* who, SpmmParams p, hipStream_t st) {
     const int64_t blocks = (int64_t)p.B * p.H * p.n_row_blocks;
     if (blocks > 0x7ffffff0) return 0;
     p.total = (int)blocks;
-    p.by_chunks = divisor(1), p.by_blocks = divisor(p.n_row_blocks), p.by_h = divisor(p.H);
+    p.by_blocks = divisor(p.n_row_blocks), p.by_h = divisor(p.H);
     static uint64_t reserved = 0;
     auto kern = spmm_tile_kernel<T, D, PART>;
     if (int rc = reserve_dynamic_lds(&reserved, reinterpret_cast<const void*>(kern), G::LDS_BYTES, who)) return rc;
