@@ -166,7 +166,8 @@ __device__ __forceinline__ void softmax_rows(const Tin* __restrict__ x, Tout* __
             float& s = part[c % NP];
             if (!ALIGNED && c == cut) {
 #if defined(__HIP_DEVICE_COMPILE__)
-                asm("" : "+v"(again[c]));  // (compared here: answers found beforehand take two scalar registers a slot until then)
+                // (compared here: answers found beforehand take two scalar registers a slot until then)
+                if constexpr (LPR == 16) asm("" : "+v"(again[c]));
 #endif
                 s = NP > 1 || c == 0 ? add_chunk<true, true>(s, v[c], again[c]) : add_chunk<true, false>(s, v[c], again[c]);
             } else {
