@@ -1,5 +1,5 @@
-"""The backward's keys' side by pairs of wavefronts against float64 where its halves, stages and exchange can go wrong, and large
-launches of it against larger ones."""
+"""The backward's keys' side by pairs of wavefronts against float64 where its halves, stages and exchange can go wrong, and that a head's
+gradients do not depend on how many others there are."""
 import pytest
 import torch
 
@@ -46,8 +46,8 @@ def test_against_float64(dev, name, L, dtype, d):
         assert float((a.double().cpu() - w).norm()) <= rel * max(float(w.norm()), 0.1 * scale)
 
 
-def test_both_sides_of_the_line(dev):
-    """1024 heads of one row block, and one head more: the shared heads agree."""
+def test_a_head_s_bits_do_not_depend_on_the_launch(dev):
+    """1024 heads of one row block, and one head more: the same bits for the heads that both have."""
     most, L, d, dtype = 1024, 128, 128, torch.bfloat16
     g = torch.Generator(device=dev).manual_seed(5)
     q, k, v, grad = (torch.randn(1, most + 1, L, d, generator=g, device=dev).to(dtype) for _ in range(4))
@@ -55,4 +55,4 @@ def test_both_sides_of_the_line(dev):
     a = step(masks, *(t[:, :most].contiguous() for t in (q, k, v, grad)), dev, dtype)
     b = step(masks, q, k, v, grad, dev, dtype)
     for x, y in zip(a, b):
-        assert float((x.float() - y[:, :most].float()).norm() / x.float().norm()) <= 4e-3
+        assert torch.equal(x, y[:, :most])

@@ -1,25 +1,32 @@
 """The float32 forward and backward on split operands against float64: what the parts hold, and what they do not (taken again in
-float32 arithmetic)."""
+float32 arithmetic).  Forwards in launches of few, some and many row blocks, which three kernels take."""
 import pytest
 import torch
 
 import acsr_helpers as A
 from r_attention import RegularAttention, attention_launcher, attention_with_grad
+from test_gpu_f32_tiles import alike, copies
 
 pytestmark = pytest.mark.gpu
 
 
-def case(dev, masks, B, H, L, d, seed, scale_q=1.0, scale_k=1.0, scale_v=1.0):
+LAUNCHES = pytest.mark.parametrize("launch", ["few", "some", "many"])
+
+
+def case(dev, masks, B, H, L, d, seed, scale_q=1.0, scale_k=1.0, scale_v=1.0, launch="few"):
     g = torch.Generator().manual_seed(seed)
     q, k, v = (torch.randn(B, H, L, d, generator=g) * s for s in (scale_q, scale_k, scale_v))
     live = sum(m.device_mask(dev) for m in masks).cpu() > 0
     s = (q.double() @ k.double().transpose(2, 3) * d ** -0.5).masked_fill(~live, float("-inf"))
     want = torch.softmax(s, -1) @ v.double()
-    attn = RegularAttention(B, L, H, d, masks, 16, 16, dev, torch.float32, scale=d ** -0.5)
-    return attn, [q.to(dev), k.to(dev).transpose(2, 3), v.to(dev)], want, live
+    n = copies(launch, B * H, L)
+    attn = RegularAttention(B, L, H * n, d, masks, 16, 16, dev, torch.float32, scale=d ** -0.5)
+    q, k, v = (t.repeat(1, n, 1, 1).to(dev) for t in (q, k, v))
+    return attn, [q, k.transpose(2, 3), v], want, live
 
 
 def error(got, want):
+    got = alike(got, got.shape[1] // want.shape[1])
     return float((got.double().cpu() - want).norm() / want.norm())
 
 
@@ -27,27 +34,30 @@ def error(got, want):
 # times what that comes to, and far below what an operand's missing part would give (2^-17)
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("q,k,v", [(1, 1, 1), (1, 1, 1e-30), (1, 1, 1e-36), (1, 1, 1e36), (1e-20, 1e20, 1), (1e-35, 1e35, 1), (1e35, 1e-35, 1), (1e-36, 1, 1)])
-def test_scales_of_the_operands(dev, d, q, k, v):
-    attn, x, want, _ = case(dev, [A.causal_windowed_pattern(401, 149)], 1, 2, 401, d, d, q, k, v)
+@LAUNCHES
+def test_scales_of_the_operands(dev, d, q, k, v, launch):
+    attn, x, want, _ = case(dev, [A.causal_windowed_pattern(401, 149)], 1, 2, 401, d, d, q, k, v, launch)
     assert error(attn(x), want) <= 1e-6
 
 
 @pytest.mark.parametrize("d", [64, 128])
-def test_scores_that_rise_along_the_walk(dev, d):
+@LAUNCHES
+def test_scores_that_rise_along_the_walk(dev, d, launch):
     """Later keys outrun the references of the first tiles by far more than an exponential holds."""
-    attn, x, want, _ = case(dev, [A.causal_windowed_pattern(300, 199)], 1, 2, 300, d, 3 * d)
+    attn, x, want, _ = case(dev, [A.causal_windowed_pattern(300, 199)], 1, 2, 300, d, 3 * d, launch=launch)
     x[1].mul_(torch.linspace(0.1, 60.0, 300, device=dev))
-    s = (x[0].double() @ x[1].double() * d ** -0.5).cpu()
+    s = (x[0][:, :2].double() @ x[1][:, :2].double() * d ** -0.5).cpu()
     live = A.causal_windowed_pattern(300, 199).device_mask(dev).cpu() > 0
-    want = torch.softmax(s.masked_fill(~live, float("-inf")), -1) @ x[2].double().cpu()
+    want = torch.softmax(s.masked_fill(~live, float("-inf")), -1) @ x[2][:, :2].double().cpu()
     assert error(attn(x), want) <= 1e-6 * float(s.abs().max())  # a score's rounding is relative to it
 
 
 @pytest.mark.parametrize("keys_along", [False, True])
 @pytest.mark.parametrize("L,d", [(400, 64), (400, 128), (96, 64)])
-def test_values_that_are_not_finite_reach_the_rows_that_see_them(dev, L, d, keys_along):
+@LAUNCHES
+def test_values_that_are_not_finite_reach_the_rows_that_see_them(dev, L, d, keys_along, launch):
     w = 40
-    attn, x, want, live = case(dev, [A.causal_windowed_pattern(L, w - 1)], 1, 2, L, d, L + d)
+    attn, x, want, live = case(dev, [A.causal_windowed_pattern(L, w - 1)], 1, 2, L, d, L + d, launch=launch)
     clean = attn(x).clone()
     x[2][:, :, 50, 3] = float("inf")
     x[2][:, :, 50, 7] = 3.4e38  # above what a bfloat16 holds
@@ -121,6 +131,7 @@ def small(at):
 
 
 def column_error(got, want):
+    got = alike(got, got.shape[1] // want.shape[1])
     return float((got[..., 5].double().cpu() - want[..., 5]).norm() / want[..., 5].norm())
 
 
@@ -163,7 +174,8 @@ def test_gradients_of_an_unlikely_key(dev, d):
 @pytest.mark.parametrize("keys_along", [False, True])
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("unlikely", [False, True])
-def test_forward_of_a_small_column(dev, d, unlikely, keys_along):
+@LAUNCHES
+def test_forward_of_a_small_column(dev, d, unlikely, keys_along, launch):
     """A column of V that is small, or that only an unlikely key has."""
     L, masks = 211, [A.causal_windowed_pattern(211, 69)]
     g = torch.Generator().manual_seed(d)
@@ -176,9 +188,11 @@ def test_forward_of_a_small_column(dev, d, unlikely, keys_along):
         small(2)(q, k, v)
     live = masks[0].device_mask(dev).cpu() > 0
     want = torch.softmax((q.double() @ k.double().transpose(2, 3) * d ** -0.5).masked_fill(~live, float("-inf")), -1) @ v.double()
-    attn = RegularAttention(1, L, 2, d, masks, 16, 16, dev, torch.float32, scale=d ** -0.5)
-    kT = k.to(dev).transpose(2, 3)
-    got = attn([q.to(dev), kT.contiguous() if keys_along else kT, v.to(dev)])
+    n = copies(launch, 2, L)
+    attn = RegularAttention(1, L, 2 * n, d, masks, 16, 16, dev, torch.float32, scale=d ** -0.5)
+    q, k, v = (t.repeat(1, n, 1, 1).to(dev) for t in (q, k, v))
+    kT = k.transpose(2, 3)
+    got = attn([q, kT.contiguous() if keys_along else kT, v])
     assert error(got, want) <= 1e-6 * (20 if unlikely else 1)
     rows = live[:, 30] if unlikely else torch.ones(L, dtype=torch.bool)
     assert column_error(got[:, :, rows.to(dev)], want[:, :, rows]) <= (2e-5 if unlikely else 1e-6)
@@ -191,7 +205,8 @@ WALKS = {"windowed": lambda L: [A.windowed_pattern(L, 23)], "gathered": lambda L
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("L", [130, 257])
 @pytest.mark.parametrize("name", list(WALKS))
-def test_rows_taken_again_on_every_walk(dev, name, L, d):
+@LAUNCHES
+def test_rows_taken_again_on_every_walk(dev, name, L, d, launch):
     """Column 0 of Q and V beyond what the parts hold, of K and dO zero: the same scores, every row in float32 arithmetic."""
     masks, B, H = WALKS[name](L), 1, 2
     g = torch.Generator().manual_seed(L + d)
@@ -206,20 +221,23 @@ def test_rows_taken_again_on_every_walk(dev, name, L, d):
     grads = [torch.nan_to_num(t) for t in torch.autograd.grad(want, wide, go.double())]
     want = want.detach()
 
+    n = copies(launch, B * H, L)
+
     def close(got, want):  # N(0, 1) columns, and column 0, which may be 2^90 times as large
+        got = alike(got, n)
         for part in (slice(0, 1), slice(1, None)):
             a, b = got[..., part].double().cpu(), want[..., part]
             assert float((a - b).abs().max()) <= 2e-5 * max(1.0, float(b.abs().max()))
 
-    attn = RegularAttention(B, L, H, d, masks, 16, 16, dev, torch.float32, scale=d ** -0.5)
-    on = [t.to(dev) for t in (q, k, v)]
+    attn = RegularAttention(B, L, H * n, d, masks, 16, 16, dev, torch.float32, scale=d ** -0.5)
+    on = [t.repeat(1, n, 1, 1).to(dev) for t in (q, k, v)]
     for kT in (on[1].transpose(2, 3), on[1].transpose(2, 3).contiguous()):
         close(attn([on[0], kT, on[2]]), want)
         out = torch.empty_like(on[0])  # without a plan table
-        attention_launcher(on[0], kT, on[2], out, attn.segments, d ** -0.5)
+        attention_launcher(on[0], kT, on[2], out, attn.segments, d ** -0.5, live_percent=attn._live_percent)
         close(out, want)
     on = [t.requires_grad_(True) for t in on]
-    for a, b in zip(torch.autograd.grad(attention_with_grad(*on, attn), on, go.to(dev)), grads):
+    for a, b in zip(torch.autograd.grad(attention_with_grad(*on, attn), on, go.repeat(1, n, 1, 1).to(dev)), grads):
         close(a, b)
 
 

@@ -18,8 +18,10 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("pattern", [lambda L: A.causal_windowed_pattern(L, 5), lambda L: A.causal_windowed_pattern(L, 128),
                                      lambda L: A.causal_windowed_pattern(L, 129), lambda L: A.dilated_pattern(L, 77, 3),
                                      lambda L: A.strided_patterns(L, 40, 16), lambda L: A.causal_windowed_pattern(L, 201),
-                                     lambda L: A.blocked_pattern(L, 200), lambda L: A.causal_windowed_pattern(L + 51, 257)],
-                         ids=["5", "128", "129", "dilated 77", "strided", "201", "blocked 200", "257"])
+                                     lambda L: A.blocked_pattern(L, 200), lambda L: A.causal_windowed_pattern(L + 51, 257),
+                                     *((lambda w: lambda L: A.causal_windowed_pattern(L + 51, w - 1))(w) for w in (32, 33, 64, 65, 256))],
+                         ids=["5", "128", "129", "dilated 77", "strided", "201", "blocked 200", "257", "edge 32", "edge 33", "edge 64", "edge 65",
+                              "edge 256"])
 @pytest.mark.parametrize("layout", ["rows", "keys"])
 def test_equals_the_two_calls(dev, layout, pattern, heads, dtype, d):
     L = 250
