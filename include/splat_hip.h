@@ -175,8 +175,8 @@ int splat_softmax(const void* x, void* y, const splat_acsr_seg* segs /* host */,
 
 /* splat_sddmm_planned without statistics (plan may be NULL), then splat_softmax of its output into `probs` ([B,H,L,T]
  * contiguous, dtype out_dtype, not overlapping out; rows without live slots and dead slots stay as they are in both).
- * Where the wavefronts of the sampled product own whole rows of at most 512 slots (float32: 256; enough row blocks for the chip, and no
- * more scores than the caches hold), they take their softmax as well, and a launch and a pass over memory are spared
+ * Where the wavefronts of the sampled product own whole rows (enough row blocks for the chip), of 16-bit scores up to 512 slots and 80 MB, of float32
+ * ones up to 256 slots (200 in launches of more than 2048 row blocks of 64 rows go without), they take their softmax as well, and a launch and a pass over memory are spared
  * (float16, 16 heads of 2000 rows, 129 slots, d = 80, with splat_spmm: 26.7 -> 21 us); elsewhere the second launch
  * follows.  Both results are those of the two calls, bit for bit.  Replaces r_sddmm.py:153-188 and r_softmax.py:126-150. */
 int splat_sddmm_softmax(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* kT, int64_t k_sb,

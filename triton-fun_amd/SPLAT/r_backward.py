@@ -310,7 +310,7 @@ def attention_backward_fused(q: torch.Tensor, kT: torch.Tensor, v: torch.Tensor,
                              lse: torch.Tensor, segments: ACSRSegments, segments_t: ACSRSegments, plan: torch.Tensor,
                              plan_t: torch.Tensor, scale: float = 1.0, sparse_rows: bool | None = None):
     """(dq, dk, dv) as ``attention_backward`` gives them, without a compressed matrix, from two launches (dQ, then dK and dV from
-    one walk) or, 16-bit types at d = 128 in launches of more than 1024 row blocks, three: ``out`` and ``lse`` are the output and the row statistic of the fused forward for the same inputs
+    one walk): ``out`` and ``lse`` are the output and the row statistic of the fused forward for the same inputs
     (``RegularAttention.forward_with_stats``), ``plan`` / ``plan_t`` the fused kernel's plans (``attention_plan``) of the
     mask's segments and of the transposed mask's.  One dtype, d in {64, 128}; operands whose rows are not contiguous
     16-byte pieces (K^T-contiguous keys among them) are copied first.  Segments of the transposed mask that keep few keys

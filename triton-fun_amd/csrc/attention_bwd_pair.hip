@@ -7,7 +7,9 @@
 // wavefronts share 32 of them: of every tile of 64 positions each computes S, P, dP and dS of its own 32, one wavefront of the pair keeps
 // dK and the other dV, and what the other one needs (dS of the one half, P of the other: 2 KiB as ready B operands) goes through
 // LDS, between two barriers a tile: its own half each wavefront accumulates before the second.  73 KiB and 256 registers a wavefront at
-// d = 128, two workgroups a CU, whose phases cover each other; 41 KiB and 168 at d = 64, three.
+// d = 128, two workgroups a CU, whose phases cover each other; 41 KiB and 168 at d = 64, three.  At d = 128 two of a lane's sixteen fragments of
+// K and V do not fit: 36 bytes of scratch, of which every tile reads 16 before its scores and 16 before dP, and the second wait is one for the
+// next tile's copies, which were requested in between.
 // lse and D belong to the positions: 64 floats each a tile, copied into LDS beside the tiles, whose swizzle serves the row-wise reads of
 // the scores and the transposing ones of the accumulation (tile_copy.hpp: dual_chunk).
 // K and V come through LDS as well, where tile 1 will lie: loaded by every wavefront for itself, 32 bytes of 32 rows an

@@ -10,6 +10,10 @@
 // Against attention_rows16.hip, which took these launches: bf16, 4 heads of 1024 rows, windows 32 / 128 / 512: d = 64 5.7 -> 4.2 us,
 // 6.6 -> 4.8, 11.2 -> 6.1; d = 128 6.7 -> 4.9, 7.9 -> 6.0, 14.4 -> 7.7; the lines are in dispatch_attn (attention.hip).
 //
+// Eight wavefronts at d = 64 on keys that lie anywhere have 44 bytes of scratch: two addresses of K's rows are read again each tile, beside K's
+// own loads and in front of them, the rest before and after the walk.  A counted wait leaves the youngest requests open, so what stands
+// between them makes it wait for more, never for less.
+//
 // Layouts are those of attention.hip (32x32x16, transposed products, one lane a row).  K's tile is free once the scores are
 // taken and V's once the output is, so that one stage of each holds the next tile's copies while the other product runs.
 #include <type_traits>

@@ -70,7 +70,8 @@ __device__ __forceinline__ void mask_half(f32x16& s, uint32_t bits) {
     }
 }
 
-// Keys c .. c + 7 of a row of K^T that may start anywhere; keys that do not exist are zero (L >= 8).
+// Keys c .. c + 7 of a row of K^T that may start anywhere (L >= 8).  Behind the row's last key there are zeros, or, in a piece that begins
+// there, some of its last keys: positions that no row sees, whose scores are masked.
 template <typename T>
 __device__ __forceinline__ u32x4 keys_piece(const T* row, int c, int L) {
     const int over = min(max(c + 8 - L, 0), 8);  // how many of them do not exist: the row's last whole piece, moved down

@@ -5,7 +5,7 @@
 // sizes whose kernels take less than that (a few hundred row blocks) run at the interpreter's speed, and a training step, whose
 // backward an autograd thread runs under the interpreter's lock, at 90 us.  Here a call reads the tensors' fields directly.
 //
-// Every entry point handles the ordinary case (tensors on the current device, rows in whole 16-byte pieces) and returns False
+// Every entry point (of the three operators together as well) handles the ordinary case (tensors on the current device, rows in whole 16-byte pieces) and returns False
 // (attend: None) for anything else, before it has done anything: the Python launchers then take the call, with their copies and
 // their messages.  The kernels are reached through the addresses that `bind` receives, so that both layers use one library.
 #include <Python.h>

@@ -533,7 +533,8 @@ static int sddmm_common(const char* who, const void* q, int64_t q_sb, int64_t q_
     // Stores around the caches pay for large outputs of whole 64-byte pieces.  The three operators, bfloat16, causal masks, d = 64 and 128, share
     // of the time with them: 150 to 540 MB of 288 to 512 slots, a multiple of 32, 0.85 to 0.99; of 200 or 304 slots, whose rows share such
     // pieces, 1.05 to 1.31, of 1000 1.25 to 1.44; and up to 80 MB, which the next operator finds in the caches, 1.02 to 1.17 (from 88 to
-    // 134 MB 0.88 to 1.17).
+    // 134 MB 0.88 to 1.17).  The product by itself is slower through the caches (32 heads of 4096 rows, 256 slots, d = 64, 67 MB: 22.4 -> 25.4 us); the
+    // two operators that read after it give that back and more.
     p.out_stream = p.out_vec && T % 32 == 0 && (int64_t)B * H * L * T * 2 > kCachedBytes;
     for (int k = 0; k < n_seg; ++k)
         if (segs[k].slot_offset % 32 != 0) p.out_stream = 0;
