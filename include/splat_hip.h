@@ -209,6 +209,19 @@ int splat_spmm_planned(const void* p, const void* v, int64_t v_sb, int64_t v_sh,
                        int32_t n_keys, int32_t n_out, int32_t T, int32_t in_dtype, int32_t out_dtype,
                        const void* plan, int64_t plan_bytes, void* stream);
 
+/* The three operators in one launch: splat_sddmm_planned's scores, splat_softmax's probabilities and splat_spmm_planned's output for q, kT, v of
+ * one 16-bit dtype (scores, probs [B,H,L,T] and out [B,H,L,d] contiguous, of that dtype; scores and probs not overlapping; n_keys rows of v).
+ * Scores and probabilities are those of the separate calls bit for bit and stay in the workgroup from one product to the next, so that nothing
+ * reads the compressed matrices.  SPLAT_E_UNSUPPORTED, with nothing launched and no error message, where the separate calls are faster
+ * (several segments of more than 64 slots together, many workgroups of rows of more than 256) and for what the kernel does not take:
+ * float32, d not a multiple of 8 or above 128, T above 512, rows that are not whole 16-byte pieces (q, v, out, and kT unless its keys
+ * are contiguous).  Replaces r_attention.py:77-100 (rsddmm_launcher, rsoftmax_launcher, rspmm_launcher). */
+int splat_operators(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* kT, int64_t k_sb, int64_t k_sh,
+                    int64_t k_sd, int64_t k_sl, const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sl, void* scores,
+                    void* probs, void* out, const splat_acsr_seg* segs /* host */, int32_t n_seg, int32_t B, int32_t H,
+                    int32_t L, int32_t n_keys, int32_t d, int32_t T, float scale, int32_t dtype, const void* plan,
+                    int64_t plan_bytes, void* stream);
+
 /* Fused forward: out = softmax_over_live_columns(scale * q.kT) . v with online softmax; the
  * compressed score matrix is never written to memory.  Equals the composition
  * rsddmm_launcher -> rsoftmax_launcher -> rspmm_launcher of RegularAttention.forward

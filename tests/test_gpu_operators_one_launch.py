@@ -1,0 +1,175 @@
+"""The three operators in one launch (splat_operators) against the three calls, bit for bit, and against float64: rows at the edges of what a row of
+LDS holds, row blocks that interleave, two segments, rows whose steps differ, heads that are padded, K along the keys, sequences that end
+inside a workgroup and inside a wavefront's rows."""
+import ctypes
+
+import pytest
+import torch
+
+import acsr_helpers as A
+import _splat_hip as hip
+from r_sddmm import live_slot_columns
+from test_gpu_operators import SENTINEL
+
+pytestmark = pytest.mark.gpu
+
+
+def _steps_differ(L):
+    """Rows of 0 to 9 slots whose steps are 1, 2 and 3 in turns: no walk in which positions are slots."""
+    mask = torch.zeros(L, L, dtype=torch.uint8)
+    for i in range(L):
+        n, step = i % 10, 1 + i % 3
+        for t in range(n):
+            if i + step * t < L:
+                mask[i, i + step * t] = 1
+    return mask
+
+
+MASKS = {"1": lambda L: A.causal_windowed_pattern(L, 0), "7": lambda L: A.causal_windowed_pattern(L, 6),
+         **{str(w): (lambda w: lambda L: A.causal_windowed_pattern(L, w - 1))(w) for w in (33, 64, 65, 128, 129, 200, 256, 257, 509, 512)},
+         "windowed 257": lambda L: A.windowed_pattern(L, 128), "blocked 64": lambda L: A.blocked_pattern(L, 64),
+         "blocked 512": lambda L: A.blocked_pattern(L, 256), "dilated 77 by 3": lambda L: A.dilated_pattern(L, 77, 3),
+         "dilated 300 by 2": lambda L: A.dilated_pattern(L, min(300, L // 2), 2), "strided": lambda L: A.strided_patterns(L, 20, 40),
+         "strided 7": lambda L: A.strided_patterns(L, 7, L // 50), "steps differ": _steps_differ}
+
+
+def _operands(dev, dtype, heads, L, d, layout, seed=0):
+    g = torch.Generator(device=dev).manual_seed(seed + L + d)
+    if layout == "tokens":
+        q, k, v = (torch.randn(1, L, heads, d, generator=g, device=dev).to(dtype).transpose(1, 2) for _ in range(3))
+    else:
+        q, k, v = (torch.randn(1, heads, L, d, generator=g, device=dev).to(dtype) for _ in range(3))
+    kT = k.transpose(2, 3)
+    return q, kT.contiguous() if layout == "keys" else kT, v
+
+
+def _one_launch(segs, q, kT, v, scale, buffers):
+    heads, L, d = q.shape[1:]
+    arr, plan = segs.seg_array(L, segs.T), segs.plan(L, q.device)
+    return hip.lib().splat_operators(q.data_ptr(), *q.stride()[:3], kT.data_ptr(), *kT.stride()[:4], v.data_ptr(), *v.stride()[:3],
+                                     *(b.data_ptr() for b in buffers), arr, len(segs), 1, heads, L, v.shape[2], d, segs.T, ctypes.c_float(scale),
+                                     hip.dtype_code(q.dtype), plan.data_ptr(), plan.numel() * plan.element_size(), hip.stream_ptr(q.device))
+
+
+def _segments(mask, dev):
+    if not isinstance(mask, list):
+        mask = [mask]
+    return A.create_acsr_segments(mask, 16, dev)
+
+
+@pytest.mark.parametrize("dtype,d,layout", [(torch.bfloat16, 64, "rows"), (torch.float16, 128, "tokens"), (torch.bfloat16, 80, "keys"),
+                                            (torch.float16, 32, "keys"), (torch.bfloat16, 104, "rows")])
+@pytest.mark.parametrize("L,heads", [(600, 3), (1037, 8), (600, 54), (700, 140)])  # (eight wavefronts a workgroup and, from 512 workgroups on, four)
+@pytest.mark.parametrize("mask", list(MASKS))
+def test_equals_the_three_calls(dev, mask, L, heads, dtype, d, layout):
+    segs = _segments(MASKS[mask](L), dev)
+    T = segs.T
+    q, kT, v = _operands(dev, dtype, heads, L, d, layout)
+    arr, code, stream, plan = segs.seg_array(L, T), hip.dtype_code(dtype), hip.stream_ptr(dev), segs.plan(L, dev)
+    sizes = [heads * L * T + 8, heads * L * T + 8, heads * L * d + 8]
+    want, got = ([torch.full((n,), SENTINEL, dtype=dtype, device=dev) for n in sizes] for _ in range(2))
+    rc = _one_launch(segs, q, kT, v, 0.2, got)
+    if T > 256 and heads != 8:  # (left to the separate calls, but for many heads of up to 64 values)
+        assert (rc == 0) == (d <= 64 and (heads == 3 or (heads == 140 and T >= 384)))
+    else:
+        assert rc == 0
+    if rc:
+        assert rc == -5 and all(torch.all(b == SENTINEL) for b in got)
+        return
+    table = (plan.data_ptr(), plan.numel() * plan.element_size())
+    rows = kT if layout != "keys" else kT.transpose(2, 3).contiguous().transpose(2, 3)
+    hip.check(hip.lib().splat_sddmm_planned(q.data_ptr(), *q.stride()[:3], rows.data_ptr(), *rows.stride()[:4], want[0].data_ptr(), arr, len(segs), 1, heads,
+                                            L, L, d, T, ctypes.c_float(0.2), code, code, None, *table, stream), "splat_sddmm_planned")
+    hip.check(hip.lib().splat_softmax(want[0].data_ptr(), want[1].data_ptr(), arr, len(segs), heads, L, T, code, code, stream), "splat_softmax")
+    hip.check(hip.lib().splat_spmm_planned(want[1].data_ptr(), v.data_ptr(), *v.stride()[:3], want[2].data_ptr(), arr, len(segs), 1, heads, L, L, d, T, code,
+                                           code, *table, stream), "splat_spmm_planned")
+    scores = [b[0][:-8].double() for b in (want, got)]
+    eps = torch.finfo(dtype).eps
+    if T > 256 and not torch.equal(*scores):
+        # (the general kernel, which takes some launches of longer rows, adds in another order: a float32 sum of d products of a size of 5 apart, rounded)
+        assert float((scores[0] - scores[1]).abs().max()) <= 8 * eps
+    else:
+        assert torch.equal(want[0], got[0]) and torch.equal(want[1], got[1])
+        if T >= 8 and len(segs) == 1:  # (shorter rows and segments are the general kernel's)
+            assert torch.equal(want[2], got[2])
+    # dead slots and what lies behind the buffers stay as they were
+    for b in got:
+        assert torch.all(b[-8:] == SENTINEL)
+    few = slice(0, 3)
+    out = torch.zeros(heads, L, d, dtype=torch.float64, device=dev)[few]
+    live_rows = torch.zeros(L, device=dev)
+    for t, fc, off in zip(segs.tuples, segs.first_cols, segs.offsets):
+        cols, live = live_slot_columns(t[2], t[3], t[4], int(t[5]), fc)
+        part = got[1][:-8].view(heads, L, T)[few, :, off:off + int(t[5])].double()
+        assert torch.all(part[:, ~live] == SENTINEL) and torch.all(got[0][:-8].view(heads, L, T)[few, :, off:off + int(t[5])].double()[:, ~live] == SENTINEL)
+        dense = torch.zeros(len(out), L, L, dtype=torch.float64, device=dev)
+        dense.scatter_add_(2, cols.clamp(0, L - 1).expand(len(out), L, -1), torch.where(live, part, 0.0))
+        out += dense @ v[0, few].double()
+        live_rows += t[4]
+    # (probabilities that sum to 1 times values of at most 6: the float32 sum of up to 512 of them, and one rounding to the type)
+    err = (got[2][:-8].view(heads, L, d)[few].double() - out).abs()
+    assert float((err - out.abs() * eps / 2 * 1.01).max()) <= 512 * 6 * 2.0 ** -24
+    rows_sum = torch.where(got[1][:-8].view(heads, L, T).double() == SENTINEL, 0.0, got[1][:-8].view(heads, L, T).double()).sum(-1)
+    assert float((rows_sum - (live_rows > 0).double()).abs().max()) <= eps + 512 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("T", [104, 128, 256, 416])
+def test_large_matrices_equal_their_halves(dev, T):
+    """Scores and probabilities that the caches do not hold are stored around them: the same bits."""
+    L, d, dtype, heads = 2048, 32, torch.bfloat16, 96 if T > 256 else 2 * -(-(84 << 20) // (4 * 2048 * T))
+    segs = _segments(A.causal_windowed_pattern(L, T - 1), dev)
+    q, kT, v = _operands(dev, dtype, heads, L, d, "rows")
+
+    def both(h0, n):
+        bufs = [torch.full((n, L, w), SENTINEL, dtype=dtype, device=dev) for w in (T, T, d)]
+        hip.check(_one_launch(segs, q[:, h0:h0 + n], kT[:, h0:h0 + n], v[:, h0:h0 + n], 0.2, bufs), "splat_operators")
+        return bufs
+    whole, parts = both(0, heads), [both(0, heads // 2), both(heads // 2, heads // 2)]
+    for i in range(3):
+        assert torch.equal(whole[i], torch.cat([x[i] for x in parts]))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("mask", ["33", "512", "strided"])
+def test_infinities_and_not_a_number(dev, dtype, mask):
+    """Scores of minus infinity weigh nothing, rows of nothing but them give zeros, NaN stays in the rows that see it: as the three calls."""
+    L, d, heads = 600, 64, 2
+    segs = _segments(MASKS[mask](L), dev)
+    T = segs.T
+    q, kT, v = _operands(dev, dtype, heads, L, d, "rows")
+    q, kT = q.clone(), kT.transpose(2, 3).clone().transpose(2, 3)
+    q[:, 0, 40:80] = 1.0
+    kT[:, 0, :, 30:60] = float("-inf")
+    kT[:, 1, 3, 100] = float("nan")
+    arr, code, stream, plan = segs.seg_array(L, T), hip.dtype_code(dtype), hip.stream_ptr(dev), segs.plan(L, dev)
+    want, got = ([torch.full((heads, L, w), SENTINEL, dtype=dtype, device=dev) for w in (T, T, d)] for _ in range(2))
+    hip.check(_one_launch(segs, q, kT, v, 1.0, got), "splat_operators")
+    table = (plan.data_ptr(), plan.numel() * plan.element_size())
+    hip.check(hip.lib().splat_sddmm_planned(q.data_ptr(), *q.stride()[:3], kT.data_ptr(), *kT.stride()[:4], want[0].data_ptr(), arr, len(segs), 1, heads,
+                                            L, L, d, T, ctypes.c_float(1.0), code, code, None, *table, stream), "splat_sddmm_planned")
+    hip.check(hip.lib().splat_softmax(want[0].data_ptr(), want[1].data_ptr(), arr, len(segs), heads, L, T, code, code, stream), "splat_softmax")
+    hip.check(hip.lib().splat_spmm_planned(want[1].data_ptr(), v.data_ptr(), *v.stride()[:3], want[2].data_ptr(), arr, len(segs), 1, heads, L, L, d, T, code,
+                                           code, *table, stream), "splat_spmm_planned")
+    for a, b in zip(got[:2], want[:2]):
+        assert torch.allclose(a.float(), b.float(), rtol=torch.finfo(dtype).eps, atol=8 * torch.finfo(dtype).eps, equal_nan=True)
+    assert torch.equal(torch.isnan(got[2]), torch.isnan(want[2]))
+    assert torch.allclose(got[2].float(), want[2].float(), rtol=0, atol=4 * torch.finfo(dtype).eps, equal_nan=True)
+
+
+def test_what_it_does_not_take(dev):
+    """Other types, dimensions, rows and addresses are left to the separate calls, before anything is written."""
+    L, heads = 300, 2
+    segs = _segments(A.causal_windowed_pattern(L, 19), dev)
+
+    def code(dtype=torch.bfloat16, d=64, segs=segs, shift=0):
+        q, kT, v = _operands(dev, dtype, heads, L, d, "rows")
+        bufs = [torch.full((heads * L * w + 8,), 7.0, dtype=dtype, device=dev) for w in (segs.T, segs.T, d)]
+        rc = _one_launch(segs, q, kT, v, 1.0, [bufs[0], bufs[1], bufs[2][shift:]])
+        torch.cuda.synchronize()
+        assert rc == 0 or all(bool(torch.all(b == 7.0)) for b in bufs)
+        return rc
+    assert code() == 0
+    assert code(dtype=torch.float32) == code(d=12) == code(d=136) == code(shift=1) == -5
+    assert code(segs=_segments(A.strided_patterns(L, 60, 16), dev)) == -5
+    L = 600
+    assert code(segs=_segments(A.causal_windowed_pattern(L, 512), dev)) == -5

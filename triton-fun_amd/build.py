@@ -16,7 +16,7 @@ LIB = os.path.join(LIB_DIR, "libsplat_hip.so")
 BENCH_LIB = os.path.join(LIB_DIR, "libsplat_bench.so")
 HOST_EXT = os.path.join(LIB_DIR, "_splat_host.so")
 
-SOURCES = ["api_common.cpp", "acsr_build.hip", "softmax.hip", "sddmm.hip", "sddmm_lines.hip", "spmm.hip", "spmm_thin.hip", "spmm_tile.hip", "spmm_t_thin.hip", "attention.hip", "attention_f32.hip", "attention_rows16.hip", "attention_shared.hip", "attention_shared_f32.hip", "backward.hip", "attention_bwd.hip", "attention_bwd_f32.hip", "attention_bwd_f32_keys.hip", "attention_bwd_pair.hip", "transpose.hip", "operators_f32.hip", "sddmm_rows16.hip"]
+SOURCES = ["api_common.cpp", "acsr_build.hip", "softmax.hip", "sddmm.hip", "sddmm_lines.hip", "spmm.hip", "spmm_thin.hip", "spmm_tile.hip", "spmm_t_thin.hip", "attention.hip", "attention_f32.hip", "attention_rows16.hip", "attention_shared.hip", "attention_shared_f32.hip", "backward.hip", "attention_bwd.hip", "attention_bwd_f32.hip", "attention_bwd_f32_keys.hip", "attention_bwd_pair.hip", "transpose.hip", "operators_f32.hip", "sddmm_rows16.hip", "operators16.hip"]
 # the measurement aids: a library of their own, so that the operator ABI holds operators only
 BENCH_SOURCES = ["api_common.cpp", "bench_probes.hip"]
 # packed fp32 VALU forms are switched off for every device compile

@@ -51,6 +51,7 @@ struct Api {
     decltype(&splat_sddmm_planned) sddmm_planned;
     decltype(&splat_softmax) softmax;
     decltype(&splat_sddmm_softmax) sddmm_softmax;
+    decltype(&splat_operators) operators;
     decltype(&splat_spmm) spmm;
     decltype(&splat_spmm_planned) spmm_planned;
     decltype(&splat_acsr_build_record) build_record;
@@ -593,6 +594,19 @@ PyObject* py_operators(PyObject*, PyObject* const* a, Py_ssize_t n) {
         if (scale == -1.0 && PyErr_Occurred()) return nullptr;
         const bool both = second.x->scalar_type() == second.out->scalar_type() && second.x->data_ptr() != second.out->data_ptr();
         const char* what;
+        // One launch, where the kernel takes it.  (K along the keys is turned on its way there, one key a lane: not where neighbouring lanes' keys lie
+        // in different lines.)
+        const Mask& planned = m[0]->plan.defined() ? *m[0] : *m[2];
+        if (both && planned.plan.defined() && first.y->size(3) == third.y->size(2) && third.x->data_ptr() == second.out->data_ptr() &&
+            third.out->scalar_type() == q->scalar_type() && !(first.turn && planned.max_step > 4)) {
+            const at::Tensor &k = *first.y, &v = *third.y, &s = *first.out;
+            const int rc = api.operators(q->data_ptr(), q->stride(0), q->stride(1), q->stride(2), k.data_ptr(), k.stride(0), k.stride(1), k.stride(2), k.stride(3),
+                                         v.data_ptr(), v.stride(0), v.stride(1), v.stride(2), s.data_ptr(), second.out->data_ptr(), out->data_ptr(),
+                                         planned.segs, planned.n_seg, q->size(0), q->size(1), q->size(2), k.size(3), q->size(3), s.size(3), (float)scale,
+                                         dtype_code(q->scalar_type()), planned.plan_ptr(), planned.plan_bytes(), stream_of(*q));
+            if (rc == 0) Py_RETURN_TRUE;
+            if (rc != SPLAT_E_UNSUPPORTED) return raise_rc("splat_operators", rc);
+        }
         if (const int rc = first.launch(*m[0], scale, both ? second.out : nullptr, &what)) return raise_rc(what, rc);
         if (!both)
             if (const int rc = second.launch(*m[1])) return raise_rc("splat_softmax", rc);
@@ -790,7 +804,7 @@ PyObject* py_bind(PyObject*, PyObject* args) {
         !take("splat_attention_bwd", api.bwd) || !take("splat_attention_bwd_keys", api.bwd_keys) ||
         !take("splat_attention_bwd_f32", api.bwd_f32) || !take("splat_attention_bwd_keys_f32", api.bwd_keys_f32) || !take("splat_sddmm", api.sddmm) ||
         !take("splat_sddmm_probs", api.sddmm_probs) || !take("splat_sddmm_planned", api.sddmm_planned) ||
-        !take("splat_softmax", api.softmax) || !take("splat_sddmm_softmax", api.sddmm_softmax) || !take("splat_spmm", api.spmm) || !take("splat_spmm_planned", api.spmm_planned) ||
+        !take("splat_softmax", api.softmax) || !take("splat_sddmm_softmax", api.sddmm_softmax) || !take("splat_operators", api.operators) || !take("splat_spmm", api.spmm) || !take("splat_spmm_planned", api.spmm_planned) ||
         !take("splat_acsr_build_record", api.build_record) || !take("splat_attention_plan_report", api.plan_report))
         return nullptr;
     Py_INCREF(err);

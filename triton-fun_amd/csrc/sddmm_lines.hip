@@ -287,7 +287,7 @@ __global__ __launch_bounds__(BM_ * 4, 4) void sddmm_lines_kernel(const SddmmPara
 #pragma unroll
                             for (int j = 0; j < 4; ++j) {
                                 const int pos = pos0 + 16 * kt + 4 * g4 + j;
-                                if (win_live(mine, pos)) row_out[win_slot(mine, pos)] = (T)(acc[half][kt][j] * out_scale);
+                                if (win_live(mine, pos)) row_out[win_slot(mine, pos)] = rounded<T>(acc[half][kt][j] * out_scale);
                             }
                     }
                     return;
@@ -296,7 +296,7 @@ __global__ __launch_bounds__(BM_ * 4, 4) void sddmm_lines_kernel(const SddmmPara
                 for (int kt = 0; kt < 2; ++kt) {
                     v4 t;
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) t[j] = (T)(acc[half][kt][j] * out_scale);
+                    for (int j = 0; j < 4; ++j) t[j] = rounded<T>(acc[half][kt][j] * out_scale);
                     const int ri = (pos0 + 16 * kt + 4 * g4 - lo4) & (R_SLOTS - 1);
                     *reinterpret_cast<v4*>(ring_mine + ri * 2) = t;
                 }

@@ -161,7 +161,7 @@ __global__ __launch_bounds__(256, 4) void sddmm_rows16_kernel(const SddmmParams 
                 }
                 vec4 x;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) x[j] = (T)s[j];
+                for (int j = 0; j < 4; ++j) x[j] = rounded<T>(s[j]);
                 const int at = ju + 4 * g - win.lo;  // of the lane's first position, from the row's first
                 if (ju >= span.lo_max && ju + 16 <= span.hi_min) {
                     __builtin_memcpy(dst + at, &x, 8);  // any alignment

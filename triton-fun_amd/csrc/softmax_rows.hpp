@@ -233,7 +233,7 @@ __device__ __forceinline__ void softmax_rows(const Tin* __restrict__ x, Tout* __
                 if (live[c] == 0xffu) {
                     vout o;
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) o[e] = (Tout)(v[c][e] * inv);
+                    for (int e = 0; e < 8; ++e) o[e] = rounded<Tout>(v[c][e] * inv);
                     if constexpr (!ALIGNED)
                         __builtin_memcpy(yr + at[c], &o, sizeof(vout));
                     else if constexpr (AROUND)
@@ -243,7 +243,7 @@ __device__ __forceinline__ void softmax_rows(const Tin* __restrict__ x, Tout* __
                 } else {
 #pragma unroll
                     for (int e = 0; e < 8; ++e)
-                        if ((live[c] >> e) & 1u) yr[at[c] + e] = (Tout)(v[c][e] * inv);
+                        if ((live[c] >> e) & 1u) yr[at[c] + e] = rounded<Tout>(v[c][e] * inv);
                 }
             }
         }

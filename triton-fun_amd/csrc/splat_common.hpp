@@ -91,6 +91,16 @@ __device__ __forceinline__ void mma16(f32x4v& acc, const Frag<f16>& a, const Fra
 // Row (within a 32-row tile) held by accumulator register j of lane group g.
 __device__ __forceinline__ constexpr int acc_row(int j, int g) { return 8 * (j >> 2) + 4 * g + (j & 3); }
 
+// x, which is the result of a product, as T: rounded to float32 first.  Left to itself the compiler multiplies and rounds to float16 in one instruction
+// in some places and not in others (v_fma_mixlo_f16), and the same value has different bits in two kernels.
+template <typename T>
+__device__ __forceinline__ T rounded(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (std::is_same_v<T, f16>) asm("" : "+v"(x));
+#endif
+    return (T)x;
+}
+
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // Store a float as element `idx` of a buffer whose element type is chosen at run time.
