@@ -213,14 +213,15 @@ int splat_spmm_planned(const void* p, const void* v, int64_t v_sb, int64_t v_sh,
  * one 16-bit dtype (scores, probs [B,H,L,T] and out [B,H,L,d] contiguous, of that dtype; scores and probs not overlapping; n_keys rows of v).
  * Scores and probabilities are those of the separate calls bit for bit and stay in the workgroup from one product to the next, so that nothing
  * reads the compressed matrices.  SPLAT_E_UNSUPPORTED, with nothing launched and no error message, where the separate calls are faster
- * (several segments of more than 64 slots together, many workgroups of rows of more than 256) and for what the kernel does not take:
+ * (several segments of more than 256 slots together, in many launches) and for what the kernel does not take:
  * float32, d not a multiple of 8 or above 128, T above 512, rows that are not whole 16-byte pieces (q, v, out, and kT unless its keys
- * are contiguous).  Replaces r_attention.py:77-100 (rsddmm_launcher, rsoftmax_launcher, rspmm_launcher). */
+ * are contiguous).  one_step: whether splat_attention_plan_report gave 0 in [3] for every block; the kernel takes no others (with a wrong
+ * answer it gives wrong results, but makes no access outside the buffers).  Replaces r_attention.py:77-100 (rsddmm_launcher, rsoftmax_launcher, rspmm_launcher). */
 int splat_operators(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* kT, int64_t k_sb, int64_t k_sh,
                     int64_t k_sd, int64_t k_sl, const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sl, void* scores,
                     void* probs, void* out, const splat_acsr_seg* segs /* host */, int32_t n_seg, int32_t B, int32_t H,
                     int32_t L, int32_t n_keys, int32_t d, int32_t T, float scale, int32_t dtype, const void* plan,
-                    int64_t plan_bytes, void* stream);
+                    int64_t plan_bytes, int32_t one_step, void* stream);
 
 /* Fused forward: out = softmax_over_live_columns(scale * q.kT) . v with online softmax; the
  * compressed score matrix is never written to memory.  Equals the composition
@@ -249,7 +250,8 @@ int splat_attention_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl,
  *   can read, 16-byte aligned; as many blocks as plan_bytes / (2*133*16*n_seg)), complete once the stream has been waited
  *   for: [0] whether some live row starts off a multiple of 8 positions of the block's walk (0 in every block: masks of large
  *   blocks, for which splat_spmm beats splat_spmm_planned), [1] tiles of 64 positions that the block walks, [2] its
- *   live positions, [3] 0.
+ *   live positions, [3] whether some segment's rows in the block differ in their column step or phase (positions of the walk are
+ *   dense columns then, not slots).
  * splat_attention_fwd_planned: as splat_attention_fwd, with the plan of the same segments and L; results
  *   are bit-identical to splat_attention_fwd.  A plan built from other segments or another L gives
  *   undefined results (only its size is checked). */

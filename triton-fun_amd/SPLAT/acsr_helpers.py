@@ -528,6 +528,11 @@ class ACSRSegments:
         entry = self._plan_entry(L, device)
         return entry[2] if entry is not None and len(entry) > 2 else 0
 
+    def one_step(self, L: int, device) -> bool:
+        """Whether no row block of the plan holds rows that differ in column step or phase; False without a plan."""
+        entry = self._plan_entry(L, device)
+        return entry is not None and len(entry) > 3 and entry[3]
+
     def native(self, L: int, device, with_plan: bool):
         """The segments as the native host path takes them (``_splat_hip.host().mask``), with the plan table or without, built
         on first use and kept where ``plan`` keeps its tables; None under stream capture when it would have to be built
@@ -548,7 +553,8 @@ class ACSRSegments:
             arr = self.seg_array(L)
             own = [t for seg in self.seg_args() for t in seg[:6] if t is not None and t is not holder]
             mask = kept[key] = _hip.host().mask(ctypes.addressof(arr), len(self), L, self.plan(L, device) if with_plan else None,
-                                                self.live_percent(L, device) if with_plan else 0, self.max_step, tuple(own))
+                                                self.live_percent(L, device) if with_plan else 0,
+                                                with_plan and self.one_step(L, device), self.max_step, tuple(own))
         return mask
 
     def seg_args(self) -> list[tuple]:

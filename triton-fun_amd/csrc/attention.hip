@@ -594,9 +594,9 @@ __global__ __launch_bounds__(256) void attn_plan_kernel(const PlanParams p) {
     if (p.report != nullptr && variant == 0) {
         __syncthreads();
         if (tid == 0) {
-            int tiles = 0;
-            for (int sg = 0; sg < n_seg; ++sg) tiles += s_plan[sg].n_tiles;
-            p.report[rb] = make_int4(s_misaligned, tiles, s_live, 0);
+            int tiles = 0, stepping = 0;
+            for (int sg = 0; sg < n_seg; ++sg) tiles += s_plan[sg].n_tiles, stepping |= s_plan[sg].uniform == 0;
+            p.report[rb] = make_int4(s_misaligned, tiles, s_live, stepping);
         }
     }
 }

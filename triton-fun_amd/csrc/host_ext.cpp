@@ -96,6 +96,7 @@ struct Mask : torch::CustomClassHolder {
     int n_seg = 0;
     int64_t rows = 0;
     int max_step = 1;
+    bool one_step = false;         // the plan's blocks walk slots (splat_operators)
     at::Tensor plan;               // may be undefined
     int live_percent = 0;          // of the positions that the plan walks, 0: unknown
     std::vector<at::Tensor> keep;  // the arrays that `segs` points into
@@ -173,20 +174,20 @@ at::Tensor transposed_keys(const at::Tensor& kT, int* rc) {
     return k;
 }
 
-// mask(arr_address, n_seg, rows, plan | None, live_percent, max_step, (tensors...)) -> capsule
+// mask(arr_address, n_seg, rows, plan | None, live_percent, one_step, max_step, (tensors...)) -> capsule
 PyObject* py_mask(PyObject*, PyObject* args) {
     unsigned long long addr;
-    int n_seg, live, max_step;
+    int n_seg, live, one_step, max_step;
     long long rows;
     PyObject *plan, *tensors;
-    if (!PyArg_ParseTuple(args, "KiLOiiO!", &addr, &n_seg, &rows, &plan, &live, &max_step, &PyTuple_Type, &tensors)) return nullptr;
+    if (!PyArg_ParseTuple(args, "KiLOipiO!", &addr, &n_seg, &rows, &plan, &live, &one_step, &max_step, &PyTuple_Type, &tensors)) return nullptr;
     if (n_seg < 1 || n_seg > SPLAT_MAX_SEGMENTS) {
         PyErr_SetString(PyExc_ValueError, "number of segments");
         return nullptr;
     }
     auto m = c10::make_intrusive<Mask>();
     std::memcpy(m->segs, reinterpret_cast<const void*>(static_cast<uintptr_t>(addr)), n_seg * sizeof(splat_acsr_seg));
-    m->n_seg = n_seg, m->rows = rows, m->live_percent = live, m->max_step = max_step;
+    m->n_seg = n_seg, m->rows = rows, m->live_percent = live, m->one_step = one_step != 0, m->max_step = max_step;
     for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(tensors); ++i) {
         PyObject* o = PyTuple_GET_ITEM(tensors, i);
         if (!THPVariable_Check(o)) continue;
@@ -594,16 +595,23 @@ PyObject* py_operators(PyObject*, PyObject* const* a, Py_ssize_t n) {
         if (scale == -1.0 && PyErr_Occurred()) return nullptr;
         const bool both = second.x->scalar_type() == second.out->scalar_type() && second.x->data_ptr() != second.out->data_ptr();
         const char* what;
-        // One launch, where the kernel takes it.  (K along the keys is turned on its way there, one key a lane: not where neighbouring lanes' keys lie
-        // in different lines.)
+        // One launch, where the kernel takes it.  (K along the keys is turned on its way there, one key a lane; where neighbouring lanes' keys lie in
+        // different lines, it is turned before.)
+        at::Tensor turned;
         const Mask& planned = m[0]->plan.defined() ? *m[0] : *m[2];
-        if (both && planned.plan.defined() && first.y->size(3) == third.y->size(2) && third.x->data_ptr() == second.out->data_ptr() &&
-            third.out->scalar_type() == q->scalar_type() && !(first.turn && planned.max_step > 4)) {
+        if (both && planned.plan.defined() && planned.one_step && first.y->size(3) == third.y->size(2) && third.x->data_ptr() == second.out->data_ptr() &&
+            third.out->scalar_type() == q->scalar_type()) {
+            if (first.turn && planned.max_step > 4) {
+                int rc = 0;
+                turned = transposed_keys(*first.y, &rc).transpose(2, 3);
+                if (rc) return raise_rc("splat_transpose_keys", rc);
+                first.y = &turned, first.turn = false;
+            }
             const at::Tensor &k = *first.y, &v = *third.y, &s = *first.out;
             const int rc = api.operators(q->data_ptr(), q->stride(0), q->stride(1), q->stride(2), k.data_ptr(), k.stride(0), k.stride(1), k.stride(2), k.stride(3),
                                          v.data_ptr(), v.stride(0), v.stride(1), v.stride(2), s.data_ptr(), second.out->data_ptr(), out->data_ptr(),
                                          planned.segs, planned.n_seg, q->size(0), q->size(1), q->size(2), k.size(3), q->size(3), s.size(3), (float)scale,
-                                         dtype_code(q->scalar_type()), planned.plan_ptr(), planned.plan_bytes(), stream_of(*q));
+                                         dtype_code(q->scalar_type()), planned.plan_ptr(), planned.plan_bytes(), planned.one_step, stream_of(*q));
             if (rc == 0) Py_RETURN_TRUE;
             if (rc != SPLAT_E_UNSUPPORTED) return raise_rc("splat_operators", rc);
         }
@@ -678,7 +686,7 @@ bool wait_for(const c10::hip::HIPStream& stream, at::Tensor& shares) {
 }
 
 // plan(arr_address, n_seg, L, table) -> (whether every live row starts on a multiple of 8 positions of its block's walk, how much of what
-// the blocks walk is live, in percent).  Fills the plan table on the current device and waits for it, so that launches on any stream
+// the blocks walk is live, in percent, whether all walk slots: no block's rows differ in step or phase).  Fills the plan table on the current device and waits for it, so that launches on any stream
 // may use it.
 PyObject* py_plan(PyObject*, PyObject* args) {
     unsigned long long addr;
@@ -696,12 +704,12 @@ PyObject* py_plan(PyObject*, PyObject* args) {
         const int rc = api.plan_report(segs, n_seg, L, table.data_ptr(), bytes, shares.data_ptr<int32_t>(), shares.nbytes(), stream.stream());
         if (rc) return refused("splat_attention_plan_report", rc, shares);
         if (!wait_for(stream, shares)) return nullptr;
-        bool aligned = true;
+        bool aligned = true, one_step = true;
         int64_t walked = 0, live = 0;
-        for (int64_t b = 0; b < blocks; ++b) aligned = aligned && sh[4 * b] == 0, walked += sh[4 * b + 1] * int64_t(64 * 128), live += sh[4 * b + 2];
+        for (int64_t b = 0; b < blocks; ++b) aligned = aligned && sh[4 * b] == 0, one_step = one_step && sh[4 * b + 3] == 0, walked += sh[4 * b + 1] * int64_t(64 * 128), live += sh[4 * b + 2];
         share_buffers()->give(std::move(shares));
         const long percent = walked > 0 ? (long)std::clamp<int64_t>((100 * live + walked - 1) / walked, 1, 100) : 1;
-        return Py_BuildValue("Nl", PyBool_FromLong(aligned), percent);
+        return Py_BuildValue("NlN", PyBool_FromLong(aligned), percent, PyBool_FromLong(one_step));
     } catch (...) {
         return raise_current();
     }
