@@ -5,11 +5,15 @@
 // three launches (or two, where the sampled product's wavefronts take the softmax) scores are read once and probabilities twice; here a workgroup
 // keeps its rows in LDS from the first product to the last.  bfloat16, causal masks, the separate launches -> this kernel, us: 128 heads of 2048 rows,
 // d = 64, 64 slots 58 -> 36, 128 78 -> 49, 256 148 -> 80, 512 224 -> 146; d = 128, 256 slots 195 -> 109, 512 274 -> 230; 8 heads of 2048, d = 64, 48 slots 11.8 -> 7.8,
-// 512 35.3 -> 18.0; float16, 16 heads of 2000, 129 slots, d = 80 20.2 -> 15.4; 64 heads of 8192, 512 slots with step 2, d = 128 551 -> 495.
+// 512 35.3 -> 18.0; float16, 16 heads of 2000, 129 slots, d = 80 20.2 -> 15.4; 64 heads of 8192, 512 slots with step 2, d = 128 551 -> 466.
 // (A first version had the general case of every place, rows whose steps differ among them, beside the common one: 300 vector and 200 scalar
 // instructions for 8 slots of a lane, 128 registers and spills, 1.1 to 1.4 times the time.)
 //
 // A workgroup is 64 rows of one (batch, head) in two halves of 32, four wavefronts or eight.
+//   Q: whole rows, once a workgroup, into the place of the scores and from there into every wavefront's operands.  Loaded straight into operands, by
+//     every wavefront for itself and 64 bytes of 16 rows an instruction, it takes more of the address path than K: 64 heads of 8192, 512 slots with step 2, d = 128
+//     495 -> 466 us, 128 heads of 2048, 512 slots 219 -> 209; 8 heads of 2048, d = 128, 48 slots 9.9 -> 8.9, 256 slots 16.0 -> 14.8 (and 13.8 with
+//     tiles of 64 keys of V); d = 64 0 to 4 %.
 //   Scores: S^T = K Q^T by 16x16x32 matrix instructions, the wavefronts of a half take turns at subtiles of 16 positions.  K goes through registers
 //     into LDS a tile at a time, two tiles ahead, in the place of V's tiles, which is free until then; or from memory straight into the operands'
 //     registers (kDirect): no barrier, but 16 lines a request and each of them twice.  That is faster for rows of up to 64 slots where eight
@@ -42,7 +46,7 @@ enum { kDirect, kStaged, kAlongKeys };
 // PS: slots that a row of LDS has room for; NW: wavefronts
 template <int D, int PS, int NW>
 struct Ops16Geom {
-    static constexpr int VK = NW == 8 && D == 64 ? 64 : 32;      // keys of a tile of V
+    static constexpr int VK = NW == 8 && (D == 64 || PS <= 256) ? 64 : 32;  // keys of a tile of V (launches of eight wavefronts have LDS for it)
     static constexpr int STAGES = PS == 256 && D == 128 && NW == 4 ? 1 : 2;  // (one: four workgroups a CU)
     static constexpr int ROWB = D * 2, V_STAGE = VK * ROWB, P_ROWB = PS * 2;
     static constexpr int V_AT = kHalfRows * P_ROWB, LDS_BYTES = V_AT + STAGES * V_STAGE;
@@ -132,15 +136,14 @@ __global__ __launch_bounds__(NW * 64, 4) void operators16_kernel(const Operators
     const PlanRec* const pt = p.plan;
     const u32x4 zero = {0u, 0u, 0u, 0u};
 
-    Frag<T> q[2][KS];  // B operands: rows 32 pr + 16 cb + li
+    // Q: whole rows into LDS, where the scores will be, and from there into the B operands; a thread's pieces are requested before anything else
+    constexpr int NQ = kHalfRows * CPR / NT;
+    u32x4 q_raw[NQ];
 #pragma unroll
-    for (int cb = 0; cb < 2; ++cb) {
-        const T* const qr = (const T*)p.q + b * p.q_sb + h * p.q_sh + (int64_t)min(r0 + rs * (32 * pr + 16 * cb + li), L - 1) * p.q_sl;
-#pragma unroll
-        for (int t = 0; t < KS; ++t) {
-            q[cb][t].v = __builtin_bit_cast(typename Frag<T>::vec, zero);
-            if (32 * t + 8 * g < d) q[cb][t] = global_frag<T>(qr + 32 * t + 8 * g);
-        }
+    for (int i = 0; i < NQ; ++i) {
+        const int f = tid + NT * i, row = f / CPR, c = f % CPR;
+        q_raw[i] = zero;
+        if (8 * c < d) q_raw[i] = *reinterpret_cast<const u32x4*>((const T*)p.q + b * p.q_sb + h * p.q_sh + (int64_t)min(r0 + rs * row, L - 1) * p.q_sl + 8 * c);
     }
 
     // ---- a segment: its walk, and where the 32 rows lie in it ----
@@ -224,6 +227,19 @@ __global__ __launch_bounds__(NW * 64, 4) void operators16_kernel(const Operators
             }
         }
     };
+    Frag<T> q[2][KS];  // B operands: rows 32 pr + 16 cb + li
+    auto q_through_lds = [&]() {
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) *reinterpret_cast<u32x4*>(smem + lds_off<ROWB, true>((tid + NT * i) / CPR, (tid + NT * i) % CPR * 16)) = q_raw[i];
+        lds_barrier();
+#pragma unroll
+        for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+            for (int t = 0; t < KS; ++t)
+                q[cb][t].v = __builtin_bit_cast(typename Frag<T>::vec, *reinterpret_cast<const u32x4*>(smem + lds_off<ROWB, true>(32 * pr + 16 * cb + li, (4 * t + g) * 16)));
+        // (tiles of K lie behind the scores' place, and scores come after a tile's barrier)
+        if constexpr (KEYS == kDirect || PS < D) lds_barrier();
+    };
     auto products = [&](const Frag<T>(&k)[KS], f32x4(&acc)[2]) {
         acc[0] = acc[1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -268,6 +284,7 @@ __global__ __launch_bounds__(NW * 64, 4) void operators16_kernel(const Operators
             advance(k_keys, ahead);
             if (more(ahead)) load_tile(ahead, rb_);
         }
+        q_through_lds();
         auto tile = [&](int stage, u32x4(&raw)[NP]) {
             if (MULTI && cur.sg != s.sg) s = enter(cur.sg);
 #pragma unroll
@@ -296,6 +313,7 @@ __global__ __launch_bounds__(NW * 64, 4) void operators16_kernel(const Operators
             if (more(cur)) tile(G::K_STAGES == 1 ? 0 : G::K_STAGE, rb_);
         }
     } else {
+        q_through_lds();
         for (int sg = 0; sg < n_seg; ++sg) {
             if (MULTI && sg != s.sg) s = enter(sg);
             auto load_k = [&](int u, Frag<T>(&k)[KS]) {
