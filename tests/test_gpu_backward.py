@@ -257,6 +257,35 @@ def test_fused_backward_at_config_3_by_comparison_of_the_two_walks(dev):
         assert float((diff / b_[:, :, listed].float().abs().clamp(min=1.0)).max()) <= 2 * torch.finfo(dtype).eps, nm
 
 
+@pytest.mark.parametrize("B,H,L,d,listed", [(1, 1, 832, 64, False), (1, 2, 960, 64, True), (1, 130, 512, 64, True), (1, 1, 560, 128, False), (1, 2, 641, 128, True)])
+def test_float32_lists_sparse_rows_from_shorter_columns_on(dev, B, H, L, d, listed):
+    """The rule for float32 passes on both sides of its line (tiles of the longest column, rounds, head dimension), and the
+    gradients of the way that it takes, through autograd: no further from float64 than the plain walk's by more than a quarter
+    (sums in another order), and within the tolerance of the type."""
+    from r_attention import attention_with_grad
+    from r_backward import keys_side_schedule
+    local, stride, scale = 24, 32, d ** -0.5
+    g = torch.Generator(device=dev).manual_seed(L + d)
+    q, k, v, go = (torch.randn(B, H, L, d, generator=g, device=dev) for _ in range(4))
+    attn = RegularAttention(B, L, H, d, A.strided_patterns(L, local, stride), 16, 16, dev, torch.float32, scale=scale)
+    for t in (q, k, v):
+        t.requires_grad_(True)
+    got = torch.autograd.grad(attention_with_grad(q, k, v, attn), (q, k, v), go)
+    assert (keys_side_schedule(attn._segments_t, L, dev, B * H, f32_d=d) is not None) == listed
+    x = [q.detach(), k.detach().transpose(2, 3), v.detach()]
+    out, lse = (t.clone() for t in attn.forward_with_stats(x))
+    plain = attn.backward_pass(x, go, lse, out, sparse_rows=False)
+    i = torch.arange(L, device=dev)
+    live = (i[None] <= i[:, None]) & ((i[None] > i[:, None] - local) | (i[None] % stride == stride - 1))
+    few = slice(0, 2)
+    q8, k8, v8 = (t.detach()[:, few].double().requires_grad_() for t in (q, k, v))
+    p8 = torch.softmax((q8 @ k8.transpose(2, 3).contiguous() * scale).masked_fill(~live, float("-inf")), -1)
+    want = torch.autograd.grad(p8 @ v8, (q8, k8, v8), go[:, few].double())
+    for nm, a, b_, w in zip(("dq", "dk", "dv"), got, plain, want):
+        err = [float((t[:, few].double() - w).norm() / w.norm()) for t in (a, b_)]
+        assert err[0] <= 1.25 * err[1] and err[0] <= 1e-5, (nm, err)
+
+
 def test_keys_entry_point_checks_its_arguments(dev):
     import _splat_hip as hip
     L, d, B, H = 256, 64, 1, 1

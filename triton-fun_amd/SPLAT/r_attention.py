@@ -326,7 +326,7 @@ class RegularAttention(nn.Module):
                     return None  # (raised again by the backward that needs it)
                 self._ensure_plan()
                 dev = self._device
-                sched = keys_side_schedule(self._segments_t, L, dev, B * H)
+                sched = keys_side_schedule(self._segments_t, L, dev, B * H, f32_d=d if self._out_dtype == torch.float32 else None)
                 keys = sched.main if sched is not None else self._segments_t
                 self._native_grad = _hip.host().grad_state(
                     self._native, keys.native(L, dev, True),

@@ -222,15 +222,22 @@ _SPARSE_ROWS_ONE_IN = 16
 # workgroups the listed rows are spread over (stretches x blocks of 128 listed rows x batch x heads): about two per slot
 _WORKGROUPS_WANTED = 512
 # the extra launch, the sum over the stretches and the scatter cost about 30 us: taken when the longest column's walk
-# (tiles of 64 queries, times the rounds in which the part runs the blocks of 128 keys) is longer than this many tiles
+# (tiles of 64 queries, times the rounds in which the part runs the blocks of 128 keys) is longer than this many tiles (16-bit types)
 _WORTH_TILES = 40
+# The same for float32 and a head dimension: a tile costs more there (products of split operands, or float32 instructions), shares are kept and added in
+# float32, and the workgroups that a long column holds up are of 64 keys.  Strided masks, a training step without and with it, us, d = 64: one head
+# of 777 rows (12 tiles) 74 -> 76, of 1024 (16) 87 -> 75, 8 heads of 1024 (14) 94 -> 77, 4 of 1500 122 -> 77, 16 of 2048 181 -> 102, 8 of 3000
+# 234 -> 103, 128 of 512 (8, two rounds) 158 -> 116; d = 128: 8 heads of 777 (10) 163 -> 132, 1024 216 -> 155, 2 of 2048 359 -> 141.  Below the line the
+# kernels of 32 heads of 512 (8) take 54 -> 58 at d = 64 and 114 -> 120 at d = 128.  Against float64, dk and dv of the listed way are closer
+# (8 heads of 1024, d = 64: 4.1e-7 and 3.8e-7 -> 3.9e-7 and 3.6e-7).
+_WORTH_TILES_F32 = {64: 14, 128: 9}
 
 
 def keys_side_schedule(segments_t: ACSRSegments, L: int, device, batch_heads: int,
-                       always: bool = False) -> KeysSideSchedule | None:
+                       always: bool = False, f32_d: int | None = None) -> KeysSideSchedule | None:
     """The ``KeysSideSchedule`` of a transposed mask, or None when no segment of it is row-sparse (or all are, or a
     sparse one lacks its rows' first columns, or two of them keep the same key), or when the walk it replaces is too short for the extra launch to pay
-    (unless ``always``).  A block of 128 consecutive keys of a strided pattern's far field holds
+    (unless ``always``; ``f32_d`` is the head dimension of a float32 pass, None of 16-bit types).  A block of 128 consecutive keys of a strided pattern's far field holds
     one live key with up to L queries: its workgroup walks up to L / 64 tiles for one row in 128, and the pass takes 5 x
     what the rest of the mask needs.  Listed row by row and cut into stretches of queries, the same entries fill a few
     workgroups each.  Built once per (L, device, number of stretches) and kept with ``segments_t`` (a host
@@ -263,8 +270,8 @@ def keys_side_schedule(segments_t: ACSRSegments, L: int, device, batch_heads: in
     if facts is False:
         return None
     sparse, first, step, cnt, key, p_min, p_max, longest_tiles = facts
-    rounds = -(-batch_heads * -(-L // 128) // 512)
-    if not always and longest_tiles * rounds < _WORTH_TILES:
+    rounds = -(-batch_heads * -(-L // (64 if f32_d else 128)) // 512)
+    if not always and longest_tiles * rounds < (_WORTH_TILES_F32[f32_d] if f32_d else _WORTH_TILES):
         return None
     n_keys = key.numel()
     per_stretch = -(-n_keys // 128) * 128
@@ -340,7 +347,8 @@ def attention_backward_fused(q: torch.Tensor, kT: torch.Tensor, v: torch.Tensor,
     delta = torch.empty((B, H, L), dtype=torch.float32, device=dev)
     dq = torch.empty((B, H, L, d), dtype=dt, device=dev)
     dk, dv = (torch.empty((B, H, L, d), dtype=dt, device=dev) for _ in range(2))
-    sched = None if sparse_rows is False else keys_side_schedule(segments_t, L, dev, B * H, always=bool(sparse_rows))
+    sched = None if sparse_rows is False else keys_side_schedule(segments_t, L, dev, B * H, always=bool(sparse_rows),
+                                                                  f32_d=d if f32 else None)
     if sched is not None:  # the row-sparse segments of the transposed mask go row by row, after the others
         segments_t, plan_t = sched.main, sched.main.plan(L, dev)
     arr = segments.seg_array(L)
