@@ -219,18 +219,21 @@ class KeysSideSchedule:
 
 # a segment of the transposed mask is listed row by row when at most one row in this many is live
 _SPARSE_ROWS_ONE_IN = 16
-# workgroups the listed rows are spread over (stretches x blocks of 128 listed rows x batch x heads): about two per slot
-_WORKGROUPS_WANTED = 512
+# workgroups the listed rows are spread over (stretches x blocks of 128 listed rows x batch x heads), and the shortest stretch in queries.
+# 16-bit types: about two workgroups per slot.  float32, the whole backward of strided masks with stretches of at least 512 / 256 / 128 / 64 queries, us: d = 64, one
+# head of 777 rows 51 / 44 / 37 / 34, 16 heads of 2048 86 / 72 / 70 / 78, 4 of 8192 94 / 81 / 82 / 95; d = 128, one of 1024 134 / 108 / 90 / 83, 8 of 2048
+# 136 / 100 / 86 / 90, 4 of 8192 205 / 168 / 170 / 188; and with 512 workgroups instead of 256, d = 128, 32 heads of 4096 528 -> 539, 128 of 1024 463 -> 479.
+_WORKGROUPS_WANTED, _WORKGROUPS_WANTED_F32 = 512, 256
+_STRETCH, _STRETCH_F32 = 512, 128
 # the extra launch, the sum over the stretches and the scatter cost about 30 us: taken when the longest column's walk
 # (tiles of 64 queries, times the rounds in which the part runs the blocks of 128 keys) is longer than this many tiles (16-bit types)
 _WORTH_TILES = 40
 # The same for float32 and a head dimension: a tile costs more there (products of split operands, or float32 instructions), shares are kept and added in
-# float32, and the workgroups that a long column holds up are of 64 keys.  Strided masks, a training step without and with it, us, d = 64: one head
-# of 777 rows (12 tiles) 74 -> 76, of 1024 (16) 87 -> 75, 8 heads of 1024 (14) 94 -> 77, 4 of 1500 122 -> 77, 16 of 2048 181 -> 102, 8 of 3000
-# 234 -> 103, 128 of 512 (8, two rounds) 158 -> 116; d = 128: 8 heads of 777 (10) 163 -> 132, 1024 216 -> 155, 2 of 2048 359 -> 141.  Below the line the
-# kernels of 32 heads of 512 (8) take 54 -> 58 at d = 64 and 114 -> 120 at d = 128.  Against float64, dk and dv of the listed way are closer
-# (8 heads of 1024, d = 64: 4.1e-7 and 3.8e-7 -> 3.9e-7 and 3.6e-7).
-_WORTH_TILES_F32 = {64: 14, 128: 9}
+# float32, and the workgroups that a long column holds up are of 64 keys.  Strided masks, a training step without and with it, us, d = 64: 32 heads
+# of 512 rows (8 tiles) 64 -> 71, one of 600 (9) 65 -> 73, 8 of 640 (9) 74 -> 73, 8 of 777 (10) 77 -> 72, 32 of 777 (12) 104 -> 72, 8 of 1024 (14)
+# 94 -> 74, 16 of 2048 (30) 182 -> 87; d = 128: one of 300 (5) 87 -> 74, 64 of 300 135 -> 111, 8 of 512 (8) 119 -> 74, 8 of 1024 215 -> 113.  (Steps of
+# up to 75 us are the host's.)  Against float64, dk and dv of the listed way are closer (8 heads of 1024, d = 64: 4.1e-7 and 3.9e-7 -> 3.8e-7 and 3.5e-7).
+_WORTH_TILES_F32 = {64: 10, 128: 5}
 
 
 def keys_side_schedule(segments_t: ACSRSegments, L: int, device, batch_heads: int,
@@ -275,10 +278,11 @@ def keys_side_schedule(segments_t: ACSRSegments, L: int, device, batch_heads: in
         return None
     n_keys = key.numel()
     per_stretch = -(-n_keys // 128) * 128
-    # stretches: enough workgroups to fill the part about twice, at least 8 tiles of 64 queries each
+    # stretches: enough workgroups to fill the part, none shorter than the shortest
     span = p_max - p_min + 1
-    want = max(1, round(_WORKGROUPS_WANTED / max(1, batch_heads * (per_stretch // 128))))
-    n_stretches = max(1, min(want, -(-span // 512)))
+    wanted, shortest = (_WORKGROUPS_WANTED_F32, _STRETCH_F32) if f32_d else (_WORKGROUPS_WANTED, _STRETCH)
+    want = max(1, round(wanted / max(1, batch_heads * (per_stretch // 128))))
+    n_stretches = max(1, min(want, -(-span // shortest)))
     sched = cache.get((L, dev.index, n_stretches))
     if sched is not None:
         return sched
