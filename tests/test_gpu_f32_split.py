@@ -255,3 +255,26 @@ def test_listed_rows_taken_again(dev, d):
     again = attn.backward_pass([far[0], k.transpose(2, 3), far[1]], go, sparse_rows=True)
     for a, b in zip(again, clean):
         assert float((a - b)[..., 1:].abs().max()) <= 2e-5 * float(b.abs().max())
+
+
+@pytest.mark.parametrize("large", [False, True])
+@pytest.mark.parametrize("L", [64, 130, 257])
+@pytest.mark.parametrize("masks", [lambda L: A.causal_windowed_pattern(L, 39), lambda L: A.dilated_pattern(L, 20, 3), lambda L: A.strided_patterns(L, 24, 16)],
+                         ids=["causal", "dilated", "strided"])
+def test_gradients_of_keys_in_many_workgroups_are_those_of_few(dev, masks, L, large):
+    """dK and dV at d = 64 in a launch beyond two workgroups a CU, whose kernel is another one, against the same heads in a launch of few: the same
+    operations in the same order, so the same bits; ``large``: rows that the split operands do not hold, one of them infinite."""
+    g = torch.Generator(device=dev).manual_seed(L)
+    x = [torch.randn(1, 2, L, 64, generator=g, device=dev) for _ in range(4)]
+    if large:
+        x[1][0, 0, L // 2] *= 1e30
+        x[3][0, 1, L // 3, 5] = float("inf")
+    times = 513 // (2 * ((L + 127) // 128) * 2) + 1
+    one, other = (RegularAttention(1, L, 2 * n, 64, masks(L), 16, 16, dev, torch.float32, scale=0.125) for n in (1, times))
+    out, lse = (t.clone() for t in one.forward_with_stats([x[0], x[1].transpose(2, 3), x[2]]))
+    few = one.backward_pass([x[0], x[1].transpose(2, 3), x[2]], x[3], lse, out)
+    q, k, v, go, out = (t.repeat(1, times, 1, 1) for t in (*x, out))
+    many = other.backward_pass([q, k.transpose(2, 3), v], go, lse.repeat(1, times, 1), out)
+    for nm, a, b in zip(("dq", "dk", "dv"), few, many):
+        assert large or bool(torch.isfinite(a).all()), nm
+        assert torch.equal(torch.nan_to_num(a.repeat(1, times, 1, 1), nan=7e37), torch.nan_to_num(b, nan=7e37)), nm

@@ -8,7 +8,7 @@
 // barriers.  A and B are split once and stay in registers.  dK + dV at d = 128 does not fit them and is a kernel of its own
 // (attention_bwd_f32_keys.hip).
 // Measured against the kernel on the float32 instructions, us: 64 heads of 2048 rows, d = 64, window 256: dQ 140 -> 97, dK + dV 181 ->
-// 135; 128 heads, window 32: 99 -> 81 and 116 -> 107; 32 heads, d = 128, window 256 / 32: dQ 142 -> 110 and 59 -> 51; one head, window 32,
+// 135; 128 heads, window 32: 99 -> 81 and 116 -> 104; 32 heads, d = 128, window 256 / 32: dQ 142 -> 110 and 59 -> 51; one head, window 32,
 // d = 64: 11.0 -> 9.7 and 10.8 -> 9.6.  Two workgroups of dQ a CU instead of three at d = 64: 110.  Relative error of dq, dk, dv
 // against float64 (norms), window 257: 5.1e-7, 5.1e-7, 4.9e-7 -> 4.3e-7, 4.3e-7, 4.2e-7.
 #include "attn_bwd.hpp"
@@ -17,14 +17,15 @@
 
 namespace splat {
 
-template <int D, bool KEYS>
-__global__ __launch_bounds__(256, D == 64 && !KEYS ? 3 : 2) void attn_bwd_f32_kernel(const BwdParams p) {
+// PER_CU: workgroups a CU that registers are kept for
+template <int D, bool KEYS, int PER_CU>
+__global__ __launch_bounds__(256, PER_CU) void attn_bwd_f32_kernel(const BwdParams p) {
     constexpr int BN = 32, ROWB = 2 * D, PLANE = BN * ROWB, TILE = 3 * PLANE;  // positions a tile; bytes of a row, a plane, an operand
     constexpr int STATS = 2 * TILE;           // lse and D of the tile's positions (dK + dV)
     constexpr int KS = D / 32, DT = D / 16;
     constexpr int CPR = D / 8;                // 8-value pieces of a row
     constexpr int NP = 2 * BN * CPR / 256;    // pieces a thread: the first half of them X's, the others Y's
-    constexpr int AHEAD = D == 64 ? 2 : 1;    // parts of fragments requested ahead of their products (as many as registers are left)
+    constexpr int AHEAD = D == 64 && !(KEYS && PER_CU == 3) ? 2 : 1;  // parts of fragments requested ahead of their products (as many as registers are left)
     constexpr float kLog2e = 1.4426950408889634f;
 
     extern __shared__ __attribute__((aligned(1024))) char smem[];  // three planes of X, three of Y, the statistics
@@ -348,21 +349,27 @@ __global__ __launch_bounds__(256, D == 64 && !KEYS ? 3 : 2) void attn_bwd_f32_ke
     }
 }
 
-template <int D, bool KEYS>
+template <int D, bool KEYS, int PER_CU>
 static int launch(const BwdParams& p0, hipStream_t st) {
     begin_launch();
     BwdParams p = p0;
     p.total = p.B * p.H * 2 * p.n_row_blocks;
     p.by_blocks = divisor(2 * p.n_row_blocks), p.by_h = divisor(p.H);
     constexpr size_t lds = 6 * 32 * D * 2 + 256;
-    auto kern = attn_bwd_f32_kernel<D, KEYS>;
+    auto kern = attn_bwd_f32_kernel<D, KEYS, PER_CU>;
     static uint64_t lds_reserved = 0;
     if (int rc = reserve_dynamic_lds(&lds_reserved, reinterpret_cast<const void*>(kern), lds, "splat_attention_bwd_f32")) return rc;
     kern<<<((p.total + 7) / 8) * 8, 256, lds, st>>>(p);
     return check_launch("splat_attention_bwd_f32");
 }
 
-int launch_bwd_dq_f32(const BwdParams& dq, int d, hipStream_t st) { return d == 64 ? launch<64, false>(dq, st) : launch<128, false>(dq, st); }
-int launch_bwd_dkv_f32(const BwdParams& dkv, int d, hipStream_t st) { return d == 64 ? launch<64, true>(dkv, st) : launch_bwd_dkv_f32_d128(dkv, st); }
+int launch_bwd_dq_f32(const BwdParams& dq, int d, hipStream_t st) { return d == 64 ? launch<64, false, 3>(dq, st) : launch<128, false, 2>(dq, st); }
+int launch_bwd_dkv_f32(const BwdParams& dkv, int d, hipStream_t st) {
+    if (d != 64) return launch_bwd_dkv_f32_d128(dkv, st);
+    // Beyond two workgroups a CU, three of them of 168 registers each (28 bytes of scratch, fragments one part ahead), us, two a CU -> three: 680 workgroups, window
+    // 128 37.3 -> 33.0; 768, window 257 to both sides 60.0 -> 51.0; 1440, window 100 62.4 -> 60.7; 2048, window 256 139 -> 133 and 139; 4096, window 32 111 -> 104.
+    // Up to that the third is of no use: 512, window 128 25.1 -> 26.6; 16, window 32 9.7 -> 9.9.
+    return (int64_t)dkv.B * dkv.H * 2 * dkv.n_row_blocks > 2 * 256 ? launch<64, true, 3>(dkv, st) : launch<64, true, 2>(dkv, st);
+}
 
 }  // namespace splat
