@@ -176,3 +176,49 @@ def test_what_it_does_not_take(dev):
     L = 600
     assert code(segs=_segments(_steps_differ(L), dev)) == -5
     assert code(segs=_segments(A.causal_windowed_pattern(L, 512), dev)) == -5
+
+
+def _three_calls(segs, q, kT, v, scale, buffers, T=None):
+    """The same through splat_sddmm_planned, splat_softmax and splat_spmm_planned."""
+    heads, L, d = q.shape[1:]
+    T = T or segs.T
+    arr, plan, code, stream = segs.seg_array(L, T), segs.plan(L, q.device), hip.dtype_code(q.dtype), hip.stream_ptr(q.device)
+    table = (plan.data_ptr(), plan.numel() * plan.element_size())
+    s, p, o = buffers
+    hip.check(hip.lib().splat_sddmm_planned(q.data_ptr(), *q.stride()[:3], kT.data_ptr(), *kT.stride()[:4], s.data_ptr(), arr, len(segs), 1, heads, L, kT.shape[3],
+                                            d, T, ctypes.c_float(scale), code, code, None, *table, stream), "splat_sddmm_planned")
+    hip.check(hip.lib().splat_softmax(s.data_ptr(), p.data_ptr(), arr, len(segs), heads, L, T, code, code, stream), "splat_softmax")
+    hip.check(hip.lib().splat_spmm_planned(p.data_ptr(), v.data_ptr(), *v.stride()[:3], o.data_ptr(), arr, len(segs), 1, heads, L, v.shape[2], d, T, code, code,
+                                           *table, stream), "splat_spmm_planned")
+
+
+@pytest.mark.parametrize("layout", ["rows", "keys"])
+@pytest.mark.parametrize("heads", [2, 80])  # (eight wavefronts a workgroup and four)
+@pytest.mark.parametrize("mask,d", [("33", 64), ("200", 128), ("strided", 64)])
+def test_columns_before_the_first_stand_for_it(dev, mask, d, heads, layout):
+    """Metadata made by hand, whose first rows begin before column 0: nothing is read in front of K and V, as with the separate calls, where such columns
+    have the first one's key and value."""
+    L = 600
+    segs = _segments(MASKS[mask](L), dev)
+    T, t = segs.T, segs.tuples[0]
+    n = int(t[5])
+    first = torch.arange(L, device=dev) - (n - 1)
+    t[2].fill_(1.0), t[3].copy_(first.to(t[3].dtype)), t[4].fill_(n), segs.first_cols[0].copy_(first)
+    q, kT, v = _operands(dev, torch.bfloat16, heads, L, d, layout)
+    want, got = ([torch.full((heads, L, w), SENTINEL, dtype=torch.bfloat16, device=dev) for w in (T, T, d)] for _ in range(2))
+    hip.check(_one_launch(segs, q, kT, v, 0.2, got), "splat_operators")
+    _three_calls(segs, q, kT.transpose(2, 3).contiguous().transpose(2, 3), v, 0.2, want)
+    for a, b in zip(got[:2], want[:2]):
+        assert torch.equal(a, b) and torch.all(a[:, :, :n] != SENTINEL)
+    columns = (first[:, None] + torch.arange(n, device=dev)).clamp(min=0)
+    q8, k8, v8 = q[0, 0].double(), kT[0, 0].double(), v[0, 0].double()
+    s = (q8 @ k8).gather(1, columns) * 0.2
+    # (one rounding of a sum of d products to the type)
+    assert float((got[0][0, :, :n].double() - s).abs().max()) <= float(s.abs().max()) * torch.finfo(torch.bfloat16).eps
+    if len(segs) == 1:
+        out = (got[1][0].double()[:, :, None] * v8[columns]).sum(1)
+        err = (got[2][0].double() - out).abs()
+        assert float((err - out.abs() * torch.finfo(torch.bfloat16).eps / 2 * 1.01).max()) <= T * 6 * 2.0 ** -24
+        assert torch.equal(got[2], want[2])
+    else:
+        assert torch.allclose(got[2].float(), want[2].float(), rtol=2 * torch.finfo(torch.bfloat16).eps, atol=1e-4)

@@ -260,7 +260,7 @@ __global__ __launch_bounds__(NW * 64, 4) void operators16_kernel(const Operators
         auto load_tile = [&](const Walk& w, u32x4(&raw)[NP]) {
 #pragma unroll
             for (int i = 0; i < NP; ++i) {
-                const int key = min(w.c0 + w.cs * (w.tile * KK + pc_key[i]), p.n_keys - 1);
+                const int key = min(max(w.c0 + w.cs * (w.tile * KK + pc_key[i]), 0), p.n_keys - 1);
                 raw[i] = zero;
                 if (8 * pc_c[i] < d) {
                     if constexpr (KEYS == kAlongKeys) {
@@ -317,7 +317,7 @@ __global__ __launch_bounds__(NW * 64, 4) void operators16_kernel(const Operators
         for (int sg = 0; sg < n_seg; ++sg) {
             if (MULTI && sg != s.sg) s = enter(sg);
             auto load_k = [&](int u, Frag<T>(&k)[KS]) {
-                const int key = min(s.c0 + s.cs * (16 * u + li), p.n_keys - 1);
+                const int key = min(max(s.c0 + s.cs * (16 * u + li), 0), p.n_keys - 1);
                 const T* const src = kb + (int64_t)key * p.k_sl + 8 * g;
 #pragma unroll
                 for (int t = 0; t < KS; ++t) {
@@ -351,7 +351,7 @@ __global__ __launch_bounds__(NW * 64, 4) void operators16_kernel(const Operators
     auto load_v = [&](const Walk& w, u32x4(&reg)[NI]) {
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
-            const int key = min(w.c0 + w.cs * (w.tile * VK + v_row[i]), p.n_keys - 1);
+            const int key = min(max(w.c0 + w.cs * (w.tile * VK + v_row[i]), 0), p.n_keys - 1);
             reg[i] = *reinterpret_cast<const u32x4*>(vbytes + key * v_rowb + v_col[i]);
         }
     };
