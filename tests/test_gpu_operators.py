@@ -888,3 +888,45 @@ def test_key_transpose_16_bit_edges(dev, L, d, dtype):
         kT = wide[..., off:off + L]
         got = A.transpose_keys(kT)
         assert got.is_contiguous() and torch.equal(got.view(torch.int16), kT.transpose(2, 3).contiguous().view(torch.int16))
+
+
+@pytest.mark.parametrize("T,d,heads", [(64, 64, 80), (40, 128, 140), (120, 64, 80), (200, 128, 80), (256, 64, 700), (256, 128, 700)])
+def test_kernels_of_the_plan_end_rows_with_the_buffer(dev, T, d, heads):
+    """Rows of 400 live columns in buffers of fewer slots, where the plan knows the mask alone: the sampled product writes nothing behind a row's last
+    slot and the last product reads nothing there.  (700 heads: more than 192 MB of probabilities, whose rows go through rings.)"""
+    import ctypes
+    import _splat_hip as hip
+    L, dtype = 600, torch.bfloat16
+    segs = A.create_acsr_segments([A.causal_windowed_pattern(L, 399)], 16, dev)
+    g = torch.Generator(device=dev).manual_seed(T)
+    q, k, v = (torch.randn(1, heads, L, d, generator=g, device=dev).to(dtype) for _ in range(3))
+    kT = k.transpose(2, 3)
+    arr, plan, code, stream = segs.seg_array(L, T), segs.plan(L, dev), hip.dtype_code(dtype), hip.stream_ptr(dev)
+    table = (plan.data_ptr(), plan.numel() * plan.element_size())
+    n, behind = heads * L * T, 4096
+    scores = [torch.full((n + behind,), SENTINEL, dtype=dtype, device=dev) for _ in range(2)]
+    args = (*q.stride()[:3], kT.data_ptr(), *kT.stride()[:4])
+    sizes = (arr, 1, 1, heads, L, L, d, T, ctypes.c_float(0.2), code, code)
+    hip.check(hip.lib().splat_sddmm_planned(q.data_ptr(), *args, scores[0].data_ptr(), *sizes, None, *table, stream), "splat_sddmm_planned")
+    hip.check(hip.lib().splat_sddmm(q.data_ptr(), *args, scores[1].data_ptr(), *sizes, stream), "splat_sddmm")
+    assert torch.equal(*scores) and torch.all(scores[0][n:] == SENTINEL)
+    i = torch.arange(L, device=dev)
+    first, cnt = (i - 399).clamp(min=0), (i + 1).clamp(max=T)
+    columns = (first[:, None] + torch.arange(T, device=dev)).clamp(max=L - 1)
+    lv = torch.arange(T, device=dev) < cnt[:, None]
+    s = (q[0, -1].double() @ kT[0, -1].double()).gather(1, columns) * 0.2
+    got = scores[0][:n].view(heads, L, T)[-1].double()
+    assert float(torch.where(lv, (got - s).abs() - s.abs() * 2.0 ** -8, 0.0).max()) <= 1e-5 and torch.all(got[~lv] == SENTINEL)
+    # probabilities: a huge value where a row's last slots are followed by the next row's first
+    p = torch.rand(heads, L, T, generator=g, device=dev).to(dtype) / T
+    p[:, ::2, :8] = 1e30
+    outs = [torch.empty(heads, L, d, dtype=dtype, device=dev) for _ in range(2)]
+    sizes = (arr, 1, 1, heads, L, L, d, T, code, code)
+    hip.check(hip.lib().splat_spmm_planned(p.data_ptr(), v.data_ptr(), *v.stride()[:3], outs[0].data_ptr(), *sizes, *table, stream), "splat_spmm_planned")
+    hip.check(hip.lib().splat_spmm(p.data_ptr(), v.data_ptr(), *v.stride()[:3], outs[1].data_ptr(), *sizes, stream), "splat_spmm")
+    for h in (0, heads - 1):
+        pd = torch.where(lv, p[h].double(), 0.0)
+        want = (pd[:, :, None] * v[0, h].double()[columns]).sum(1)
+        most = (pd[:, :, None] * v[0, h].double()[columns].abs()).sum(1)
+        for o in outs:  # (a float32 sum of at most T products, one rounding to the type)
+            assert float(((o[h].double() - want).abs() - want.abs() * 2.0 ** -8 - most * T * 2.0 ** -24).max()) <= 0

@@ -44,11 +44,12 @@ def _operands(dev, dtype, heads, L, d, layout, seed=0):
     return q, kT.contiguous() if layout == "keys" else kT, v
 
 
-def _one_launch(segs, q, kT, v, scale, buffers):
+def _one_launch(segs, q, kT, v, scale, buffers, T=None):
     heads, L, d = q.shape[1:]
-    arr, plan = segs.seg_array(L, segs.T), segs.plan(L, q.device)
+    T = T or segs.T
+    arr, plan = segs.seg_array(L, T), segs.plan(L, q.device)
     return hip.lib().splat_operators(q.data_ptr(), *q.stride()[:3], kT.data_ptr(), *kT.stride()[:4], v.data_ptr(), *v.stride()[:3],
-                                     *(b.data_ptr() for b in buffers), arr, len(segs), 1, heads, L, v.shape[2], d, segs.T, ctypes.c_float(scale),
+                                     *(b.data_ptr() for b in buffers), arr, len(segs), 1, heads, L, v.shape[2], d, T, ctypes.c_float(scale),
                                      hip.dtype_code(q.dtype), plan.data_ptr(), plan.numel() * plan.element_size(), segs.one_step(L, q.device), hip.stream_ptr(q.device))
 
 
@@ -219,6 +220,25 @@ def test_columns_before_the_first_stand_for_it(dev, mask, d, heads, layout):
         out = (got[1][0].double()[:, :, None] * v8[columns]).sum(1)
         err = (got[2][0].double() - out).abs()
         assert float((err - out.abs() * torch.finfo(torch.bfloat16).eps / 2 * 1.01).max()) <= T * 6 * 2.0 ** -24
+        assert torch.equal(got[2], want[2])
+    else:
+        assert torch.allclose(got[2].float(), want[2].float(), rtol=2 * torch.finfo(torch.bfloat16).eps, atol=1e-4)
+
+
+@pytest.mark.parametrize("layout", ["rows", "keys"])
+@pytest.mark.parametrize("L,heads", [(600, 2), (600, 80)])
+@pytest.mark.parametrize("mask,T,d", [("128", 64, 64), ("128", 40, 128), ("200", 64, 80), ("512", 256, 64), ("512", 129, 128), ("dilated 77 by 3", 33, 64), ("windowed 257", 128, 64),
+                                      ("blocked 512", 200, 128), ("strided 100", 110, 64), ("strided 7", 30, 64)])
+def test_rows_longer_than_the_buffers_rows(dev, mask, T, d, L, heads, layout):
+    """Rows of more live columns than a compressed row has slots end with the last slot, in all three results, as with the separate calls."""
+    segs = _segments(MASKS[mask](L), dev)
+    assert segs.T > T
+    q, kT, v = _operands(dev, torch.bfloat16, heads, L, d, layout)
+    want, got = ([torch.full((heads * L * w + 8,), SENTINEL, dtype=torch.bfloat16, device=dev) for w in (T, T, d)] for _ in range(2))
+    hip.check(_one_launch(segs, q, kT, v, 0.2, got, T), "splat_operators")
+    _three_calls(segs, q, kT.transpose(2, 3).contiguous().transpose(2, 3), v, 0.2, want, T)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    if len(segs) == 1:
         assert torch.equal(got[2], want[2])
     else:
         assert torch.allclose(got[2].float(), want[2].float(), rtol=2 * torch.finfo(torch.bfloat16).eps, atol=1e-4)

@@ -276,6 +276,14 @@ __device__ __forceinline__ PlanRec plan_uniform_load(const PlanRec* p) {
     return *reinterpret_cast<const_plan_rec*>(reinterpret_cast<uintptr_t>(p));
 }
 
+// A span of the plan table for a buffer whose rows own `most` slots of the segment.  The table knows the mask alone: rows that are longer end after
+// those slots, and neither a tile behind them may pass for one without a mask nor may positions far behind them share a place in LDS with live ones.
+// (With room for all of them both bounds are the table's: no row ends further than `most` positions behind the first or the last of their beginnings.)
+__device__ __forceinline__ WaveSpan planned_span(const PlanRec& r, int most) {
+    most = min(most, 0x3fffffff);
+    return WaveSpan{r[0], r[1], min(r[2], r[0] + most), min(r[3], r[1] + most)};
+}
+
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
 // Transposing LDS read: the 16 lanes of a block address 4 rows x 16 columns of 16-bit elements (lane s:

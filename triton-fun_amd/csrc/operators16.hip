@@ -163,9 +163,9 @@ __global__ __launch_bounds__(NW * 64, 4) void operators16_kernel(const Operators
         const PlanRec s0 = plan_uniform_load(pt + plan_span_at(n_rb, n_seg, rb, sg, 2 * half)), s1 = plan_uniform_load(pt + plan_span_at(n_rb, n_seg, rb, sg, 2 * half + 1));
         const PlanRec sp = pr ? s1 : s0;
         s.sg = sg, s.c0 = r[0], s.cs = r[1];
-        s.span = WaveSpan{sp[0], sp[1], sp[2], sp[3]};
+        s.span = planned_span(sp, p.seg[sg].max_cnt);
         s.first = max(min(s0[0], s1[0]), 0), s.end = min(max(max(s0[3], s1[3]), 0), r[2] * kBN);
-        s.apart = ((max(sp[3], 0) + 31) & ~31) - (sp[0] & ~31) <= PS;
+        s.apart = ((max(s.span.hi_max, 0) + 31) & ~31) - (sp[0] & ~31) <= PS;
 #pragma unroll
         for (int cb = 0; cb < 2; ++cb) {
             const PlanRec w = row_rec(sg, 32 * pr + 16 * cb + li);

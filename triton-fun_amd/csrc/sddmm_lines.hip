@@ -186,7 +186,7 @@ __global__ __launch_bounds__(BM_ * 4, 4) void sddmm_lines_kernel(const SddmmPara
         if constexpr (PLANNED) {
             // the table holds the spans of 32 rows: wider than this wavefront's 16, which only makes the tests below pass less often
             const PlanRec r = plan_uniform_load(pt + plan_span_at(n_rb, p.n_seg, rb, sg, wave >> 1));
-            span = WaveSpan{r[0], r[1], r[2], r[3]};
+            span = planned_span(r, p.seg[sg].max_cnt);
         } else {
             span = wave_span(mine, uniform);
         }

@@ -127,7 +127,7 @@ __global__ __launch_bounds__(512, 4) void spmm_thin_kernel(const SpmmParams p) {
         {
             // the table holds the spans of 32 rows: wider than this wavefront's 16, which only makes the tests below pass less often
             const PlanRec r = plan_uniform_load(pt + plan_span_at(n_rb, p.n_seg, rb, sg, wave >> 1));
-            span = WaveSpan{r[0], r[1], r[2], r[3]};
+            span = planned_span(r, p.seg[sg].max_cnt);
         }
         const int lmin = span.lo_min, hmax = span.hi_max;
         const T* const prow = pb + (int64_t)min(my_r, L - 1) * p.T + off;
