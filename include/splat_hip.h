@@ -213,7 +213,8 @@ int splat_spmm_planned(const void* p, const void* v, int64_t v_sb, int64_t v_sh,
  * one 16-bit dtype (scores, probs [B,H,L,T] and out [B,H,L,d] contiguous, of that dtype; scores and probs not overlapping; n_keys rows of v).
  * Scores and probabilities are those of the separate calls bit for bit and stay in the workgroup from one product to the next, so that nothing
  * reads the compressed matrices.  SPLAT_E_UNSUPPORTED, with nothing launched and no error message, where the separate calls are faster
- * (several segments of more than 256 slots together, in many launches) and for what the kernel does not take:
+ * (several segments of more than 256 slots together, in many launches), where scores, probs or out share memory with another of them or with an
+ * operand (the separate calls are ordered, the workgroups of one launch are not) and for what the kernel does not take:
  * float32, d not a multiple of 8 or above 128, T above 512, rows that are not whole 16-byte pieces (q, v, out, and kT unless its keys
  * are contiguous).  one_step: whether splat_attention_plan_report gave 0 in [3] for every block; the kernel takes no others (with a wrong
  * answer it gives wrong results, but makes no access outside the buffers).  Replaces r_attention.py:77-100 (rsddmm_launcher, rsoftmax_launcher, rspmm_launcher). */

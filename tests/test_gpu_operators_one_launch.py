@@ -242,3 +242,50 @@ def test_rows_longer_than_the_buffers_rows(dev, mask, T, d, L, heads, layout):
         assert torch.equal(got[2], want[2])
     else:
         assert torch.allclose(got[2].float(), want[2].float(), rtol=2 * torch.finfo(torch.bfloat16).eps, atol=1e-4)
+
+
+def test_results_that_share_memory_with_operands_are_left_to_the_separate_calls(dev):
+    """No launch in which one workgroup stores what another still reads: results over an operand, from its first byte to its last one, over each other, or
+    over rows between an operand's; neighbours in memory are taken."""
+    heads, L, d, dtype = 2, 256, 64, torch.bfloat16
+    segs = _segments(A.causal_windowed_pattern(L, d - 1), dev)
+    n = heads * L * d
+    assert segs.T == d  # (so that all six have one size)
+    for operand in range(3):
+        for result in range(3):
+            for shift, taken in ((0, False), (8, False), (-8, False), (n - 8, False), (8 - n, False), (n, True), (-n, True)):
+                pool = torch.full((10 * n,), SENTINEL, dtype=dtype, device=dev)
+                at = 3 * n + operand * n  # the operand is where it is, the result around it, the others further on
+                ops = [pool[at:at + n] if i == operand else torch.randn(n, device=dev).to(dtype) for i in range(3)]
+                ops[operand].copy_(torch.randn(n, device=dev))
+                bufs = [pool[at + shift:at + shift + n] if i == result else torch.empty(n, dtype=dtype, device=dev) for i in range(3)]
+                q, k, v = (t.view(1, heads, L, d) for t in ops)
+                rc = _one_launch(segs, q, k.transpose(2, 3), v, 0.2, bufs)
+                assert rc == (0 if taken else -5), (operand, result, shift)
+    pool = torch.randn(8 * n, device=dev).to(dtype)
+    q, k, v, s, p, o = (pool[i * n:(i + 1) * n] for i in range(6))
+    x = (q.view(1, heads, L, d), k.view(1, heads, L, d).transpose(2, 3), v.view(1, heads, L, d))
+    assert _one_launch(segs, *x, 0.2, [s, p, o]) == 0
+    for bufs in ([s, pool[3 * n + 8:4 * n + 8], o], [s, p, s], [s, p, p]):
+        assert _one_launch(segs, *x, 0.2, bufs) == -5
+    wide = torch.randn(1, heads, L, 2 * d, device=dev).to(dtype)  # rows of K with room between them
+    assert _one_launch(segs, x[0], wide[..., :d].transpose(2, 3), x[2], 0.2, [s, p, wide.view(-1)[d:d + n]]) == -5
+
+
+@pytest.mark.parametrize("layout", ["rows", "keys"])
+@pytest.mark.parametrize("which", ["q", "k"])
+def test_a_modules_own_buffers_as_operands(dev, which, layout):
+    """The output of the call before (the module's buffer) as q or K of the next call: as with a copy of it."""
+    from r_attention import RegularAttention
+    heads, L, d = 24, 512, 64
+    g = torch.Generator(device=dev).manual_seed(3)
+    q, k, v, w = (torch.randn(1, heads, L, d, generator=g, device=dev).to(torch.bfloat16) for _ in range(4))
+    attn, other = (RegularAttention(1, L, heads, d, A.causal_windowed_pattern(L, d - 1), 16, 16, dev, torch.bfloat16, scale=0.125, fused=False) for _ in range(2))
+    first = attn([q, k.transpose(2, 3), v])
+    if layout == "keys" and which != "q":
+        x = lambda t: [q, t.view(1, heads, d, L), w]  # noqa: E731
+    else:
+        x = lambda t: [t, k.transpose(2, 3), w] if which == "q" else [q, t.transpose(2, 3), w]  # noqa: E731
+    want = other(x(first.clone()))
+    got = attn(x(first))
+    assert torch.equal(got, want)

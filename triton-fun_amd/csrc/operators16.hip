@@ -649,13 +649,22 @@ extern "C" int splat_operators(const void* q, int64_t q_sb, int64_t q_sh, int64_
     auto whole = [](const void* ptr, std::initializer_list<int64_t> strides) {
         return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0 && std::all_of(strides.begin(), strides.end(), [](int64_t s) { return s % 8 == 0; });
     };
+    // In separate launches an operand has been read before a later result takes its memory (K in the output of the call before, say); here workgroups
+    // store results while others still read.
+    const Extent results[] = {extent_of(scores, 2, {{B * (int64_t)H * L, T}, {T, 1}}), extent_of(probs, 2, {{B * (int64_t)H * L, T}, {T, 1}}),
+                              extent_of(out, 2, {{B * (int64_t)H * L, d}, {d, 1}})};
+    const Extent operands[] = {extent_of(q, 2, {{B, q_sb}, {H, q_sh}, {L, q_sl}, {d, 1}}), extent_of(kT, 2, {{B, k_sb}, {H, k_sh}, {d, k_sd}, {n_keys, k_sl}}),
+                               extent_of(v, 2, {{B, v_sb}, {H, v_sh}, {n_keys, v_sl}, {d, 1}})};
+    bool apart = !results[0].meets(results[1]) && !results[0].meets(results[2]) && !results[1].meets(results[2]);
+    for (const Extent& r : results)
+        for (const Extent& o : operands) apart = apart && !r.meets(o);
     const bool kt = k_sd != 1;
     p.row_stride = common_row_stride(segs, n_seg);
     const int64_t blocks = 2 * (int64_t)B * H * count_row_blocks(L, kPlanBM, p.row_stride);
     // The separate launches are faster on several segments of more than 256 slots together, whose scores go into LDS one by one: 368 slots, d = 64, 64 to
     // 512 workgroups 0.78 to 0.98 of their time, beyond 1.06 to 1.21; d = 128, 64 workgroups 1.09, 256 0.83, beyond 1.10 to 1.28.
     const bool pays = n_seg == 1 || T <= 256 || (d <= 64 ? blocks <= 512 : blocks >= 128 && blocks <= 256);
-    if (!pays || !one_step || dtype == SPLAT_F32 || d % 8 != 0 || d > 128 || T > 512 || blocks > 0x7ffffff0 || !whole(q, {q_sb, q_sh, q_sl}) || !whole(v, {v_sb, v_sh, v_sl}) ||
+    if (!pays || !apart || !one_step || dtype == SPLAT_F32 || d % 8 != 0 || d > 128 || T > 512 || blocks > 0x7ffffff0 || !whole(q, {q_sb, q_sh, q_sl}) || !whole(v, {v_sb, v_sh, v_sl}) ||
         !whole(out, {}) || (!kt && !whole(kT, {k_sb, k_sh, k_sl})))
         return SPLAT_E_UNSUPPORTED;
     p.q = q, p.k = kT, p.v = v, p.scores = scores, p.probs = probs, p.out = out;

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <initializer_list>
 #include <type_traits>
 
 #include "../../include/splat_hip.h"
@@ -32,6 +33,23 @@ int check_launch(const char* what);
 // Raise a kernel's dynamic LDS limit once per device (the attribute belongs to the device's copy of the kernel, so a
 // process that uses several GPUs needs it on each): `done` is a bit mask over device ordinals, one per kernel.
 int reserve_dynamic_lds(uint64_t* done, const void* kernel, size_t bytes, const char* who);
+
+// The bytes from the first element of a strided operand to its last one.
+struct Extent {
+    uintptr_t first, end;
+    bool meets(const Extent& o) const { return first < o.end && o.first < end; }
+};
+struct Dim {
+    int64_t size, stride;
+};
+inline Extent extent_of(const void* base, int element_bytes, std::initializer_list<Dim> dims) {
+    Extent e{reinterpret_cast<uintptr_t>(base), reinterpret_cast<uintptr_t>(base) + element_bytes};
+    for (const Dim& d : dims) {
+        const int64_t reach = (d.size - 1) * d.stride * element_bytes;
+        (reach < 0 ? e.first : e.end) += reach;
+    }
+    return e;
+}
 
 // f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>)
 template <int N, int I = 0, typename F>
