@@ -272,16 +272,21 @@ def test_results_that_share_memory_with_operands_are_left_to_the_separate_calls(
     assert _one_launch(segs, x[0], wide[..., :d].transpose(2, 3), x[2], 0.2, [s, p, wide.view(-1)[d:d + n]]) == -5
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("layout", ["rows", "keys"])
-@pytest.mark.parametrize("which", ["q", "k"])
-def test_a_modules_own_buffers_as_operands(dev, which, layout):
-    """The output of the call before (the module's buffer) as q or K of the next call: as with a copy of it."""
+@pytest.mark.parametrize("which", ["q", "k", "probabilities as k"])
+def test_a_modules_own_buffers_as_operands(dev, which, layout, dtype):
+    """The output of the call before (the module's buffer) as q or K of the next call, or its probabilities where a row has as many slots as a head has
+    values: as with a copy."""
     from r_attention import RegularAttention
     heads, L, d = 24, 512, 64
     g = torch.Generator(device=dev).manual_seed(3)
-    q, k, v, w = (torch.randn(1, heads, L, d, generator=g, device=dev).to(torch.bfloat16) for _ in range(4))
-    attn, other = (RegularAttention(1, L, heads, d, A.causal_windowed_pattern(L, d - 1), 16, 16, dev, torch.bfloat16, scale=0.125, fused=False) for _ in range(2))
+    q, k, v, w = (torch.randn(1, heads, L, d, generator=g, device=dev).to(dtype) for _ in range(4))
+    attn, other = (RegularAttention(1, L, heads, d, A.causal_windowed_pattern(L, d - 1), 16, 16, dev, dtype, scale=0.125, fused=False) for _ in range(2))
+    attn.rsoftmax_output.zero_()  # (dead slots)
     first = attn([q, k.transpose(2, 3), v])
+    if which == "probabilities as k":
+        first = attn.rsoftmax_output
     if layout == "keys" and which != "q":
         x = lambda t: [q, t.view(1, heads, d, L), w]  # noqa: E731
     else:

@@ -507,6 +507,14 @@ static int sddmm_common(const char* who, const void* q, int64_t q_sb, int64_t q_
     p.row_lse = row_lse;
     p.plan = nullptr;
     p.probs = probs;
+    if (probs) {
+        // where the probabilities take the place of an operand, other workgroups may still read it: the softmax waits for all of them in a launch of its own
+        const int size = in_dtype == SPLAT_F32 ? 4 : 2;
+        const Extent to = extent_of(probs, out_dtype == SPLAT_F32 ? 4 : 2, {{(int64_t)B * H * L, T}, {T, 1}});
+        if (to.meets(extent_of(q, size, {{B, q_sb}, {H, q_sh}, {L, q_sl}, {d, 1}})) ||
+            to.meets(extent_of(kT, size, {{B, k_sb}, {H, k_sh}, {d, k_sd}, {n_keys, k_sl}})))
+            p.probs = nullptr;
+    }
     p.probs_vec = T % 8 == 0 && ((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(probs)) & 31) == 0;
     if (plan) {
         if ((reinterpret_cast<uintptr_t>(plan) & 15) != 0) return fail(SPLAT_E_ALIGN, "%s: the plan must be 16-byte aligned", who);
