@@ -286,6 +286,22 @@ def test_float32_lists_sparse_rows_from_shorter_columns_on(dev, B, H, L, d, list
         assert err[0] <= 1.25 * err[1] and err[0] <= 1e-5, (nm, err)
 
 
+@pytest.mark.parametrize("d,local,stride,L,heads,listed", [
+    (64, 24, 32, 576, 56, False), (64, 24, 32, 640, 51, True),    # up to 512 workgroups of 64 keys: 9 and 10 tiles
+    (64, 24, 32, 320, 104, False), (64, 24, 32, 384, 87, True), (64, 24, 32, 384, 128, True), (64, 24, 32, 512, 65, True),  # up to 768: 5, 6 and 8 tiles
+    (64, 64, 64, 320, 250, False), (64, 64, 64, 384, 160, True),  # up to 1536: 4 and 5 tiles
+    (64, 16, 128, 320, 480, False), (64, 64, 64, 320, 320, True),  # beyond: 3 and 4 tiles
+    (128, 64, 64, 320, 102, False), (128, 64, 64, 384, 85, True), (128, 64, 64, 256, 130, False), (128, 64, 64, 320, 104, True),
+    (128, 64, 64, 192, 400, False), (128, 64, 64, 256, 200, True)])
+def test_float32_lists_sparse_rows_by_tiles_and_workgroups(dev, d, local, stride, L, heads, listed):
+    """Both sides of every line of the rule: the least tiles of the longest column in launches of so many workgroups."""
+    from r_backward import keys_side_schedule
+    attn = RegularAttention(1, L, heads, d, A.strided_patterns(L, local, stride), 16, 16, dev, torch.float32, scale=1.0)
+    attn._ensure_transposed()
+    assert (keys_side_schedule(attn._segments_t, L, dev, heads, f32_d=d) is not None) == listed
+    assert keys_side_schedule(attn._segments_t, L, dev, heads, always=True, f32_d=d) is not None
+
+
 def test_keys_entry_point_checks_its_arguments(dev):
     import _splat_hip as hip
     L, d, B, H = 256, 64, 1, 1

@@ -18,6 +18,7 @@ an array or tensor against its metadata and raises ``SplatError`` instead.
 """
 from __future__ import annotations
 
+import math
 from typing import Any, Sequence
 
 import numpy as np
@@ -228,12 +229,15 @@ _STRETCH, _STRETCH_F32 = 512, 128
 # the extra launch, the sum over the stretches and the scatter cost about 30 us: taken when the longest column's walk
 # (tiles of 64 queries, times the rounds in which the part runs the blocks of 128 keys) is longer than this many tiles (16-bit types)
 _WORTH_TILES = 40
-# The same for float32 and a head dimension: a tile costs more there (products of split operands, or float32 instructions), shares are kept and added in
-# float32, and the workgroups that a long column holds up are of 64 keys.  Strided masks, a training step without and with it, us, d = 64: 32 heads
-# of 512 rows (8 tiles) 64 -> 71, one of 600 (9) 65 -> 73, 8 of 640 (9) 74 -> 73, 8 of 777 (10) 77 -> 72, 32 of 777 (12) 104 -> 72, 8 of 1024 (14)
-# 94 -> 74, 16 of 2048 (30) 182 -> 87; d = 128: one of 300 (5) 87 -> 74, 64 of 300 135 -> 111, 8 of 512 (8) 119 -> 74, 8 of 1024 215 -> 113.  (Steps of
-# up to 75 us are the host's.)  Against float64, dk and dv of the listed way are closer (8 heads of 1024, d = 64: 4.1e-7 and 3.9e-7 -> 3.8e-7 and 3.5e-7).
-_WORTH_TILES_F32 = {64: 10, 128: 5}
+# The same for float32, by head dimension: the least tiles of the longest column, up to so many workgroups of 64 keys.  A tile costs more there (products of
+# split operands, or float32 instructions) and shares are kept and added in float32.  Up to 512 workgroups at d = 64 a step is the host's (of up to 75 us) and a
+# launch more is in its way: strided masks, a training step without and with it, us: 32 heads of 512 rows (8 tiles) 64 -> 71, one of 600 (9) 65 -> 73, 8 of
+# 777 (10) 77 -> 72, 16 of 2048 (30) 182 -> 87; d = 128, one of 300 (5) 87 -> 74, 8 of 1024 215 -> 113.  Beyond, three workgroups a CU at d = 64 (768) and
+# two at d = 128 (512) make a round, shares of the time with three masks: d = 64, 3 tiles 1.04 to 1.12 from 520 to 3000 workgroups; 4 tiles 1.02 to
+# 1.08 up to 800, 0.92 to 1.06 from 1025 to 1536, 0.96 to 1.01 beyond; 5 tiles 0.92 to 1.05 up to 768 (two of the masks 1.02 to 1.05), 0.90 to 1.02 up to 1024, 0.86 to
+# 0.96 beyond; 6 tiles and more 0.75 to 0.98 from 518 on; d = 128, 3 tiles 0.97 to 1.10 up to 700, 0.96 to 0.99 from 768 on, 4 tiles 0.92 to 1.01, 2 tiles 0.98
+# to 1.02.  Against float64, dk and dv of the listed way are closer (8 heads of 1024, d = 64: 4.1e-7 and 3.9e-7 -> 3.8e-7 and 3.5e-7).
+_WORTH_TILES_F32 = {64: ((512, 10), (768, 6), (1536, 5), (math.inf, 4)), 128: ((512, 5), (768, 4), (math.inf, 3))}
 
 
 def keys_side_schedule(segments_t: ACSRSegments, L: int, device, batch_heads: int,
@@ -273,8 +277,11 @@ def keys_side_schedule(segments_t: ACSRSegments, L: int, device, batch_heads: in
     if facts is False:
         return None
     sparse, first, step, cnt, key, p_min, p_max, longest_tiles = facts
-    rounds = -(-batch_heads * -(-L // (64 if f32_d else 128)) // 512)
-    if not always and longest_tiles * rounds < (_WORTH_TILES_F32[f32_d] if f32_d else _WORTH_TILES):
+    if f32_d:
+        worth = longest_tiles >= next(tiles for most, tiles in _WORTH_TILES_F32[f32_d] if batch_heads * -(-L // 64) <= most)
+    else:
+        worth = longest_tiles * -(-batch_heads * -(-L // 128) // 512) >= _WORTH_TILES
+    if not always and not worth:
         return None
     n_keys = key.numel()
     per_stretch = -(-n_keys // 128) * 128
