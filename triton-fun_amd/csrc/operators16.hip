@@ -603,12 +603,13 @@ static int launch_operators16(const Operators16Params& p, int64_t blocks, int dt
     auto by_segments = [&](auto t, auto dd, auto ps, auto nw) {
         return p.n_seg > 1 ? by_layout(t, dd, ps, nw, std::true_type{}) : by_layout(t, dd, ps, nw, std::false_type{});
     };
-    // Eight wavefronts up to two workgroups a CU, of short rows and of several segments one.  bfloat16, as shares of the separate launches' time, four and eight: 40 to
+    // Eight wavefronts up to two workgroups a CU, of short rows one.  bfloat16, as shares of the separate launches' time, four and eight: 40 to
     // 64 slots, d = 64, 256 workgroups 0.71 and 0.63, 384 0.73 and 0.77; 256 slots, d = 64, 256 workgroups 0.77 and 0.61, 512 0.68 and 0.62, 1024
-    // 0.71 and 0.76, d = 128, 1024 0.76 and 0.90; two segments, 228 slots, d = 64, 256 workgroups 0.97 and 0.77, 640 0.87 and 0.95.  Longer rows have two
-    // workgroups a CU in any case: 512 slots, d = 128, 4096 workgroups 0.94 and 0.84.
+    // 0.71 and 0.76, d = 128, 1024 0.76 and 0.90; two segments of 10 to 64 slots together 288 to 512 workgroups 0.79 to 0.88 and 0.81 to 0.90; of 83 to 256 (17 masks,
+    // d = 32 to 128, rows of K and K along the keys) 288 to 512 0.84 to 1.09 and 0.83 to 1.01, 576 and 640 0.84 to 1.02 and 0.89 to 1.15, beyond 0.67 to 1.09 and
+    // 0.78 to 1.29.  Longer rows have two workgroups a CU in any case: 512 slots, d = 128, 4096 workgroups 0.94 and 0.84.
     auto by_waves = [&](auto t, auto dd, auto ps) {
-        return blocks <= (p.T <= 64 || p.n_seg > 1 ? 256 : 512) ? by_segments(t, dd, ps, std::integral_constant<int, 8>{})
+        return blocks <= (p.T <= 64 ? 256 : 512) ? by_segments(t, dd, ps, std::integral_constant<int, 8>{})
                                                                 : by_segments(t, dd, ps, std::integral_constant<int, 4>{});
     };
     auto by_slots = [&](auto t, auto dd) {
@@ -619,6 +620,21 @@ static int launch_operators16(const Operators16Params& p, int64_t blocks, int dt
     };
     auto by_d = [&](auto t) { return p.d <= 64 ? by_slots(t, std::integral_constant<int, 64>{}) : by_slots(t, std::integral_constant<int, 128>{}); };
     return dtype == SPLAT_BF16 ? by_d(bf16{}) : by_d(f16{});
+}
+
+// The separate launches are faster on some masks of several segments, whose scores go into LDS one by one.  Shares of their time, bfloat16, two segments
+// (23 masks, heads of 1024 and 4096 rows, graphs of the forwards):
+// More than 256 slots together: rows of K, d = 32 and 64, 16 and 32 workgroups 0.97 to 1.10, 80 to 448 0.72 to 0.99, 512 at d = 64 0.90 to 0.99, at d = 32
+// 0.93 to 1.03, beyond 1.06 to 1.21; K along the keys, which is turned tile by tile, 16 to 96 workgroups 0.94 to 1.17, 128 to 448 0.70 to 1.01; d = 128, rows 64
+// workgroups 1.09, 128 to 256 0.77 to 0.97, beyond 1.10 to 1.28, keys 128 0.91 to 1.10, 192 and 256 0.76 to 0.95.
+// 129 to 256 slots, more than 512 workgroups, scores that the sampled product's wavefronts take the softmax of (own_rows_fit): d = 32 and 64 up to 2048
+// workgroups 0.78 to 1.06, at 3072 and 4096 0.89 to 1.09; d = 96 0.82 to 1.04; d = 128 up to 768 0.90 to 0.96, 1024 and 1536 0.93 to 1.07, beyond 0.86 to 1.08 with
+// a mean of 0.99.  Larger scores 0.69 to 1.01, fewer slots 0.67 to 1.01.
+static bool one_launch_pays(int n_seg, int T, int d, bool kt, int64_t blocks, int64_t score_bytes) {
+    if (n_seg == 1 || T <= 128) return true;
+    if (T > 256) return d <= 64 ? blocks >= (kt ? 128 : 80) && blocks <= (d <= 32 ? 448 : 512) : blocks >= (kt ? 192 : 128) && blocks <= 256;
+    if (score_bytes > kCachedBytes) return true;
+    return d <= 64 ? blocks <= 2048 : d <= 96 || blocks <= 768 || blocks > 1536;
 }
 
 }  // namespace splat
@@ -661,10 +677,7 @@ extern "C" int splat_operators(const void* q, int64_t q_sb, int64_t q_sh, int64_
     const bool kt = k_sd != 1;
     p.row_stride = common_row_stride(segs, n_seg);
     const int64_t blocks = 2 * (int64_t)B * H * count_row_blocks(L, kPlanBM, p.row_stride);
-    // The separate launches are faster on several segments of more than 256 slots together, whose scores go into LDS one by one: 368 slots, d = 64, 64 to
-    // 512 workgroups 0.78 to 0.98 of their time, beyond 1.06 to 1.21; d = 128, 64 workgroups 1.09, 256 0.83, beyond 1.10 to 1.28.
-    const bool pays = n_seg == 1 || T <= 256 || (d <= 64 ? blocks <= 512 : blocks >= 128 && blocks <= 256);
-    if (!pays || !apart || !one_step || dtype == SPLAT_F32 || d % 8 != 0 || d > 128 || T > 512 || blocks > 0x7ffffff0 || !whole(q, {q_sb, q_sh, q_sl}) || !whole(v, {v_sb, v_sh, v_sl}) ||
+    if (!apart || !one_launch_pays(n_seg, T, d, kt, blocks, (int64_t)B * H * L * T * 2) || !one_step || dtype == SPLAT_F32 || d % 8 != 0 || d > 128 || T > 512 || blocks > 0x7ffffff0 || !whole(q, {q_sb, q_sh, q_sl}) || !whole(v, {v_sb, v_sh, v_sl}) ||
         !whole(out, {}) || (!kt && !whole(kT, {k_sb, k_sh, k_sl})))
         return SPLAT_E_UNSUPPORTED;
     p.q = q, p.k = kT, p.v = v, p.scores = scores, p.probs = probs, p.out = out;
