@@ -318,3 +318,26 @@ def test_which_launches_of_two_segments_are_one(dev, T, d, layout, blocks, taken
         for a, b in zip(bufs, want):  # (long rows may be added in another order: one rounding apart)
             assert torch.equal(a == SENTINEL, b == SENTINEL)
             assert float(((a.float() - b.float()).abs() - eps * b.float().abs()).max()) <= 1e-4
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("mask,d", [("dilated 60 by 5", 64), ("dilated 40 by 8", 96), ("dilated 300 by 2", 128), ("dilated 300 by 2", 64), ("dilated 77 by 3", 128), ("512", 128)])
+def test_keys_that_are_turned_before_and_inside(dev, mask, d, dtype):
+    """A module's forward in many workgroups with K along the keys, on both sides of the rule for turning it first, is the one with rows of K, bit for bit;
+    two sequences whose heads lie between each other's in memory."""
+    from r_attention import RegularAttention
+    B, H, L = 2, 36, 640
+    pattern = {"dilated 60 by 5": lambda L: A.dilated_pattern(L, 60, 5), "dilated 40 by 8": lambda L: A.dilated_pattern(L, 40, 8), **MASKS}[mask](L)
+    g = torch.Generator(device=dev).manual_seed(d)
+    q, k, v = (torch.randn(H, B, L, d, generator=g, device=dev).to(dtype).transpose(0, 1) for _ in range(3))
+    attn = RegularAttention(B, L, H, d, pattern, 16, 16, dev, dtype, scale=0.2, fused=False)
+    dead = [b.fill_(SENTINEL) for b in (attn.rsddmm_output, attn.rsoftmax_output)]
+    want = [t.clone() for t in (attn([q, k.transpose(2, 3), v]), *dead)]
+    along = k.transpose(2, 3).contiguous()
+    got = attn([q, along, v])
+    for a, b in zip((got, *dead), want):
+        assert torch.equal(a, b)
+    each = RegularAttention(1, L, H, d, pattern, 16, 16, dev, dtype, scale=0.2, fused=False)  # one sequence after the other
+    for i in range(B):
+        one = each([q[i:i + 1], k[i:i + 1].transpose(2, 3), v[i:i + 1]])
+        assert torch.equal(one[0], want[0][i])

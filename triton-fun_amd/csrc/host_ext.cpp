@@ -595,13 +595,16 @@ PyObject* py_operators(PyObject*, PyObject* const* a, Py_ssize_t n) {
         if (scale == -1.0 && PyErr_Occurred()) return nullptr;
         const bool both = second.x->scalar_type() == second.out->scalar_type() && second.x->data_ptr() != second.out->data_ptr();
         const char* what;
-        // One launch, where the kernel takes it.  (K along the keys is turned on its way there, one key a lane; where neighbouring lanes' keys lie in
-        // different lines, it is turned before.)
+        // One launch, where the kernel takes it.  K along the keys is turned on its way there, one key a lane; where the separate launches would turn it
+        // and neighbouring lanes' keys lie further apart, it is turned before.  Shares of the separate launches' time, 640 to 4096 workgroups, inside and turned
+        // before (mean; bfloat16, one segment, graphs of the forwards): no step 0.48 to 0.95 (0.70) and 0.55 to 0.91 (0.76); steps of 2 to 4, up to 256 slots
+        // 0.61 to 0.91 (0.77) and 0.63 to 0.86 (0.78), longer rows d = 32 and 64 0.70 to 0.95 (0.83) and 0.67 to 0.89 (0.79), d = 80 and 128 0.78 to 1.05 (0.92)
+        // and 0.72 to 0.92 (0.83); steps of 5 to 8 0.59 to 0.92 (0.77) and 0.58 to 0.87 (0.76).
         at::Tensor turned;
         const Mask& planned = m[0]->plan.defined() ? *m[0] : *m[2];
         if (both && planned.plan.defined() && planned.one_step && first.y->size(3) == third.y->size(2) && third.x->data_ptr() == second.out->data_ptr() &&
             third.out->scalar_type() == q->scalar_type()) {
-            if (first.turn && planned.max_step > 4) {
+            if (first.turn && (planned.max_step > 4 || (planned.max_step > 1 && first.out->size(3) > 256 && q->size(3) > 64))) {
                 int rc = 0;
                 turned = transposed_keys(*first.y, &rc).transpose(2, 3);
                 if (rc) return raise_rc("splat_transpose_keys", rc);
