@@ -341,3 +341,50 @@ def test_keys_that_are_turned_before_and_inside(dev, mask, d, dtype):
     for i in range(B):
         one = each([q[i:i + 1], k[i:i + 1].transpose(2, 3), v[i:i + 1]])
         assert torch.equal(one[0], want[0][i])
+
+
+@pytest.mark.parametrize("mask", ["33", "64", "200", "512", "blocked 512", "dilated 77 by 3", "dilated 300 by 2", "strided", "strided 100"])
+@pytest.mark.parametrize("heads", [2, 54])
+def test_infinities_and_not_a_number_in_values(dev, mask, heads):
+    """Rows that see a value of infinity or NaN have it; no row that the three calls leave finite is any other here, nor any other column."""
+    L, d, dtype = 600, 64, torch.bfloat16
+    segs = _segments(MASKS[mask](L), dev)
+    q, kT, v = _operands(dev, dtype, heads, L, d, "rows")
+    v = v.clone()
+    rows, columns = [0, 100, 333, L - 1], [3, 5, 6, 7]
+    for r, c, x in zip(rows, columns, (float("inf"), float("nan"), float("-inf"), float("nan"))):
+        v[:, 0, r, c] = x
+    want, got = ([torch.full((heads, L, w), SENTINEL, dtype=dtype, device=dev) for w in (segs.T, segs.T, d)] for _ in range(2))
+    hip.check(_one_launch(segs, q, kT, v, 0.2, got), "splat_operators")
+    _three_calls(segs, q, kT, v, 0.2, want)
+    finite = torch.isfinite(got[2])
+    assert torch.all(finite | ~torch.isfinite(want[2])) and torch.all(finite[1:])
+    for r, c in zip(rows, columns):
+        sees = torch.zeros(L, dtype=torch.bool, device=dev)
+        for t, fc in zip(segs.tuples, segs.first_cols):
+            cols, live = live_slot_columns(t[2], t[3], t[4], int(t[5]), fc)
+            sees |= ((cols == r) & live).any(1)
+        assert not torch.any(finite[0, sees, c])
+    assert torch.all(finite[0][:, [c for c in range(d) if c not in columns]])
+    both = finite & torch.isfinite(want[2])
+    assert torch.allclose(got[2][both].float(), want[2][both].float(), rtol=2 * torch.finfo(dtype).eps, atol=1e-4)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("L,heads", [(600, 8), (1037, 40)])
+@pytest.mark.parametrize("mask", ["257", "509", "512", "blocked 512", "dilated 300 by 2", "strided 200"])
+def test_probabilities_of_long_rows_are_the_softmax_of_their_scores(dev, mask, L, heads, dtype):
+    """Rows of more than 256 slots, whose scores some separate launches add in another order: the probabilities are splat_softmax's of the scores that are
+    stored beside them, bit for bit."""
+    segs = _segments(MASKS[mask](L), dev)
+    d, T = 64, segs.T
+    assert T > 256
+    q, kT, v = _operands(dev, dtype, heads, L, d, "rows")
+    got = [torch.full((heads, L, w), SENTINEL, dtype=dtype, device=dev) for w in (T, T, d)]
+    rc = _one_launch(segs, q, kT, v, 0.2, got)
+    assert rc == 0 or (rc == -5 and len(segs) > 1 and heads == 40)
+    if rc == 0:
+        again = torch.full_like(got[1], SENTINEL)
+        hip.check(hip.lib().splat_softmax(got[0].data_ptr(), again.data_ptr(), segs.seg_array(L, T), len(segs), heads, L, T, hip.dtype_code(dtype),
+                                          hip.dtype_code(dtype), hip.stream_ptr(dev)), "splat_softmax")
+        assert torch.equal(got[1], again)
