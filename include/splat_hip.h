@@ -177,8 +177,8 @@ int splat_softmax(const void* x, void* y, const splat_acsr_seg* segs /* host */,
  * contiguous, dtype out_dtype, not overlapping out; rows without live slots and dead slots stay as they are in both).
  * Where the wavefronts of the sampled product own whole rows (enough row blocks for the chip), of 16-bit scores up to 512 slots and 80 MB, of float32
  * ones up to 256 slots (200 in launches of more than 2048 row blocks of 64 rows go without), they take their softmax as well, and a launch and a pass over memory are spared
- * (float16, 16 heads of 2000 rows, 129 slots, d = 80, with splat_spmm: 26.7 -> 21 us); elsewhere the second launch
- * follows.  Both results are those of the two calls, bit for bit.  Replaces r_sddmm.py:153-188 and r_softmax.py:126-150. */
+ * (float16, 16 heads of 2000 rows, 129 slots, d = 80, with splat_spmm: 26.7 -> 21 us); elsewhere, and where probs shares memory with q or kT, the
+ * second launch follows.  Both results are those of the two calls, bit for bit.  Replaces r_sddmm.py:153-188 and r_softmax.py:126-150. */
 int splat_sddmm_softmax(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* kT, int64_t k_sb,
                         int64_t k_sh, int64_t k_sd, int64_t k_sl, void* out, void* probs,
                         const splat_acsr_seg* segs /* host */, int32_t n_seg, int32_t B, int32_t H, int32_t L,
@@ -209,15 +209,19 @@ int splat_spmm_planned(const void* p, const void* v, int64_t v_sb, int64_t v_sh,
                        int32_t n_keys, int32_t n_out, int32_t T, int32_t in_dtype, int32_t out_dtype,
                        const void* plan, int64_t plan_bytes, void* stream);
 
-/* The three operators in one launch: splat_sddmm_planned's scores, splat_softmax's probabilities and splat_spmm_planned's output for q, kT, v of
- * one 16-bit dtype (scores, probs [B,H,L,T] and out [B,H,L,d] contiguous, of that dtype; scores and probs not overlapping; n_keys rows of v).
- * Scores and probabilities are those of the separate calls bit for bit and stay in the workgroup from one product to the next, so that nothing
- * reads the compressed matrices.  SPLAT_E_UNSUPPORTED, with nothing launched and no error message, where the separate calls are faster
- * (several segments of more than 256 slots together, in many launches), where scores, probs or out share memory with another of them or with an
- * operand (the separate calls are ordered, the workgroups of one launch are not) and for what the kernel does not take:
+/* The three operators in one launch: splat_sddmm_planned's scores, splat_softmax's probabilities of them and splat_spmm_planned's output for q, kT, v
+ * of one 16-bit dtype (scores, probs [B,H,L,T] and out [B,H,L,d] contiguous, of that dtype; n_keys rows of v).  Scores and probabilities stay in the
+ * workgroup from one product to the next, so that nothing reads the compressed matrices.  Up to 256 slots scores and probabilities are those of the
+ * separate calls bit for bit; of longer rows the scores may differ from them, where those run the general kernel, by the order of the float32 additions of a
+ * product of d values, and the probabilities are splat_softmax's of the scores stored here, bit for bit, in either case.  The output is splat_spmm_planned's up to the
+ * order of the additions (the same bits for one segment of at least 8 slots).  Rows of more live columns than they have slots end with the last slot.
+ * SPLAT_E_UNSUPPORTED, with nothing launched and no error message, where the separate calls are faster (several segments of more than 128 slots together, by
+ * their slots, d, kT's layout and the number of workgroups), where scores, probs or out share memory with another of them or with an operand (the
+ * separate calls are ordered, the workgroups of one launch are not) and for what the kernel does not take:
  * float32, d not a multiple of 8 or above 128, T above 512, rows that are not whole 16-byte pieces (q, v, out, and kT unless its keys
  * are contiguous).  one_step: whether splat_attention_plan_report gave 0 in [3] for every block; the kernel takes no others (with a wrong
- * answer it gives wrong results, but makes no access outside the buffers).  Replaces r_attention.py:77-100 (rsddmm_launcher, rsoftmax_launcher, rspmm_launcher). */
+ * answer, or a plan built from other metadata, it gives wrong results, but makes no access outside the buffers; columns outside [0, n_keys) stand for the
+ * nearest one).  Replaces r_attention.py:77-100 (rsddmm_launcher, rsoftmax_launcher, rspmm_launcher). */
 int splat_operators(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* kT, int64_t k_sb, int64_t k_sh,
                     int64_t k_sd, int64_t k_sl, const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sl, void* scores,
                     void* probs, void* out, const splat_acsr_seg* segs /* host */, int32_t n_seg, int32_t B, int32_t H,

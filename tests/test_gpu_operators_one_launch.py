@@ -1,4 +1,4 @@
-"""The three operators in one launch (splat_operators) against the three calls, bit for bit, and against float64: rows at the edges of what a row of
+"""The three operators in one launch (splat_operators) against the three calls, bit for bit where those add in its order, and against float64: rows at the edges of what a row of
 LDS holds, row blocks that interleave, two segments, rows whose steps differ, heads that are padded, K along the keys, sequences that end
 inside a workgroup and inside a wavefront's rows."""
 import ctypes

@@ -4,8 +4,8 @@ Mirrors the reference's ``SPLAT/r_attention.py``: ``RegularAttention`` (:12-100)
 signature, attribute names and ``forward([q, kT, v])``; ``unit`` (:102-110) keeps its signature.
 
 Differences, all opt-in or invisible to a caller of the reference:
-  * ``forward`` runs the fused online-softmax kernel by default (``fused=False`` gives the three launches);
-    the two [B, H, L, T] intermediates are therefore allocated on first use, not in ``__init__``;
+  * ``forward`` runs the fused online-softmax kernel by default (``fused=False`` gives the three operators, whose
+    compressed matrices are in memory afterwards, in one to four launches); the two [B, H, L, T] intermediates are therefore allocated on first use, not in ``__init__``;
   * ``scale`` (default 1.0: the reference applies no softmax scale) multiplies the scores;
   * ``mask`` may be a list of lists (reference), an array / tensor, a ``MaskPattern`` or a list of
     ``MaskPattern`` segments (several affine segments per row).

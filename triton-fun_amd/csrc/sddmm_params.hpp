@@ -33,7 +33,10 @@ struct SddmmParams {
     int probs_vec;  // T % 8 == 0, and out and probs start on 32-byte boundaries
 };
 
-// Whether softmax_own_rows pays.  Float32: rows of up to 256 slots (of 300 1.05 of the time of a launch for each, of 512 1.03 to 1.13).  16-bit
+// Whether softmax_own_rows pays.  (The figures are of the three operators as two launches and three.  16-bit forwards whose masks step alike within a block and whose
+// rows are whole 16-byte pieces are one launch since, operators16.hip, but for several segments where that does not pay; here come the others, rows of other
+// addresses or strides, blocks whose rows step differently, and calls of these two operators alone.)
+//  Float32: rows of up to 256 slots (of 300 1.05 of the time of a launch for each, of 512 1.03 to 1.13).  16-bit
 // types: rows of up to 512 slots and scores that the caches hold: causal masks of 33 to 256 slots, d = 64 and 128, the three operators 0.68 to 0.99 of
 // the time up to 80 MB of scores, the two alone 0.82 to 1.25 from 100 to 170 MB.  (Scores and probabilities are stored through the caches
 // then: 4096 rows of 200 slots, 16 heads, d = 128 60 -> 41 us, of which 53 around them.)  Of rows of more than 256 slots the workgroups that have
